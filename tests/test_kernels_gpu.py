@@ -137,6 +137,46 @@ def test_decode_attention(group, ctx):
     assert_close(out, expect, msg=f"group={group} ctx={ctx}")
 
 
+@pytest.mark.parametrize("hd,group,dtype,cache_dtype,window", [
+    (128, 7, torch.bfloat16, torch.bfloat16, 0),
+    (128, 4, torch.bfloat16, torch.bfloat16, 150),
+    (64, 3, torch.bfloat16, torch.float8_e4m3fn, 0),
+    (256, 5, torch.bfloat16, torch.float8_e4m3fn, 33),
+    (128, 8, torch.float16, torch.float16, 0),
+    (64, 1, torch.float16, torch.float8_e4m3fn, 1),
+])
+@pytest.mark.parametrize("n", [6, 300])  # split and unsplit keys
+def test_decode_attention_edges(hd, group, dtype, cache_dtype, window, n):
+    """Ragged rows at the edges of a wave's 32 keys, a workgroup's 128
+    and a cache block; rows of the last block that no token has written
+    hold NaN. Tolerance: the output's own rounding, 2^-8 (bf16) or
+    2^-11 (fp16) of values up to 4, once more for the order of sums."""
+    hip = _hip()
+    Hkv = 2
+    lens = [1, 31, 33, 64, 129, 640]
+    ctx = [lens[i % 6] for i in range(n)]
+    q, cache, bt, qsl, sl = _make_paged(n, [1] * n, ctx, Hkv * group, Hkv,
+                                        D=hd)
+    q = q.to(dtype)
+    cache = cache.to(cache_dtype)
+    nan = torch.tensor(float("nan"), device="cuda").to(cache_dtype)
+    raw = cache if cache_dtype != torch.float8_e4m3fn \
+        else cache.view(torch.uint8)
+    for i in range(6):
+        if ctx[i] % 64:
+            raw[:, bt[i, ctx[i] // 64], :, ctx[i] % 64:] = \
+                nan.view(raw.dtype) if raw.dtype == torch.uint8 else nan
+    out = hip.attention_unified(q, cache, bt, qsl, sl, hd**-0.5,
+                                num_decodes=n, max_seq_len=max(ctx),
+                                max_query_len=1, sliding_window=window)
+    rows = list(range(6))
+    expect = ref.attention_unified(
+        q[rows].float(), cache.float(), bt[rows], qsl[:7], sl[rows],
+        hd**-0.5, num_decodes=6, sliding_window=window)
+    atol = 2 * 4 * (2**-8 if dtype == torch.bfloat16 else 2**-11)
+    assert_close(out[rows], expect, atol=atol, rtol=atol / 4)
+
+
 @pytest.mark.parametrize("group", [4])
 @pytest.mark.parametrize(
     "q_lens,ctx_lens",

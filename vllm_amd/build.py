@@ -39,6 +39,11 @@ SOURCES = [
     CSRC / "bindings.cpp",
 ]
 
+# These kernels keep matrix-core accumulators in ordinary vector
+# registers: they are rescaled by the vector ALU between products, and
+# through the accumulation registers every rescale is a copy each way.
+VGPR_ACCUMULATORS = {"attention_decode"}
+
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("PYTORCH_ROCM_ARCH", "gfx950")
 
@@ -101,6 +106,8 @@ def build(verbose: bool = True) -> Path:
         if src.suffix == ".hip":
             cmd.insert(1, "-x")
             cmd.insert(2, "hip")
+        if src.stem in VGPR_ACCUMULATORS:
+            cmd += ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
         cmds.append(cmd)
         objs.append(str(obj))
 

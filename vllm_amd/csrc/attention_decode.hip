@@ -1,22 +1,35 @@
 // Paged decode attention for MI355X (gfx950, CDNA4).
 //
-// Design (MI355X-first, not a port):
-//   Decode attention is HBM-bandwidth bound: per context token and KV head
-//   the kernel reads 2*D*2 bytes of K+V and does GQA_group*4*D flops —
-//   arithmetic intensity = group flops/byte (≈4-8), far below the
-//   157 TF / 6.3 TB/s = 25 flops/byte VALU roofline. So this kernel is a
-//   pure-VALU streaming kernel tuned for the load path, not MFMA:
-//   16B/lane short8 K/V loads (G13), 16-lane thread groups per token,
-//   flash-decoding partitions of PART tokens with a separate LSE-merge
-//   reduce kernel for long contexts.
+// What bounds it: one pass over the cached keys and values. At 2..16
+// flops per byte everything else only has to stay out of the way of the
+// loads, so the kernel keeps as many bytes in flight as registers allow
+// and spends few issue slots per byte:
+//   - A wave owns 32 keys at a time and never meets another wave before
+//     the end, so there is no barrier in the loop. The next 32 keys are
+//     loaded as soon as the registers of the current ones are free.
+//   - Scores are S^T = K Q^T on the matrix cores: a K row goes from HBM
+//     straight into the A fragment (16 B per lane), the query heads of
+//     the group are the 16 columns. No cross-lane sum per key and head,
+//     which is what the vector-ALU form of this kernel spent its time on.
+//   - O^T = V^T P^T: V passes through this wave's own LDS slice to be
+//     transposed on the read. The lane that holds the scores of keys
+//     (4g..4g+3, 16+4g..) holds exactly the P^T fragment of those keys
+//     when the contraction runs over keys in that order, so P never
+//     moves between lanes.
+//   - P stays at more than 16 bits: it is split in two 16-bit parts
+//     (p = hi + lo, error 2^-17) and multiplied twice; the matrix cores
+//     are idle here anyway. Sums and outputs are fp32.
+// Against the vector-ALU form it replaced (16 lanes per token, dot
+// products reduced with shuffles), us per layer at 32 query and 8 KV
+// heads of 128:
+//   1 x 1000 keys 46 -> 13; 256 x 129..2176 keys 346 -> 227 (5.3 TB/s);
+//   1024 x 129..176 keys 215 -> 128 (5.0 TB/s);
+//   64 x 4096..8192 keys, fp8 cache 371 -> 154 (5.2 TB/s).
 //
-//   The KV cache layout [2, blocks, kv_heads, block_size=64, D] keeps each
-//   (block, head) tile contiguous (16 KB at D=128), so a partition is a
-//   handful of fully-coalesced streams.
+// The KV cache layout [2, blocks, kv_heads, block_size=64, D] keeps each
+// (block, head) tile contiguous (16 KB at D=128).
 //
-// Role of the reference's paged_attention (csrc/rocm/attention.cu:321,1420),
-// re-designed: the reference packs GQA into MFMA16 tiles; on MI355X the
-// memory-bound regime makes VALU dot products simpler and just as fast.
+// Role of the reference's paged_attention (csrc/rocm/attention.cu:321,1420).
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
@@ -25,24 +38,31 @@
 
 namespace vllm_amd {
 
-// Tunables. PART must be a multiple of the token-iteration width
-// (BLOCK/16 tokens per iteration) and of the cache block size (64).
-constexpr int DEC_BLOCK = 256;          // threads per workgroup (4 waves)
-constexpr int DEC_PART = 512;           // context tokens per partition
-constexpr int MAX_GROUP = 8;            // max GQA ratio handled in registers
+constexpr int DEC_WAVES = 4;
+constexpr int DEC_BLOCK = DEC_WAVES * WAVE_SIZE;
+constexpr int DEC_KEYS = 32;    // keys per wave and step
+constexpr int MAX_GROUP = 8;    // query heads per KV head
+constexpr float DEC_NEG = -3.0e38f;
+constexpr float DEC_LOG2E = 1.4426950408889634f;
 
-// One workgroup: (decode seq, kv head, partition). Computes the partial
-// attention output for GROUP query heads over PART context tokens with an
-// unnormalized softmax (running max m, exp-sum l), writing either the
-// final bf16 output (single partition) or fp32 partials + (m, l) scratch.
-//
-// Thread layout: 16 lanes per token (lane d covers dims 8d..8d+7 as one
-// short8 = 16 B load), so a 256-thread block streams 16 tokens per
-// iteration; DEC_PART/16 = 32 iterations.
-// HD = head_dim (64/128/256). LPT = HD/8 lanes cover one token's dims
-// (8 dims per lane, one 16 B load); SLOTS = DEC_BLOCK/LPT token slots
-// stream in parallel, two tokens per slot-iteration.
-template <typename Tag, typename CTag, int GROUP, bool FINAL, int HD>
+// Bytes of a V row are moved in 32 B segments (16 columns, what one
+// transposing read takes from a row). Rotating the segments by the row
+// spreads the rows a read touches over all 64 banks.
+template <int HD> DEVINL int v_slot(int row, int seg) {
+  if constexpr (HD == 64) return seg ^ ((row >> 1) & 3);
+  return seg ^ (row & 7);
+}
+
+// First key this row attends, rounded down so that a wave's 32 keys
+// never leave a cache block.
+DEVINL int dec_base(int ctx, int window) {
+  return window > 0 ? (max(0, ctx - window) & ~(DEC_KEYS - 1)) : 0;
+}
+
+// One workgroup: (kv head, decode row, partition of part_len keys).
+// Writes the final 16-bit output (FINAL) or fp32 partials with their
+// running maximum (log2 domain) and sum.
+template <typename Tag, typename CTag, bool FINAL, int HD>
 __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
     short* __restrict__ out,            // FINAL: [Tdec, Hq, D] (16-bit)
     float* __restrict__ tmp_out,        // else: [Tdec, Hq, parts, D]
@@ -52,244 +72,328 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
                                         // [2, blocks, Hkv, 64, D]
     const int* __restrict__ block_table,   // [num_reqs, max_blocks]
     const int* __restrict__ seq_lens,      // [num_reqs]
-    const float scale, const int num_q_heads, const int num_kv_heads,
-    const int head_dim, const int max_blocks_per_req, const int num_parts,
+    const float scale_log2, const int group, const int num_kv_heads,
+    const int max_blocks_per_req, const int num_parts, const int part_len,
     const int64_t kv_plane_stride,      // elements between K and V planes
     const int64_t q_stride,             // elements between q token rows
     const int sliding_window) {
-  const int seq = blockIdx.x;       // decode row == request row
-  const int kvh = blockIdx.y;
+  using elem = typename CacheTraits<CTag>::elem;
+  constexpr bool FP8 = sizeof(elem) == 1;
+  constexpr int EPV = 16 / sizeof(elem);          // elements per 16 B
+  constexpr int KF = HD / 32;                     // MFMA steps over D
+  constexpr int KN = HD * (int)sizeof(elem) / 64; // 16 B K loads per row
+  constexpr int VN = DEC_KEYS * HD / EPV / WAVE_SIZE;
+  constexpr int DS = HD / 16;                     // output column tiles
+  constexpr int V_BYTES = DEC_KEYS * HD * 2;      // per wave
+
+  const int kvh = blockIdx.x;
+  const int seq = blockIdx.y;       // decode row == request row
   const int part = blockIdx.z;
   const int ctx = seq_lens[seq];
-
-  int t_begin = part * DEC_PART;
-  int t_end = min(ctx, t_begin + DEC_PART);
-  if (sliding_window > 0) {
-    // Query position is ctx-1; keys < ctx - sliding_window are masked.
-    t_begin = max(t_begin, ctx - sliding_window);
-  }
-  const int hq0 = kvh * GROUP;  // first query head of this group
+  const int num_q_heads = num_kv_heads * group;
+  const int hq0 = kvh * group;
+  const int t_lo = sliding_window > 0 ? max(0, ctx - sliding_window) : 0;
+  const int t_begin = dec_base(ctx, sliding_window) + part * part_len;
+  const int t_end = min(ctx, t_begin + part_len);
 
   if (t_begin >= t_end) {
-    if (!FINAL && threadIdx.x < GROUP * 2) {
+    if (!FINAL && threadIdx.x < group * 2) {
       const int g = threadIdx.x / 2;
-      float* lse = tmp_lse +
-          (((int64_t)seq * num_q_heads + hq0 + g) * num_parts + part) * 2;
-      lse[threadIdx.x % 2] = (threadIdx.x % 2 == 0) ? -3.0e38f : 0.f;
+      tmp_lse[(((int64_t)seq * num_q_heads + hq0 + g) * num_parts + part) *
+                  2 + threadIdx.x % 2] =
+          (threadIdx.x % 2 == 0) ? DEC_NEG : 0.f;
     }
     return;
   }
 
-  constexpr int LPT = HD / 8;                   // lanes per token
-  constexpr int SLOTS_PER_WAVE = WAVE_SIZE / LPT;
-  constexpr int SLOTS = DEC_BLOCK / LPT;
-  const int lane_d = threadIdx.x & (LPT - 1);   // dim-slice owner
-  const int slot = (threadIdx.x / LPT) % SLOTS_PER_WAVE;
-  const int wave = threadIdx.x / WAVE_SIZE;     // 0..3
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lane = threadIdx.x % WAVE_SIZE;
+  const int l16 = lane & 15;
+  const int l4 = lane >> 4;
 
-  // LDS: physical block ids + cross-wave merge scratch.
-  __shared__ int blk_ids[DEC_PART / 64];
-  __shared__ float ml_red[4][GROUP][2];       // per-wave (m, l)
-  __shared__ float o_red[4][GROUP][HD];       // per-wave accumulators
+  // V slices of the waves; reused for the merge of the waves at the end
+  // (group <= 8 of the 16 columns, so it always fits).
+  __shared__ __align__(16) char lds[DEC_WAVES * V_BYTES];
+  __shared__ float ml_red[DEC_WAVES][MAX_GROUP][2];
+  char* v_lds = lds + wave * V_BYTES;
 
-  if (threadIdx.x < DEC_PART / 64) {
-    const int cache_blk = (part * DEC_PART) / 64 + threadIdx.x;
-    blk_ids[threadIdx.x] =
-        block_table[(int64_t)seq * max_blocks_per_req + cache_blk];
-  }
-  __syncthreads();
-
-  // Q fragment: each lane16 holds its 8-dim slice for all GROUP heads.
-  float qf[GROUP][8];
+  // B fragments of the queries: column l16 is a head of the group, the
+  // others repeat head 0 and are never written out.
+  s16x8 qf[KF];
   {
-    const short* qbase =
-        q + (int64_t)seq * q_stride + hq0 * head_dim + lane_d * 8;
+    const short* qb = q + (int64_t)seq * q_stride +
+                      (int64_t)(hq0 + (l16 < group ? l16 : 0)) * HD;
 #pragma unroll
-    for (int g = 0; g < GROUP; ++g) {
-      s16x8 v = *reinterpret_cast<const s16x8*>(qbase + g * head_dim);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) qf[g][j] = to_f32<Tag>(v[j]) * scale;
+    for (int kk = 0; kk < KF; ++kk) {
+      // With an fp8 cache a 16 B load is two fragments' worth of one
+      // row, so the dims of a step are interleaved differently.
+      const int d = FP8 ? (kk >> 1) * 64 + l4 * 16 + (kk & 1) * 8
+                        : kk * 32 + l4 * 8;
+      qf[kk] = *reinterpret_cast<const s16x8*>(qb + d);
     }
   }
 
-  // ---- single pass: online softmax per (wave, slot) ----------------------
-  // Each slot streams tokens t = t_begin + wave*4 + slot + 16*i. K and V
-  // rows are read once, 16 B per lane (G13); no syncthreads in the loop, so
-  // the 4 waves keep the HBM pipeline full independently.
-  const int64_t head_tile_stride = (int64_t)64 * head_dim;  // one (blk,head)
-  float m_s[GROUP], l_s[GROUP], acc[GROUP][8];
+  const int* bt = block_table + (int64_t)seq * max_blocks_per_req;
+  auto tile_of = [&](int key0) {
+    return kv_cache +
+           ((int64_t)bt[key0 >> 6] * num_kv_heads + kvh) * (64 * HD) +
+           (key0 & 63) * HD;
+  };
+  i32x4 kr[2][KN], vr[VN];
+  auto load_k = [&](const elem* tile) {
 #pragma unroll
-  for (int g = 0; g < GROUP; ++g) {
-    m_s[g] = -3.0e38f;
-    l_s[g] = 0.f;
+    for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-  }
+      for (int i = 0; i < KN; ++i)
+        kr[s][i] = *reinterpret_cast<const i32x4*>(
+            tile + (s * 16 + l16) * HD + (i * 4 + l4) * EPV);
+  };
+  auto load_v = [&](const elem* tile) {
+#pragma unroll
+    for (int i = 0; i < VN; ++i)
+      vr[i] = *reinterpret_cast<const i32x4*>(
+          tile + kv_plane_stride + (i * WAVE_SIZE + lane) * EPV);
+  };
 
-  // Two tokens per (wave, slot) iteration: doubles the K/V loads in
-  // flight per lane and halves the online-softmax update chain.
-  const int t0_base = t_begin + wave * SLOTS_PER_WAVE + slot;
-  for (int t = t0_base; t < t_end; t += 2 * SLOTS) {
-    const int t1 = t + SLOTS;
-    const bool has1 = t1 < t_end;
-    using CT = CacheTraits<CTag>;
-    using cvec = typename CT::vec8;
-    const int local0 = t - part * DEC_PART;
-    const typename CT::elem* base0 = kv_cache +
-        ((int64_t)blk_ids[local0 / 64] * num_kv_heads + kvh) *
-            head_tile_stride +
-        (int64_t)(t % 64) * head_dim + lane_d * 8;
-    const int local1 = has1 ? t1 - part * DEC_PART : local0;
-    const typename CT::elem* base1 = has1 ? kv_cache +
-        ((int64_t)blk_ids[local1 / 64] * num_kv_heads + kvh) *
-            head_tile_stride +
-        (int64_t)(t1 % 64) * head_dim + lane_d * 8 : base0;
-    cvec k0 = *reinterpret_cast<const cvec*>(base0);
-    cvec v0 = *reinterpret_cast<const cvec*>(base0 + kv_plane_stride);
-    cvec k1 = *reinterpret_cast<const cvec*>(base1);
-    cvec v1 = *reinterpret_cast<const cvec*>(base1 + kv_plane_stride);
-    float kf0[8], vf0[8], kf1[8], vf1[8];
+  float m_run = DEC_NEG, l_run = 0.f;   // of head l16; l: this lane's keys
+  f32x4 o[DS];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      kf0[j] = CT::get(k0, j);
-      vf0[j] = CT::get(v0, j);
-      kf1[j] = CT::get(k1, j);
-      vf1[j] = CT::get(v1, j);
+  for (int i = 0; i < DS; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // One step of 32 keys; with NEXT the loads of the wave's next 32 are
+  // issued as the registers become free (a template flag and not a test
+  // inside, so that the waits count exactly the older loads).
+  auto step = [&](int key0, auto has_next) {
+    constexpr bool NEXT = decltype(has_next)::value;
+    const elem* next_tile =
+        NEXT ? tile_of(key0 + DEC_WAVES * DEC_KEYS) : nullptr;
+    // ---- S^T: rows are keys, columns heads -----------------------------
+    f32x4 s[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < KF; ++kk) {
+        s16x8 a;
+        if constexpr (FP8) {
+          const i32x4 r = kr[t][kk >> 1];
+          const int2 x = fp8x4_widen<Tag>(r[(kk & 1) * 2]);
+          const int2 y = fp8x4_widen<Tag>(r[(kk & 1) * 2 + 1]);
+          a = __builtin_bit_cast(s16x8, (i32x4){x.x, x.y, y.x, y.y});
+        } else {
+          a = __builtin_bit_cast(s16x8, kr[t][kk]);
+        }
+        s[t] = mfma16<Tag>(a, qf[kk], s[t]);
+      }
+    }
+    if constexpr (NEXT) load_k(next_tile);
+
+    // ---- V to LDS, rows outside [t_lo, t_end) as zeros ------------------
+    // (a stale cache row may hold anything, and 0 * NaN is NaN).
+    const bool edge = key0 < t_lo || key0 + DEC_KEYS > t_end;
+    if (edge) {
+#pragma unroll
+      for (int i = 0; i < VN; ++i) {
+        const int key = key0 + (i * WAVE_SIZE + lane) * EPV / HD;
+        const bool in = (key >= t_lo) & (key < t_end);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vr[i][j] = in ? vr[i][j] : 0;
+      }
     }
 #pragma unroll
-    for (int g = 0; g < GROUP; ++g) {
-      float sc0 = 0.f, sc1 = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        sc0 += qf[g][j] * kf0[j];
-        sc1 += qf[g][j] * kf1[j];
-      }
-      // Reduce over the LPT dim lanes of this slot (consecutive lanes).
-#pragma unroll
-      for (int off = 1; off < LPT; off <<= 1) {
-        sc0 += __shfl_xor(sc0, off, 64);
-        sc1 += __shfl_xor(sc1, off, 64);
-      }
-      if (!has1) sc1 = -3.0e38f;
-      const float m_new = fmaxf(m_s[g], fmaxf(sc0, sc1));
-      const float p0 = __expf(sc0 - m_new);
-      const float p1 = has1 ? __expf(sc1 - m_new) : 0.f;
-      if (m_new > m_s[g]) {
-        const float corr = __expf(m_s[g] - m_new);
-        l_s[g] = l_s[g] * corr + p0 + p1;
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          acc[g][j] = acc[g][j] * corr + p0 * vf0[j] + p1 * vf1[j];
-        m_s[g] = m_new;
+    for (int i = 0; i < VN; ++i) {
+      const int e = (i * WAVE_SIZE + lane) * EPV;
+      const int row = e / HD;
+      const i32x4 v = vr[i];
+      const int c16 = (e % HD) / 8;   // 16 B chunk of the 16-bit row
+      char* dst = v_lds + row * (HD * 2) + v_slot<HD>(row, c16 >> 1) * 32;
+      if constexpr (FP8) {
+        const int2 a = fp8x4_widen<Tag>(v[0]), b = fp8x4_widen<Tag>(v[1]);
+        const int2 c = fp8x4_widen<Tag>(v[2]), d = fp8x4_widen<Tag>(v[3]);
+        i32x4* p = reinterpret_cast<i32x4*>(dst);
+        p[0] = i32x4{a.x, a.y, b.x, b.y};
+        p[1] = i32x4{c.x, c.y, d.x, d.y};
       } else {
-        l_s[g] += p0 + p1;
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          acc[g][j] += p0 * vf0[j] + p1 * vf1[j];
+        *reinterpret_cast<i32x4*>(dst + (c16 & 1) * 16) = v;
       }
     }
-  }
+    if constexpr (NEXT) load_v(next_tile);
 
-  // ---- merge the slots within each wave (butterfly over lanes LPT..32) ---
+    // ---- running softmax, log2 domain ----------------------------------
+    // A key outside the row's range scores DEC_NEG and weighs nothing
+    // even where the whole step is outside it.
+    bool in[2][4];
+    float mx = DEC_NEG;
 #pragma unroll
-  for (int off = LPT; off <= 32; off <<= 1) {
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int g = 0; g < GROUP; ++g) {
-      const float m_o = __shfl_xor(m_s[g], off, 64);
-      const float l_o = __shfl_xor(l_s[g], off, 64);
-      const float M = fmaxf(m_s[g], m_o);
-      const float c1 = __expf(m_s[g] - M);
-      const float c2 = __expf(m_o - M);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float a_o = __shfl_xor(acc[g][j], off, 64);
-        acc[g][j] = acc[g][j] * c1 + a_o * c2;
+      for (int r = 0; r < 4; ++r) {
+        const int key = key0 + t * 16 + l4 * 4 + r;
+        in[t][r] = (key >= t_lo) & (key < t_end);
+        s[t][r] = in[t][r] ? s[t][r] * scale_log2 : DEC_NEG;
+        mx = fmaxf(mx, s[t][r]);
       }
-      l_s[g] = l_s[g] * c1 + l_o * c2;
-      m_s[g] = M;
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(m_run, mx);
+    if (__any(m_new > m_run)) {
+      const float f = __builtin_amdgcn_exp2f(m_run - m_new);
+      l_run *= f;
+#pragma unroll
+      for (int i = 0; i < DS; ++i) o[i] *= f;
+      m_run = m_new;
     }
+    i32x4 hi, lo;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; r += 2) {
+        const float e0 = __builtin_amdgcn_exp2f(s[t][r] - m_run);
+        const float e1 = __builtin_amdgcn_exp2f(s[t][r + 1] - m_run);
+        const float p0 = in[t][r] ? e0 : 0.f;
+        const float p1 = in[t][r + 1] ? e1 : 0.f;
+        l_run += p0 + p1;
+        const int h = pack2<Tag>(p0, p1);
+        hi[t * 2 + r / 2] = h;
+        lo[t * 2 + r / 2] =
+            pack2<Tag>(p0 - unpack_lo<Tag>(h), p1 - unpack_hi<Tag>(h));
+      }
+    const s16x8 p_hi = __builtin_bit_cast(s16x8, hi);
+    const s16x8 p_lo = __builtin_bit_cast(s16x8, lo);
+
+    // ---- O^T += V^T P^T -------------------------------------------------
+    // LDS operations of one wave complete in order; the fences only keep
+    // the compiler from moving them.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int row = l4 * 4 + (l16 >> 2);
+#pragma unroll
+    for (int i = 0; i < DS; ++i) {
+      const int off = (l16 & 3) * 8;
+      const s16x4 a = lds_read_tr(v_lds + row * (HD * 2) +
+                                  v_slot<HD>(row, i) * 32 + off);
+      const s16x4 b = lds_read_tr(v_lds + (row + 16) * (HD * 2) +
+                                  v_slot<HD>(row + 16, i) * 32 + off);
+      const s16x8 v = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+      o[i] = mfma16<Tag>(v, p_lo, o[i]);
+      o[i] = mfma16<Tag>(v, p_hi, o[i]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+
+  int key0 = t_begin + wave * DEC_KEYS;
+  if (key0 < t_end) {
+    const elem* tile = tile_of(key0);
+    load_k(tile);
+    load_v(tile);
+    for (; key0 + DEC_WAVES * DEC_KEYS < t_end; key0 += DEC_WAVES * DEC_KEYS)
+      step(key0, std::true_type{});
+    step(key0, std::false_type{});
   }
 
-  // ---- merge the 4 waves via LDS ------------------------------------------
-  if ((threadIdx.x & 63) < LPT) {
+  // ---- merge the waves ----------------------------------------------------
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  __syncthreads();   // every wave is done with its V slice
+  float* o_red = reinterpret_cast<float*>(lds);  // [wave][MAX_GROUP][HD]
+  static_assert(MAX_GROUP * HD * 4 <= V_BYTES, "merge scratch");
+  if (l16 < group) {
 #pragma unroll
-    for (int g = 0; g < GROUP; ++g) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o_red[wave][g][lane_d * 8 + j] = acc[g][j];
-      if (lane_d == 0) {
-        ml_red[wave][g][0] = m_s[g];
-        ml_red[wave][g][1] = l_s[g];
-      }
+    for (int i = 0; i < DS; ++i)
+      *reinterpret_cast<f32x4*>(
+          o_red + (wave * MAX_GROUP + l16) * HD + i * 16 + l4 * 4) = o[i];
+    if (l4 == 0) {
+      ml_red[wave][l16][0] = m_run;
+      ml_red[wave][l16][1] = l_run;
     }
   }
   __syncthreads();
-  // HD threads: one per dim; every thread recomputes the scalar merge.
-  if (threadIdx.x < HD) {
-    const int d = threadIdx.x;
+  for (int e = threadIdx.x; e < group * HD; e += DEC_BLOCK) {
+    const int g = e / HD;
+    const int d = e % HD;
+    float M = DEC_NEG;
 #pragma unroll
-    for (int g = 0; g < GROUP; ++g) {
-      float M = fmaxf(fmaxf(ml_red[0][g][0], ml_red[1][g][0]),
-                      fmaxf(ml_red[2][g][0], ml_red[3][g][0]));
-      float L = 0.f, o = 0.f;
+    for (int w = 0; w < DEC_WAVES; ++w) M = fmaxf(M, ml_red[w][g][0]);
+    float L = 0.f, acc = 0.f;
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const float c = __expf(ml_red[w][g][0] - M);
-        L += ml_red[w][g][1] * c;
-        o += o_red[w][g][d] * c;
-      }
-      if (FINAL) {
-        const float inv_l = L > 0.f ? 1.f / L : 0.f;
-        out[((int64_t)seq * num_q_heads + hq0 + g) * head_dim + d] =
-            from_f32<Tag>(o * inv_l);
-      } else {
-        tmp_out[((((int64_t)seq * num_q_heads + hq0 + g) * num_parts + part) *
-                 head_dim) + d] = o;
-        if (d == 0) {
-          float* lse = tmp_lse +
-              (((int64_t)seq * num_q_heads + hq0 + g) * num_parts + part) * 2;
-          lse[0] = M;
-          lse[1] = L;
-        }
+    for (int w = 0; w < DEC_WAVES; ++w) {
+      const float c = __builtin_amdgcn_exp2f(ml_red[w][g][0] - M);
+      L += ml_red[w][g][1] * c;
+      acc += o_red[(w * MAX_GROUP + g) * HD + d] * c;
+    }
+    if constexpr (FINAL) {
+      const float inv_l = L > 0.f || L != L ? 1.f / L : 0.f;
+      out[((int64_t)seq * num_q_heads + hq0 + g) * HD + d] =
+          from_f32<Tag>(acc * inv_l);
+    } else {
+      const int64_t row =
+          ((int64_t)seq * num_q_heads + hq0 + g) * num_parts + part;
+      tmp_out[row * HD + d] = acc;
+      if (d == 0) {
+        tmp_lse[row * 2] = M;
+        tmp_lse[row * 2 + 1] = L;
       }
     }
   }
 }
 
-// Merge per-partition partials: out = sum_p o_p * exp(m_p - M) / sum_p
-// l_p * exp(m_p - M). Grid (Tdec, Hq), block = D threads (one per dim).
-template <typename Tag>
-__global__ void paged_decode_reduce_kernel(
+// Merge per-partition partials: out = sum_p o_p 2^(m_p - M) / sum_p l_p
+// 2^(m_p - M). One wave per (row, head); lane p weighs partition p, then
+// every lane sums its own dims over the partitions (independent loads).
+template <typename Tag, int HD>
+__global__ __launch_bounds__(WAVE_SIZE) void paged_decode_reduce_kernel(
     short* __restrict__ out,           // [Tdec, Hq, D]
     const float* __restrict__ tmp_out, // [Tdec, Hq, parts, D]
     const float* __restrict__ tmp_lse, // [Tdec, Hq, parts, 2]
     const int* __restrict__ seq_lens, const int num_parts,
-    const int head_dim, const int num_q_heads) {
-  const int seq = blockIdx.x;
-  const int h = blockIdx.y;
-  const int d = threadIdx.x;
-  const int used_parts = min(num_parts, (seq_lens[seq] + DEC_PART - 1) /
-                                            DEC_PART);
-  const float* lse =
-      tmp_lse + (((int64_t)seq * num_q_heads + h) * num_parts) * 2;
-  float M = -3.0e38f;
-  for (int p = 0; p < used_parts; ++p) M = fmaxf(M, lse[p * 2]);
-  float L = 0.f;
-  for (int p = 0; p < used_parts; ++p)
-    L += lse[p * 2 + 1] * __expf(lse[p * 2] - M);
-  const float inv_l = L > 0.f ? 1.f / L : 0.f;
-  const float* o_base =
-      tmp_out + (((int64_t)seq * num_q_heads + h) * num_parts) * head_dim;
-  float o = 0.f;
-  for (int p = 0; p < used_parts; ++p)
-    o += o_base[p * head_dim + d] * __expf(lse[p * 2] - M);
-  out[((int64_t)seq * num_q_heads + h) * head_dim + d] =
-      from_f32<Tag>(o * inv_l);
+    const int part_len, const int num_q_heads, const int sliding_window) {
+  constexpr int V = HD / WAVE_SIZE;   // dims per lane (1, 2 or 4)
+  const int h = blockIdx.x;
+  const int seq = blockIdx.y;
+  const int lane = threadIdx.x;
+  const int ctx = seq_lens[seq];
+  const int span = ctx - dec_base(ctx, sliding_window);
+  const int used = min(num_parts, (span + part_len - 1) / part_len);
+  const int64_t row = ((int64_t)seq * num_q_heads + h) * num_parts;
+  float M = DEC_NEG, L = 0.f, acc[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) acc[j] = 0.f;
+  for (int p0 = 0; p0 < used; p0 += WAVE_SIZE) {
+    const int n = min(WAVE_SIZE, used - p0);
+    float m = DEC_NEG, l = 0.f;
+    if (lane < n) {
+      m = tmp_lse[(row + p0 + lane) * 2];
+      l = tmp_lse[(row + p0 + lane) * 2 + 1];
+    }
+    const float m_new = fmaxf(M, wave_reduce_max(m));
+    const float f = __builtin_amdgcn_exp2f(M - m_new);
+    const float w = __builtin_amdgcn_exp2f(m - m_new);
+    L = L * f + wave_reduce_sum(l * w);
+    M = m_new;
+#pragma unroll
+    for (int j = 0; j < V; ++j) acc[j] *= f;
+    const float* src = tmp_out + (row + p0) * HD + lane * V;
+#pragma unroll 8
+    for (int p = 0; p < n; ++p) {
+      const float wp = __shfl(w, p, 64);
+#pragma unroll
+      for (int j = 0; j < V; ++j) acc[j] += src[(int64_t)p * HD + j] * wp;
+    }
+  }
+  const float inv_l = L > 0.f || L != L ? 1.f / L : 0.f;
+#pragma unroll
+  for (int j = 0; j < V; ++j)
+    out[((int64_t)seq * num_q_heads + h) * HD + lane * V + j] =
+        from_f32<Tag>(acc[j] * inv_l);
 }
 
 // ---------------------------------------------------------------------------
 // Host launcher. q: [Tdec, Hq, D] (contiguous slice of the step's q);
 // out: [Tdec, Hq, D]; kv_cache: [2, blocks, Hkv, 64, D];
 // block_table/seq_lens cover the decode rows (rows 0..Tdec-1).
+// tmp_out [Tdec, Hq, parts, D] and tmp_lse [Tdec, Hq, parts, 2] say into
+// how many partitions a row's keys are split; empty means one.
 void paged_decode_attention(torch::Tensor out, torch::Tensor q,
                             torch::Tensor kv_cache,
                             torch::Tensor block_table,
@@ -310,82 +414,79 @@ void paged_decode_attention(torch::Tensor out, torch::Tensor q,
   TORCH_CHECK(kv_cache.size(3) == 64, "cache block_size must be 64");
   TORCH_CHECK(group >= 1 && group <= MAX_GROUP && num_q_heads ==
               group * num_kv_heads, "GQA group must be 1..8, got ", group);
-  const int num_parts =
-      (int)((max_seq_len + DEC_PART - 1) / DEC_PART);
+  int num_parts = 1;
+  if (tmp_out.numel() > 0) {
+    TORCH_CHECK(tmp_out.dim() == 4 && tmp_lse.dim() == 4 &&
+                tmp_out.is_contiguous() && tmp_lse.is_contiguous() &&
+                tmp_out.size(0) == num_seqs && tmp_lse.size(0) == num_seqs &&
+                tmp_out.size(1) == num_q_heads &&
+                tmp_lse.size(1) == num_q_heads &&
+                tmp_out.size(2) == tmp_lse.size(2) &&
+                tmp_out.size(3) == head_dim && tmp_lse.size(3) == 2,
+                "decode scratch must be [T, Hq, parts, D] and "
+                "[T, Hq, parts, 2]");
+    num_parts = tmp_out.size(2);
+  }
+  // A window starts on a multiple of 32 keys, up to 31 before it.
+  int64_t span = std::max<int64_t>(max_seq_len, 1);
+  if (sliding_window > 0)
+    span = std::min(span, sliding_window + DEC_KEYS - 1);
+  const int unit = DEC_WAVES * DEC_KEYS;
+  const int part_len =
+      (int)((span + (int64_t)num_parts * unit - 1) /
+            ((int64_t)num_parts * unit)) * unit;
   const int max_blocks = block_table.size(1);
+  const float scale_log2 = (float)scale * DEC_LOG2E;
   auto stream = c10::hip::getCurrentHIPStream().stream();
 
-  dim3 grid(num_seqs, num_kv_heads, num_parts);
-  dim3 block(DEC_BLOCK);
+  dim3 grid(num_kv_heads, num_seqs, num_parts);
 
-#define LAUNCH_DEC_HD(TAG, CTAG, G, FIN, HD)                                 \
-  hipLaunchKernelGGL((paged_decode_kernel<TAG, CTAG, G, FIN, HD>), grid,     \
-                     block,                                                  \
-                     0, stream, (short*)out.data_ptr(),                      \
-                     FIN ? nullptr : tmp_out.data_ptr<float>(),              \
-                     FIN ? nullptr : tmp_lse.data_ptr<float>(),              \
-                     (const short*)q.data_ptr(),                             \
-                     (const CacheTraits<CTAG>::elem*)kv_cache.data_ptr(),    \
-                     block_table.data_ptr<int>(), seq_lens.data_ptr<int>(),  \
-                     (float)scale, num_q_heads, num_kv_heads, head_dim,      \
-                     max_blocks, num_parts, kv_cache.stride(0),              \
-                     q.stride(0), (int)sliding_window)
-
-#define LAUNCH_DEC(TAG, CTAG, G, FIN)                                        \
-  switch (head_dim) {                                                        \
-    case 64: LAUNCH_DEC_HD(TAG, CTAG, G, FIN, 64); break;                    \
-    case 256: LAUNCH_DEC_HD(TAG, CTAG, G, FIN, 256); break;                  \
-    default: LAUNCH_DEC_HD(TAG, CTAG, G, FIN, 128); break;                   \
-  }
-
-#define DISPATCH_GROUP(TAG, CTAG, FIN)                                       \
-  switch (group) {                                                           \
-    case 1: LAUNCH_DEC(TAG, CTAG, 1, FIN); break;                            \
-    case 2: LAUNCH_DEC(TAG, CTAG, 2, FIN); break;                            \
-    case 4: LAUNCH_DEC(TAG, CTAG, 4, FIN); break;                            \
-    case 5: LAUNCH_DEC(TAG, CTAG, 5, FIN); break;                            \
-    case 6: LAUNCH_DEC(TAG, CTAG, 6, FIN); break;                            \
-    case 8: LAUNCH_DEC(TAG, CTAG, 8, FIN); break;                            \
-    case 3: LAUNCH_DEC(TAG, CTAG, 3, FIN); break;                            \
-    case 7: LAUNCH_DEC(TAG, CTAG, 7, FIN); break;                            \
-    default: TORCH_CHECK(false, "unsupported GQA group ", group);            \
-  }
-
-#define DISPATCH_CACHE(TAG, FIN)                                             \
-  if (kv_cache.scalar_type() == torch::kFloat8_e4m3fn) {                     \
-    DISPATCH_GROUP(TAG, FP8CacheTag, FIN);                                   \
-  } else {                                                                   \
-    DISPATCH_GROUP(TAG, TAG, FIN);                                           \
-  }
-
-  const bool is_bf16 = q.scalar_type() == torch::kBFloat16;
-  if (num_parts == 1) {
-    if (is_bf16) { DISPATCH_CACHE(BF16Tag, true); }
-    else         { DISPATCH_CACHE(FP16Tag, true); }
-  } else {
-    if (is_bf16) { DISPATCH_CACHE(BF16Tag, false); }
-    else         { DISPATCH_CACHE(FP16Tag, false); }
-    HIP_CHECK_KERNEL();
-    dim3 rgrid(num_seqs, num_q_heads);
-    if (is_bf16) {
-      hipLaunchKernelGGL((paged_decode_reduce_kernel<BF16Tag>), rgrid,
-                         dim3(head_dim), 0, stream, (short*)out.data_ptr(),
-                         tmp_out.data_ptr<float>(),
-                         tmp_lse.data_ptr<float>(), seq_lens.data_ptr<int>(),
-                         num_parts, head_dim, num_q_heads);
-    } else {
-      hipLaunchKernelGGL((paged_decode_reduce_kernel<FP16Tag>), rgrid,
-                         dim3(head_dim), 0, stream, (short*)out.data_ptr(),
-                         tmp_out.data_ptr<float>(),
-                         tmp_lse.data_ptr<float>(), seq_lens.data_ptr<int>(),
-                         num_parts, head_dim, num_q_heads);
+  auto launch = [&](auto tag, auto ctag, auto dim, auto fin) {
+    using Tag = decltype(tag);
+    using CTag = decltype(ctag);
+    constexpr int HD = decltype(dim)::value;
+    constexpr bool FINAL = decltype(fin)::value;
+    hipLaunchKernelGGL(
+        (paged_decode_kernel<Tag, CTag, FINAL, HD>), grid, dim3(DEC_BLOCK),
+        0, stream, (short*)out.data_ptr(),
+        FINAL ? nullptr : tmp_out.data_ptr<float>(),
+        FINAL ? nullptr : tmp_lse.data_ptr<float>(),
+        (const short*)q.data_ptr(),
+        (const typename CacheTraits<CTag>::elem*)kv_cache.data_ptr(),
+        block_table.data_ptr<int>(), seq_lens.data_ptr<int>(), scale_log2,
+        group, num_kv_heads, max_blocks, num_parts, part_len,
+        kv_cache.stride(0), q.stride(0), (int)sliding_window);
+    if constexpr (!FINAL) {
+      HIP_CHECK_KERNEL();
+      hipLaunchKernelGGL(
+          (paged_decode_reduce_kernel<Tag, HD>), dim3(num_q_heads, num_seqs),
+          dim3(WAVE_SIZE), 0, stream, (short*)out.data_ptr(),
+          tmp_out.data_ptr<float>(), tmp_lse.data_ptr<float>(),
+          seq_lens.data_ptr<int>(), num_parts, part_len, num_q_heads,
+          (int)sliding_window);
     }
-  }
+  };
+  auto by_dim = [&](auto tag, auto ctag, auto fin) {
+    if (head_dim == 64)
+      launch(tag, ctag, std::integral_constant<int, 64>{}, fin);
+    else if (head_dim == 128)
+      launch(tag, ctag, std::integral_constant<int, 128>{}, fin);
+    else
+      launch(tag, ctag, std::integral_constant<int, 256>{}, fin);
+  };
+  const bool fp8c = kv_cache.scalar_type() == torch::kFloat8_e4m3fn;
+  auto by_type = [&](auto fin) {
+    if (q.scalar_type() == torch::kBFloat16) {
+      if (fp8c) by_dim(BF16Tag{}, FP8CacheTag{}, fin);
+      else      by_dim(BF16Tag{}, BF16Tag{}, fin);
+    } else {
+      if (fp8c) by_dim(FP16Tag{}, FP8CacheTag{}, fin);
+      else      by_dim(FP16Tag{}, FP16Tag{}, fin);
+    }
+  };
+  if (num_parts == 1) by_type(std::true_type{});
+  else                by_type(std::false_type{});
   HIP_CHECK_KERNEL();
-#undef DISPATCH_CACHE
-#undef DISPATCH_GROUP
-#undef LAUNCH_DEC
-#undef LAUNCH_DEC_HD
 }
 
 }  // namespace vllm_amd

@@ -118,6 +118,75 @@ template <> struct CacheTraits<FP8CacheTag> {
 };
 
 // ---------------------------------------------------------------------------
+// Matrix-core helpers. The 16-bit element type selects the instruction:
+// bf16 and fp16 bits share the fragment registers (s16x8), so a kernel
+// templated on the tag must go through these rather than name one
+// builtin.
+typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
+
+template <typename Tag> DEVINL f32x4 mfma16(s16x8 a, s16x8 b, f32x4 c);
+template <> DEVINL f32x4 mfma16<BF16Tag>(s16x8 a, s16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+      __builtin_bit_cast(b16x8, a), __builtin_bit_cast(b16x8, b), c, 0, 0, 0);
+}
+template <> DEVINL f32x4 mfma16<FP16Tag>(s16x8 a, s16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(
+      __builtin_bit_cast(h16x8, a), __builtin_bit_cast(h16x8, b), c, 0, 0, 0);
+}
+template <typename Tag> DEVINL f32x16 mfma32(s16x8 a, s16x8 b, f32x16 c);
+template <> DEVINL f32x16 mfma32<BF16Tag>(s16x8 a, s16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+      __builtin_bit_cast(b16x8, a), __builtin_bit_cast(b16x8, b), c, 0, 0, 0);
+}
+template <> DEVINL f32x16 mfma32<FP16Tag>(s16x8 a, s16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(
+      __builtin_bit_cast(h16x8, a), __builtin_bit_cast(h16x8, b), c, 0, 0, 0);
+}
+
+// Two floats rounded (nearest even) to a packed 16-bit pair.
+template <typename Tag> DEVINL int pack2(float a, float b);
+template <> DEVINL int pack2<BF16Tag>(float a, float b) {
+  return __builtin_bit_cast(
+      int, __builtin_convertvector((f32x2){a, b}, b16x2));
+}
+template <> DEVINL int pack2<FP16Tag>(float a, float b) {
+  return __builtin_bit_cast(
+      int, __builtin_convertvector((f32x2){a, b}, h16x2));
+}
+template <typename Tag> DEVINL float unpack_lo(int v) {
+  return to_f32<Tag>((short)v);
+}
+template <typename Tag> DEVINL float unpack_hi(int v) {
+  return to_f32<Tag>((short)(v >> 16));
+}
+
+// Four e4m3 bytes to four 16-bit values (exact for both types).
+template <typename Tag> DEVINL int2 fp8x4_widen(int v);
+template <> DEVINL int2 fp8x4_widen<BF16Tag>(int v) {
+  return {__builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
+                                      v, 1.0f, false)),
+          __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
+                                      v, 1.0f, true))};
+}
+template <> DEVINL int2 fp8x4_widen<FP16Tag>(int v) {
+  return {__builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(
+                                      v, 1.0f, false)),
+          __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(
+                                      v, 1.0f, true))};
+}
+
+// Transposing LDS read: the 16 lanes of a group address a block of 4
+// rows x 16 columns of 16-bit values (lane i: row i / 4, columns
+// (i % 4) * 4 .. + 3) and lane i receives column i, rows 0..3.
+DEVINL s16x4 lds_read_tr(const void* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s16x4*)p);
+}
+
+// ---------------------------------------------------------------------------
 // Wave reductions (64 lanes).
 DEVINL float wave_reduce_sum(float v) {
 #pragma unroll

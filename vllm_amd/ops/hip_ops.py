@@ -22,8 +22,30 @@ torch.ops.load_library(str(_SO))
 
 _C = torch.ops.vllm_amd
 
-# Decode flash-partition size — must match DEC_PART in attention_decode.hip.
-_DEC_PART = 512
+# Decode attention: one workgroup takes at least this many keys (4 waves
+# of 32), at most 16 times as many, and 2 workgroups fit on each of the
+# 256 CUs.
+_DEC_UNIT = 128
+_DEC_MAX_UNITS = 16
+_DEC_FILL = 512
+
+
+def _decode_parts(rows, kv_heads, max_seq_len, sliding_window):
+    """Into how many partitions a row's keys are split. Every partition
+    costs a pass over its fp32 partials, so no more than fill the chip:
+    16 rows x 4096 keys (8 KV heads of 128) take 52 us in 4 partitions,
+    58 in 16. Partitions of more than 2048 keys leave ragged batches
+    waiting for their longest row; below that more partitions only
+    cost: 256 rows x 129..2176 keys take 227 us in 2, 248 in 9; 64 rows
+    x 4096..8192 fp8 keys 154 us in 4, 180 in 32. At most 64, the lanes
+    of the merging wave."""
+    span = max(max_seq_len, 1)
+    if sliding_window > 0:
+        span = min(span, sliding_window + 31)
+    units = -(-span // _DEC_UNIT)
+    parts = max(-(-_DEC_FILL // max(rows * kv_heads, 1)),
+                -(-units // _DEC_MAX_UNITS))
+    return max(1, min(parts, units, 64))
 
 
 def rms_norm(x, weight, eps):
@@ -121,7 +143,8 @@ def attention_unified(
 
     if num_decodes > 0:
         q_dec = q[:num_decodes]
-        num_parts = (max_seq_len + _DEC_PART - 1) // _DEC_PART
+        num_parts = _decode_parts(num_decodes, kv_cache.shape[2],
+                                  max_seq_len, sliding_window)
         if num_parts > 1:
             tmp_out = torch.empty(
                 num_decodes, num_heads, num_parts, head_dim,

@@ -89,7 +89,9 @@ class DecodeGraphRunner:
 
     BATCH_BUCKETS = (1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256,
                      384, 512, 768, 1024)
-    DEC_PART = 512  # must match attention_decode.hip
+    # Granularity of the context bound a graph is captured for (the
+    # decode kernel splits its keys by that bound, not by real lengths).
+    DEC_PART = 512
 
     def __init__(self, runner: "ModelRunner"):
         self.runner = runner
