@@ -159,13 +159,12 @@ def test_decode_attention_edges(hd, group, dtype, cache_dtype, window, n):
                                         D=hd)
     q = q.to(dtype)
     cache = cache.to(cache_dtype)
-    nan = torch.tensor(float("nan"), device="cuda").to(cache_dtype)
     raw = cache if cache_dtype != torch.float8_e4m3fn \
         else cache.view(torch.uint8)
+    nan = float("nan") if raw is cache else 0x7F
     for i in range(6):
         if ctx[i] % 64:
-            raw[:, bt[i, ctx[i] // 64], :, ctx[i] % 64:] = \
-                nan.view(raw.dtype) if raw.dtype == torch.uint8 else nan
+            raw[:, bt[i, ctx[i] // 64], :, ctx[i] % 64:] = nan
     out = hip.attention_unified(q, cache, bt, qsl, sl, hd**-0.5,
                                 num_decodes=n, max_seq_len=max(ctx),
                                 max_query_len=1, sliding_window=window)
@@ -205,6 +204,48 @@ def test_prefill_attention(group, q_lens, ctx_lens):
     expect = ref.attention_unified(q, cache, bt, qsl, sl, scale,
                                    num_decodes=num_decodes)
     assert_close(out, expect)
+
+
+@pytest.mark.parametrize("hd,group,dtype,cache_dtype,window,scale", [
+    (128, 7, torch.bfloat16, torch.bfloat16, 0, 0.09),
+    (128, 4, torch.bfloat16, torch.bfloat16, 5, 0.5),
+    (128, 4, torch.float16, torch.float16, 0, 0.5),
+    (64, 3, torch.bfloat16, torch.float8_e4m3fn, 0, -0.125),
+    (64, 1, torch.float16, torch.float8_e4m3fn, 70, 0.125),
+    (256, 5, torch.bfloat16, torch.bfloat16, 200, 0.06),
+    (256, 2, torch.bfloat16, torch.float8_e4m3fn, 0, 0.06),
+])
+def test_prefill_attention_edges(hd, group, dtype, cache_dtype, window,
+                                 scale):
+    """Portions that end on, before and after the edges of a row tile
+    (128 rows = tokens x heads) and of a key tile, after contexts of the
+    same kind; an empty portion; unwritten rows of the last block hold
+    NaN; scores large enough for the running maximum to move. Tolerance:
+    weights and outputs rounded to 16 bits (2^-8 bf16, 2^-11 fp16), of
+    values up to 4."""
+    hip = _hip()
+    Hkv = 2
+    q_lens = [2, 33, 64, 0, 65, 129]
+    ctx = [2, 64, 64 + 63, 9, 65 + 300, 129]
+    n = len(ctx)
+    q, cache, bt, qsl, sl = _make_paged(n, q_lens, ctx, Hkv * group, Hkv,
+                                        D=hd)
+    q = q.to(dtype)
+    cache = cache.to(cache_dtype)
+    raw = cache if cache_dtype != torch.float8_e4m3fn \
+        else cache.view(torch.uint8)
+    nan = float("nan") if raw is cache else 0x7F
+    for i in range(n):
+        if ctx[i] % 64:
+            raw[:, bt[i, ctx[i] // 64], :, ctx[i] % 64:] = nan
+    out = hip.attention_unified(q, cache, bt, qsl, sl, scale,
+                                num_decodes=0, max_seq_len=max(ctx),
+                                max_query_len=max(q_lens),
+                                sliding_window=window)
+    expect = ref.attention_unified(q.float(), cache.float(), bt, qsl, sl,
+                                   scale, sliding_window=window)
+    atol = 3 * 4 * (2**-8 if dtype == torch.bfloat16 else 2**-11)
+    assert_close(out, expect, atol=atol, rtol=atol / 4)
 
 
 def test_model_forward_matches_cpu_reference():

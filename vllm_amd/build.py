@@ -42,7 +42,7 @@ SOURCES = [
 # These kernels keep matrix-core accumulators in ordinary vector
 # registers: they are rescaled by the vector ALU between products, and
 # through the accumulation registers every rescale is a copy each way.
-VGPR_ACCUMULATORS = {"attention_decode"}
+VGPR_ACCUMULATORS = {"attention_decode", "attention_prefill"}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("PYTORCH_ROCM_ARCH", "gfx950")

@@ -128,7 +128,7 @@ def attention_unified(
     max_query_len=0,
 ):
     """Dispatch decode rows (first num_decodes, query_len==1) to the
-    partitioned VALU decode kernel and the rest to the MFMA prefill
+    partitioned decode kernel and the rest to the MFMA prefill
     kernel. max_seq_len/max_query_len come from the scheduler (CPU) so
     no device sync is needed here."""
     num_tokens, num_heads, head_dim = q.shape
