@@ -163,6 +163,19 @@ template <typename Tag> DEVINL float unpack_hi(int v) {
   return to_f32<Tag>((short)(v >> 16));
 }
 
+// acc plus the two values of a packed pair, in fp32.
+template <typename Tag> DEVINL float add_pair(int v, float acc);
+template <> DEVINL float add_pair<BF16Tag>(int v, float acc) {
+  return __builtin_amdgcn_fdot2_f32_bf16(
+      __builtin_bit_cast(b16x2, v), __builtin_bit_cast(b16x2, 0x3f803f80),
+      acc, false);
+}
+template <> DEVINL float add_pair<FP16Tag>(int v, float acc) {
+  return __builtin_amdgcn_fdot2(
+      __builtin_bit_cast(h16x2, v), __builtin_bit_cast(h16x2, 0x3c003c00),
+      acc, false);
+}
+
 // Four e4m3 bytes to four 16-bit values (exact for both types).
 template <typename Tag> DEVINL int2 fp8x4_widen(int v);
 template <> DEVINL int2 fp8x4_widen<BF16Tag>(int v) {
@@ -185,6 +198,26 @@ DEVINL s16x4 lds_read_tr(const void* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
       (__attribute__((address_space(3))) s16x4*)p);
 }
+
+// 64 lanes x 16 B from global memory straight into LDS: lane i's 16 bytes
+// land at dst + 16 * i (dst the same in all lanes). No register receives
+// anything, so the kernel waits itself (lds_fill_wait, then a barrier for
+// the other waves' parts): the compiler would wait for every fill under
+// way before each LDS read, having no means to tell the tiles apart.
+DEVINL void lds_fill16(const void* src, void* dst) {
+  const uint32_t at = (uint32_t)(uintptr_t)(
+      __attribute__((address_space(3))) void*)dst;
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off"
+      :
+      : "s"(at), "v"(src)
+      : "memory", "m0");
+}
+// vmcnt(0); the builtin, so that the compiler knows its own older loads to
+// be done as well and does not wait again after the next fill.
+DEVINL void lds_fill_wait() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 
 // ---------------------------------------------------------------------------
 // Wave reductions (64 lanes).
