@@ -564,6 +564,53 @@ def test_mla_decode_kernel(T, Hq, ctx):
     assert_close(out, expect, atol=4e-2, rtol=4e-2)
 
 
+@pytest.mark.parametrize("heads,bs,dtype", [
+    (128, 64, torch.bfloat16),   # whole tiles from one cache block
+    (130, 16, torch.bfloat16),   # second head group nearly empty
+    (20, 128, torch.float16),    # idle waves
+])
+def test_mla_attention_edges(heads, bs, dtype):
+    """Decode rows and prompt portions around the 64-key tile, an empty
+    portion, padded partitions; unwritten rows of the last block hold
+    NaN. Tolerance: weights of decode rows and all outputs are rounded to
+    16 bits, values up to 4."""
+    hip = _hip()
+    q_lens = [1, 1, 1, 2, 0, 65, 40]
+    ctx = [1, 65, 700, 64, 5, 130, 40]
+    n, T = len(ctx), sum(q_lens)
+    nb = -(-max(ctx) // bs)
+    cache = torch.randn(n * nb, bs, 576, device="cuda", dtype=dtype)
+    bt = torch.randperm(n * nb, device="cuda").int().view(n, nb)
+    for i, c in enumerate(ctx):
+        if c % bs:
+            cache[bt[i, c // bs], c % bs:] = float("nan")
+    qn = torch.randn(T, heads, 512, device="cuda", dtype=dtype)
+    qp = torch.randn(T, heads, 64, device="cuda", dtype=dtype)
+    qsl = torch.tensor([0] + [sum(q_lens[:i + 1]) for i in range(n)],
+                       device="cuda", dtype=torch.int32)
+    sl = torch.tensor(ctx, device="cuda", dtype=torch.int32)
+    out = hip.mla_attention(qn, qp, cache, bt, qsl, sl, 0.07,
+                            num_decodes=3, max_seq_len=max(ctx))
+    expect = ref.mla_attention(qn.float(), qp.float(), cache.float(), bt,
+                               qsl, sl, 0.07)
+    atol = 2 * 4 * (2**-8 if dtype == torch.bfloat16 else 2**-11)
+    assert_close(out, expect, atol=atol, rtol=atol / 4)
+
+
+@pytest.mark.parametrize("T,H,K,N", [(1, 3, 128, 512), (65, 2, 512, 128),
+                                     (130, 1, 256, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_head_matmul(T, H, K, N, dtype):
+    """Strided head slices, ragged token tiles, several K steps. fp32
+    sums: off by the result's own rounding (2^-8, 2^-11) at most."""
+    hip = _hip()
+    x = torch.randn(T, H, K + 64, device="cuda", dtype=dtype)[..., :K]
+    w = torch.randn(H, K, N, device="cuda", dtype=dtype) * K**-0.5
+    assert_close(hip.head_matmul(x, w), ref.head_matmul(x, w),
+                 atol=2**-9, rtol=2**-8 if dtype == torch.bfloat16
+                 else 2**-10)
+
+
 def test_mla_unified_dispatch_mixed_batch():
     """ops.mla_attention routes decode rows to the kernel and prefill
     rows to the torch path; both must agree with the all-torch result."""

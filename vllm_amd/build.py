@@ -25,6 +25,7 @@ SOURCES = [
     CSRC / "comms.hip",
     CSRC / "moe.hip",
     CSRC / "mla.hip",
+    CSRC / "head_matmul.hip",
     CSRC / "quant_fp8.hip",
     CSRC / "attention_decode.hip",
     CSRC / "attention_prefill.hip",
@@ -42,7 +43,7 @@ SOURCES = [
 # These kernels keep matrix-core accumulators in ordinary vector
 # registers: they are rescaled by the vector ALU between products, and
 # through the accumulation registers every rescale is a copy each way.
-VGPR_ACCUMULATORS = {"attention_decode", "attention_prefill"}
+VGPR_ACCUMULATORS = {"attention_decode", "attention_prefill", "mla", "head_matmul"}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("PYTORCH_ROCM_ARCH", "gfx950")

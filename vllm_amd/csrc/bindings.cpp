@@ -55,6 +55,11 @@ void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
                 torch::Tensor kv_cache, torch::Tensor block_table,
                 torch::Tensor seq_lens, double scale, int64_t max_seq_len,
                 torch::Tensor tmp_out, torch::Tensor tmp_lse);
+void mla_prefill(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
+                 torch::Tensor kv_cache, torch::Tensor block_table,
+                 torch::Tensor query_start_loc, torch::Tensor seq_lens,
+                 double scale, int64_t num_decodes);
+torch::Tensor head_matmul(torch::Tensor x, torch::Tensor w);
 torch::Tensor scalar_rms_norm(torch::Tensor x, torch::Tensor gain,
                               double eps, torch::ScalarType out_dtype);
 torch::Tensor add_scaled_scalar_norm(
@@ -193,6 +198,10 @@ TORCH_LIBRARY(vllm_amd, m) {
         "Tensor kv_cache, Tensor block_table, Tensor seq_lens, "
         "float scale, int max_seq_len, Tensor(b!) tmp_out, "
         "Tensor(c!) tmp_lse) -> ()");
+  m.def("mla_prefill(Tensor(a!) out, Tensor q_nope, Tensor q_pe, "
+        "Tensor kv_cache, Tensor block_table, Tensor query_start_loc, "
+        "Tensor seq_lens, float scale, int num_decodes) -> ()");
+  m.def("head_matmul(Tensor x, Tensor w) -> Tensor");
   m.def("scalar_rms_norm(Tensor x, Tensor gain, float eps, "
         "ScalarType out_dtype) -> Tensor");
   m.def("add_scaled_scalar_norm(Tensor(a!) residual, Tensor y, Tensor gain, "
@@ -292,6 +301,8 @@ TORCH_LIBRARY_IMPL(vllm_amd, CUDA, m) {
   m.impl("moe_gemm_shuf", &vllm_amd::moe_gemm_shuf);
   m.impl("moe_combine", &vllm_amd::moe_combine);
   m.impl("mla_decode", &vllm_amd::mla_decode);
+  m.impl("mla_prefill", &vllm_amd::mla_prefill);
+  m.impl("head_matmul", &vllm_amd::head_matmul);
   m.impl("scalar_rms_norm", &vllm_amd::scalar_rms_norm);
   m.impl("add_scaled_scalar_norm", &vllm_amd::add_scaled_scalar_norm);
   m.impl("token_shift", &vllm_amd::token_shift);

@@ -1,28 +1,41 @@
-// MLA decode attention for CDNA4 (gfx950).
+// MLA attention for CDNA4 (gfx950): decode rows and prompt portions over
+// the compressed latent KV cache.
 //
-// Absorbed-MQA decode over the compressed latent KV cache (blueprint:
-// reference vllm/model_executor/layers/attention/mla_attention.py:40-190
-// "data-movement friendly" decode path): queries are pre-absorbed
-// through W_UK so every head attends with dim L+R (kv_lora 512 + rope
-// 64 = 576) against ONE shared latent stream, and the value is the
-// first L dims of the same stream. That makes decode a GEMM-shaped
-// problem — Q[32 heads, 576] x K^T[576, 32 tok] and P[32, 32] x
-// V[32 tok, 512] per tile — so this kernel runs on MFMA 16x16x32-bf16,
-// unlike the GQA decode kernel (attention_decode.hip) which is
-// VALU-bound at 1-16 queries/KV head.
-//
-// Block = 4 waves = 32 heads x 32-token KV subtiles:
-//   QK:  wave(mtile=w&1, ntile=w>>1): 18 MFMAs over the 576 dim.
-//   softmax: per-head online max/sum shared through LDS (wave-redundant
-//   recompute from LDS keeps the update single-barrier).
-//   PV:  wave w owns V columns [w*128, (w+1)*128); P staged [h][t] bf16.
-// The KV subtile is staged once: [tok][576] (QK reads rows) plus a
-// scatter-transposed copy of the first 512 dims [dim][tok] (PV reads
-// rows) — ~70 KB LDS, 2 blocks/CU.
-//
-// Grid (num_decodes, num_parts, ceil(Hq/32)); partitions of 1024 tokens
-// produce fp32 partials + (m, l) merged by mla_reduce_kernel — same
-// flash-partition scheme as the GQA decode kernel.
+// Absorbed-MQA form (blueprint: reference
+// vllm/model_executor/layers/attention/mla_attention.py:40-190): queries
+// are carried through W_UK first, so all heads of a token attend with dim
+// L+R (512 + 64) against ONE shared latent stream whose first 512 dims
+// are the value as well. Every cached row meets 2 * 1088 flops per head:
+// with 128 heads that is 240 flops per byte, so the matrix cores bound it
+// and the tile is laid out for them:
+//   - A workgroup is one token and 128 heads, eight waves of 16 heads. A
+//     wave keeps its queries (72 registers) and all 512 output columns
+//     (128 registers) for the whole pass; two waves per SIMD fit, so one
+//     wave's softmax and LDS latency run under another's products.
+//     (32-head waves would read half the LDS bytes per flop, but need 400
+//     registers before the first temporary.)
+//   - 16x16x32 MFMA: S^T = K Q^T with the heads as columns, so a lane
+//     holds 16 of 64 keys of one head and P^T is already the fragment
+//     O^T = V^T P^T needs when the keys are taken in the order the score
+//     registers hold them: P never leaves its lane.
+//   - One LDS copy of 64 latent rows serves both products: K fragments
+//     are plain 16 B reads, V^T fragments transposing reads of the same
+//     rows. 16 B chunks of a row are exchanged so that neither kind of
+//     read meets a bank twice.
+//   - Two such tiles alternate; they are filled straight from global
+//     memory (no registers), one tile ahead, one barrier per tile.
+//   - Where the weights keep more than 16 bits (hi + lo, prompts),
+//     accumulators are rescaled only when a head's maximum has grown by
+//     2^8. Where they are rounded to 16 (decode), the largest is kept at
+//     one and the rounded weights are summed: 3 % slower, 4 % closer to
+//     64-bit results.
+// Decode rows are split over a few partitions of the keys when there are
+// fewer rows than CUs; fp32 partials (256 KB per row and partition) are
+// merged by mla_reduce_kernel, so partitions are few and long.
+// 128 heads: 128 rows x 129..2176 keys 1025 -> 128 us with the merge (four
+// waves of 16 heads on 32-key tiles, V stored transposed, before); prompts
+// of 300, 1300 and 2301 tokens 1.6 ms (600 TFLOP/s counting P once; a
+// composition of library products in fp32 before, 24 ms).
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
@@ -36,324 +49,375 @@ namespace mla {
 
 constexpr int LORA = 512;
 constexpr int ROPE = 64;
-constexpr int DK = LORA + ROPE;  // 576
-constexpr int HG = 32;           // heads per block
-constexpr int SUB = 32;          // KV tokens per subtile
-constexpr int PART = 1024;       // tokens per grid partition
-constexpr int THREADS = 256;
-constexpr float NEG_INF = -1e30f;
+constexpr int DK = LORA + ROPE;   // 576
+constexpr int HG = 128;           // heads per workgroup
+constexpr int SUB = 64;           // keys per LDS tile
+constexpr int WAVES = 8;
+constexpr int THREADS = WAVES * WAVE_SIZE;
+constexpr int CHUNKS = DK / 8;    // 16 B chunks per row
+constexpr int TILE_BYTES = SUB * DK * 2;
+constexpr int BUFS = 2;
+constexpr int FILL = SUB * CHUNKS / THREADS;  // 16 B loads a thread and tile
+constexpr float NEG = -3.0e38f;
+constexpr float GROWTH = 8.f;
 
-DEVINL int swz(int row, int byte_off) { return byte_off ^ ((row & 7) << 4); }
+// A row is 4.5 x 256 B, so odd rows start half a bank period later. The
+// eight chunks of each 128 B are exchanged by a number that differs over
+// eight row pairs (K reads: 16 rows, one chunk) and in more than its last
+// bit over four (V reads: 8 rows, two neighbouring chunks).
+DEVINL int chunk_slot(int row, int c) {
+  const int x = (row >> 1) & 7;
+  return c ^ (((x & 3) << 1) | (x >> 2));
+}
 
-template <typename Tag>
-__launch_bounds__(THREADS) __global__
-void mla_decode_kernel(short* __restrict__ out,           // [T, Hq, LORA]
-                       const short* __restrict__ q_nope,  // [T, Hq, LORA]
-                       const short* __restrict__ q_pe,    // [T, Hq, ROPE]
-                       const short* __restrict__ kv,      // [NB, BS, DK]
-                       const int* __restrict__ block_table, int bt_stride,
-                       const int* __restrict__ seq_lens, float scale,
-                       int num_heads, int block_size,
-                       float* __restrict__ tmp_out,  // [T, Hq, parts, LORA]
-                       float* __restrict__ tmp_lse,  // [T, Hq, parts, 2]
-                       int max_parts) {
-  const int seq = blockIdx.x;
-  const int part = blockIdx.y;
+// One workgroup: (token row, partition of part_len keys, head group).
+// PROMPT: blockIdx.x counts the batch's prompt tokens from the last one
+// (the last tokens of a portion have most keys); otherwise blockIdx.x is a
+// decode row and blockIdx.y a partition. SPLIT_P keeps the weights at more than 16 bits
+// (hi + lo parts, two products).
+template <typename Tag, bool PROMPT, bool SPLIT_P>
+__launch_bounds__(THREADS, 2) __global__
+void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
+                const short* __restrict__ q_nope,  // [T, Hq, LORA]
+                const short* __restrict__ q_pe,    // [T, Hq, ROPE]
+                const short* __restrict__ kv,      // [NB, BS, DK]
+                const int* __restrict__ block_table, int bt_stride,
+                const int* __restrict__ query_start_loc,
+                const int* __restrict__ seq_lens, float scale_log2,
+                int num_heads, int block_size, int num_decodes,
+                int num_reqs,
+                float* __restrict__ tmp_out,  // [T, Hq, parts, LORA]
+                float* __restrict__ tmp_lse,  // [T, Hq, parts, 2]
+                int num_parts, int part_len) {
+  int req, row, ctx, part = 0;
+  if constexpr (PROMPT) {
+    row = query_start_loc[num_reqs] - 1 - (int)blockIdx.x;
+    if (row < query_start_loc[num_decodes]) return;
+    req = num_decodes;              // the last request starting at or before
+    for (int end = num_reqs; end - req > 1;) {
+      const int mid = (req + end) / 2;
+      if (query_start_loc[mid] <= row) req = mid;
+      else end = mid;
+    }
+    ctx = seq_lens[req] - (query_start_loc[req + 1] - 1 - row);
+  } else {
+    req = row = blockIdx.x;
+    part = blockIdx.y;
+    ctx = seq_lens[req];
+  }
   const int hg0 = blockIdx.z * HG;
-  const int ctx = seq_lens[seq];
-  const int t_begin = part * PART;
-  if (t_begin >= ctx) return;
-  const int t_end = min(t_begin + PART, ctx);
-  const bool single = gridDim.y == 1;
+  const int t_begin = part * part_len;
+  const int t_end = min(ctx, t_begin + part_len);
+  if (t_begin >= t_end) return;
 
-  __shared__ short k_lds[SUB * DK];       // [tok][576], swizzled 16B slots
-  __shared__ short vt_lds[LORA * SUB];    // [dim][tok]
-  __shared__ short p_lds[HG * SUB];       // [head][tok] bf16
-  __shared__ float m_st[HG], l_st[HG], f_st[HG];
-  __shared__ float wmax[2][HG], wsum[2][HG];
+  __shared__ __align__(16) char lds[BUFS * TILE_BYTES];
 
-  const int tid = threadIdx.x;
-  const int wave = tid / WAVE_SIZE;
-  const int lane = tid % WAVE_SIZE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lane = threadIdx.x % WAVE_SIZE;
   const int l16 = lane & 15;
   const int l4 = lane >> 4;
-  const int mtile = wave & 1;
-  const int ntile = wave >> 1;
+  const int head = hg0 + wave * 16 + l16;
+  const bool busy = hg0 + wave * 16 < num_heads;
 
-  if (tid < HG) {
-    m_st[tid] = NEG_INF;
-    l_st[tid] = 0.f;
-  }
-  // Running max per owned head row, kept REDUNDANTLY in registers by
-  // the two waves sharing an mtile (identical deterministic updates
-  // from LDS wmax) — m_st is written only by owner lanes and read only
-  // across barriers, so there is no read/write race in the softmax
-  // phase.
-  float m_reg[4] = {NEG_INF, NEG_INF, NEG_INF, NEG_INF};
-
-  // Q fragments: wave's rows are heads mtile*16 + l16 of this group.
-  const int head = hg0 + mtile * 16 + l16;
-  const bool head_ok = head < num_heads;
-  const long qn_row = ((long)seq * num_heads + (head_ok ? head : 0)) * LORA;
-  const long qp_row = ((long)seq * num_heads + (head_ok ? head : 0)) * ROPE;
-  s16x8 qfrag[18];
+  s16x8 qf[DK / 32];
+  {
+    const int64_t h = (int64_t)row * num_heads + min(head, num_heads - 1);
+    const short* qn = q_nope + h * LORA + l4 * 8;
+    const short* qp = q_pe + h * ROPE + l4 * 8;
 #pragma unroll
-  for (int kf = 0; kf < 18; ++kf) {
-    const int f = kf * 32 + l4 * 8;
-    s16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (head_ok)
-      v = (f < LORA)
-              ? *reinterpret_cast<const s16x8*>(q_nope + qn_row + f)
-              : *reinterpret_cast<const s16x8*>(q_pe + qp_row + (f - LORA));
-    qfrag[kf] = v;
+    for (int kk = 0; kk < LORA / 32; ++kk)
+      qf[kk] = *reinterpret_cast<const s16x8*>(qn + kk * 32);
+#pragma unroll
+    for (int kk = 0; kk < ROPE / 32; ++kk)
+      qf[LORA / 32 + kk] = *reinterpret_cast<const s16x8*>(qp + kk * 32);
   }
 
-  // PV accumulators: wave owns V cols [wave*128, wave*128+128) for both
-  // head mtiles: acc[mt][nf] covers heads mt*16.. x cols nf*16..
-  f32x4 o_acc[2][8];
+  const int* bt = block_table + (int64_t)req * bt_stride;
+  // Each wave fills 8 rows. Rows past the end repeat the last one: their
+  // weight is zero, and what a stale row holds could be NaN.
+  auto fill = [&](int sub0, int buf) {
+    int ln = lane;
+    asm("" : "+v"(ln));  // recompute the places each time: no registers
+    const int last = t_end - 1 - sub0;
+    char* dst = lds + buf * TILE_BYTES + wave * (FILL * WAVE_SIZE * 16);
+    auto place = [&](int i, int& rr, int& e) {
+      const int c = i * WAVE_SIZE + ln;
+      const int r8 = c / CHUNKS;
+      const int r = wave * (SUB / WAVES) + r8;
+      e = chunk_slot(r, c - r8 * CHUNKS) * 8;
+      rr = min(r, last);
+    };
+    int rr, e;
+    if (block_size % SUB == 0) {   // the tile is part of one cache block
+      const int b = sub0 / block_size;
+      const short* base =
+          kv + ((int64_t)bt[b] * block_size + (sub0 - b * block_size)) * DK;
 #pragma unroll
-  for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-    for (int nf = 0; nf < 8; ++nf) o_acc[mt][nf] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const float sc2 = scale * 1.4426950408889634f;  // log2(e)
-  __syncthreads();
-
-  for (int sub0 = t_begin; sub0 < t_end; sub0 += SUB) {
-    // ---- stage: 32 tokens x 1152B; 2304 16B chunks over 256 threads.
-    {
-      for (int c = tid; c < SUB * (DK / 8); c += THREADS) {
-        const int tok = c / (DK / 8);
-        const int f8 = c % (DK / 8);      // 8-elem feature chunk
-        const int t_glob = sub0 + tok;
-        s16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (t_glob < t_end) {
-          const int blk = block_table[seq * bt_stride + t_glob / block_size];
-          v = *reinterpret_cast<const s16x8*>(
-              kv + ((long)blk * block_size + t_glob % block_size) * DK +
-              f8 * 8);
-        }
-        *reinterpret_cast<s16x8*>(reinterpret_cast<char*>(k_lds) +
-                                  tok * (DK * 2) + swz(tok, f8 * 16)) = v;
-        if (f8 * 8 < LORA) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            vt_lds[(f8 * 8 + j) * SUB + tok] = v[j];
-        }
+      for (int i = 0; i < FILL; ++i) {
+        place(i, rr, e);
+        lds_fill16(base + (rr * DK + e), dst + i * WAVE_SIZE * 16);
+      }
+    } else {
+      for (int i = 0; i < FILL; ++i) {
+        place(i, rr, e);
+        const int t = sub0 + rr;
+        const int b = t / block_size;
+        lds_fill16(kv + ((int64_t)bt[b] * block_size + (t - b * block_size)) *
+                            DK + e,
+                   dst + i * WAVE_SIZE * 16);
       }
     }
-    __syncthreads();
+  };
 
-    // ---- QK: S[16h x 16t] for (mtile, ntile).
-    f32x4 s_frag = {0.f, 0.f, 0.f, 0.f};
-    {
-      const int tok = ntile * 16 + l16;  // B-frag col
+  // Byte places of this lane's fragments in a tile. The exchange of chunks
+  // only touches the low three bits of a chunk and repeats every 16 rows,
+  // so all other parts of an address are constants.
+  int k_at[2], v_at[4];
+  k_at[0] = l16 * (DK * 2) + chunk_slot(l16, l4) * 16;
+  k_at[1] = k_at[0] ^ 64;
+  {
+    const int r = l4 * 4 + (l16 >> 2);
 #pragma unroll
-      for (int kf = 0; kf < 18; ++kf) {
-        s16x8 bfrag = *reinterpret_cast<const s16x8*>(
-            reinterpret_cast<const char*>(k_lds) + tok * (DK * 2) +
-            swz(tok, kf * 64 + l4 * 16));
-        s_frag = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qfrag[kf], bfrag,
-                                                         s_frag, 0, 0, 0);
+    for (int j = 0; j < 4; ++j)
+      v_at[j] = r * (DK * 2) + chunk_slot(r, j * 2 + ((l16 & 3) >> 1)) * 16 +
+                (l16 & 1) * 8;
+  }
+
+  float m_run = NEG, l_run = 0.f;  // of this head, log2 domain; l: own keys
+  f32x4 o[LORA / 16];
+#pragma unroll
+  for (int i = 0; i < LORA / 16; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  fill(t_begin, 0);
+  int buf = 0;
+  for (int sub0 = t_begin; sub0 < t_end; sub0 += SUB, buf ^= 1) {
+    // The tile has landed for this wave, then for all; and every wave is
+    // done with the tile before, whose place the next one takes.
+    lds_fill_wait();
+    __syncthreads();
+    if (sub0 + SUB < t_end) fill(sub0 + SUB, buf ^ 1);
+    if (!busy) continue;
+    const char* t = lds + buf * TILE_BYTES;
+    // ---- S^T: 64 keys x 16 heads -----------------------------------------
+    f32x4 s[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      s[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < DK / 32; ++kk) {
+        const s16x8 a = *reinterpret_cast<const s16x8*>(
+            t + k_at[kk & 1] + n * 16 * (DK * 2) + (kk >> 1) * 128);
+        s[n] = mfma16<Tag>(a, qf[kk], s[n]);
       }
     }
-    // C-frag: col=lane&15=token, row=l4*4+r=head-in-mtile.
-    const int tok_g = sub0 + ntile * 16 + l16;
-    const bool tok_ok = tok_g < t_end;
-    float s_val[4];
-    float wm = NEG_INF;
+    // ---- softmax: s[n][r] is key n*16 + l4*4 + r -------------------------
+    const int left = t_end - sub0 - l4 * 4;
+    float mx = NEG;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      s_val[r] = tok_ok ? s_frag[r] * sc2 : NEG_INF;
-      // per-head max needs a reduce over tokens (lanes l16); do all 4
-      // head rows: each lane carries 4 heads, reduce each row below.
-    }
-    // Reduce max over the 16 token lanes for each of the 4 head rows.
-    float rowmax[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float v = s_val[r];
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1)
-        v = fmaxf(v, __shfl_xor(v, off, 64));
-      rowmax[r] = v;
-    }
-    if (l16 == 0) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        wmax[ntile][mtile * 16 + l4 * 4 + r] = rowmax[r];
-    }
-    __syncthreads();
-
-    // ---- softmax update (wave-redundant from LDS).
-    float factor[4], m_new[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int h = mtile * 16 + l4 * 4 + r;
-      const float mo = m_reg[r];
-      m_new[r] = fmaxf(mo, fmaxf(wmax[0][h], wmax[1][h]));
-      factor[r] = exp2f(mo - m_new[r]);  // exp2(-inf - x) = 0 first time
-      m_reg[r] = m_new[r];
-    }
-    float rowsum[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float p = tok_ok ? exp2f(s_val[r] - m_new[r]) : 0.f;
-      p_lds[(mtile * 16 + l4 * 4 + r) * SUB + ntile * 16 + l16] =
-          from_f32<Tag>(p);
-      float v = p;
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-      rowsum[r] = v;
-    }
-    if (l16 == 0) {
+    for (int n = 0; n < 4; ++n)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int h = mtile * 16 + l4 * 4 + r;
-        wsum[ntile][h] = rowsum[r];
-        if (ntile == 0) {
-          m_st[h] = m_new[r];
-          f_st[h] = factor[r];
-        }
+        s[n][r] = n * 16 + r < left ? s[n][r] * scale_log2 : NEG;
+        mx = __builtin_amdgcn_fmed3f(mx, s[n][r], INFINITY);
       }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (__any(mx - m_run > (SPLIT_P ? GROWTH : 0.f))) {
+      const float m_new = fmaxf(m_run, mx);
+      const float f = __builtin_amdgcn_exp2f(m_run - m_new);
+      l_run *= f;
+#pragma unroll
+      for (int i = 0; i < LORA / 16; ++i) o[i] *= f;
+      m_run = m_new;
     }
-    __syncthreads();
-
-    // ---- PV: o_acc[mt] covers heads mt*16 + (l4*4 + r) rows.
+    // ---- O^T += V^T P^T, 32 keys at a time -------------------------------
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      // rescale accumulators by this subtile's factor per head row
+    for (int c = 0; c < 2; ++c) {
+      i32x4 hi, lo;
 #pragma unroll
-      for (int nf = 0; nf < 8; ++nf) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          o_acc[mt][nf][r] *= f_st[mt * 16 + l4 * 4 + r];
+      for (int j = 0; j < 4; ++j) {
+        const f32x4& sc = s[c * 2 + (j >> 1)];
+        const float p0 = __builtin_amdgcn_exp2f(sc[(j & 1) * 2] - m_run);
+        const float p1 = __builtin_amdgcn_exp2f(sc[(j & 1) * 2 + 1] - m_run);
+        hi[j] = pack2<Tag>(p0, p1);
+        l_run = SPLIT_P ? l_run + (p0 + p1) : add_pair<Tag>(hi[j], l_run);
+        lo[j] = SPLIT_P ? pack2<Tag>(p0 - unpack_lo<Tag>(hi[j]),
+                                     p1 - unpack_hi<Tag>(hi[j])) : 0;
       }
-      const int arow = mt * 16 + l16;  // A-frag head row
-      s16x8 afrag = *reinterpret_cast<const s16x8*>(
-          p_lds + arow * SUB + l4 * 8);
+      const s16x8 p_hi = __builtin_bit_cast(s16x8, hi);
+      const s16x8 p_lo = __builtin_bit_cast(s16x8, lo);
 #pragma unroll
-      for (int nf = 0; nf < 8; ++nf) {
-        const int col = wave * 128 + nf * 16 + l16;
-        s16x8 bfrag = *reinterpret_cast<const s16x8*>(
-            vt_lds + col * SUB + l4 * 8);
-        o_acc[mt][nf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            afrag, bfrag, o_acc[mt][nf], 0, 0, 0);
-      }
-    }
-    // l state update (one lane per head).
-    if (wave == 0 && tid < HG)
-      l_st[tid] = l_st[tid] * f_st[tid] + wsum[0][tid] + wsum[1][tid];
-    __syncthreads();
-  }
-
-  // ---- write out. o_acc rows: head = mt*16 + l4*4 + r; col = wave*128
-  // + nf*16 + l16.
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt) {
-#pragma unroll
-    for (int nf = 0; nf < 8; ++nf) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int h = hg0 + mt * 16 + l4 * 4 + r;
-        if (h >= num_heads) continue;
-        const int col = wave * 128 + nf * 16 + l16;
-        const float l = l_st[mt * 16 + l4 * 4 + r];
-        if (single) {
-          out[((long)seq * num_heads + h) * LORA + col] =
-              from_f32<Tag>(o_acc[mt][nf][r] / l);
-        } else {
-          tmp_out[(((long)seq * num_heads + h) * max_parts + part) * LORA +
-                  col] = o_acc[mt][nf][r];
-        }
+      for (int i = 0; i < LORA / 16; ++i) {
+        const char* at = t + v_at[i & 3] + c * 32 * (DK * 2) + (i >> 2) * 128;
+        const s16x4 a = lds_read_tr(at);
+        const s16x4 b = lds_read_tr(at + 16 * (DK * 2));
+        const s16x8 v = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+        if constexpr (SPLIT_P) o[i] = mfma16<Tag>(v, p_lo, o[i]);
+        o[i] = mfma16<Tag>(v, p_hi, o[i]);
       }
     }
   }
-  if (!single && wave == 0 && tid < HG) {
-    const int h = hg0 + tid;
-    if (h < num_heads) {
-      const long base = (((long)seq * num_heads + h) * max_parts + part) * 2;
-      tmp_lse[base] = m_st[tid];      // log2-domain max
-      tmp_lse[base + 1] = l_st[tid];  // sum
+
+  l_run += __shfl_xor(l_run, 16, 64);
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (head >= num_heads) return;
+  const int64_t hrow = (int64_t)row * num_heads + head;
+  if (PROMPT || num_parts == 1) {
+    const float inv_l = 1.f / l_run;
+    short* ob = out + hrow * LORA + l4 * 4;
+#pragma unroll
+    for (int i = 0; i < LORA / 16; ++i) {
+      int2 v;
+      v.x = pack2<Tag>(o[i][0] * inv_l, o[i][1] * inv_l);
+      v.y = pack2<Tag>(o[i][2] * inv_l, o[i][3] * inv_l);
+      *reinterpret_cast<int2*>(ob + i * 16) = v;
+    }
+  } else {
+    float* ob = tmp_out + (hrow * num_parts + part) * LORA + l4 * 4;
+#pragma unroll
+    for (int i = 0; i < LORA / 16; ++i)
+      *reinterpret_cast<f32x4*>(ob + i * 16) = o[i];
+    if (l4 == 0) {
+      tmp_lse[(hrow * num_parts + part) * 2] = m_run;
+      tmp_lse[(hrow * num_parts + part) * 2 + 1] = l_run;
     }
   }
 }
 
 // Merge partitions: out[s,h,:] = sum_p w_p * tmp[s,h,p,:] / sum_p w_p l_p
-// with w_p = exp2(m_p - m_max). Grid (T, Hq), 256 threads over 512 cols.
+// with w_p = exp2(m_p - m_max). One wave per (row, head), 8 columns each.
 template <typename Tag>
-__global__ void mla_reduce_kernel(short* __restrict__ out,
-                                  const float* __restrict__ tmp_out,
-                                  const float* __restrict__ tmp_lse,
-                                  const int* __restrict__ seq_lens,
-                                  int num_heads, int max_parts) {
-  const int seq = blockIdx.x;
-  const int h = blockIdx.y;
-  const int parts = min((seq_lens[seq] + PART - 1) / PART, max_parts);
-  const long lse_base = (((long)seq * num_heads + h) * max_parts) * 2;
-  float m = NEG_INF;
-  for (int p = 0; p < parts; ++p) m = fmaxf(m, tmp_lse[lse_base + p * 2]);
+__launch_bounds__(WAVE_SIZE) __global__
+void mla_reduce_kernel(short* __restrict__ out,
+                       const float* __restrict__ tmp_out,
+                       const float* __restrict__ tmp_lse,
+                       const int* __restrict__ seq_lens, int num_heads,
+                       int num_parts, int part_len) {
+  const int h = blockIdx.x;
+  const int seq = blockIdx.y;
+  const int parts = min((seq_lens[seq] + part_len - 1) / part_len, num_parts);
+  if (parts <= 0) return;
+  const int64_t hrow = (int64_t)seq * num_heads + h;
+  const float* lse = tmp_lse + hrow * num_parts * 2;
+  float m = NEG;
+  for (int p = 0; p < parts; ++p) m = fmaxf(m, lse[p * 2]);
   float l = 0.f;
-  for (int p = 0; p < parts; ++p)
-    l += exp2f(tmp_lse[lse_base + p * 2] - m) * tmp_lse[lse_base + p * 2 + 1];
-  const float inv_l = 1.f / l;
-  const long o_base = ((long)seq * num_heads + h) * (long)max_parts * LORA;
-  for (int c = threadIdx.x; c < LORA; c += blockDim.x) {
-    float acc = 0.f;
-    for (int p = 0; p < parts; ++p)
-      acc += exp2f(tmp_lse[lse_base + p * 2] - m) *
-             tmp_out[o_base + (long)p * LORA + c];
-    out[((long)seq * num_heads + h) * LORA + c] = from_f32<Tag>(acc * inv_l);
+  f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  const float* src = tmp_out + hrow * num_parts * LORA + threadIdx.x * 8;
+#pragma unroll 4
+  for (int p = 0; p < parts; ++p) {
+    const float w = __builtin_amdgcn_exp2f(lse[p * 2] - m);
+    l += w * lse[p * 2 + 1];
+    acc[0] += w * *reinterpret_cast<const f32x4*>(src + (int64_t)p * LORA);
+    acc[1] += w * *reinterpret_cast<const f32x4*>(src + (int64_t)p * LORA + 4);
   }
+  const float inv_l = 1.f / l;
+  i32x4 v;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    v[j] = pack2<Tag>(acc[j >> 1][(j & 1) * 2] * inv_l,
+                      acc[j >> 1][(j & 1) * 2 + 1] * inv_l);
+  *reinterpret_cast<i32x4*>(out + hrow * LORA + threadIdx.x * 8) = v;
+}
+
+static void check(const torch::Tensor& out, const torch::Tensor& q_nope,
+                  const torch::Tensor& q_pe, const torch::Tensor& kv_cache) {
+  TORCH_CHECK(q_nope.dim() == 3 && q_nope.size(2) == LORA,
+              "mla kernel expects kv_lora_rank=512");
+  TORCH_CHECK(q_pe.size(2) == ROPE, "mla kernel expects rope dim 64");
+  TORCH_CHECK(kv_cache.size(2) == DK);
+  TORCH_CHECK(q_nope.is_contiguous() && q_pe.is_contiguous() &&
+              out.is_contiguous() && kv_cache.is_contiguous());
+  TORCH_CHECK(out.scalar_type() == q_nope.scalar_type() &&
+              q_pe.scalar_type() == q_nope.scalar_type() &&
+              kv_cache.scalar_type() == q_nope.scalar_type());
+  TORCH_CHECK(q_nope.scalar_type() == torch::kBFloat16 ||
+                  q_nope.scalar_type() == torch::kHalf,
+              "mla kernel: bf16/fp16 only");
 }
 
 }  // namespace mla
 
+// Decode rows. tmp_out [T, Hq, parts, 512] and tmp_lse [T, Hq, parts, 2]
+// say into how many partitions the keys are split; empty means one.
 void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
                 torch::Tensor kv_cache, torch::Tensor block_table,
                 torch::Tensor seq_lens, double scale, int64_t max_seq_len,
                 torch::Tensor tmp_out, torch::Tensor tmp_lse) {
   using namespace mla;
-  TORCH_CHECK(q_nope.dim() == 3 && q_nope.size(2) == LORA,
-              "mla_decode expects kv_lora_rank=512");
-  TORCH_CHECK(q_pe.size(2) == ROPE, "mla_decode expects rope dim 64");
-  TORCH_CHECK(kv_cache.size(2) == DK);
-  TORCH_CHECK(q_nope.is_contiguous() && q_pe.is_contiguous() &&
-              out.is_contiguous() && kv_cache.is_contiguous());
-  TORCH_CHECK(out.scalar_type() == q_nope.scalar_type());
+  check(out, q_nope, q_pe, kv_cache);
   const int T = (int)q_nope.size(0);
+  if (T == 0) return;
   const int Hq = (int)q_nope.size(1);
   const int bs = (int)kv_cache.size(1);
-  const int parts = std::max<int>(1, (int)((max_seq_len + PART - 1) / PART));
-  if (parts > 1)
-    TORCH_CHECK(tmp_out.numel() >= (long)T * Hq * parts * LORA &&
-                tmp_lse.numel() >= (long)T * Hq * parts * 2);
+  int parts = 1;
+  if (tmp_out.numel() > 0) {
+    TORCH_CHECK(tmp_out.dim() == 4 && tmp_lse.dim() == 4 &&
+                tmp_out.is_contiguous() && tmp_lse.is_contiguous() &&
+                tmp_out.size(0) == T && tmp_lse.size(0) == T &&
+                tmp_out.size(1) == Hq && tmp_lse.size(1) == Hq &&
+                tmp_out.size(2) == tmp_lse.size(2) &&
+                tmp_out.size(3) == LORA && tmp_lse.size(3) == 2,
+                "mla scratch must be [T, Hq, parts, 512] and "
+                "[T, Hq, parts, 2]");
+    parts = (int)tmp_out.size(2);
+  }
+  const int part_len =
+      ceil_div(ceil_div((int)std::max<int64_t>(max_seq_len, 1), parts), SUB) *
+      SUB;
   auto stream = c10::hip::getCurrentHIPStream().stream();
   dim3 grid(T, parts, ceil_div(Hq, HG));
   auto launch = [&](auto tag) {
     using Tag = decltype(tag);
     hipLaunchKernelGGL(
-        (mla_decode_kernel<Tag>), grid, dim3(THREADS), 0, stream,
+        (mla_kernel<Tag, false, false>), grid, dim3(THREADS), 0, stream,
+        (short*)out.data_ptr(), (const short*)q_nope.data_ptr(),
+        (const short*)q_pe.data_ptr(), (const short*)kv_cache.data_ptr(),
+        block_table.data_ptr<int>(), (int)block_table.size(1), nullptr,
+        seq_lens.data_ptr<int>(), (float)scale * 1.4426950408889634f, Hq, bs,
+        T, T, parts > 1 ? tmp_out.data_ptr<float>() : nullptr,
+        parts > 1 ? tmp_lse.data_ptr<float>() : nullptr, parts, part_len);
+    if (parts > 1) {
+      HIP_CHECK_KERNEL();
+      hipLaunchKernelGGL((mla_reduce_kernel<Tag>), dim3(Hq, T),
+                         dim3(WAVE_SIZE), 0, stream, (short*)out.data_ptr(),
+                         tmp_out.data_ptr<float>(), tmp_lse.data_ptr<float>(),
+                         seq_lens.data_ptr<int>(), Hq, parts, part_len);
+    }
+  };
+  if (q_nope.scalar_type() == torch::kBFloat16) launch(BF16Tag{});
+  else launch(FP16Tag{});
+  HIP_CHECK_KERNEL();
+}
+
+// Prompt portions: requests num_decodes.. of the batch; q/out cover the
+// whole step.
+void mla_prefill(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
+                 torch::Tensor kv_cache, torch::Tensor block_table,
+                 torch::Tensor query_start_loc, torch::Tensor seq_lens,
+                 double scale, int64_t num_decodes) {
+  using namespace mla;
+  check(out, q_nope, q_pe, kv_cache);
+  const int reqs = (int)seq_lens.size(0);
+  const int rows = (int)(q_nope.size(0) - num_decodes);
+  if (reqs <= num_decodes || rows <= 0) return;
+  TORCH_CHECK(query_start_loc.numel() > reqs);
+  const int Hq = (int)q_nope.size(1);
+  auto stream = c10::hip::getCurrentHIPStream().stream();
+  dim3 grid(rows, 1, ceil_div(Hq, HG));
+  auto launch = [&](auto tag) {
+    using Tag = decltype(tag);
+    hipLaunchKernelGGL(
+        (mla_kernel<Tag, true, true>), grid, dim3(THREADS), 0, stream,
         (short*)out.data_ptr(), (const short*)q_nope.data_ptr(),
         (const short*)q_pe.data_ptr(), (const short*)kv_cache.data_ptr(),
         block_table.data_ptr<int>(), (int)block_table.size(1),
-        seq_lens.data_ptr<int>(), (float)scale, Hq, bs,
-        parts > 1 ? tmp_out.data_ptr<float>() : nullptr,
-        parts > 1 ? tmp_lse.data_ptr<float>() : nullptr, parts);
-    if (parts > 1) {
-      hipLaunchKernelGGL((mla_reduce_kernel<Tag>), dim3(T, Hq), dim3(256),
-                         0, stream, (short*)out.data_ptr(),
-                         tmp_out.data_ptr<float>(),
-                         tmp_lse.data_ptr<float>(),
-                         seq_lens.data_ptr<int>(), Hq, parts);
-    }
+        query_start_loc.data_ptr<int>(), seq_lens.data_ptr<int>(),
+        (float)scale * 1.4426950408889634f, Hq, (int)kv_cache.size(1),
+        (int)num_decodes, reqs, nullptr, nullptr, 1, 0x7fffff00);
   };
-  if (q_nope.scalar_type() == torch::kBFloat16)
-    launch(BF16Tag{});
-  else if (q_nope.scalar_type() == torch::kHalf)
-    launch(FP16Tag{});
-  else
-    TORCH_CHECK(false, "mla_decode: bf16/fp16 only");
+  if (q_nope.scalar_type() == torch::kBFloat16) launch(BF16Tag{});
+  else launch(FP16Tag{});
   HIP_CHECK_KERNEL();
 }
 

@@ -120,9 +120,7 @@ class DeepseekMLAAttention(nn.Module):
         self.rotary_emb(positions, q_pe, k_pe)
 
         # Absorb W_UK: q' [T, h, lora].
-        q_absorbed = torch.einsum(
-            "thn,hnl->thl", q_nope.float(), self.w_uk.float()
-        ).to(hidden.dtype)
+        q_absorbed = ops.head_matmul(q_nope, self.w_uk)
 
         ctx = get_forward_context()
         meta = ctx.attn_metadata
@@ -139,8 +137,7 @@ class DeepseekMLAAttention(nn.Module):
                 num_decodes=meta.num_decodes, max_seq_len=meta.max_seq_len,
             )
         # Un-absorb W_UV: [T, h, v].
-        out = torch.einsum("thl,hlv->thv", o_c.float(),
-                           self.w_uv.float()).to(hidden.dtype)
+        out = ops.head_matmul(o_c, self.w_uv)
         return self.o_proj(out.reshape(T, -1))
 
     def _profile_attention(self, q_absorbed, q_pe, c_kv, k_pe, meta):

@@ -145,6 +145,12 @@ def mla_attention(q_nope, q_pe, kv_cache, block_table, query_start_loc,
     )
 
 
+def head_matmul(x, w):
+    """x [T, H, K] times a matrix of its own per head, w [H, K, N]:
+    [T, H, N], summed in fp32."""
+    return get_backend(x.device).head_matmul(x, w)
+
+
 def grouped_topk(gating, topk, renormalize=True, num_groups=0,
                  topk_groups=0, scoring_func="softmax", e_score_bias=None,
                  routed_scaling_factor=1.0):

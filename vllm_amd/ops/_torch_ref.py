@@ -275,6 +275,11 @@ def mla_attention(
     return out
 
 
+def head_matmul(x, w):
+    """x [T, H, K] times a matrix of its own per head, w [H, K, N]."""
+    return torch.einsum("thk,hkn->thn", x.float(), w.float()).to(x.dtype)
+
+
 def grouped_topk(
     gating, topk, renormalize=True, num_groups=0, topk_groups=0,
     scoring_func="softmax", e_score_bias=None, routed_scaling_factor=1.0,

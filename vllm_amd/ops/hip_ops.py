@@ -211,7 +211,22 @@ from vllm_amd.ops._torch_ref import (  # noqa: E402,F401
     topk_softmax,
 )
 
-_MLA_PART = 1024  # must match mla::PART in csrc/mla.hip
+# MLA decode: one workgroup (128 heads of a row) fits on each of the 256
+# CUs; a partition of its keys costs 256 KB of fp32 partials written and
+# read.
+_MLA_FILL = 256
+_MLA_PART_MIN = 128
+
+
+def _mla_parts(rows, heads, max_seq_len):
+    """Into how many partitions a row's keys are split: as many as fill
+    the chip and no more (128 heads, us: 128 rows x 129..2176 keys 182 in
+    one, 116 in 2, 140 in 4; 32 x 8192 keys 125 in 8, 150 in 16), none
+    shorter than two tiles (one row x 1000 keys 36 in 4, 27 in 8; x 4000
+    39 in 16, 33 in 32, 37 in 63), at most 64."""
+    groups = rows * -(-heads // 128)
+    return max(1, min(-(-_MLA_FILL // max(groups, 1)),
+                      -(-max_seq_len // _MLA_PART_MIN), 64))
 
 
 def mla_decode(q_nope, q_pe, kv_cache, block_table, seq_lens, scale,
@@ -222,7 +237,7 @@ def mla_decode(q_nope, q_pe, kv_cache, block_table, seq_lens, scale,
     out = torch.empty(T, Hq, lora, dtype=q_nope.dtype, device=q_nope.device)
     if max_seq_len <= 0:
         max_seq_len = int(seq_lens.max().item())
-    parts = max(1, -(-max_seq_len // _MLA_PART))
+    parts = _mla_parts(T, Hq, max_seq_len)
     if parts > 1:
         tmp_out = torch.empty(T, Hq, parts, lora, dtype=torch.float32,
                               device=q_nope.device)
@@ -238,29 +253,41 @@ def mla_decode(q_nope, q_pe, kv_cache, block_table, seq_lens, scale,
 
 def mla_attention(q_nope, q_pe, kv_cache, block_table, query_start_loc,
                   seq_lens, scale, num_decodes=0, max_seq_len=0):
-    """Decode rows (query_len==1, first num_decodes) on the HIP MFMA
-    kernel; prefill rows on the torch composition (MLA prefill runs per
-    scheduler chunk — a bounded, non-steady-state path)."""
+    """Decode rows (query_len==1, first num_decodes) and prompt rows on
+    the MFMA kernel (csrc/mla.hip). Other latent widths, types or cache
+    types take the torch composition."""
     T = q_nope.shape[0]
-    num_reqs = seq_lens.shape[0]
     use_hip = (q_nope.shape[2] == 512 and q_pe.shape[2] == 64
                and q_nope.dtype in (torch.bfloat16, torch.float16)
+               and q_pe.dtype == q_nope.dtype
                and kv_cache.dtype == q_nope.dtype)
-    if num_decodes > 0 and use_hip:
-        out_dec = mla_decode(
-            q_nope[:num_decodes].contiguous(),
-            q_pe[:num_decodes].contiguous(), kv_cache,
+    if not use_hip:
+        return _torch_ref.mla_attention(
+            q_nope, q_pe, kv_cache, block_table, query_start_loc, seq_lens,
+            scale)
+    q_nope, q_pe = q_nope.contiguous(), q_pe.contiguous()
+    if num_decodes == T:
+        return mla_decode(q_nope, q_pe, kv_cache, block_table,
+                          seq_lens[:num_decodes], scale, max_seq_len)
+    out = torch.empty_like(q_nope)
+    if num_decodes > 0:
+        out[:num_decodes] = mla_decode(
+            q_nope[:num_decodes], q_pe[:num_decodes], kv_cache,
             block_table, seq_lens[:num_decodes], scale, max_seq_len)
-        if num_decodes == T:
-            return out_dec
-        qsl = query_start_loc[num_decodes:] - num_decodes
-        out_pre = _torch_ref.mla_attention(
-            q_nope[num_decodes:], q_pe[num_decodes:], kv_cache,
-            block_table[num_decodes:], qsl, seq_lens[num_decodes:], scale)
-        return torch.cat([out_dec, out_pre], dim=0)
-    return _torch_ref.mla_attention(
-        q_nope, q_pe, kv_cache, block_table, query_start_loc, seq_lens,
-        scale)
+    _C.mla_prefill(out, q_nope, q_pe, kv_cache, block_table,
+                   query_start_loc, seq_lens, scale, num_decodes)
+    return out
+
+
+def head_matmul(x, w):
+    """out[t, h] = x[t, h] @ w[h], fp32 sums, result in x's type."""
+    if (x.dtype in (torch.bfloat16, torch.float16) and x.dtype == w.dtype
+            and w.shape[1] % 128 == 0 and w.shape[2] % 128 == 0
+            and w.is_contiguous() and x.stride(2) == 1
+            and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0
+            and x.data_ptr() % 16 == 0):
+        return _C.head_matmul(x, w)
+    return _torch_ref.head_matmul(x, w)
 
 
 _MOE_BM = 64  # must match moe::BM in csrc/moe.hip
