@@ -611,6 +611,44 @@ def test_head_matmul(T, H, K, N, dtype):
                  else 2**-10)
 
 
+@pytest.mark.parametrize("T,H,I,E,K,act", [
+    (33, 128, 128, 6, 2, "relu2"),    # streamed, part of a 64-row tile
+    (1100, 128, 64, 128, 2, "silu"),  # streamed, counted by blocks of rows
+    (70, 256, 192, 5, 2, "silu"),     # 128-row tiles, ragged last columns
+    (260, 128, 128, 3, 1, "relu2"),
+    (1100, 128, 192, 4, 2, "silu"),   # 256-row tiles
+    (400, 384, 128, 2, 1, "relu2"),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_moe_forms(T, H, I, E, K, act, dtype):
+    """Each form of the expert products, half of the rows on one expert
+    and none on the last. Against 64 bits; three roundings to the type
+    (activation, expert's output, sum) and fp32 sums bound the error."""
+    hip = _hip()
+    hidden = torch.randn(T, H, device="cuda", dtype=dtype)
+    g = 2 if act == "silu" else 1
+    w13 = torch.randn(E, g * I, H, device="cuda", dtype=dtype) * H**-0.5
+    w2 = torch.randn(E, H, I, device="cuda", dtype=dtype) * I**-0.5
+    ti = torch.randint(0, E - 1, (T, K), device="cuda", dtype=torch.int32)
+    ti[: T // 2, 0] = 0
+    tw = torch.rand(T, K, device="cuda")
+    out = hip.fused_moe(hidden, w13, w2, tw, ti, act).double()
+    expect, bound = torch.zeros_like(out), torch.zeros_like(out)
+    for e in range(E):
+        t, k = (ti == e).nonzero(as_tuple=True)
+        y = hidden[t].double() @ w13[e].double().T
+        a = (torch.nn.functional.silu(y[:, :I]) * y[:, I:] if g == 2
+             else y.relu() ** 2)
+        w = tw[t, k].double()[:, None]
+        y, mag = a @ w2[e].double().T, a.abs() @ w2[e].double().abs().T
+        expect.index_add_(0, t, w * y)
+        bound.index_add_(0, t, w * (mag + y.abs()))
+    # Rounding to p significant bits is off by 2^-p of the value: p = 8, 11.
+    eps = 2**-8 if dtype == torch.bfloat16 else 2**-11
+    assert ((out - expect).abs()
+            <= 1.1 * eps * (bound + expect.abs()) + 2**-20).all()
+
+
 def test_mla_unified_dispatch_mixed_batch():
     """ops.mla_attention routes decode rows to the kernel and prefill
     rows to the torch path; both must agree with the all-torch result."""

@@ -43,7 +43,8 @@ SOURCES = [
 # These kernels keep matrix-core accumulators in ordinary vector
 # registers: they are rescaled by the vector ALU between products, and
 # through the accumulation registers every rescale is a copy each way.
-VGPR_ACCUMULATORS = {"attention_decode", "attention_prefill", "mla", "head_matmul"}
+VGPR_ACCUMULATORS = {"attention_decode", "attention_prefill", "mla", "head_matmul",
+                     "moe"}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("PYTORCH_ROCM_ARCH", "gfx950")

@@ -38,19 +38,20 @@ void dynamic_quant_fp8(torch::Tensor out, torch::Tensor scales,
 void scale_rows_cols(torch::Tensor y, torch::Tensor row_scales,
                      torch::Tensor col_scales,
                      c10::optional<torch::Tensor> bias);
-void moe_align(torch::Tensor topk_ids, int64_t num_experts,
+void moe_align(torch::Tensor topk_ids, int64_t num_experts, int64_t tile_rows,
                torch::Tensor sorted, torch::Tensor expert_tiles,
-               torch::Tensor inv_perm, torch::Tensor counts,
-               torch::Tensor fill, torch::Tensor off);
+               torch::Tensor inv_perm, torch::Tensor scratch);
+int64_t moe_tile_rows(int64_t form);
 void moe_gemm(torch::Tensor a, torch::Tensor b, torch::Tensor c,
               torch::Tensor sorted, torch::Tensor expert_tiles,
-              int64_t topk_div, int64_t total_flat);
+              int64_t topk_div, int64_t total_flat, int64_t act,
+              int64_t form);
 void moe_combine(torch::Tensor out, torch::Tensor y,
                  torch::Tensor topk_weights, torch::Tensor inv_perm);
 void moe_gemm_shuf(torch::Tensor a, torch::Tensor b_shuf, torch::Tensor c,
                    torch::Tensor sorted, torch::Tensor expert_tiles,
                    int64_t n, int64_t k, int64_t topk_div,
-                   int64_t total_flat);
+                   int64_t total_flat, int64_t act);
 void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
                 torch::Tensor kv_cache, torch::Tensor block_table,
                 torch::Tensor seq_lens, double scale, int64_t max_seq_len,
@@ -184,16 +185,18 @@ TORCH_LIBRARY(vllm_amd, m) {
         " -> ()");
   m.def("scale_rows_cols(Tensor(a!) y, Tensor row_scales, Tensor col_scales,"
         " Tensor? bias) -> ()");
-  m.def("moe_align(Tensor topk_ids, int num_experts, Tensor(a!) sorted, "
-        "Tensor(b!) expert_tiles, Tensor(c!) inv_perm, Tensor(d!) counts, "
-        "Tensor(e!) fill, Tensor(f!) off) -> ()");
+  m.def("moe_align(Tensor topk_ids, int num_experts, int tile_rows, "
+        "Tensor(a!) sorted, Tensor(b!) expert_tiles, Tensor(c!) inv_perm, "
+        "Tensor(d!) scratch) -> ()");
+  m.def("moe_tile_rows(int form) -> int", &vllm_amd::moe_tile_rows);
   m.def("moe_gemm(Tensor a, Tensor b, Tensor(a!) c, Tensor sorted, "
-        "Tensor expert_tiles, int topk_div, int total_flat) -> ()");
+        "Tensor expert_tiles, int topk_div, int total_flat, int act, "
+        "int form) -> ()");
   m.def("moe_combine(Tensor(a!) out, Tensor y, Tensor topk_weights, "
         "Tensor inv_perm) -> ()");
   m.def("moe_gemm_shuf(Tensor a, Tensor b_shuf, Tensor(a!) c, "
         "Tensor sorted, Tensor expert_tiles, int n, int k, int topk_div, "
-        "int total_flat) -> ()");
+        "int total_flat, int act) -> ()");
   m.def("mla_decode(Tensor(a!) out, Tensor q_nope, Tensor q_pe, "
         "Tensor kv_cache, Tensor block_table, Tensor seq_lens, "
         "float scale, int max_seq_len, Tensor(b!) tmp_out, "

@@ -215,9 +215,21 @@ DEVINL void lds_fill16(const void* src, void* dst) {
       : "s"(at), "v"(src)
       : "memory", "m0");
 }
-// vmcnt(0); the builtin, so that the compiler knows its own older loads to
-// be done as well and does not wait again after the next fill.
-DEVINL void lds_fill_wait() { __builtin_amdgcn_s_waitcnt(0x0f70); }
+// At most N (< 64) of this wave's loads still under way; the builtin, so
+// that the compiler knows its own older loads to be done as well and does
+// not wait again after the next fill.
+template <int N = 0> DEVINL void lds_fill_wait() {
+  static_assert(N >= 0 && N < 64);
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+}
+// Workgroup barrier that waits for this wave's LDS operations but not for
+// its loads (__syncthreads may wait for both).
+DEVINL void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
 
 // ---------------------------------------------------------------------------
 // Wave reductions (64 lanes).

@@ -3,21 +3,30 @@
 // Role of the reference's Triton grouped GEMM
 // (vllm/model_executor/layers/fused_moe/fused_moe.py:299) and
 // moe_align_block_size (csrc/libtorch_stable/moe/moe_align_sum_kernels.cu:326),
-// redesigned as hand-written MFMA kernels: tokens are sorted by expert
-// into BLOCK_M=64 tiles on-device (no host sync — shapes depend only on
-// (T, topk, E), so the whole MoE layer is hipGraph-capturable), then a
-// tiled 16x16x32-bf16 MFMA GEMM streams each expert's weights from HBM
-// once per m-tile. Decode-shape MoE is weight-bound (~32 flops per
-// weight byte at BM=64), so the kernel targets the HBM roofline, not
-// peak MFMA.
+// as hand-written MFMA kernels: (token, slot) rows are sorted by expert
+// into tiles on the device (no host sync; shapes depend only on (T, topk,
+// E), so the whole layer is hipGraph-capturable), then two products run
+// over the tiles. The activation is the first product's epilogue: gate
+// and up rows of the same columns belong to one workgroup.
+//
+// Two forms of the product, chosen by the average number of rows an
+// expert gets (ops/hip_ops.py):
+//   moe_stream_kernel  few rows: every weight is read once and used for at
+//                      most 64 rows, so HBM bounds it. Weights go straight
+//                      into MFMA fragments, no LDS and no barrier in the
+//                      loop. Weights may be stored in fragment order
+//                      ([E][N/16][K/32][64 lanes][8], ops/hip_ops.py
+//                      moe_shuffle_weights): then a wave's load is one run
+//                      of 1 KB.
+//   moe_tile_kernel    many rows: the matrix cores bound it; 128 or 256 x
+//                      256 tiles through LDS.
 //
 // Pipeline (ops/hip_ops.py fused_moe):
 //   moe_align: counts -> tile-aligned offsets -> sorted flat ids + the
-//              inverse permutation (combine is deterministic, no atomics)
-//   moe_gemm(hidden, w13)   -> y [EM, 2I]   (A rows gathered via sorted)
-//   silu_and_mul(y)         -> act [EM, I]  (existing elementwise kernel)
-//   moe_gemm(act, w2)       -> y2 [EM, H]   (A rows in sorted order)
-//   moe_combine: out[t] = sum_k w[t,k] * y2[inv_perm[t*K+k]]
+//              inverse permutation (combine is deterministic)
+//   moe_gemm(hidden, w13) + activation -> act [EM, I] (rows gathered)
+//   moe_gemm(act, w2)                  -> y [EM, H]   (rows in tile order)
+//   moe_combine: out[t] = sum_k w[t,k] * y[inv_perm[t*K+k]]
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
@@ -29,305 +38,536 @@ namespace vllm_amd {
 
 namespace moe {
 
-constexpr int BM = 64;    // token rows per tile (must divide align padding)
-constexpr int BN = 128;   // output cols per block
-constexpr int BK = 64;    // K step staged in LDS
+constexpr int BM = 64;    // token rows per tile of the few-row kernels
 constexpr int THREADS = 256;
 constexpr int SENTINEL = 0x7fffffff;
+constexpr int MAX_EXPERTS = 1024;
 
 // --------------------------------------------------------------------------
-// Alignment kernels.
-__global__ void zero_kernel(int* counts, int* fill, int e) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < e) {
-    counts[i] = 0;
-    fill[i] = 0;
-  }
-}
+// Alignment. Counting and placing with one atomic per row on global
+// counters costs 113 us at 32768 rows (every row of an expert waits for
+// the one before); counters in LDS, one set per block of 2048 rows, and a
+// prefix over the blocks cost 29 us. Up to 2048 rows one workgroup does it
+// all in one launch (four before).
+constexpr int ALIGN_ROWS = 2048;   // rows per block
 
-__global__ void count_kernel(const int* __restrict__ topk_ids, int total,
-                             int* __restrict__ counts) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < total) atomicAdd(&counts[topk_ids[i]], 1);
-}
-
-// One block: tile-aligned exclusive offsets, expert id per tile, sorted
-// array pre-filled with SENTINEL. E <= a few hundred, EM up to ~1M.
-__global__ void scan_kernel(const int* __restrict__ counts, int e,
-                            int* __restrict__ off,
-                            int* __restrict__ expert_tiles, int max_tiles,
-                            int* __restrict__ sorted, int em_max) {
-  __shared__ int total_tiles_sh;
-  if (threadIdx.x == 0) {
-    int tok_off = 0;
-    for (int i = 0; i < e; ++i) {
-      off[i] = tok_off;
-      tok_off += (counts[i] + BM - 1) / BM * BM;
-    }
-    total_tiles_sh = tok_off / BM;
-  }
-  __syncthreads();
-  const int total_tiles = total_tiles_sh;
-  for (int t = threadIdx.x; t < max_tiles; t += blockDim.x) {
-    int ex = -1;
-    if (t < total_tiles) {
-      // tile t belongs to the expert whose [off, off+aligned) covers it.
-      // Linear scan per tile is fine: E small, one block total.
-      for (int i = e - 1; i >= 0; --i) {
-        if (t * BM >= off[i]) {
-          ex = i;
-          break;
-        }
-      }
-    }
-    expert_tiles[t] = ex;
-  }
-  for (int i = threadIdx.x; i < em_max; i += blockDim.x)
-    sorted[i] = SENTINEL;
-}
-
-__global__ void scatter_kernel(const int* __restrict__ topk_ids, int total,
-                               const int* __restrict__ off,
-                               int* __restrict__ fill,
-                               int* __restrict__ sorted,
-                               int* __restrict__ inv_perm) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  int e = topk_ids[i];
-  int pos = off[e] + atomicAdd(&fill[e], 1);
-  sorted[pos] = i;
-  inv_perm[i] = pos;
-}
-
-// --------------------------------------------------------------------------
-// Grouped GEMM: C[m, n] = sum_k A[row(m), k] * B[expert(m), n, k].
-// Per 16x16x32 MFMA: A-frag lane&15 = row, k = (lane>>4)*8 + j;
-// B-frag lane&15 = col, same k split; C-frag col = lane&15,
-// row = (lane>>4)*4 + reg (conventions proven in attention_prefill.hip).
-//
-// LDS XOR swizzle (guide T2): byte offset ^= (row&7)<<4 spreads the 16
-// same-column rows of a fragment read across 8 distinct 16B slots.
-DEVINL int swz(int row, int byte_off) { return byte_off ^ ((row & 7) << 4); }
-
-template <typename Tag>
-__launch_bounds__(THREADS) __global__
-void moe_gemm_kernel(const short* __restrict__ A, long lda,
-                     const short* __restrict__ B, long expert_stride,
-                     long ldb, short* __restrict__ C, long ldc,
-                     const int* __restrict__ sorted,
-                     const int* __restrict__ expert_tiles, int K, int N,
-                     int topk_div, int total_flat) {
-  const int tile_m = blockIdx.y;
-  const int n0 = blockIdx.x * BN;
-  const int expert = expert_tiles[tile_m];
-  if (expert < 0) return;  // padding tile
-
-  __shared__ short a_lds[BM * BK];  // [row][k], swizzled rows
-  __shared__ short b_lds[BN * BK];  // [col][k], swizzled cols
-  __shared__ int rows_sh[BM];       // A source row per tile row (-1 pad)
-  __shared__ int cval_sh[BM];       // sorted id per tile row (C row valid)
-
+// counts[e] -> off[e] = first row of expert e in tile order, and what the
+// products read per tile. Called by all THREADS threads of one workgroup.
+DEVINL void place_experts(const int* counts, int* off, int e, int bm,
+                          int* __restrict__ expert_tiles, int max_tiles,
+                          int* __restrict__ sorted, int* scan) {
   const int tid = threadIdx.x;
-  if (tid < BM) {
-    int sid = sorted[tile_m * BM + tid];
-    cval_sh[tid] = (sid < total_flat) ? 1 : 0;
-    rows_sh[tid] = (sid < total_flat)
-                       ? (topk_div > 0 ? sid / topk_div : tile_m * BM + tid)
-                       : -1;
-  }
+  const int per = (e + THREADS - 1) / THREADS;
+  int tiles = 0;
+  for (int i = tid * per; i < min(e, (tid + 1) * per); ++i)
+    tiles += (counts[i] + bm - 1) / bm;
+  scan[tid] = tiles;
   __syncthreads();
-
-  const int wave = tid / WAVE_SIZE;
-  const int lane = tid % WAVE_SIZE;
-  const int l16 = lane & 15;
-  const int l4 = lane >> 4;       // 0..3: k-quarter for A/B frags
-  const int wm = wave & 1;        // m 32-half (2 m-frags of 16)
-  const int wn = wave >> 1;       // n 64-half (4 n-frags of 16)
-
-  f32x4 acc[2][4];
-#pragma unroll
-  for (int m = 0; m < 2; ++m)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const short* b_exp = B + (long)expert * expert_stride;
-
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    // Stage A: BM rows x 64 cols bf16 = BM x 128B; 16B per thread-chunk.
-    {
-#pragma unroll
-      for (int it = 0; it < BM * 8 / THREADS; ++it) {
-        const int idx = it * THREADS + tid;
-        const int r = idx >> 3;
-        const int cb = (idx & 7) * 16;   // byte col 0..112
-        const int arow = rows_sh[r];
-        s16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (arow >= 0)
-          v = *reinterpret_cast<const s16x8*>(A + (long)arow * lda + k0 +
-                                              (cb >> 1));
-        *reinterpret_cast<s16x8*>(
-            reinterpret_cast<char*>(a_lds) + r * 128 + swz(r, cb)) = v;
-      }
-    }
-    // Stage B: 128 rows (n) x 64 cols = 128 x 128B; 4 x 16B per thread.
-    {
-#pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        const int idx = it * THREADS + tid;   // 0..1023
-        const int n = idx >> 3;
-        const int cb = (idx & 7) * 16;
-        s16x8 v = *reinterpret_cast<const s16x8*>(
-            b_exp + (long)(n0 + n) * ldb + k0 + (cb >> 1));
-        *reinterpret_cast<s16x8*>(
-            reinterpret_cast<char*>(b_lds) + n * 128 + swz(n, cb)) = v;
-      }
-    }
+  for (int d = 1; d < THREADS; d <<= 1) {
+    const int v = tid >= d ? scan[tid - d] : 0;
     __syncthreads();
-    // 2 K-steps of 32 within the tile.
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      const int kb = kk * 64 + l4 * 16;  // byte offset of this lane's 8 elems
-      s16x8 afrag[2];
-#pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        const int arow = wm * 32 + m * 16 + l16;
-        afrag[m] = *reinterpret_cast<const s16x8*>(
-            reinterpret_cast<const char*>(a_lds) + arow * 128 +
-            swz(arow, kb));
-      }
-#pragma unroll
-      for (int nf = 0; nf < 4; ++nf) {
-        const int bcol = wn * 64 + nf * 16 + l16;
-        s16x8 bfrag = *reinterpret_cast<const s16x8*>(
-            reinterpret_cast<const char*>(b_lds) + bcol * 128 +
-            swz(bcol, kb));
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-          acc[m][nf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              afrag[m], bfrag, acc[m][nf], 0, 0, 0);
-      }
-    }
+    scan[tid] += v;
     __syncthreads();
   }
+  int t = scan[tid] - tiles;
+  const int total = scan[THREADS - 1];
+  for (int i = tid * per; i < min(e, (tid + 1) * per); ++i) {
+    const int n = counts[i];
+    off[i] = t * bm;
+    for (int k = 0; k < n; k += bm) expert_tiles[t++] = i;
+    for (int k = n; k % bm != 0; ++k) sorted[off[i] + k] = SENTINEL;
+  }
+  for (int i = total + tid; i < max_tiles; i += THREADS) expert_tiles[i] = -1;
+  __syncthreads();
+}
 
-  // Epilogue: C rows are sorted positions; skip padding rows.
-#pragma unroll
-  for (int m = 0; m < 2; ++m) {
-#pragma unroll
-    for (int nf = 0; nf < 4; ++nf) {
-      const int n = n0 + wn * 64 + nf * 16 + l16;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int mrow = wm * 32 + m * 16 + l4 * 4 + r;
-        if (cval_sh[mrow])
-          C[(long)(tile_m * BM + mrow) * ldc + n] =
-              from_f32<Tag>(acc[m][nf][r]);
-      }
+__global__ __launch_bounds__(THREADS) void align_small_kernel(
+    const int* __restrict__ ids, int total, int e, int bm,
+    int* __restrict__ expert_tiles, int max_tiles, int* __restrict__ sorted,
+    int* __restrict__ inv_perm) {
+  __shared__ int counts[MAX_EXPERTS], off[MAX_EXPERTS], scan[THREADS];
+  for (int i = threadIdx.x; i < e; i += THREADS) counts[i] = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < total; i += THREADS)
+    atomicAdd(&counts[ids[i]], 1);
+  __syncthreads();
+  place_experts(counts, off, e, bm, expert_tiles, max_tiles, sorted, scan);
+  for (int i = threadIdx.x; i < total; i += THREADS) {
+    const int pos = atomicAdd(&off[ids[i]], 1);
+    sorted[pos] = i;
+    inv_perm[i] = pos;
+  }
+}
+
+// part[b][e]: rows of expert e in block b.
+__global__ __launch_bounds__(THREADS) void align_count_kernel(
+    const int* __restrict__ ids, int total, int e, int* __restrict__ part) {
+  __shared__ int counts[MAX_EXPERTS];
+  for (int i = threadIdx.x; i < e; i += THREADS) counts[i] = 0;
+  __syncthreads();
+  const int end = min(total, ((int)blockIdx.x + 1) * ALIGN_ROWS);
+  for (int i = blockIdx.x * ALIGN_ROWS + threadIdx.x; i < end; i += THREADS)
+    atomicAdd(&counts[ids[i]], 1);
+  __syncthreads();
+  for (int i = threadIdx.x; i < e; i += THREADS)
+    part[(int64_t)blockIdx.x * e + i] = counts[i];
+}
+
+// part[b][e] -> first row of block b's rows of expert e.
+__global__ __launch_bounds__(THREADS) void align_place_kernel(
+    int* __restrict__ part, int blocks, int e, int bm,
+    int* __restrict__ expert_tiles, int max_tiles, int* __restrict__ sorted) {
+  __shared__ int counts[MAX_EXPERTS], off[MAX_EXPERTS], scan[THREADS];
+  for (int i = threadIdx.x; i < e; i += THREADS) {
+    int n = 0;
+    for (int b = 0; b < blocks; ++b) n += part[(int64_t)b * e + i];
+    counts[i] = n;
+  }
+  __syncthreads();
+  place_experts(counts, off, e, bm, expert_tiles, max_tiles, sorted, scan);
+  for (int i = threadIdx.x; i < e; i += THREADS) {
+    int at = off[i];
+    for (int b = 0; b < blocks; ++b) {
+      const int n = part[(int64_t)b * e + i];
+      part[(int64_t)b * e + i] = at;
+      at += n;
     }
   }
 }
 
-// --------------------------------------------------------------------------
-// Fragment-major grouped GEMM: B is pre-shuffled at weight-load time
-// into MFMA-fragment order [E][N/16][K/32][64 lanes][8 elems] so each
-// wave reads its B-fragment as ONE coalesced 16B/lane chunk straight
-// from HBM. A-fragments load per-lane from global (scattered but tiny —
-// <1% of traffic, L3-resident across the N/128 blocks sharing the
-// m-tile). ZERO LDS and ZERO barriers in the k-loop: nothing forces a
-// vmcnt(0) drain, so the compiler pipelines the weight stream at full
-// depth (the staged-LDS variant stalls on the barrier drain — guide
-// §Composed models). This is the MI355X-first inference layout:
-// weights are written once and streamed billions of times, so they
-// belong in consumer order.
-template <typename Tag>
-__launch_bounds__(THREADS) __global__
-void moe_gemm_shuf_kernel(const short* __restrict__ A, long lda,
-                          const short* __restrict__ B, long expert_stride,
-                          short* __restrict__ C, long ldc,
-                          const int* __restrict__ sorted,
-                          const int* __restrict__ expert_tiles, int K,
-                          int N, int topk_div, int total_flat) {
-  const int tile_m = blockIdx.y;
-  const int n0 = blockIdx.x * BN;
-  const int expert = expert_tiles[tile_m];
-  if (expert < 0) return;  // padding tile
+__global__ __launch_bounds__(THREADS) void align_scatter_kernel(
+    const int* __restrict__ ids, int total, int e,
+    const int* __restrict__ part, int* __restrict__ sorted,
+    int* __restrict__ inv_perm) {
+  __shared__ int off[MAX_EXPERTS];
+  for (int i = threadIdx.x; i < e; i += THREADS)
+    off[i] = part[(int64_t)blockIdx.x * e + i];
+  __syncthreads();
+  const int end = min(total, ((int)blockIdx.x + 1) * ALIGN_ROWS);
+  for (int i = blockIdx.x * ALIGN_ROWS + threadIdx.x; i < end; i += THREADS) {
+    const int pos = atomicAdd(&off[ids[i]], 1);
+    sorted[pos] = i;
+    inv_perm[i] = pos;
+  }
+}
 
-  const int tid = threadIdx.x;
-  const int wave = tid / WAVE_SIZE;
-  const int lane = tid % WAVE_SIZE;
+// --------------------------------------------------------------------------
+// What the epilogue of a product does.
+enum Act { NONE = 0, SILU_GATED = 1, RELU2 = 2 };
+
+DEVINL float silu_mul(float g, float u) { return g / (1.f + __expf(-g)) * u; }
+DEVINL float relu2(float x) {
+  const float r = fmaxf(x, 0.f);
+  return r * r;
+}
+
+// Which (row tile, column block) a workgroup takes; every eighth workgroup
+// runs on the same XCD. `split` column parts are spread over the XCDs and
+// groups of 8 / split row tiles over the XCDs of a part: what an XCD runs
+// at a time then shares weights (the tiles of an expert) and rows (the
+// blocks of its part) in its L2. split 0: a run of neighbours in (column
+// block, row tile) order per XCD, for grids too small to deal out.
+DEVINL bool tile_of_block(int m_tiles, int n_blocks, int split, int& m,
+                          int& n) {
+  const int x = (int)blockIdx.x & 7;
+  const int l = (int)blockIdx.x >> 3;
+  if (split == 0) {
+    const int total = m_tiles * n_blocks;
+    const int per = (total + 7) / 8;
+    const int p = x * per + l;
+    if (l >= per || p >= total) return false;
+    m = p % m_tiles;
+    n = p / m_tiles;
+    return true;
+  }
+  const int gm = 8 / split;
+  const int nb = (n_blocks + split - 1) / split;
+  const int n_lo = x % split * nb;
+  const int nn = min(nb, n_blocks - n_lo);
+  if (nn <= 0) return false;
+  const int q = l % (gm * nn);
+  m = (l / (gm * nn) * gm + x / split) * gm + q % gm;
+  n = n_lo + q / gm;
+  return m < m_tiles;
+}
+
+// The split for a grid, and the number of workgroups it takes. Measured on
+// 64 experts x 512 rows (160 row tiles; 16 and 28 column blocks): 3.57 ms
+// without, 3.43 in 4 parts; 128 x 256 rows with 6 column blocks 0.62 and
+// 0.56 in 2.
+static int split_of_grid(int m_tiles, int n_blocks) {
+  for (int split = 4; split >= 1; split /= 2) {
+    const int gm = 8 / split;
+    if (ceil_div(n_blocks, split) * split * 10 <= n_blocks * 11)
+      return m_tiles >= 2 * gm * gm ? split : 0;
+  }
+  return 0;
+}
+static int64_t blocks_of_grid(int m_tiles, int n_blocks, int split) {
+  if (split == 0) return ((int64_t)m_tiles * n_blocks + 7) / 8 * 8;
+  const int gm = 8 / split;
+  return (int64_t)ceil_div(ceil_div(m_tiles, gm), gm) * gm *
+         ceil_div(n_blocks, split) * 8;
+}
+
+// --------------------------------------------------------------------------
+// Few rows. A workgroup takes 64 weight rows (32 gate + 32 up rows for
+// gated experts) of an expert and up to 64 token rows; its four waves take
+// a quarter of K each and add up at the end. A wave reads 64 weight rows
+// 128 B at a time straight into A fragments, the next 128 B while it
+// multiplies; token rows are B fragments, from L2. Two workgroups per CU
+// keep 128 KB of weights in flight. At 64 rows the matrix cores are 15 %
+// busy, so rows of padding cost nothing; 16-row groups past the tile's
+// last row are left out.
+constexpr int ST_W = 64;     // weight rows per workgroup
+constexpr int ST_U = 2;      // 32-wide K steps per load
+
+template <typename Tag, int ACT, int STEP, int MT>
+DEVINL void stream_body(const short* const (&wp)[4],
+                        const short* const (&xp)[4], int s0, int s1,
+                        f32x4* red, int wave, int lane, int rows,
+                        short* __restrict__ C, int64_t ldc, int n0, int N) {
   const int l16 = lane & 15;
   const int l4 = lane >> 4;
-  const int wm = wave & 1;   // m 32-half (2 m-frags)
-  const int wn = wave >> 1;  // n 64-half (4 n-frags)
-
-  // Per-lane A row pointers (A-frag: lane&15 = row, k = (lane>>4)*8+j).
-  // Padding rows read row 0 (real data); their C rows are masked at the
-  // epilogue and never mix into valid rows (MFMA rows are independent).
-  const short* a_ptr[2];
-  bool cval[2][4];
+  f32x4 acc[4][MT];
 #pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    const int r = tile_m * BM + wm * 32 + m * 16 + l16;
-    const int sid = sorted[r];
-    const long arow =
-        (sid < total_flat)
-            ? (topk_div > 0 ? (long)(sid / topk_div) : (long)r)
-            : 0;
-    a_ptr[m] = A + arow * lda + l4 * 8;
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const int crow = tile_m * BM + wm * 32 + m * 16 + l4 * 4 + rr;
-      cval[m][rr] = sorted[crow] < total_flat;
+    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  s16x8 wf[ST_U][4], xf[ST_U][MT], wn[ST_U][4], xn[ST_U][MT];
+  auto load = [&](int s, auto& w, auto& x) {
+#pragma unroll
+    for (int u = 0; u < ST_U; ++u) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        w[u][i] = *reinterpret_cast<const s16x8*>(wp[i] + (int64_t)(s + u) * STEP);
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+        x[u][j] = *reinterpret_cast<const s16x8*>(xp[j] + (s + u) * 32);
     }
-  }
-
-  f32x4 acc[2][4];
+  };
+  auto multiply = [&](auto& w, auto& x) {
 #pragma unroll
-  for (int m = 0; m < 2; ++m)
+    for (int u = 0; u < ST_U; ++u)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // B fragment stream for this wave: frags at n-tiles n0/16 + wn*4 + nf,
-  // granule 64 lanes x 8 elems; consecutive k-steps are contiguous 1 KB
-  // lines, so each wave walks 4 linear HBM streams. A re-reads hit the
-  // L3 (the m-tile's rows are shared by all N/128 blocks).
-  const int ksteps = K / 32;
-  const short* bptr[4];
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-  for (int nf = 0; nf < 4; ++nf)
-    bptr[nf] = B + (long)expert * expert_stride +
-               ((long)((n0 >> 4) + wn * 4 + nf) * ksteps) * 512 + lane * 8;
-
-  // No LDS, no barriers: the compiler software-pipelines the 6 loads +
-  // 8 MFMAs per k-step with fine-grained s_waitcnt.
-  for (int ks = 0; ks < ksteps; ++ks) {
-    s16x8 afrag[2];
+        for (int j = 0; j < MT; ++j)
+          acc[i][j] = mfma16<Tag>(w[u][i], x[u][j], acc[i][j]);
+  };
+  int s = s0;
+  if (s + ST_U <= s1) {
+    load(s, wf, xf);
+    for (; s + 2 * ST_U <= s1; s += ST_U) {
+      load(s + ST_U, wn, xn);
+      multiply(wf, xf);
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
-      afrag[m] = *reinterpret_cast<const s16x8*>(a_ptr[m] + ks * 32);
+      for (int u = 0; u < ST_U; ++u) {
 #pragma unroll
-    for (int nf = 0; nf < 4; ++nf) {
-      const s16x8 bfrag =
-          *reinterpret_cast<const s16x8*>(bptr[nf] + (long)ks * 512);
+        for (int i = 0; i < 4; ++i) wf[u][i] = wn[u][i];
 #pragma unroll
-      for (int m = 0; m < 2; ++m)
-        acc[m][nf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            afrag[m], bfrag, acc[m][nf], 0, 0, 0);
-    }
-  }
-
-#pragma unroll
-  for (int m = 0; m < 2; ++m) {
-#pragma unroll
-    for (int nf = 0; nf < 4; ++nf) {
-      const int n = n0 + wn * 64 + nf * 16 + l16;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (cval[m][r])
-          C[(long)(tile_m * BM + wm * 32 + m * 16 + l4 * 4 + r) * ldc + n] =
-              from_f32<Tag>(acc[m][nf][r]);
+        for (int j = 0; j < MT; ++j) xf[u][j] = xn[u][j];
       }
     }
+    multiply(wf, xf);
+    s += ST_U;
+  }
+  for (; s < s1; ++s) {   // an odd step is left
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const s16x8 w =
+          *reinterpret_cast<const s16x8*>(wp[i] + (int64_t)s * STEP);
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+        acc[i][j] = mfma16<Tag>(
+            w, *reinterpret_cast<const s16x8*>(xp[j] + s * 32), acc[i][j]);
+    }
+  }
+
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+      red[((wave * 4 + i) * MT + j) * WAVE_SIZE + lane] = acc[i][j];
+  __syncthreads();
+  auto sum = [&](int i, int j) {
+    f32x4 v = red[(i * MT + j) * WAVE_SIZE + lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w)
+      v += red[((w * 4 + i) * MT + j) * WAVE_SIZE + lane];
+    return v;
+  };
+  // Each wave finishes a share of the 16 x 16 tiles: column l16 is a token
+  // row, the four values are neighbouring columns of the output.
+  constexpr int PARTS = ACT == SILU_GATED ? 2 : 4;
+#pragma unroll
+  for (int u = 0; u < PARTS * MT / 4 + (PARTS * MT % 4 != 0); ++u) {
+    const int unit = u * 4 + wave;
+    if (unit >= PARTS * MT) break;
+    const int p = unit % PARTS;
+    const int j = unit / PARTS;
+    f32x4 v = sum(p, j);
+    if constexpr (ACT == SILU_GATED) {
+      const f32x4 up = sum(p + 2, j);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = silu_mul(v[r], up[r]);
+    } else if constexpr (ACT == RELU2) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = relu2(v[r]);
+    }
+    const int row = j * 16 + l16;
+    const int col = n0 + p * 16 + l4 * 4;
+    if (row < rows && col < N) {
+      int2 o;
+      o.x = pack2<Tag>(v[0], v[1]);
+      o.y = pack2<Tag>(v[2], v[3]);
+      *reinterpret_cast<int2*>(C + (int64_t)row * ldc + col) = o;
+    }
+  }
+}
+
+// Rows of this tile that hold a (token, slot) pair: they come first.
+template <int TM>
+DEVINL int rows_of_tile(const int* __restrict__ sorted, int tile,
+                        int total_flat) {
+  int n = 0;
+#pragma unroll
+  for (int i = 0; i < TM; i += WAVE_SIZE)
+    n += __popcll(__ballot(
+        sorted[tile * TM + i + (threadIdx.x % WAVE_SIZE)] < total_flat));
+  return n;
+}
+
+template <typename Tag, int ACT, bool SHUF>
+__launch_bounds__(THREADS, 2) __global__
+void moe_stream_kernel(const short* __restrict__ A, int64_t lda,
+                       const short* __restrict__ W, int64_t expert_stride,
+                       short* __restrict__ C, int64_t ldc,
+                       const int* __restrict__ sorted,
+                       const int* __restrict__ expert_tiles, int K, int N,
+                       int topk_div, int total_flat, int m_tiles,
+                       int n_blocks, int split) {
+  int tile, blk;
+  if (!tile_of_block(m_tiles, n_blocks, split, tile, blk)) return;
+  const int expert = expert_tiles[tile];
+  if (expert < 0) return;  // padding tile
+  __shared__ __align__(16) f32x4 red[4 * 4 * 4 * WAVE_SIZE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lane = threadIdx.x % WAVE_SIZE;
+  const int l16 = lane & 15;
+  const int l4 = lane >> 4;
+  const int rows = rows_of_tile<BM>(sorted, tile, total_flat);
+  const int n0 = blk * (ACT == SILU_GATED ? ST_W / 2 : ST_W);
+
+  const short* wp[4];
+  const short* we = W + expert * expert_stride;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    // 16 rows, whole ones: N is a multiple of 16 where SHUF.
+    const int r0 = n0 + (ACT == SILU_GATED ? i & 1 : i) * 16;
+    const int up = ACT == SILU_GATED ? (i >> 1) * N : 0;
+    if constexpr (SHUF)
+      wp[i] = we + (int64_t)(min(r0, N - 16) + up) * K + lane * 8;
+    else
+      wp[i] = we + (int64_t)(min(r0 + l16, N - 1) + up) * K + l4 * 8;
+  }
+  const short* xp[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = tile * BM + min(j * 16 + l16, rows - 1);
+    xp[j] = A + (topk_div > 0 ? sorted[r] / topk_div : r) * lda + l4 * 8;
+  }
+  constexpr int STEP = SHUF ? 16 * 32 : 32;   // elements to the next step
+  const int steps = K / 32;
+  const int s0 = steps * wave / 4, s1 = steps * (wave + 1) / 4;
+  short* c = C + (int64_t)tile * BM * ldc;
+  if (rows <= 16)
+    stream_body<Tag, ACT, STEP, 1>(wp, xp, s0, s1, red, wave, lane, rows, c, ldc,
+                             n0, N);
+  else if (rows <= 32)
+    stream_body<Tag, ACT, STEP, 2>(wp, xp, s0, s1, red, wave, lane, rows, c, ldc,
+                             n0, N);
+  else
+    stream_body<Tag, ACT, STEP, 4>(wp, xp, s0, s1, red, wave, lane, rows, c, ldc,
+                             n0, N);
+}
+
+// --------------------------------------------------------------------------
+// Many rows. TM x 256 tiles (128 gate + 128 up weight rows for gated
+// experts) by eight waves, two a SIMD; K goes by 64 (whole 128 B lines: by
+// 32 it was 10 % slower), stages are filled straight from global memory
+// and rotate, one barrier a stage. The product is formed transposed
+// (weight rows are the A operand), so a lane ends up with four
+// neighbouring columns of one row. 32-row groups without a row are left
+// out, by wave, so padding costs fills but few products.
+//   WM 4, 256 rows: waves of 64 x 128, half the traffic from L2 per
+//                   product, two stages. 64 experts x 512 rows (7168,
+//                   2048): 3.43 ms with everything, 1024 rows x 8 experts
+//                   (4096, 14336) 3.2 ms: 900 TFLOP/s.
+//   WM 2, 128 rows: waves of 64 x 64, three stages. Better where an expert
+//                   has fewer than about 190 rows (128 rows: 1.40 against
+//                   1.46 ms), worse above (512 rows: 3.86).
+// (Four waves of 64 x 128 or 128 x 128 left the matrix cores waiting for a
+// single wave per SIMD; three stages of 32 fetch half lines.)
+constexpr int TL_W = 256;
+constexpr int TL_K = 64;
+constexpr int TL_THREADS = 8 * WAVE_SIZE;
+constexpr int TL_ROW = TL_K * 2;                     // bytes of a row
+constexpr int TL_CH = TL_ROW / 16;                   // 16 B chunks of a row
+constexpr int TL_FR = WAVE_SIZE / TL_CH;             // rows a fill moves
+
+// The eight chunks of a row are exchanged by the row / 2, so that the 16
+// rows a fragment read takes the same chunk from lie on all banks.
+DEVINL int tl_swap(int row) { return (row >> 1) & 7; }
+
+template <typename Tag, int ACT, int WM>
+__launch_bounds__(TL_THREADS, 2) __global__
+void moe_tile_kernel(const short* __restrict__ A, int64_t lda,
+                     const short* __restrict__ W, int64_t expert_stride,
+                     short* __restrict__ C, int64_t ldc,
+                     const int* __restrict__ sorted,
+                     const int* __restrict__ expert_tiles, int K, int N,
+                     int topk_div, int total_flat, int m_tiles,
+                     int n_blocks, int split) {
+  constexpr int TL_M = WM * 64;
+  constexpr int TL_STAGES = WM == 4 ? 2 : 3;
+  constexpr int TL_WN = 8 / WM;            // waves along the weight rows
+  constexpr int TL_WW = TL_W / TL_WN;      // weight rows of a wave
+  constexpr int TL_WI = TL_WW / 32;
+  constexpr int TL_MI = 2;                 // 32-row groups of a wave
+  constexpr int TL_STAGE = (TL_M + TL_W) * TL_ROW;   // bytes
+  constexpr int TL_FA = TL_M / TL_FR / 8;  // fills per wave
+  constexpr int TL_FW = TL_W / TL_FR / 8;
+  int tile, blk;
+  if (!tile_of_block(m_tiles, n_blocks, split, tile, blk)) return;
+  const int expert = expert_tiles[tile];
+  if (expert < 0) return;  // padding tile
+  __shared__ __align__(16) char lds[TL_STAGES * TL_STAGE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lane = threadIdx.x % WAVE_SIZE;
+  const int l32 = lane & 31;
+  const int half = lane >> 5;
+  const int wm = wave / TL_WN;   // (a SIMD's two waves take other rows)
+  const int wn = wave % TL_WN;
+  const int rows = rows_of_tile<TL_M>(sorted, tile, total_flat);
+  const int n0 = blk * (ACT == SILU_GATED ? TL_W / 2 : TL_W);
+
+  const int frow = lane / TL_CH;
+  const short* ap[TL_FA];
+#pragma unroll
+  for (int i = 0; i < TL_FA; ++i) {
+    const int lr = (wave * TL_FA + i) * TL_FR + frow;
+    const int r = tile * TL_M + min(lr, rows - 1);
+    ap[i] = A + (topk_div > 0 ? sorted[r] / topk_div : r) * lda +
+            ((lane % TL_CH) ^ tl_swap(lr)) * 8;
+  }
+  const short* wp[TL_FW];
+#pragma unroll
+  for (int i = 0; i < TL_FW; ++i) {
+    const int r = (wave * TL_FW + i) * TL_FR + frow;
+    int64_t src;
+    if constexpr (ACT == SILU_GATED)   // a wave's gate rows, their up rows
+      src = min(n0 + r / TL_WW * (TL_WW / 2) + r % (TL_WW / 2), N - 1) +
+            r / (TL_WW / 2) % 2 * (int64_t)N;
+    else
+      src = min(n0 + r, N - 1);
+    wp[i] = W + expert * expert_stride + src * K +
+            ((lane % TL_CH) ^ tl_swap(r)) * 8;
+  }
+  auto fill = [&](int step, int stage) {
+    char* dst = lds + stage * TL_STAGE;
+#pragma unroll
+    for (int i = 0; i < TL_FA; ++i)
+      lds_fill16(ap[i] + step * TL_K, dst + (wave * TL_FA + i) * 1024);
+    dst += TL_M * TL_ROW;
+#pragma unroll
+    for (int i = 0; i < TL_FW; ++i)
+      lds_fill16(wp[i] + step * TL_K, dst + (wave * TL_FW + i) * 1024);
+  };
+
+  f32x16 acc[TL_WI][TL_MI];
+#pragma unroll
+  for (int i = 0; i < TL_WI; ++i)
+#pragma unroll
+    for (int j = 0; j < TL_MI; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  // 32-row groups of this wave that hold a row at all.
+  const int groups = min(TL_MI, (rows - wm * TL_MI * 32 + 31) / 32);
+  const int steps = K / TL_K;
+  int at[TL_K / 16];   // byte places of this lane's fragments of a row group
+#pragma unroll
+  for (int kk = 0; kk < TL_K / 16; ++kk)
+    at[kk] = l32 * TL_ROW + (((kk * 2 + half) ^ tl_swap(l32)) * 16);
+#pragma unroll
+  for (int i = 0; i < TL_STAGES - 1; ++i)
+    if (i < steps) fill(i, i);
+  int stage = 0;
+  for (int s = 0; s < steps; ++s) {
+    // This stage has landed when at most the next one's fills are under
+    // way; past the barrier every wave is done with the stage before.
+    if (TL_STAGES > 2 && s + 1 < steps) lds_fill_wait<TL_FA + TL_FW>();
+    else lds_fill_wait();
+    lds_barrier();
+    if (s + TL_STAGES - 1 < steps)
+      fill(s + TL_STAGES - 1, stage == 0 ? TL_STAGES - 1 : stage - 1);
+    const char* a = lds + stage * TL_STAGE + wm * TL_MI * 32 * TL_ROW;
+    const char* w = lds + stage * TL_STAGE + TL_M * TL_ROW + wn * TL_WW * TL_ROW;
+    auto multiply = [&](auto n) {
+      constexpr int J = decltype(n)::value;
+#pragma unroll
+      for (int kk = 0; kk < TL_K / 16; ++kk) {
+        s16x8 af[J], wf[TL_WI];
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+          af[j] = *reinterpret_cast<const s16x8*>(a + j * 32 * TL_ROW + at[kk]);
+#pragma unroll
+        for (int i = 0; i < TL_WI; ++i)
+          wf[i] = *reinterpret_cast<const s16x8*>(w + i * 32 * TL_ROW + at[kk]);
+#pragma unroll
+        for (int i = 0; i < TL_WI; ++i)
+#pragma unroll
+          for (int j = 0; j < J; ++j)
+            acc[i][j] = mfma32<Tag>(wf[i], af[j], acc[i][j]);
+      }
+    };
+    if (groups >= 2) multiply(std::integral_constant<int, 2>{});
+    else if (groups == 1) multiply(std::integral_constant<int, 1>{});
+    stage = stage == TL_STAGES - 1 ? 0 : stage + 1;
+  }
+
+  // Register r of acc[i][j]: weight row i*32 + 8*(r/4) + 4*half + r%4,
+  // token row j*32 + l32.
+#pragma unroll
+  for (int j = 0; j < TL_MI; ++j) {
+    const int row = wm * TL_MI * 32 + j * 32 + l32;
+    if (row >= rows) continue;
+    short* c = C + ((int64_t)tile * TL_M + row) * ldc;
+#pragma unroll
+    for (int i = 0; i < (ACT == SILU_GATED ? TL_WI / 2 : TL_WI); ++i)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        f32x4 v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float x = acc[i][j][b * 4 + r];
+          if constexpr (ACT == SILU_GATED)
+            v[r] = silu_mul(x, acc[i + TL_WI / 2][j][b * 4 + r]);
+          else if constexpr (ACT == RELU2)
+            v[r] = relu2(x);
+          else
+            v[r] = x;
+        }
+        const int col = n0 + wn * (ACT == SILU_GATED ? TL_WW / 2 : TL_WW) + i * 32 +
+                        b * 8 + half * 4;
+        if (col < N) {
+          int2 o;
+          o.x = pack2<Tag>(v[0], v[1]);
+          o.y = pack2<Tag>(v[2], v[3]);
+          *reinterpret_cast<int2*>(c + col) = o;
+        }
+      }
   }
 }
 
@@ -360,70 +600,140 @@ __global__ void combine_kernel(short* __restrict__ out,
 
 // Host-side entry points -----------------------------------------------------
 
-void moe_align(torch::Tensor topk_ids, int64_t num_experts,
+// Rows per tile of the forms of the product: 0 streams weights, 1 and 2
+// are the 128- and 256-row tiles.
+int64_t moe_tile_rows(int64_t form) {
+  TORCH_CHECK(form >= 0 && form <= 2);
+  return form == 2 ? 256 : form == 1 ? 128 : moe::BM;
+}
+
+// scratch: ceil(total / 2048) * num_experts ints where total > 2048.
+void moe_align(torch::Tensor topk_ids, int64_t num_experts, int64_t tile_rows,
                torch::Tensor sorted, torch::Tensor expert_tiles,
-               torch::Tensor inv_perm, torch::Tensor counts,
-               torch::Tensor fill, torch::Tensor off) {
+               torch::Tensor inv_perm, torch::Tensor scratch) {
   using namespace moe;
   TORCH_CHECK(topk_ids.scalar_type() == torch::kInt32 &&
               topk_ids.is_contiguous());
   const int total = (int)topk_ids.numel();
   const int e = (int)num_experts;
-  const int em_max = (int)sorted.numel();
+  const int bm = (int)tile_rows;
   const int max_tiles = (int)expert_tiles.numel();
-  TORCH_CHECK(counts.numel() >= e && fill.numel() >= e && off.numel() >= e);
+  TORCH_CHECK(e >= 1 && e <= MAX_EXPERTS, "moe_align: 1..", MAX_EXPERTS,
+              " experts, got ", e);
+  TORCH_CHECK(bm >= 1 && sorted.numel() >= (int64_t)max_tiles * bm &&
+              (int64_t)max_tiles * bm >=
+                  total + (int64_t)std::min(e, total) * (bm - 1) - (bm - 1));
   TORCH_CHECK(inv_perm.numel() >= total);
+  if (total == 0) return;
+  const int blocks = ceil_div(total, ALIGN_ROWS);
   auto stream = c10::hip::getCurrentHIPStream().stream();
   const int* ids = topk_ids.data_ptr<int>();
-  hipLaunchKernelGGL(zero_kernel, dim3(ceil_div(e, 256)), dim3(256), 0,
-                     stream, counts.data_ptr<int>(), fill.data_ptr<int>(), e);
-  hipLaunchKernelGGL(count_kernel, dim3(ceil_div(total, 256)), dim3(256), 0,
-                     stream, ids, total, counts.data_ptr<int>());
-  hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(256), 0, stream,
-                     counts.data_ptr<int>(), e, off.data_ptr<int>(),
-                     expert_tiles.data_ptr<int>(), max_tiles,
-                     sorted.data_ptr<int>(), em_max);
-  hipLaunchKernelGGL(scatter_kernel, dim3(ceil_div(total, 256)), dim3(256),
-                     0, stream, ids, total, off.data_ptr<int>(),
-                     fill.data_ptr<int>(), sorted.data_ptr<int>(),
-                     inv_perm.data_ptr<int>());
+  if (blocks == 1) {
+    hipLaunchKernelGGL(align_small_kernel, dim3(1), dim3(THREADS), 0, stream,
+                       ids, total, e, bm, expert_tiles.data_ptr<int>(),
+                       max_tiles, sorted.data_ptr<int>(),
+                       inv_perm.data_ptr<int>());
+  } else {
+    TORCH_CHECK(scratch.scalar_type() == torch::kInt32 &&
+                scratch.numel() >= (int64_t)blocks * e);
+    int* part = scratch.data_ptr<int>();
+    hipLaunchKernelGGL(align_count_kernel, dim3(blocks), dim3(THREADS), 0,
+                       stream, ids, total, e, part);
+    hipLaunchKernelGGL(align_place_kernel, dim3(1), dim3(THREADS), 0, stream,
+                       part, blocks, e, bm, expert_tiles.data_ptr<int>(),
+                       max_tiles, sorted.data_ptr<int>());
+    hipLaunchKernelGGL(align_scatter_kernel, dim3(blocks), dim3(THREADS), 0,
+                       stream, ids, total, e, part, sorted.data_ptr<int>(),
+                       inv_perm.data_ptr<int>());
+  }
   HIP_CHECK_KERNEL();
 }
 
-void moe_gemm(torch::Tensor a, torch::Tensor b, torch::Tensor c,
-              torch::Tensor sorted, torch::Tensor expert_tiles,
-              int64_t topk_div, int64_t total_flat) {
+static void run_gemm(const torch::Tensor& a, const torch::Tensor& b,
+                     int64_t b_rows, bool shuf, torch::Tensor& c,
+                     const torch::Tensor& sorted,
+                     const torch::Tensor& expert_tiles, int64_t topk_div,
+                     int64_t total_flat, int64_t act, int64_t form) {
   using namespace moe;
-  TORCH_CHECK(a.dim() == 2 && b.dim() == 3 && c.dim() == 2);
+  TORCH_CHECK(a.dim() == 2 && c.dim() == 2);
   TORCH_CHECK(a.is_contiguous() && b.is_contiguous() && c.is_contiguous());
   TORCH_CHECK(a.scalar_type() == b.scalar_type() &&
               a.scalar_type() == c.scalar_type());
   const int K = (int)a.size(1);
-  const int N = (int)b.size(1);
-  TORCH_CHECK(b.size(2) == K, "B inner dim mismatch");
-  TORCH_CHECK(K % BK == 0, "K must be a multiple of ", BK);
-  TORCH_CHECK(N % BN == 0, "N must be a multiple of ", BN);
+  const int N = (int)c.size(1);
+  TORCH_CHECK(act >= NONE && act <= RELU2);
+  TORCH_CHECK(b_rows == (act == SILU_GATED ? 2 : 1) * (int64_t)N);
+  TORCH_CHECK(K % (form > 0 ? TL_K : 32) == 0 && N % (shuf ? 16 : 4) == 0,
+              "K must be a multiple of 32 (64 for tiles), N of 4 (16 in "
+              "fragment order)");
+  const int bm = (int)moe_tile_rows(form);
   const int em = (int)c.size(0);
-  TORCH_CHECK(em % BM == 0 && em / BM <= (int)expert_tiles.numel());
-  TORCH_CHECK(c.size(1) == N);
+  const int m_tiles = em / bm;
+  TORCH_CHECK(em % bm == 0 && m_tiles <= (int)expert_tiles.numel() &&
+              em <= sorted.numel());
+  TORCH_CHECK(topk_div > 0 || a.size(0) >= em);
+  if (em == 0) return;
+  const int cols = (form > 0 ? TL_W : ST_W) / (act == SILU_GATED ? 2 : 1);
+  const int n_blocks = ceil_div(N, cols);
+  const int split = form > 0 ? split_of_grid(m_tiles, n_blocks) : 0;
+  const int64_t blocks = blocks_of_grid(m_tiles, n_blocks, split);
+  TORCH_CHECK(blocks < (1ll << 30));
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  dim3 grid(N / BN, em / BM);
-  auto launch = [&](auto tag) {
+  dim3 grid((unsigned)blocks);
+  auto launch = [&](auto tag, auto act_tag) {
     using Tag = decltype(tag);
-    hipLaunchKernelGGL(
-        (moe_gemm_kernel<Tag>), grid, dim3(THREADS), 0, stream,
-        (const short*)a.data_ptr(), a.size(1), (const short*)b.data_ptr(),
-        b.size(1) * b.size(2), b.size(2), (short*)c.data_ptr(), c.size(1),
-        sorted.data_ptr<int>(), expert_tiles.data_ptr<int>(), K, N,
-        (int)topk_div, (int)total_flat);
+    constexpr int ACT = decltype(act_tag)::value;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(
+          kernel, grid, dim3(form > 0 ? TL_THREADS : THREADS), 0, stream,
+          (const short*)a.data_ptr(),
+          a.size(1), (const short*)b.data_ptr(), b_rows * K,
+          (short*)c.data_ptr(), c.size(1), sorted.data_ptr<int>(),
+          expert_tiles.data_ptr<int>(), K, N, (int)topk_div, (int)total_flat,
+          m_tiles, n_blocks, split);
+    };
+    if (form == 2)      go(moe_tile_kernel<Tag, ACT, 4>);
+    else if (form == 1) go(moe_tile_kernel<Tag, ACT, 2>);
+    else if (shuf)      go(moe_stream_kernel<Tag, ACT, true>);
+    else                go(moe_stream_kernel<Tag, ACT, false>);
+  };
+  auto by_act = [&](auto tag) {
+    if (act == SILU_GATED)
+      launch(tag, std::integral_constant<int, SILU_GATED>{});
+    else if (act == RELU2)
+      launch(tag, std::integral_constant<int, RELU2>{});
+    else
+      launch(tag, std::integral_constant<int, NONE>{});
   };
   if (a.scalar_type() == torch::kBFloat16)
-    launch(BF16Tag{});
+    by_act(BF16Tag{});
   else if (a.scalar_type() == torch::kHalf)
-    launch(FP16Tag{});
+    by_act(FP16Tag{});
   else
     TORCH_CHECK(false, "moe_gemm: bf16/fp16 only");
   HIP_CHECK_KERNEL();
+}
+
+// c [EM, N] = act(a rows x b[expert]^T); b [E, N, K], or [E, 2N, K] for the
+// gated activation. topk_div > 0: a's rows are tokens, gathered through
+// `sorted`; 0: a's rows are in tile order already.
+void moe_gemm(torch::Tensor a, torch::Tensor b, torch::Tensor c,
+              torch::Tensor sorted, torch::Tensor expert_tiles,
+              int64_t topk_div, int64_t total_flat, int64_t act,
+              int64_t form) {
+  TORCH_CHECK(b.dim() == 3 && b.size(2) == a.size(1), "B inner dim mismatch");
+  run_gemm(a, b, b.size(1), false, c, sorted, expert_tiles, topk_div,
+           total_flat, act, form);
+}
+
+// The same with b in fragment order, [E, n * k].
+void moe_gemm_shuf(torch::Tensor a, torch::Tensor b_shuf, torch::Tensor c,
+                   torch::Tensor sorted, torch::Tensor expert_tiles,
+                   int64_t n, int64_t k, int64_t topk_div,
+                   int64_t total_flat, int64_t act) {
+  TORCH_CHECK(a.size(1) == k && b_shuf.numel() % (n * k) == 0);
+  run_gemm(a, b_shuf, n, true, c, sorted, expert_tiles, topk_div, total_flat,
+           act, 0);
 }
 
 void moe_combine(torch::Tensor out, torch::Tensor y,
@@ -455,45 +765,5 @@ void moe_combine(torch::Tensor out, torch::Tensor y,
   HIP_CHECK_KERNEL();
 }
 
-
-void moe_gemm_shuf(torch::Tensor a, torch::Tensor b_shuf, torch::Tensor c,
-                   torch::Tensor sorted, torch::Tensor expert_tiles,
-                   int64_t n, int64_t k, int64_t topk_div,
-                   int64_t total_flat) {
-  using namespace moe;
-  TORCH_CHECK(a.dim() == 2 && c.dim() == 2);
-  TORCH_CHECK(a.is_contiguous() && b_shuf.is_contiguous() &&
-              c.is_contiguous());
-  TORCH_CHECK(a.scalar_type() == b_shuf.scalar_type() &&
-              a.scalar_type() == c.scalar_type());
-  const int K = (int)k;
-  const int N = (int)n;
-  TORCH_CHECK(a.size(1) == K);
-  TORCH_CHECK(K % 64 == 0 && N % BN == 0);
-  const int em = (int)c.size(0);
-  TORCH_CHECK(em % BM == 0 && em / BM <= (int)expert_tiles.numel());
-  TORCH_CHECK(c.size(1) == N);
-  const long expert_stride = (long)(N / 16) * (K / 32) * 512;
-  TORCH_CHECK(b_shuf.numel() % expert_stride == 0);
-  auto stream = c10::hip::getCurrentHIPStream().stream();
-  dim3 grid(N / BN, em / BM);
-  auto launch = [&](auto tag) {
-    using Tag = decltype(tag);
-    hipLaunchKernelGGL(
-        (moe_gemm_shuf_kernel<Tag>), grid, dim3(THREADS), 0, stream,
-        (const short*)a.data_ptr(), a.size(1),
-        (const short*)b_shuf.data_ptr(), expert_stride,
-        (short*)c.data_ptr(), c.size(1), sorted.data_ptr<int>(),
-        expert_tiles.data_ptr<int>(), K, N, (int)topk_div,
-        (int)total_flat);
-  };
-  if (a.scalar_type() == torch::kBFloat16)
-    launch(BF16Tag{});
-  else if (a.scalar_type() == torch::kHalf)
-    launch(FP16Tag{});
-  else
-    TORCH_CHECK(false, "moe_gemm_shuf: bf16/fp16 only");
-  HIP_CHECK_KERNEL();
-}
 
 }  // namespace vllm_amd

@@ -290,13 +290,21 @@ def head_matmul(x, w):
     return _torch_ref.head_matmul(x, w)
 
 
-_MOE_BM = 64  # must match moe::BM in csrc/moe.hip
+# Form of the expert products by the average number of rows an expert
+# gets: below 24 weights are streamed past at most 64 rows (16 rows x 64
+# experts of 7168 x 2048: 1.10 ms against 1.04 in tiles; 2 rows 0.79 / 0.90;
+# 12 rows x 8 experts of 4096 x 14336 0.52 / 0.65), below 192 tiles of 128
+# rows, from there 256.
+_MOE_TILES_FROM = 24
+_MOE_WIDE_TILES_FROM = 192
 
 
 def _moe_hip_ok(hidden, w13, w2, activation):
     if activation not in ("silu", "relu2"):
         return False
     if hidden.dtype not in (torch.bfloat16, torch.float16):
+        return False
+    if w13.shape[0] > 1024:  # moe_align's counters are in LDS
         return False
     H = hidden.shape[1]
     n1 = w13.shape[1]
@@ -311,7 +319,7 @@ def moe_shuffle_weights(w):
     """Pre-shuffle expert weights [E, N, K] into MFMA fragment-major
     order [E][N/16][K/32][64 lanes][8 elems]: each wave's B-fragment
     becomes one coalesced 16B/lane HBM read (csrc/moe.hip
-    moe_gemm_shuf_kernel). One-time cost at weight load."""
+    moe_stream_kernel). One-time cost at weight load."""
     E, N, K = w.shape
     v = w.view(E, N // 16, 16, K // 32, 4, 8)
     v = v.permute(0, 1, 3, 4, 2, 5)
@@ -326,36 +334,41 @@ def fused_moe_hip(hidden, w13, w2, topk_weights, topk_ids,
     (role of the reference's fused_moe.py:299 + moe_align_sum_kernels.cu).
     """
     T, H = hidden.shape
-    E, twoI, _ = w13.shape      # ungated experts: the up width itself
+    E, n1, _ = w13.shape
     I = w2.shape[2]
     k = topk_ids.shape[1]
     total = T * k
     dev = hidden.device
-    em_max = -(-(total + E * (_MOE_BM - 1)) // _MOE_BM) * _MOE_BM
+    shuf = w13_shuf is not None or w2_shuf is not None
+    form = (0 if shuf or total < _MOE_TILES_FROM * E else
+            1 if total < _MOE_WIDE_TILES_FROM * E else 2)
+    bm = _C.moe_tile_rows(form)
+    tiles = (total + min(E, total) * (bm - 1)) // bm
+    em = tiles * bm
     ids32 = topk_ids.to(torch.int32).contiguous()
-    sorted_ids = torch.empty(em_max, dtype=torch.int32, device=dev)
-    expert_tiles = torch.empty(em_max // _MOE_BM, dtype=torch.int32,
-                               device=dev)
-    inv_perm = torch.empty(total, dtype=torch.int32, device=dev)
-    scratch = torch.empty(3 * E, dtype=torch.int32, device=dev)
-    counts, fill, off = scratch[:E], scratch[E:2 * E], scratch[2 * E:]
-    _C.moe_align(ids32, E, sorted_ids, expert_tiles, inv_perm, counts,
-                 fill, off)
-    y = torch.empty(em_max, twoI, dtype=hidden.dtype, device=dev)
+    blocks = -(-total // 2048)
+    scratch = torch.empty(
+        em + tiles + total + (blocks * E if blocks > 1 else 0),
+        dtype=torch.int32, device=dev)
+    sorted_ids, expert_tiles, inv_perm, part = scratch.split(
+        [em, tiles, total, scratch.numel() - em - tiles - total])
+    _C.moe_align(ids32, E, bm, sorted_ids, expert_tiles, inv_perm, part)
+    act_kind = 2 if activation == "relu2" else 1
+    act = torch.empty(em, I, dtype=hidden.dtype, device=dev)
     if w13_shuf is not None:
-        _C.moe_gemm_shuf(hidden, w13_shuf, y, sorted_ids, expert_tiles,
-                         twoI, H, k, total)
+        _C.moe_gemm_shuf(hidden, w13_shuf, act, sorted_ids, expert_tiles,
+                         n1, H, k, total, act_kind)
     else:
-        _C.moe_gemm(hidden, w13, y, sorted_ids, expert_tiles, k, total)
-    act = _C.relu2(y) if activation == "relu2" else silu_and_mul(y)
-    y2 = torch.empty(em_max, H, dtype=hidden.dtype, device=dev)
+        _C.moe_gemm(hidden, w13, act, sorted_ids, expert_tiles, k, total,
+                    act_kind, form)
+    y = torch.empty(em, H, dtype=hidden.dtype, device=dev)
     if w2_shuf is not None:
-        _C.moe_gemm_shuf(act, w2_shuf, y2, sorted_ids, expert_tiles,
-                         H, I, 0, total)
+        _C.moe_gemm_shuf(act, w2_shuf, y, sorted_ids, expert_tiles,
+                         H, I, 0, total, 0)
     else:
-        _C.moe_gemm(act, w2, y2, sorted_ids, expert_tiles, 0, total)
+        _C.moe_gemm(act, w2, y, sorted_ids, expert_tiles, 0, total, 0, form)
     out = torch.empty(T, H, dtype=hidden.dtype, device=dev)
-    _C.moe_combine(out, y2, topk_weights.float().contiguous(), inv_perm)
+    _C.moe_combine(out, y, topk_weights.float().contiguous(), inv_perm)
     return out
 
 
