@@ -649,6 +649,44 @@ def test_moe_forms(T, H, I, E, K, act, dtype):
             <= 1.1 * eps * (bound + expect.abs()) + 2**-20).all()
 
 
+@pytest.mark.parametrize("nd,qls,ctxs,H,bs,at_once", [
+    (0, [130], [130], 3, 64, 3),               # no context before it
+    (2, [1, 1, 200, 57, 131], [70, 300, 200, 311, 131], 10, 16, 4),
+    (0, [1, 300, 128], [1, 300, 128], 16, 64, 16),
+    (1, [1, 129, 255], [5, 640, 257], 2, 80, 1),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_mla_heads(nd, qls, ctxs, H, bs, at_once, dtype, monkeypatch):
+    """Prompt portions with keys and values carried out of the latent
+    space: ragged tiles, contexts before the portion, several passes over
+    the heads. Scores of unit variance are off by at most 4 * 2^-8 (2^-11)
+    through rounded queries and keys, values up to 4 by as much, the
+    result once more; the reference's own roundings double that."""
+    hip = _hip()
+    n, S, T = len(qls), max(ctxs), sum(qls)
+    nb = (S + bs - 1) // bs
+    cache = torch.randn(n * nb, bs, 576, device="cuda", dtype=dtype)
+    bt = torch.randperm(n * nb, device="cuda").to(torch.int32).view(n, nb)
+    q = torch.randn(T, H, 192, device="cuda", dtype=dtype)
+    qn, qp = q[..., :128], q[..., 128:].contiguous()
+    wk = torch.randn(H, 128, 512, device="cuda", dtype=dtype) * 512**-0.5
+    wv = torch.randn(H, 512, 128, device="cuda", dtype=dtype) * 512**-0.5
+    qsl = torch.tensor([sum(qls[:i]) for i in range(n + 1)], device="cuda",
+                       dtype=torch.int32)
+    sl = torch.tensor(ctxs, device="cuda", dtype=torch.int32)
+    monkeypatch.setattr(hip, "_MLA_PROMPT_SCRATCH",
+                        at_once * (n - nd) * S * 512)
+    assert hip._mla_prompt_heads(qn, wk, wv, cache, n, 1.0, nd, max(qls),
+                                 S) == at_once
+    out = hip.mla_heads(qn, qp, wk, wv, cache, bt, qsl, sl, 192**-0.5,
+                        num_decodes=nd, max_query_len=max(qls),
+                        max_seq_len=S)
+    expect = ref.mla_heads(qn.float(), qp.float(), wk.float(), wv.float(),
+                           cache.float(), bt, qsl, sl, 192**-0.5)
+    atol = 2 * 4 * (2**-8 if dtype == torch.bfloat16 else 2**-11)
+    assert_close(out, expect, atol=atol, rtol=atol / 4)
+
+
 def test_mla_unified_dispatch_mixed_batch():
     """ops.mla_attention routes decode rows to the kernel and prefill
     rows to the torch path; both must agree with the all-torch result."""

@@ -25,6 +25,7 @@ SOURCES = [
     CSRC / "comms.hip",
     CSRC / "moe.hip",
     CSRC / "mla.hip",
+    CSRC / "mla_prompt.hip",
     CSRC / "head_matmul.hip",
     CSRC / "quant_fp8.hip",
     CSRC / "attention_decode.hip",
@@ -43,8 +44,8 @@ SOURCES = [
 # These kernels keep matrix-core accumulators in ordinary vector
 # registers: they are rescaled by the vector ALU between products, and
 # through the accumulation registers every rescale is a copy each way.
-VGPR_ACCUMULATORS = {"attention_decode", "attention_prefill", "mla", "head_matmul",
-                     "moe"}
+VGPR_ACCUMULATORS = {"attention_decode", "attention_prefill", "mla",
+                     "mla_prompt", "head_matmul", "moe"}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("PYTORCH_ROCM_ARCH", "gfx950")

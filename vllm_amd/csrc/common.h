@@ -191,6 +191,21 @@ template <> DEVINL int2 fp8x4_widen<FP16Tag>(int v) {
                                       v, 1.0f, true))};
 }
 
+// Column l32 of a 32 x 32 product holds rows 8*b + 4*half + 0..3 in
+// registers 4*b ..; the lower half wave receives all eight rows of b, the
+// upper one those of b + 1: one 16 B store a lane, 32 B in a row (8 B
+// stores: 30 % slower where a kernel is bound by what it writes).
+template <typename Tag> DEVINL i32x4 row_chunk(const f32x16& c, int b) {
+  const unsigned x0 = pack2<Tag>(c[b * 4], c[b * 4 + 1]);
+  const unsigned x1 = pack2<Tag>(c[b * 4 + 2], c[b * 4 + 3]);
+  const unsigned y0 = pack2<Tag>(c[b * 4 + 4], c[b * 4 + 5]);
+  const unsigned y1 = pack2<Tag>(c[b * 4 + 6], c[b * 4 + 7]);
+  const auto s0 = __builtin_amdgcn_permlane32_swap(x0, y0, false, false);
+  const auto s1 = __builtin_amdgcn_permlane32_swap(x1, y1, false, false);
+  const int a0 = s0[0], a1 = s1[0], b0 = s0[1], b1 = s1[1];
+  return i32x4{a0, a1, b0, b1};
+}
+
 // Transposing LDS read: the 16 lanes of a group address a block of 4
 // rows x 16 columns of 16-bit values (lane i: row i / 4, columns
 // (i % 4) * 4 .. + 3) and lane i receives column i, rows 0..3.

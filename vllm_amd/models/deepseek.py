@@ -7,9 +7,10 @@ models/deepseek_v2.py) and mla.py (model_executor/layers/mla.py:36):
 - MLA: per-token KV compressed to kv_lora_rank (512) + rope dim (64) —
   the paged cache stores 576 values/token/layer regardless of head
   count, which is what makes 128-head attention fit 288 GB HBM3E.
-- Decode/prefill run in the ABSORBED space: q_nope is folded through
-  W_UK so attention works directly on the compressed cache; W_UV is
-  applied after (no per-token KV decompression).
+- Decode runs in the ABSORBED space: q_nope is folded through W_UK so
+  attention works directly on the compressed cache; W_UV is applied
+  after (no per-token KV decompression). Prompt portions of many tokens
+  decompress their context instead (ops.mla_heads chooses).
 - MoE: sigmoid scoring, group-limited top-k (n_group/topk_group),
   routed_scaling_factor, plus dense shared experts; leading
   first_dense_layers use a dense MLP.
@@ -119,25 +120,24 @@ class DeepseekMLAAttention(nn.Module):
         k_pe = k_pe.contiguous()
         self.rotary_emb(positions, q_pe, k_pe)
 
-        # Absorb W_UK: q' [T, h, lora].
-        q_absorbed = ops.head_matmul(q_nope, self.w_uk)
-
         ctx = get_forward_context()
         meta = ctx.attn_metadata
         if not ctx.kv_caches:
-            o_c = self._profile_attention(q_absorbed, q_pe, c_kv,
-                                          k_pe.squeeze(1), meta)
+            o_c = self._profile_attention(
+                ops.head_matmul(q_nope, self.w_uk), q_pe, c_kv,
+                k_pe.squeeze(1), meta)
+            out = ops.head_matmul(o_c, self.w_uv)
         else:
             kv_cache = ctx.kv_caches[self.layer_idx]
             ops.concat_and_cache_mla(c_kv, k_pe.squeeze(1), kv_cache,
                                      meta.slot_mapping)
-            o_c = ops.mla_attention(
-                q_absorbed, q_pe, kv_cache, meta.block_table,
-                meta.query_start_loc, meta.seq_lens, self.scale,
-                num_decodes=meta.num_decodes, max_seq_len=meta.max_seq_len,
+            out = ops.mla_heads(
+                q_nope, q_pe, self.w_uk, self.w_uv, kv_cache,
+                meta.block_table, meta.query_start_loc, meta.seq_lens,
+                self.scale, num_decodes=meta.num_decodes,
+                max_query_len=meta.max_query_len,
+                max_seq_len=meta.max_seq_len,
             )
-        # Un-absorb W_UV: [T, h, v].
-        out = ops.head_matmul(o_c, self.w_uv)
         return self.o_proj(out.reshape(T, -1))
 
     def _profile_attention(self, q_absorbed, q_pe, c_kv, k_pe, meta):

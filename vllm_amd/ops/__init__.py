@@ -145,6 +145,22 @@ def mla_attention(q_nope, q_pe, kv_cache, block_table, query_start_loc,
     )
 
 
+def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
+              query_start_loc, seq_lens, scale, num_decodes=0,
+              max_query_len=0, max_seq_len=0):
+    backend = get_backend(q_nope.device)
+    if backend is not _torch_ref:
+        return backend.mla_heads(
+            q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
+            query_start_loc, seq_lens, scale, num_decodes=num_decodes,
+            max_query_len=max_query_len, max_seq_len=max_seq_len,
+        )
+    return backend.mla_heads(
+        q_nope, q_pe, w_uk, w_uv, kv_cache, block_table, query_start_loc,
+        seq_lens, scale
+    )
+
+
 def head_matmul(x, w):
     """x [T, H, K] times a matrix of its own per head, w [H, K, N]:
     [T, H, N], summed in fp32."""

@@ -229,6 +229,16 @@ def concat_and_cache_mla(c_kv, k_pe, kv_cache, slot_mapping):
     kv_cache[blk, off, lora:] = k_pe
 
 
+def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
+              query_start_loc, seq_lens, scale):
+    """MLA attention from per-head queries [T, Hq, nope] to per-head
+    results [T, Hq, v]: queries go through W_UK [Hq, nope, lora], results
+    through W_UV [Hq, lora, v]."""
+    o = mla_attention(head_matmul(q_nope, w_uk), q_pe, kv_cache,
+                      block_table, query_start_loc, seq_lens, scale)
+    return head_matmul(o, w_uv)
+
+
 def mla_attention(
     q_nope,       # [T, Hq, d_nope]  (already absorbed: d_nope == kv_lora)
     q_pe,         # [T, Hq, d_rope]

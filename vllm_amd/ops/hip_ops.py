@@ -290,6 +290,72 @@ def head_matmul(x, w):
     return _torch_ref.head_matmul(x, w)
 
 
+_MLA_PROMPT_SCRATCH = 512 << 20   # bytes
+
+
+def _mla_prompt_heads(q_nope, w_uk, w_uv, kv_cache, reqs, scale,
+                      num_decodes, max_query_len, max_seq_len):
+    """How many heads at a time prompt portions attend with keys and
+    values carried out of the latent space (csrc/mla_prompt.hip); 0:
+    in it (csrc/mla.hip). Carrying them out costs by context row, the
+    latent form by query (0.25 us plus 0.38 per 1000 keys, for 128 heads
+    and no fewer than 256 queries, which fill the chip), so the line is a
+    number of queries per request that grows with the context. 8 requests,
+    us per head / latent: 96 tokens of 512 273 / 317, of 1024 530 / 466;
+    160 of 2048 1218 / 1185, 192 1199 / 1420; 192 of 4096 2532 / 2478. Only
+    the longest context is known here: shorter ones cost less than this
+    says, most so per head."""
+    T, Hq, nope = q_nope.shape
+    rows, reqs = T - num_decodes, reqs - num_decodes
+    S = max(max_seq_len, 128)
+    if (nope != 128 or w_uk.shape[2] != 512 or w_uv.shape[2] != 128
+            or kv_cache.shape[2] != 576 or scale <= 0 or max_query_len <= 0
+            or max_seq_len <= 0 or not 0 < reqs < 65536 or rows <= 0
+            or max(rows, 256) * (800 + S) < reqs * 200 * S
+            or q_nope.dtype not in (torch.bfloat16, torch.float16)
+            or any(t.dtype != q_nope.dtype for t in (w_uk, w_uv, kv_cache))
+            or not all(t.is_contiguous() for t in (w_uk, w_uv, kv_cache))
+            or q_nope.stride(2) != 1 or q_nope.stride(0) % 8
+            or q_nope.stride(1) % 8 or q_nope.data_ptr() % 16):
+        return 0
+    return min(Hq, _MLA_PROMPT_SCRATCH // (reqs * max_seq_len * 512))
+
+
+def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
+              query_start_loc, seq_lens, scale, num_decodes=0,
+              max_query_len=0, max_seq_len=0):
+    """MLA attention from per-head queries to per-head results. Decode
+    rows and short portions work on the latent rows themselves; portions
+    of many tokens carry their context's keys and values out of the latent
+    space first."""
+    T = q_nope.shape[0]
+    reqs = seq_lens.shape[0]
+
+    def latent(n, reqs):
+        o = mla_attention(head_matmul(q_nope[:n], w_uk), q_pe[:n], kv_cache,
+                          block_table[:reqs], query_start_loc[:reqs + 1],
+                          seq_lens[:reqs], scale, num_decodes=num_decodes,
+                          max_seq_len=max_seq_len)
+        return head_matmul(o, w_uv)
+
+    heads = _mla_prompt_heads(q_nope, w_uk, w_uv, kv_cache, reqs, scale,
+                              num_decodes, max_query_len, max_seq_len)
+    if heads == 0:
+        return latent(T, reqs)
+    out = torch.empty(T, q_nope.shape[1], w_uv.shape[2], dtype=q_nope.dtype,
+                      device=q_nope.device)
+    if num_decodes > 0:
+        out[:num_decodes] = latent(num_decodes, num_decodes)
+    rows = (reqs - num_decodes) * max_seq_len
+    scratch = torch.empty(rows * (64 + heads * 256), dtype=q_nope.dtype,
+                          device=q_nope.device)
+    _C.mla_prompt_attention(out, q_nope, q_pe.contiguous(), w_uk, w_uv,
+                            kv_cache, block_table, query_start_loc, seq_lens,
+                            scale, num_decodes, max_query_len, max_seq_len,
+                            scratch)
+    return out
+
+
 # Form of the expert products by the average number of rows an expert
 # gets: below 24 weights are streamed past at most 64 rows (16 rows x 64
 # experts of 7168 x 2048: 1.10 ms against 1.04 in tiles; 2 rows 0.79 / 0.90;
