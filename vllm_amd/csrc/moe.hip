@@ -398,8 +398,9 @@ void moe_stream_kernel(const short* __restrict__ A, int64_t lda,
 // 32 it was 10 % slower), stages are filled straight from global memory
 // and rotate, one barrier a stage. The product is formed transposed
 // (weight rows are the A operand), so a lane ends up with four
-// neighbouring columns of one row. 32-row groups without a row are left
-// out, by wave, so padding costs fills but few products.
+// neighbouring columns of one row, eight after a trade with the other half
+// wave (16 B stores: the second product 5 % faster). 32-row groups without
+// a row are left out, by wave, so padding costs fills but few products.
 //   WM 4, 256 rows: waves of 64 x 128, half the traffic from L2 per
 //                   product, two stages. 64 experts x 512 rows (7168,
 //                   2048): 3.43 ms with everything, 1024 rows x 8 experts
@@ -545,29 +546,23 @@ void moe_tile_kernel(const short* __restrict__ A, int64_t lda,
     if (row >= rows) continue;
     short* c = C + ((int64_t)tile * TL_M + row) * ldc;
 #pragma unroll
-    for (int i = 0; i < (ACT == SILU_GATED ? TL_WI / 2 : TL_WI); ++i)
+    for (int i = 0; i < (ACT == SILU_GATED ? TL_WI / 2 : TL_WI); ++i) {
+      f32x16 v = acc[i][j];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        f32x4 v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float x = acc[i][j][b * 4 + r];
-          if constexpr (ACT == SILU_GATED)
-            v[r] = silu_mul(x, acc[i + TL_WI / 2][j][b * 4 + r]);
-          else if constexpr (ACT == RELU2)
-            v[r] = relu2(x);
-          else
-            v[r] = x;
-        }
-        const int col = n0 + wn * (ACT == SILU_GATED ? TL_WW / 2 : TL_WW) + i * 32 +
-                        b * 8 + half * 4;
-        if (col < N) {
-          int2 o;
-          o.x = pack2<Tag>(v[0], v[1]);
-          o.y = pack2<Tag>(v[2], v[3]);
-          *reinterpret_cast<int2*>(c + col) = o;
-        }
+      for (int r = 0; r < 16; ++r) {
+        if constexpr (ACT == SILU_GATED)
+          v[r] = silu_mul(v[r], acc[i + TL_WI / 2][j][r]);
+        else if constexpr (ACT == RELU2)
+          v[r] = relu2(v[r]);
       }
+#pragma unroll
+      for (int b = 0; b < 4; b += 2) {
+        const i32x4 o = row_chunk<Tag>(v, b);
+        const int col = n0 + wn * (ACT == SILU_GATED ? TL_WW / 2 : TL_WW) +
+                        i * 32 + b * 8 + half * 8;
+        if (col < N) *reinterpret_cast<i32x4*>(c + col) = o;
+      }
+    }
   }
 }
 
@@ -663,9 +658,10 @@ static void run_gemm(const torch::Tensor& a, const torch::Tensor& b,
   const int N = (int)c.size(1);
   TORCH_CHECK(act >= NONE && act <= RELU2);
   TORCH_CHECK(b_rows == (act == SILU_GATED ? 2 : 1) * (int64_t)N);
-  TORCH_CHECK(K % (form > 0 ? TL_K : 32) == 0 && N % (shuf ? 16 : 4) == 0,
-              "K must be a multiple of 32 (64 for tiles), N of 4 (16 in "
-              "fragment order)");
+  TORCH_CHECK(K % (form > 0 ? TL_K : 32) == 0 &&
+                  N % (shuf ? 16 : form > 0 ? 8 : 4) == 0,
+              "K must be a multiple of 32, N of 4 (tiles: 64 and 8; in "
+              "fragment order N of 16)");
   const int bm = (int)moe_tile_rows(form);
   const int em = (int)c.size(0);
   const int m_tiles = em / bm;
