@@ -687,6 +687,33 @@ def test_mla_heads(nd, qls, ctxs, H, bs, at_once, dtype, monkeypatch):
     assert_close(out, expect, atol=atol, rtol=atol / 4)
 
 
+@pytest.mark.parametrize("T,H", [(1, 3), (5, 128), (70, 65)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_mla_prepare(T, H, dtype):
+    """Strided inputs, a padding slot, untouched rows stay. fp32 math of
+    the same 16-bit values: one rounding, or its neighbour."""
+    hip = _hip()
+    q = torch.randn(T, H, 192, device="cuda", dtype=dtype)[..., 128:]
+    kv_a = torch.randn(T, 584, device="cuda", dtype=dtype)[:, :576]
+    w = torch.randn(512, device="cuda", dtype=dtype)
+    cs = torch.randn(100, 64, device="cuda")
+    pos = torch.randint(0, 100, (T,), device="cuda")
+    cache = torch.randn(12, 16, 576, device="cuda", dtype=dtype)
+    want = cache.float()
+    slots = torch.randperm(12 * 16, device="cuda")[:T]
+    pad = torch.cat([slots[:-1], slots.new_tensor([-1])])
+    out = hip.mla_prepare(pos, q, kv_a, w, 1e-5, cs, cache, pad)
+    keep = slice(0, T - 1)
+    ref.mla_prepare(pos[keep], q[keep].float(), kv_a[keep].float(),
+                    w.float(), 1e-5, cs, want, slots[keep])
+    qf = q.float().contiguous()
+    ref.apply_rope(pos, qf, torch.zeros_like(qf), cs, 64)
+    tol = dict(atol=2**-12, rtol=2**-7 if dtype == torch.bfloat16
+               else 2**-10)
+    assert_close(out, qf, **tol)
+    assert_close(cache, want, **tol)
+
+
 def test_mla_unified_dispatch_mixed_batch():
     """ops.mla_attention routes decode rows to the kernel and prefill
     rows to the torch path; both must agree with the all-torch result."""

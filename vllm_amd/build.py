@@ -26,6 +26,7 @@ SOURCES = [
     CSRC / "moe.hip",
     CSRC / "mla.hip",
     CSRC / "mla_prompt.hip",
+    CSRC / "mla_prepare.hip",
     CSRC / "head_matmul.hip",
     CSRC / "quant_fp8.hip",
     CSRC / "attention_decode.hip",

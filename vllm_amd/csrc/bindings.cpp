@@ -56,6 +56,10 @@ void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
                 torch::Tensor kv_cache, torch::Tensor block_table,
                 torch::Tensor seq_lens, double scale, int64_t max_seq_len,
                 torch::Tensor tmp_out, torch::Tensor tmp_lse);
+torch::Tensor mla_prepare(torch::Tensor positions, torch::Tensor q_pe,
+                          torch::Tensor kv_a, torch::Tensor weight,
+                          double eps, torch::Tensor cos_sin,
+                          torch::Tensor kv_cache, torch::Tensor slots);
 void mla_prompt_attention(torch::Tensor out, torch::Tensor q_nope,
                           torch::Tensor q_pe, torch::Tensor w_uk,
                           torch::Tensor w_uv, torch::Tensor kv_cache,
@@ -210,6 +214,10 @@ TORCH_LIBRARY(vllm_amd, m) {
         "float scale, int max_seq_len, Tensor(b!) tmp_out, "
         "Tensor(c!) tmp_lse) -> ()");
   m.def(
+      "mla_prepare(Tensor positions, Tensor q_pe, Tensor kv_a, "
+      "Tensor weight, float eps, Tensor cos_sin, Tensor(a!) kv_cache, "
+      "Tensor slots) -> Tensor");
+  m.def(
       "mla_prompt_attention(Tensor(a!) out, Tensor q_nope, Tensor q_pe, "
       "Tensor w_uk, Tensor w_uv, Tensor kv_cache, Tensor block_table, "
       "Tensor query_start_loc, Tensor seq_lens, float scale, "
@@ -317,6 +325,7 @@ TORCH_LIBRARY_IMPL(vllm_amd, CUDA, m) {
   m.impl("moe_gemm_shuf", &vllm_amd::moe_gemm_shuf);
   m.impl("moe_combine", &vllm_amd::moe_combine);
   m.impl("mla_decode", &vllm_amd::mla_decode);
+  m.impl("mla_prepare", &vllm_amd::mla_prepare);
   m.impl("mla_prompt_attention", &vllm_amd::mla_prompt_attention);
   m.impl("mla_prefill", &vllm_amd::mla_prefill);
   m.impl("head_matmul", &vllm_amd::head_matmul);

@@ -113,24 +113,23 @@ class DeepseekMLAAttention(nn.Module):
         q_nope, q_pe = q[..., : self.qk_nope], q[..., self.qk_nope:]
 
         kv_a = self.kv_a_proj_with_mqa(hidden)
-        c_kv = self.kv_a_layernorm(kv_a[:, : self.kv_lora].contiguous())
-        k_pe = kv_a[:, self.kv_lora:].unsqueeze(1)  # [T, 1, rope]
-
-        q_pe = q_pe.contiguous()
-        k_pe = k_pe.contiguous()
-        self.rotary_emb(positions, q_pe, k_pe)
-
         ctx = get_forward_context()
         meta = ctx.attn_metadata
         if not ctx.kv_caches:
+            c_kv = self.kv_a_layernorm(kv_a[:, : self.kv_lora].contiguous())
+            q_pe = q_pe.contiguous()
+            k_pe = kv_a[:, self.kv_lora:].unsqueeze(1).contiguous()
+            self.rotary_emb(positions, q_pe, k_pe)
             o_c = self._profile_attention(
                 ops.head_matmul(q_nope, self.w_uk), q_pe, c_kv,
                 k_pe.squeeze(1), meta)
             out = ops.head_matmul(o_c, self.w_uv)
         else:
             kv_cache = ctx.kv_caches[self.layer_idx]
-            ops.concat_and_cache_mla(c_kv, k_pe.squeeze(1), kv_cache,
-                                     meta.slot_mapping)
+            q_pe = ops.mla_prepare(
+                positions, q_pe, kv_a, self.kv_a_layernorm.weight,
+                self.kv_a_layernorm.eps, self.rotary_emb.cos_sin_cache,
+                kv_cache, meta.slot_mapping)
             out = ops.mla_heads(
                 q_nope, q_pe, self.w_uk, self.w_uv, kv_cache,
                 meta.block_table, meta.query_start_loc, meta.seq_lens,

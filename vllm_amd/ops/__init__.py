@@ -145,6 +145,13 @@ def mla_attention(q_nope, q_pe, kv_cache, block_table, query_start_loc,
     )
 
 
+def mla_prepare(positions, q_pe, kv_a, weight, eps, cos_sin_cache, kv_cache,
+                slot_mapping):
+    return get_backend(q_pe.device).mla_prepare(
+        positions, q_pe, kv_a, weight, eps, cos_sin_cache, kv_cache,
+        slot_mapping)
+
+
 def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
               query_start_loc, seq_lens, scale, num_decodes=0,
               max_query_len=0, max_seq_len=0):

@@ -229,6 +229,20 @@ def concat_and_cache_mla(c_kv, k_pe, kv_cache, slot_mapping):
     kv_cache[blk, off, lora:] = k_pe
 
 
+def mla_prepare(positions, q_pe, kv_a, weight, eps, cos_sin_cache, kv_cache,
+                slot_mapping):
+    """kv_a [T, lora + rope]: the latent part normalized, the key part
+    rotated, both written to the cache; q_pe [T, Hq, rope] rotated,
+    returned contiguous."""
+    lora = weight.shape[0]
+    c_kv = rms_norm(kv_a[:, :lora].contiguous(), weight, eps)
+    q_pe = q_pe.contiguous()
+    k_pe = kv_a[:, lora:].unsqueeze(1).contiguous()
+    apply_rope(positions, q_pe, k_pe, cos_sin_cache, k_pe.shape[-1])
+    concat_and_cache_mla(c_kv, k_pe.squeeze(1), kv_cache, slot_mapping)
+    return q_pe
+
+
 def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
               query_start_loc, seq_lens, scale):
     """MLA attention from per-head queries [T, Hq, nope] to per-head

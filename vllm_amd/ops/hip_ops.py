@@ -290,6 +290,32 @@ def head_matmul(x, w):
     return _torch_ref.head_matmul(x, w)
 
 
+def mla_prepare(positions, q_pe, kv_a, weight, eps, cos_sin_cache, kv_cache,
+                slot_mapping):
+    """Norm, rotations and cache write of an MLA block's projections in
+    one launch where rows are 16 B aligned and everything has one 16-bit
+    type; else step by step."""
+    aligned = all(
+        x.stride(-1) == 1 and x.data_ptr() % 16 == 0
+        and all(n % 8 == 0 for n in x.stride()[:-1])
+        for x in (q_pe, kv_a, weight))
+    if (aligned and q_pe.shape[2] == 64 and weight.shape[0] == 512
+            and kv_a.shape[1] == 576 and kv_cache.shape[2] == 576
+            and kv_cache.is_contiguous() and cos_sin_cache.shape[-1] == 64
+            and q_pe.dtype in (torch.bfloat16, torch.float16)
+            and all(x.dtype == q_pe.dtype
+                    for x in (kv_a, weight, kv_cache))):
+        return _C.mla_prepare(positions, q_pe, kv_a, weight, eps,
+                              cos_sin_cache, kv_cache, slot_mapping)
+    lora = weight.shape[0]
+    c_kv = rms_norm(kv_a[:, :lora].contiguous(), weight, eps)
+    q_pe = q_pe.contiguous()
+    k_pe = kv_a[:, lora:].unsqueeze(1).contiguous()
+    apply_rope(positions, q_pe, k_pe, cos_sin_cache, k_pe.shape[-1])
+    concat_and_cache_mla(c_kv, k_pe.squeeze(1), kv_cache, slot_mapping)
+    return q_pe
+
+
 _MLA_PROMPT_SCRATCH = 512 << 20   # bytes
 
 
