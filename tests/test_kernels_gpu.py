@@ -714,6 +714,41 @@ def test_mla_prepare(T, H, dtype):
     assert_close(cache, want, **tol)
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D,rot,bs", [
+    (1, 4, 1, 64, 64, 16), (9, 32, 8, 128, 128, 64), (3, 5, 5, 80, 16, 16),
+    (70, 40, 8, 256, 128, 64)])
+@pytest.mark.parametrize("dtype,fp8", [
+    (torch.bfloat16, False), (torch.float16, False), (torch.bfloat16, True)])
+def test_rope_and_cache(T, Hq, Hkv, D, rot, bs, dtype, fp8):
+    """Slices of one projection, partial rotation, a padding slot. The
+    same fp32 math on 16-bit values as rotation and cache write apart:
+    the cached bytes are the same."""
+    hip = _hip()
+    qkv = torch.randn(T, (Hq + 2 * Hkv) * D, device="cuda", dtype=dtype)
+    both = qkv.clone()
+    cs = torch.randn(100, rot, device="cuda")
+    pos = torch.randint(0, 100, (T,), device="cuda")
+    cache = torch.zeros(2, 12, Hkv, bs, D, device="cuda", dtype=dtype)
+    if fp8:
+        cache = cache.to(torch.float8_e4m3fn)
+    want = cache.clone()
+    slots = torch.randperm(12 * bs, device="cuda")[:T]
+    if T > 1:
+        slots[T // 2] = -1
+
+    def split(x):
+        return [y.view(T, -1, D) for y in
+                x.split([Hq * D, Hkv * D, Hkv * D], dim=1)]
+
+    q, k, v = split(qkv)
+    hip.rope_and_cache(pos, q, k, v, cs, rot, True, cache, slots)
+    q2, k2, v2 = split(both)
+    hip.apply_rope(pos, q2, k2, cs, rot)
+    hip.reshape_and_cache(k2, v2, want, slots)
+    assert torch.equal(q, q2)
+    assert torch.equal(cache.view(torch.uint8), want.view(torch.uint8))
+
+
 def test_mla_unified_dispatch_mixed_batch():
     """ops.mla_attention routes decode rows to the kernel and prefill
     rows to the torch path; both must agree with the all-torch result."""

@@ -17,6 +17,10 @@ torch::Tensor gelu_and_mul(torch::Tensor x);
 void rotary_embedding(torch::Tensor positions, torch::Tensor q,
                       torch::Tensor k, torch::Tensor cos_sin_cache,
                       int64_t rot);
+void rope_and_cache(torch::Tensor positions, torch::Tensor q,
+                    torch::Tensor k, torch::Tensor v,
+                    torch::Tensor cos_sin_cache, int64_t rot,
+                    torch::Tensor kv_cache, torch::Tensor slot_mapping);
 void reshape_and_cache(torch::Tensor key, torch::Tensor value,
                        torch::Tensor kv_cache, torch::Tensor slot_mapping);
 void paged_decode_attention(torch::Tensor out, torch::Tensor q,
@@ -182,6 +186,10 @@ TORCH_LIBRARY(vllm_amd, m) {
   m.def("gelu_and_mul(Tensor x) -> Tensor");
   m.def("rotary_embedding(Tensor positions, Tensor(a!) q, Tensor(b!) k, "
         "Tensor cos_sin_cache, int rot) -> ()");
+  m.def(
+      "rope_and_cache(Tensor positions, Tensor(a!) q, Tensor k, Tensor v, "
+      "Tensor cos_sin_cache, int rot, Tensor(b!) kv_cache, "
+      "Tensor slot_mapping) -> ()");
   m.def("reshape_and_cache(Tensor key, Tensor value, Tensor(a!) kv_cache, "
         "Tensor slot_mapping) -> ()");
   m.def("paged_decode_attention(Tensor(a!) out, Tensor q, Tensor kv_cache, "
@@ -310,6 +318,7 @@ TORCH_LIBRARY_IMPL(vllm_amd, CUDA, m) {
   m.impl("silu_and_mul", &vllm_amd::silu_and_mul);
   m.impl("gelu_and_mul", &vllm_amd::gelu_and_mul);
   m.impl("rotary_embedding", &vllm_amd::rotary_embedding);
+  m.impl("rope_and_cache", &vllm_amd::rope_and_cache);
   m.impl("reshape_and_cache", &vllm_amd::reshape_and_cache);
   m.impl("paged_decode_attention", &vllm_amd::paged_decode_attention);
   m.impl("prefill_attention", &vllm_amd::prefill_attention);

@@ -206,6 +206,26 @@ template <typename Tag> DEVINL i32x4 row_chunk(const f32x16& c, int b) {
   return i32x4{a0, a1, b0, b1};
 }
 
+// Rotates 8 pairs (x1[j], x2[j]) by the angles p0 + j of a table row
+// [cos(half) | sin(half)].
+template <typename Tag>
+DEVINL void rope8(s16x8& x1, s16x8& x2, const float* __restrict__ cs,
+                  int half, int p0) {
+  f32x4 c[2], s[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    c[i] = *reinterpret_cast<const f32x4*>(cs + p0 + i * 4);
+    s[i] = *reinterpret_cast<const f32x4*>(cs + half + p0 + i * 4);
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float a = to_f32<Tag>(x1[j]), b = to_f32<Tag>(x2[j]);
+    const float cj = c[j >> 2][j & 3], sj = s[j >> 2][j & 3];
+    x1[j] = from_f32<Tag>(__builtin_fmaf(a, cj, -(b * sj)));
+    x2[j] = from_f32<Tag>(__builtin_fmaf(a, sj, b * cj));
+  }
+}
+
 // Transposing LDS read: the 16 lanes of a group address a block of 4
 // rows x 16 columns of 16-bit values (lane i: row i / 4, columns
 // (i % 4) * 4 .. + 3) and lane i receives column i, rows 0..3.

@@ -26,26 +26,6 @@ constexpr int ROPE = 64;
 constexpr int Q_THREADS = 4 * WAVE_SIZE;
 constexpr int THREADS = Q_THREADS + WAVE_SIZE;
 
-// Rotates 8 pairs (x1[j], x2[j]) by the angles p0 + j of a table row
-// [cos(32) | sin(32)].
-template <typename Tag>
-DEVINL void rotate8(s16x8& x1, s16x8& x2, const float* __restrict__ cs,
-                    int p0) {
-  f32x4 c[2], s[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    c[i] = *reinterpret_cast<const f32x4*>(cs + p0 + i * 4);
-    s[i] = *reinterpret_cast<const f32x4*>(cs + ROPE / 2 + p0 + i * 4);
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const float a = to_f32<Tag>(x1[j]), b = to_f32<Tag>(x2[j]);
-    const float cj = c[j >> 2][j & 3], sj = s[j >> 2][j & 3];
-    x1[j] = from_f32<Tag>(a * cj - b * sj);
-    x2[j] = from_f32<Tag>(b * cj + a * sj);
-  }
-}
-
 template <typename Tag>
 __launch_bounds__(THREADS) __global__
 void mla_prepare_kernel(short* __restrict__ q_out,        // [T, H, ROPE]
@@ -65,7 +45,7 @@ void mla_prepare_kernel(short* __restrict__ q_out,        // [T, H, ROPE]
       const short* src = q + t * q_row + h * q_head + p0;
       s16x8 x1 = *reinterpret_cast<const s16x8*>(src);
       s16x8 x2 = *reinterpret_cast<const s16x8*>(src + ROPE / 2);
-      rotate8<Tag>(x1, x2, cs, p0);
+      rope8<Tag>(x1, x2, cs, ROPE / 2, p0);
       short* dst = q_out + (t * heads + h) * ROPE + p0;
       *reinterpret_cast<s16x8*>(dst) = x1;
       *reinterpret_cast<s16x8*>(dst + ROPE / 2) = x2;
@@ -94,7 +74,7 @@ void mla_prepare_kernel(short* __restrict__ q_out,        // [T, H, ROPE]
     const short* src = row + LORA + lane * 8;
     s16x8 x1 = *reinterpret_cast<const s16x8*>(src);
     s16x8 x2 = *reinterpret_cast<const s16x8*>(src + ROPE / 2);
-    rotate8<Tag>(x1, x2, cs, lane * 8);
+    rope8<Tag>(x1, x2, cs, ROPE / 2, lane * 8);
     *reinterpret_cast<s16x8*>(dst + LORA + lane * 8) = x1;
     *reinterpret_cast<s16x8*>(dst + LORA + ROPE / 2 + lane * 8) = x2;
   }

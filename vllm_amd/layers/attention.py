@@ -38,9 +38,13 @@ class Attention(nn.Module):
         self.kv_group = kv_group
 
     def forward(
-        self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
+        self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+        rotary=None
     ) -> torch.Tensor:
         """q: [T, Hq, D] or [T, Hq*D]; k/v likewise -> [T, Hq*D].
+
+        rotary = (positions, RotaryEmbedding) rotates q and k on the way:
+        q in place, k as it is written to the cache.
 
         Inputs may be strided head-slices of the fused QKV projection —
         the HIP kernels take row strides, so no contiguity copies here.
@@ -59,6 +63,8 @@ class Attention(nn.Module):
             # Memory-profiling run: no cache allocated; compute attention
             # over just the new tokens (worst-case activation footprint is
             # what matters, not values).
+            if rotary is not None:
+                rotary[1](rotary[0], q, k)
             return self._profile_attention(q, k, v, meta).reshape(T, -1)
 
         kv_cache = ctx.kv_caches[self.layer_idx]
@@ -66,7 +72,13 @@ class Attention(nn.Module):
                  and meta.block_table_w is not None)
         slot_mapping = meta.slot_mapping_w if use_w else meta.slot_mapping
         block_table = meta.block_table_w if use_w else meta.block_table
-        ops.reshape_and_cache(k, v, kv_cache, slot_mapping)
+        if rotary is not None:
+            positions, rope = rotary
+            ops.rope_and_cache(positions, q, k, v, rope.cos_sin_cache,
+                               rope.rotary_dim, rope.is_neox, kv_cache,
+                               slot_mapping)
+        else:
+            ops.reshape_and_cache(k, v, kv_cache, slot_mapping)
         out = ops.attention_unified(
             q,
             kv_cache,

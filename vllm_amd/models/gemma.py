@@ -89,8 +89,8 @@ class GemmaAttention(nn.Module):
             q.reshape(-1, self.head_dim).contiguous()).view(q.shape)
         k = self.k_norm(
             k.reshape(-1, self.head_dim).contiguous()).view(k.shape)
-        self.rotary_emb(positions, q, k)
-        return self.o_proj(self.attn(q, k, v))
+        return self.o_proj(
+            self.attn(q, k, v, rotary=(positions, self.rotary_emb)))
 
 
 class GemmaDecoderLayer(nn.Module):

@@ -131,8 +131,7 @@ class LlamaAttention(nn.Module):
                 q.reshape(-1, self.head_dim).contiguous()).view(q.shape)
             k = self.k_norm(
                 k.reshape(-1, self.head_dim).contiguous()).view(k.shape)
-        self.rotary_emb(positions, q, k)
-        out = self.attn(q, k, v)
+        out = self.attn(q, k, v, rotary=(positions, self.rotary_emb))
         return self.o_proj(out, reduce_results=reduce_results)
 
 

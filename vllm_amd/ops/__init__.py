@@ -65,6 +65,14 @@ def apply_rope(positions, q, k, cos_sin_cache, rotary_dim, is_neox=True):
     )
 
 
+def rope_and_cache(positions, q, k, v, cos_sin_cache, rotary_dim, is_neox,
+                   kv_cache, slot_mapping):
+    """Rotates q in place and writes rotated k, and v, to the cache."""
+    return get_backend(q.device).rope_and_cache(
+        positions, q, k, v, cos_sin_cache, rotary_dim, is_neox, kv_cache,
+        slot_mapping)
+
+
 def silu_and_mul(x):
     return get_backend(x.device).silu_and_mul(x)
 

@@ -115,6 +115,25 @@ def reshape_and_cache(key, value, kv_cache, slot_mapping):
     _C.reshape_and_cache(key, value, kv_cache, slot_mapping)
 
 
+def rope_and_cache(positions, q, k, v, cos_sin_cache, rotary_dim, is_neox,
+                   kv_cache, slot_mapping):
+    """One launch where heads split into 16 B pieces (csrc/elementwise.hip
+    rope_cache_kernel), else rotation and cache write."""
+    D = q.shape[2]
+    if (is_neox and rotary_dim % 16 == 0 and D % 16 == 0
+            and 16 <= rotary_dim <= D == v.shape[2]
+            and q.dtype in (torch.bfloat16, torch.float16)
+            and kv_cache.dtype in (q.dtype, torch.float8_e4m3fn)
+            and kv_cache.is_contiguous()
+            and all(x.data_ptr() % 16 == 0 and x.dtype == q.dtype
+                    for x in (q, k, v))):
+        _C.rope_and_cache(positions, q, k, v, cos_sin_cache, rotary_dim,
+                          kv_cache, slot_mapping)
+    else:
+        apply_rope(positions, q, k, cos_sin_cache, rotary_dim, is_neox)
+        reshape_and_cache(k, v, kv_cache, slot_mapping)
+
+
 def attention_unified(
     q,
     kv_cache,
