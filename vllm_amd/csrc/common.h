@@ -250,6 +250,18 @@ DEVINL void lds_fill16(const void* src, void* dst) {
       : "s"(at), "v"(src)
       : "memory", "m0");
 }
+// The same from base + at, base the same in all lanes.
+DEVINL void lds_fill16(const void* base, uint32_t at, void* dst) {
+  const uint32_t to = (uint32_t)(uintptr_t)(
+      __attribute__((address_space(3))) void*)dst;
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2"
+      :
+      : "s"(to), "v"(at), "s"(base)
+      : "memory", "m0");
+}
 // At most N (< 64) of this wave's loads still under way; the builtin, so
 // that the compiler knows its own older loads to be done as well and does
 // not wait again after the next fill.

@@ -78,6 +78,7 @@ DEVINL void place_experts(const int* counts, int* off, int e, int bm,
     for (int k = n; k % bm != 0; ++k) sorted[off[i] + k] = SENTINEL;
   }
   for (int i = total + tid; i < max_tiles; i += THREADS) expert_tiles[i] = -1;
+  if (tid == 0) expert_tiles[max_tiles] = total;
   __syncthreads();
 }
 
@@ -162,52 +163,52 @@ DEVINL float relu2(float x) {
 }
 
 // Which (row tile, column block) a workgroup takes; every eighth workgroup
-// runs on the same XCD. `split` column parts are spread over the XCDs and
-// groups of 8 / split row tiles over the XCDs of a part: what an XCD runs
-// at a time then shares weights (the tiles of an expert) and rows (the
-// blocks of its part) in its L2. split 0: a run of neighbours in (column
-// block, row tile) order per XCD, for grids too small to deal out.
-DEVINL bool tile_of_block(int m_tiles, int n_blocks, int split, int& m,
+// runs on the same XCD. Streamed weights: each XCD takes a run of
+// neighbours in (column block, row tile) order.
+DEVINL bool tile_of_block(int m_tiles, int n_blocks, int& m, int& n) {
+  const int total = m_tiles * n_blocks;
+  const int per = (total + 7) / 8;
+  const int l = (int)blockIdx.x >> 3;
+  const int p = ((int)blockIdx.x & 7) * per + l;
+  if (l >= per || p >= total) return false;
+  m = p % m_tiles;
+  n = p / m_tiles;
+  return true;
+}
+// Tiles: `split` parts of the column blocks times 8 / split parts of the
+// row tiles that hold rows, one part of each per XCD; eight row tiles by
+// some column blocks run there at a time, so tiles of an expert share
+// weights and blocks share rows in its L2.
+DEVINL bool tile_of_block(int tiles, int n_blocks, int split, int& m,
                           int& n) {
+  constexpr int GROUP = 8;
   const int x = (int)blockIdx.x & 7;
   const int l = (int)blockIdx.x >> 3;
-  if (split == 0) {
-    const int total = m_tiles * n_blocks;
-    const int per = (total + 7) / 8;
-    const int p = x * per + l;
-    if (l >= per || p >= total) return false;
-    m = p % m_tiles;
-    n = p / m_tiles;
-    return true;
-  }
-  const int gm = 8 / split;
-  const int nb = (n_blocks + split - 1) / split;
-  const int n_lo = x % split * nb;
-  const int nn = min(nb, n_blocks - n_lo);
-  if (nn <= 0) return false;
-  const int q = l % (gm * nn);
-  m = (l / (gm * nn) * gm + x / split) * gm + q % gm;
-  n = n_lo + q / gm;
-  return m < m_tiles;
+  const int parts = 8 / split, y = x / split, c = x % split;
+  const int m0 = tiles * y / parts, mm = tiles * (y + 1) / parts - m0;
+  const int n_lo = n_blocks * c / split;
+  const int nn = n_blocks * (c + 1) / split - n_lo;
+  if (l >= mm * nn) return false;
+  const int g = l / (GROUP * nn), q = l - g * (GROUP * nn);
+  const int rows = min(GROUP, mm - g * GROUP);
+  m = m0 + g * GROUP + q % rows;
+  n = n_lo + q / rows;
+  return true;
 }
 
-// The split for a grid, and the number of workgroups it takes. Measured on
-// 64 experts x 512 rows (160 row tiles; 16 and 28 column blocks): 3.57 ms
-// without, 3.43 in 4 parts; 128 x 256 rows with 6 column blocks 0.62 and
-// 0.56 in 2.
+// Into how many parts the column blocks go: three or more blocks each and
+// no more than a tenth of unevenness, more only where row tiles are few.
+// Measured in 8 / 4 / 2 / 1 parts, ms: 8 experts, 4096 x 14336 (112 and 16
+// blocks), 96 rows 0.63 / 0.67 / 0.71 / 0.78; 64 experts, 7168 x 2048 (16
+// and 28), 512 rows 3.33 / 3.16 / 3.16 / 3.18; 128 experts, 2048 x 768 (6
+// and 8), 64 rows 0.32 / 0.32 / 0.30 / 0.30.
 static int split_of_grid(int m_tiles, int n_blocks) {
-  for (int split = 4; split >= 1; split /= 2) {
-    const int gm = 8 / split;
-    if (ceil_div(n_blocks, split) * split * 10 <= n_blocks * 11)
-      return m_tiles >= 2 * gm * gm ? split : 0;
-  }
-  return 0;
-}
-static int64_t blocks_of_grid(int m_tiles, int n_blocks, int split) {
-  if (split == 0) return ((int64_t)m_tiles * n_blocks + 7) / 8 * 8;
-  const int gm = 8 / split;
-  return (int64_t)ceil_div(ceil_div(m_tiles, gm), gm) * gm *
-         ceil_div(n_blocks, split) * 8;
+  int split = 8;
+  while (split > 1 && (n_blocks < 3 * split ||
+                       ceil_div(n_blocks, split) * split * 10 > n_blocks * 11))
+    split /= 2;
+  while (split < 8 && m_tiles < 2 * (8 / split)) split *= 2;
+  return split;
 }
 
 // --------------------------------------------------------------------------
@@ -240,7 +241,8 @@ DEVINL void stream_body(const short* const (&wp)[4],
     for (int u = 0; u < ST_U; ++u) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        w[u][i] = *reinterpret_cast<const s16x8*>(wp[i] + (int64_t)(s + u) * STEP);
+        w[u][i] =
+            *reinterpret_cast<const s16x8*>(wp[i] + (int64_t)(s + u) * STEP);
 #pragma unroll
       for (int j = 0; j < MT; ++j)
         x[u][j] = *reinterpret_cast<const s16x8*>(xp[j] + (s + u) * 32);
@@ -348,7 +350,7 @@ void moe_stream_kernel(const short* __restrict__ A, int64_t lda,
                        int topk_div, int total_flat, int m_tiles,
                        int n_blocks, int split) {
   int tile, blk;
-  if (!tile_of_block(m_tiles, n_blocks, split, tile, blk)) return;
+  if (!tile_of_block(m_tiles, n_blocks, tile, blk)) return;
   const int expert = expert_tiles[tile];
   if (expert < 0) return;  // padding tile
   __shared__ __align__(16) f32x4 red[4 * 4 * 4 * WAVE_SIZE];
@@ -382,14 +384,14 @@ void moe_stream_kernel(const short* __restrict__ A, int64_t lda,
   const int s0 = steps * wave / 4, s1 = steps * (wave + 1) / 4;
   short* c = C + (int64_t)tile * BM * ldc;
   if (rows <= 16)
-    stream_body<Tag, ACT, STEP, 1>(wp, xp, s0, s1, red, wave, lane, rows, c, ldc,
-                             n0, N);
+    stream_body<Tag, ACT, STEP, 1>(wp, xp, s0, s1, red, wave, lane, rows, c,
+                                   ldc, n0, N);
   else if (rows <= 32)
-    stream_body<Tag, ACT, STEP, 2>(wp, xp, s0, s1, red, wave, lane, rows, c, ldc,
-                             n0, N);
+    stream_body<Tag, ACT, STEP, 2>(wp, xp, s0, s1, red, wave, lane, rows, c,
+                                   ldc, n0, N);
   else
-    stream_body<Tag, ACT, STEP, 4>(wp, xp, s0, s1, red, wave, lane, rows, c, ldc,
-                             n0, N);
+    stream_body<Tag, ACT, STEP, 4>(wp, xp, s0, s1, red, wave, lane, rows, c,
+                                   ldc, n0, N);
 }
 
 // --------------------------------------------------------------------------
@@ -402,17 +404,21 @@ void moe_stream_kernel(const short* __restrict__ A, int64_t lda,
 // wave (16 B stores: the second product 5 % faster). 32-row groups without
 // a row are left out, by wave, so padding costs fills but few products.
 //   WM 4, 256 rows: waves of 64 x 128, half the traffic from L2 per
-//                   product, two stages. 64 experts x 512 rows (7168,
-//                   2048): 3.43 ms with everything, 1024 rows x 8 experts
-//                   (4096, 14336) 3.2 ms: 900 TFLOP/s.
-//   WM 2, 128 rows: waves of 64 x 64, three stages. Better where an expert
-//                   has fewer than about 190 rows (128 rows: 1.40 against
-//                   1.46 ms), worse above (512 rows: 3.86).
+//                   product, two stages, reads and products of the two
+//                   halves of the workgroup in turn (all waves in step:
+//                   3.41 ms for 64 experts x 512 rows of 7168 x 2048, 3.16
+//                   now; 8 experts x 1024 rows of 4096 x 14336 3.18 and
+//                   2.87: 1000 TFLOP/s). Products alone would take 2.5 ms,
+//                   fills alone 2.9: weights that miss L2 bound it.
+//   WM 2, 128 rows: waves of 64 x 64, three stages. For experts of few
+//                   rows, and for what is left of an expert's rows after
+//                   whole tiles of 256.
 // (Four waves of 64 x 128 or 128 x 128 left the matrix cores waiting for a
-// single wave per SIMD; three stages of 32 fetch half lines.)
+// single wave per SIMD; five stages of 32 fetch half lines: 2 % slower.)
 constexpr int TL_W = 256;
 constexpr int TL_K = 64;
 constexpr int TL_THREADS = 8 * WAVE_SIZE;
+constexpr int TL_LDS = 144 * 1024;                   // bytes of the stages
 constexpr int TL_ROW = TL_K * 2;                     // bytes of a row
 constexpr int TL_CH = TL_ROW / 16;                   // 16 B chunks of a row
 constexpr int TL_FR = WAVE_SIZE / TL_CH;             // rows a fill moves
@@ -421,15 +427,13 @@ constexpr int TL_FR = WAVE_SIZE / TL_CH;             // rows a fill moves
 // rows a fragment read takes the same chunk from lie on all banks.
 DEVINL int tl_swap(int row) { return (row >> 1) & 7; }
 
+// One tile by waves of (8 / WM columns of) WM rows of 64; `row0` is its
+// first row in tile order.
 template <typename Tag, int ACT, int WM>
-__launch_bounds__(TL_THREADS, 2) __global__
-void moe_tile_kernel(const short* __restrict__ A, int64_t lda,
-                     const short* __restrict__ W, int64_t expert_stride,
-                     short* __restrict__ C, int64_t ldc,
-                     const int* __restrict__ sorted,
-                     const int* __restrict__ expert_tiles, int K, int N,
-                     int topk_div, int total_flat, int m_tiles,
-                     int n_blocks, int split) {
+DEVINL void tile_body(char* lds, const short* __restrict__ A, int64_t lda,
+                      const short* __restrict__ W, short* __restrict__ C,
+                      int64_t ldc, const int* __restrict__ sorted, int K,
+                      int N, int topk_div, int row0, int rows, int n0) {
   constexpr int TL_M = WM * 64;
   constexpr int TL_STAGES = WM == 4 ? 2 : 3;
   constexpr int TL_WN = 8 / WM;            // waves along the weight rows
@@ -437,53 +441,46 @@ void moe_tile_kernel(const short* __restrict__ A, int64_t lda,
   constexpr int TL_WI = TL_WW / 32;
   constexpr int TL_MI = 2;                 // 32-row groups of a wave
   constexpr int TL_STAGE = (TL_M + TL_W) * TL_ROW;   // bytes
+  static_assert(TL_STAGES * TL_STAGE <= TL_LDS);
   constexpr int TL_FA = TL_M / TL_FR / 8;  // fills per wave
   constexpr int TL_FW = TL_W / TL_FR / 8;
-  int tile, blk;
-  if (!tile_of_block(m_tiles, n_blocks, split, tile, blk)) return;
-  const int expert = expert_tiles[tile];
-  if (expert < 0) return;  // padding tile
-  __shared__ __align__(16) char lds[TL_STAGES * TL_STAGE];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
   const int l32 = lane & 31;
   const int half = lane >> 5;
   const int wm = wave / TL_WN;   // (a SIMD's two waves take other rows)
   const int wn = wave % TL_WN;
-  const int rows = rows_of_tile<TL_M>(sorted, tile, total_flat);
-  const int n0 = blk * (ACT == SILU_GATED ? TL_W / 2 : TL_W);
 
   const int frow = lane / TL_CH;
-  const short* ap[TL_FA];
+  uint32_t ap[TL_FA], wp[TL_FW];   // byte places in A and W
 #pragma unroll
   for (int i = 0; i < TL_FA; ++i) {
     const int lr = (wave * TL_FA + i) * TL_FR + frow;
-    const int r = tile * TL_M + min(lr, rows - 1);
-    ap[i] = A + (topk_div > 0 ? sorted[r] / topk_div : r) * lda +
-            ((lane % TL_CH) ^ tl_swap(lr)) * 8;
+    const int r = row0 + min(lr, rows - 1);
+    ap[i] = (uint32_t)(topk_div > 0 ? sorted[r] / topk_div : r) *
+                (uint32_t)lda * 2 +
+            ((lane % TL_CH) ^ tl_swap(lr)) * 16;
   }
-  const short* wp[TL_FW];
 #pragma unroll
   for (int i = 0; i < TL_FW; ++i) {
     const int r = (wave * TL_FW + i) * TL_FR + frow;
-    int64_t src;
+    uint32_t src;
     if constexpr (ACT == SILU_GATED)   // a wave's gate rows, their up rows
       src = min(n0 + r / TL_WW * (TL_WW / 2) + r % (TL_WW / 2), N - 1) +
-            r / (TL_WW / 2) % 2 * (int64_t)N;
+            r / (TL_WW / 2) % 2 * N;
     else
       src = min(n0 + r, N - 1);
-    wp[i] = W + expert * expert_stride + src * K +
-            ((lane % TL_CH) ^ tl_swap(r)) * 8;
+    wp[i] = src * (uint32_t)K * 2 + ((lane % TL_CH) ^ tl_swap(r)) * 16;
   }
   auto fill = [&](int step, int stage) {
     char* dst = lds + stage * TL_STAGE;
 #pragma unroll
     for (int i = 0; i < TL_FA; ++i)
-      lds_fill16(ap[i] + step * TL_K, dst + (wave * TL_FA + i) * 1024);
+      lds_fill16(A + step * TL_K, ap[i], dst + (wave * TL_FA + i) * 1024);
     dst += TL_M * TL_ROW;
 #pragma unroll
     for (int i = 0; i < TL_FW; ++i)
-      lds_fill16(wp[i] + step * TL_K, dst + (wave * TL_FW + i) * 1024);
+      lds_fill16(W + step * TL_K, wp[i], dst + (wave * TL_FW + i) * 1024);
   };
 
   f32x16 acc[TL_WI][TL_MI];
@@ -501,41 +498,112 @@ void moe_tile_kernel(const short* __restrict__ A, int64_t lda,
 #pragma unroll
   for (int kk = 0; kk < TL_K / 16; ++kk)
     at[kk] = l32 * TL_ROW + (((kk * 2 + half) ^ tl_swap(l32)) * 16);
-#pragma unroll
-  for (int i = 0; i < TL_STAGES - 1; ++i)
-    if (i < steps) fill(i, i);
-  int stage = 0;
-  for (int s = 0; s < steps; ++s) {
-    // This stage has landed when at most the next one's fills are under
-    // way; past the barrier every wave is done with the stage before.
-    if (TL_STAGES > 2 && s + 1 < steps) lds_fill_wait<TL_FA + TL_FW>();
-    else lds_fill_wait();
-    lds_barrier();
-    if (s + TL_STAGES - 1 < steps)
-      fill(s + TL_STAGES - 1, stage == 0 ? TL_STAGES - 1 : stage - 1);
-    const char* a = lds + stage * TL_STAGE + wm * TL_MI * 32 * TL_ROW;
-    const char* w = lds + stage * TL_STAGE + TL_M * TL_ROW + wn * TL_WW * TL_ROW;
-    auto multiply = [&](auto n) {
+  if constexpr (WM == 4) {
+    // Waves 4..7 run one slot behind waves 0..3, their neighbours on the
+    // SIMDs: one half multiplies 32 of K while the other reads the next 32
+    // into fragments, a barrier a slot, four slots a stage. The next stage
+    // is filled from the first slot on (the laggards read its place last
+    // in the slot before) and has landed for all when the fourth ends.
+    // The number of row groups is a constant of the loop: merging
+    // accumulators of several branches would copy them.
+    const int lag = wave >> 2;
+    const char* a0 = lds + wm * TL_MI * 32 * TL_ROW;
+    const char* w0 = lds + TL_M * TL_ROW + wn * TL_WW * TL_ROW;
+    auto run = [&](auto n) {
       constexpr int J = decltype(n)::value;
+      s16x8 af[2][J > 0 ? J : 1], wf[2][TL_WI];
+      auto read = [&](int stage, int k0) {
+        if constexpr (J > 0) {
 #pragma unroll
-      for (int kk = 0; kk < TL_K / 16; ++kk) {
-        s16x8 af[J], wf[TL_WI];
+          for (int k = 0; k < 2; ++k) {
 #pragma unroll
-        for (int j = 0; j < J; ++j)
-          af[j] = *reinterpret_cast<const s16x8*>(a + j * 32 * TL_ROW + at[kk]);
+            for (int j = 0; j < J; ++j)
+              af[k][j] = *reinterpret_cast<const s16x8*>(
+                  a0 + stage * TL_STAGE + j * 32 * TL_ROW + at[k0 + k]);
 #pragma unroll
-        for (int i = 0; i < TL_WI; ++i)
-          wf[i] = *reinterpret_cast<const s16x8*>(w + i * 32 * TL_ROW + at[kk]);
+            for (int i = 0; i < TL_WI; ++i)
+              wf[k][i] = *reinterpret_cast<const s16x8*>(
+                  w0 + stage * TL_STAGE + i * 32 * TL_ROW + at[k0 + k]);
+          }
+        }
+      };
+      auto multiply = [&]() {
+        if constexpr (J > 0) {
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < TL_WI; ++i)
+          for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int i = 0; i < TL_WI; ++i)
+#pragma unroll
+              for (int j = 0; j < J; ++j)
+                acc[i][j] = mfma32<Tag>(wf[k][i], af[k][j], acc[i][j]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      if (lag) lds_barrier();   // (as many barriers for every wave)
+#pragma unroll 1
+      for (int s = 0; s < steps; ++s) {
+        const int stage = s & 1;
+        if (s + 1 < steps) fill(s + 1, stage ^ 1);
+        read(stage, 0);
+        lds_barrier();
+        multiply();
+        lds_barrier();
+        read(stage, 2);
+        if (lag) lds_fill_wait();
+        lds_barrier();
+        multiply();
+        if (!lag) lds_fill_wait();
+        lds_barrier();
+      }
+      if (!lag) lds_barrier();
+    };
+    fill(0, 0);
+    lds_fill_wait();
+    lds_barrier();
+    if (groups >= 2) run(std::integral_constant<int, 2>{});
+    else if (groups == 1) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 0>{});
+  } else {
+#pragma unroll
+    for (int i = 0; i < TL_STAGES - 1; ++i)
+      if (i < steps) fill(i, i);
+    int stage = 0;
+    for (int s = 0; s < steps; ++s) {
+      // This stage has landed when at most the next one's fills are under
+      // way; past the barrier every wave is done with the stage before.
+      if (TL_STAGES > 2 && s + 1 < steps) lds_fill_wait<TL_FA + TL_FW>();
+      else lds_fill_wait();
+      lds_barrier();
+      if (s + TL_STAGES - 1 < steps)
+        fill(s + TL_STAGES - 1, stage == 0 ? TL_STAGES - 1 : stage - 1);
+      const char* a = lds + stage * TL_STAGE + wm * TL_MI * 32 * TL_ROW;
+      const char* w =
+          lds + stage * TL_STAGE + (TL_M + wn * TL_WW) * TL_ROW;
+      auto multiply = [&](auto n) {
+        constexpr int J = decltype(n)::value;
+#pragma unroll
+        for (int kk = 0; kk < TL_K / 16; ++kk) {
+          s16x8 af[J], wf[TL_WI];
 #pragma unroll
           for (int j = 0; j < J; ++j)
-            acc[i][j] = mfma32<Tag>(wf[i], af[j], acc[i][j]);
-      }
-    };
-    if (groups >= 2) multiply(std::integral_constant<int, 2>{});
-    else if (groups == 1) multiply(std::integral_constant<int, 1>{});
-    stage = stage == TL_STAGES - 1 ? 0 : stage + 1;
+            af[j] =
+                *reinterpret_cast<const s16x8*>(a + j * 32 * TL_ROW + at[kk]);
+#pragma unroll
+          for (int i = 0; i < TL_WI; ++i)
+            wf[i] =
+                *reinterpret_cast<const s16x8*>(w + i * 32 * TL_ROW + at[kk]);
+#pragma unroll
+          for (int i = 0; i < TL_WI; ++i)
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+              acc[i][j] = mfma32<Tag>(wf[i], af[j], acc[i][j]);
+        }
+      };
+      if (groups >= 2) multiply(std::integral_constant<int, 2>{});
+      else if (groups == 1) multiply(std::integral_constant<int, 1>{});
+      stage = stage == TL_STAGES - 1 ? 0 : stage + 1;
+    }
   }
 
   // Register r of acc[i][j]: weight row i*32 + 8*(r/4) + 4*half + r%4,
@@ -544,7 +612,7 @@ void moe_tile_kernel(const short* __restrict__ A, int64_t lda,
   for (int j = 0; j < TL_MI; ++j) {
     const int row = wm * TL_MI * 32 + j * 32 + l32;
     if (row >= rows) continue;
-    short* c = C + ((int64_t)tile * TL_M + row) * ldc;
+    short* c = C + (int64_t)(row0 + row) * ldc;
 #pragma unroll
     for (int i = 0; i < (ACT == SILU_GATED ? TL_WI / 2 : TL_WI); ++i) {
       f32x16 v = acc[i][j];
@@ -564,6 +632,31 @@ void moe_tile_kernel(const short* __restrict__ A, int64_t lda,
       }
     }
   }
+}
+
+template <typename Tag, int ACT, int TM>
+__launch_bounds__(TL_THREADS, 2) __global__
+void moe_tile_kernel(const short* __restrict__ A, int64_t lda,
+                     const short* __restrict__ W, int64_t expert_stride,
+                     short* __restrict__ C, int64_t ldc,
+                     const int* __restrict__ sorted,
+                     const int* __restrict__ expert_tiles, int K, int N,
+                     int topk_div, int total_flat, int m_tiles,
+                     int n_blocks, int split) {
+  int tile, blk;
+  if (!tile_of_block(expert_tiles[m_tiles], n_blocks, split, tile, blk))
+    return;
+  const int expert = expert_tiles[tile];
+  __shared__ __align__(16) char lds[TL_LDS];
+  const int rows = rows_of_tile<TM>(sorted, tile, total_flat);
+  const int n0 = blk * (ACT == SILU_GATED ? TL_W / 2 : TL_W);
+  W += expert * expert_stride;
+  if (TM == 128 || rows <= 128)
+    tile_body<Tag, ACT, 2>(lds, A, lda, W, C, ldc, sorted, K, N, topk_div,
+                           tile * TM, rows, n0);
+  else
+    tile_body<Tag, ACT, 4>(lds, A, lda, W, C, ldc, sorted, K, N, topk_div,
+                           tile * TM, rows, n0);
 }
 
 // --------------------------------------------------------------------------
@@ -612,7 +705,7 @@ void moe_align(torch::Tensor topk_ids, int64_t num_experts, int64_t tile_rows,
   const int total = (int)topk_ids.numel();
   const int e = (int)num_experts;
   const int bm = (int)tile_rows;
-  const int max_tiles = (int)expert_tiles.numel();
+  const int max_tiles = (int)expert_tiles.numel() - 1;
   TORCH_CHECK(e >= 1 && e <= MAX_EXPERTS, "moe_align: 1..", MAX_EXPERTS,
               " experts, got ", e);
   TORCH_CHECK(bm >= 1 && sorted.numel() >= (int64_t)max_tiles * bm &&
@@ -665,14 +758,20 @@ static void run_gemm(const torch::Tensor& a, const torch::Tensor& b,
   const int bm = (int)moe_tile_rows(form);
   const int em = (int)c.size(0);
   const int m_tiles = em / bm;
-  TORCH_CHECK(em % bm == 0 && m_tiles <= (int)expert_tiles.numel() &&
+  TORCH_CHECK(em % bm == 0 && m_tiles == (int)expert_tiles.numel() - 1 &&
               em <= sorted.numel());
   TORCH_CHECK(topk_div > 0 || a.size(0) >= em);
   if (em == 0) return;
   const int cols = (form > 0 ? TL_W : ST_W) / (act == SILU_GATED ? 2 : 1);
   const int n_blocks = ceil_div(N, cols);
-  const int split = form > 0 ? split_of_grid(m_tiles, n_blocks) : 0;
-  const int64_t blocks = blocks_of_grid(m_tiles, n_blocks, split);
+  const int split = split_of_grid(m_tiles, n_blocks);
+  const int64_t blocks =
+      form > 0 ? (int64_t)ceil_div(m_tiles, 8 / split) *
+                     ceil_div(n_blocks, split) * 8
+               : ((int64_t)m_tiles * n_blocks + 7) / 8 * 8;
+  // (Tiles address rows and an expert's weights with 32 bits.)
+  TORCH_CHECK(form == 0 || (a.numel() * 2 < (1ll << 32) &&
+                            b_rows * K * 2 < (1ll << 32)));
   TORCH_CHECK(blocks < (1ll << 30));
   auto stream = c10::hip::getCurrentHIPStream().stream();
   dim3 grid((unsigned)blocks);
@@ -688,8 +787,8 @@ static void run_gemm(const torch::Tensor& a, const torch::Tensor& b,
           expert_tiles.data_ptr<int>(), K, N, (int)topk_div, (int)total_flat,
           m_tiles, n_blocks, split);
     };
-    if (form == 2)      go(moe_tile_kernel<Tag, ACT, 4>);
-    else if (form == 1) go(moe_tile_kernel<Tag, ACT, 2>);
+    if (form == 2)      go(moe_tile_kernel<Tag, ACT, 256>);
+    else if (form == 1) go(moe_tile_kernel<Tag, ACT, 128>);
     else if (shuf)      go(moe_stream_kernel<Tag, ACT, true>);
     else                go(moe_stream_kernel<Tag, ACT, false>);
   };

@@ -402,10 +402,12 @@ def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
 
 
 # Form of the expert products by the average number of rows an expert
-# gets: below 24 weights are streamed past at most 64 rows (16 rows x 64
-# experts of 7168 x 2048: 1.10 ms against 1.04 in tiles; 2 rows 0.79 / 0.90;
-# 12 rows x 8 experts of 4096 x 14336 0.52 / 0.65), below 192 tiles of 128
-# rows, from there 256.
+# gets: below 24 weights are streamed past at most 64 rows, below 192 tiles
+# of 128 rows, from there 256. ms streamed / 128 / 256: 8 experts of 4096 x
+# 14336, 12 rows 0.54 / 0.57 / 0.59, 32 rows 0.74 / 0.61 / 0.62, 128 rows
+# 1.49 / 0.69 / 0.86, 256 rows 2.74 / 1.14 / 0.99; 64 experts of 7168 x
+# 2048, 16 rows 1.11 / 1.00 / 1.00, 64 rows 1.89 / 1.17 / 1.17, 192 rows
+# 4.21 / 1.79 / 1.79, 512 rows 10.2 / 3.70 / 3.20.
 _MOE_TILES_FROM = 24
 _MOE_WIDE_TILES_FROM = 192
 
@@ -453,16 +455,18 @@ def fused_moe_hip(hidden, w13, w2, topk_weights, topk_ids,
     shuf = w13_shuf is not None or w2_shuf is not None
     form = (0 if shuf or total < _MOE_TILES_FROM * E else
             1 if total < _MOE_WIDE_TILES_FROM * E else 2)
+    if max(T * H, (total + E * 256) * I, n1 * H) >= 1 << 31:
+        form = 0    # tiles address 4 GB
     bm = _C.moe_tile_rows(form)
     tiles = (total + min(E, total) * (bm - 1)) // bm
     em = tiles * bm
     ids32 = topk_ids.to(torch.int32).contiguous()
     blocks = -(-total // 2048)
     scratch = torch.empty(
-        em + tiles + total + (blocks * E if blocks > 1 else 0),
+        em + tiles + 1 + total + (blocks * E if blocks > 1 else 0),
         dtype=torch.int32, device=dev)
     sorted_ids, expert_tiles, inv_perm, part = scratch.split(
-        [em, tiles, total, scratch.numel() - em - tiles - total])
+        [em, tiles + 1, total, scratch.numel() - em - tiles - 1 - total])
     _C.moe_align(ids32, E, bm, sorted_ids, expert_tiles, inv_perm, part)
     act_kind = 2 if activation == "relu2" else 1
     act = torch.empty(em, I, dtype=hidden.dtype, device=dev)
