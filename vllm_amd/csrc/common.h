@@ -234,6 +234,20 @@ DEVINL s16x4 lds_read_tr(const void* p) {
       (__attribute__((address_space(3))) s16x4*)p);
 }
 
+// Order for the scheduler, said after STEPS steps of LDS reads and MFMAS
+// products each: AHEAD reads come first, then PER further ones after each
+// step. By itself it tends to wait for every read just before its product
+// where registers are short.
+template <int AHEAD, int PER, int STEPS, int MFMAS = 1>
+DEVINL void reads_ahead() {
+  __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, MFMAS, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, PER, 0);
+  }
+}
+
 // 64 lanes x 16 B from global memory straight into LDS: lane i's 16 bytes
 // land at dst + 16 * i (dst the same in all lanes). No register receives
 // anything, so the kernel waits itself (lds_fill_wait, then a barrier for

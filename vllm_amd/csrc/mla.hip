@@ -22,6 +22,10 @@
 //     are plain 16 B reads, V^T fragments transposing reads of the same
 //     rows. 16 B chunks of a row are exchanged so that neither kind of
 //     read meets a bank twice.
+//   - Reads run four and more products ahead of their use, in an order the
+//     scheduler is told: left alone it waits for each read just before its
+//     product (115 -> 90 us for the decode rows below, 1.60 -> 1.32 ms for
+//     the prompts).
 //   - Two such tiles alternate; they are filled straight from global
 //     memory (no registers), one tile ahead, one barrier per tile.
 //   - Where the weights keep more than 16 bits (hi + lo, prompts),
@@ -32,9 +36,9 @@
 // Decode rows are split over a few partitions of the keys when there are
 // fewer rows than CUs; fp32 partials (256 KB per row and partition) are
 // merged by mla_reduce_kernel, so partitions are few and long.
-// 128 heads: 128 rows x 129..2176 keys 1025 -> 128 us with the merge (four
+// 128 heads: 128 rows x 129..2176 keys 1025 -> 90 us with the merge (four
 // waves of 16 heads on 32-key tiles, V stored transposed, before); prompts
-// of 300, 1300 and 2301 tokens 1.6 ms (600 TFLOP/s counting P once; a
+// of 300, 1300 and 2301 tokens 1.32 ms (750 TFLOP/s counting P once; a
 // composition of library products in fp32 before, 24 ms).
 
 #include <torch/all.h>
@@ -62,12 +66,16 @@ constexpr float NEG = -3.0e38f;
 constexpr float GROWTH = 8.f;
 
 // A row is 4.5 x 256 B, so odd rows start half a bank period later. The
-// eight chunks of each 128 B are exchanged by a number that differs over
-// eight row pairs (K reads: 16 rows, one chunk) and in more than its last
-// bit over four (V reads: 8 rows, two neighbouring chunks).
+// eight chunks of each 128 B are exchanged by a number that differs in more
+// than its last bit over rows 0..7 and 8..15 (V reads: 8 rows, two
+// neighbouring chunks) and keeps a part of a K read off its own banks: 16 B
+// reads are served 16 lanes at a time, lanes 0..3, 12..15, 20..23 and
+// 24..27 first, that is one chunk of rows 0..3 and 12..15 and its
+// neighbour of rows 4..11. (With lanes 0..15 in mind alone every K read met
+// each bank twice.)
 DEVINL int chunk_slot(int row, int c) {
   const int x = (row >> 1) & 7;
-  return c ^ (((x & 3) << 1) | (x >> 2));
+  return c ^ ((((x & 3) ^ ((x >> 2) << 1)) << 1) | (x >> 2));
 }
 
 // One workgroup: (token row, partition of part_len keys, head group).
@@ -201,15 +209,16 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
     // ---- S^T: 64 keys x 16 heads -----------------------------------------
     f32x4 s[4];
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      s[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < 4; ++n) s[n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kk = 0; kk < DK / 32; ++kk) {
+    for (int kk = 0; kk < DK / 32; ++kk)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
         const s16x8 a = *reinterpret_cast<const s16x8*>(
             t + k_at[kk & 1] + n * 16 * (DK * 2) + (kk >> 1) * 128);
         s[n] = mfma16<Tag>(a, qf[kk], s[n]);
       }
-    }
+    reads_ahead<4, 1, DK / 32 * 4>();
     // ---- softmax: s[n][r] is key n*16 + l4*4 + r -------------------------
     const int left = t_end - sub0 - l4 * 4;
     float mx = NEG;
@@ -255,6 +264,7 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
         if constexpr (SPLIT_P) o[i] = mfma16<Tag>(v, p_lo, o[i]);
         o[i] = mfma16<Tag>(v, p_hi, o[i]);
       }
+      reads_ahead<SPLIT_P ? 4 : 8, 2, LORA / 16, SPLIT_P ? 2 : 1>();
     }
   }
 

@@ -10,9 +10,9 @@
 //   mla_prompt_kernel   causal attention over them
 // Keys and values are rounded to the cache's type, as queries and results
 // are in the latent form; weights keep more than 16 bits (hi + lo).
-// 128 heads, prompts of 300, 1300 and 2301 tokens: 2.02 -> 0.74 ms with
+// 128 heads, prompts of 300, 1300 and 2301 tokens: 2.02 -> 0.71 ms with
 // everything between queries and results (latent form before); one of
-// 8192 13.1 -> 3.8 ms, four of 2048 4.48 -> 1.45 ms.
+// 8192 13.1 -> 3.7 ms, four of 2048 4.48 -> 1.45 ms.
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
@@ -49,9 +49,10 @@ DEVINL int seg256_chunk(int row, int c) {
 // (weights are the A operand; W_UV's fragments are transposing reads), so a
 // lane ends up with runs of columns of one token. A workgroup goes on to
 // the next heads without draining its stages (4 of them: 3 % of a prompt's
-// time). Groups of heads are neighbours in the grid: an XCD meets every
-// eighth group, whose weights stay in its L2. 3901 tokens x 128 heads: 0.22
-// ms, 590 TFLOP/s, 1.2 TB/s written.
+// time); the loop is one of two, for keys and for values, without a branch
+// among its reads. Groups of heads are neighbours in the grid: an XCD meets
+// every eighth group, whose weights stay in its L2. 3901 tokens x 128 heads:
+// 0.19 ms, 690 TFLOP/s, 1.3 TB/s written.
 constexpr int EX_M = 128;
 constexpr int EX_K = 64;
 constexpr int EX_THREADS = 8 * WAVE_SIZE;
@@ -134,64 +135,70 @@ void mla_expand_kernel(short* __restrict__ k_out,   // [heads, reqs, S, D]
                (((int64_t)h * reqs + r) * S + t0) * D + wn * 64 + half * 8;
   fill(0);
   fill(1);
+  auto run = [&](auto kind) {   // (no branch among the reads)
+    constexpr bool VALUES = decltype(kind)::value;
 #pragma unroll 1
-  for (int s = 0; s < all; ++s) {
-    // This stage has landed when only the next one's fills are under way;
-    // past the barrier every wave is done with the stage before it.
-    if (s + 1 < all) lds_fill_wait<3 * EX_FILLS>();
-    else lds_fill_wait();
-    lds_barrier();
-    if (s + 2 < all) fill(s + 2);
-    const char* t = lds + s % EX_STAGES * EX_STAGE;
+    for (int s = 0; s < all; ++s) {
+      // This stage has landed when only the next one's fills are under way;
+      // past the barrier every wave is done with the stage before it.
+      if (s + 1 < all) lds_fill_wait<3 * EX_FILLS>();
+      else lds_fill_wait();
+      lds_barrier();
+      if (s + 2 < all) fill(s + 2);
+      const char* t = lds + s % EX_STAGES * EX_STAGE;
 #pragma unroll
-    for (int kk = 0; kk < EX_K / 16; ++kk) {
-      s16x8 x[2], w[2];
+      for (int kk = 0; kk < EX_K / 16; ++kk) {
+        s16x8 x[2], w[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int row = wm * 64 + j * 32 + l32;
+          x[j] = *reinterpret_cast<const s16x8*>(
+              t + row * 128 + chunk128(row, kk * 2 + half) * 16);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          if constexpr (VALUES) {
+            const int l = kk * 16 + half * 8 + ((lane & 15) >> 2);
+            const int seg = wn * 4 + i * 2 + ((lane >> 4) & 1);
+            const char* at = t + 2 * EX_PART + (lane & 3) * 8;
+            const s16x4 a = lds_read_tr(at + l * 256 + seg256(l, seg) * 32);
+            const s16x4 b =
+                lds_read_tr(at + (l + 4) * 256 + seg256(l + 4, seg) * 32);
+            w[i] = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+          } else {
+            const int row = wn * 64 + i * 32 + l32;
+            w[i] = *reinterpret_cast<const s16x8*>(
+                t + EX_PART + row * 128 + chunk128(row, kk * 2 + half) * 16);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[i][j] = mfma32<Tag>(w[i], x[j], acc[i][j]);
+      }
+      reads_ahead<VALUES ? 9 : 6, VALUES ? 3 : 2, EX_K / 16 * 2, 2>();
+      if ((s + 1) % STEPS) continue;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int row = wm * 64 + j * 32 + l32;
-        x[j] = *reinterpret_cast<const s16x8*>(
-            t + row * 128 + chunk128(row, kk * 2 + half) * 16);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int b = 0; b < 4; b += 2) {
+            f32x16& c = acc[i][j];
+            const i32x4 w = row_chunk<Tag>(c, b);
+            if (t0 + row < ctx)
+              *reinterpret_cast<i32x4*>(out + row * D + i * 32 + b * 8) = w;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) c[b * 4 + e] = 0.f;
+          }
       }
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        if (values) {
-          const int l = kk * 16 + half * 8 + ((lane & 15) >> 2);
-          const int seg = wn * 4 + i * 2 + ((lane >> 4) & 1);
-          const char* at = t + 2 * EX_PART + (lane & 3) * 8;
-          const s16x4 a = lds_read_tr(at + l * 256 + seg256(l, seg) * 32);
-          const s16x4 b =
-              lds_read_tr(at + (l + 4) * 256 + seg256(l + 4, seg) * 32);
-          w[i] = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
-        } else {
-          const int row = wn * 64 + i * 32 + l32;
-          w[i] = *reinterpret_cast<const s16x8*>(
-              t + EX_PART + row * 128 + chunk128(row, kk * 2 + half) * 16);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = mfma32<Tag>(w[i], x[j], acc[i][j]);
+      out += (int64_t)reqs * S * D;
     }
-    if ((s + 1) % STEPS) continue;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int row = wm * 64 + j * 32 + l32;
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int b = 0; b < 4; b += 2) {
-          f32x16& c = acc[i][j];
-          const i32x4 w = row_chunk<Tag>(c, b);
-          if (t0 + row < ctx)
-            *reinterpret_cast<i32x4*>(out + row * D + i * 32 + b * 8) = w;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) c[b * 4 + e] = 0.f;
-        }
-    }
-    out += (int64_t)reqs * S * D;
-  }
+  };
+  if (values) run(std::true_type{});
+  else run(std::false_type{});
   if (write_pe && h == 0) {
     for (int c = threadIdx.x; c < EX_M * 8; c += EX_THREADS)
       if (t0 + (c >> 3) < ctx)

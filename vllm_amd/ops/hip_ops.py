@@ -238,13 +238,13 @@ _MLA_PART_MIN = 128
 
 
 def _mla_parts(rows, heads, max_seq_len):
-    """Into how many partitions a row's keys are split: as many as fill
-    the chip and no more (128 heads, us: 128 rows x 129..2176 keys 182 in
-    one, 116 in 2, 140 in 4; 32 x 8192 keys 125 in 8, 150 in 16), none
-    shorter than two tiles (one row x 1000 keys 36 in 4, 27 in 8; x 4000
-    39 in 16, 33 in 32, 37 in 63), at most 64."""
+    """Into how many partitions a row's keys are split: as many as run at
+    a time and no more (128 heads, us in 1 / 2 / 4 / 8: 200 rows x 129..2176
+    keys 139 / 151 / 149; 128 rows 128 / 90 / 115; 32 rows x 8192 441 / 237
+    / 134 / 105, 16 132), none shorter than two tiles (one row x 1000 keys
+    24 in 8, 22 in 16; x 4000 31 in 16, 29 in 32, 35 in 63), at most 64."""
     groups = rows * -(-heads // 128)
-    return max(1, min(-(-_MLA_FILL // max(groups, 1)),
+    return max(1, min(_MLA_FILL // max(groups, 1),
                       -(-max_seq_len // _MLA_PART_MIN), 64))
 
 
@@ -343,20 +343,21 @@ def _mla_prompt_heads(q_nope, w_uk, w_uv, kv_cache, reqs, scale,
     """How many heads at a time prompt portions attend with keys and
     values carried out of the latent space (csrc/mla_prompt.hip); 0:
     in it (csrc/mla.hip). Carrying them out costs by context row, the
-    latent form by query (0.25 us plus 0.38 per 1000 keys, for 128 heads
-    and no fewer than 256 queries, which fill the chip), so the line is a
-    number of queries per request that grows with the context. 8 requests,
-    us per head / latent: 96 tokens of 512 273 / 317, of 1024 530 / 466;
-    160 of 2048 1218 / 1185, 192 1199 / 1420; 192 of 4096 2532 / 2478. Only
-    the longest context is known here: shorter ones cost less than this
-    says, most so per head."""
+    latent form by query (a part for each and a part per key; 200 at
+    least, which fill the chip), so the line is a number of queries per
+    request that grows with the context. us per head / latent, 8 requests:
+    96 tokens of 512 256 / 260, 128 266 / 345; 192 of 2048 1174 / 1130, 256
+    of 4096 2433 / 2660; 32 requests: 32 of 128 272 / 251, 64 of 256 505 /
+    547; one: 128 of 2048 147 / 164, 64 of 8192 563 / 515. Only the longest
+    context is known here: shorter ones cost less than this says, most so
+    per head."""
     T, Hq, nope = q_nope.shape
     rows, reqs = T - num_decodes, reqs - num_decodes
     S = max(max_seq_len, 128)
     if (nope != 128 or w_uk.shape[2] != 512 or w_uv.shape[2] != 128
             or kv_cache.shape[2] != 576 or scale <= 0 or max_query_len <= 0
             or max_seq_len <= 0 or not 0 < reqs < 65536 or rows <= 0
-            or max(rows, 256) * (800 + S) < reqs * 200 * S
+            or max(rows, 200) * (800 + S) < reqs * 255 * S
             or q_nope.dtype not in (torch.bfloat16, torch.float16)
             or any(t.dtype != q_nope.dtype for t in (w_uk, w_uv, kv_cache))
             or not all(t.is_contiguous() for t in (w_uk, w_uv, kv_cache))
