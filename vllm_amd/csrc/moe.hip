@@ -404,12 +404,13 @@ void moe_stream_kernel(const short* __restrict__ A, int64_t lda,
 // wave (16 B stores: the second product 5 % faster). 32-row groups without
 // a row are left out, by wave, so padding costs fills but few products.
 //   WM 4, 256 rows: waves of 64 x 128, half the traffic from L2 per
-//                   product, two stages, reads and products of the two
-//                   halves of the workgroup in turn (all waves in step:
-//                   3.41 ms for 64 experts x 512 rows of 7168 x 2048, 3.16
-//                   now; 8 experts x 1024 rows of 4096 x 14336 3.18 and
-//                   2.87: 1000 TFLOP/s). Products alone would take 2.5 ms,
-//                   fills alone 2.9: weights that miss L2 bound it.
+//                   product, reads and products of the two halves of the
+//                   workgroup in turn, weights filled two steps ahead.
+//                   64 experts x 512 rows of 7168 x 2048: all waves in step
+//                   3.41 ms, in turn 3.24, weights ahead 3.17; 8 experts x
+//                   1024 rows of 4096 x 14336 3.18, 2.90, 2.82 (1020
+//                   TFLOP/s). Products alone would take 2.5 ms, with
+//                   weights always in L2 2.6.
 //   WM 2, 128 rows: waves of 64 x 64, three stages. For experts of few
 //                   rows, and for what is left of an expert's rows after
 //                   whole tiles of 256.
@@ -418,7 +419,7 @@ void moe_stream_kernel(const short* __restrict__ A, int64_t lda,
 constexpr int TL_W = 256;
 constexpr int TL_K = 64;
 constexpr int TL_THREADS = 8 * WAVE_SIZE;
-constexpr int TL_LDS = 144 * 1024;                   // bytes of the stages
+constexpr int TL_LDS = 160 * 1024;                   // all there is
 constexpr int TL_ROW = TL_K * 2;                     // bytes of a row
 constexpr int TL_CH = TL_ROW / 16;                   // 16 B chunks of a row
 constexpr int TL_FR = WAVE_SIZE / TL_CH;             // rows a fill moves
@@ -472,15 +473,19 @@ DEVINL void tile_body(char* lds, const short* __restrict__ A, int64_t lda,
       src = min(n0 + r, N - 1);
     wp[i] = src * (uint32_t)K * 2 + ((lane % TL_CH) ^ tl_swap(r)) * 16;
   }
-  auto fill = [&](int step, int stage) {
-    char* dst = lds + stage * TL_STAGE;
+  auto fill_a = [&](int step, char* dst) {
 #pragma unroll
     for (int i = 0; i < TL_FA; ++i)
       lds_fill16(A + step * TL_K, ap[i], dst + (wave * TL_FA + i) * 1024);
-    dst += TL_M * TL_ROW;
+  };
+  auto fill_w = [&](int step, char* dst) {
 #pragma unroll
     for (int i = 0; i < TL_FW; ++i)
       lds_fill16(W + step * TL_K, wp[i], dst + (wave * TL_FW + i) * 1024);
+  };
+  auto fill = [&](int step, int stage) {
+    fill_a(step, lds + stage * TL_STAGE);
+    fill_w(step, lds + stage * TL_STAGE + TL_M * TL_ROW);
   };
 
   f32x16 acc[TL_WI][TL_MI];
@@ -501,29 +506,32 @@ DEVINL void tile_body(char* lds, const short* __restrict__ A, int64_t lda,
   if constexpr (WM == 4) {
     // Waves 4..7 run one slot behind waves 0..3, their neighbours on the
     // SIMDs: one half multiplies 32 of K while the other reads the next 32
-    // into fragments, a barrier a slot, four slots a stage. The next stage
-    // is filled from the first slot on (the laggards read its place last
-    // in the slot before) and has landed for all when the fourth ends.
+    // into fragments, a barrier a slot, four slots a step. A step's first
+    // slot starts the fills of the next step's rows and of the weights one
+    // further on, which come from HBM (three places for weights, two for
+    // rows; the laggards read the places these take last in the slot
+    // before). When its fourth ends, all the next step needs has landed.
     // The number of row groups is a constant of the loop: merging
     // accumulators of several branches would copy them.
     const int lag = wave >> 2;
+    constexpr int AB = TL_M * TL_ROW, WB = TL_W * TL_ROW;
     const char* a0 = lds + wm * TL_MI * 32 * TL_ROW;
-    const char* w0 = lds + TL_M * TL_ROW + wn * TL_WW * TL_ROW;
+    const char* w0 = lds + 2 * AB + wn * TL_WW * TL_ROW;
     auto run = [&](auto n) {
       constexpr int J = decltype(n)::value;
       s16x8 af[2][J > 0 ? J : 1], wf[2][TL_WI];
-      auto read = [&](int stage, int k0) {
+      auto read = [&](int stage, int wst, int k0) {
         if constexpr (J > 0) {
 #pragma unroll
           for (int k = 0; k < 2; ++k) {
 #pragma unroll
             for (int j = 0; j < J; ++j)
               af[k][j] = *reinterpret_cast<const s16x8*>(
-                  a0 + stage * TL_STAGE + j * 32 * TL_ROW + at[k0 + k]);
+                  a0 + stage * AB + j * 32 * TL_ROW + at[k0 + k]);
 #pragma unroll
             for (int i = 0; i < TL_WI; ++i)
               wf[k][i] = *reinterpret_cast<const s16x8*>(
-                  w0 + stage * TL_STAGE + i * 32 * TL_ROW + at[k0 + k]);
+                  w0 + wst * WB + i * 32 * TL_ROW + at[k0 + k]);
           }
         }
       };
@@ -542,24 +550,34 @@ DEVINL void tile_body(char* lds, const short* __restrict__ A, int64_t lda,
       };
       if (lag) lds_barrier();   // (as many barriers for every wave)
 #pragma unroll 1
-      for (int s = 0; s < steps; ++s) {
+      for (int s = 0, wst = 0; s < steps; ++s) {
         const int stage = s & 1;
-        if (s + 1 < steps) fill(s + 1, stage ^ 1);
-        read(stage, 0);
+        if (s + 1 < steps) fill_a(s + 1, lds + (stage ^ 1) * AB);
+        if (s + 2 < steps)
+          fill_w(s + 2, lds + 2 * AB + (wst == 0 ? 2 : wst - 1) * WB);
+        auto landed = [&]() {
+          if (s + 2 < steps) lds_fill_wait<TL_FW>();
+          else lds_fill_wait();
+        };
+        read(stage, wst, 0);
         lds_barrier();
         multiply();
         lds_barrier();
-        read(stage, 2);
-        if (lag) lds_fill_wait();
+        read(stage, wst, 2);
+        if (lag) landed();
         lds_barrier();
         multiply();
-        if (!lag) lds_fill_wait();
+        if (!lag) landed();
         lds_barrier();
+        wst = wst == 2 ? 0 : wst + 1;
       }
       if (!lag) lds_barrier();
     };
-    fill(0, 0);
-    lds_fill_wait();
+    fill_a(0, lds);
+    fill_w(0, lds + 2 * AB);
+    if (steps > 1) fill_w(1, lds + 2 * AB + WB);
+    if (steps > 1) lds_fill_wait<TL_FW>();
+    else lds_fill_wait();
     lds_barrier();
     if (groups >= 2) run(std::integral_constant<int, 2>{});
     else if (groups == 1) run(std::integral_constant<int, 1>{});
