@@ -128,8 +128,9 @@ class FusedMoE(nn.Module):
         # lazily on the first GPU forward; freed by invalidate_shuffled
         # when weights change). Costs a second copy of the expert
         # weights — the MI355X trade: 288 GB HBM buys coalesced,
-        # barrier-free weight streams. Opt-in via VLLM_AMD_MOE_SHUF=1
-        # (the staged-LDS kernel measured faster at decode batch>=256).
+        # barrier-free weight streams. Opt-in via VLLM_AMD_MOE_SHUF=1:
+        # a few percent for batches of few rows per expert, the others
+        # run in tiles that take the plain weights.
         self._w13_shuf = None
         self._w2_shuf = None
 
@@ -233,10 +234,10 @@ class FusedMoE(nn.Module):
     def _maybe_shuffled(self, hidden):
         import os
 
-        # Fragment-major streaming is opt-in (VLLM_AMD_MOE_SHUF=1): on
-        # MI355X the staged-LDS grouped GEMM measured faster at decode
-        # batch >= 256 (the barrier-free stream wins only at tiny
-        # batches; see profiles/r02_summary.md).
+        # Fragment-major streaming is opt-in (VLLM_AMD_MOE_SHUF=1): 1 to
+        # 10 % faster where an expert gets few rows (8 experts of 4096 x
+        # 14336: 1 token 165 -> 146 us, 48 tokens 518 -> 500), for a
+        # second copy of the weights.
         if (not hidden.is_cuda
                 or os.environ.get("VLLM_AMD_MOE_SHUF", "0") != "1"):
             return None, None

@@ -453,11 +453,12 @@ def fused_moe_hip(hidden, w13, w2, topk_weights, topk_ids,
     k = topk_ids.shape[1]
     total = T * k
     dev = hidden.device
-    shuf = w13_shuf is not None or w2_shuf is not None
-    form = (0 if shuf or total < _MOE_TILES_FROM * E else
+    form = (0 if total < _MOE_TILES_FROM * E else
             1 if total < _MOE_WIDE_TILES_FROM * E else 2)
     if max(T * H, (total + E * 256) * I, n1 * H) >= 1 << 31:
         form = 0    # tiles address 4 GB
+    if form > 0:    # (they take the weights in their own order)
+        w13_shuf = w2_shuf = None
     bm = _C.moe_tile_rows(form)
     tiles = (total + min(E, total) * (bm - 1)) // bm
     em = tiles * bm
