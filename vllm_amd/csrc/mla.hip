@@ -35,8 +35,9 @@
 //     64-bit results.
 // Decode rows are split over a few partitions of the keys when there are
 // fewer rows than CUs; fp32 partials (256 KB per row and partition) are
-// merged by mla_reduce_kernel, so partitions are few and long.
-// 128 heads: 128 rows x 129..2176 keys 1025 -> 90 us with the merge (four
+// merged by mla_reduce_kernel, so partitions are few and long, and rows
+// that fit one are written at once.
+// 128 heads: 128 rows x 129..2176 keys 1025 -> 88 us with the merge (four
 // waves of 16 heads on 32-key tiles, V stored transposed, before); prompts
 // of 300, 1300 and 2301 tokens 1.32 ms (750 TFLOP/s counting P once; a
 // composition of library products in fp32 before, 24 ms).
@@ -272,7 +273,7 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
   l_run += __shfl_xor(l_run, 32, 64);
   if (head >= num_heads) return;
   const int64_t hrow = (int64_t)row * num_heads + head;
-  if (PROMPT || num_parts == 1) {
+  if (PROMPT || num_parts == 1 || ctx <= part_len) {   // nothing to merge
     const float inv_l = 1.f / l_run;
     short* ob = out + hrow * LORA + l4 * 4;
 #pragma unroll
@@ -306,7 +307,7 @@ void mla_reduce_kernel(short* __restrict__ out,
   const int h = blockIdx.x;
   const int seq = blockIdx.y;
   const int parts = min((seq_lens[seq] + part_len - 1) / part_len, num_parts);
-  if (parts <= 0) return;
+  if (parts <= 1) return;   // the row fits one partition: it is done
   const int64_t hrow = (int64_t)seq * num_heads + h;
   const float* lse = tmp_lse + hrow * num_parts * 2;
   float m = NEG;
