@@ -749,6 +749,32 @@ def test_rope_and_cache(T, Hq, Hkv, D, rot, bs, dtype, fp8):
     assert torch.equal(cache.view(torch.uint8), want.view(torch.uint8))
 
 
+@pytest.mark.parametrize("T", [1, 70])
+def test_mla_a_projections_as_one(T):
+    """One product over both weights, through a move of the module, and
+    the norm of rows of a wider matrix: the same as apart but for the order
+    of fp32 sums, one rounding of values up to about 4 (2^-8 of them)."""
+    from vllm_amd.config import get_model_spec
+    from vllm_amd.models.deepseek import DeepseekMLAAttention
+
+    block = DeepseekMLAAttention(get_model_spec("deepseek-v3-lite"), 0,
+                                 torch.bfloat16, 64)
+    for p in block.parameters():
+        p.data.normal_(std=0.01)
+    block = block.cuda()
+    q, kv = block.q_a_proj.weight, block.kv_a_proj_with_mqa.weight
+    assert kv.data_ptr() == q.data_ptr() + 2 * q.numel()
+    x = torch.randn(T, q.shape[1], device="cuda", dtype=torch.bfloat16)
+    q_a, kv_a = block._a_projs(x)
+    assert not T > 1 or not q_a.is_contiguous()
+    assert_close(q_a, x.float() @ q.float().T, atol=2**-8, rtol=2**-7)
+    assert_close(kv_a, x.float() @ kv.float().T, atol=2**-8, rtol=2**-7)
+    assert torch.equal(block.q_a_layernorm(q_a),
+                       block.q_a_layernorm(q_a.contiguous()))
+    kv.data = kv.data.clone()     # no longer behind the other: apart
+    assert_close(block._a_projs(x)[1], kv_a, atol=2**-8, rtol=2**-7)
+
+
 def test_mla_unified_dispatch_mixed_batch():
     """ops.mla_attention routes decode rows to the kernel and prefill
     rows to the torch path; both must agree with the all-torch result."""

@@ -22,10 +22,11 @@ template <typename Tag, int BLOCK>
 __global__ void rms_norm_kernel(short* __restrict__ out,
                                 const short* __restrict__ in,
                                 const short* __restrict__ weight,
-                                const float eps, const int hidden) {
+                                const float eps, const int hidden,
+                                const int64_t in_stride) {
   __shared__ float red[BLOCK / WAVE_SIZE];
   const int64_t row = blockIdx.x;
-  const short* x = in + row * hidden;
+  const short* x = in + row * in_stride;
   short* o = out + row * hidden;
 
   float ss = 0.f;
@@ -332,9 +333,16 @@ static inline void check_rows_16b(const torch::Tensor& t, const char* name) {
   }
 
 torch::Tensor rms_norm(torch::Tensor x, torch::Tensor weight, double eps) {
-  check_16b(x, "x");
-  auto out = torch::empty_like(x);
+  // Contiguous, or the rows of a wider matrix.
+  const bool rows_of = x.dim() == 2 && x.stride(1) == 1 &&
+                       x.stride(0) % 8 == 0 &&
+                       (uintptr_t)x.data_ptr() % 16 == 0;
+  if (!rows_of) check_16b(x, "x");
+  TORCH_CHECK(x.scalar_type() == torch::kBFloat16 ||
+              x.scalar_type() == torch::kHalf, "x must be bf16 or fp16");
+  auto out = torch::empty(x.sizes(), x.options());
   const int hidden = x.size(-1);
+  const int64_t stride = x.is_contiguous() ? hidden : x.stride(0);
   TORCH_CHECK(hidden % 8 == 0, "hidden must be a multiple of 8");
   const int64_t rows = x.numel() / hidden;
   constexpr int BLOCK = 256;
@@ -343,7 +351,8 @@ torch::Tensor rms_norm(torch::Tensor x, torch::Tensor weight, double eps) {
   hipLaunchKernelGGL((rms_norm_kernel<TAG, BLOCK>), dim3(rows),          \
                      dim3(BLOCK), 0, stream,                             \
                      (short*)out.data_ptr(), (const short*)x.data_ptr(), \
-                     (const short*)weight.data_ptr(), (float)eps, hidden)
+                     (const short*)weight.data_ptr(), (float)eps, hidden, \
+                     stride)
   DISPATCH_16B(x, LAUNCH_RMS);
 #undef LAUNCH_RMS
   HIP_CHECK_KERNEL();

@@ -89,6 +89,40 @@ class DeepseekMLAAttention(nn.Module):
             self.qk_rope, self.qk_rope, max_position, theta=spec.rope_theta,
             rope_scaling=spec.rope_scaling,
         )
+        self._join_a_projs()
+
+    def _apply(self, fn, recurse=True):
+        super()._apply(fn, recurse)
+        self._join_a_projs()
+        return self
+
+    def _join_a_projs(self) -> None:
+        """Lays the weights of the two projections of the hidden state one
+        behind the other, so that _a_projs can take them as one matrix."""
+        if self.q_a_proj is None:
+            return
+        q, kv = self.q_a_proj.weight, self.kv_a_proj_with_mqa.weight
+        if q.numel() == 0 or q.dtype != kv.dtype or q.device != kv.device:
+            return
+        both = torch.cat([q.data, kv.data])
+        q.data, kv.data = both[: q.shape[0]], both[q.shape[0]:]
+
+    def _a_projs(self, hidden):
+        """q_a_proj and kv_a_proj_with_mqa of hidden. As one product where
+        their weights lie one behind the other in one storage (us for 1536
+        + 576 rows of 7168, apart / as one: 1 token 20.7 / 10.6, 128 30.8 /
+        22.7, 3901 132 / 102, 8192 215 / 218)."""
+        q, kv = self.q_a_proj.weight, self.kv_a_proj_with_mqa.weight
+        if (hidden.is_cuda and hidden.shape[0] <= 4096 and q.numel() > 0
+                and kv.numel() > 0 and q.dtype == kv.dtype
+                and q.is_contiguous() and kv.is_contiguous()
+                and q.untyped_storage().data_ptr()
+                == kv.untyped_storage().data_ptr()
+                and kv.storage_offset() == q.storage_offset() + q.numel()):
+            n, k = q.shape
+            both = torch.as_strided(q, (n + kv.shape[0], k), (k, 1))
+            return ops.linear(hidden, both).split([n, kv.shape[0]], dim=1)
+        return self.q_a_proj(hidden), self.kv_a_proj_with_mqa(hidden)
 
     def load_kv_b_proj(self, kv_b_weight: torch.Tensor) -> None:
         """kv_b_proj.weight [Hq*(nope+v), lora] (full) -> absorbed splits
@@ -106,13 +140,14 @@ class DeepseekMLAAttention(nn.Module):
     def forward(self, positions, hidden):
         T = hidden.shape[0]
         if self.q_a_proj is not None:
-            q = self.q_b_proj(self.q_a_layernorm(self.q_a_proj(hidden)))
+            q_a, kv_a = self._a_projs(hidden)
+            q = self.q_b_proj(self.q_a_layernorm(q_a))
         else:
             q = self.q_proj(hidden)
+            kv_a = self.kv_a_proj_with_mqa(hidden)
         q = q.view(T, self.num_heads, self.qk_head_dim)
         q_nope, q_pe = q[..., : self.qk_nope], q[..., self.qk_nope:]
 
-        kv_a = self.kv_a_proj_with_mqa(hidden)
         ctx = get_forward_context()
         meta = ctx.attn_metadata
         if not ctx.kv_caches:
