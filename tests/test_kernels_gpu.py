@@ -176,6 +176,31 @@ def test_decode_attention_edges(hd, group, dtype, cache_dtype, window, n):
     assert_close(out[rows], expect, atol=atol, rtol=atol / 4)
 
 
+@pytest.mark.parametrize("n,longest", [(300, 700), (3, 700), (300, 90)])
+def test_decode_rows_without_keys(n, longest):
+    """A row of length 0 (a captured step's padding) gives exact zeros,
+    whether its keys would be split or not, and leaves the others alone.
+    The memory that results are taken from holds NaN."""
+    hip = _hip()
+    q, cache, bt, qsl, sl = _make_paged(n, [1] * n, [longest] * n, 8, 2)
+    sl[1::2] = 0
+    junk = torch.full_like(q, float("nan"))
+    del junk
+    out = hip.attention_unified(q, cache, bt, qsl, sl, 0.1, num_decodes=n,
+                                max_seq_len=longest, max_query_len=1)
+    assert (out[1::2] == 0).all() and out[::2].isfinite().all()
+    lat = torch.randn(n * 2, 64, 576, device="cuda", dtype=torch.bfloat16)
+    bt = torch.arange(n * 2, device="cuda", dtype=torch.int32).view(n, 2)
+    sl.clamp_(max=128)
+    for heads in (20, 130):
+        qn = torch.randn(n, heads, 512, device="cuda", dtype=torch.bfloat16)
+        junk = torch.full_like(qn, float("nan"))
+        del junk
+        out = hip.mla_decode(qn, qn[..., :64].contiguous(), lat, bt, sl,
+                             0.07, 128)
+        assert (out[1::2] == 0).all() and out[::2].isfinite().all()
+
+
 @pytest.mark.parametrize("group", [4])
 @pytest.mark.parametrize(
     "q_lens,ctx_lens",

@@ -97,6 +97,10 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
   const int t_end = min(ctx, t_begin + part_len);
 
   if (t_begin >= t_end) {
+    // A row without keys (padding) is zero, also where nothing merges it.
+    if constexpr (FINAL)
+      for (int e = threadIdx.x; e < group * HD; e += DEC_BLOCK)
+        out[((int64_t)seq * num_q_heads + hq0) * HD + e] = 0;
     if (!FINAL && threadIdx.x < group * 2) {
       const int g = threadIdx.x / 2;
       tmp_lse[(((int64_t)seq * num_q_heads + hq0 + g) * num_parts + part) *

@@ -117,7 +117,15 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
   const int hg0 = blockIdx.z * HG;
   const int t_begin = part * part_len;
   const int t_end = min(ctx, t_begin + part_len);
-  if (t_begin >= t_end) return;
+  if (t_begin >= t_end) {
+    if (!PROMPT && part == 0) {   // a row without keys (padding) is zero
+      const int n = min(HG, num_heads - hg0) * (LORA / 8);
+      short* ob = out + ((int64_t)row * num_heads + hg0) * LORA;
+      for (int c = threadIdx.x; c < n; c += THREADS)
+        *reinterpret_cast<i32x4*>(ob + c * 8) = i32x4{0, 0, 0, 0};
+    }
+    return;
+  }
 
   __shared__ __align__(16) char lds[BUFS * TILE_BYTES];
 
