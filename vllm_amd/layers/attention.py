@@ -90,6 +90,7 @@ class Attention(nn.Module):
             sliding_window=self.sliding_window,
             max_seq_len=meta.max_seq_len,
             max_query_len=meta.max_query_len,
+            max_decode_len=meta.max_decode_len,
         )
         return out.reshape(T, -1)
 

@@ -171,6 +171,7 @@ class DeepseekMLAAttention(nn.Module):
                 self.scale, num_decodes=meta.num_decodes,
                 max_query_len=meta.max_query_len,
                 max_seq_len=meta.max_seq_len,
+                max_decode_len=meta.max_decode_len,
             )
         return self.o_proj(out.reshape(T, -1))
 

@@ -98,6 +98,7 @@ def attention_unified(
     sliding_window: int = 0,
     max_seq_len: int = 0,
     max_query_len: int = 0,
+    max_decode_len: int = 0,
 ):
     """Varlen attention over the paged KV cache (prefill + decode mixed).
 
@@ -105,11 +106,13 @@ def attention_unified(
     num_kv_heads, block_size, head_dim]; returns [num_tokens, num_heads,
     head_dim]. Requests are ordered decodes-first (query_len==1).
     max_seq_len/max_query_len are CPU-known hints so the GPU path never
-    syncs to size its scratch.
+    syncs to size its scratch; max_decode_len bounds the contexts of the
+    decode rows alone (0: max_seq_len does).
     """
     return get_backend(q.device).attention_unified(
         q, kv_cache, block_table, query_start_loc, seq_lens, scale,
         num_decodes, sliding_window, max_seq_len, max_query_len,
+        max_decode_len,
     )
 
 
@@ -162,13 +165,14 @@ def mla_prepare(positions, q_pe, kv_a, weight, eps, cos_sin_cache, kv_cache,
 
 def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
               query_start_loc, seq_lens, scale, num_decodes=0,
-              max_query_len=0, max_seq_len=0):
+              max_query_len=0, max_seq_len=0, max_decode_len=0):
     backend = get_backend(q_nope.device)
     if backend is not _torch_ref:
         return backend.mla_heads(
             q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
             query_start_loc, seq_lens, scale, num_decodes=num_decodes,
             max_query_len=max_query_len, max_seq_len=max_seq_len,
+            max_decode_len=max_decode_len,
         )
     return backend.mla_heads(
         q_nope, q_pe, w_uk, w_uv, kv_cache, block_table, query_start_loc,

@@ -115,6 +115,7 @@ def attention_unified(
     sliding_window=0,
     max_seq_len=0,
     max_query_len=0,
+    max_decode_len=0,
 ):
     num_tokens, num_heads, head_dim = q.shape
     num_kv_heads = kv_cache.shape[2]

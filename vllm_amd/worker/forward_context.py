@@ -42,6 +42,10 @@ class AttentionMetadata:
     # order (decodes first) — indexes the runner's state tensors. None
     # for models without such state.
     state_rows: Optional[torch.Tensor] = None
+    # Longest context among the first num_decodes requests: their keys
+    # are split by it, whatever prompts ride along. 0: not known, then
+    # max_seq_len stands for it.
+    max_decode_len: int = 0
 
 
 @dataclass
