@@ -81,9 +81,9 @@ def test_mla_decode_split_ignores_prompts(hip, rows, monkeypatch):
     assert split(8192) == split(0)
 
 
-def test_runner_tells_decode_lengths(monkeypatch):
-    """The runner's steps say how long their decode rows are, with and
-    without prompts beside them."""
+def test_runner_tells_lengths(monkeypatch):
+    """The runner's mixed steps say how long their decode rows are, and
+    how long their prompts' contexts."""
     from vllm_amd.entrypoints.llm import LLM
     from vllm_amd.layers import attention
     from vllm_amd.sampling_params import SamplingParams
@@ -91,10 +91,12 @@ def test_runner_tells_decode_lengths(monkeypatch):
     real, seen = attention.ops, []
 
     def spy(q, kv, bt, qsl, sl, scale, **kw):
-        nd = kw["num_decodes"]
+        meta = attention.get_forward_context().attn_metadata
+        nd = meta.num_decodes
         if 0 < nd < len(sl):
-            seen.append((kw["max_decode_len"], int(sl[:nd].max()),
-                         kw["max_seq_len"]))
+            assert kw["max_decode_len"] == int(sl[:nd].max())
+            assert meta.max_prompt_len == int(sl[nd:].max())
+            seen.append(kw["max_decode_len"] < kw["max_seq_len"])
         return real.attention_unified(q, kv, bt, qsl, sl, scale, **kw)
 
     monkeypatch.setattr(attention, "ops", types.SimpleNamespace(
@@ -107,5 +109,46 @@ def test_runner_tells_decode_lengths(monkeypatch):
                  SamplingParams(temperature=0.0, max_tokens=8,
                                 ignore_eos=True))
     llm.shutdown()
-    assert all(told == real_max for told, real_max, _ in seen)
-    assert any(told < longest for told, _, longest in seen)
+    assert any(seen)
+
+
+def _mla_prompts(hip, monkeypatch, decodes, prompts, H=128, **kw):
+    """The arguments of the per-head prompt kernel for 400-token prompts
+    beside decode rows of 8192 keys."""
+    n, t = decodes + prompts, decodes + prompts * 400
+    q = torch.empty(t, H, 192, dtype=torch.bfloat16)
+    monkeypatch.setattr(hip, "mla_attention",
+                        lambda q, *a, **k: torch.empty_like(q))
+    monkeypatch.setattr(hip, "head_matmul", lambda x, w: torch.empty(
+        x.shape[0], x.shape[1], w.shape[2], dtype=x.dtype))
+    hip._C.calls.clear()
+    hip.mla_heads(
+        q[..., :128], q[..., 128:],
+        torch.empty(H, 128, 512, dtype=torch.bfloat16),
+        torch.empty(H, 512, 128, dtype=torch.bfloat16),
+        torch.empty(1, 64, 576, dtype=torch.bfloat16),
+        torch.zeros(n, 1, dtype=torch.int32), _lens(*range(n + 1)),
+        _lens(*[400] * n), 0.07, num_decodes=decodes, max_query_len=400,
+        max_seq_len=8192 if decodes else 400, **kw)
+    (a,) = hip._C.args("mla_prompt_attention")
+    return a[12], a[13].numel()   # S, scratch
+
+
+def test_mla_prompt_scratch_ignores_decodes(hip, monkeypatch):
+    """Prompts' scratch is sized by the prompts' own contexts."""
+    alone = _mla_prompts(hip, monkeypatch, 0, 20)
+    beside = _mla_prompts(hip, monkeypatch, 1, 20, max_decode_len=8192,
+                          max_prompt_len=400)
+    assert alone == beside == (400, 20 * 400 * (64 + 128 * 256))
+
+
+def test_mla_prompt_heads_at_a_time(hip, monkeypatch):
+    """Heads that do not fit at once go in multiples of eight, one per
+    XCD, while eight fit."""
+    S, numel = _mla_prompts(hip, monkeypatch, 1, 60)
+    per = 60 * S
+    heads = (numel // per - 64) // 256
+    assert numel == per * (64 + heads * 256) and 1 <= heads < 8
+    monkeypatch.setattr(hip, "_MLA_PROMPT_SCRATCH", 13 * 60 * S * 512)
+    _, numel = _mla_prompts(hip, monkeypatch, 1, 60)
+    assert (numel // per - 64) // 256 == 8

@@ -219,7 +219,8 @@ void mla_expand_kernel(short* __restrict__ k_out,   // [heads, reqs, S, D]
 // barrier a tile: 80 KB, two workgroups a CU, one's softmax under the
 // other's products. Accumulators are rescaled when a maximum has grown by
 // 2^8. 3901 tokens as above: 0.50 ms, 820 TFLOP/s with both halves of the
-// weights. All tiles of a head run on one XCD, late ones (most keys) first.
+// weights. All tiles of a head run on one XCD, late ones (most keys) first;
+// where fewer than eight heads run at a time, a head's tiles go to several.
 constexpr int PA_M = 128;
 constexpr int PA_KEYS = 64;
 constexpr int PA_THREADS = 4 * WAVE_SIZE;
@@ -247,8 +248,9 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
                        const int* __restrict__ seq_lens, float scale_log2,
                        int num_heads, int head0, int heads, int num_decodes,
                        int S, int tiles) {
-  const int seq = (int)blockIdx.x >> 3;
-  const int h = seq / tiles * 8 + ((int)blockIdx.x & 7);
+  const int lanes = min(heads, 8);
+  const int seq = (int)blockIdx.x / lanes;
+  const int h = seq / tiles * lanes + (int)blockIdx.x % lanes;
   if (h >= heads) return;
   const int r = blockIdx.y;
   const int req = num_decodes + r;
@@ -487,9 +489,11 @@ void mla_prompt_attention(torch::Tensor out, torch::Tensor q_nope,
           (int)block_table.size(1), seq_lens.data_ptr<int>(),
           (int)kv_cache.size(1), (int)num_decodes, (int)S, heads, per, h0 == 0);
       HIP_CHECK_KERNEL();
+      const int lanes = std::min(heads, 8);
       hipLaunchKernelGGL(
           (mla_prompt_kernel<Tag>),
-          dim3(ceil_div(heads, 8) * 8 * tiles, (int)reqs), dim3(PA_THREADS),
+          dim3(ceil_div(heads, lanes) * lanes * tiles, (int)reqs),
+          dim3(PA_THREADS),
           0, stream, (short*)out.data_ptr(), (const short*)q_nope.data_ptr(),
           q_nope.stride(0), q_nope.stride(1), (const short*)q_pe.data_ptr(),
           k, v, pe, query_start_loc.data_ptr<int>(),

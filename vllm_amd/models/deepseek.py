@@ -172,6 +172,7 @@ class DeepseekMLAAttention(nn.Module):
                 max_query_len=meta.max_query_len,
                 max_seq_len=meta.max_seq_len,
                 max_decode_len=meta.max_decode_len,
+                max_prompt_len=meta.max_prompt_len,
             )
         return self.o_proj(out.reshape(T, -1))
 

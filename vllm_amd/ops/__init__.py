@@ -165,14 +165,15 @@ def mla_prepare(positions, q_pe, kv_a, weight, eps, cos_sin_cache, kv_cache,
 
 def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
               query_start_loc, seq_lens, scale, num_decodes=0,
-              max_query_len=0, max_seq_len=0, max_decode_len=0):
+              max_query_len=0, max_seq_len=0, max_decode_len=0,
+              max_prompt_len=0):
     backend = get_backend(q_nope.device)
     if backend is not _torch_ref:
         return backend.mla_heads(
             q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
             query_start_loc, seq_lens, scale, num_decodes=num_decodes,
             max_query_len=max_query_len, max_seq_len=max_seq_len,
-            max_decode_len=max_decode_len,
+            max_decode_len=max_decode_len, max_prompt_len=max_prompt_len,
         )
     return backend.mla_heads(
         q_nope, q_pe, w_uk, w_uv, kv_cache, block_table, query_start_loc,

@@ -42,10 +42,12 @@ class AttentionMetadata:
     # order (decodes first) — indexes the runner's state tensors. None
     # for models without such state.
     state_rows: Optional[torch.Tensor] = None
-    # Longest context among the first num_decodes requests: their keys
-    # are split by it, whatever prompts ride along. 0: not known, then
-    # max_seq_len stands for it.
+    # Longest context among the first num_decodes requests and among the
+    # others: what one kind's kernels split and allocate by does not
+    # depend on the other kind. 0: not known, then max_seq_len stands
+    # for it.
     max_decode_len: int = 0
+    max_prompt_len: int = 0
 
 
 @dataclass

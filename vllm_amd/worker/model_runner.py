@@ -1408,6 +1408,7 @@ class ModelRunner:
             max_query_len=int(max(n for _, n in items)),
             max_seq_len=max_seq_len,
             max_decode_len=int(seq_lens[:num_decodes].max(initial=0)),
+            max_prompt_len=int(seq_lens[num_decodes:].max(initial=0)),
             num_decodes=num_decodes,
             state_rows=(torch.tensor(
                 [self._row_of[rid] for rid, _ in items],
