@@ -875,3 +875,32 @@ def test_moe_shuffled_weight_gemm(T, H, I, E, K):
     expect = ref.fused_moe(hidden.float(), w13.float(), w2.float(), tw, ti)
     assert_close(out, base, atol=1e-3, rtol=1e-3)  # same math, same order
     assert_close(out, expect, atol=8e-2, rtol=8e-2)
+
+
+@pytest.mark.parametrize("heads,bs,dtype", [
+    (128, 64, torch.bfloat16),
+    (130, 16, torch.bfloat16),
+    (20, 64, torch.float16),
+])
+@pytest.mark.parametrize("bound", [1300, 500, 0])
+def test_mla_prompt_keys_split(heads, bs, dtype, bound):
+    """Few prompt tokens after long contexts: their keys go over
+    partitions, of which some rows fill one, some all, by a bound that is
+    exact, too short (the last partition takes what is left) or missing.
+    Tolerance: queries and keys are exact here, so only the results'
+    rounding and the order of sums are left, of values up to 4."""
+    hip = _hip()
+    q_lens, ctx = [1, 2, 0, 5, 1], [70, 1300, 9, 640, 33]
+    n, T, nb = 5, sum(q_lens), -(-1300 // bs)
+    cache = torch.randn(n * nb, bs, 576, device="cuda", dtype=dtype)
+    bt = torch.randperm(n * nb, device="cuda").int().view(n, nb)
+    qn = torch.randn(T, heads, 512, device="cuda", dtype=dtype)
+    qp = torch.randn(T, heads, 64, device="cuda", dtype=dtype)
+    qsl = torch.tensor([0, 1, 3, 3, 8, 9], device="cuda", dtype=torch.int32)
+    sl = torch.tensor(ctx, device="cuda", dtype=torch.int32)
+    out = hip.mla_attention(qn, qp, cache, bt, qsl, sl, 0.07, num_decodes=1,
+                            max_prompt_len=bound)
+    expect = ref.mla_attention(qn.float(), qp.float(), cache.float(), bt,
+                               qsl, sl, 0.07)
+    atol = 2 * 4 * (2**-8 if dtype == torch.bfloat16 else 2**-11)
+    assert_close(out, expect, atol=atol, rtol=atol / 4)

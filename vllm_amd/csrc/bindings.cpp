@@ -75,7 +75,8 @@ void mla_prompt_attention(torch::Tensor out, torch::Tensor q_nope,
 void mla_prefill(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
                  torch::Tensor kv_cache, torch::Tensor block_table,
                  torch::Tensor query_start_loc, torch::Tensor seq_lens,
-                 double scale, int64_t num_decodes);
+                 double scale, int64_t num_decodes, int64_t max_seq_len,
+                 torch::Tensor tmp_out, torch::Tensor tmp_lse);
 torch::Tensor head_matmul(torch::Tensor x, torch::Tensor w);
 torch::Tensor scalar_rms_norm(torch::Tensor x, torch::Tensor gain,
                               double eps, torch::ScalarType out_dtype);
@@ -232,7 +233,8 @@ TORCH_LIBRARY(vllm_amd, m) {
       "int num_decodes, int max_query_len, int S, Tensor(b!) scratch) -> ()");
   m.def("mla_prefill(Tensor(a!) out, Tensor q_nope, Tensor q_pe, "
         "Tensor kv_cache, Tensor block_table, Tensor query_start_loc, "
-        "Tensor seq_lens, float scale, int num_decodes) -> ()");
+        "Tensor seq_lens, float scale, int num_decodes, int max_seq_len, "
+        "Tensor(b!) tmp_out, Tensor(c!) tmp_lse) -> ()");
   m.def("head_matmul(Tensor x, Tensor w) -> Tensor");
   m.def("scalar_rms_norm(Tensor x, Tensor gain, float eps, "
         "ScalarType out_dtype) -> Tensor");

@@ -33,10 +33,11 @@
 //     2^8. Where they are rounded to 16 (decode), the largest is kept at
 //     one and the rounded weights are summed: 3 % slower, 4 % closer to
 //     64-bit results.
-// Decode rows are split over a few partitions of the keys when there are
-// fewer rows than CUs; fp32 partials (256 KB per row and partition) are
-// merged by mla_reduce_kernel, so partitions are few and long, and rows
-// that fit one are written at once.
+// Rows are split over a few partitions of the keys when there are fewer
+// than CUs; fp32 partials (256 KB per row and partition) are merged by
+// mla_reduce_kernel, so partitions are few and long, and rows that fit one
+// are written at once. A portion of 2 tokens after 8190 takes 56 us in
+// 64 partitions, with the products around it, and 510 in one.
 // 128 heads: 128 rows x 129..2176 keys 1025 -> 88 us with the merge (four
 // waves of 16 heads on 32-key tiles, V stored transposed, before); prompts
 // of 300, 1300 and 2301 tokens 1.32 ms (750 TFLOP/s counting P once; a
@@ -79,12 +80,27 @@ DEVINL int chunk_slot(int row, int c) {
   return c ^ ((((x & 3) ^ ((x >> 2) << 1)) << 1) | (x >> 2));
 }
 
-// One workgroup: (token row, partition of part_len keys, head group).
+// The request of a prompt token: the last one starting at or before its
+// row. Returns how many keys the token sees.
+DEVINL int prompt_keys(int row, const int* __restrict__ query_start_loc,
+                       const int* __restrict__ seq_lens, int num_decodes,
+                       int num_reqs, int& req) {
+  req = num_decodes;
+  for (int end = num_reqs; end - req > 1;) {
+    const int mid = (req + end) / 2;
+    if (query_start_loc[mid] <= row) req = mid;
+    else end = mid;
+  }
+  return seq_lens[req] - (query_start_loc[req + 1] - 1 - row);
+}
+
+// One workgroup: (token row, partition of part_len keys, head group); the
+// last partition takes what is left.
 // PROMPT: blockIdx.x counts the batch's prompt tokens from the last one
 // (the last tokens of a portion have most keys); otherwise blockIdx.x is a
-// decode row and blockIdx.y a partition. SPLIT_P keeps the weights at more than 16 bits
-// (hi + lo parts, two products).
-template <typename Tag, bool PROMPT, bool SPLIT_P>
+// decode row. PARTS: blockIdx.y is a partition. SPLIT_P keeps the weights
+// at more than 16 bits (hi + lo parts, two products).
+template <typename Tag, bool PROMPT, bool SPLIT_P, bool PARTS>
 __launch_bounds__(THREADS, 2) __global__
 void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
                 const short* __restrict__ q_nope,  // [T, Hq, LORA]
@@ -95,28 +111,25 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
                 const int* __restrict__ seq_lens, float scale_log2,
                 int num_heads, int block_size, int num_decodes,
                 int num_reqs,
-                float* __restrict__ tmp_out,  // [T, Hq, parts, LORA]
-                float* __restrict__ tmp_lse,  // [T, Hq, parts, 2]
+                float* __restrict__ tmp_out,  // [rows, Hq, parts, LORA]
+                float* __restrict__ tmp_lse,  // [rows, Hq, parts, 2]
                 int num_parts, int part_len) {
-  int req, row, ctx, part = 0;
+  int req, row, ctx, first = 0;   // first: row 0 of the scratch
   if constexpr (PROMPT) {
     row = query_start_loc[num_reqs] - 1 - (int)blockIdx.x;
-    if (row < query_start_loc[num_decodes]) return;
-    req = num_decodes;              // the last request starting at or before
-    for (int end = num_reqs; end - req > 1;) {
-      const int mid = (req + end) / 2;
-      if (query_start_loc[mid] <= row) req = mid;
-      else end = mid;
-    }
-    ctx = seq_lens[req] - (query_start_loc[req + 1] - 1 - row);
+    first = query_start_loc[num_decodes];
+    if (row < first) return;
+    ctx = prompt_keys(row, query_start_loc, seq_lens, num_decodes, num_reqs,
+                      req);
   } else {
     req = row = blockIdx.x;
-    part = blockIdx.y;
     ctx = seq_lens[req];
   }
   const int hg0 = blockIdx.z * HG;
-  const int t_begin = part * part_len;
-  const int t_end = min(ctx, t_begin + part_len);
+  const int part = PARTS ? blockIdx.y : 0;
+  const int t_begin = PARTS ? part * part_len : 0;
+  const int t_end =
+      PARTS && part + 1 < num_parts ? min(ctx, t_begin + part_len) : ctx;
   if (t_begin >= t_end) {
     if (!PROMPT && part == 0) {   // a row without keys (padding) is zero
       const int n = min(HG, num_heads - hg0) * (LORA / 8);
@@ -281,7 +294,7 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
   l_run += __shfl_xor(l_run, 32, 64);
   if (head >= num_heads) return;
   const int64_t hrow = (int64_t)row * num_heads + head;
-  if (PROMPT || num_parts == 1 || ctx <= part_len) {   // nothing to merge
+  if (!PARTS || num_parts == 1 || ctx <= part_len) {   // nothing to merge
     const float inv_l = 1.f / l_run;
     short* ob = out + hrow * LORA + l4 * 4;
 #pragma unroll
@@ -292,37 +305,51 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
       *reinterpret_cast<int2*>(ob + i * 16) = v;
     }
   } else {
-    float* ob = tmp_out + (hrow * num_parts + part) * LORA + l4 * 4;
+    const int64_t at =
+        ((int64_t)(row - first) * num_heads + head) * num_parts + part;
+    float* ob = tmp_out + at * LORA + l4 * 4;
 #pragma unroll
     for (int i = 0; i < LORA / 16; ++i)
       *reinterpret_cast<f32x4*>(ob + i * 16) = o[i];
     if (l4 == 0) {
-      tmp_lse[(hrow * num_parts + part) * 2] = m_run;
-      tmp_lse[(hrow * num_parts + part) * 2 + 1] = l_run;
+      tmp_lse[at * 2] = m_run;
+      tmp_lse[at * 2 + 1] = l_run;
     }
   }
 }
 
 // Merge partitions: out[s,h,:] = sum_p w_p * tmp[s,h,p,:] / sum_p w_p l_p
 // with w_p = exp2(m_p - m_max). One wave per (row, head), 8 columns each.
-template <typename Tag>
+template <typename Tag, bool PROMPT>
 __launch_bounds__(WAVE_SIZE) __global__
 void mla_reduce_kernel(short* __restrict__ out,
                        const float* __restrict__ tmp_out,
                        const float* __restrict__ tmp_lse,
-                       const int* __restrict__ seq_lens, int num_heads,
-                       int num_parts, int part_len) {
+                       const int* __restrict__ query_start_loc,
+                       const int* __restrict__ seq_lens, int num_decodes,
+                       int num_reqs, int num_heads, int num_parts,
+                       int part_len) {
   const int h = blockIdx.x;
-  const int seq = blockIdx.y;
-  const int parts = min((seq_lens[seq] + part_len - 1) / part_len, num_parts);
+  int row = blockIdx.y, ctx;
+  const int64_t trow = (int64_t)row * num_heads + h;
+  if constexpr (PROMPT) {
+    int req;
+    row += query_start_loc[num_decodes];
+    if (row >= query_start_loc[num_reqs]) return;
+    ctx = prompt_keys(row, query_start_loc, seq_lens, num_decodes, num_reqs,
+                      req);
+  } else {
+    ctx = seq_lens[row];
+  }
+  const int parts = min((ctx + part_len - 1) / part_len, num_parts);
   if (parts <= 1) return;   // the row fits one partition: it is done
-  const int64_t hrow = (int64_t)seq * num_heads + h;
-  const float* lse = tmp_lse + hrow * num_parts * 2;
+  const int64_t hrow = (int64_t)row * num_heads + h;
+  const float* lse = tmp_lse + trow * num_parts * 2;
   float m = NEG;
   for (int p = 0; p < parts; ++p) m = fmaxf(m, lse[p * 2]);
   float l = 0.f;
   f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-  const float* src = tmp_out + hrow * num_parts * LORA + threadIdx.x * 8;
+  const float* src = tmp_out + trow * num_parts * LORA + threadIdx.x * 8;
 #pragma unroll 4
   for (int p = 0; p < parts; ++p) {
     const float w = __builtin_amdgcn_exp2f(lse[p * 2] - m);
@@ -355,10 +382,30 @@ static void check(const torch::Tensor& out, const torch::Tensor& q_nope,
               "mla kernel: bf16/fp16 only");
 }
 
+// Into how many partitions scratch [rows, Hq, parts, 512] and
+// [rows, Hq, parts, 2] splits the keys; empty means one.
+static int parts_of(const torch::Tensor& tmp_out,
+                    const torch::Tensor& tmp_lse, int64_t rows, int64_t Hq) {
+  if (tmp_out.numel() == 0) return 1;
+  TORCH_CHECK(tmp_out.dim() == 4 && tmp_lse.dim() == 4 &&
+              tmp_out.is_contiguous() && tmp_lse.is_contiguous() &&
+              tmp_out.size(0) == rows && tmp_lse.size(0) == rows &&
+              tmp_out.size(1) == Hq && tmp_lse.size(1) == Hq &&
+              tmp_out.size(2) == tmp_lse.size(2) &&
+              tmp_out.size(3) == LORA && tmp_lse.size(3) == 2,
+              "mla scratch must be [rows, Hq, parts, 512] and "
+              "[rows, Hq, parts, 2]");
+  return (int)tmp_out.size(2);
+}
+
+static int part_length(int64_t max_seq_len, int parts) {
+  return ceil_div(ceil_div((int)std::max<int64_t>(max_seq_len, 1), parts),
+                  SUB) * SUB;
+}
+
 }  // namespace mla
 
-// Decode rows. tmp_out [T, Hq, parts, 512] and tmp_lse [T, Hq, parts, 2]
-// say into how many partitions the keys are split; empty means one.
+// Decode rows; the scratch says into how many partitions their keys go.
 void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
                 torch::Tensor kv_cache, torch::Tensor block_table,
                 torch::Tensor seq_lens, double scale, int64_t max_seq_len,
@@ -369,27 +416,14 @@ void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
   if (T == 0) return;
   const int Hq = (int)q_nope.size(1);
   const int bs = (int)kv_cache.size(1);
-  int parts = 1;
-  if (tmp_out.numel() > 0) {
-    TORCH_CHECK(tmp_out.dim() == 4 && tmp_lse.dim() == 4 &&
-                tmp_out.is_contiguous() && tmp_lse.is_contiguous() &&
-                tmp_out.size(0) == T && tmp_lse.size(0) == T &&
-                tmp_out.size(1) == Hq && tmp_lse.size(1) == Hq &&
-                tmp_out.size(2) == tmp_lse.size(2) &&
-                tmp_out.size(3) == LORA && tmp_lse.size(3) == 2,
-                "mla scratch must be [T, Hq, parts, 512] and "
-                "[T, Hq, parts, 2]");
-    parts = (int)tmp_out.size(2);
-  }
-  const int part_len =
-      ceil_div(ceil_div((int)std::max<int64_t>(max_seq_len, 1), parts), SUB) *
-      SUB;
+  const int parts = parts_of(tmp_out, tmp_lse, T, Hq);
+  const int part_len = part_length(max_seq_len, parts);
   auto stream = c10::hip::getCurrentHIPStream().stream();
   dim3 grid(T, parts, ceil_div(Hq, HG));
   auto launch = [&](auto tag) {
     using Tag = decltype(tag);
     hipLaunchKernelGGL(
-        (mla_kernel<Tag, false, false>), grid, dim3(THREADS), 0, stream,
+        (mla_kernel<Tag, false, false, true>), grid, dim3(THREADS), 0, stream,
         (short*)out.data_ptr(), (const short*)q_nope.data_ptr(),
         (const short*)q_pe.data_ptr(), (const short*)kv_cache.data_ptr(),
         block_table.data_ptr<int>(), (int)block_table.size(1), nullptr,
@@ -398,10 +432,11 @@ void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
         parts > 1 ? tmp_lse.data_ptr<float>() : nullptr, parts, part_len);
     if (parts > 1) {
       HIP_CHECK_KERNEL();
-      hipLaunchKernelGGL((mla_reduce_kernel<Tag>), dim3(Hq, T),
+      hipLaunchKernelGGL((mla_reduce_kernel<Tag, false>), dim3(Hq, T),
                          dim3(WAVE_SIZE), 0, stream, (short*)out.data_ptr(),
                          tmp_out.data_ptr<float>(), tmp_lse.data_ptr<float>(),
-                         seq_lens.data_ptr<int>(), Hq, parts, part_len);
+                         nullptr, seq_lens.data_ptr<int>(), T, T, Hq, parts,
+                         part_len);
     }
   };
   if (q_nope.scalar_type() == torch::kBFloat16) launch(BF16Tag{});
@@ -410,11 +445,12 @@ void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
 }
 
 // Prompt portions: requests num_decodes.. of the batch; q/out cover the
-// whole step.
+// whole step, the scratch the prompt tokens.
 void mla_prefill(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
                  torch::Tensor kv_cache, torch::Tensor block_table,
                  torch::Tensor query_start_loc, torch::Tensor seq_lens,
-                 double scale, int64_t num_decodes) {
+                 double scale, int64_t num_decodes, int64_t max_seq_len,
+                 torch::Tensor tmp_out, torch::Tensor tmp_lse) {
   using namespace mla;
   check(out, q_nope, q_pe, kv_cache);
   const int reqs = (int)seq_lens.size(0);
@@ -423,20 +459,37 @@ void mla_prefill(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
   TORCH_CHECK(query_start_loc.numel() > reqs);
   const int Hq = (int)q_nope.size(1);
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  dim3 grid(rows, 1, ceil_div(Hq, HG));
-  auto launch = [&](auto tag) {
+  const int parts = parts_of(tmp_out, tmp_lse, rows, Hq);
+  const int part_len = part_length(max_seq_len, parts);
+  dim3 grid(rows, parts, ceil_div(Hq, HG));
+  auto launch = [&](auto tag, auto split) {
     using Tag = decltype(tag);
+    constexpr bool PARTS = decltype(split)::value;
     hipLaunchKernelGGL(
-        (mla_kernel<Tag, true, true>), grid, dim3(THREADS), 0, stream,
+        (mla_kernel<Tag, true, true, PARTS>), grid, dim3(THREADS), 0, stream,
         (short*)out.data_ptr(), (const short*)q_nope.data_ptr(),
         (const short*)q_pe.data_ptr(), (const short*)kv_cache.data_ptr(),
         block_table.data_ptr<int>(), (int)block_table.size(1),
         query_start_loc.data_ptr<int>(), seq_lens.data_ptr<int>(),
         (float)scale * 1.4426950408889634f, Hq, (int)kv_cache.size(1),
-        (int)num_decodes, reqs, nullptr, nullptr, 1, 0x7fffff00);
+        (int)num_decodes, reqs, PARTS ? tmp_out.data_ptr<float>() : nullptr,
+        PARTS ? tmp_lse.data_ptr<float>() : nullptr, parts, part_len);
+    if constexpr (PARTS) {
+      HIP_CHECK_KERNEL();
+      hipLaunchKernelGGL((mla_reduce_kernel<Tag, true>), dim3(Hq, rows),
+                         dim3(WAVE_SIZE), 0, stream, (short*)out.data_ptr(),
+                         tmp_out.data_ptr<float>(), tmp_lse.data_ptr<float>(),
+                         query_start_loc.data_ptr<int>(),
+                         seq_lens.data_ptr<int>(), (int)num_decodes, reqs, Hq,
+                         parts, part_len);
+    }
   };
-  if (q_nope.scalar_type() == torch::kBFloat16) launch(BF16Tag{});
-  else launch(FP16Tag{});
+  auto by_parts = [&](auto tag) {
+    if (parts > 1) launch(tag, std::true_type{});
+    else           launch(tag, std::false_type{});
+  };
+  if (q_nope.scalar_type() == torch::kBFloat16) by_parts(BF16Tag{});
+  else by_parts(FP16Tag{});
   HIP_CHECK_KERNEL();
 }
 

@@ -253,6 +253,18 @@ def _mla_parts(rows, heads, max_seq_len):
                       -(-max_seq_len // _MLA_PART_MIN), 64))
 
 
+def _mla_scratch(q, max_seq_len):
+    """Partials of the partitions of q's rows [T, Hq, lora]; empty for one
+    partition."""
+    T, Hq, lora = q.shape
+    parts = _mla_parts(T, Hq, max_seq_len)
+    if parts == 1:
+        none = q.new_empty(0, dtype=torch.float32)
+        return none, none
+    return (q.new_empty(T, Hq, parts, lora, dtype=torch.float32),
+            q.new_empty(T, Hq, parts, 2, dtype=torch.float32))
+
+
 def mla_decode(q_nope, q_pe, kv_cache, block_table, seq_lens, scale,
                max_seq_len):
     """Absorbed-MQA MLA decode on the MFMA kernel (csrc/mla.hip);
@@ -261,25 +273,18 @@ def mla_decode(q_nope, q_pe, kv_cache, block_table, seq_lens, scale,
     out = torch.empty(T, Hq, lora, dtype=q_nope.dtype, device=q_nope.device)
     if max_seq_len <= 0:
         max_seq_len = int(seq_lens.max().item())
-    parts = _mla_parts(T, Hq, max_seq_len)
-    if parts > 1:
-        tmp_out = torch.empty(T, Hq, parts, lora, dtype=torch.float32,
-                              device=q_nope.device)
-        tmp_lse = torch.empty(T, Hq, parts, 2, dtype=torch.float32,
-                              device=q_nope.device)
-    else:
-        tmp_out = q_nope.new_empty(0, dtype=torch.float32)
-        tmp_lse = tmp_out
     _C.mla_decode(out, q_nope, q_pe, kv_cache, block_table, seq_lens,
-                  scale, max_seq_len, tmp_out, tmp_lse)
+                  scale, max_seq_len, *_mla_scratch(q_nope, max_seq_len))
     return out
 
 
 def mla_attention(q_nope, q_pe, kv_cache, block_table, query_start_loc,
-                  seq_lens, scale, num_decodes=0, max_seq_len=0):
+                  seq_lens, scale, num_decodes=0, max_seq_len=0,
+                  max_prompt_len=0):
     """Decode rows (query_len==1, first num_decodes) and prompt rows on
     the MFMA kernel (csrc/mla.hip). Other latent widths, types or cache
-    types take the torch composition."""
+    types take the torch composition. max_prompt_len bounds the prompts'
+    contexts (0: max_seq_len does, or they are not split)."""
     T = q_nope.shape[0]
     use_hip = (q_nope.shape[2] == 512 and q_pe.shape[2] == 64
                and q_nope.dtype in (torch.bfloat16, torch.float16)
@@ -298,8 +303,10 @@ def mla_attention(q_nope, q_pe, kv_cache, block_table, query_start_loc,
         out[:num_decodes] = mla_decode(
             q_nope[:num_decodes], q_pe[:num_decodes], kv_cache,
             block_table, seq_lens[:num_decodes], scale, max_seq_len)
+    bound = max_prompt_len or max_seq_len
     _C.mla_prefill(out, q_nope, q_pe, kv_cache, block_table,
-                   query_start_loc, seq_lens, scale, num_decodes)
+                   query_start_loc, seq_lens, scale, num_decodes, bound,
+                   *_mla_scratch(q_nope[num_decodes:], bound))
     return out
 
 
@@ -349,20 +356,24 @@ def _mla_prompt_heads(q_nope, w_uk, w_uv, kv_cache, reqs, scale,
     values carried out of the latent space (csrc/mla_prompt.hip); 0:
     in it (csrc/mla.hip). Carrying them out costs by context row, the
     latent form by query (a part for each and a part per key; 200 at
-    least, which fill the chip), so the line is a number of queries per
-    request that grows with the context. us per head / latent, 8 requests:
-    96 tokens of 512 256 / 260, 128 266 / 345; 192 of 2048 1174 / 1130, 256
-    of 4096 2433 / 2660; 32 requests: 32 of 128 272 / 251, 64 of 256 505 /
-    547; one: 128 of 2048 147 / 164, 64 of 8192 563 / 515. Only the longest
-    context is known here: shorter ones cost less than this says, most so
-    per head."""
+    least, which fill the chip, or 256 pieces of queries whose keys are
+    split), so the line is a number of queries per request that grows with
+    the context. us per head / latent, 8 requests: 96 tokens of 512 260 /
+    261, 128 267 / 342; 192 of 2048 1233 / 1181, 256 of 4096 2492 / 2786;
+    32 requests: 32 of 128 265 / 242, 64 of 256 521 / 552; one: 64 of 512
+    54 / 62, 128 of 2048 150 / 136, 160 154 / 175, 192 of 8192 655 / 623,
+    256 629 / 692. Only the longest context is known here: shorter ones
+    cost less than this says, most so per head."""
     T, Hq, nope = q_nope.shape
     rows, reqs = T - num_decodes, reqs - num_decodes
     S = max(max_seq_len, 128)
+    parts = _mla_parts(rows, Hq, S)
+    cost = (max(rows, 200) * (800 + S) if parts == 1 else
+            256 * (800 + S // parts))
     if (nope != 128 or w_uk.shape[2] != 512 or w_uv.shape[2] != 128
             or kv_cache.shape[2] != 576 or scale <= 0 or max_query_len <= 0
             or max_seq_len <= 0 or not 0 < reqs < 65536 or rows <= 0
-            or max(rows, 200) * (800 + S) < reqs * 255 * S
+            or cost < reqs * 255 * S
             or q_nope.dtype not in (torch.bfloat16, torch.float16)
             or any(t.dtype != q_nope.dtype for t in (w_uk, w_uv, kv_cache))
             or not all(t.is_contiguous() for t in (w_uk, w_uv, kv_cache))
@@ -393,7 +404,8 @@ def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
         o = mla_attention(head_matmul(q_nope[:n], w_uk), q_pe[:n], kv_cache,
                           block_table[:reqs], query_start_loc[:reqs + 1],
                           seq_lens[:reqs], scale, num_decodes=num_decodes,
-                          max_seq_len=max_decode_len or max_seq_len)
+                          max_seq_len=max_decode_len or max_seq_len,
+                          max_prompt_len=max_prompt_len or max_seq_len)
         return head_matmul(o, w_uv)
 
     S = max_prompt_len or max_seq_len
