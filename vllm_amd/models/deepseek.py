@@ -96,10 +96,27 @@ class DeepseekMLAAttention(nn.Module):
         self._join_a_projs()
         return self
 
+    def _joined_a_projs(self):
+        """The weights of the two projections of the hidden state as one
+        matrix, or None where they do not lie one behind the other in one
+        storage."""
+        q, kv = self.q_a_proj.weight, self.kv_a_proj_with_mqa.weight
+        if (q.numel() == 0 or kv.numel() == 0 or q.dtype != kv.dtype
+                or q.device != kv.device
+                or not q.is_contiguous() or not kv.is_contiguous()
+                or q.untyped_storage().data_ptr()
+                != kv.untyped_storage().data_ptr()
+                or kv.storage_offset() != q.storage_offset() + q.numel()):
+            return None
+        n, k = q.shape
+        return torch.as_strided(q, (n + kv.shape[0], k), (k, 1))
+
     def _join_a_projs(self) -> None:
         """Lays the weights of the two projections of the hidden state one
-        behind the other, so that _a_projs can take them as one matrix."""
-        if self.q_a_proj is None:
+        behind the other, so that _a_projs can take them as one matrix.
+        Weights that lie so already stay where they are: a move that
+        changes nothing leaves captured graphs and shared memory valid."""
+        if self.q_a_proj is None or self._joined_a_projs() is not None:
             return
         q, kv = self.q_a_proj.weight, self.kv_a_proj_with_mqa.weight
         if q.numel() == 0 or q.dtype != kv.dtype or q.device != kv.device:
@@ -112,17 +129,12 @@ class DeepseekMLAAttention(nn.Module):
         their weights lie one behind the other in one storage (us for 1536
         + 576 rows of 7168, apart / as one: 1 token 20.7 / 10.6, 128 30.8 /
         22.7, 3901 132 / 102, 8192 215 / 218)."""
-        q, kv = self.q_a_proj.weight, self.kv_a_proj_with_mqa.weight
-        if (hidden.is_cuda and hidden.shape[0] <= 4096 and q.numel() > 0
-                and kv.numel() > 0 and q.dtype == kv.dtype
-                and q.is_contiguous() and kv.is_contiguous()
-                and q.untyped_storage().data_ptr()
-                == kv.untyped_storage().data_ptr()
-                and kv.storage_offset() == q.storage_offset() + q.numel()):
-            n, k = q.shape
-            both = torch.as_strided(q, (n + kv.shape[0], k), (k, 1))
-            return ops.linear(hidden, both).split([n, kv.shape[0]], dim=1)
-        return self.q_a_proj(hidden), self.kv_a_proj_with_mqa(hidden)
+        both = (self._joined_a_projs()
+                if hidden.is_cuda and hidden.shape[0] <= 4096 else None)
+        if both is None:
+            return self.q_a_proj(hidden), self.kv_a_proj_with_mqa(hidden)
+        n = self.q_a_proj.weight.shape[0]
+        return ops.linear(hidden, both).split([n, both.shape[0] - n], dim=1)
 
     def load_kv_b_proj(self, kv_b_weight: torch.Tensor) -> None:
         """kv_b_proj.weight [Hq*(nope+v), lora] (full) -> absorbed splits
