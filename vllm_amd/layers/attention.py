@@ -12,6 +12,7 @@ import torch
 import torch.nn as nn
 
 from vllm_amd import ops
+from vllm_amd.layers.hooks import hooked
 from vllm_amd.worker.forward_context import get_forward_context
 
 
@@ -59,12 +60,13 @@ class Attention(nn.Module):
         if v.dim() == 2:
             v = v.view(T, self.num_kv_heads, self.head_dim)
 
+        if rotary is not None and (not ctx.kv_caches or hooked(rotary[1])):
+            rotary[1](rotary[0], q, k)
+            rotary = None
         if not ctx.kv_caches:
             # Memory-profiling run: no cache allocated; compute attention
             # over just the new tokens (worst-case activation footprint is
             # what matters, not values).
-            if rotary is not None:
-                rotary[1](rotary[0], q, k)
             return self._profile_attention(q, k, v, meta).reshape(T, -1)
 
         kv_cache = ctx.kv_caches[self.layer_idx]

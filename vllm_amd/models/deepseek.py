@@ -33,6 +33,7 @@ from vllm_amd.layers.linear import (
     ReplicatedLinear,
     RowParallelLinear,
 )
+from vllm_amd.layers.hooks import hooked
 from vllm_amd.layers.rotary import RotaryEmbedding
 from vllm_amd.parallel.state import get_tp_world_size
 from vllm_amd.worker.forward_context import get_forward_context
@@ -129,11 +130,14 @@ class DeepseekMLAAttention(nn.Module):
         their weights lie one behind the other in one storage (us for 1536
         + 576 rows of 7168, apart / as one: 1 token 20.7 / 10.6, 128 30.8 /
         22.7, 3901 132 / 102, 8192 215 / 218)."""
-        both = (self._joined_a_projs()
-                if hidden.is_cuda and hidden.shape[0] <= 4096 else None)
+        q, kv = self.q_a_proj, self.kv_a_proj_with_mqa
+        both = None
+        if (hidden.is_cuda and hidden.shape[0] <= 4096 and q.bias is None
+                and kv.bias is None and not hooked(q, kv)):
+            both = self._joined_a_projs()
         if both is None:
-            return self.q_a_proj(hidden), self.kv_a_proj_with_mqa(hidden)
-        n = self.q_a_proj.weight.shape[0]
+            return q(hidden), kv(hidden)
+        n = q.weight.shape[0]
         return ops.linear(hidden, both).split([n, both.shape[0] - n], dim=1)
 
     def load_kv_b_proj(self, kv_b_weight: torch.Tensor) -> None:
@@ -149,6 +153,15 @@ class DeepseekMLAAttention(nn.Module):
         self.w_uk.data.copy_(w[:, : self.qk_nope])
         self.w_uv.data.copy_(w[:, self.qk_nope:].transpose(1, 2))
 
+    def _prepare(self, positions, q_pe, kv_a):
+        """The normalized latent and the rotated parts of queries and keys,
+        module by module."""
+        c_kv = self.kv_a_layernorm(kv_a[:, : self.kv_lora].contiguous())
+        q_pe = q_pe.contiguous()
+        k_pe = kv_a[:, self.kv_lora:].unsqueeze(1).contiguous()
+        self.rotary_emb(positions, q_pe, k_pe)
+        return c_kv, q_pe, k_pe.squeeze(1)
+
     def forward(self, positions, hidden):
         T = hidden.shape[0]
         if self.q_a_proj is not None:
@@ -163,20 +176,21 @@ class DeepseekMLAAttention(nn.Module):
         ctx = get_forward_context()
         meta = ctx.attn_metadata
         if not ctx.kv_caches:
-            c_kv = self.kv_a_layernorm(kv_a[:, : self.kv_lora].contiguous())
-            q_pe = q_pe.contiguous()
-            k_pe = kv_a[:, self.kv_lora:].unsqueeze(1).contiguous()
-            self.rotary_emb(positions, q_pe, k_pe)
+            c_kv, q_pe, k_pe = self._prepare(positions, q_pe, kv_a)
             o_c = self._profile_attention(
-                ops.head_matmul(q_nope, self.w_uk), q_pe, c_kv,
-                k_pe.squeeze(1), meta)
+                ops.head_matmul(q_nope, self.w_uk), q_pe, c_kv, k_pe, meta)
             out = ops.head_matmul(o_c, self.w_uv)
         else:
             kv_cache = ctx.kv_caches[self.layer_idx]
-            q_pe = ops.mla_prepare(
-                positions, q_pe, kv_a, self.kv_a_layernorm.weight,
-                self.kv_a_layernorm.eps, self.rotary_emb.cos_sin_cache,
-                kv_cache, meta.slot_mapping)
+            if hooked(self.kv_a_layernorm, self.rotary_emb):
+                c_kv, q_pe, k_pe = self._prepare(positions, q_pe, kv_a)
+                ops.concat_and_cache_mla(c_kv, k_pe, kv_cache,
+                                         meta.slot_mapping)
+            else:
+                q_pe = ops.mla_prepare(
+                    positions, q_pe, kv_a, self.kv_a_layernorm.weight,
+                    self.kv_a_layernorm.eps, self.rotary_emb.cos_sin_cache,
+                    kv_cache, meta.slot_mapping)
             out = ops.mla_heads(
                 q_nope, q_pe, self.w_uk, self.w_uv, kv_cache,
                 meta.block_table, meta.query_start_loc, meta.seq_lens,
