@@ -81,6 +81,32 @@ def test_mla_decode_split_ignores_prompts(hip, rows, monkeypatch):
     assert split(8192) == split(0)
 
 
+@pytest.mark.parametrize("tokens,topk,E,H,form", [
+    (64, 8, 64, 7168, 0),      # one streamed tile holds any expert's rows
+    (65, 8, 64, 7168, 1),      # no longer
+    (767, 8, 256, 7168, 1),
+    (95, 2, 8, 4096, 0),       # 8 x 16 tiles leave half the chip idle
+    (96, 2, 8, 4096, 1),
+    (500, 1, 128, 2048, 0),    # below 4 rows an expert
+    (512, 1, 128, 2048, 1),
+    (1536, 8, 64, 7168, 2),
+])
+def test_expert_form(hip, tokens, topk, E, H, form):
+    """Where rows may meet in few experts the weights are not streamed
+    once per 64 of them."""
+    I = 64
+    w13 = torch.empty(E, 2 * I, 1).expand(E, 2 * I, H)
+    w2 = torch.empty(E, H, 1).expand(E, H, I)
+    rows = (64, 128, 256)[form]
+    hip._C.moe_tile_rows = lambda f: (64, 128, 256)[f]
+    hip.fused_moe_hip(torch.empty(tokens, H, dtype=torch.bfloat16), w13, w2,
+                      torch.empty(tokens, topk),
+                      torch.zeros(tokens, topk, dtype=torch.int32))
+    gemms = hip._C.args("moe_gemm")
+    assert [a[8] for a in gemms] == [form, form]
+    assert hip._C.args("moe_align")[0][2] == rows
+
+
 def test_runner_tells_lengths(monkeypatch):
     """The runner's mixed steps say how long their decode rows are, and
     how long their prompts' contexts."""

@@ -435,6 +435,31 @@ def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
 # 4.21 / 1.79 / 1.79, 512 rows 10.2 / 3.70 / 3.20.
 _MOE_TILES_FROM = 24
 _MOE_WIDE_TILES_FROM = 192
+# The average says little where rows meet in few experts (equal prompts,
+# padded rows of a captured step): weights of an expert with more than 64
+# rows are streamed once per 64. So tiles also from 4 rows an expert where
+# an expert may get more than 64 (the batch holds more tokens) and one tile
+# per expert fills the chip. us streamed / 128, experts chosen evenly | by
+# half of the tokens | all the same: 64 experts of 7168 x 2048, 8 a token,
+# 80 tokens 1018 / 993 | 1023 / 985 | 350 / 201, 191 tokens 1177 / 1018 |
+# 1255 / 1005 | 526 / 225; 256 experts, 767 tokens 4591 / 3890 | 4916 /
+# 4004 | 1854 / 679; 128 of 2048 x 768, 65 tokens 237 / 238 | 216 / 219 |
+# 67 / 60. Not filled: 8 experts of 4096 x 14336, 2 a token, 65 tokens 530 /
+# 555 | 559 / 562 | 400 / 312. Fewer than 4: 128 of 2048 x 768, 1 a token,
+# 192 tokens 188 / 204 | 145 / 148 | 55 / 58.
+_MOE_STREAM_ROWS = 64
+_MOE_CHIP_TILES = 256
+
+
+def _moe_form(tokens, total, E, H):
+    """0 streamed, 1 and 2 tiles of 128 and 256 rows, for total (token,
+    expert) pairs of tokens rows of H, no pair twice."""
+    if total >= _MOE_WIDE_TILES_FROM * E:
+        return 2
+    if total >= _MOE_TILES_FROM * E:
+        return 1
+    return int(tokens > _MOE_STREAM_ROWS and total >= 4 * E
+               and E * -(-H // 256) >= _MOE_CHIP_TILES)
 
 
 def _moe_hip_ok(hidden, w13, w2, activation):
@@ -477,8 +502,7 @@ def fused_moe_hip(hidden, w13, w2, topk_weights, topk_ids,
     k = topk_ids.shape[1]
     total = T * k
     dev = hidden.device
-    form = (0 if total < _MOE_TILES_FROM * E else
-            1 if total < _MOE_WIDE_TILES_FROM * E else 2)
+    form = _moe_form(T, total, E, H)
     if max(T * H, (total + E * 256) * I, n1 * H) >= 1 << 31:
         form = 0    # tiles address 4 GB
     if form > 0:    # (they take the weights in their own order)
