@@ -904,3 +904,46 @@ def test_mla_prompt_keys_split(heads, bs, dtype, bound):
                                qsl, sl, 0.07)
     atol = 2 * 4 * (2**-8 if dtype == torch.bfloat16 else 2**-11)
     assert_close(out, expect, atol=atol, rtol=atol / 4)
+
+
+@pytest.mark.parametrize("T", [40, 1100])  # one block of rows, two
+def test_moe_more_experts_than_lds_counters(T):
+    """More experts than LDS counters take the same path, captured too:
+    no synchronisation, each replay gives the eager bytes. Every row's
+    result against its two experts in 64 bits, within three roundings to
+    bf16 (2^-8 each) of sums of magnitudes."""
+    hip = _hip()
+    E, H, I, K = 1500, 128, 64, 2
+    bf = torch.bfloat16
+    x = torch.randn(T, H, device="cuda", dtype=bf)
+    w13 = torch.randn(E, 2 * I, H, device="cuda", dtype=bf) * H**-0.5
+    w2 = torch.randn(E, H, I, device="cuda", dtype=bf) * I**-0.5
+    assert hip._moe_hip_ok(x, w13, w2, "silu")
+    ids = torch.stack([torch.randperm(E, device="cuda")[:K]
+                       for _ in range(T)]).int()
+    ids[: T // 2, 0], ids[: T // 2, 1] = E - 1, 3
+    w = torch.rand(T, K, device="cuda")
+    out = hip.fused_moe(x, w13, w2, w, ids)
+    y = torch.matmul(w13[ids.long()].double(), x.double()[:, None, :, None])
+    a = torch.nn.functional.silu(y[:, :, :I]) * y[:, :, I:]
+    w2d, wd = w2[ids.long()].double(), w.double()[..., None, None]
+    terms = torch.matmul(w2d, a) * wd
+    bound = (torch.matmul(w2d.abs(), a.abs()) * wd).sum(1) + terms.abs().sum(1)
+    expect = terms.sum(1)
+    err = (out.double()[..., None] - expect).abs()
+    assert (err <= 1.1 * 2**-8 * (bound + expect.abs()) + 2**-20).all()
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        hip.fused_moe(x, w13, w2, w, ids)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        again = hip.fused_moe(x, w13, w2, w, ids)
+    for _ in range(3):
+        again.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(again, out)
+        assert torch.equal(hip.fused_moe(x, w13, w2, w, ids), out)

@@ -41,14 +41,15 @@ namespace moe {
 constexpr int BM = 64;    // token rows per tile of the few-row kernels
 constexpr int THREADS = 256;
 constexpr int SENTINEL = 0x7fffffff;
-constexpr int MAX_EXPERTS = 1024;
+constexpr int LDS_EXPERTS = 1024;   // whose counters fit LDS
 
 // --------------------------------------------------------------------------
 // Alignment. Counting and placing with one atomic per row on global
 // counters costs 113 us at 32768 rows (every row of an expert waits for
 // the one before); counters in LDS, one set per block of 2048 rows, and a
 // prefix over the blocks cost 29 us. Up to 2048 rows one workgroup does it
-// all in one launch (four before).
+// all in one launch (four before). Counters of more than 1024 experts
+// (LDS false) are in the scratch instead, one set per block all the same.
 constexpr int ALIGN_ROWS = 2048;   // rows per block
 
 // counts[e] -> off[e] = first row of expert e in tile order, and what the
@@ -82,11 +83,14 @@ DEVINL void place_experts(const int* counts, int* off, int e, int bm,
   __syncthreads();
 }
 
+template <bool LDS>
 __global__ __launch_bounds__(THREADS) void align_small_kernel(
     const int* __restrict__ ids, int total, int e, int bm,
     int* __restrict__ expert_tiles, int max_tiles, int* __restrict__ sorted,
-    int* __restrict__ inv_perm) {
-  __shared__ int counts[MAX_EXPERTS], off[MAX_EXPERTS], scan[THREADS];
+    int* __restrict__ inv_perm, int* counters) {
+  __shared__ int lds[LDS ? 2 * LDS_EXPERTS : 1], scan[THREADS];
+  int* counts = LDS ? lds : counters;
+  int* off = counts + (LDS ? LDS_EXPERTS : e);
   for (int i = threadIdx.x; i < e; i += THREADS) counts[i] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < total; i += THREADS)
@@ -101,24 +105,32 @@ __global__ __launch_bounds__(THREADS) void align_small_kernel(
 }
 
 // part[b][e]: rows of expert e in block b.
+template <bool LDS>
 __global__ __launch_bounds__(THREADS) void align_count_kernel(
-    const int* __restrict__ ids, int total, int e, int* __restrict__ part) {
-  __shared__ int counts[MAX_EXPERTS];
+    const int* __restrict__ ids, int total, int e, int* part) {
+  __shared__ int lds[LDS ? LDS_EXPERTS : 1];
+  int* counts = LDS ? lds : part + (int64_t)blockIdx.x * e;
   for (int i = threadIdx.x; i < e; i += THREADS) counts[i] = 0;
   __syncthreads();
   const int end = min(total, ((int)blockIdx.x + 1) * ALIGN_ROWS);
   for (int i = blockIdx.x * ALIGN_ROWS + threadIdx.x; i < end; i += THREADS)
     atomicAdd(&counts[ids[i]], 1);
-  __syncthreads();
-  for (int i = threadIdx.x; i < e; i += THREADS)
-    part[(int64_t)blockIdx.x * e + i] = counts[i];
+  if constexpr (LDS) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < e; i += THREADS)
+      part[(int64_t)blockIdx.x * e + i] = counts[i];
+  }
 }
 
 // part[b][e] -> first row of block b's rows of expert e.
+template <bool LDS>
 __global__ __launch_bounds__(THREADS) void align_place_kernel(
     int* __restrict__ part, int blocks, int e, int bm,
-    int* __restrict__ expert_tiles, int max_tiles, int* __restrict__ sorted) {
-  __shared__ int counts[MAX_EXPERTS], off[MAX_EXPERTS], scan[THREADS];
+    int* __restrict__ expert_tiles, int max_tiles, int* __restrict__ sorted,
+    int* counters) {
+  __shared__ int lds[LDS ? 2 * LDS_EXPERTS : 1], scan[THREADS];
+  int* counts = LDS ? lds : counters;
+  int* off = counts + (LDS ? LDS_EXPERTS : e);
   for (int i = threadIdx.x; i < e; i += THREADS) {
     int n = 0;
     for (int b = 0; b < blocks; ++b) n += part[(int64_t)b * e + i];
@@ -136,14 +148,17 @@ __global__ __launch_bounds__(THREADS) void align_place_kernel(
   }
 }
 
+template <bool LDS>
 __global__ __launch_bounds__(THREADS) void align_scatter_kernel(
-    const int* __restrict__ ids, int total, int e,
-    const int* __restrict__ part, int* __restrict__ sorted,
-    int* __restrict__ inv_perm) {
-  __shared__ int off[MAX_EXPERTS];
-  for (int i = threadIdx.x; i < e; i += THREADS)
-    off[i] = part[(int64_t)blockIdx.x * e + i];
-  __syncthreads();
+    const int* __restrict__ ids, int total, int e, int* part,
+    int* __restrict__ sorted, int* __restrict__ inv_perm) {
+  __shared__ int lds[LDS ? LDS_EXPERTS : 1];
+  int* off = LDS ? lds : part + (int64_t)blockIdx.x * e;
+  if constexpr (LDS) {
+    for (int i = threadIdx.x; i < e; i += THREADS)
+      off[i] = part[(int64_t)blockIdx.x * e + i];
+    __syncthreads();
+  }
   const int end = min(total, ((int)blockIdx.x + 1) * ALIGN_ROWS);
   for (int i = blockIdx.x * ALIGN_ROWS + threadIdx.x; i < end; i += THREADS) {
     const int pos = atomicAdd(&off[ids[i]], 1);
@@ -713,7 +728,8 @@ int64_t moe_tile_rows(int64_t form) {
   return form == 2 ? 256 : form == 1 ? 128 : moe::BM;
 }
 
-// scratch: ceil(total / 2048) * num_experts ints where total > 2048.
+// scratch: ceil(total / 2048) * num_experts ints where total > 2048, and
+// 2 * num_experts more for more than 1024 experts.
 void moe_align(torch::Tensor topk_ids, int64_t num_experts, int64_t tile_rows,
                torch::Tensor sorted, torch::Tensor expert_tiles,
                torch::Tensor inv_perm, torch::Tensor scratch) {
@@ -724,8 +740,7 @@ void moe_align(torch::Tensor topk_ids, int64_t num_experts, int64_t tile_rows,
   const int e = (int)num_experts;
   const int bm = (int)tile_rows;
   const int max_tiles = (int)expert_tiles.numel() - 1;
-  TORCH_CHECK(e >= 1 && e <= MAX_EXPERTS, "moe_align: 1..", MAX_EXPERTS,
-              " experts, got ", e);
+  TORCH_CHECK(e >= 1, "moe_align: no experts");
   TORCH_CHECK(bm >= 1 && sorted.numel() >= (int64_t)max_tiles * bm &&
               (int64_t)max_tiles * bm >=
                   total + (int64_t)std::min(e, total) * (bm - 1) - (bm - 1));
@@ -734,24 +749,33 @@ void moe_align(torch::Tensor topk_ids, int64_t num_experts, int64_t tile_rows,
   const int blocks = ceil_div(total, ALIGN_ROWS);
   auto stream = c10::hip::getCurrentHIPStream().stream();
   const int* ids = topk_ids.data_ptr<int>();
-  if (blocks == 1) {
-    hipLaunchKernelGGL(align_small_kernel, dim3(1), dim3(THREADS), 0, stream,
-                       ids, total, e, bm, expert_tiles.data_ptr<int>(),
-                       max_tiles, sorted.data_ptr<int>(),
-                       inv_perm.data_ptr<int>());
-  } else {
-    TORCH_CHECK(scratch.scalar_type() == torch::kInt32 &&
-                scratch.numel() >= (int64_t)blocks * e);
-    int* part = scratch.data_ptr<int>();
-    hipLaunchKernelGGL(align_count_kernel, dim3(blocks), dim3(THREADS), 0,
-                       stream, ids, total, e, part);
-    hipLaunchKernelGGL(align_place_kernel, dim3(1), dim3(THREADS), 0, stream,
-                       part, blocks, e, bm, expert_tiles.data_ptr<int>(),
-                       max_tiles, sorted.data_ptr<int>());
-    hipLaunchKernelGGL(align_scatter_kernel, dim3(blocks), dim3(THREADS), 0,
-                       stream, ids, total, e, part, sorted.data_ptr<int>(),
-                       inv_perm.data_ptr<int>());
-  }
+  const int64_t parts = blocks > 1 ? (int64_t)blocks * e : 0;
+  TORCH_CHECK(scratch.scalar_type() == torch::kInt32 &&
+              scratch.is_contiguous() &&
+              scratch.numel() >= parts + (e > LDS_EXPERTS ? 2 * e : 0));
+  int* part = scratch.data_ptr<int>();
+  auto launch = [&](auto in_lds) {
+    constexpr bool LDS = decltype(in_lds)::value;
+    if (blocks == 1) {
+      hipLaunchKernelGGL(align_small_kernel<LDS>, dim3(1), dim3(THREADS), 0,
+                         stream, ids, total, e, bm,
+                         expert_tiles.data_ptr<int>(), max_tiles,
+                         sorted.data_ptr<int>(), inv_perm.data_ptr<int>(),
+                         part);
+      return;
+    }
+    hipLaunchKernelGGL(align_count_kernel<LDS>, dim3(blocks), dim3(THREADS),
+                       0, stream, ids, total, e, part);
+    hipLaunchKernelGGL(align_place_kernel<LDS>, dim3(1), dim3(THREADS), 0,
+                       stream, part, blocks, e, bm,
+                       expert_tiles.data_ptr<int>(), max_tiles,
+                       sorted.data_ptr<int>(), part + parts);
+    hipLaunchKernelGGL(align_scatter_kernel<LDS>, dim3(blocks),
+                       dim3(THREADS), 0, stream, ids, total, e, part,
+                       sorted.data_ptr<int>(), inv_perm.data_ptr<int>());
+  };
+  if (e <= LDS_EXPERTS) launch(std::true_type{});
+  else                  launch(std::false_type{});
   HIP_CHECK_KERNEL();
 }
 

@@ -467,8 +467,6 @@ def _moe_hip_ok(hidden, w13, w2, activation):
         return False
     if hidden.dtype not in (torch.bfloat16, torch.float16):
         return False
-    if w13.shape[0] > 1024:  # moe_align's counters are in LDS
-        return False
     H = hidden.shape[1]
     n1 = w13.shape[1]
     if activation == "relu2":
@@ -513,7 +511,8 @@ def fused_moe_hip(hidden, w13, w2, topk_weights, topk_ids,
     ids32 = topk_ids.to(torch.int32).contiguous()
     blocks = -(-total // 2048)
     scratch = torch.empty(
-        em + tiles + 1 + total + (blocks * E if blocks > 1 else 0),
+        em + tiles + 1 + total + (blocks * E if blocks > 1 else 0)
+        + (2 * E if E > 1024 else 0),
         dtype=torch.int32, device=dev)
     sorted_ids, expert_tiles, inv_perm, part = scratch.split(
         [em, tiles + 1, total, scratch.numel() - em - tiles - 1 - total])
