@@ -907,6 +907,7 @@ def test_mla_prompt_keys_split(heads, bs, dtype, bound):
 
 
 @pytest.mark.parametrize("T", [40, 1100])  # one block of rows, two
+@torch.inference_mode()   # as the runner captures
 def test_moe_more_experts_than_lds_counters(T):
     """More experts than LDS counters take the same path, captured too:
     no synchronisation, each replay gives the eager bytes. Every row's
