@@ -451,13 +451,10 @@ DEVINL void tile_body(char* lds, const short* __restrict__ A, int64_t lda,
                       int64_t ldc, const int* __restrict__ sorted, int K,
                       int N, int topk_div, int row0, int rows, int n0) {
   constexpr int TL_M = WM * 64;
-  constexpr int TL_STAGES = WM == 4 ? 2 : 3;
   constexpr int TL_WN = 8 / WM;            // waves along the weight rows
   constexpr int TL_WW = TL_W / TL_WN;      // weight rows of a wave
   constexpr int TL_WI = TL_WW / 32;
   constexpr int TL_MI = 2;                 // 32-row groups of a wave
-  constexpr int TL_STAGE = (TL_M + TL_W) * TL_ROW;   // bytes
-  static_assert(TL_STAGES * TL_STAGE <= TL_LDS);
   constexpr int TL_FA = TL_M / TL_FR / 8;  // fills per wave
   constexpr int TL_FW = TL_W / TL_FR / 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
@@ -498,10 +495,6 @@ DEVINL void tile_body(char* lds, const short* __restrict__ A, int64_t lda,
     for (int i = 0; i < TL_FW; ++i)
       lds_fill16(W + step * TL_K, wp[i], dst + (wave * TL_FW + i) * 1024);
   };
-  auto fill = [&](int step, int stage) {
-    fill_a(step, lds + stage * TL_STAGE);
-    fill_w(step, lds + stage * TL_STAGE + TL_M * TL_ROW);
-  };
 
   f32x16 acc[TL_WI][TL_MI];
 #pragma unroll
@@ -530,6 +523,7 @@ DEVINL void tile_body(char* lds, const short* __restrict__ A, int64_t lda,
     // accumulators of several branches would copy them.
     const int lag = wave >> 2;
     constexpr int AB = TL_M * TL_ROW, WB = TL_W * TL_ROW;
+    static_assert(2 * AB + 3 * WB <= TL_LDS);
     const char* a0 = lds + wm * TL_MI * 32 * TL_ROW;
     const char* w0 = lds + 2 * AB + wn * TL_WW * TL_ROW;
     auto run = [&](auto n) {
@@ -598,6 +592,13 @@ DEVINL void tile_body(char* lds, const short* __restrict__ A, int64_t lda,
     else if (groups == 1) run(std::integral_constant<int, 1>{});
     else run(std::integral_constant<int, 0>{});
   } else {
+    constexpr int TL_STAGES = 3;
+    constexpr int TL_STAGE = (TL_M + TL_W) * TL_ROW;   // bytes
+    static_assert(TL_STAGES * TL_STAGE <= TL_LDS);
+    auto fill = [&](int step, int stage) {
+      fill_a(step, lds + stage * TL_STAGE);
+      fill_w(step, lds + stage * TL_STAGE + TL_M * TL_ROW);
+    };
 #pragma unroll
     for (int i = 0; i < TL_STAGES - 1; ++i)
       if (i < steps) fill(i, i);
@@ -605,7 +606,7 @@ DEVINL void tile_body(char* lds, const short* __restrict__ A, int64_t lda,
     for (int s = 0; s < steps; ++s) {
       // This stage has landed when at most the next one's fills are under
       // way; past the barrier every wave is done with the stage before.
-      if (TL_STAGES > 2 && s + 1 < steps) lds_fill_wait<TL_FA + TL_FW>();
+      if (s + 1 < steps) lds_fill_wait<TL_FA + TL_FW>();
       else lds_fill_wait();
       lds_barrier();
       if (s + TL_STAGES - 1 < steps)
