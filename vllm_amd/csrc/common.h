@@ -1,6 +1,6 @@
 // Common device helpers for vllm_amd CDNA4 (gfx950) kernels.
 //
-// Written for MI355X only: wave64, 32-bank LDS, MFMA matrix cores,
+// Written for MI355X only: wave64, 64-bank LDS, MFMA matrix cores,
 // HBM3E. No CUDA-compat paths.
 #pragma once
 
@@ -72,10 +72,6 @@ template <> DEVINL short from_f32<FP16Tag>(float f) { return f16_from_f32(f); }
 // v_cvt_pk_fp8_f32, RNE) — the software bit manipulation this replaced
 // cost ~20 VALU ops per element and made the fp8-KV decode kernel
 // conversion-bound instead of HBM-bound.
-DEVINL float fp8_e4m3_to_f32(uint8_t v) {
-  return __builtin_amdgcn_cvt_f32_fp8((uint32_t)v, 0);
-}
-
 DEVINL uint8_t f32_to_fp8_e4m3(float f) {
   union { float f; uint32_t u; } c;
   c.f = f;
@@ -87,11 +83,6 @@ DEVINL uint8_t f32_to_fp8_e4m3(float f) {
   return (uint8_t)__builtin_amdgcn_cvt_pk_fp8_f32(cl, cl, 0, false);
 }
 
-// Packed pair converts for vectorized cache reads: 2 elements/instr.
-DEVINL f32x2 fp8x2_e4m3_to_f32x2(uint16_t v2) {
-  return __builtin_amdgcn_cvt_pk_f32_fp8((uint32_t)v2, false);
-}
-
 // Cache element traits: the KV cache may be narrower than the compute
 // dtype. vec8 loads 8 cache elements (16 B bf16/fp16, 8 B fp8).
 typedef uint8_t u8x8 __attribute__((ext_vector_type(8)));
@@ -101,19 +92,16 @@ template <typename CTag> struct CacheTraits;
 template <> struct CacheTraits<BF16Tag> {
   using elem = short;
   using vec8 = s16x8;
-  static DEVINL float get(vec8 v, int j) { return bf16_to_f32(v[j]); }
   static DEVINL elem put(float f) { return f32_to_bf16(f); }
 };
 template <> struct CacheTraits<FP16Tag> {
   using elem = short;
   using vec8 = s16x8;
-  static DEVINL float get(vec8 v, int j) { return f16_to_f32(v[j]); }
   static DEVINL elem put(float f) { return f16_from_f32(f); }
 };
 template <> struct CacheTraits<FP8CacheTag> {
   using elem = uint8_t;
   using vec8 = u8x8;
-  static DEVINL float get(vec8 v, int j) { return fp8_e4m3_to_f32(v[j]); }
   static DEVINL elem put(float f) { return f32_to_fp8_e4m3(f); }
 };
 
