@@ -22,8 +22,9 @@
 // Against the vector-ALU form it replaced (16 lanes per token, dot
 // products reduced with shuffles), us per layer at 32 query and 8 KV
 // heads of 128:
-//   1 x 1000 keys 46 -> 13; 256 x 129..2176 keys 346 -> 227 (5.3 TB/s);
-//   1024 x 129..176 keys 215 -> 128 (5.0 TB/s);
+//   1 x 1000 keys 46 -> 13; 256 x 129..2176 keys 349 -> 228 (5.3 TB/s);
+//   1024 x 129..176 keys 206 -> 124 (5.2 TB/s; 132 with the last 32 keys
+//   of a row read whole);
 //   64 x 4096..8192 keys, fp8 cache 371 -> 154 (5.2 TB/s).
 //
 // The KV cache layout [2, blocks, kv_heads, block_size=64, D] keeps each
@@ -144,19 +145,28 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
            (key0 & 63) * HD;
   };
   i32x4 kr[2][KN], vr[VN];
-  auto load_k = [&](const elem* tile) {
+  // Rows of a step that the row does not attend repeat the nearest one it
+  // does: they cost no bytes.
+  auto load_k = [&](const elem* tile, int key0) {
+    const int lo = t_lo - key0, hi = t_end - 1 - key0;
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+    for (int s = 0; s < 2; ++s) {
+      const int r = min(max(s * 16 + l16, lo), hi);
 #pragma unroll
       for (int i = 0; i < KN; ++i)
         kr[s][i] = *reinterpret_cast<const i32x4*>(
-            tile + (s * 16 + l16) * HD + (i * 4 + l4) * EPV);
+            tile + r * HD + (i * 4 + l4) * EPV);
+    }
   };
-  auto load_v = [&](const elem* tile) {
+  auto load_v = [&](const elem* tile, int key0) {
+    const int lo = t_lo - key0, hi = t_end - 1 - key0;
 #pragma unroll
-    for (int i = 0; i < VN; ++i)
-      vr[i] = *reinterpret_cast<const i32x4*>(
-          tile + kv_plane_stride + (i * WAVE_SIZE + lane) * EPV);
+    for (int i = 0; i < VN; ++i) {
+      const int e = (i * WAVE_SIZE + lane) * EPV;
+      const int r = min(max(e / HD, lo), hi);
+      vr[i] = *reinterpret_cast<const i32x4*>(tile + kv_plane_stride +
+                                              r * HD + e % HD);
+    }
   };
 
   float m_run = DEC_NEG, l_run = 0.f;   // of head l16; l: this lane's keys
@@ -190,7 +200,7 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
         s[t] = mfma16<Tag>(a, qf[kk], s[t]);
       }
     }
-    if constexpr (NEXT) load_k(next_tile);
+    if constexpr (NEXT) load_k(next_tile, key0 + DEC_WAVES * DEC_KEYS);
 
     // ---- V to LDS, rows outside [t_lo, t_end) as zeros ------------------
     // (a stale cache row may hold anything, and 0 * NaN is NaN).
@@ -221,7 +231,7 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
         *reinterpret_cast<i32x4*>(dst + (c16 & 1) * 16) = v;
       }
     }
-    if constexpr (NEXT) load_v(next_tile);
+    if constexpr (NEXT) load_v(next_tile, key0 + DEC_WAVES * DEC_KEYS);
 
     // ---- running softmax, log2 domain ----------------------------------
     // A key outside the row's range scores DEC_NEG and weighs nothing
@@ -289,8 +299,8 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
   int key0 = t_begin + wave * DEC_KEYS;
   if (key0 < t_end) {
     const elem* tile = tile_of(key0);
-    load_k(tile);
-    load_v(tile);
+    load_k(tile, key0);
+    load_v(tile, key0);
     for (; key0 + DEC_WAVES * DEC_KEYS < t_end; key0 += DEC_WAVES * DEC_KEYS)
       step(key0, std::true_type{});
     step(key0, std::false_type{});
