@@ -176,6 +176,45 @@ def test_decode_attention_edges(hd, group, dtype, cache_dtype, window, n):
     assert_close(out[rows], expect, atol=atol, rtol=atol / 4)
 
 
+def _check_decode_rows(n, lens, Hkv, group, hd, dtype, cache_dtype, window,
+                       bound=0):
+    """Rows of the given lengths in turn against fp32, unwritten rows of
+    their last block NaN. Tolerance: the output's own rounding, 2^-8
+    (bf16) or 2^-11 (fp16) of values up to 4, once more for the order of
+    sums."""
+    hip = _hip()
+    ctx = [lens[i % len(lens)] for i in range(n)]
+    q, cache, bt, qsl, sl = _make_paged(n, [1] * n, ctx, Hkv * group, Hkv,
+                                        D=hd)
+    q, cache = q.to(dtype), cache.to(cache_dtype)
+    raw = cache if cache_dtype != torch.float8_e4m3fn \
+        else cache.view(torch.uint8)
+    rows = sorted({*range(len(lens)), n - 1})
+    for i in rows:
+        if ctx[i] % 64:
+            raw[:, bt[i, ctx[i] // 64], :, ctx[i] % 64:] = \
+                float("nan") if raw is cache else 0x7F
+    out = hip.attention_unified(q, cache, bt, qsl, sl, hd**-0.5,
+                                num_decodes=n,
+                                max_seq_len=bound or max(ctx),
+                                max_query_len=1, sliding_window=window)
+    expect = ref.attention_unified(
+        q[rows].float(), cache.float(), bt[rows], qsl[:len(rows) + 1],
+        sl[rows], hd**-0.5, num_decodes=len(rows), sliding_window=window)
+    atol = 2 * 4 * (2**-8 if dtype == torch.bfloat16 else 2**-11)
+    assert_close(out[rows], expect, atol=atol, rtol=atol / 4)
+
+
+@pytest.mark.parametrize("dtype,group,window", [
+    (torch.bfloat16, 3, 0), (torch.float16, 8, 0), (torch.bfloat16, 1, 33)])
+@pytest.mark.parametrize("n", [7, 300])  # split and unsplit keys
+def test_decode_attention_16_key_steps(dtype, group, window, n):
+    """Heads of 256 take 16 keys a step: rows around 16 keys, a
+    workgroup's 64 and a cache block."""
+    _check_decode_rows(n, [1, 15, 17, 63, 65, 128, 641], 2, group, 256,
+                       dtype, dtype, window)
+
+
 @pytest.mark.parametrize("n,longest", [(300, 700), (3, 700), (300, 90)])
 def test_decode_rows_without_keys(n, longest):
     """A row of length 0 (a captured step's padding) gives exact zeros,

@@ -4,9 +4,10 @@
 // flops per byte everything else only has to stay out of the way of the
 // loads, so the kernel keeps as many bytes in flight as registers allow
 // and spends few issue slots per byte:
-//   - A wave owns 32 keys at a time and never meets another wave before
-//     the end, so there is no barrier in the loop. The next 32 keys are
-//     loaded as soon as the registers of the current ones are free.
+//   - A wave owns 32 keys at a time (16 where rows are 512 B) and never
+//     meets another wave before the end, so there is no barrier in the
+//     loop. The next keys are loaded as soon as the registers of the
+//     current ones are free.
 //   - Scores are S^T = K Q^T on the matrix cores: a K row goes from HBM
 //     straight into the A fragment (16 B per lane), the query heads of
 //     the group are the 16 columns. No cross-lane sum per key and head,
@@ -41,7 +42,7 @@ namespace vllm_amd {
 
 constexpr int DEC_WAVES = 4;
 constexpr int DEC_BLOCK = DEC_WAVES * WAVE_SIZE;
-constexpr int DEC_KEYS = 32;    // keys per wave and step
+constexpr int DEC_KEYS = 32;    // keys per wave and step, at most
 constexpr int MAX_GROUP = 8;    // query heads per KV head
 constexpr float DEC_NEG = -3.0e38f;
 constexpr float DEC_LOG2E = 1.4426950408889634f;
@@ -54,6 +55,18 @@ template <int HD> DEVINL int v_slot(int row, int seg) {
   return seg ^ (row & 7);
 }
 
+// Keys per wave and step. 32 rows of 512 B each for keys and values, the
+// queries and 16 x 256 outputs are more registers than the two workgroups
+// of a CU have (340; one workgroup then, values moved between register
+// files): 16 a step instead takes 228. us: 16 x 750..1500 keys, 16 KV heads
+// 58 -> 53, 64 x 300..3000 (4) 102 -> 98, 256 x 150..300 through a window of
+// 128 (16, three query heads each) 146 -> 102. At 128 columns 16 keys are no
+// faster for long rows (256 x 129..2176 228 -> 231).
+template <typename CTag, int HD>
+constexpr int dec_keys =
+    HD == 256 && sizeof(typename CacheTraits<CTag>::elem) == 2 ? 16
+                                                               : DEC_KEYS;
+
 // First key this row attends, rounded down so that a wave's 32 keys
 // never leave a cache block.
 DEVINL int dec_base(int ctx, int window) {
@@ -64,7 +77,7 @@ DEVINL int dec_base(int ctx, int window) {
 // Writes the final 16-bit output (FINAL) or fp32 partials with their
 // running maximum (log2 domain) and sum.
 template <typename Tag, typename CTag, bool FINAL, int HD>
-__global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
+__global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
     short* __restrict__ out,            // FINAL: [Tdec, Hq, D] (16-bit)
     float* __restrict__ tmp_out,        // else: [Tdec, Hq, parts, D]
     float* __restrict__ tmp_lse,        // else: [Tdec, Hq, parts, 2]
@@ -81,11 +94,13 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
   using elem = typename CacheTraits<CTag>::elem;
   constexpr bool FP8 = sizeof(elem) == 1;
   constexpr int EPV = 16 / sizeof(elem);          // elements per 16 B
+  constexpr int KEYS = dec_keys<CTag, HD>;
+  constexpr int KT = KEYS / 16;                   // score tiles
   constexpr int KF = HD / 32;                     // MFMA steps over D
   constexpr int KN = HD * (int)sizeof(elem) / 64; // 16 B K loads per row
-  constexpr int VN = DEC_KEYS * HD / EPV / WAVE_SIZE;
+  constexpr int VN = KEYS * HD / EPV / WAVE_SIZE;
   constexpr int DS = HD / 16;                     // output column tiles
-  constexpr int V_BYTES = DEC_KEYS * HD * 2;      // per wave
+  constexpr int V_BYTES = KEYS * HD * 2;          // per wave
 
   const int kvh = blockIdx.x;
   const int seq = blockIdx.y;       // decode row == request row
@@ -144,13 +159,13 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
            ((int64_t)bt[key0 >> 6] * num_kv_heads + kvh) * (64 * HD) +
            (key0 & 63) * HD;
   };
-  i32x4 kr[2][KN], vr[VN];
+  i32x4 kr[KT][KN], vr[VN];
   // Rows of a step that the row does not attend repeat the nearest one it
   // does: they cost no bytes.
   auto load_k = [&](const elem* tile, int key0) {
     const int lo = t_lo - key0, hi = t_end - 1 - key0;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
+    for (int s = 0; s < KT; ++s) {
       const int r = min(max(s * 16 + l16, lo), hi);
 #pragma unroll
       for (int i = 0; i < KN; ++i)
@@ -174,17 +189,18 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
 #pragma unroll
   for (int i = 0; i < DS; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // One step of 32 keys; with NEXT the loads of the wave's next 32 are
+  // One step of KEYS keys; with NEXT the loads of the wave's next ones are
   // issued as the registers become free (a template flag and not a test
   // inside, so that the waits count exactly the older loads).
+  constexpr int STRIDE = DEC_WAVES * KEYS;
   auto step = [&](int key0, auto has_next) {
     constexpr bool NEXT = decltype(has_next)::value;
     const elem* next_tile =
-        NEXT ? tile_of(key0 + DEC_WAVES * DEC_KEYS) : nullptr;
+        NEXT ? tile_of(key0 + STRIDE) : nullptr;
     // ---- S^T: rows are keys, columns heads -----------------------------
-    f32x4 s[2];
+    f32x4 s[KT];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < KT; ++t) {
       s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kk = 0; kk < KF; ++kk) {
@@ -200,11 +216,11 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
         s[t] = mfma16<Tag>(a, qf[kk], s[t]);
       }
     }
-    if constexpr (NEXT) load_k(next_tile, key0 + DEC_WAVES * DEC_KEYS);
+    if constexpr (NEXT) load_k(next_tile, key0 + STRIDE);
 
     // ---- V to LDS, rows outside [t_lo, t_end) as zeros ------------------
     // (a stale cache row may hold anything, and 0 * NaN is NaN).
-    const bool edge = key0 < t_lo || key0 + DEC_KEYS > t_end;
+    const bool edge = key0 < t_lo || key0 + KEYS > t_end;
     if (edge) {
 #pragma unroll
       for (int i = 0; i < VN; ++i) {
@@ -231,15 +247,15 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
         *reinterpret_cast<i32x4*>(dst + (c16 & 1) * 16) = v;
       }
     }
-    if constexpr (NEXT) load_v(next_tile, key0 + DEC_WAVES * DEC_KEYS);
+    if constexpr (NEXT) load_v(next_tile, key0 + STRIDE);
 
     // ---- running softmax, log2 domain ----------------------------------
     // A key outside the row's range scores DEC_NEG and weighs nothing
     // even where the whole step is outside it.
-    bool in[2][4];
+    bool in[KT][4];
     float mx = DEC_NEG;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < KT; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int key = key0 + t * 16 + l4 * 4 + r;
@@ -257,9 +273,9 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
       for (int i = 0; i < DS; ++i) o[i] *= f;
       m_run = m_new;
     }
-    i32x4 hi, lo;
+    i32x4 hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < KT; ++t)
 #pragma unroll
       for (int r = 0; r < 4; r += 2) {
         const float e0 = __builtin_amdgcn_exp2f(s[t][r] - m_run);
@@ -286,6 +302,13 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
       const int off = (l16 & 3) * 8;
       const s16x4 a = lds_read_tr(v_lds + row * (HD * 2) +
                                   v_slot<HD>(row, i) * 32 + off);
+      if constexpr (KT == 1) {
+        o[i] = mfma16<Tag>(a, __builtin_shufflevector(p_lo, p_lo, 0, 1, 2, 3),
+                           o[i]);
+        o[i] = mfma16<Tag>(a, __builtin_shufflevector(p_hi, p_hi, 0, 1, 2, 3),
+                           o[i]);
+        continue;
+      }
       const s16x4 b = lds_read_tr(v_lds + (row + 16) * (HD * 2) +
                                   v_slot<HD>(row + 16, i) * 32 + off);
       const s16x8 v = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -296,12 +319,12 @@ __global__ __launch_bounds__(DEC_BLOCK) void paged_decode_kernel(
     __builtin_amdgcn_wave_barrier();
   };
 
-  int key0 = t_begin + wave * DEC_KEYS;
+  int key0 = t_begin + wave * KEYS;
   if (key0 < t_end) {
     const elem* tile = tile_of(key0);
     load_k(tile, key0);
     load_v(tile, key0);
-    for (; key0 + DEC_WAVES * DEC_KEYS < t_end; key0 += DEC_WAVES * DEC_KEYS)
+    for (; key0 + STRIDE < t_end; key0 += STRIDE)
       step(key0, std::true_type{});
     step(key0, std::false_type{});
   }

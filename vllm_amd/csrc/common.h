@@ -113,6 +113,7 @@ template <> struct CacheTraits<FP8CacheTag> {
 typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
 
 template <typename Tag> DEVINL f32x4 mfma16(s16x8 a, s16x8 b, f32x4 c);
@@ -123,6 +124,15 @@ template <> DEVINL f32x4 mfma16<BF16Tag>(s16x8 a, s16x8 b, f32x4 c) {
 template <> DEVINL f32x4 mfma16<FP16Tag>(s16x8 a, s16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(
       __builtin_bit_cast(h16x8, a), __builtin_bit_cast(h16x8, b), c, 0, 0, 0);
+}
+// The same over 16 instead of 32.
+template <typename Tag> DEVINL f32x4 mfma16(s16x4 a, s16x4 b, f32x4 c);
+template <> DEVINL f32x4 mfma16<BF16Tag>(s16x4 a, s16x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+}
+template <> DEVINL f32x4 mfma16<FP16Tag>(s16x4 a, s16x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16f16(
+      __builtin_bit_cast(h16x4, a), __builtin_bit_cast(h16x4, b), c, 0, 0, 0);
 }
 template <typename Tag> DEVINL f32x16 mfma32(s16x8 a, s16x8 b, f32x16 c);
 template <> DEVINL f32x16 mfma32<BF16Tag>(s16x8 a, s16x8 b, f32x16 c) {
