@@ -215,6 +215,40 @@ def test_decode_attention_16_key_steps(dtype, group, window, n):
                        dtype, dtype, window)
 
 
+@pytest.mark.parametrize("hd,group,dtype,cache_dtype,window,bound", [
+    (128, 4, torch.bfloat16, torch.bfloat16, 0, 0),
+    (128, 7, torch.float16, torch.float8_e4m3fn, 40, 0),
+    (64, 8, torch.bfloat16, torch.bfloat16, 0, 512),
+    (64, 1, torch.float16, torch.float16, 33, 0),
+    (256, 2, torch.bfloat16, torch.bfloat16, 0, 0),
+    (256, 3, torch.bfloat16, torch.float8_e4m3fn, 17, 0),
+    (128, 2, torch.bfloat16, torch.bfloat16, 0, 512),
+])
+def test_decode_attention_wave_rows(hd, group, dtype, cache_dtype, window,
+                                    bound):
+    """Many short rows, a wave each: rows around the steps of 16 and 32
+    keys, a number of rows that is no multiple of a workgroup's four, a
+    bound far above the rows as a captured step has."""
+    lens = [1, 15, 16, 17, 31, 33, 64, 127, 128, 97]
+    if bound:
+        lens += [129, 480, 512]
+    _check_decode_rows(2063 if bound else 803, lens, 2, group, hd, dtype,
+                       cache_dtype, window, bound)
+
+
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_decode_wave_rows_without_keys(hd):
+    hip = _hip()
+    n = 801
+    q, cache, bt, qsl, sl = _make_paged(n, [1] * n, [40] * n, 8, 2, D=hd)
+    sl[1::2] = 0
+    junk = torch.full_like(q, float("nan"))
+    del junk
+    out = hip.attention_unified(q, cache, bt, qsl, sl, 0.1, num_decodes=n,
+                                max_seq_len=40, max_query_len=1)
+    assert (out[1::2] == 0).all() and out[::2].isfinite().all()
+
+
 @pytest.mark.parametrize("n,longest", [(300, 700), (3, 700), (300, 90)])
 def test_decode_rows_without_keys(n, longest):
     """A row of length 0 (a captured step's padding) gives exact zeros,

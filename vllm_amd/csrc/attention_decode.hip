@@ -73,10 +73,12 @@ DEVINL int dec_base(int ctx, int window) {
   return window > 0 ? (max(0, ctx - window) & ~(DEC_KEYS - 1)) : 0;
 }
 
-// One workgroup: (kv head, decode row, partition of part_len keys).
-// Writes the final 16-bit output (FINAL) or fp32 partials with their
-// running maximum (log2 domain) and sum.
-template <typename Tag, typename CTag, bool FINAL, int HD>
+// WPR 4: one workgroup is (kv head, decode row, partition of part_len
+// keys) and a wave takes every fourth step of them. WPR 1: a wave is a row
+// of its own, whole, for batches of short rows. Writes the final 16-bit
+// output (FINAL) or fp32 partials with their running maximum (log2 domain)
+// and sum.
+template <typename Tag, typename CTag, bool FINAL, int HD, int WPR>
 __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
     short* __restrict__ out,            // FINAL: [Tdec, Hq, D] (16-bit)
     float* __restrict__ tmp_out,        // else: [Tdec, Hq, parts, D]
@@ -87,10 +89,12 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
     const int* __restrict__ block_table,   // [num_reqs, max_blocks]
     const int* __restrict__ seq_lens,      // [num_reqs]
     const float scale_log2, const int group, const int num_kv_heads,
-    const int max_blocks_per_req, const int num_parts, const int part_len,
+    const int num_seqs, const int max_blocks_per_req, const int num_parts,
+    const int part_len,
     const int64_t kv_plane_stride,      // elements between K and V planes
     const int64_t q_stride,             // elements between q token rows
     const int sliding_window) {
+  static_assert(WPR == DEC_WAVES || (WPR == 1 && FINAL));
   using elem = typename CacheTraits<CTag>::elem;
   constexpr bool FP8 = sizeof(elem) == 1;
   constexpr int EPV = 16 / sizeof(elem);          // elements per 16 B
@@ -102,9 +106,13 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
   constexpr int DS = HD / 16;                     // output column tiles
   constexpr int V_BYTES = KEYS * HD * 2;          // per wave
 
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lane = threadIdx.x % WAVE_SIZE;
   const int kvh = blockIdx.x;
-  const int seq = blockIdx.y;       // decode row == request row
-  const int part = blockIdx.z;
+  // Decode row == request row.
+  const int seq = WPR > 1 ? blockIdx.y : blockIdx.y * DEC_WAVES + wave;
+  if (WPR == 1 && seq >= num_seqs) return;   // (no barrier below then)
+  const int part = WPR > 1 ? blockIdx.z : 0;
   const int ctx = seq_lens[seq];
   const int num_q_heads = num_kv_heads * group;
   const int hq0 = kvh * group;
@@ -115,7 +123,8 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
   if (t_begin >= t_end) {
     // A row without keys (padding) is zero, also where nothing merges it.
     if constexpr (FINAL)
-      for (int e = threadIdx.x; e < group * HD; e += DEC_BLOCK)
+      for (int e = WPR > 1 ? threadIdx.x : lane; e < group * HD;
+           e += WPR * WAVE_SIZE)
         out[((int64_t)seq * num_q_heads + hq0) * HD + e] = 0;
     if (!FINAL && threadIdx.x < group * 2) {
       const int g = threadIdx.x / 2;
@@ -126,8 +135,6 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
     return;
   }
 
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
-  const int lane = threadIdx.x % WAVE_SIZE;
   const int l16 = lane & 15;
   const int l4 = lane >> 4;
 
@@ -192,7 +199,7 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
   // One step of KEYS keys; with NEXT the loads of the wave's next ones are
   // issued as the registers become free (a template flag and not a test
   // inside, so that the waits count exactly the older loads).
-  constexpr int STRIDE = DEC_WAVES * KEYS;
+  constexpr int STRIDE = WPR * KEYS;
   auto step = [&](int key0, auto has_next) {
     constexpr bool NEXT = decltype(has_next)::value;
     const elem* next_tile =
@@ -319,7 +326,7 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
     __builtin_amdgcn_wave_barrier();
   };
 
-  int key0 = t_begin + wave * KEYS;
+  int key0 = t_begin + (WPR > 1 ? wave * KEYS : 0);
   if (key0 < t_end) {
     const elem* tile = tile_of(key0);
     load_k(tile, key0);
@@ -332,6 +339,21 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
   // ---- merge the waves ----------------------------------------------------
   l_run += __shfl_xor(l_run, 16, 64);
   l_run += __shfl_xor(l_run, 32, 64);
+  if constexpr (WPR == 1) {   // nothing to merge
+    const float inv_l = l_run > 0.f || l_run != l_run ? 1.f / l_run : 0.f;
+    if (l16 < group) {
+      short* ob =
+          out + ((int64_t)seq * num_q_heads + hq0 + l16) * HD + l4 * 4;
+#pragma unroll
+      for (int i = 0; i < DS; ++i) {
+        int2 v;
+        v.x = pack2<Tag>(o[i][0] * inv_l, o[i][1] * inv_l);
+        v.y = pack2<Tag>(o[i][2] * inv_l, o[i][3] * inv_l);
+        *reinterpret_cast<int2*>(ob + i * 16) = v;
+      }
+    }
+    return;
+  }
   __syncthreads();   // every wave is done with its V slice
   float* o_red = reinterpret_cast<float*>(lds);  // [wave][MAX_GROUP][HD]
   static_assert(MAX_GROUP * HD * 4 <= V_BYTES, "merge scratch");
@@ -476,22 +498,38 @@ void paged_decode_attention(torch::Tensor out, torch::Tensor q,
   const float scale_log2 = (float)scale * DEC_LOG2E;
   auto stream = c10::hip::getCurrentHIPStream().stream();
 
-  dim3 grid(num_kv_heads, num_seqs, num_parts);
+  // Rows of a few steps leave three of a workgroup's four waves idle, and
+  // starting and merging it costs more than its keys: from half the waves
+  // that run at a time on, each takes a row of at most 128 keys of its own;
+  // of up to 512 (the least that a captured step is told) where rows fill
+  // the chip twice over. us, workgroup / wave a row, 32/8 heads of 128: 1024
+  // rows x 1..32 keys 49 / 20, 33..64 56 / 35, 129..176 125 / 121, 512 377 /
+  // 378; 128 x 1..128 11.1 / 9.3; 64 x 128 7.6 / 8.8, 512 x 1..512 104 / 106.
+  // Heads of 256: 512 x 128 97.6 / 99.3, 1..128 49 / 45, 1..512 195 / 207.
+  const int64_t units = (int64_t)num_seqs * num_kv_heads;
+  const bool wave_rows =
+      num_parts == 1 &&
+      ((span <= 128 && units >= (head_dim == 64 ? 1536 : 1024)) ||
+       (span <= 512 && units >= 4096 && head_dim <= 128));
+  const dim3 grid(num_kv_heads,
+                  wave_rows ? ceil_div(num_seqs, DEC_WAVES) : num_seqs,
+                  num_parts);
 
-  auto launch = [&](auto tag, auto ctag, auto dim, auto fin) {
+  auto launch = [&](auto tag, auto ctag, auto dim, auto fin, auto wpr) {
     using Tag = decltype(tag);
     using CTag = decltype(ctag);
     constexpr int HD = decltype(dim)::value;
     constexpr bool FINAL = decltype(fin)::value;
+    constexpr int WPR = decltype(wpr)::value;
     hipLaunchKernelGGL(
-        (paged_decode_kernel<Tag, CTag, FINAL, HD>), grid, dim3(DEC_BLOCK),
-        0, stream, (short*)out.data_ptr(),
+        (paged_decode_kernel<Tag, CTag, FINAL, HD, WPR>), grid,
+        dim3(DEC_BLOCK), 0, stream, (short*)out.data_ptr(),
         FINAL ? nullptr : tmp_out.data_ptr<float>(),
         FINAL ? nullptr : tmp_lse.data_ptr<float>(),
         (const short*)q.data_ptr(),
         (const typename CacheTraits<CTag>::elem*)kv_cache.data_ptr(),
         block_table.data_ptr<int>(), seq_lens.data_ptr<int>(), scale_log2,
-        group, num_kv_heads, max_blocks, num_parts, part_len,
+        group, num_kv_heads, num_seqs, max_blocks, num_parts, part_len,
         kv_cache.stride(0), q.stride(0), (int)sliding_window);
     if constexpr (!FINAL) {
       HIP_CHECK_KERNEL();
@@ -503,26 +541,29 @@ void paged_decode_attention(torch::Tensor out, torch::Tensor q,
           (int)sliding_window);
     }
   };
-  auto by_dim = [&](auto tag, auto ctag, auto fin) {
+  auto by_dim = [&](auto tag, auto ctag, auto fin, auto wpr) {
     if (head_dim == 64)
-      launch(tag, ctag, std::integral_constant<int, 64>{}, fin);
+      launch(tag, ctag, std::integral_constant<int, 64>{}, fin, wpr);
     else if (head_dim == 128)
-      launch(tag, ctag, std::integral_constant<int, 128>{}, fin);
+      launch(tag, ctag, std::integral_constant<int, 128>{}, fin, wpr);
     else
-      launch(tag, ctag, std::integral_constant<int, 256>{}, fin);
+      launch(tag, ctag, std::integral_constant<int, 256>{}, fin, wpr);
   };
   const bool fp8c = kv_cache.scalar_type() == torch::kFloat8_e4m3fn;
-  auto by_type = [&](auto fin) {
+  auto by_type = [&](auto fin, auto wpr) {
     if (q.scalar_type() == torch::kBFloat16) {
-      if (fp8c) by_dim(BF16Tag{}, FP8CacheTag{}, fin);
-      else      by_dim(BF16Tag{}, BF16Tag{}, fin);
+      if (fp8c) by_dim(BF16Tag{}, FP8CacheTag{}, fin, wpr);
+      else      by_dim(BF16Tag{}, BF16Tag{}, fin, wpr);
     } else {
-      if (fp8c) by_dim(FP16Tag{}, FP8CacheTag{}, fin);
-      else      by_dim(FP16Tag{}, FP16Tag{}, fin);
+      if (fp8c) by_dim(FP16Tag{}, FP8CacheTag{}, fin, wpr);
+      else      by_dim(FP16Tag{}, FP16Tag{}, fin, wpr);
     }
   };
-  if (num_parts == 1) by_type(std::true_type{});
-  else                by_type(std::false_type{});
+  using one = std::integral_constant<int, 1>;
+  using four = std::integral_constant<int, DEC_WAVES>;
+  if (wave_rows)           by_type(std::true_type{}, one{});
+  else if (num_parts == 1) by_type(std::true_type{}, four{});
+  else                     by_type(std::false_type{}, four{});
   HIP_CHECK_KERNEL();
 }
 
