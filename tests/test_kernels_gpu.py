@@ -1021,3 +1021,74 @@ def test_moe_more_experts_than_lds_counters(T):
         torch.cuda.synchronize()
         assert torch.equal(again, out)
         assert torch.equal(hip.fused_moe(x, w13, w2, w, ids), out)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_mla_prompt_key_ranges(dtype):
+    """Keys outside fp16's range, far below one, or of very different size
+    in the two halves of a head or in neighbouring blocks of tokens, with
+    queries that make up for it: the powers of two cancel, so tolerances
+    are those of ordinary heads (test_mla_heads)."""
+    hip = _hip()
+    n, H = 300, 8
+    cache = torch.randn(5, 64, 576, device="cuda", dtype=dtype)
+    bt = torch.randperm(5, device="cuda").int()[None]
+    q = torch.randn(n, H, 192, device="cuda", dtype=dtype)
+    wk = torch.randn(H, 128, 512, device="cuda", dtype=dtype) * 512**-0.5
+    wv = torch.randn(H, 512, 128, device="cuda", dtype=dtype) * 512**-0.5
+    big = 20 if dtype == torch.bfloat16 else 8
+    for h, lo, hi, e in [(0, 0, 128, big), (1, 0, 128, -big),
+                         (2, 0, 64, big // 2), (3, 64, 128, -big // 2),
+                         (4, 0, 128, big * 3 if big == 20 else 9)]:
+        wk[h, lo:hi] *= 2.0**e
+        q[:, h, lo:hi] *= 2.0**-e
+    q[5, 6] = 0
+    # Tokens 64..127 carry larger latents, weighed down by their rotary part.
+    cache[bt[0, 1], :, :512] *= 32
+    qsl = torch.tensor([0, n], device="cuda", dtype=torch.int32)
+    out = hip.mla_heads(q[..., :128], q[..., 128:], wk, wv, cache, bt, qsl,
+                        qsl[1:].clone(), 192**-0.5, max_query_len=n,
+                        max_seq_len=n)
+    expect = ref.mla_heads(q[..., :128].double(), q[..., 128:].double(),
+                           wk.double(), wv.double(), cache.double(), bt, qsl,
+                           qsl[1:].clone(), 192**-0.5)
+    assert out.isfinite().all()
+    err = (out - expect).double().norm(dim=(0, 2))
+    rel = err / expect.norm(dim=(0, 2))
+    assert (rel < 4 * (2**-8 if dtype == torch.bfloat16 else 2**-11)).all(), \
+        rel
+
+
+def test_mla_prompt_precision(monkeypatch):
+    """In sharp softmaxes (scores of deviation 4) the per-head form is no
+    further from 64 bits than the latent one: there a query's 512 values
+    are rounded to bf16 and decide the error, here a key's are fp16, an
+    eighth of that; what both share, values and results in bf16, is about
+    0.6 of the latent form's error."""
+    hip = _hip()
+    n, H, bf = 250, 16, torch.bfloat16
+    cache = torch.randn(4, 64, 576, device="cuda", dtype=bf)
+    bt = torch.randperm(4, device="cuda").int()[None]
+    q = torch.randn(n, H, 192, device="cuda", dtype=bf) * 8
+    wk = torch.randn(H, 128, 512, device="cuda", dtype=bf) * 900**-0.5
+    wv = torch.randn(H, 512, 128, device="cuda", dtype=bf) * 900**-0.5
+    qsl = torch.tensor([0, n], device="cuda", dtype=torch.int32)
+    args = (cache, bt, qsl, qsl[1:].clone(), 192**-0.5)
+    rule, err = hip._mla_prompt_heads, {}
+    expect = None
+    for name, form in (("heads", rule), ("latent", lambda *a: 0)):
+        monkeypatch.setattr(hip, "_mla_prompt_heads", form)
+        out = hip.mla_heads(q[..., :128], q[..., 128:], wk, wv, *args,
+                            max_query_len=n, max_seq_len=n).double()
+        if expect is None:
+            expect = torch.empty_like(out)
+            rows = cache[bt[0].long()].flatten(0, 1)[:n].double()
+            hide = torch.ones(n, n, device="cuda").triu(1).bool()
+            for h in range(H):
+                k = rows[:, :512] @ wk[h].double().T
+                s = (q[:, h, :128].double() @ k.T
+                     + q[:, h, 128:].double() @ rows[:, 512:].T)
+                p = (s * 192**-0.5).masked_fill(hide, -torch.inf).softmax(-1)
+                expect[:, h] = p @ (rows[:, :512] @ wv[h].double())
+        err[name] = ((out - expect).norm() / expect.norm()).item()
+    assert err["heads"] < 0.8 * err["latent"], err

@@ -71,7 +71,8 @@ void mla_prompt_attention(torch::Tensor out, torch::Tensor q_nope,
                           torch::Tensor query_start_loc,
                           torch::Tensor seq_lens, double scale,
                           int64_t num_decodes, int64_t max_query_len,
-                          int64_t S, torch::Tensor scratch);
+                          int64_t S, torch::Tensor scratch,
+                          torch::Tensor exps);
 void mla_prefill(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
                  torch::Tensor kv_cache, torch::Tensor block_table,
                  torch::Tensor query_start_loc, torch::Tensor seq_lens,
@@ -230,7 +231,8 @@ TORCH_LIBRARY(vllm_amd, m) {
       "mla_prompt_attention(Tensor(a!) out, Tensor q_nope, Tensor q_pe, "
       "Tensor w_uk, Tensor w_uv, Tensor kv_cache, Tensor block_table, "
       "Tensor query_start_loc, Tensor seq_lens, float scale, "
-      "int num_decodes, int max_query_len, int S, Tensor(b!) scratch) -> ()");
+      "int num_decodes, int max_query_len, int S, Tensor(b!) scratch, "
+      "Tensor(c!) exps) -> ()");
   m.def("mla_prefill(Tensor(a!) out, Tensor q_nope, Tensor q_pe, "
         "Tensor kv_cache, Tensor block_table, Tensor query_start_loc, "
         "Tensor seq_lens, float scale, int num_decodes, int max_seq_len, "

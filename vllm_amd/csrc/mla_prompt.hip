@@ -8,8 +8,16 @@
 //   mla_expand_kernel   keys, values and rotary parts of each request's
 //                       context, from the paged latent cache, per head
 //   mla_prompt_kernel   causal attention over them
-// Keys and values are rounded to the cache's type, as queries and results
-// are in the latent form; weights keep more than 16 bits (hi + lo).
+// Values are rounded to the cache's type, as results are in the latent
+// form; weights keep more than 16 bits (hi + lo). Keys are fp16 for a bf16
+// cache too: in sharp softmaxes the 128 roundings of a key weigh more than
+// the 512 of a query carried into the latent space. 5 prompts of 283 tokens,
+// queries of deviation 1 / 4 / 8, distance to 64 bits in thousandths: keys in
+// bf16 2.36 / 3.11 / 3.68, the latent form 2.37 / 3.08 / 3.61, keys in fp16
+// 2.27 / 2.34 / 2.36 (fp16 products run 2 % slower, power bound); with an
+// fp16 cache 0.295 / 0.389 / 0.460, the latent form 0.296 / 0.385 / 0.451.
+// So that no key leaves fp16's range, 64 tokens x 64 columns share a power of
+// two, which is one unless their largest is below 1/4 or from 2^15.
 // 128 heads, prompts of 300, 1300 and 2301 tokens: 2.02 -> 0.71 ms with
 // everything between queries and results (latent form before); one of
 // 8192 13.1 -> 3.7 ms, four of 2048 4.48 -> 1.45 ms.
@@ -17,6 +25,8 @@
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -41,6 +51,23 @@ DEVINL int seg256_chunk(int row, int c) {
   return seg256(row, c >> 1) * 2 + (c & 1);
 }
 
+// The powers of two that a block of keys and a row of queries are divided
+// by on the way to fp16 (infinities and NaN by none). A row's is free, so
+// its largest always lies below 2^14, with 2^28 of full precision under it.
+DEVINL int exponent(float largest) {
+  return (int)(__float_as_uint(largest) >> 23) - 127;
+}
+DEVINL int key_shift(float largest) {
+  const int e = exponent(largest);
+  return e == 128 || (e >= -2 && e <= 14) ? 0 : max(e, -60);
+}
+DEVINL int query_shift(float largest) {
+  const int e = exponent(largest);
+  return e == 128 ? 0 : max(e - 13, -60);
+}
+// exps of a head and request: two per 64 tokens.
+DEVINL int exps_per_request(int S) { return (S + 63) / 64 * 2; }
+
 // --------------------------------------------------------------------------
 // Keys and values of EX_M context tokens for one head. Eight waves of
 // 64 tokens x 64 columns, the first half of the columns keys, the second
@@ -64,8 +91,9 @@ static_assert(EX_M == D && EX_PART == EX_K * D * 2);
 
 template <typename Tag>
 __launch_bounds__(EX_THREADS, 2) __global__
-void mla_expand_kernel(short* __restrict__ k_out,   // [heads, reqs, S, D]
+void mla_expand_kernel(short* __restrict__ k_out,   // [heads, reqs, S, D] fp16
                        short* __restrict__ v_out,   // [heads, reqs, S, D]
+                       int* __restrict__ k_exp,     // [heads, reqs, S/64, 2]
                        short* __restrict__ pe_out,  // [reqs, S, ROPE]
                        const short* __restrict__ w_uk,  // [heads, D, LORA]
                        const short* __restrict__ w_uv,  // [heads, LORA, D]
@@ -179,6 +207,29 @@ void mla_expand_kernel(short* __restrict__ k_out,   // [heads, reqs, S, D]
       }
       reads_ahead<VALUES ? 9 : 6, VALUES ? 3 : 2, EX_K / 16 * 2, 2>();
       if ((s + 1) % STEPS) continue;
+      if constexpr (!VALUES) {
+        float mx = 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+              mx = __builtin_amdgcn_fmed3f(mx, fabsf(acc[i][j][e]), INFINITY);
+        int shift = 0;
+        if (__any(!(mx < 32768.f)) || !__any(mx >= 0.25f)) {
+          shift = key_shift(__uint_as_float(__builtin_amdgcn_readfirstlane(
+              __float_as_uint(wave_reduce_max(mx)))));
+          const float f = __builtin_ldexpf(1.f, -shift);
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] *= f;
+        }
+        if (lane == 0 && t0 + wm * 64 < ctx)
+          k_exp[((int64_t)(h + s / STEPS) * reqs + r) * exps_per_request(S) +
+                (t0 / 64 + wm) * 2 + wn] = shift;
+      }
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int row = wm * 64 + j * 32 + l32;
@@ -187,7 +238,8 @@ void mla_expand_kernel(short* __restrict__ k_out,   // [heads, reqs, S, D]
 #pragma unroll
           for (int b = 0; b < 4; b += 2) {
             f32x16& c = acc[i][j];
-            const i32x4 w = row_chunk<Tag>(c, b);
+            const i32x4 w = VALUES ? row_chunk<Tag>(c, b)
+                                   : row_chunk<FP16Tag>(c, b);
             if (t0 + row < ctx)
               *reinterpret_cast<i32x4*>(out + row * D + i * 32 + b * 8) = w;
 #pragma unroll
@@ -243,6 +295,7 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
                        const short* __restrict__ q_pe,     // [T, Hq, ROPE]
                        const short* __restrict__ k,        // [heads, reqs, S, D]
                        const short* __restrict__ v,
+                       const int* __restrict__ k_exp,
                        const short* __restrict__ pe,       // [reqs, S, ROPE]
                        const int* __restrict__ query_start_loc,
                        const int* __restrict__ seq_lens, float scale_log2,
@@ -271,6 +324,12 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
   const int tok_safe = min(tok, ql - 1);
   const int qpos = pos0 + tok_safe;
 
+  const int kt_end = (pos0 + min(row0 + PA_M, ql) - 1) / PA_KEYS + 1;
+  const int* ke =
+      k_exp + ((int64_t)h * gridDim.y + r) * exps_per_request(S);
+  int shifted = 0;
+  for (int i = lane; i < kt_end * 2; i += WAVE_SIZE) shifted |= ke[i];
+
   s16x8 qf[(D + ROPE) / 16];
   {
     const short* qn = q_nope + (q_start + tok_safe) * q_row +
@@ -283,6 +342,31 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
 #pragma unroll
     for (int kk = 0; kk < ROPE / 16; ++kk)
       qf[D / 16 + kk] = *reinterpret_cast<const s16x8*>(qp + kk * 16);
+  }
+  // A bf16 query has fewer bits than fp16; the scale takes its power of two
+  // back.
+  float scale = scale_log2;
+  if constexpr (std::is_same_v<Tag, BF16Tag>) {
+    float mx = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < D / 16; ++kk)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        mx = fmaxf(mx, fabsf(bf16_to_f32(qf[kk][e])));
+    const int shift = query_shift(half_max(mx));
+    const float f = __builtin_ldexpf(1.f, -shift);
+    scale = __builtin_ldexpf(scale_log2, shift);
+#pragma unroll
+    for (int kk = 0; kk < (D + ROPE) / 16; ++kk) {
+      i32x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float a = bf16_to_f32(qf[kk][e * 2]) * f;
+        const float b = bf16_to_f32(qf[kk][e * 2 + 1]) * f;
+        w[e] = kk < D / 16 ? pack2<FP16Tag>(a, b) : pack2<BF16Tag>(a, b);
+      }
+      qf[kk] = __builtin_bit_cast(s16x8, w);
+    }
   }
 
   const int64_t base = ((int64_t)h * gridDim.y + r) * S;
@@ -322,92 +406,101 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
 
   const int wave_first = pos0 + row0 + wave * 32;
   const int wave_last = pos0 + min(row0 + wave * 32 + 31, ql - 1);
-  const int kt_end = (pos0 + min(row0 + PA_M, ql) - 1) / PA_KEYS + 1;
   fill(0, 0);
+  auto run = [&](auto shifts) {
+    constexpr bool SHIFTS = decltype(shifts)::value;
 #pragma unroll 1
-  for (int kt = 0; kt < kt_end; ++kt) {
-    lds_fill_wait();
-    lds_barrier();
-    if (kt + 1 < kt_end) fill(kt + 1, (kt + 1) & 1);
-    if (kt * PA_KEYS > wave_last) continue;   // no key for these tokens
-    const char* t = lds + (kt & 1) * PA_BUF;
-    // --- S^T: 64 keys x 32 tokens ----------------------------------------
-    f32x16 s[2];
+    for (int kt = 0; kt < kt_end; ++kt) {
+      lds_fill_wait();
+      lds_barrier();
+      if (kt + 1 < kt_end) fill(kt + 1, (kt + 1) & 1);
+      if (kt * PA_KEYS > wave_last) continue;   // no key for these tokens
+      const char* t = lds + (kt & 1) * PA_BUF;
+      // --- S^T: 64 keys x 32 tokens ----------------------------------------
+      f32x16 s[2];
 #pragma unroll
-    for (int n = 0; n < 2; ++n) {
+      for (int n = 0; n < 2; ++n) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) s[n][e] = 0.f;
-      const int key = n * 32 + l32;
+        for (int e = 0; e < 16; ++e) s[n][e] = 0.f;
+        const int key = n * 32 + l32;
 #pragma unroll
-      for (int kk = 0; kk < D / 16; ++kk)
-        s[n] = mfma32<Tag>(
-            *reinterpret_cast<const s16x8*>(
-                t + key * 256 + chunk256(key, kk * 2 + half) * 16),
-            qf[kk], s[n]);
+        for (int kk = 0; kk < D / 16; ++kk) {
+          s[n] = mfma32<FP16Tag>(
+              *reinterpret_cast<const s16x8*>(
+                  t + key * 256 + chunk256(key, kk * 2 + half) * 16),
+              qf[kk], s[n]);
+          if (SHIFTS && kk == D / 32 - 1)
+            s[n] *= __builtin_ldexpf(1.f,
+                                     min(ke[kt * 2] - ke[kt * 2 + 1], 127));
+        }
+        if constexpr (SHIFTS) s[n] *= __builtin_ldexpf(1.f, ke[kt * 2 + 1]);
 #pragma unroll
-      for (int kk = 0; kk < ROPE / 16; ++kk)
-        s[n] = mfma32<Tag>(
-            *reinterpret_cast<const s16x8*>(
-                t + 2 * PA_K + key * 128 + chunk128(key, kk * 2 + half) * 16),
-            qf[D / 16 + kk], s[n]);
-    }
-    // Register e of s[n] is key n*32 + 8*(e/4) + 4*half + e%4.
-    if (kt * PA_KEYS + PA_KEYS - 1 > wave_first) {
-      const int left = qpos - kt * PA_KEYS - half * 4;
-#pragma unroll
-      for (int n = 0; n < 2; ++n)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          s[n][e] = n * 32 + 8 * (e >> 2) + (e & 3) <= left ? s[n][e] : NEG;
-    }
-    float mx = NEG;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      mx = __builtin_amdgcn_fmed3f(mx, s[0][e], INFINITY);
-      mx = __builtin_amdgcn_fmed3f(mx, s[1][e], INFINITY);
-    }
-    mx = half_max(mx) * scale_log2;
-    if (__any(mx - m_run > GROWTH)) {
-      const float m_new = fmaxf(m_run, mx);
-      const float f = __builtin_amdgcn_exp2f(m_run - m_new);
-      l_run *= f;
-#pragma unroll
-      for (int i = 0; i < D / 32; ++i) o[i] *= f;
-      m_run = m_new;
-    }
-    // --- O^T += V^T P^T, 16 keys at a time -------------------------------
-    const int vrow = half * 4 + ((lane & 15) >> 2);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      i32x4 hi, lo;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int e = (c & 1) * 8 + j * 2;
-        const float p0 = __builtin_amdgcn_exp2f(
-            __builtin_fmaf(s[c >> 1][e], scale_log2, -m_run));
-        const float p1 = __builtin_amdgcn_exp2f(
-            __builtin_fmaf(s[c >> 1][e + 1], scale_log2, -m_run));
-        hi[j] = pack2<Tag>(p0, p1);
-        l_run += p0 + p1;
-        lo[j] = pack2<Tag>(p0 - unpack_lo<Tag>(hi[j]),
-                           p1 - unpack_hi<Tag>(hi[j]));
+        for (int kk = 0; kk < ROPE / 16; ++kk)
+          s[n] = mfma32<Tag>(
+              *reinterpret_cast<const s16x8*>(
+                  t + 2 * PA_K + key * 128 + chunk128(key, kk * 2 + half) * 16),
+              qf[D / 16 + kk], s[n]);
       }
-      const s16x8 p_hi = __builtin_bit_cast(s16x8, hi);
-      const s16x8 p_lo = __builtin_bit_cast(s16x8, lo);
-      const int r0 = c * 16 + vrow;
+      // Register e of s[n] is key n*32 + 8*(e/4) + 4*half + e%4.
+      if (kt * PA_KEYS + PA_KEYS - 1 > wave_first) {
+        const int left = qpos - kt * PA_KEYS - half * 4;
 #pragma unroll
-      for (int i = 0; i < D / 32; ++i) {
-        const int seg = i * 2 + ((lane >> 4) & 1);
-        const char* at = t + PA_K + (lane & 3) * 8;
-        const s16x4 a = lds_read_tr(at + r0 * 256 + seg256(r0, seg) * 32);
-        const s16x4 b =
-            lds_read_tr(at + (r0 + 8) * 256 + seg256(r0 + 8, seg) * 32);
-        const s16x8 vf = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
-        o[i] = mfma32<Tag>(vf, p_lo, o[i]);
-        o[i] = mfma32<Tag>(vf, p_hi, o[i]);
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            s[n][e] = n * 32 + 8 * (e >> 2) + (e & 3) <= left ? s[n][e] : NEG;
+      }
+      float mx = NEG;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        mx = __builtin_amdgcn_fmed3f(mx, s[0][e], INFINITY);
+        mx = __builtin_amdgcn_fmed3f(mx, s[1][e], INFINITY);
+      }
+      mx = half_max(mx) * scale;
+      if (__any(mx - m_run > GROWTH)) {
+        const float m_new = fmaxf(m_run, mx);
+        const float f = __builtin_amdgcn_exp2f(m_run - m_new);
+        l_run *= f;
+#pragma unroll
+        for (int i = 0; i < D / 32; ++i) o[i] *= f;
+        m_run = m_new;
+      }
+      // --- O^T += V^T P^T, 16 keys at a time -------------------------------
+      const int vrow = half * 4 + ((lane & 15) >> 2);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        i32x4 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int e = (c & 1) * 8 + j * 2;
+          const float p0 = __builtin_amdgcn_exp2f(
+              __builtin_fmaf(s[c >> 1][e], scale, -m_run));
+          const float p1 = __builtin_amdgcn_exp2f(
+              __builtin_fmaf(s[c >> 1][e + 1], scale, -m_run));
+          hi[j] = pack2<Tag>(p0, p1);
+          l_run += p0 + p1;
+          lo[j] = pack2<Tag>(p0 - unpack_lo<Tag>(hi[j]),
+                             p1 - unpack_hi<Tag>(hi[j]));
+        }
+        const s16x8 p_hi = __builtin_bit_cast(s16x8, hi);
+        const s16x8 p_lo = __builtin_bit_cast(s16x8, lo);
+        const int r0 = c * 16 + vrow;
+#pragma unroll
+        for (int i = 0; i < D / 32; ++i) {
+          const int seg = i * 2 + ((lane >> 4) & 1);
+          const char* at = t + PA_K + (lane & 3) * 8;
+          const s16x4 a = lds_read_tr(at + r0 * 256 + seg256(r0, seg) * 32);
+          const s16x4 b =
+              lds_read_tr(at + (r0 + 8) * 256 + seg256(r0 + 8, seg) * 32);
+          const s16x8 vf = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+          o[i] = mfma32<Tag>(vf, p_lo, o[i]);
+          o[i] = mfma32<Tag>(vf, p_hi, o[i]);
+        }
       }
     }
-  }
+  };
+  if (__any(shifted != 0)) run(std::true_type{});
+  else run(std::false_type{});
 
   l_run += __shfl_xor(l_run, 32, 64);
   const float inv_l = 1.f / l_run;
@@ -429,7 +522,8 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
 // Prompt portions (requests num_decodes..) of a step; out, q_nope and q_pe
 // [T, Hq, 128 / 128 / 64] cover the whole step. scratch holds per head
 // 2 x [reqs, S, 128] and once [reqs, S, 64] values, S >= every context; as
-// many heads as fit run at a time.
+// many heads as fit run at a time. exps [heads at a time, reqs,
+// ceil(S / 64), 2] are the keys' exponents.
 void mla_prompt_attention(torch::Tensor out, torch::Tensor q_nope,
                           torch::Tensor q_pe, torch::Tensor w_uk,
                           torch::Tensor w_uv, torch::Tensor kv_cache,
@@ -437,7 +531,8 @@ void mla_prompt_attention(torch::Tensor out, torch::Tensor q_nope,
                           torch::Tensor query_start_loc,
                           torch::Tensor seq_lens, double scale,
                           int64_t num_decodes, int64_t max_query_len,
-                          int64_t S, torch::Tensor scratch) {
+                          int64_t S, torch::Tensor scratch,
+                          torch::Tensor exps) {
   using namespace mla_prompt;
   TORCH_CHECK(q_nope.dim() == 3 && q_nope.size(2) == D &&
               q_pe.dim() == 3 && q_pe.size(2) == ROPE &&
@@ -468,6 +563,8 @@ void mla_prompt_attention(torch::Tensor out, torch::Tensor q_nope,
   const int at_once = (int)std::min<int64_t>(
       Hq, (scratch.numel() - pe_size) / (2 * head_size));
   TORCH_CHECK(at_once >= 1, "mla prompts: scratch holds no head");
+  TORCH_CHECK(exps.scalar_type() == torch::kInt32 && exps.is_contiguous() &&
+              exps.numel() >= at_once * reqs * ((S + 63) / 64 * 2));
   short* pe = (short*)scratch.data_ptr();
   short* k = pe + pe_size;
   short* v = k + at_once * head_size;
@@ -483,7 +580,8 @@ void mla_prompt_attention(torch::Tensor out, torch::Tensor q_nope,
           (mla_expand_kernel<Tag>),
           dim3(ceil_div(heads, per), token_tiles, (int)reqs),
           dim3(EX_THREADS), 0,
-          stream, k, v, pe, (const short*)w_uk.data_ptr() + h0 * D * LORA,
+          stream, k, v, exps.data_ptr<int>(), pe,
+          (const short*)w_uk.data_ptr() + h0 * D * LORA,
           (const short*)w_uv.data_ptr() + h0 * D * LORA,
           (const short*)kv_cache.data_ptr(), block_table.data_ptr<int>(),
           (int)block_table.size(1), seq_lens.data_ptr<int>(),
@@ -496,7 +594,7 @@ void mla_prompt_attention(torch::Tensor out, torch::Tensor q_nope,
           dim3(PA_THREADS),
           0, stream, (short*)out.data_ptr(), (const short*)q_nope.data_ptr(),
           q_nope.stride(0), q_nope.stride(1), (const short*)q_pe.data_ptr(),
-          k, v, pe, query_start_loc.data_ptr<int>(),
+          k, v, exps.data_ptr<int>(), pe, query_start_loc.data_ptr<int>(),
           seq_lens.data_ptr<int>(), (float)scale * 1.4426950408889634f,
           (int)Hq, h0, heads, (int)num_decodes, (int)S, tiles);
       HIP_CHECK_KERNEL();

@@ -420,9 +420,12 @@ def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
     rows = (reqs - num_decodes) * S
     scratch = torch.empty(rows * (64 + heads * 256), dtype=q_nope.dtype,
                           device=q_nope.device)
+    exps = torch.empty(heads * (reqs - num_decodes) * -(-S // 64) * 2,
+                       dtype=torch.int32, device=q_nope.device)
     _C.mla_prompt_attention(out, q_nope, q_pe.contiguous(), w_uk, w_uv,
                             kv_cache, block_table, query_start_loc, seq_lens,
-                            scale, num_decodes, max_query_len, S, scratch)
+                            scale, num_decodes, max_query_len, S, scratch,
+                            exps)
     return out
 
 
