@@ -178,3 +178,53 @@ def test_mla_prompt_heads_at_a_time(hip, monkeypatch):
     monkeypatch.setattr(hip, "_MLA_PROMPT_SCRATCH", 13 * 60 * S * 512)
     _, numel = _mla_prompts(hip, monkeypatch, 1, 60)
     assert (numel // per - 64) // 256 == 8
+
+
+def _odd(*shape):
+    """A contiguous bf16 tensor that begins 2 B past a 16 B boundary."""
+    n = 1
+    for x in shape:
+        n *= x
+    flat = torch.empty(n + 8, dtype=torch.bfloat16)
+    at = next(i for i in range(8)
+              if flat[i:].data_ptr() % 16 == 2)
+    return flat[at:at + n].view(shape)
+
+
+def test_odd_places_take_plain_loads(hip, monkeypatch):
+    """Operands that do not begin on 16 B never reach a kernel that fills
+    LDS from them directly."""
+    bf, H, I, E = torch.bfloat16, 128, 64, 2
+    hip._C.moe_tile_rows = lambda f: (64, 128, 256)[f]
+    weights = (torch.empty(E, 2 * I, H, dtype=bf),
+               torch.empty(E, H, I, dtype=bf))
+    for x, w13, w2, form in (
+            (torch.empty(600, H, dtype=bf), *weights, 2),
+            (_odd(600, H), *weights, 0),
+            (torch.empty(600, H, dtype=bf), _odd(E, 2 * I, H), weights[1],
+             0)):
+        hip._C.calls.clear()
+        hip.fused_moe_hip(x, w13, w2, torch.empty(600, 1),
+                          torch.zeros(600, 1, dtype=torch.int32))
+        assert [a[8] for a in hip._C.args("moe_gemm")] == [form, form]
+
+    hip._C.calls.clear()
+    hip.head_matmul(torch.randn(3, 2, 128).to(bf), _odd(2, 128, 128).zero_())
+    assert not hip._C.calls
+
+    q = torch.empty(400, 128, 192, dtype=bf)[..., :128]
+    w_uk = torch.empty(128, 128, 512, dtype=bf)
+    w_uv = torch.empty(128, 512, 128, dtype=bf)
+    cache = torch.empty(1, 64, 576, dtype=bf)
+    args = (1, 0.07, 0, 400, 400)
+    assert hip._mla_prompt_heads(q, w_uk, w_uv, cache, *args) == 128
+    for odd in ((_odd(128, 128, 512), w_uv, cache),
+                (w_uk, _odd(128, 512, 128), cache),
+                (w_uk, w_uv, _odd(1, 64, 576))):
+        assert hip._mla_prompt_heads(q, *odd, *args) == 0
+    one = torch.ones(1, dtype=torch.int32)
+    hip.mla_attention(torch.zeros(1, 4, 512, dtype=bf),
+                      torch.zeros(1, 4, 64, dtype=bf),
+                      _odd(1, 64, 576).zero_(), one[None] * 0,
+                      _lens(0, 1), one, 0.07, num_decodes=1, max_seq_len=1)
+    assert not hip._C.calls

@@ -140,7 +140,8 @@ torch::Tensor head_matmul(torch::Tensor x, torch::Tensor w) {
                x.scalar_type() == torch::kHalf), "head_matmul: bf16/fp16 only");
   TORCH_CHECK(w.is_contiguous() && x.stride(2) == 1 &&
               x.stride(0) % 8 == 0 && x.stride(1) % 8 == 0 &&
-              (uintptr_t)x.data_ptr() % 16 == 0,
+              (uintptr_t)x.data_ptr() % 16 == 0 &&
+              (uintptr_t)w.data_ptr() % 16 == 0,
               "head_matmul: rows must be 16 B aligned");
   const int T = (int)x.size(0), H = (int)x.size(1), K = (int)x.size(2);
   const int N = (int)w.size(2);

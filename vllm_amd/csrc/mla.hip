@@ -373,7 +373,8 @@ static void check(const torch::Tensor& out, const torch::Tensor& q_nope,
   TORCH_CHECK(q_pe.size(2) == ROPE, "mla kernel expects rope dim 64");
   TORCH_CHECK(kv_cache.size(2) == DK);
   TORCH_CHECK(q_nope.is_contiguous() && q_pe.is_contiguous() &&
-              out.is_contiguous() && kv_cache.is_contiguous());
+              out.is_contiguous() && kv_cache.is_contiguous() &&
+              (uintptr_t)kv_cache.data_ptr() % 16 == 0);
   TORCH_CHECK(out.scalar_type() == q_nope.scalar_type() &&
               q_pe.scalar_type() == q_nope.scalar_type() &&
               kv_cache.scalar_type() == q_nope.scalar_type());

@@ -549,8 +549,9 @@ void mla_prompt_attention(torch::Tensor out, torch::Tensor q_nope,
               w_uk.is_contiguous() && w_uv.is_contiguous() &&
               kv_cache.is_contiguous() && scratch.is_contiguous());
   TORCH_CHECK(q_nope.stride(2) == 1 && q_nope.stride(0) % 8 == 0 &&
-              q_nope.stride(1) % 8 == 0 &&
-              (uintptr_t)q_nope.data_ptr() % 16 == 0);
+              q_nope.stride(1) % 8 == 0);
+  for (const auto& x : {q_nope, w_uk, w_uv, kv_cache, scratch})
+    TORCH_CHECK((uintptr_t)x.data_ptr() % 16 == 0);
   const auto type = q_nope.scalar_type();
   TORCH_CHECK(type == torch::kBFloat16 || type == torch::kHalf);
   for (const auto& x : {out, q_pe, w_uk, w_uv, kv_cache, scratch})

@@ -812,9 +812,12 @@ static void run_gemm(const torch::Tensor& a, const torch::Tensor& b,
       form > 0 ? (int64_t)ceil_div(m_tiles, 8 / split) *
                      ceil_div(n_blocks, split) * 8
                : ((int64_t)m_tiles * n_blocks + 7) / 8 * 8;
-  // (Tiles address rows and an expert's weights with 32 bits.)
+  // (Tiles address rows and an expert's weights with 32 bits, and fill LDS
+  // from them 16 B at a time.)
   TORCH_CHECK(form == 0 || (a.numel() * 2 < (1ll << 32) &&
-                            b_rows * K * 2 < (1ll << 32)));
+                            b_rows * K * 2 < (1ll << 32) &&
+                            (uintptr_t)a.data_ptr() % 16 == 0 &&
+                            (uintptr_t)b.data_ptr() % 16 == 0));
   TORCH_CHECK(blocks < (1ll << 30));
   auto stream = c10::hip::getCurrentHIPStream().stream();
   dim3 grid((unsigned)blocks);

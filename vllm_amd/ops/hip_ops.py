@@ -48,6 +48,12 @@ def _decode_parts(rows, kv_heads, max_seq_len, sliding_window):
     return max(1, min(parts, units, 64))
 
 
+def _aligned(*tensors):
+    """Operands that kernels fill LDS from directly, 16 B at a time, must
+    begin on 16 B; views into odd places take a form with plain loads."""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def rms_norm(x, weight, eps):
     return _C.rms_norm(x, weight, eps)
 
@@ -289,7 +295,7 @@ def mla_attention(q_nope, q_pe, kv_cache, block_table, query_start_loc,
     use_hip = (q_nope.shape[2] == 512 and q_pe.shape[2] == 64
                and q_nope.dtype in (torch.bfloat16, torch.float16)
                and q_pe.dtype == q_nope.dtype
-               and kv_cache.dtype == q_nope.dtype)
+               and kv_cache.dtype == q_nope.dtype and _aligned(kv_cache))
     if not use_hip:
         return _torch_ref.mla_attention(
             q_nope, q_pe, kv_cache, block_table, query_start_loc, seq_lens,
@@ -316,7 +322,7 @@ def head_matmul(x, w):
             and w.shape[1] % 128 == 0 and w.shape[2] % 128 == 0
             and w.is_contiguous() and x.stride(2) == 1
             and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0
-            and x.data_ptr() % 16 == 0):
+            and _aligned(x, w)):
         return _C.head_matmul(x, w)
     return _torch_ref.head_matmul(x, w)
 
@@ -378,7 +384,8 @@ def _mla_prompt_heads(q_nope, w_uk, w_uv, kv_cache, reqs, scale,
             or any(t.dtype != q_nope.dtype for t in (w_uk, w_uv, kv_cache))
             or not all(t.is_contiguous() for t in (w_uk, w_uv, kv_cache))
             or q_nope.stride(2) != 1 or q_nope.stride(0) % 8
-            or q_nope.stride(1) % 8 or q_nope.data_ptr() % 16):
+            or q_nope.stride(1) % 8
+            or not _aligned(q_nope, w_uk, w_uv, kv_cache)):
         return 0
     heads = min(Hq, _MLA_PROMPT_SCRATCH // (reqs * max_seq_len * 512))
     # The kernel deals eight heads at a time to the eight XCDs.
@@ -504,8 +511,9 @@ def fused_moe_hip(hidden, w13, w2, topk_weights, topk_ids,
     total = T * k
     dev = hidden.device
     form = _moe_form(T, total, E, H)
-    if max(T * H, (total + E * 256) * I, n1 * H) >= 1 << 31:
-        form = 0    # tiles address 4 GB
+    if (max(T * H, (total + E * 256) * I, n1 * H) >= 1 << 31
+            or not _aligned(hidden, w13, w2)):
+        form = 0    # tiles address 4 GB, by 16 B
     if form > 0:    # (they take the weights in their own order)
         w13_shuf = w2_shuf = None
     bm = _C.moe_tile_rows(form)
