@@ -874,8 +874,9 @@ def test_mla_a_projections_as_one(T):
 
 
 def test_mla_unified_dispatch_mixed_batch():
-    """ops.mla_attention routes decode rows to the kernel and prefill
-    rows to the torch path; both must agree with the all-torch result."""
+    """hip_ops.mla_attention runs decode rows (mla_decode) and prompt rows
+    (mla_prefill) of one batch on the kernel; both must agree with the
+    all-torch result."""
     hip = _hip()
     lora, rope, bs, Hq = 512, 64, 16, 32
     T_dec, ql_pre, ctx_pre = 3, 5, 40
@@ -933,7 +934,7 @@ def test_prefill_attention_head_dim_sweep(hd, q_lens, ctx_lens):
 ])
 def test_moe_shuffled_weight_gemm(T, H, I, E, K):
     """Fragment-major pre-shuffled weight stream (moe_gemm_shuf) must
-    match the staged-LDS grouped GEMM and the fp32 reference."""
+    match the stream of plain weights and the fp32 reference."""
     hip = _hip()
     hidden = torch.randn(T, H, dtype=torch.bfloat16, device="cuda") * 0.3
     w13 = torch.randn(E, 2 * I, H, dtype=torch.bfloat16, device="cuda") * 0.2

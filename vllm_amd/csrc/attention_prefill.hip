@@ -29,8 +29,8 @@
 //   - Results are stored 16 B a lane (8 B: 59 us for the short prompts
 //     below, 53 now).
 // Against 16x16x32 fragments on 16-row waves with V scattered into LDS:
-// one 8192-token prompt, 32/8 heads of 128: 4.70 -> 0.61 ms (900 TFLOP/s);
-// 64 prompts of 33..223 tokens: 207 -> 53 us; 4 x 2048 tokens, 16/8 heads
+// one 8192-token prompt, 32/8 heads of 128: 4.70 -> 0.67 ms (820 TFLOP/s);
+// 64 prompts of 33..223 tokens: 207 -> 54 us; 4 x 2048 tokens, 16/8 heads
 // of 256: 2.59 -> 0.26 ms.
 //
 // Role of the reference's triton_unified_attention.py:179 (prefill side)

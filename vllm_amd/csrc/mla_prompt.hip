@@ -18,9 +18,9 @@
 // fp16 cache 0.295 / 0.389 / 0.460, the latent form 0.296 / 0.385 / 0.451.
 // So that no key leaves fp16's range, 64 tokens x 64 columns share a power of
 // two, which is one unless their largest is below 1/4 or from 2^15.
-// 128 heads, prompts of 300, 1300 and 2301 tokens: 2.02 -> 0.71 ms with
+// 128 heads, prompts of 300, 1300 and 2301 tokens: 2.02 -> 0.63 ms with
 // everything between queries and results (latent form before); one of
-// 8192 13.1 -> 3.7 ms, four of 2048 4.48 -> 1.45 ms.
+// 8192 13.1 -> 3.80 ms, four of 2048 4.48 -> 1.36 ms.
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
