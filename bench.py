@@ -1,15 +1,14 @@
-"""Flagship serving benchmark (driver contract).
+"""Flagship serving benchmark.
 
-Measures whole-node output tokens/sec on the BASELINE.json headline
-config: Llama-3-8B bf16, synthetic random prompts of the CI benchmark
+Measures whole-node output tokens/sec of Llama-3-8B in bf16, synthetic random prompts of the CI benchmark
 shape (random 128-token inputs), random-init (dummy) weights, continuous
 decode at a fixed running batch.
 
     python bench.py --gpus N --steps K --warmup W
 
-For N>1 the driver launches this under torch.distributed.run with one
-rank per GPU; ranks form a TP=N group over RCCL/xGMI (the reference's
-headline TP configs). One "step" is one engine iteration:
+For N>1 this is launched under torch.distributed.run with one rank per
+GPU; ranks form a TP=N group over RCCL/xGMI (the reference's headline TP
+configs). One "step" is one engine iteration:
 after warmup (which absorbs the prefill of the whole batch) every step
 is a full-batch decode producing `batch` output tokens.
 

@@ -1,6 +1,6 @@
 """Serving benchmark: output tokens/sec + TTFT/ITL percentiles at a fixed
 request rate (role of the reference's `vllm bench serve`,
-vllm/benchmarks/serve.py — the BASELINE.json metric's latency half).
+vllm/benchmarks/serve.py).
 
 Drives the full serving path in-process (FastAPI app via ASGI transport:
 HTTP parsing, SSE streaming, detokenization) with synthetic random

@@ -4,7 +4,7 @@ GPU tests run TWO processes sharing one GPU: hipIpc handle exchange over
 a gloo process group, then the one-shot / two-shot kernels reduce across
 the two processes' buffers — the full production path (init, connect,
 flag protocol, parity reuse, graph capture) minus the multi-device xGMI
-hop, which the driver's round-end 8-GPU scale run covers.
+hop, which only an eight-GPU run covers.
 """
 
 import multiprocessing as mp

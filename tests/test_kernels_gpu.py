@@ -391,7 +391,7 @@ def test_model_forward_matches_cpu_reference():
     gpu = run("cuda", "bf16")
     cpu = run("cpu", "fp32")
     cos = torch.nn.functional.cosine_similarity(gpu, cpu, dim=-1)
-    # bf16 2-layer stack vs fp32: tighter than the round-1 gate (0.99 /
+    # bf16 2-layer stack vs fp32: tighter than an earlier gate (0.99 /
     # 0.8 argmax, loose enough to hide drift) while leaving bf16
     # headroom; op-level tests carry the per-kernel tolerances.
     assert cos.min() > 0.995, cos

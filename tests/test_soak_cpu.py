@@ -4,7 +4,7 @@ scheduling, spec decode and a pool small enough to force preemption —
 all at once. Asserts (a) every request completes with the requested
 token count, (b) the whole run is bit-deterministic across two
 executions (catches cross-feature state leaks the targeted tests
-miss — the round-2 window-reclaim corruption was exactly this class)."""
+miss, as a corruption by early reclaimed window blocks once was)."""
 
 import numpy as np
 

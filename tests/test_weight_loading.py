@@ -267,7 +267,7 @@ def test_dummy_shard_matches_loaders_at_high_tp(monkeypatch):
     """dummy_shard must produce EXACTLY what the checkpoint loaders
     produce from the same full tensors, for every rank at tp=4 and
     tp=8 (incl. KV-head replication) — the gloo tests only cover tp=2,
-    but the driver's scale run shards at tp=8."""
+    while eight-GPU runs shard at tp=8."""
     import torch
 
     import vllm_amd.layers.linear as L

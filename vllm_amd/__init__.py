@@ -7,8 +7,7 @@ parallelism, OpenAI-compatible API) designed for AMD Instinct MI355X
 LDS-staged tiles for the hot ops, RCCL over xGMI for collectives, and
 hipGraph-captured decode steps.
 
-Reference feature map: vllm-project/vllm. This is not a
-port — the architecture is MI355X-first.
+The features are those of vllm-project/vllm. This is not a port — the architecture is MI355X-first.
 """
 
 __version__ = "0.1.0"

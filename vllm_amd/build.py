@@ -1,7 +1,7 @@
 """In-tree build of the vllm_amd HIP/CDNA4 extension (gfx950 only).
 
 Drives hipcc directly (no JIT cache — the .so lands next to the package
-so the gpurun snapshot carries it). Usage:
+and travels with the tree). Usage:
 
     python -m vllm_amd.build           # build vllm_amd/_C.so
     python -m vllm_amd.build --check   # build only if sources newer

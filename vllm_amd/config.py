@@ -3,8 +3,8 @@
 One composite ``EngineConfig`` threads through every constructor, same
 discipline as the reference's VllmConfig (vllm/config/vllm.py:331).
 Model architectures are described by an explicit ``ModelSpec`` so the
-engine runs fully offline: built-in presets cover the benchmark configs
-and any local HF ``config.json`` can also be loaded.
+engine runs fully offline: built-in presets cover the benchmarked
+models, and any local HF ``config.json`` can also be loaded.
 """
 
 from __future__ import annotations
@@ -197,7 +197,7 @@ class ModelSpec:
         return 1
 
 
-# Built-in presets matching BASELINE.json's named configs.
+# Built-in presets: the benchmarked models, and tiny ones for tests.
 MODEL_PRESETS: dict[str, ModelSpec] = {
     # Tiny llava-style vision-language model (CPU tests).
     "tiny-llava": ModelSpec(
@@ -1237,8 +1237,8 @@ def _spec_from_hf_config(path: str) -> ModelSpec:
         architecture = "qwen3_moe"
     elif "phi3" in arch:
         # Phi-3 is llama-structured (fused qkv/gate_up checkpoints);
-        # longrope scaling beyond the original 4k context is a tracked
-        # round-2 item — contexts <= original_max_position need none.
+        # longrope scaling beyond the original 4k context is not
+        # built — contexts <= original_max_position need none.
         architecture = "phi3"
     elif "qwen3" in arch:
         architecture = "qwen3"

@@ -346,7 +346,7 @@ class LLMEngine:
         pp = self.config.parallel_config.pipeline_parallel_size
         if pp > 1 and (params.pooling or params.prompt_logprobs):
             # Hidden states / logits live on the LAST pp stage while the
-            # driver is stage 0; routing them back is a round-2 item.
+            # driver is stage 0; they are not routed back.
             raise ValueError(
                 "pooling and prompt_logprobs require pp=1")
         if params.guided_choice:

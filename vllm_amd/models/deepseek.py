@@ -1,5 +1,5 @@
 """DeepSeek-V3-style decoder: MLA attention + sigmoid group-routed MoE
-with shared experts (BASELINE config 5).
+with shared experts.
 
 Structure mirrors the reference's deepseek_v2.py (vllm/model_executor/
 models/deepseek_v2.py) and mla.py (model_executor/layers/mla.py:36):

@@ -1,4 +1,4 @@
-"""Mixtral (sparse MoE decoder: Mixtral 8x7B).
+"""Mixtral (sparse MoE decoder, as Mixtral 8x7B).
 
 Structure mirrors the reference's mixtral.py (vllm/model_executor/models/
 mixtral.py) — Llama-style GQA attention + per-layer top-2-of-8 FusedMoE

@@ -152,8 +152,8 @@ def quantize_model_fp8(model: torch.nn.Module) -> None:
     """Quantize every dense linear to W8A8 fp8 after load (per-channel
     weight scales; activations get per-token scales at run time). The
     lm_head stays in model dtype (logit sensitivity — same choice as the
-    reference's fp8 config), as do MoE expert weights (grouped-GEMM path
-    is bf16 this round) and the embedding."""
+    reference's fp8 config), as do MoE expert weights (the grouped products
+    take 16-bit weights) and the embedding."""
     from vllm_amd.layers.linear import (
         ColumnParallelLinear,
         ReplicatedLinear,

@@ -13,7 +13,7 @@ blocks — they never grow during decode).
 Decoder block (pre-norm): self-attn -> cross-attn -> GELU MLP.
 Learned decoder positions (OPT-style, no offset). TP shards the
 projections; the encoder itself is replicated (runs once per request).
-PP is not supported for encoder-decoder this round (the encoder states
+PP is not supported for encoder-decoder models (the encoder states
 would need to ship between stages) — single-stage only, enforced at
 construction.
 """

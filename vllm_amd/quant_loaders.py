@@ -5,7 +5,7 @@ AWQ (4-bit, group-scaled, zero-pointed) checkpoints are DEQUANTIZED at
 load into the model dtype, so any AWQ-packed model runs today; combining
 with `--quantization fp8` re-quantizes the dequantized weights to W8A8
 for the fp8 MFMA path. A native int4 dequant-GEMM kernel (keeping the 4×
-weight-memory saving at run time) is a tracked round-2 item.
+weight-memory saving at run time) is not built.
 
 AWQ packing: qweight int32 [K, N/8] — eight 4-bit values per int32
 along the OUTPUT dim in the interleaved order [0, 2, 4, 6, 1, 3, 5, 7];
