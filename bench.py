@@ -1,16 +1,16 @@
 """Flagship serving benchmark.
 
-Measures whole-node output tokens/sec of Llama-3-8B in bf16, synthetic random prompts of the CI benchmark
-shape (random 128-token inputs), random-init (dummy) weights, continuous
-decode at a fixed running batch.
+Measures whole-node output tokens/sec of Llama-3-8B in bf16, synthetic
+random prompts of the CI benchmark shape (random 128-token inputs),
+random-init (dummy) weights, continuous decode at a fixed running batch.
 
     python bench.py --gpus N --steps K --warmup W
 
 For N>1 this is launched under torch.distributed.run with one rank per
 GPU; ranks form a TP=N group over RCCL/xGMI (the reference's headline TP
-configs). One "step" is one engine iteration:
-after warmup (which absorbs the prefill of the whole batch) every step
-is a full-batch decode producing `batch` output tokens.
+configs). One "step" is one engine iteration: after warmup (which absorbs
+the prefill of the whole batch) every step is a full-batch decode producing
+`batch` output tokens.
 
 Timing: barrier + torch.cuda.synchronize on both sides of exactly
 --steps engine steps; elapsed is MAX over ranks; rank 0 prints one JSON
