@@ -1,0 +1,126 @@
+"""Linear layers on few rows (csrc/stream_linear.hip): sizes at the edges
+of its forms, parts and epilogues against fp32 products of the same
+operands."""
+
+import pytest
+import torch
+
+from vllm_amd.layers.activation import SiluAndMul
+from vllm_amd.layers.linear import ReplicatedLinear, gated_silu
+
+gpu = pytest.mark.gpu
+
+
+def _operands(m, n, k, dtype):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m * 7919 + n * 31 + k)
+    x = torch.randn(m, k, dtype=dtype, device="cuda", generator=g)
+    w = torch.randn(n, k, dtype=dtype, device="cuda", generator=g)
+    return x, w * k ** -0.5
+
+
+def _check(out, expect, dtype):
+    # fp32 sums of exact products: what is left is the rounding of the
+    # result (half a unit of the last of 7 stored bits in bf16, of 10 in
+    # fp16: 2^-8 and 2^-11 of the value) and, near zero, of sums of terms
+    # of size 1 (K * 2^-24 at the very most, K up to 14336).
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    err = (out.float() - expect).abs() - expect.abs() * unit
+    assert err.max() <= 1e-3, err.max()
+
+
+# Row groups of 8, 16, 32 and 64 at both ends; columns that end within a
+# tile; one step of K for all waves, K split over workgroups, every form.
+SHAPES = [(1, 8, 64), (8, 16, 128), (9, 2112, 7168), (16, 24, 192),
+          (17, 4096, 4096), (32, 1000, 576), (33, 4104, 14336),
+          (64, 2112, 7168), (64, 4096, 4096), (1, 4096, 4096),
+          (64, 6144, 4096), (5, 28672, 512), (64, 28672, 512),
+          (40, 22016, 256), (64, 37888, 256), (3, 128256, 128)]
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_linear(m, n, k, dtype):
+    from vllm_amd.ops import hip_ops
+    x, w = _operands(m, n, k, dtype)
+    bias = torch.randn(n, dtype=dtype, device="cuda")
+    expect = x.float() @ w.float().t()
+    _check(hip_ops.linear(x, w), expect, dtype)
+    _check(hip_ops.linear(x, w, bias), expect + bias.float(), dtype)
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_linear_silu_and_mul(m, n, k, dtype):
+    from vllm_amd.ops import hip_ops
+    x, w = _operands(m, 2 * n if n < 60000 else n, k, dtype)
+    gate, up = (x.float() @ w.float().t()).chunk(2, -1)
+    expect = torch.nn.functional.silu(gate) * up
+    _check(hip_ops.linear_silu_and_mul(x, w), expect, dtype)
+
+
+@gpu
+def test_views_and_other_streams():
+    """Operands that begin off 16 B take the library; launches on several
+    streams whose K is split do not count each other's workgroups."""
+    from vllm_amd.ops import hip_ops
+    x, w = _operands(33, 2112, 7168, torch.bfloat16)
+    expect = x.float() @ w.float().t()
+    odd = torch.empty(x.numel() + 1, dtype=x.dtype, device="cuda")[1:]
+    odd.view(x.shape).copy_(x)
+    _check(hip_ops.linear(odd.view(x.shape), w), expect, x.dtype)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    outs = []
+    for _ in range(4):
+        for s in streams:
+            with torch.cuda.stream(s):
+                outs.append(hip_ops.linear(x, w))
+    torch.cuda.synchronize()
+    for out in outs:
+        assert torch.equal(out, outs[0])
+    _check(outs[0], expect, x.dtype)
+
+
+@gpu
+def test_replays():
+    """A captured product counts in its own counters: replays beside eager
+    calls on the same and on another stream give the same."""
+    from vllm_amd.ops import hip_ops
+    x, w = _operands(33, 2112, 7168, torch.bfloat16)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        eager = hip_ops.linear(x, w)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = hip_ops.linear(x, w)
+    for _ in range(4):
+        out.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            again = hip_ops.linear(x, w)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        assert torch.equal(again, eager)
+
+
+def test_gated_silu_calls_what_is_hooked():
+    """The fused pass goes past the modules only where nothing would be
+    left out: a hook, a bias or an adapter still runs."""
+    proj = ReplicatedLinear(64, 32, dtype=torch.float32)
+    torch.nn.init.normal_(proj.weight)
+    act = SiluAndMul()
+    x = torch.randn(3, 64)
+    expect = act(proj(x))
+    assert torch.equal(gated_silu(proj, act, x), expect)
+    seen = []
+    handle = proj.register_forward_hook(lambda *a: seen.append(1))
+    assert torch.equal(gated_silu(proj, act, x), expect)
+    assert seen == [1]
+    handle.remove()
+    proj.bias = torch.nn.Parameter(torch.ones(32), requires_grad=False)
+    assert torch.equal(gated_silu(proj, act, x), act(proj(x)))

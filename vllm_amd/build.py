@@ -38,6 +38,7 @@ SOURCES = [
     CSRC / "latent_attention.hip",
     CSRC / "latent_attention_tiles.hip",
     CSRC / "ssd.hip",
+    CSRC / "stream_linear.hip",
     CSRC / "gemm_hipblaslt.cpp",
     CSRC / "bindings.cpp",
 ]
@@ -46,7 +47,8 @@ SOURCES = [
 # registers: they are rescaled by the vector ALU between products, and
 # through the accumulation registers every rescale is a copy each way.
 VGPR_ACCUMULATORS = {"attention_decode", "attention_prefill", "mla",
-                     "mla_prompt", "head_matmul", "moe"}
+                     "mla_prompt", "head_matmul", "moe",
+                     "stream_linear"}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("PYTORCH_ROCM_ARCH", "gfx950")

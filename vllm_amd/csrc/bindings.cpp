@@ -36,6 +36,7 @@ void prefill_attention(torch::Tensor out, torch::Tensor q,
                        int64_t max_query_len, int64_t sliding_window);
 torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
                         c10::optional<torch::Tensor> bias);
+torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w);
 torch::Tensor lt_linear_fp8(torch::Tensor a, torch::Tensor w);
 void dynamic_quant_fp8(torch::Tensor out, torch::Tensor scales,
                        torch::Tensor x);
@@ -202,6 +203,7 @@ TORCH_LIBRARY(vllm_amd, m) {
         "float scale, int num_decodes, int max_query_len, "
         "int sliding_window) -> ()");
   m.def("lt_linear(Tensor a, Tensor w, Tensor? bias) -> Tensor");
+  m.def("linear_silu_and_mul(Tensor a, Tensor w) -> Tensor");
   m.def("lt_linear_fp8(Tensor a, Tensor w) -> Tensor");
   m.def("dynamic_quant_fp8(Tensor(a!) out, Tensor(b!) scales, Tensor x)"
         " -> ()");
@@ -327,6 +329,7 @@ TORCH_LIBRARY_IMPL(vllm_amd, CUDA, m) {
   m.impl("paged_decode_attention", &vllm_amd::paged_decode_attention);
   m.impl("prefill_attention", &vllm_amd::prefill_attention);
   m.impl("lt_linear", &vllm_amd::lt_linear);
+  m.impl("linear_silu_and_mul", &vllm_amd::linear_silu_and_mul);
   m.impl("lt_linear_fp8", &vllm_amd::lt_linear_fp8);
   m.impl("dynamic_quant_fp8", &vllm_amd::dynamic_quant_fp8);
   m.impl("scale_rows_cols", &vllm_amd::scale_rows_cols);

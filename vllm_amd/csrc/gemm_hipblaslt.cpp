@@ -27,6 +27,12 @@
 
 namespace vllm_amd {
 
+// stream_linear.hip
+bool stream_linear_takes(const torch::Tensor& x, const torch::Tensor& w,
+                         int64_t n);
+torch::Tensor stream_linear(const torch::Tensor& x, const torch::Tensor& w,
+                            const c10::optional<torch::Tensor>& bias);
+
 namespace {
 
 #define HIP_CHECK(expr)                                              \
@@ -311,9 +317,16 @@ torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
   auto sizes = a.sizes().vec();
   const int64_t K = sizes.back();
   auto a2 = a.reshape({-1, K}).contiguous();
+  sizes.back() = w.size(0);
+  // Few rows stream the weights through a kernel of our own (which side is
+  // faster at which size: stream_linear.hip).
+  if (w.dim() == 2 && stream_linear_takes(a2, w, w.size(0)) &&
+      (!bias.has_value() ||
+       (bias->scalar_type() == a2.scalar_type() && bias->is_contiguous() &&
+        bias->numel() == w.size(0))))
+    return stream_linear(a2, w, bias).reshape(sizes);
   auto out = torch::empty({a2.size(0), w.size(0)}, a.options());
   run_matmul(out, a2, w, bias);
-  sizes.back() = w.size(0);
   return out.reshape(sizes);
 }
 

@@ -1,0 +1,476 @@
+// Linear layers on few rows for MI355X (gfx950):
+//   out[M, N] = x[M, K] @ w[N, K]^T (+ bias), 16-bit operands, fp32 sums,
+// and the same with silu(gate) * up of two halves of w as the epilogue.
+//
+// Up to 64 rows every weight is used too little for anything but HBM to
+// bound the product, if the weights keep coming. Three things decide that:
+//
+//  * Whole 128 B lines. A wave that loads fragments directly takes 64 B of
+//    16 rows at a time; each half line costs as much as a whole one on the
+//    way from L2, and rows of x, read again by every workgroup, run into
+//    that first (4096 x 4096, us for 1 / 8 / 64 rows: fragments directly
+//    8.1 / 9.5 / 23.9, through LDS in whole lines 8.1 / 8.4 / 13.1).
+//  * No waiting on other waves. A wave takes every WV-th run of 64 columns
+//    of K for all rows of its workgroup's tile, so it fills its own ring in
+//    LDS (8 rows x 128 B an instruction, no registers) and waits for its own
+//    fills only; sums meet once, at the end. Each line enters a workgroup
+//    once. Workgroups begin at different places of K, so that they do not
+//    all ask for the same lines of x at a time (28672 x 4096, 64 rows: 48.8
+//    -> 45.7 us).
+//  * Enough workgroups of equal size (plan() below). Narrow layers split K
+//    over workgroups; the last one to arrive adds up the parts in their
+//    order. Parts are written and read past the caches that the XCDs do not
+//    share, a release fence would write back all of L2 (2112 x 7168, 64
+//    rows in three parts: 33 us with fences, 14.7 without, 21.3 in one).
+//
+// us on weights from HBM, tuned library products -> these (floor at 6 TB/s):
+//                   1 row          8 rows         32 rows        64 rows
+//    4096 x 4096    10.5 ->  8.4   10.6 ->  8.4   11.8 -> 10.7   13.8 -> 13.1   (5.6)
+//    6144 x 4096    13.3 -> 11.8   14.5 -> 11.5   15.2 -> 13.9   17.9 -> 17.2   (8.4)
+//   28672 x 4096    51.7 -> 42.7   47.6 -> 42.4   48.3 -> 44.5   54.6 -> 47.4   (39)
+//    4096 x 14336   25.5 -> 23.2   25.7 -> 23.5   31.9 -> 27.1   37.6 -> 32.9   (20)
+//    2112 x 7168    12.2 ->  9.1   12.0 -> 10.6   15.8 -> 11.9   19.3 -> 14.7   (5.0)
+
+#include <torch/all.h>
+#include <c10/hip/HIPStream.h>
+
+#include <algorithm>
+#include <map>
+#include <mutex>
+
+#include "common.h"
+
+namespace vllm_amd {
+
+// gemm_hipblaslt.cpp, elementwise.hip
+torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
+                        c10::optional<torch::Tensor> bias);
+torch::Tensor silu_and_mul(torch::Tensor x);
+
+namespace {
+
+constexpr int SL_ROWS = 64;      // rows of x at most
+constexpr int SL_K = 64;         // columns of K per step of a wave: 128 B
+constexpr int SL_FILL = 1024;    // bytes of a fill: 8 rows x 128 B
+constexpr int SL_PARTS = 8;      // of K, over workgroups
+constexpr int SL_JOBS = 1024;    // column tiles whose K is split
+constexpr int SL_LDS = 160 * 1024;
+
+// Forms: 16-row groups of w per workgroup, waves, ring steps per wave.
+struct Form { int ni, wv, d; };
+constexpr Form SL_FORMS[] = {{1, 8, 4}, {2, 4, 2}, {4, 4, 2},
+                             {6, 4, 2}, {8, 2, 2}, {10, 2, 2}};
+constexpr int SL_NFORMS = sizeof(SL_FORMS) / sizeof(Form);
+
+// xg: groups of 8 rows of x.
+constexpr int ring_bytes(Form f, int xg) {
+  return f.wv * f.d * (2 * f.ni + xg) * SL_FILL;
+}
+constexpr int sums_bytes(Form f, int xg) {
+  return f.wv * f.ni * ((xg + 1) / 2) * WAVE_SIZE * 16;
+}
+constexpr int lds_bytes(Form f, int xg) {
+  return ring_bytes(f, xg) > sums_bytes(f, xg) ? ring_bytes(f, xg)
+                                               : sums_bytes(f, xg);
+}
+
+// Parts of sums travel between workgroups of different XCDs, whose L2s do
+// not see each other: agent-scope accesses go past them.
+DEVINL void put_part(f32x4* p, f32x4 v) {
+  const i32x4 b = __builtin_bit_cast(i32x4, v);
+  uint64_t* q = reinterpret_cast<uint64_t*>(p);
+  __hip_atomic_store(q, (uint64_t)(uint32_t)b[0] | (uint64_t)b[1] << 32,
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, (uint64_t)(uint32_t)b[2] | (uint64_t)b[3] << 32,
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+DEVINL f32x4 get_part(const f32x4* p) {
+  const uint64_t* q = reinterpret_cast<const uint64_t*>(p);
+  const uint64_t a =
+      __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint64_t b =
+      __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __builtin_bit_cast(
+      f32x4, (i32x4){(int)a, (int)(a >> 32), (int)b, (int)(b >> 32)});
+}
+
+// N: columns of out. SILU: w has 2N rows, gate then up; a tile is NI / 2
+// groups of gate rows and the NI / 2 groups of the same columns' up rows.
+template <typename Tag, int NI, int XG, int WV, int D, bool SILU>
+__global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
+    short* __restrict__ out, const short* __restrict__ x,
+    const short* __restrict__ w, const short* __restrict__ bias, const int M,
+    const int N, const int K, const int n_tiles, const int parts,
+    f32x4* __restrict__ part_sums, unsigned* __restrict__ arrived) {
+  constexpr int MT = (XG + 1) / 2;      // 16-row groups of x
+  constexpr int FILLS = 2 * NI + XG;
+  constexpr int STEP = FILLS * SL_FILL;
+  constexpr int NO = SILU ? NI / 2 : NI;
+  static_assert(D > 1 && (D - 1) * FILLS < 64, "what a wait can count");
+  extern __shared__ __align__(16) char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lane = threadIdx.x % WAVE_SIZE;
+  const int l16 = lane & 15;
+  const int l4 = lane >> 4;
+  const int tile = blockIdx.x % n_tiles;
+  const int part = blockIdx.x / n_tiles;
+  const int n0 = tile * NO * 16;
+
+  // Steps of this workgroup's part of K, every WV-th for this wave.
+  const int steps = K / SL_K;
+  const int s0 = steps * part / parts;
+  const int s1 = steps * (part + 1) / parts;
+  const int n = s1 - s0 > wave ? (s1 - s0 - wave + WV - 1) / WV : 0;
+  const int turn = n > 0 ? (int)((blockIdx.x / 8) % (unsigned)n) : 0;
+
+  // Byte places of this lane's pieces in the tile's rows; rows past the
+  // end repeat the last. 16 B chunk c of row r lies at c ^ (r / 2 & 7), so
+  // that the 16 rows of a fragment read meet no bank twice.
+  const int frow = lane >> 3;
+  const char* wbase = reinterpret_cast<const char*>(w + (int64_t)n0 * K);
+  uint32_t wat[2 * NI], xat[XG];
+#pragma unroll
+  for (int i = 0; i < 2 * NI; ++i) {
+    const int r = i * 8 + frow;
+    const int c = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+    const int half = SILU && i >= NI ? 1 : 0;
+    wat[i] = (uint32_t)(min(r - half * NO * 16, N - 1 - n0) + half * N) *
+                 (uint32_t)(K * 2) + c;
+  }
+#pragma unroll
+  for (int i = 0; i < XG; ++i) {
+    const int r = i * 8 + frow;
+    xat[i] = (uint32_t)min(r, M - 1) * (uint32_t)(K * 2) +
+             ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+  }
+  char* ring = lds + wave * (D * STEP);
+  auto fill = [&](int i, int slot) {
+    i = min(i, n - 1) + turn;
+    const int64_t k = (int64_t)(s0 + wave + (i >= n ? i - n : i) * WV) *
+                      (SL_K * 2);
+    char* to = ring + slot * STEP;
+#pragma unroll
+    for (int j = 0; j < 2 * NI; ++j)
+      lds_fill16(wbase + k, wat[j], to + j * SL_FILL);
+#pragma unroll
+    for (int j = 0; j < XG; ++j)
+      lds_fill16(reinterpret_cast<const char*>(x) + k, xat[j],
+                 to + (2 * NI + j) * SL_FILL);
+  };
+
+  f32x4 acc[NI][MT];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // The product is formed transposed: a lane ends up with four neighbouring
+  // columns of row l16. (Of 8 rows the upper lanes repeat the lower.)
+  const int xrow = XG == 1 ? l16 & 7 : l16;
+  auto multiply = [&](int slot) {
+    const char* from = ring + slot * STEP;
+    s16x8 wf[2][NI], xf[2][MT];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        wf[u][i] = *reinterpret_cast<const s16x8*>(
+            from + (i * 16 + l16) * 128 +
+            ((u * 4 + l4) ^ ((l16 >> 1) & 7)) * 16);
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+        xf[u][j] = *reinterpret_cast<const s16x8*>(
+            from + 2 * NI * SL_FILL + (j * 16 + xrow) * 128 +
+            ((u * 4 + l4) ^ ((xrow >> 1) & 7)) * 16);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+          acc[i][j] = mfma16<Tag>(wf[u][i], xf[u][j], acc[i][j]);
+  };
+  if (n > 0) {
+    // Short waves fill the last step more than once: the counts that the
+    // waits go by stay the same.
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d) fill(d, d);
+    int slot = 0, i = 0;
+    for (; i + D - 1 < n; ++i) {
+      fill(i + D - 1, slot == 0 ? D - 1 : slot - 1);
+      lds_fill_wait<(D - 1) * FILLS>();
+      asm volatile("" ::: "memory");
+      multiply(slot);
+      // Read before it is filled again.
+      __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+      asm volatile("" ::: "memory");
+      slot = slot + 1 == D ? 0 : slot + 1;
+    }
+    lds_fill_wait();
+    asm volatile("" ::: "memory");
+    for (; i < n; ++i) {
+      multiply(slot);
+      slot = slot + 1 == D ? 0 : slot + 1;
+    }
+  }
+
+  // Sums of all waves; each wave goes on with a share of the tiles.
+  constexpr int T = NI * MT;
+  constexpr int TO = NO * MT;
+  constexpr int PER = (TO + WV - 1) / WV;
+  f32x4* red = reinterpret_cast<f32x4*>(lds);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+      red[(wave * T + i * MT + j) * WAVE_SIZE + lane] = acc[i][j];
+  __syncthreads();
+  constexpr int H = SILU ? 2 : 1;
+  f32x4 v[PER][H];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int t = u * WV + wave;
+    if (t >= TO) break;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      v[u][h] = red[(h * TO + t) * WAVE_SIZE + lane];
+#pragma unroll
+      for (int q = 1; q < WV; ++q)
+        v[u][h] += red[(q * T + h * TO + t) * WAVE_SIZE + lane];
+    }
+  }
+  if (parts > 1) {
+    f32x4* sums = part_sums + (int64_t)tile * parts * T * WAVE_SIZE + lane;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int t = u * WV + wave;
+      if (t >= TO) break;
+#pragma unroll
+      for (int h = 0; h < H; ++h)
+        put_part(sums + (part * T + h * TO + t) * WAVE_SIZE, v[u][h]);
+    }
+    // Written through before this workgroup counts as arrived.
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    asm volatile("" ::: "memory");
+    __syncthreads();
+    unsigned* last = reinterpret_cast<unsigned*>(lds);
+    if (threadIdx.x == 0) {
+      const unsigned before = __hip_atomic_fetch_add(
+          arrived + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // All have arrived: zero again for the next launch.
+      if (before == (unsigned)parts - 1)
+        __hip_atomic_store(arrived + tile, 0u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      *last = before == (unsigned)parts - 1;
+    }
+    __syncthreads();
+    if (!*last) return;
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int t = u * WV + wave;
+      if (t >= TO) break;
+#pragma unroll
+      for (int h = 0; h < H; ++h) {
+        v[u][h] = get_part(sums + (h * TO + t) * WAVE_SIZE);
+        for (int q = 1; q < parts; ++q)
+          v[u][h] += get_part(sums + (q * T + h * TO + t) * WAVE_SIZE);
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int t = u * WV + wave;
+    if (t >= TO) break;
+    const int row = (t % MT) * 16 + l16;
+    const int col = n0 + (t / MT) * 16 + l4 * 4;
+    f32x4 o = v[u][0];
+    if constexpr (SILU) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        o[r] = o[r] / (1.f + __expf(-o[r])) * v[u][1][r];
+    }
+    if (row >= M || col >= N || (XG == 1 && l16 >= 8)) continue;
+    if (!SILU && bias != nullptr) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] += to_f32<Tag>(bias[col + r]);
+    }
+    *reinterpret_cast<int2*>(out + (int64_t)row * N + col) =
+        int2{pack2<Tag>(o[0], o[1]), pack2<Tag>(o[2], o[3])};
+  }
+}
+
+struct Plan { int form, parts; };
+
+// Form and parts of K by an estimate of the time: weights at 6 TB/s; all
+// that enters workgroups (x again in each) at 15 TB/s; what the fullest CU
+// takes in at 60 GB/s, evened out by two fifths where neighbours still run;
+// 1.5 us and the traffic of the partial sums where K is split. The constants
+// are those that come closest to the best of all forms over 15 layers of
+// 2112 x 7168 to 128256 x 4096 at 1 to 64 rows: 2 % from it on average.
+Plan plan(int xg, int64_t rows_w, int K, bool silu) {
+  Plan best{-1, 1};
+  double least = 1e30;
+  for (int i = 0; i < SL_NFORMS; ++i) {
+    const Form f = SL_FORMS[i];
+    if (lds_bytes(f, xg) > SL_LDS || (silu && f.ni % 2 != 0)) continue;
+    const int64_t tiles = (rows_w + f.ni * 16 - 1) / (f.ni * 16);
+    for (int parts : {1, 2, 3, 4, 6, 8}) {
+      if (parts > 1 && (tiles > SL_JOBS || tiles * parts > 1100 ||
+                        K / SL_K / parts < f.wv))
+        continue;
+      const double mb = (f.ni * 16 + xg * 8) * 2e-6 * K / parts;
+      const double jobs = (double)(tiles * parts);
+      const double cus = (double)((tiles * parts + 255) / 256);
+      const double load =
+          cus > 1 && lds_bytes(f, xg) * 2 > SL_LDS
+              ? cus
+              : 0.6 * cus + 0.4 * std::max(1.0, jobs / 256);
+      double t = std::max({(double)rows_w * K * 2e-6 / 6.0, jobs * mb / 15.0,
+                           load * mb / 0.06});
+      if (parts > 1) t += 1.5 + 0.02 * parts * f.ni * xg;
+      if (t < least) {
+        least = t;
+        best = {i, parts};
+      }
+    }
+  }
+  return best;
+}
+
+// Zeroed counters of the workgroups that arrived; every launch leaves them
+// zero. One set per stream, whose launches follow each other; 32 sets at
+// most. Two kinds of call clear counters of their own: those of a graph,
+// which may run beside the stream that it was captured on, and those of
+// streams that are not torch's (their ids are even handles), which may end
+// and come back as another stream while work is under way.
+torch::Tensor arrival_counters(const torch::Tensor& like) {
+  constexpr size_t SETS = 32;
+  auto opt = like.options().dtype(torch::kInt);
+  const auto stream = c10::hip::getCurrentHIPStream();
+  const int64_t id = stream.id();
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if ((id != 0 && id % 2 == 0) ||
+      hipStreamIsCapturing(stream.stream(), &capturing) != hipSuccess ||
+      capturing != hipStreamCaptureStatusNone)
+    return torch::zeros({SL_JOBS}, opt);
+  // (Never destroyed: the runtime may be gone by then.)
+  static auto* sets = new std::map<std::pair<int, int64_t>, torch::Tensor>();
+  static std::mutex mu;
+  std::lock_guard<std::mutex> guard(mu);
+  const auto key = std::make_pair((int)like.get_device(), id);
+  auto it = sets->find(key);
+  if (it != sets->end()) return it->second;
+  auto t = torch::zeros({SL_JOBS}, opt);
+  if (sets->size() < SETS) sets->emplace(key, t);
+  return t;
+}
+
+template <typename Tag, int I, int XG, bool SILU>
+void launch_form(torch::Tensor& out, const torch::Tensor& x,
+                 const torch::Tensor& w, const short* bias, int N,
+                 int parts) {
+  constexpr Form f = SL_FORMS[I];
+  if constexpr (lds_bytes(f, XG) <= SL_LDS && (!SILU || f.ni % 2 == 0)) {
+    const int M = (int)x.size(0), K = (int)x.size(1);
+    const int cols = f.ni * 16 / (SILU ? 2 : 1);
+    const int tiles = ceil_div(N, cols);
+    torch::Tensor sums, arrived;
+    if (parts > 1) {
+      sums = torch::empty({(int64_t)tiles * parts * f.ni * ((XG + 1) / 2) *
+                           WAVE_SIZE * 4},
+                          x.options().dtype(torch::kFloat));
+      arrived = arrival_counters(x);
+    }
+    hipLaunchKernelGGL(
+        (stream_linear_kernel<Tag, f.ni, XG, f.wv, f.d, SILU>),
+        dim3(tiles * parts), dim3(f.wv * WAVE_SIZE), lds_bytes(f, XG),
+        c10::hip::getCurrentHIPStream().stream(), (short*)out.data_ptr(),
+        (const short*)x.data_ptr(), (const short*)w.data_ptr(), bias, M, N, K,
+        tiles, parts, parts > 1 ? (f32x4*)sums.data_ptr() : nullptr,
+        parts > 1 ? (unsigned*)arrived.data_ptr() : nullptr);
+  } else {
+    TORCH_CHECK(false, "stream_linear: form does not fit");
+  }
+}
+
+template <typename Tag, bool SILU>
+void launch(torch::Tensor& out, const torch::Tensor& x,
+            const torch::Tensor& w, const short* bias, int N) {
+  const int groups = ceil_div((int)x.size(0), 8);
+  const int xg = groups <= 2 ? groups : groups <= 4 ? 4 : 8;
+  const Plan p = plan(xg, w.size(0), (int)x.size(1), SILU);
+  auto by_rows = [&](auto form) {
+    constexpr int I = decltype(form)::value;
+    if (xg == 1) launch_form<Tag, I, 1, SILU>(out, x, w, bias, N, p.parts);
+    else if (xg == 2) launch_form<Tag, I, 2, SILU>(out, x, w, bias, N, p.parts);
+    else if (xg == 4) launch_form<Tag, I, 4, SILU>(out, x, w, bias, N, p.parts);
+    else launch_form<Tag, I, 8, SILU>(out, x, w, bias, N, p.parts);
+  };
+  static_assert(SL_NFORMS == 6);
+  switch (p.form) {
+    case 0: return by_rows(std::integral_constant<int, 0>{});
+    case 1: return by_rows(std::integral_constant<int, 1>{});
+    case 2: return by_rows(std::integral_constant<int, 2>{});
+    case 3: return by_rows(std::integral_constant<int, 3>{});
+    case 4: return by_rows(std::integral_constant<int, 4>{});
+    case 5: return by_rows(std::integral_constant<int, 5>{});
+    default: TORCH_CHECK(false, "stream_linear: no form");
+  }
+}
+
+}  // namespace
+
+// Whether stream_linear takes the product: x [M, K] and w [rows, K], both
+// contiguous; out has n columns.
+bool stream_linear_takes(const torch::Tensor& x, const torch::Tensor& w,
+                         int64_t n) {
+  const int64_t K = x.size(1);
+  return x.size(0) > 0 && x.size(0) <= SL_ROWS && n > 0 && n % 4 == 0 &&
+         K > 0 && K % SL_K == 0 && K < (1 << 24) &&
+         w.size(0) < (1 << 30) && (w.size(0) + 160) * K * 2 < (1ll << 32) &&
+         (x.scalar_type() == torch::kBFloat16 ||
+          x.scalar_type() == torch::kHalf) &&
+         w.scalar_type() == x.scalar_type() && w.size(1) == K &&
+         x.is_contiguous() && w.is_contiguous() &&
+         (uintptr_t)x.data_ptr() % 16 == 0 &&
+         (uintptr_t)w.data_ptr() % 16 == 0;
+}
+
+// x, w and bias as stream_linear_takes and lt_linear have checked them.
+torch::Tensor stream_linear(const torch::Tensor& x, const torch::Tensor& w,
+                            const c10::optional<torch::Tensor>& bias) {
+  const int64_t N = w.size(0);
+  auto out = torch::empty({x.size(0), N}, x.options());
+  const short* b = bias.has_value() ? (const short*)bias->data_ptr() : nullptr;
+  if (x.scalar_type() == torch::kBFloat16)
+    launch<BF16Tag, false>(out, x, w, b, (int)N);
+  else
+    launch<FP16Tag, false>(out, x, w, b, (int)N);
+  HIP_CHECK_KERNEL();
+  return out;
+}
+
+// silu(x @ gate^T) * (x @ up^T), w = [gate; up]; in one launch where
+// stream_linear takes it (the products are then not rounded in between).
+torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w) {
+  TORCH_CHECK(w.dim() == 2 && w.size(0) % 2 == 0 && a.dim() >= 1 &&
+              a.size(-1) == w.size(1) && a.scalar_type() == w.scalar_type(),
+              "linear_silu_and_mul: [.., K] x [2N, K]");
+  auto sizes = a.sizes().vec();
+  auto x = a.reshape({-1, sizes.back()}).contiguous();
+  const int64_t N = w.size(0) / 2;
+  sizes.back() = N;
+  if (!stream_linear_takes(x, w, N))
+    return silu_and_mul(lt_linear(x, w, c10::nullopt)).reshape(sizes);
+  auto out = torch::empty({x.size(0), N}, x.options());
+  if (x.scalar_type() == torch::kBFloat16)
+    launch<BF16Tag, true>(out, x, w, nullptr, (int)N);
+  else
+    launch<FP16Tag, true>(out, x, w, nullptr, (int)N);
+  HIP_CHECK_KERNEL();
+  return out.reshape(sizes);
+}
+
+}  // namespace vllm_amd

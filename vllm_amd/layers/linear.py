@@ -17,7 +17,8 @@ import torch
 import torch.nn as nn
 
 from vllm_amd import ops
-
+from vllm_amd.layers.activation import SiluAndMul
+from vllm_amd.layers.hooks import hooked
 from vllm_amd.parallel.state import (
     get_tp_rank,
     get_tp_world_size,
@@ -64,6 +65,20 @@ def _maybe_apply_lora(module, x, y):
     y2 = y.reshape(-1, y.shape[-1])
     apply_lora_slices(x2, y2, ctx.lora_ids, ctx.lora_manager, slices)
     return y
+
+
+def gated_silu(proj, act, x):
+    """act(proj(x)) of a gated MLP: one pass over the weights where
+    nothing happens between the two but the activation."""
+    if (type(proj) in (MergedColumnParallelLinear, ReplicatedLinear)
+            and type(act) is SiluAndMul
+            and proj.bias is None
+            and getattr(proj, "weight_fp8", None) is None
+            and getattr(proj, "lora_slices", None) is None
+            and not getattr(proj, "gather_output", False)
+            and not hooked(proj, act)):
+        return ops.linear_silu_and_mul(x, proj.weight)
+    return act(proj(x))
 
 
 class ReplicatedLinear(nn.Module):

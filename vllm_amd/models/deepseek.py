@@ -32,6 +32,7 @@ from vllm_amd.layers.linear import (
     MergedColumnParallelLinear,
     ReplicatedLinear,
     RowParallelLinear,
+    gated_silu,
 )
 from vllm_amd.layers.hooks import hooked
 from vllm_amd.layers.rotary import RotaryEmbedding
@@ -236,7 +237,8 @@ class DeepseekDenseMLP(nn.Module):
         self.act_fn = SiluAndMul()
 
     def forward(self, x):
-        return self.down_proj(self.act_fn(self.gate_up_proj(x)))
+        return self.down_proj(
+            gated_silu(self.gate_up_proj, self.act_fn, x))
 
 
 class DeepseekMoE(nn.Module):

@@ -39,7 +39,7 @@ from vllm_amd.layers.attention import PooledWindowAttention
 from vllm_amd.layers.embedding import ParallelLMHead, VocabParallelEmbedding
 from vllm_amd.layers.fused_moe import FusedMoE, TokenTableRouter
 from vllm_amd.layers.layernorm import RMSNorm, ScalarRMSNorm
-from vllm_amd.layers.linear import ReplicatedLinear
+from vllm_amd.layers.linear import ReplicatedLinear, gated_silu
 from vllm_amd.layers.token_shift import TokenShift
 from vllm_amd.parallel.state import get_tp_world_size
 
@@ -111,7 +111,8 @@ class GadilixExpert(nn.Module):
         self.act_fn = SiluAndMul()
 
     def forward(self, x):
-        return self.down_proj(self.act_fn(self.gate_up_proj(x)))
+        return self.down_proj(
+            gated_silu(self.gate_up_proj, self.act_fn, x))
 
 
 class GadilixMoE(nn.Module):

@@ -21,6 +21,7 @@ from vllm_amd.layers.linear import (
     MergedColumnParallelLinear,
     QKVParallelLinear,
     RowParallelLinear,
+    gated_silu,
 )
 from vllm_amd.layers.rotary import RotaryEmbedding
 from vllm_amd.parallel.state import (
@@ -57,8 +58,7 @@ class LlamaMLP(nn.Module):
 
     def forward(self, x, reduce_results: bool = True):
         if self.gated:
-            x = self.gate_up_proj(x)
-            x = self.act_fn(x)
+            x = gated_silu(self.gate_up_proj, self.act_fn, x)
         else:
             x = self.up_proj(x)
             if self.plain_act == "gelu":

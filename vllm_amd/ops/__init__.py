@@ -121,6 +121,11 @@ def linear(x, weight, bias=None):
     return get_backend(x.device).linear(x, weight, bias)
 
 
+def linear_silu_and_mul(x, weight):
+    """silu_and_mul(x @ weight.T), weight = [gate; up]."""
+    return get_backend(x.device).linear_silu_and_mul(x, weight)
+
+
 def linear_fp8(x, w_fp8, w_scale, bias=None):
     """W8A8 fp8 linear: dynamic per-token activation scales, per-channel
     weight scales. fp8 MFMA GEMM on GPU; bit-matching fp32 simulation on

@@ -151,6 +151,10 @@ def linear(x, weight, bias=None):
     return F.linear(x, weight, bias)
 
 
+def linear_silu_and_mul(x, weight):
+    return silu_and_mul(F.linear(x, weight))
+
+
 FP8_MAX = 448.0  # OCP e4m3fn max finite
 
 

@@ -95,6 +95,16 @@ def linear(x, weight, bias=None):
     return _C.lt_linear(x, weight, bias)
 
 
+def linear_silu_and_mul(x, weight):
+    # The activation as the product's epilogue where few rows stream the
+    # weights (csrc/stream_linear.hip); other shapes take two launches.
+    n2, k = weight.shape
+    if (x.dtype == torch.float32 or n2 % 16 or k % 64
+            or x.numel() > 64 * k or x.numel() == 0):
+        return silu_and_mul(linear(x, weight))
+    return _C.linear_silu_and_mul(x, weight)
+
+
 def quant_fp8_dynamic(x):
     # Per-token dynamic quant (csrc/quant_fp8.hip): one workgroup/row.
     M, K = x.shape
