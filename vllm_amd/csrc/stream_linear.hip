@@ -35,6 +35,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <mutex>
 
@@ -59,7 +60,8 @@ constexpr int SL_LDS = 160 * 1024;
 // Forms: 16-row groups of w per workgroup, waves, ring steps per wave.
 struct Form { int ni, wv, d; };
 constexpr Form SL_FORMS[] = {{1, 8, 4}, {2, 4, 2}, {4, 4, 2},
-                             {6, 4, 2}, {8, 2, 2}, {10, 2, 2}};
+                             {6, 4, 2}, {8, 4, 2}, {8, 2, 2},
+                             {10, 2, 2}};
 constexpr int SL_NFORMS = sizeof(SL_FORMS) / sizeof(Form);
 
 // xg: groups of 8 rows of x.
@@ -303,18 +305,24 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
 
 struct Plan { int form, parts; };
 
-// Form and parts of K by an estimate of the time: weights at 6 TB/s; all
-// that enters workgroups (x again in each) at 15 TB/s; what the fullest CU
-// takes in at 60 GB/s, evened out by two fifths where neighbours still run;
-// 1.5 us and the traffic of the partial sums where K is split. The constants
-// are those that come closest to the best of all forms over 15 layers of
-// 2112 x 7168 to 128256 x 4096 at 1 to 64 rows: 2 % from it on average.
+// Form and parts of K by an estimate of the time, of which these bound it
+// (added as fourth powers): weights at 6 TB/s; all that enters workgroups, x
+// again in each, at 15 TB/s; what the fullest CU takes in at 60 GB/s, evened
+// out by two fifths where neighbours still run. A workgroup's start costs
+// 0.2 us of its CU, splitting K 1.5 us and the traffic of partial sums. The
+// constants are those that come closest to the best of all forms over 15
+// layers of 2112 x 7168 to 128256 x 4096 at 1 to 64 rows: 1.3 % from it on
+// average, 7 % at most.
 Plan plan(int xg, int64_t rows_w, int K, bool silu) {
   Plan best{-1, 1};
   double least = 1e30;
+  auto fourth = [](double v) { return v * v * v * v; };
   for (int i = 0; i < SL_NFORMS; ++i) {
     const Form f = SL_FORMS[i];
-    if (lds_bytes(f, xg) > SL_LDS || (silu && f.ni % 2 != 0)) continue;
+    // Two waves have too little on the way where four fit.
+    if (lds_bytes(f, xg) > SL_LDS || (f.wv == 2 && xg < 8) ||
+        (silu && f.ni % 2 != 0))
+      continue;
     const int64_t tiles = (rows_w + f.ni * 16 - 1) / (f.ni * 16);
     for (int parts : {1, 2, 3, 4, 6, 8}) {
       if (parts > 1 && (tiles > SL_JOBS || tiles * parts > 1100 ||
@@ -327,9 +335,11 @@ Plan plan(int xg, int64_t rows_w, int K, bool silu) {
           cus > 1 && lds_bytes(f, xg) * 2 > SL_LDS
               ? cus
               : 0.6 * cus + 0.4 * std::max(1.0, jobs / 256);
-      double t = std::max({(double)rows_w * K * 2e-6 / 6.0, jobs * mb / 15.0,
-                           load * mb / 0.06});
-      if (parts > 1) t += 1.5 + 0.02 * parts * f.ni * xg;
+      double t = std::sqrt(std::sqrt(fourth(rows_w * 2e-6 * K / 6.0) +
+                                     fourth(jobs * mb / 15.0) +
+                                     fourth(load * mb / 0.06))) +
+                 0.2 * jobs / 256;
+      if (parts > 1) t += 1.5 + 0.04 * parts * f.ni * xg;
       if (t < least) {
         least = t;
         best = {i, parts};
@@ -372,7 +382,8 @@ void launch_form(torch::Tensor& out, const torch::Tensor& x,
                  const torch::Tensor& w, const short* bias, int N,
                  int parts) {
   constexpr Form f = SL_FORMS[I];
-  if constexpr (lds_bytes(f, XG) <= SL_LDS && (!SILU || f.ni % 2 == 0)) {
+  if constexpr (lds_bytes(f, XG) <= SL_LDS && (f.wv > 2 || XG == 8) &&
+                (!SILU || f.ni % 2 == 0)) {
     const int M = (int)x.size(0), K = (int)x.size(1);
     const int cols = f.ni * 16 / (SILU ? 2 : 1);
     const int tiles = ceil_div(N, cols);
@@ -408,7 +419,7 @@ void launch(torch::Tensor& out, const torch::Tensor& x,
     else if (xg == 4) launch_form<Tag, I, 4, SILU>(out, x, w, bias, N, p.parts);
     else launch_form<Tag, I, 8, SILU>(out, x, w, bias, N, p.parts);
   };
-  static_assert(SL_NFORMS == 6);
+  static_assert(SL_NFORMS == 7);
   switch (p.form) {
     case 0: return by_rows(std::integral_constant<int, 0>{});
     case 1: return by_rows(std::integral_constant<int, 1>{});
@@ -416,6 +427,7 @@ void launch(torch::Tensor& out, const torch::Tensor& x,
     case 3: return by_rows(std::integral_constant<int, 3>{});
     case 4: return by_rows(std::integral_constant<int, 4>{});
     case 5: return by_rows(std::integral_constant<int, 5>{});
+    case 6: return by_rows(std::integral_constant<int, 6>{});
     default: TORCH_CHECK(false, "stream_linear: no form");
   }
 }
