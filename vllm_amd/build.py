@@ -24,6 +24,7 @@ SOURCES = [
     CSRC / "elementwise.hip",
     CSRC / "comms.hip",
     CSRC / "moe.hip",
+    CSRC / "moe_tiles.hip",
     CSRC / "mla.hip",
     CSRC / "mla_prompt.hip",
     CSRC / "mla_prepare.hip",
@@ -93,8 +94,7 @@ def needs_build() -> bool:
     if not OUT_SO.exists():
         return True
     so_mtime = OUT_SO.stat().st_mtime
-    deps = list(SOURCES) + [CSRC / "common.h",
-                            CSRC / "pooled_attention.h", Path(__file__)]
+    deps = list(SOURCES) + sorted(CSRC.glob("*.h")) + [Path(__file__)]
     return any(p.stat().st_mtime > so_mtime for p in deps)
 
 

@@ -18,7 +18,7 @@
 //                      ([E][N/16][K/32][64 lanes][8], ops/hip_ops.py
 //                      moe_shuffle_weights): then a wave's load is one run
 //                      of 1 KB.
-//   moe_tile_kernel    many rows: the matrix cores bound it; 128 or 256 x
+//   moe_tiles.hip      many rows: the matrix cores bound it; 128 or 256 x
 //                      256 tiles through LDS.
 //
 // Pipeline (ops/hip_ops.py fused_moe):
@@ -32,7 +32,8 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
-#include "common.h"
+#include "moe.h"
+#include "tile_product.h"
 
 namespace vllm_amd {
 
@@ -168,49 +169,6 @@ __global__ __launch_bounds__(THREADS) void align_scatter_kernel(
 }
 
 // --------------------------------------------------------------------------
-// What the epilogue of a product does.
-enum Act { NONE = 0, SILU_GATED = 1, RELU2 = 2 };
-
-DEVINL float silu_mul(float g, float u) { return g / (1.f + __expf(-g)) * u; }
-DEVINL float relu2(float x) {
-  const float r = fmaxf(x, 0.f);
-  return r * r;
-}
-
-// Which (row tile, column block) a workgroup takes; every eighth workgroup
-// runs on the same XCD. Streamed weights: each XCD takes a run of
-// neighbours in (column block, row tile) order.
-DEVINL bool tile_of_block(int m_tiles, int n_blocks, int& m, int& n) {
-  const int total = m_tiles * n_blocks;
-  const int per = (total + 7) / 8;
-  const int l = (int)blockIdx.x >> 3;
-  const int p = ((int)blockIdx.x & 7) * per + l;
-  if (l >= per || p >= total) return false;
-  m = p % m_tiles;
-  n = p / m_tiles;
-  return true;
-}
-// Tiles: `split` parts of the column blocks times 8 / split parts of the
-// row tiles that hold rows, one part of each per XCD; eight row tiles by
-// some column blocks run there at a time, so tiles of an expert share
-// weights and blocks share rows in its L2.
-DEVINL bool tile_of_block(int tiles, int n_blocks, int split, int& m,
-                          int& n) {
-  constexpr int GROUP = 8;
-  const int x = (int)blockIdx.x & 7;
-  const int l = (int)blockIdx.x >> 3;
-  const int parts = 8 / split, y = x / split, c = x % split;
-  const int m0 = tiles * y / parts, mm = tiles * (y + 1) / parts - m0;
-  const int n_lo = n_blocks * c / split;
-  const int nn = n_blocks * (c + 1) / split - n_lo;
-  if (l >= mm * nn) return false;
-  const int g = l / (GROUP * nn), q = l - g * (GROUP * nn);
-  const int rows = min(GROUP, mm - g * GROUP);
-  m = m0 + g * GROUP + q % rows;
-  n = n_lo + q / rows;
-  return true;
-}
-
 // Into how many parts the column blocks go: three or more blocks each and
 // no more than a tenth of unevenness, more only where row tiles are few.
 // Measured in 8 / 4 / 2 / 1 parts, ms: 8 experts, 4096 x 14336 (112 and 16
@@ -343,18 +301,6 @@ DEVINL void stream_body(const short* const (&wp)[4],
   }
 }
 
-// Rows of this tile that hold a (token, slot) pair: they come first.
-template <int TM>
-DEVINL int rows_of_tile(const int* __restrict__ sorted, int tile,
-                        int total_flat) {
-  int n = 0;
-#pragma unroll
-  for (int i = 0; i < TM; i += WAVE_SIZE)
-    n += __popcll(__ballot(
-        sorted[tile * TM + i + (threadIdx.x % WAVE_SIZE)] < total_flat));
-  return n;
-}
-
 template <typename Tag, int ACT, bool SHUF>
 __launch_bounds__(THREADS, 2) __global__
 void moe_stream_kernel(const short* __restrict__ A, int64_t lda,
@@ -363,7 +309,7 @@ void moe_stream_kernel(const short* __restrict__ A, int64_t lda,
                        const int* __restrict__ sorted,
                        const int* __restrict__ expert_tiles, int K, int N,
                        int topk_div, int total_flat, int m_tiles,
-                       int n_blocks, int split) {
+                       int n_blocks) {
   int tile, blk;
   if (!tile_of_block(m_tiles, n_blocks, tile, blk)) return;
   const int expert = expert_tiles[tile];
@@ -407,290 +353,6 @@ void moe_stream_kernel(const short* __restrict__ A, int64_t lda,
   else
     stream_body<Tag, ACT, STEP, 4>(wp, xp, s0, s1, red, wave, lane, rows, c,
                                    ldc, n0, N);
-}
-
-// --------------------------------------------------------------------------
-// Many rows. TM x 256 tiles (128 gate + 128 up weight rows for gated
-// experts) by eight waves, two a SIMD; K goes by 64 (whole 128 B lines: by
-// 32 it was 10 % slower), stages are filled straight from global memory
-// and rotate, one barrier a stage. The product is formed transposed
-// (weight rows are the A operand), so a lane ends up with four
-// neighbouring columns of one row, eight after a trade with the other half
-// wave (16 B stores: the second product 5 % faster). 32-row groups without
-// a row are left out, by wave, so padding costs fills but few products.
-//   WM 4, 256 rows: waves of 64 x 128, half the traffic from L2 per
-//                   product, reads and products of the two halves of the
-//                   workgroup in turn, weights filled two steps ahead.
-//                   64 experts x 512 rows of 7168 x 2048: all waves in step
-//                   3.41 ms, in turn 3.24, weights ahead 3.17; 8 experts x
-//                   1024 rows of 4096 x 14336 3.18, 2.90, 2.82 (1020
-//                   TFLOP/s). Products alone would take 2.5 ms, with
-//                   weights always in L2 2.6.
-//   WM 2, 128 rows: waves of 64 x 64, three stages. For experts of few
-//                   rows, and for what is left of an expert's rows after
-//                   whole tiles of 256.
-// (Four waves of 64 x 128 or 128 x 128 left the matrix cores waiting for a
-// single wave per SIMD; five stages of 32 fetch half lines: 2 % slower.)
-constexpr int TL_W = 256;
-constexpr int TL_K = 64;
-constexpr int TL_THREADS = 8 * WAVE_SIZE;
-constexpr int TL_LDS = 160 * 1024;                   // all there is
-constexpr int TL_ROW = TL_K * 2;                     // bytes of a row
-constexpr int TL_CH = TL_ROW / 16;                   // 16 B chunks of a row
-constexpr int TL_FR = WAVE_SIZE / TL_CH;             // rows a fill moves
-
-// The eight chunks of a row are exchanged by the row / 2, so that the 16
-// rows a fragment read takes the same chunk from lie on all banks.
-DEVINL int tl_swap(int row) { return (row >> 1) & 7; }
-
-// One tile by waves of (8 / WM columns of) WM rows of 64; `row0` is its
-// first row in tile order.
-template <typename Tag, int ACT, int WM>
-DEVINL void tile_body(char* lds, const short* __restrict__ A, int64_t lda,
-                      const short* __restrict__ W, short* __restrict__ C,
-                      int64_t ldc, const int* __restrict__ sorted, int K,
-                      int N, int topk_div, int row0, int rows, int n0) {
-  constexpr int TL_M = WM * 64;
-  constexpr int TL_WN = 8 / WM;            // waves along the weight rows
-  constexpr int TL_WW = TL_W / TL_WN;      // weight rows of a wave
-  constexpr int TL_WI = TL_WW / 32;
-  constexpr int TL_MI = 2;                 // 32-row groups of a wave
-  constexpr int TL_FA = TL_M / TL_FR / 8;  // fills per wave
-  constexpr int TL_FW = TL_W / TL_FR / 8;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
-  const int lane = threadIdx.x % WAVE_SIZE;
-  const int l32 = lane & 31;
-  const int half = lane >> 5;
-  const int wm = wave / TL_WN;   // (a SIMD's two waves take other rows)
-  const int wn = wave % TL_WN;
-
-  const int frow = lane / TL_CH;
-  uint32_t ap[TL_FA], wp[TL_FW];   // byte places in A and W
-#pragma unroll
-  for (int i = 0; i < TL_FA; ++i) {
-    const int lr = (wave * TL_FA + i) * TL_FR + frow;
-    const int r = row0 + min(lr, rows - 1);
-    ap[i] = (uint32_t)(topk_div > 0 ? sorted[r] / topk_div : r) *
-                (uint32_t)lda * 2 +
-            ((lane % TL_CH) ^ tl_swap(lr)) * 16;
-  }
-#pragma unroll
-  for (int i = 0; i < TL_FW; ++i) {
-    const int r = (wave * TL_FW + i) * TL_FR + frow;
-    uint32_t src;
-    if constexpr (ACT == SILU_GATED)   // a wave's gate rows, their up rows
-      src = min(n0 + r / TL_WW * (TL_WW / 2) + r % (TL_WW / 2), N - 1) +
-            r / (TL_WW / 2) % 2 * N;
-    else
-      src = min(n0 + r, N - 1);
-    wp[i] = src * (uint32_t)K * 2 + ((lane % TL_CH) ^ tl_swap(r)) * 16;
-  }
-  auto fill_a = [&](int step, char* dst) {
-#pragma unroll
-    for (int i = 0; i < TL_FA; ++i)
-      lds_fill16(A + step * TL_K, ap[i], dst + (wave * TL_FA + i) * 1024);
-  };
-  auto fill_w = [&](int step, char* dst) {
-#pragma unroll
-    for (int i = 0; i < TL_FW; ++i)
-      lds_fill16(W + step * TL_K, wp[i], dst + (wave * TL_FW + i) * 1024);
-  };
-
-  f32x16 acc[TL_WI][TL_MI];
-#pragma unroll
-  for (int i = 0; i < TL_WI; ++i)
-#pragma unroll
-    for (int j = 0; j < TL_MI; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  // 32-row groups of this wave that hold a row at all.
-  const int groups = min(TL_MI, (rows - wm * TL_MI * 32 + 31) / 32);
-  const int steps = K / TL_K;
-  int at[TL_K / 16];   // byte places of this lane's fragments of a row group
-#pragma unroll
-  for (int kk = 0; kk < TL_K / 16; ++kk)
-    at[kk] = l32 * TL_ROW + (((kk * 2 + half) ^ tl_swap(l32)) * 16);
-  if constexpr (WM == 4) {
-    // Waves 4..7 run one slot behind waves 0..3, their neighbours on the
-    // SIMDs: one half multiplies 32 of K while the other reads the next 32
-    // into fragments, a barrier a slot, four slots a step. A step's first
-    // slot starts the fills of the next step's rows and of the weights one
-    // further on, which come from HBM (three places for weights, two for
-    // rows; the laggards read the places these take last in the slot
-    // before). When its fourth ends, all the next step needs has landed.
-    // The number of row groups is a constant of the loop: merging
-    // accumulators of several branches would copy them.
-    const int lag = wave >> 2;
-    constexpr int AB = TL_M * TL_ROW, WB = TL_W * TL_ROW;
-    static_assert(2 * AB + 3 * WB <= TL_LDS);
-    const char* a0 = lds + wm * TL_MI * 32 * TL_ROW;
-    const char* w0 = lds + 2 * AB + wn * TL_WW * TL_ROW;
-    auto run = [&](auto n) {
-      constexpr int J = decltype(n)::value;
-      s16x8 af[2][J > 0 ? J : 1], wf[2][TL_WI];
-      auto read = [&](int stage, int wst, int k0) {
-        if constexpr (J > 0) {
-#pragma unroll
-          for (int k = 0; k < 2; ++k) {
-#pragma unroll
-            for (int j = 0; j < J; ++j)
-              af[k][j] = *reinterpret_cast<const s16x8*>(
-                  a0 + stage * AB + j * 32 * TL_ROW + at[k0 + k]);
-#pragma unroll
-            for (int i = 0; i < TL_WI; ++i)
-              wf[k][i] = *reinterpret_cast<const s16x8*>(
-                  w0 + wst * WB + i * 32 * TL_ROW + at[k0 + k]);
-          }
-        }
-      };
-      auto multiply = [&]() {
-        if constexpr (J > 0) {
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int i = 0; i < TL_WI; ++i)
-#pragma unroll
-              for (int j = 0; j < J; ++j)
-                acc[i][j] = mfma32<Tag>(wf[k][i], af[k][j], acc[i][j]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      };
-      if (lag) lds_barrier();   // (as many barriers for every wave)
-#pragma unroll 1
-      for (int s = 0, wst = 0; s < steps; ++s) {
-        const int stage = s & 1;
-        if (s + 1 < steps) fill_a(s + 1, lds + (stage ^ 1) * AB);
-        if (s + 2 < steps)
-          fill_w(s + 2, lds + 2 * AB + (wst == 0 ? 2 : wst - 1) * WB);
-        auto landed = [&]() {
-          if (s + 2 < steps) lds_fill_wait<TL_FW>();
-          else lds_fill_wait();
-        };
-        read(stage, wst, 0);
-        lds_barrier();
-        multiply();
-        lds_barrier();
-        read(stage, wst, 2);
-        if (lag) landed();
-        lds_barrier();
-        multiply();
-        if (!lag) landed();
-        lds_barrier();
-        wst = wst == 2 ? 0 : wst + 1;
-      }
-      if (!lag) lds_barrier();
-    };
-    fill_a(0, lds);
-    fill_w(0, lds + 2 * AB);
-    if (steps > 1) fill_w(1, lds + 2 * AB + WB);
-    if (steps > 1) lds_fill_wait<TL_FW>();
-    else lds_fill_wait();
-    lds_barrier();
-    if (groups >= 2) run(std::integral_constant<int, 2>{});
-    else if (groups == 1) run(std::integral_constant<int, 1>{});
-    else run(std::integral_constant<int, 0>{});
-  } else {
-    constexpr int TL_STAGES = 3;
-    constexpr int TL_STAGE = (TL_M + TL_W) * TL_ROW;   // bytes
-    static_assert(TL_STAGES * TL_STAGE <= TL_LDS);
-    auto fill = [&](int step, int stage) {
-      fill_a(step, lds + stage * TL_STAGE);
-      fill_w(step, lds + stage * TL_STAGE + TL_M * TL_ROW);
-    };
-#pragma unroll
-    for (int i = 0; i < TL_STAGES - 1; ++i)
-      if (i < steps) fill(i, i);
-    int stage = 0;
-    for (int s = 0; s < steps; ++s) {
-      // This stage has landed when at most the next one's fills are under
-      // way; past the barrier every wave is done with the stage before.
-      if (s + 1 < steps) lds_fill_wait<TL_FA + TL_FW>();
-      else lds_fill_wait();
-      lds_barrier();
-      if (s + TL_STAGES - 1 < steps)
-        fill(s + TL_STAGES - 1, stage == 0 ? TL_STAGES - 1 : stage - 1);
-      const char* a = lds + stage * TL_STAGE + wm * TL_MI * 32 * TL_ROW;
-      const char* w =
-          lds + stage * TL_STAGE + (TL_M + wn * TL_WW) * TL_ROW;
-      auto multiply = [&](auto n) {
-        constexpr int J = decltype(n)::value;
-#pragma unroll
-        for (int kk = 0; kk < TL_K / 16; ++kk) {
-          s16x8 af[J], wf[TL_WI];
-#pragma unroll
-          for (int j = 0; j < J; ++j)
-            af[j] =
-                *reinterpret_cast<const s16x8*>(a + j * 32 * TL_ROW + at[kk]);
-#pragma unroll
-          for (int i = 0; i < TL_WI; ++i)
-            wf[i] =
-                *reinterpret_cast<const s16x8*>(w + i * 32 * TL_ROW + at[kk]);
-#pragma unroll
-          for (int i = 0; i < TL_WI; ++i)
-#pragma unroll
-            for (int j = 0; j < J; ++j)
-              acc[i][j] = mfma32<Tag>(wf[i], af[j], acc[i][j]);
-        }
-      };
-      if (groups >= 2) multiply(std::integral_constant<int, 2>{});
-      else if (groups == 1) multiply(std::integral_constant<int, 1>{});
-      stage = stage == TL_STAGES - 1 ? 0 : stage + 1;
-    }
-  }
-
-  // Register r of acc[i][j]: weight row i*32 + 8*(r/4) + 4*half + r%4,
-  // token row j*32 + l32.
-#pragma unroll
-  for (int j = 0; j < TL_MI; ++j) {
-    const int row = wm * TL_MI * 32 + j * 32 + l32;
-    if (row >= rows) continue;
-    short* c = C + (int64_t)(row0 + row) * ldc;
-#pragma unroll
-    for (int i = 0; i < (ACT == SILU_GATED ? TL_WI / 2 : TL_WI); ++i) {
-      f32x16 v = acc[i][j];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        if constexpr (ACT == SILU_GATED)
-          v[r] = silu_mul(v[r], acc[i + TL_WI / 2][j][r]);
-        else if constexpr (ACT == RELU2)
-          v[r] = relu2(v[r]);
-      }
-#pragma unroll
-      for (int b = 0; b < 4; b += 2) {
-        const i32x4 o = row_chunk<Tag>(v, b);
-        const int col = n0 + wn * (ACT == SILU_GATED ? TL_WW / 2 : TL_WW) +
-                        i * 32 + b * 8 + half * 8;
-        if (col < N) *reinterpret_cast<i32x4*>(c + col) = o;
-      }
-    }
-  }
-}
-
-template <typename Tag, int ACT, int TM>
-__launch_bounds__(TL_THREADS, 2) __global__
-void moe_tile_kernel(const short* __restrict__ A, int64_t lda,
-                     const short* __restrict__ W, int64_t expert_stride,
-                     short* __restrict__ C, int64_t ldc,
-                     const int* __restrict__ sorted,
-                     const int* __restrict__ expert_tiles, int K, int N,
-                     int topk_div, int total_flat, int m_tiles,
-                     int n_blocks, int split) {
-  int tile, blk;
-  if (!tile_of_block(expert_tiles[m_tiles], n_blocks, split, tile, blk))
-    return;
-  const int expert = expert_tiles[tile];
-  __shared__ __align__(16) char lds[TL_LDS];
-  const int rows = rows_of_tile<TM>(sorted, tile, total_flat);
-  const int n0 = blk * (ACT == SILU_GATED ? TL_W / 2 : TL_W);
-  W += expert * expert_stride;
-  if (TM == 128 || rows <= 128)
-    tile_body<Tag, ACT, 2>(lds, A, lda, W, C, ldc, sorted, K, N, topk_div,
-                           tile * TM, rows, n0);
-  else
-    tile_body<Tag, ACT, 4>(lds, A, lda, W, C, ldc, sorted, K, N, topk_div,
-                           tile * TM, rows, n0);
 }
 
 // --------------------------------------------------------------------------
@@ -794,7 +456,7 @@ static void run_gemm(const torch::Tensor& a, const torch::Tensor& b,
   const int N = (int)c.size(1);
   TORCH_CHECK(act >= NONE && act <= RELU2);
   TORCH_CHECK(b_rows == (act == SILU_GATED ? 2 : 1) * (int64_t)N);
-  TORCH_CHECK(K % (form > 0 ? TL_K : 32) == 0 &&
+  TORCH_CHECK(K % (form > 0 ? TP_K : 32) == 0 &&
                   N % (shuf ? 16 : form > 0 ? 8 : 4) == 0,
               "K must be a multiple of 32, N of 4 (tiles: 64 and 8; in "
               "fragment order N of 16)");
@@ -820,23 +482,35 @@ static void run_gemm(const torch::Tensor& a, const torch::Tensor& b,
                             (uintptr_t)b.data_ptr() % 16 == 0));
   TORCH_CHECK(blocks < (1ll << 30));
   auto stream = c10::hip::getCurrentHIPStream().stream();
+  if (form > 0) {
+    TORCH_CHECK(a.scalar_type() == torch::kBFloat16 ||
+                    a.scalar_type() == torch::kHalf,
+                "moe_gemm: bf16/fp16 only");
+    launch_tiles({(const short*)a.data_ptr(), a.size(1),
+                  (const short*)b.data_ptr(), b_rows * K,
+                  (short*)c.data_ptr(), c.size(1), sorted.data_ptr<int>(),
+                  expert_tiles.data_ptr<int>(), K, N, (int)topk_div,
+                  (int)total_flat, m_tiles, n_blocks, split},
+                 (int)form, (int)act, a.scalar_type() == torch::kBFloat16,
+                 (unsigned)blocks, stream);
+    HIP_CHECK_KERNEL();
+    return;
+  }
   dim3 grid((unsigned)blocks);
   auto launch = [&](auto tag, auto act_tag) {
     using Tag = decltype(tag);
     constexpr int ACT = decltype(act_tag)::value;
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(
-          kernel, grid, dim3(form > 0 ? TL_THREADS : THREADS), 0, stream,
+          kernel, grid, dim3(THREADS), 0, stream,
           (const short*)a.data_ptr(),
           a.size(1), (const short*)b.data_ptr(), b_rows * K,
           (short*)c.data_ptr(), c.size(1), sorted.data_ptr<int>(),
           expert_tiles.data_ptr<int>(), K, N, (int)topk_div, (int)total_flat,
-          m_tiles, n_blocks, split);
+          m_tiles, n_blocks);
     };
-    if (form == 2)      go(moe_tile_kernel<Tag, ACT, 256>);
-    else if (form == 1) go(moe_tile_kernel<Tag, ACT, 128>);
-    else if (shuf)      go(moe_stream_kernel<Tag, ACT, true>);
-    else                go(moe_stream_kernel<Tag, ACT, false>);
+    if (shuf) go(moe_stream_kernel<Tag, ACT, true>);
+    else      go(moe_stream_kernel<Tag, ACT, false>);
   };
   auto by_act = [&](auto tag) {
     if (act == SILU_GATED)

@@ -1,0 +1,149 @@
+// Grouped expert products for experts of many rows (gfx950): 128 or 256 x
+// 256 tiles of tile_product.h, the matrix cores bound them. The product is
+// formed transposed (weight rows are the A operand), so a lane ends up with
+// four neighbouring columns of one row, eight after a trade with the other
+// half wave (16 B stores). Gated experts: a tile is 128 gate rows and the up
+// rows of the same columns, a wave's gate groups before its up groups, and
+// the activation is the epilogue.
+//
+// Tiles of at most 128 rows (what is left of an expert after whole tiles,
+// or experts of few rows) lay the four waves out along the weights; 32-row
+// groups without a row are left out.
+//
+// 64 experts of 7168 x 2048, 4096 tokens of 8, 50 to 1925 rows an expert:
+// 1.76 + 0.98 ms (eight waves by halves in turn 2.01 + 1.10); 512 rows each
+// 1.50 + 0.86 (1.28 and 1.12 PFLOP/s: the second, of 32 stages, pays the
+// start and end of its tiles). What uneven rows cost beyond their padding
+// is weights read twice: tiles of an expert that are not in step do not
+// meet in L2 (8.3 GB instead of 4.1 in the first product).
+
+#include <torch/all.h>
+#include <c10/hip/HIPStream.h>
+
+#include "moe.h"
+#include "tile_product.h"
+
+namespace vllm_amd {
+
+namespace moe {
+
+// One tile by TileProduct; `row0` is its first row in tile order.
+template <typename Tag, int ACT, int WGM, int NI, int MI, int PA>
+DEVINL void tile_body(char* lds, const TileArgs& t, const short* w,
+                      const int row0, const int rows, const int n0) {
+  using P = TileProduct<Tag, WGM, NI, MI, PA, 3>;
+  static_assert(P::TN == TL_W && P::WW * P::WGN == TL_W);
+  constexpr bool GATED = ACT == SILU_GATED;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lane = threadIdx.x % WAVE_SIZE;
+  const int l32 = lane & 31;
+  const int half = lane >> 5;
+  const int N = t.N;
+
+  uint32_t ap[P::FA], wp[P::FW];   // byte places of this lane's pieces
+#pragma unroll
+  for (int i = 0; i < P::FA; ++i) {
+    const int lr = (wave * P::FA + i) * 8 + (lane >> 3);
+    const int r = row0 + min(lr, rows - 1);
+    ap[i] = (uint32_t)(t.topk_div > 0 ? t.sorted[r] / t.topk_div : r) *
+                (uint32_t)t.lda * 2 +
+            ((lane & 7) ^ tp_swap(lr)) * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < P::FW; ++i) {
+    const int r = (wave * P::FW + i) * 8 + (lane >> 3);
+    int src;
+    if constexpr (GATED)   // a wave's gate rows, their up rows
+      src = min(n0 + r / P::WW * (P::WW / 2) + r % (P::WW / 2), N - 1) +
+            r / (P::WW / 2) % 2 * N;
+    else
+      src = min(n0 + r, N - 1);
+    wp[i] = (uint32_t)src * (uint32_t)t.K * 2 +
+            ((lane & 7) ^ tp_swap(r)) * 16;
+  }
+  P::run(
+      lds, t.K / TP_K, rows,
+      [&](int s, int i, char* dst) { lds_fill16(t.a + s * TP_K, ap[i], dst); },
+      [&](int s, int i, char* dst) { lds_fill16(w + s * TP_K, wp[i], dst); },
+      [&](auto n, auto& acc) {
+        constexpr int J = decltype(n)::value;
+        constexpr int NO = GATED ? NI / 2 : NI;
+        // Register r of acc[i][j]: weight row i*32 + 8*(r/4) + 4*half + r%4
+        // of the wave, row l32 of its group j.
+        const int wm = wave / P::WGN, wn = wave % P::WGN;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const int row = (j * WGM + wm) * 32 + l32;
+          if (row >= rows) continue;
+          short* c = t.c + (int64_t)(row0 + row) * t.ldc;
+#pragma unroll
+          for (int i = 0; i < NO; ++i) {
+            f32x16 v = acc[i][j];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              if constexpr (GATED)
+                v[r] = silu_mul(v[r], acc[i + NI / 2][j][r]);
+              else if constexpr (ACT == RELU2)
+                v[r] = relu2(v[r]);
+            }
+#pragma unroll
+            for (int b = 0; b < 4; b += 2) {
+              const i32x4 o = row_chunk<Tag>(v, b);
+              const int col = n0 + wn * NO * 32 + i * 32 + b * 8 + half * 8;
+              if (col < N) *reinterpret_cast<i32x4*>(c + col) = o;
+            }
+          }
+        }
+      });
+}
+
+template <typename Tag, int ACT, int TM>
+__launch_bounds__(TP_THREADS, 1) __global__
+void moe_tile_kernel(const TileArgs t) {
+  int tile, blk;
+  if (!tile_of_block(t.expert_tiles[t.m_tiles], t.n_blocks, t.split, tile,
+                     blk))
+    return;
+  using Whole = TileProduct<Tag, 2, 4, 4, 2, 3>;
+  using Half = TileProduct<Tag, 1, 2, 4, 3, 3>;
+  static_assert(Whole::TM == 256 && Half::TM == 128);
+  __shared__ __align__(16) char lds[TM == 256 ? Whole::LDS : Half::LDS];
+  const int rows = rows_of_tile<TM>(t.sorted, tile, t.total_flat);
+  const int n0 = blk * (ACT == SILU_GATED ? TL_W / 2 : TL_W);
+  const short* w = t.w + t.expert_tiles[tile] * t.expert_stride;
+  if constexpr (TM == 256) {
+    if (rows > 128) {
+      tile_body<Tag, ACT, 2, 4, 4, 2>(lds, t, w, tile * TM, rows, n0);
+      return;
+    }
+  }
+  tile_body<Tag, ACT, 1, 2, 4, 3>(lds, t, w, tile * TM, rows, n0);
+}
+
+void launch_tiles(const TileArgs& t, int form, int act, bool bf16,
+                  unsigned blocks, hipStream_t stream) {
+  auto launch = [&](auto tag, auto act_tag) {
+    using Tag = decltype(tag);
+    constexpr int ACT = decltype(act_tag)::value;
+    if (form == 2)
+      hipLaunchKernelGGL((moe_tile_kernel<Tag, ACT, 256>), dim3(blocks),
+                         dim3(TP_THREADS), 0, stream, t);
+    else
+      hipLaunchKernelGGL((moe_tile_kernel<Tag, ACT, 128>), dim3(blocks),
+                         dim3(TP_THREADS), 0, stream, t);
+  };
+  auto by_act = [&](auto tag) {
+    if (act == SILU_GATED)
+      launch(tag, std::integral_constant<int, SILU_GATED>{});
+    else if (act == RELU2)
+      launch(tag, std::integral_constant<int, RELU2>{});
+    else
+      launch(tag, std::integral_constant<int, NONE>{});
+  };
+  if (bf16) by_act(BF16Tag{});
+  else      by_act(FP16Tag{});
+}
+
+}  // namespace moe
+
+}  // namespace vllm_amd

@@ -1,0 +1,219 @@
+// Product of a tile of rows with a tile of weight rows by four waves, one
+// a SIMD (gfx950): acc += W[TN, K] @ X[TM, K]^T, 16-bit operands in
+// LDS, fp32 sums in accumulation registers. Compile files that use it
+// without -amdgpu-mfma-vgpr-form: 256 accumulators a lane leave no room in
+// the vector registers.
+//
+// What bounds it. A wave of 128 x 128 reads 8 fragments of 32 x 16 from LDS
+// for 16 products of 32 x 32 x 16 (64 B a clock of the 128 that LDS gives;
+// eight waves of 64 x 128 read 96, and with what is filled that is all there
+// is). With one wave a SIMD nothing else hides a wait, so nothing waits:
+//  * fragments of the next 16 columns are read one at a time between this
+//    step's products, the order of products being that in which fragments
+//    arrive (pinned by scheduling barriers: the compiler would move reads to
+//    their use);
+//  * fills go straight from global memory to LDS, a few between products of
+//    every step: all at once they back up behind each other;
+//  * one barrier per 64 columns, before the last of their four steps, by
+//    when all of their fragments are in registers. From there on their
+//    places are filled again, that of the rows first. (Beside 256 x 256
+//    tiles LDS has two places for rows and three for weights, which come
+//    from further away.)
+// 8192 x 28672 x 4096 in bf16: 1.39 PFLOP/s, 8192 x 4096 x 14336 1.44 (eight
+// waves by halves in turn 1.0; the tuned library 1.57 and 1.60).
+#pragma once
+
+#include <type_traits>
+
+#include "common.h"
+
+namespace vllm_amd {
+
+constexpr int TP_K = 64;                  // columns of a stage: 128 B lines
+constexpr int TP_ROW = TP_K * 2;          // bytes of a row of a stage
+constexpr int TP_FILL = 1024;             // bytes of a fill: 8 rows
+constexpr int TP_THREADS = 4 * WAVE_SIZE;
+
+// 16 B chunk c of row r of a stage lies at c ^ tp_swap(r), so that the rows
+// of a fragment read meet no bank twice.
+DEVINL int tp_swap(int row) { return (row >> 1) & 7; }
+
+// Order of the fragments of a step (weights and rows in turn) and of its
+// products: each as soon as both fragments are there.
+template <int NI, int J> struct TpOrder {
+  bool w[NI + J]{};
+  int ix[NI + J]{}, i[NI * J + 1]{}, j[NI * J + 1]{};
+  constexpr TpOrder() {
+    int nw = 0, na = 0, n = 0;
+    for (int r = 0; r < NI + J; ++r) {
+      const bool tw = nw < NI && (nw <= na || na == J);
+      w[r] = tw;
+      ix[r] = tw ? nw : na;
+      for (int q = 0; q < (tw ? na : nw); ++q) {
+        i[n] = tw ? nw : q;
+        j[n] = tw ? q : na;
+        ++n;
+      }
+      (tw ? nw : na)++;
+    }
+  }
+};
+
+// WGM: waves along the rows (4 / WGM along the weights). NI, MI: 32-row
+// groups of weights and of rows a wave takes. PA, PW: stages of rows and of
+// weights that LDS holds. The waves' groups of rows alternate, so that in a
+// tile with few rows they have as many each.
+template <typename Tag, int WGM, int NI, int MI, int PA, int PW>
+struct TileProduct {
+  static constexpr int WGN = 4 / WGM;
+  static constexpr int TM = WGM * MI * 32;
+  static constexpr int TN = WGN * NI * 32;
+  static constexpr int AB = TM * TP_ROW;     // bytes of a stage
+  static constexpr int WB = TN * TP_ROW;
+  static constexpr int FA = TM / 8 / 4;      // fills a wave
+  static constexpr int FW = TN / 8 / 4;
+  static constexpr int LDS = PA * AB + PW * WB;
+  static constexpr int WW = NI * 32;         // weight rows of a wave
+  static_assert(PA >= 2 && PW >= PA && LDS <= 160 * 1024);
+
+  // fill_a(step, i, dst) and fill_w: the wave's i-th fill of 8 rows of a
+  // stage, rows (wave * FA + i) * 8 .. of the tile. done(J, acc) gets the
+  // sums of the J groups of rows of this wave that hold any of `rows`.
+  template <typename FillA, typename FillW, typename Done>
+  static DEVINL void run(char* lds, const int steps, const int rows,
+                         FillA fill_a, FillW fill_w, Done done) {
+    const int wave =
+        __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+    const int wm = wave / WGN;
+    const int groups = (min(rows, TM) + 31) / 32;
+    const int mine = (groups - wm + WGM - 1) / WGM;
+    auto go = [&](auto n) {
+      constexpr int J = decltype(n)::value;
+      f32x16 acc[NI][J > 0 ? J : 1];
+      loop<J>(lds, steps, wave, fill_a, fill_w, acc);
+      done(n, acc);
+      // What was filled past the end must not land in another workgroup's
+      // LDS.
+      lds_fill_wait();
+    };
+    if (mine >= MI) go(std::integral_constant<int, MI>{});
+    else if (MI > 3 && mine == 3) go(std::integral_constant<int, 3>{});
+    else if (MI > 2 && mine == 2) go(std::integral_constant<int, 2>{});
+    else if (MI > 1 && mine == 1) go(std::integral_constant<int, 1>{});
+    else go(std::integral_constant<int, 0>{});
+  }
+
+ private:
+  template <int J, typename FillA, typename FillW, int JA>
+  static DEVINL void loop(char* lds, const int steps, const int wave,
+                          FillA fill_a, FillW fill_w, f32x16 (&acc)[NI][JA]) {
+    constexpr TpOrder<NI, J> O{};
+    constexpr int M = NI * J, F = NI + J;
+    constexpr int G = M > 1 ? M / 2 : 1;     // pairs of products of a step
+    const int lane = threadIdx.x % WAVE_SIZE;
+    const int l32 = lane & 31;
+    const int half = lane >> 5;
+    const int wm = wave / WGN, wn = wave % WGN;
+    int at[4];   // byte places of this lane's fragments of a group
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      at[k] = l32 * TP_ROW + ((k * 2 + half) ^ tp_swap(l32)) * 16;
+    char* const wlds = lds + PA * AB;
+    const char* const a0 = lds + wm * 32 * TP_ROW;
+    const char* const w0 = wlds + wn * WW * TP_ROW;
+    auto fa = [&](int s, int i, int place) {
+      fill_a(min(s, steps - 1), i,
+             lds + place * AB + (wave * FA + i) * TP_FILL);
+    };
+    auto fw = [&](int s, int i, int place) {
+      fill_w(min(s, steps - 1), i,
+             wlds + place * WB + (wave * FW + i) * TP_FILL);
+    };
+    s16x8 af[2][J > 0 ? J : 1], wf[2][NI];
+    auto read = [&](int to, int ap, int wp, int k, int r) {
+      if constexpr (J > 0) {
+        if (O.w[r])
+          wf[to][O.ix[r]] = *reinterpret_cast<const s16x8*>(
+              w0 + wp * WB + O.ix[r] * 32 * TP_ROW + at[k]);
+        else
+          af[to][O.ix[r]] = *reinterpret_cast<const s16x8*>(
+              a0 + ap * AB + O.ix[r] * WGM * 32 * TP_ROW + at[k]);
+      }
+    };
+    // Products from fragments `cur`; between them READS of the next step's
+    // fragments, by the pair in which they come (all in the first half where
+    // a barrier follows), and n fills.
+    auto step = [&](const int cur, const bool soon, auto reads, const int n,
+                    auto fills) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+#pragma unroll
+        for (int r = 0; r < F; ++r)
+          if (r * G / (soon ? 2 * F : F) == g) reads(r);
+#pragma unroll
+        for (int f = 0; f < n; ++f)
+          if ((2 * f + 1) * G / (2 * n) == g) fills(f);
+        if constexpr (M > 1) {
+#pragma unroll
+          for (int q = 2 * g; q < 2 * g + 2; ++q)
+            acc[O.i[q]][O.j[q]] = mfma32<Tag>(
+                wf[cur][O.i[q]], af[cur][O.j[q]], acc[O.i[q]][O.j[q]]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if constexpr (J > 0) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    }
+    // In the order in which the loop goes on: what it waits for is counted.
+    constexpr int AHEAD_A = FW + (PA - 2) * (FA + FW);
+    constexpr int AHEAD_W = (PW - 2) * (FA + FW);
+    constexpr int AHEAD = AHEAD_A < AHEAD_W ? AHEAD_A : AHEAD_W;
+    static_assert(AHEAD + FA < 64);
+#pragma unroll
+    for (int t = 1 - PW; t < 0; ++t) {
+      if (t + PA - 1 >= 0) {
+#pragma unroll
+        for (int i = t + PA - 1 == 0 ? 0 : FA / 2; i < FA; ++i)
+          fa(t + PA - 1, i, t + PA - 1);
+      }
+#pragma unroll
+      for (int i = 0; i < FW; ++i) fw(t + PW - 1, i, t + PW - 1);
+      if (t + PA >= 1) {
+#pragma unroll
+        for (int i = 0; i < FA / 2; ++i) fa(t + PA, i, (t + PA) % PA);
+      }
+    }
+    lds_fill_wait<AHEAD>();
+    lds_barrier();
+#pragma unroll
+    for (int r = 0; r < F; ++r) read(0, 0, 0, 0, r);
+    int ap = 0, wp = 0;
+#pragma unroll 1
+    for (int s = 0; s < steps; ++s) {
+      const int an = ap == PA - 1 ? 0 : ap + 1, al = ap == 0 ? PA - 1 : ap - 1;
+      const int wn_ = wp == PW - 1 ? 0 : wp + 1, wl = wp == 0 ? PW - 1 : wp - 1;
+      step(0, false, [&](int r) { read(1, ap, wp, 1, r); }, FA / 2,
+           [&](int f) { fa(s + PA - 1, FA / 2 + f, al); });
+      step(1, false, [&](int r) { read(0, ap, wp, 2, r); }, FW / 2,
+           [&](int f) { fw(s + PW - 1, f, wl); });
+      step(0, true, [&](int r) { read(1, ap, wp, 3, r); }, FW / 2,
+           [&](int f) { fw(s + PW - 1, FW / 2 + f, wl); });
+      // The next stage has landed when only what was filled after it is
+      // under way; past the barrier no wave reads this one again.
+      lds_fill_wait<AHEAD>();
+      lds_barrier();
+      step(1, true, [&](int r) { read(0, an, wn_, 0, r); }, FA / 2,
+           [&](int f) { fa(s + PA, f, ap); });
+      ap = an;
+      wp = wn_;
+    }
+  }
+};
+
+}  // namespace vllm_amd
