@@ -39,6 +39,7 @@
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
 
+#include "arrivals.h"
 #include "common.h"
 
 namespace vllm_amd {
@@ -47,6 +48,7 @@ constexpr int DEC_WAVES = 4;
 constexpr int DEC_BLOCK = DEC_WAVES * WAVE_SIZE;
 constexpr int DEC_KEYS = 32;    // keys per wave and step, at most
 constexpr int MAX_GROUP = 8;    // query heads per KV head
+constexpr int MAX_PARTS = 64;   // partitions of a row: lanes of a wave
 constexpr float DEC_NEG = -3.0e38f;
 constexpr float DEC_LOG2E = 1.4426950408889634f;
 
@@ -78,14 +80,17 @@ DEVINL int dec_base(int ctx, int window) {
 
 // WPR 4: one workgroup is (kv head, decode row, partition of part_len
 // keys) and a wave takes every fourth step of them. WPR 1: a wave is a row
-// of its own, whole, for batches of short rows. Writes the final 16-bit
-// output (FINAL) or fp32 partials with their running maximum (log2 domain)
-// and sum.
-template <typename Tag, typename CTag, bool FINAL, int HD, int WPR>
+// of its own, whole, for batches of short rows. A row of several partitions
+// (only where not WHOLE) leaves fp32 partials with their running maximum
+// (log2 domain) and sum; the last of its workgroups to arrive merges them.
+// (A second launch for that: 1 x 1000 keys 9.2 us, now 8.2; 4 x 8192 29.5,
+// now 25.9; 64 x 4096..8192 fp8 keys 156.2, now 156.0.)
+template <typename Tag, typename CTag, bool WHOLE, int HD, int WPR>
 __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
-    short* __restrict__ out,            // FINAL: [Tdec, Hq, D] (16-bit)
-    float* __restrict__ tmp_out,        // else: [Tdec, Hq, parts, D]
-    float* __restrict__ tmp_lse,        // else: [Tdec, Hq, parts, 2]
+    short* __restrict__ out,            // [Tdec, Hq, D] (16-bit)
+    float* __restrict__ tmp_out,        // [Tdec, Hq, parts, D]
+    float* __restrict__ tmp_lse,        // [Tdec, Hq, parts, 2]
+    unsigned* __restrict__ arrived,     // [Tdec, Hkv]
     const short* __restrict__ q,        // [Tdec, Hq, D]
     const typename CacheTraits<CTag>::elem* __restrict__ kv_cache,
                                         // [2, blocks, Hkv, 64, D]
@@ -97,7 +102,7 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
     const int64_t kv_plane_stride,      // elements between K and V planes
     const int64_t q_stride,             // elements between q token rows
     const int sliding_window) {
-  static_assert(WPR == DEC_WAVES || (WPR == 1 && FINAL));
+  static_assert(WPR == DEC_WAVES || (WPR == 1 && WHOLE));
   using elem = typename CacheTraits<CTag>::elem;
   constexpr bool FP8 = sizeof(elem) == 1;
   constexpr int EPV = 16 / sizeof(elem);          // elements per 16 B
@@ -120,21 +125,18 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
   const int num_q_heads = num_kv_heads * group;
   const int hq0 = kvh * group;
   const int t_lo = sliding_window > 0 ? max(0, ctx - sliding_window) : 0;
-  const int t_begin = dec_base(ctx, sliding_window) + part * part_len;
+  const int t_first = dec_base(ctx, sliding_window);
+  const int t_begin = t_first + part * part_len;
   const int t_end = min(ctx, t_begin + part_len);
+  // Partitions of this row that hold keys.
+  const int used =
+      WHOLE ? 1 : min(num_parts, (ctx - t_first + part_len - 1) / part_len);
 
   if (t_begin >= t_end) {
-    // A row without keys (padding) is zero, also where nothing merges it.
-    if constexpr (FINAL)
+    if (part == 0)   // a row without keys (padding) is zero
       for (int e = WPR > 1 ? threadIdx.x : lane; e < group * HD;
            e += WPR * WAVE_SIZE)
         out[((int64_t)seq * num_q_heads + hq0) * HD + e] = 0;
-    if (!FINAL && threadIdx.x < group * 2) {
-      const int g = threadIdx.x / 2;
-      tmp_lse[(((int64_t)seq * num_q_heads + hq0 + g) * num_parts + part) *
-                  2 + threadIdx.x % 2] =
-          (threadIdx.x % 2 == 0) ? DEC_NEG : 0.f;
-    }
     return;
   }
 
@@ -371,83 +373,93 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
     }
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < group * HD; e += DEC_BLOCK) {
+  auto store4 = [&](int g, int d, f32x4 v) {
+    *reinterpret_cast<int2*>(
+        out + ((int64_t)seq * num_q_heads + hq0 + g) * HD + d) =
+        int2{pack2<Tag>(v[0], v[1]), pack2<Tag>(v[2], v[3])};
+  };
+  for (int e = threadIdx.x * 4; e < group * HD; e += DEC_BLOCK * 4) {
     const int g = e / HD;
     const int d = e % HD;
     float M = DEC_NEG;
 #pragma unroll
     for (int w = 0; w < DEC_WAVES; ++w) M = fmaxf(M, ml_red[w][g][0]);
-    float L = 0.f, acc = 0.f;
+    float L = 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < DEC_WAVES; ++w) {
       const float c = __builtin_amdgcn_exp2f(ml_red[w][g][0] - M);
       L += ml_red[w][g][1] * c;
-      acc += o_red[(w * MAX_GROUP + g) * HD + d] * c;
+      acc += *reinterpret_cast<const f32x4*>(
+                 o_red + (w * MAX_GROUP + g) * HD + d) *
+             c;
     }
-    if constexpr (FINAL) {
-      const float inv_l = L > 0.f || L != L ? 1.f / L : 0.f;
-      out[((int64_t)seq * num_q_heads + hq0 + g) * HD + d] =
-          from_f32<Tag>(acc * inv_l);
+    if (WHOLE || used == 1) {
+      store4(g, d, acc * (L > 0.f || L != L ? 1.f / L : 0.f));
     } else {
       const int64_t row =
           ((int64_t)seq * num_q_heads + hq0 + g) * num_parts + part;
-      tmp_out[row * HD + d] = acc;
+      part_put(reinterpret_cast<f32x4*>(tmp_out + row * HD + d), acc);
       if (d == 0) {
-        tmp_lse[row * 2] = M;
-        tmp_lse[row * 2 + 1] = L;
+        part_put(tmp_lse + row * 2, M);
+        part_put(tmp_lse + row * 2 + 1, L);
       }
     }
   }
-}
-
-// Merge per-partition partials: out = sum_p o_p 2^(m_p - M) / sum_p l_p
-// 2^(m_p - M). One wave per (row, head); lane p weighs partition p, then
-// every lane sums its own dims over the partitions (independent loads).
-template <typename Tag, int HD>
-__global__ __launch_bounds__(WAVE_SIZE) void paged_decode_reduce_kernel(
-    short* __restrict__ out,           // [Tdec, Hq, D]
-    const float* __restrict__ tmp_out, // [Tdec, Hq, parts, D]
-    const float* __restrict__ tmp_lse, // [Tdec, Hq, parts, 2]
-    const int* __restrict__ seq_lens, const int num_parts,
-    const int part_len, const int num_q_heads, const int sliding_window) {
-  constexpr int V = HD / WAVE_SIZE;   // dims per lane (1, 2 or 4)
-  const int h = blockIdx.x;
-  const int seq = blockIdx.y;
-  const int lane = threadIdx.x;
-  const int ctx = seq_lens[seq];
-  const int span = ctx - dec_base(ctx, sliding_window);
-  const int used = min(num_parts, (span + part_len - 1) / part_len);
-  const int64_t row = ((int64_t)seq * num_q_heads + h) * num_parts;
-  float M = DEC_NEG, L = 0.f, acc[V];
+  if constexpr (!WHOLE) {
+    // ---- merge the partitions: sum_p o_p 2^(m_p - M) / sum_p l_p 2^(m_p -
+    // M), the weights of each head in LDS ----------------------------------
+    if (used == 1) return;
+    float* w_lds = reinterpret_cast<float*>(lds);   // [group][MAX_PARTS]
+    static_assert(MAX_GROUP * MAX_PARTS * 4 + 4 <= (int)sizeof(lds));
+    if (!last_to_arrive(
+            arrived + (int64_t)seq * num_kv_heads + kvh, used,
+            reinterpret_cast<unsigned*>(w_lds + MAX_GROUP * MAX_PARTS)))
+      return;
+    const int64_t row0 = ((int64_t)seq * num_q_heads + hq0) * num_parts;
+    // Parts come from beyond L2: all that a thread needs is on its way at
+    // once, weights and the first eight partitions of its columns.
+    constexpr int AT_ONCE = 8;
+    f32x4 first[AT_ONCE];
+    const int e0 = threadIdx.x * 4;
+    auto part_of = [&](int e, int p) {
+      return reinterpret_cast<const f32x4*>(
+          tmp_out + (row0 + (int64_t)(e / HD) * num_parts + p) * HD + e % HD);
+    };
 #pragma unroll
-  for (int j = 0; j < V; ++j) acc[j] = 0.f;
-  for (int p0 = 0; p0 < used; p0 += WAVE_SIZE) {
-    const int n = min(WAVE_SIZE, used - p0);
-    float m = DEC_NEG, l = 0.f;
-    if (lane < n) {
-      m = tmp_lse[(row + p0 + lane) * 2];
-      l = tmp_lse[(row + p0 + lane) * 2 + 1];
+    for (int p = 0; p < AT_ONCE; ++p)
+      if (e0 < group * HD && p < used) first[p] = part_get(part_of(e0, p));
+    constexpr int HEADS = MAX_GROUP / DEC_WAVES;
+    float m[HEADS], l[HEADS];
+#pragma unroll
+    for (int i = 0; i < HEADS; ++i) {   // lane p: partition p
+      const int g = wave + i * DEC_WAVES;
+      const bool in = g < group && lane < used;
+      const float* lse = tmp_lse + (row0 + (int64_t)g * num_parts + lane) * 2;
+      m[i] = in ? part_get(lse) : DEC_NEG;
+      l[i] = in ? part_get(lse + 1) : 0.f;
     }
-    const float m_new = fmaxf(M, wave_reduce_max(m));
-    const float f = __builtin_amdgcn_exp2f(M - m_new);
-    const float w = __builtin_amdgcn_exp2f(m - m_new);
-    L = L * f + wave_reduce_sum(l * w);
-    M = m_new;
 #pragma unroll
-    for (int j = 0; j < V; ++j) acc[j] *= f;
-    const float* src = tmp_out + (row + p0) * HD + lane * V;
-#pragma unroll 8
-    for (int p = 0; p < n; ++p) {
-      const float wp = __shfl(w, p, 64);
+    for (int i = 0; i < HEADS; ++i) {
+      const float w = __builtin_amdgcn_exp2f(m[i] - wave_reduce_max(m[i]));
+      const float L = wave_reduce_sum(l[i] * w);
+      w_lds[(wave + i * DEC_WAVES) * MAX_PARTS + lane] =
+          L > 0.f || L != L ? w * (1.f / L) : 0.f;
+    }
+    __syncthreads();
+    for (int e = e0; e < group * HD; e += DEC_BLOCK * 4) {
+      const float* w = w_lds + e / HD * MAX_PARTS;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < V; ++j) acc[j] += src[(int64_t)p * HD + j] * wp;
+      for (int p = 0; p < AT_ONCE; ++p)
+        if (p < used) acc += (e == e0 ? first[p] : part_get(part_of(e, p))) *
+                             w[p];
+#pragma unroll 4
+      for (int p = AT_ONCE; p < used; ++p)
+        acc += part_get(part_of(e, p)) * w[p];
+      store4(e / HD, e % HD, acc);
     }
   }
-  const float inv_l = L > 0.f || L != L ? 1.f / L : 0.f;
-#pragma unroll
-  for (int j = 0; j < V; ++j)
-    out[((int64_t)seq * num_q_heads + h) * HD + lane * V + j] =
-        from_f32<Tag>(acc[j] * inv_l);
 }
 
 // ---------------------------------------------------------------------------
@@ -487,7 +499,7 @@ void paged_decode_attention(torch::Tensor out, torch::Tensor q,
                 tmp_out.size(3) == head_dim && tmp_lse.size(3) == 2,
                 "decode scratch must be [T, Hq, parts, D] and "
                 "[T, Hq, parts, 2]");
-    num_parts = tmp_out.size(2);
+    num_parts = std::min((int)tmp_out.size(2), MAX_PARTS);
   }
   // A window starts on a multiple of 32 keys, up to 31 before it.
   int64_t span = std::max<int64_t>(max_seq_len, 1);
@@ -518,48 +530,43 @@ void paged_decode_attention(torch::Tensor out, torch::Tensor q,
                   wave_rows ? ceil_div(num_seqs, DEC_WAVES) : num_seqs,
                   num_parts);
 
-  auto launch = [&](auto tag, auto ctag, auto dim, auto fin, auto wpr) {
+  torch::Tensor arrived;
+  if (num_parts > 1) arrived = arrival_counters(q, units);
+
+  auto launch = [&](auto tag, auto ctag, auto dim, auto whole, auto wpr) {
     using Tag = decltype(tag);
     using CTag = decltype(ctag);
     constexpr int HD = decltype(dim)::value;
-    constexpr bool FINAL = decltype(fin)::value;
+    constexpr bool WHOLE = decltype(whole)::value;
     constexpr int WPR = decltype(wpr)::value;
     hipLaunchKernelGGL(
-        (paged_decode_kernel<Tag, CTag, FINAL, HD, WPR>), grid,
+        (paged_decode_kernel<Tag, CTag, WHOLE, HD, WPR>), grid,
         dim3(DEC_BLOCK), 0, stream, (short*)out.data_ptr(),
-        FINAL ? nullptr : tmp_out.data_ptr<float>(),
-        FINAL ? nullptr : tmp_lse.data_ptr<float>(),
+        WHOLE ? nullptr : tmp_out.data_ptr<float>(),
+        WHOLE ? nullptr : tmp_lse.data_ptr<float>(),
+        WHOLE ? nullptr : (unsigned*)arrived.data_ptr<int>(),
         (const short*)q.data_ptr(),
         (const typename CacheTraits<CTag>::elem*)kv_cache.data_ptr(),
         block_table.data_ptr<int>(), seq_lens.data_ptr<int>(), scale_log2,
         group, num_kv_heads, num_seqs, max_blocks, num_parts, part_len,
         kv_cache.stride(0), q.stride(0), (int)sliding_window);
-    if constexpr (!FINAL) {
-      HIP_CHECK_KERNEL();
-      hipLaunchKernelGGL(
-          (paged_decode_reduce_kernel<Tag, HD>), dim3(num_q_heads, num_seqs),
-          dim3(WAVE_SIZE), 0, stream, (short*)out.data_ptr(),
-          tmp_out.data_ptr<float>(), tmp_lse.data_ptr<float>(),
-          seq_lens.data_ptr<int>(), num_parts, part_len, num_q_heads,
-          (int)sliding_window);
-    }
   };
-  auto by_dim = [&](auto tag, auto ctag, auto fin, auto wpr) {
+  auto by_dim = [&](auto tag, auto ctag, auto whole, auto wpr) {
     if (head_dim == 64)
-      launch(tag, ctag, std::integral_constant<int, 64>{}, fin, wpr);
+      launch(tag, ctag, std::integral_constant<int, 64>{}, whole, wpr);
     else if (head_dim == 128)
-      launch(tag, ctag, std::integral_constant<int, 128>{}, fin, wpr);
+      launch(tag, ctag, std::integral_constant<int, 128>{}, whole, wpr);
     else
-      launch(tag, ctag, std::integral_constant<int, 256>{}, fin, wpr);
+      launch(tag, ctag, std::integral_constant<int, 256>{}, whole, wpr);
   };
   const bool fp8c = kv_cache.scalar_type() == torch::kFloat8_e4m3fn;
-  auto by_type = [&](auto fin, auto wpr) {
+  auto by_type = [&](auto whole, auto wpr) {
     if (q.scalar_type() == torch::kBFloat16) {
-      if (fp8c) by_dim(BF16Tag{}, FP8CacheTag{}, fin, wpr);
-      else      by_dim(BF16Tag{}, BF16Tag{}, fin, wpr);
+      if (fp8c) by_dim(BF16Tag{}, FP8CacheTag{}, whole, wpr);
+      else      by_dim(BF16Tag{}, BF16Tag{}, whole, wpr);
     } else {
-      if (fp8c) by_dim(FP16Tag{}, FP8CacheTag{}, fin, wpr);
-      else      by_dim(FP16Tag{}, FP16Tag{}, fin, wpr);
+      if (fp8c) by_dim(FP16Tag{}, FP8CacheTag{}, whole, wpr);
+      else      by_dim(FP16Tag{}, FP16Tag{}, whole, wpr);
     }
   };
   using one = std::integral_constant<int, 1>;

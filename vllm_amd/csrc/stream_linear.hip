@@ -19,9 +19,8 @@
 //    -> 45.7 us).
 //  * Enough workgroups of equal size (plan() below). Narrow layers split K
 //    over workgroups; the last one to arrive adds up the parts in their
-//    order. Parts are written and read past the caches that the XCDs do not
-//    share, a release fence would write back all of L2 (2112 x 7168, 64
-//    rows in three parts: 33 us with fences, 14.7 without, 21.3 in one).
+//    order (arrivals.h; 2112 x 7168, 64 rows: 14.7 us in three parts, 21.3
+//    in one).
 //
 // us on weights from HBM, tuned library products -> these (floor at 6 TB/s):
 //                   1 row          8 rows         32 rows        64 rows
@@ -36,9 +35,7 @@
 
 #include <algorithm>
 #include <cmath>
-#include <map>
-#include <mutex>
-
+#include "arrivals.h"
 #include "common.h"
 
 namespace vllm_amd {
@@ -74,26 +71,6 @@ constexpr int sums_bytes(Form f, int xg) {
 constexpr int lds_bytes(Form f, int xg) {
   return ring_bytes(f, xg) > sums_bytes(f, xg) ? ring_bytes(f, xg)
                                                : sums_bytes(f, xg);
-}
-
-// Parts of sums travel between workgroups of different XCDs, whose L2s do
-// not see each other: agent-scope accesses go past them.
-DEVINL void put_part(f32x4* p, f32x4 v) {
-  const i32x4 b = __builtin_bit_cast(i32x4, v);
-  uint64_t* q = reinterpret_cast<uint64_t*>(p);
-  __hip_atomic_store(q, (uint64_t)(uint32_t)b[0] | (uint64_t)b[1] << 32,
-                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(q + 1, (uint64_t)(uint32_t)b[2] | (uint64_t)b[3] << 32,
-                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-DEVINL f32x4 get_part(const f32x4* p) {
-  const uint64_t* q = reinterpret_cast<const uint64_t*>(p);
-  const uint64_t a =
-      __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint64_t b =
-      __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return __builtin_bit_cast(
-      f32x4, (i32x4){(int)a, (int)(a >> 32), (int)b, (int)(b >> 32)});
 }
 
 // N: columns of out. SILU: w has 2N rows, gate then up; a tile is NI / 2
@@ -250,34 +227,20 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
       if (t >= TO) break;
 #pragma unroll
       for (int h = 0; h < H; ++h)
-        put_part(sums + (part * T + h * TO + t) * WAVE_SIZE, v[u][h]);
+        part_put(sums + (part * T + h * TO + t) * WAVE_SIZE, v[u][h]);
     }
-    // Written through before this workgroup counts as arrived.
-    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
-    asm volatile("" ::: "memory");
-    __syncthreads();
-    unsigned* last = reinterpret_cast<unsigned*>(lds);
-    if (threadIdx.x == 0) {
-      const unsigned before = __hip_atomic_fetch_add(
-          arrived + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      // All have arrived: zero again for the next launch.
-      if (before == (unsigned)parts - 1)
-        __hip_atomic_store(arrived + tile, 0u, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-      *last = before == (unsigned)parts - 1;
-    }
-    __syncthreads();
-    if (!*last) return;
-    asm volatile("" ::: "memory");
+    if (!last_to_arrive(arrived + tile, parts,
+                        reinterpret_cast<unsigned*>(lds)))
+      return;
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
       const int t = u * WV + wave;
       if (t >= TO) break;
 #pragma unroll
       for (int h = 0; h < H; ++h) {
-        v[u][h] = get_part(sums + (h * TO + t) * WAVE_SIZE);
+        v[u][h] = part_get(sums + (h * TO + t) * WAVE_SIZE);
         for (int q = 1; q < parts; ++q)
-          v[u][h] += get_part(sums + (q * T + h * TO + t) * WAVE_SIZE);
+          v[u][h] += part_get(sums + (q * T + h * TO + t) * WAVE_SIZE);
       }
     }
   }
@@ -349,34 +312,6 @@ Plan plan(int xg, int64_t rows_w, int K, bool silu) {
   return best;
 }
 
-// Zeroed counters of the workgroups that arrived; every launch leaves them
-// zero. One set per stream, whose launches follow each other; 32 sets at
-// most. Two kinds of call clear counters of their own: those of a graph,
-// which may run beside the stream that it was captured on, and those of
-// streams that are not torch's (their ids are even handles), which may end
-// and come back as another stream while work is under way.
-torch::Tensor arrival_counters(const torch::Tensor& like) {
-  constexpr size_t SETS = 32;
-  auto opt = like.options().dtype(torch::kInt);
-  const auto stream = c10::hip::getCurrentHIPStream();
-  const int64_t id = stream.id();
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if ((id != 0 && id % 2 == 0) ||
-      hipStreamIsCapturing(stream.stream(), &capturing) != hipSuccess ||
-      capturing != hipStreamCaptureStatusNone)
-    return torch::zeros({SL_JOBS}, opt);
-  // (Never destroyed: the runtime may be gone by then.)
-  static auto* sets = new std::map<std::pair<int, int64_t>, torch::Tensor>();
-  static std::mutex mu;
-  std::lock_guard<std::mutex> guard(mu);
-  const auto key = std::make_pair((int)like.get_device(), id);
-  auto it = sets->find(key);
-  if (it != sets->end()) return it->second;
-  auto t = torch::zeros({SL_JOBS}, opt);
-  if (sets->size() < SETS) sets->emplace(key, t);
-  return t;
-}
-
 template <typename Tag, int I, int XG, bool SILU>
 void launch_form(torch::Tensor& out, const torch::Tensor& x,
                  const torch::Tensor& w, const short* bias, int N,
@@ -392,7 +327,7 @@ void launch_form(torch::Tensor& out, const torch::Tensor& x,
       sums = torch::empty({(int64_t)tiles * parts * f.ni * ((XG + 1) / 2) *
                            WAVE_SIZE * 4},
                           x.options().dtype(torch::kFloat));
-      arrived = arrival_counters(x);
+      arrived = arrival_counters(x, tiles);
     }
     hipLaunchKernelGGL(
         (stream_linear_kernel<Tag, f.ni, XG, f.wv, f.d, SILU>),
