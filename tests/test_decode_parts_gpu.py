@@ -91,3 +91,45 @@ def test_replays_and_streams():
         assert torch.equal(out, expect)
         for o in beside:
             assert torch.equal(o, expect)
+
+
+# More tiles than rows and fewer, one of each; a portion shorter than a
+# tile, after cached tokens; heads in groups of 1, 7 and 8; rows in one and
+# in several partitions; a window; an fp8 cache; a negative scale.
+@pytest.mark.parametrize("rows,new,past,hq,hkv,hd,window,dtype,cache,scale", [
+    ([1000], [70], [0], 32, 8, 128, 0, torch.bfloat16, None, 0.09),
+    ([0, 1, 129, 3000], [1, 300], [5, 64], 14, 2, 128, 0, torch.float16,
+     None, 0.09),
+    ([500] * 40, [2], [1], 8, 8, 64, 0, torch.bfloat16, None, -0.1),
+    ([2000, 60], [513, 40, 129], [100, 0, 700], 16, 2, 128, 200,
+     torch.bfloat16, None, 0.09),
+    ([700, 1500, 64], [200], [31], 8, 2, 128, 0, torch.bfloat16,
+     torch.float8_e4m3fn, 0.09),
+])
+def test_mixed(rows, new, past, hq, hkv, hd, window, dtype, cache, scale):
+    """Rows and portions in one launch against each in its own: the same
+    work by the same code, so the same but for the order in which the
+    compiler adds (a unit of fp32 sums, the result's rounding)."""
+    from vllm_amd.ops import hip_ops
+    ctx = rows + [n + p for n, p in zip(new, past)]
+    q, kv, table, _, lens = _rows(ctx, hq, hkv, hd, dtype, cache or dtype)
+    q = torch.randn(len(rows) + sum(new), hq, hd, device="cuda").to(dtype)
+    qsl = torch.tensor([0] + [1] * len(rows) + new, device="cuda").cumsum(
+        0).to(torch.int32)
+    n = len(rows)
+    none = q.new_empty(0, dtype=torch.float32)
+    parts = hip_ops._decode_parts(n, hkv, max(rows), window)
+    tmp = (torch.empty(n, hq, parts, hd, device="cuda"),
+           torch.empty(n, hq, parts, 2, device="cuda")) if parts > 1 else (
+               none, none)
+    one, two = torch.empty_like(q), torch.empty_like(q)
+    ops = hip_ops._C
+    ops.mixed_attention(one, q, kv, table, qsl, lens, scale, n, max(rows),
+                        max(new), window, *tmp)
+    ops.paged_decode_attention(two[:n], q[:n], kv, table, lens, scale,
+                               max(rows), window, *tmp)
+    ops.prefill_attention(two, q, kv, table, qsl, lens, scale, n, max(new),
+                          window)
+    tol = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    torch.testing.assert_close(one.float(), two.float(), rtol=tol,
+                               atol=1e-6)

@@ -228,3 +228,25 @@ def test_odd_places_take_plain_loads(hip, monkeypatch):
                       _odd(1, 64, 576).zero_(), one[None] * 0,
                       _lens(0, 1), one, 0.07, num_decodes=1, max_seq_len=1)
     assert not hip._C.calls
+
+
+@pytest.mark.parametrize("rows,keys,new,heads,hd,mixed", [
+    (96, 4000, 1000, 32, 128, True),
+    (8, 1000, 2000, 32, 128, True),
+    (1, 1000, 8191, 32, 128, False),     # nothing to run beside
+    (256, 300, 500, 32, 128, False),     # a wave a row
+    (8, 1000, 200, 72, 128, False),      # nine heads a KV head
+    (8, 1000, 200, 32, 256, False),
+    (8, 1000, 2000, 32, 64, True),
+])
+def test_rows_beside_portions(hip, rows, keys, new, heads, hd, mixed):
+    q = torch.empty(rows + new, heads, hd, dtype=torch.bfloat16)
+    kv = torch.empty(2, 1, 8, 64, hd, dtype=torch.bfloat16)
+    hip.attention_unified(
+        q, kv, torch.zeros(rows + 1, 1, dtype=torch.int32),
+        _lens(*range(rows + 2)), _lens(*[keys] * rows, new), 0.1,
+        num_decodes=rows, max_seq_len=max(keys, new), max_query_len=new,
+        max_decode_len=keys)
+    names = [n for n, _ in hip._C.calls]
+    assert names == (["mixed_attention"] if mixed else
+                     ["paged_decode_attention", "prefill_attention"])

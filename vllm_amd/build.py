@@ -32,6 +32,7 @@ SOURCES = [
     CSRC / "quant_fp8.hip",
     CSRC / "attention_decode.hip",
     CSRC / "attention_prefill.hip",
+    CSRC / "attention_mixed.hip",
     CSRC / "pooled_attention.hip",
     CSRC / "pooled_attention_prefill.hip",
     CSRC / "pooled_attention_decode.hip",
@@ -48,7 +49,8 @@ SOURCES = [
 # These kernels keep matrix-core accumulators in ordinary vector
 # registers: they are rescaled by the vector ALU between products, and
 # through the accumulation registers every rescale is a copy each way.
-VGPR_ACCUMULATORS = {"attention_decode", "attention_prefill", "mla",
+VGPR_ACCUMULATORS = {"attention_decode", "attention_prefill",
+                     "attention_mixed", "mla",
                      "mla_prompt", "head_matmul", "moe",
                      "stream_linear"}
 

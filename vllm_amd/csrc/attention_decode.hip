@@ -1,481 +1,26 @@
-// Paged decode attention for MI355X (gfx950, CDNA4).
-//
-// What bounds it: one pass over the cached keys and values. At 2..16
-// flops per byte everything else only has to stay out of the way of the
-// loads, so the kernel keeps as many bytes in flight as registers allow
-// and spends few issue slots per byte:
-//   - A wave owns 32 keys at a time (16 where rows are 512 B) and never
-//     meets another wave before the end, so there is no barrier in the
-//     loop. The next keys are loaded as soon as the registers of the
-//     current ones are free.
-//   - Scores are S^T = K Q^T on the matrix cores: a K row goes from HBM
-//     straight into the A fragment (16 B per lane), the query heads of
-//     the group are the 16 columns. No cross-lane sum per key and head,
-//     which is what the vector-ALU form of this kernel spent its time on.
-//   - O^T = V^T P^T: V passes through this wave's own LDS slice to be
-//     transposed on the read. The lane that holds the scores of keys
-//     (4g..4g+3, 16+4g..) holds exactly the P^T fragment of those keys
-//     when the contraction runs over keys in that order, so P never
-//     moves between lanes.
-//   - P stays at more than 16 bits: it is split in two 16-bit parts
-//     (p = hi + lo, error 2^-17) and multiplied twice; the matrix cores
-//     are idle here anyway. Sums and outputs are fp32. Results are as far
-//     from 64 bits as with fp32 weights, to six digits (1.64328e-3 at 1 x
-//     1000 keys, 1.66106e-3 at 1024 x 129..176, fp16 2.07694e-4 at 40 x
-//     100..4000).
-// Against the vector-ALU form it replaced (16 lanes per token, dot
-// products reduced with shuffles), us per layer at 32 query and 8 KV
-// heads of 128:
-//   1 x 1000 keys 46 -> 13; 256 x 129..2176 keys 349 -> 228 (5.3 TB/s);
-//   1024 x 129..176 keys 206 -> 121 (5.3 TB/s; 132 with the last 32 keys
-//   of a row read whole);
-//   64 x 4096..8192 keys, fp8 cache 371 -> 160 (5.2 TB/s).
-//
-// The KV cache layout [2, blocks, kv_heads, block_size=64, D] keeps each
-// (block, head) tile contiguous (16 KB at D=128).
-//
-// Role of the reference's paged_attention (csrc/rocm/attention.cu:321,1420).
+// Paged decode attention: kernel and host launcher. What bounds the work and
+// how it is laid out: attention_decode.h.
 
-#include <torch/all.h>
 #include <c10/hip/HIPStream.h>
 
-#include "arrivals.h"
-#include "common.h"
+#include "attention.h"
 
 namespace vllm_amd {
 
-constexpr int DEC_WAVES = 4;
-constexpr int DEC_BLOCK = DEC_WAVES * WAVE_SIZE;
-constexpr int DEC_KEYS = 32;    // keys per wave and step, at most
-constexpr int MAX_GROUP = 8;    // query heads per KV head
-constexpr int MAX_PARTS = 64;   // partitions of a row: lanes of a wave
-constexpr float DEC_NEG = -3.0e38f;
-constexpr float DEC_LOG2E = 1.4426950408889634f;
-
-// Bytes of a V row are moved in 32 B segments (16 columns, what one
-// transposing read takes from a row). Rotating the segments by the row
-// spreads the rows a read touches over all 64 banks.
-template <int HD> DEVINL int v_slot(int row, int seg) {
-  if constexpr (HD == 64) return seg ^ ((row >> 1) & 3);
-  return seg ^ (row & 7);
-}
-
-// Keys per wave and step. 32 rows of 512 B each for keys and values, the
-// queries and 16 x 256 outputs are more registers than the two workgroups
-// of a CU have (340; one workgroup then, values moved between register
-// files): 16 a step instead takes 228. us: 16 x 750..1500 keys, 16 KV heads
-// 58 -> 53, 64 x 300..3000 (4) 102 -> 98, 256 x 150..300 through a window of
-// 128 (16, three query heads each) 146 -> 102. At 128 columns 16 keys are no
-// faster for long rows (256 x 129..2176 228 -> 231).
-template <typename CTag, int HD>
-constexpr int dec_keys =
-    HD == 256 && sizeof(typename CacheTraits<CTag>::elem) == 2 ? 16
-                                                               : DEC_KEYS;
-
-// First key this row attends, rounded down so that a wave's 32 keys
-// never leave a cache block.
-DEVINL int dec_base(int ctx, int window) {
-  return window > 0 ? (max(0, ctx - window) & ~(DEC_KEYS - 1)) : 0;
-}
-
-// WPR 4: one workgroup is (kv head, decode row, partition of part_len
-// keys) and a wave takes every fourth step of them. WPR 1: a wave is a row
-// of its own, whole, for batches of short rows. A row of several partitions
-// (only where not WHOLE) leaves fp32 partials with their running maximum
-// (log2 domain) and sum; the last of its workgroups to arrive merges them.
-// (A second launch for that: 1 x 1000 keys 9.2 us, now 8.2; 4 x 8192 29.5,
-// now 25.9; 64 x 4096..8192 fp8 keys 156.2, now 156.0.)
 template <typename Tag, typename CTag, bool WHOLE, int HD, int WPR>
 __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
-    short* __restrict__ out,            // [Tdec, Hq, D] (16-bit)
-    float* __restrict__ tmp_out,        // [Tdec, Hq, parts, D]
-    float* __restrict__ tmp_lse,        // [Tdec, Hq, parts, 2]
-    unsigned* __restrict__ arrived,     // [Tdec, Hkv]
-    const short* __restrict__ q,        // [Tdec, Hq, D]
-    const typename CacheTraits<CTag>::elem* __restrict__ kv_cache,
-                                        // [2, blocks, Hkv, 64, D]
-    const int* __restrict__ block_table,   // [num_reqs, max_blocks]
-    const int* __restrict__ seq_lens,      // [num_reqs]
-    const float scale_log2, const int group, const int num_kv_heads,
-    const int num_seqs, const int max_blocks_per_req, const int num_parts,
-    const int part_len,
-    const int64_t kv_plane_stride,      // elements between K and V planes
-    const int64_t q_stride,             // elements between q token rows
-    const int sliding_window) {
-  static_assert(WPR == DEC_WAVES || (WPR == 1 && WHOLE));
-  using elem = typename CacheTraits<CTag>::elem;
-  constexpr bool FP8 = sizeof(elem) == 1;
-  constexpr int EPV = 16 / sizeof(elem);          // elements per 16 B
-  constexpr int KEYS = dec_keys<CTag, HD>;
-  constexpr int KT = KEYS / 16;                   // score tiles
-  constexpr int KF = HD / 32;                     // MFMA steps over D
-  constexpr int KN = HD * (int)sizeof(elem) / 64; // 16 B K loads per row
-  constexpr int VN = KEYS * HD / EPV / WAVE_SIZE;
-  constexpr int DS = HD / 16;                     // output column tiles
-  constexpr int V_BYTES = KEYS * HD * 2;          // per wave
-
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
-  const int lane = threadIdx.x % WAVE_SIZE;
-  const int kvh = blockIdx.x;
-  // Decode row == request row.
-  const int seq = WPR > 1 ? blockIdx.y : blockIdx.y * DEC_WAVES + wave;
-  if (WPR == 1 && seq >= num_seqs) return;   // (no barrier below then)
-  const int part = WPR > 1 ? blockIdx.z : 0;
-  const int ctx = seq_lens[seq];
-  const int num_q_heads = num_kv_heads * group;
-  const int hq0 = kvh * group;
-  const int t_lo = sliding_window > 0 ? max(0, ctx - sliding_window) : 0;
-  const int t_first = dec_base(ctx, sliding_window);
-  const int t_begin = t_first + part * part_len;
-  const int t_end = min(ctx, t_begin + part_len);
-  // Partitions of this row that hold keys.
-  const int used =
-      WHOLE ? 1 : min(num_parts, (ctx - t_first + part_len - 1) / part_len);
-
-  if (t_begin >= t_end) {
-    if (part == 0)   // a row without keys (padding) is zero
-      for (int e = WPR > 1 ? threadIdx.x : lane; e < group * HD;
-           e += WPR * WAVE_SIZE)
-        out[((int64_t)seq * num_q_heads + hq0) * HD + e] = 0;
-    return;
-  }
-
-  const int l16 = lane & 15;
-  const int l4 = lane >> 4;
-
-  // V slices of the waves; reused for the merge of the waves at the end
-  // (group <= 8 of the 16 columns, so it always fits).
-  __shared__ __align__(16) char lds[DEC_WAVES * V_BYTES];
-  __shared__ float ml_red[DEC_WAVES][MAX_GROUP][2];
-  char* v_lds = lds + wave * V_BYTES;
-
-  // B fragments of the queries: column l16 is a head of the group, the
-  // others repeat head 0 and are never written out.
-  s16x8 qf[KF];
-  {
-    const short* qb = q + (int64_t)seq * q_stride +
-                      (int64_t)(hq0 + (l16 < group ? l16 : 0)) * HD;
-#pragma unroll
-    for (int kk = 0; kk < KF; ++kk) {
-      // With an fp8 cache a 16 B load is two fragments' worth of one
-      // row, so the dims of a step are interleaved differently.
-      const int d = FP8 ? (kk >> 1) * 64 + l4 * 16 + (kk & 1) * 8
-                        : kk * 32 + l4 * 8;
-      qf[kk] = *reinterpret_cast<const s16x8*>(qb + d);
-    }
-  }
-
-  const int* bt = block_table + (int64_t)seq * max_blocks_per_req;
-  auto tile_of = [&](int key0) {
-    return kv_cache +
-           ((int64_t)bt[key0 >> 6] * num_kv_heads + kvh) * (64 * HD) +
-           (key0 & 63) * HD;
-  };
-  i32x4 kr[KT][KN], vr[VN];
-  // Rows of a step that the row does not attend repeat the nearest one it
-  // does: they cost no bytes.
-  auto load_k = [&](const elem* tile, int key0) {
-    const int lo = t_lo - key0, hi = t_end - 1 - key0;
-#pragma unroll
-    for (int s = 0; s < KT; ++s) {
-      const int r = min(max(s * 16 + l16, lo), hi);
-#pragma unroll
-      for (int i = 0; i < KN; ++i)
-        kr[s][i] = *reinterpret_cast<const i32x4*>(
-            tile + r * HD + (i * 4 + l4) * EPV);
-    }
-  };
-  auto load_v = [&](const elem* tile, int key0) {
-    const int lo = t_lo - key0, hi = t_end - 1 - key0;
-#pragma unroll
-    for (int i = 0; i < VN; ++i) {
-      const int e = (i * WAVE_SIZE + lane) * EPV;
-      const int r = min(max(e / HD, lo), hi);
-      vr[i] = *reinterpret_cast<const i32x4*>(tile + kv_plane_stride +
-                                              r * HD + e % HD);
-    }
-  };
-
-  float m_run = DEC_NEG, l_run = 0.f;   // of head l16; l: this lane's keys
-  f32x4 o[DS];
-#pragma unroll
-  for (int i = 0; i < DS; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // One step of KEYS keys; with NEXT the loads of the wave's next ones are
-  // issued as the registers become free (a template flag and not a test
-  // inside, so that the waits count exactly the older loads).
-  constexpr int STRIDE = WPR * KEYS;
-  auto step = [&](int key0, auto has_next) {
-    constexpr bool NEXT = decltype(has_next)::value;
-    const elem* next_tile =
-        NEXT ? tile_of(key0 + STRIDE) : nullptr;
-    // ---- S^T: rows are keys, columns heads -----------------------------
-    f32x4 s[KT];
-#pragma unroll
-    for (int t = 0; t < KT; ++t) {
-      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kk = 0; kk < KF; ++kk) {
-        s16x8 a;
-        if constexpr (FP8) {
-          const i32x4 r = kr[t][kk >> 1];
-          const int2 x = fp8x4_widen<Tag>(r[(kk & 1) * 2]);
-          const int2 y = fp8x4_widen<Tag>(r[(kk & 1) * 2 + 1]);
-          a = __builtin_bit_cast(s16x8, (i32x4){x.x, x.y, y.x, y.y});
-        } else {
-          a = __builtin_bit_cast(s16x8, kr[t][kk]);
-        }
-        s[t] = mfma16<Tag>(a, qf[kk], s[t]);
-      }
-    }
-    if constexpr (NEXT) load_k(next_tile, key0 + STRIDE);
-
-    // ---- V to LDS, rows outside [t_lo, t_end) as zeros ------------------
-    // (a stale cache row may hold anything, and 0 * NaN is NaN).
-    const bool edge = key0 < t_lo || key0 + KEYS > t_end;
-    if (edge) {
-#pragma unroll
-      for (int i = 0; i < VN; ++i) {
-        const int key = key0 + (i * WAVE_SIZE + lane) * EPV / HD;
-        const bool in = (key >= t_lo) & (key < t_end);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) vr[i][j] = in ? vr[i][j] : 0;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < VN; ++i) {
-      const int e = (i * WAVE_SIZE + lane) * EPV;
-      const int row = e / HD;
-      const i32x4 v = vr[i];
-      const int c16 = (e % HD) / 8;   // 16 B chunk of the 16-bit row
-      char* dst = v_lds + row * (HD * 2) + v_slot<HD>(row, c16 >> 1) * 32;
-      if constexpr (FP8) {
-        const int2 a = fp8x4_widen<Tag>(v[0]), b = fp8x4_widen<Tag>(v[1]);
-        const int2 c = fp8x4_widen<Tag>(v[2]), d = fp8x4_widen<Tag>(v[3]);
-        i32x4* p = reinterpret_cast<i32x4*>(dst);
-        p[0] = i32x4{a.x, a.y, b.x, b.y};
-        p[1] = i32x4{c.x, c.y, d.x, d.y};
-      } else {
-        *reinterpret_cast<i32x4*>(dst + (c16 & 1) * 16) = v;
-      }
-    }
-    if constexpr (NEXT) load_v(next_tile, key0 + STRIDE);
-
-    // ---- running softmax, log2 domain ----------------------------------
-    // A key outside the row's range scores DEC_NEG and weighs nothing
-    // even where the whole step is outside it.
-    bool in[KT][4];
-    float mx = DEC_NEG;
-#pragma unroll
-    for (int t = 0; t < KT; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int key = key0 + t * 16 + l4 * 4 + r;
-        in[t][r] = (key >= t_lo) & (key < t_end);
-        s[t][r] = in[t][r] ? s[t][r] * scale_log2 : DEC_NEG;
-        mx = fmaxf(mx, s[t][r]);
-      }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m_run, mx);
-    if (__any(m_new > m_run)) {
-      const float f = __builtin_amdgcn_exp2f(m_run - m_new);
-      l_run *= f;
-#pragma unroll
-      for (int i = 0; i < DS; ++i) o[i] *= f;
-      m_run = m_new;
-    }
-    i32x4 hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
-#pragma unroll
-    for (int t = 0; t < KT; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; r += 2) {
-        const float e0 = __builtin_amdgcn_exp2f(s[t][r] - m_run);
-        const float e1 = __builtin_amdgcn_exp2f(s[t][r + 1] - m_run);
-        const float p0 = in[t][r] ? e0 : 0.f;
-        const float p1 = in[t][r + 1] ? e1 : 0.f;
-        l_run += p0 + p1;
-        const int h = pack2<Tag>(p0, p1);
-        hi[t * 2 + r / 2] = h;
-        lo[t * 2 + r / 2] =
-            pack2<Tag>(p0 - unpack_lo<Tag>(h), p1 - unpack_hi<Tag>(h));
-      }
-    const s16x8 p_hi = __builtin_bit_cast(s16x8, hi);
-    const s16x8 p_lo = __builtin_bit_cast(s16x8, lo);
-
-    // ---- O^T += V^T P^T -------------------------------------------------
-    // LDS operations of one wave complete in order; the fences only keep
-    // the compiler from moving them.
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    const int row = l4 * 4 + (l16 >> 2);
-#pragma unroll
-    for (int i = 0; i < DS; ++i) {
-      const int off = (l16 & 3) * 8;
-      const s16x4 a = lds_read_tr(v_lds + row * (HD * 2) +
-                                  v_slot<HD>(row, i) * 32 + off);
-      if constexpr (KT == 1) {
-        o[i] = mfma16<Tag>(a, __builtin_shufflevector(p_lo, p_lo, 0, 1, 2, 3),
-                           o[i]);
-        o[i] = mfma16<Tag>(a, __builtin_shufflevector(p_hi, p_hi, 0, 1, 2, 3),
-                           o[i]);
-        continue;
-      }
-      const s16x4 b = lds_read_tr(v_lds + (row + 16) * (HD * 2) +
-                                  v_slot<HD>(row + 16, i) * 32 + off);
-      const s16x8 v = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
-      o[i] = mfma16<Tag>(v, p_lo, o[i]);
-      o[i] = mfma16<Tag>(v, p_hi, o[i]);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  };
-
-  int key0 = t_begin + (WPR > 1 ? wave * KEYS : 0);
-  if (key0 < t_end) {
-    const elem* tile = tile_of(key0);
-    load_k(tile, key0);
-    load_v(tile, key0);
-    for (; key0 + STRIDE < t_end; key0 += STRIDE)
-      step(key0, std::true_type{});
-    step(key0, std::false_type{});
-  }
-
-  // ---- merge the waves ----------------------------------------------------
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
-  if constexpr (WPR == 1) {   // nothing to merge
-    const float inv_l = l_run > 0.f || l_run != l_run ? 1.f / l_run : 0.f;
-    if (l16 < group) {
-      short* ob =
-          out + ((int64_t)seq * num_q_heads + hq0 + l16) * HD + l4 * 4;
-#pragma unroll
-      for (int i = 0; i < DS; ++i) {
-        int2 v;
-        v.x = pack2<Tag>(o[i][0] * inv_l, o[i][1] * inv_l);
-        v.y = pack2<Tag>(o[i][2] * inv_l, o[i][3] * inv_l);
-        *reinterpret_cast<int2*>(ob + i * 16) = v;
-      }
-    }
-    return;
-  }
-  __syncthreads();   // every wave is done with its V slice
-  float* o_red = reinterpret_cast<float*>(lds);  // [wave][MAX_GROUP][HD]
-  static_assert(MAX_GROUP * HD * 4 <= V_BYTES, "merge scratch");
-  if (l16 < group) {
-#pragma unroll
-    for (int i = 0; i < DS; ++i)
-      *reinterpret_cast<f32x4*>(
-          o_red + (wave * MAX_GROUP + l16) * HD + i * 16 + l4 * 4) = o[i];
-    if (l4 == 0) {
-      ml_red[wave][l16][0] = m_run;
-      ml_red[wave][l16][1] = l_run;
-    }
-  }
-  __syncthreads();
-  auto store4 = [&](int g, int d, f32x4 v) {
-    *reinterpret_cast<int2*>(
-        out + ((int64_t)seq * num_q_heads + hq0 + g) * HD + d) =
-        int2{pack2<Tag>(v[0], v[1]), pack2<Tag>(v[2], v[3])};
-  };
-  for (int e = threadIdx.x * 4; e < group * HD; e += DEC_BLOCK * 4) {
-    const int g = e / HD;
-    const int d = e % HD;
-    float M = DEC_NEG;
-#pragma unroll
-    for (int w = 0; w < DEC_WAVES; ++w) M = fmaxf(M, ml_red[w][g][0]);
-    float L = 0.f;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < DEC_WAVES; ++w) {
-      const float c = __builtin_amdgcn_exp2f(ml_red[w][g][0] - M);
-      L += ml_red[w][g][1] * c;
-      acc += *reinterpret_cast<const f32x4*>(
-                 o_red + (w * MAX_GROUP + g) * HD + d) *
-             c;
-    }
-    if (WHOLE || used == 1) {
-      store4(g, d, acc * (L > 0.f || L != L ? 1.f / L : 0.f));
-    } else {
-      const int64_t row =
-          ((int64_t)seq * num_q_heads + hq0 + g) * num_parts + part;
-      part_put(reinterpret_cast<f32x4*>(tmp_out + row * HD + d), acc);
-      if (d == 0) {
-        part_put(tmp_lse + row * 2, M);
-        part_put(tmp_lse + row * 2 + 1, L);
-      }
-    }
-  }
-  if constexpr (!WHOLE) {
-    // ---- merge the partitions: sum_p o_p 2^(m_p - M) / sum_p l_p 2^(m_p -
-    // M), the weights of each head in LDS ----------------------------------
-    if (used == 1) return;
-    float* w_lds = reinterpret_cast<float*>(lds);   // [group][MAX_PARTS]
-    static_assert(MAX_GROUP * MAX_PARTS * 4 + 4 <= (int)sizeof(lds));
-    if (!last_to_arrive(
-            arrived + (int64_t)seq * num_kv_heads + kvh, used,
-            reinterpret_cast<unsigned*>(w_lds + MAX_GROUP * MAX_PARTS)))
-      return;
-    const int64_t row0 = ((int64_t)seq * num_q_heads + hq0) * num_parts;
-    // Parts come from beyond L2: all that a thread needs is on its way at
-    // once, weights and the first eight partitions of its columns.
-    constexpr int AT_ONCE = 8;
-    f32x4 first[AT_ONCE];
-    const int e0 = threadIdx.x * 4;
-    auto part_of = [&](int e, int p) {
-      return reinterpret_cast<const f32x4*>(
-          tmp_out + (row0 + (int64_t)(e / HD) * num_parts + p) * HD + e % HD);
-    };
-#pragma unroll
-    for (int p = 0; p < AT_ONCE; ++p)
-      if (e0 < group * HD && p < used) first[p] = part_get(part_of(e0, p));
-    constexpr int HEADS = MAX_GROUP / DEC_WAVES;
-    float m[HEADS], l[HEADS];
-#pragma unroll
-    for (int i = 0; i < HEADS; ++i) {   // lane p: partition p
-      const int g = wave + i * DEC_WAVES;
-      const bool in = g < group && lane < used;
-      const float* lse = tmp_lse + (row0 + (int64_t)g * num_parts + lane) * 2;
-      m[i] = in ? part_get(lse) : DEC_NEG;
-      l[i] = in ? part_get(lse + 1) : 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < HEADS; ++i) {
-      const float w = __builtin_amdgcn_exp2f(m[i] - wave_reduce_max(m[i]));
-      const float L = wave_reduce_sum(l[i] * w);
-      w_lds[(wave + i * DEC_WAVES) * MAX_PARTS + lane] =
-          L > 0.f || L != L ? w * (1.f / L) : 0.f;
-    }
-    __syncthreads();
-    for (int e = e0; e < group * HD; e += DEC_BLOCK * 4) {
-      const float* w = w_lds + e / HD * MAX_PARTS;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int p = 0; p < AT_ONCE; ++p)
-        if (p < used) acc += (e == e0 ? first[p] : part_get(part_of(e, p))) *
-                             w[p];
-#pragma unroll 4
-      for (int p = AT_ONCE; p < used; ++p)
-        acc += part_get(part_of(e, p)) * w[p];
-      store4(e / HD, e % HD, acc);
-    }
-  }
+    const DecodeArgs<CTag> a) {
+  __shared__ __align__(16) char lds[dec_lds<CTag, HD>];
+  decode_rows<Tag, CTag, WHOLE, HD, WPR>(a, blockIdx.x, blockIdx.y,
+                                         blockIdx.z, lds);
 }
 
-// ---------------------------------------------------------------------------
-// Host launcher. q: [Tdec, Hq, D] (contiguous slice of the step's q);
-// out: [Tdec, Hq, D]; kv_cache: [2, blocks, Hkv, 64, D];
-// block_table/seq_lens cover the decode rows (rows 0..Tdec-1).
-// tmp_out [Tdec, Hq, parts, D] and tmp_lse [Tdec, Hq, parts, 2] say into
-// how many partitions a row's keys are split; empty means one.
-void paged_decode_attention(torch::Tensor out, torch::Tensor q,
-                            torch::Tensor kv_cache,
-                            torch::Tensor block_table,
-                            torch::Tensor seq_lens, double scale,
-                            int64_t max_seq_len, int64_t sliding_window,
-                            torch::Tensor tmp_out, torch::Tensor tmp_lse) {
-  const int num_seqs = q.size(0);
-  if (num_seqs == 0) return;
+// Checks the operands of num_seqs decode rows and lays them out.
+DecodePlan plan_decode(const torch::Tensor& out, const torch::Tensor& q,
+                       const torch::Tensor& kv_cache, int num_seqs,
+                       double scale, int64_t max_seq_len,
+                       int64_t sliding_window, const torch::Tensor& tmp_out,
+                       const torch::Tensor& tmp_lse) {
   const int num_q_heads = q.size(1);
   const int head_dim = q.size(2);
   const int num_kv_heads = kv_cache.size(2);
@@ -509,10 +54,6 @@ void paged_decode_attention(torch::Tensor out, torch::Tensor q,
   const int part_len =
       (int)((span + (int64_t)num_parts * unit - 1) /
             ((int64_t)num_parts * unit)) * unit;
-  const int max_blocks = block_table.size(1);
-  const float scale_log2 = (float)scale * DEC_LOG2E;
-  auto stream = c10::hip::getCurrentHIPStream().stream();
-
   // Rows of a few steps leave three of a workgroup's four waves idle, and
   // starting and merging it costs more than its keys: from half the waves
   // that run at a time on, each takes a row of at most 128 keys of its own;
@@ -526,30 +67,44 @@ void paged_decode_attention(torch::Tensor out, torch::Tensor q,
       num_parts == 1 &&
       ((span <= 128 && units >= (head_dim == 64 ? 1536 : 1024)) ||
        (span <= 512 && units >= 4096 && head_dim <= 128));
-  const dim3 grid(num_kv_heads,
-                  wave_rows ? ceil_div(num_seqs, DEC_WAVES) : num_seqs,
-                  num_parts);
-
   torch::Tensor arrived;
   if (num_parts > 1) arrived = arrival_counters(q, units);
+  return {num_parts, part_len, wave_rows, (float)scale * DEC_LOG2E, arrived};
+}
+
+// ---------------------------------------------------------------------------
+// Host launcher. q: [Tdec, Hq, D] (contiguous slice of the step's q);
+// out: [Tdec, Hq, D]; kv_cache: [2, blocks, Hkv, 64, D];
+// block_table/seq_lens cover the decode rows (rows 0..Tdec-1).
+// tmp_out [Tdec, Hq, parts, D] and tmp_lse [Tdec, Hq, parts, 2] say into
+// how many partitions a row's keys are split; empty means one.
+void paged_decode_attention(torch::Tensor out, torch::Tensor q,
+                            torch::Tensor kv_cache,
+                            torch::Tensor block_table,
+                            torch::Tensor seq_lens, double scale,
+                            int64_t max_seq_len, int64_t sliding_window,
+                            torch::Tensor tmp_out, torch::Tensor tmp_lse) {
+  const int num_seqs = q.size(0);
+  if (num_seqs == 0) return;
+  const int head_dim = q.size(2);
+  const DecodePlan p =
+      plan_decode(out, q, kv_cache, num_seqs, scale, max_seq_len,
+                  sliding_window, tmp_out, tmp_lse);
+  auto stream = c10::hip::getCurrentHIPStream().stream();
+  const dim3 grid((unsigned)kv_cache.size(2),
+                  p.wave_rows ? ceil_div(num_seqs, DEC_WAVES) : num_seqs,
+                  p.num_parts);
 
   auto launch = [&](auto tag, auto ctag, auto dim, auto whole, auto wpr) {
     using Tag = decltype(tag);
     using CTag = decltype(ctag);
     constexpr int HD = decltype(dim)::value;
-    constexpr bool WHOLE = decltype(whole)::value;
-    constexpr int WPR = decltype(wpr)::value;
     hipLaunchKernelGGL(
-        (paged_decode_kernel<Tag, CTag, WHOLE, HD, WPR>), grid,
-        dim3(DEC_BLOCK), 0, stream, (short*)out.data_ptr(),
-        WHOLE ? nullptr : tmp_out.data_ptr<float>(),
-        WHOLE ? nullptr : tmp_lse.data_ptr<float>(),
-        WHOLE ? nullptr : (unsigned*)arrived.data_ptr<int>(),
-        (const short*)q.data_ptr(),
-        (const typename CacheTraits<CTag>::elem*)kv_cache.data_ptr(),
-        block_table.data_ptr<int>(), seq_lens.data_ptr<int>(), scale_log2,
-        group, num_kv_heads, num_seqs, max_blocks, num_parts, part_len,
-        kv_cache.stride(0), q.stride(0), (int)sliding_window);
+        (paged_decode_kernel<Tag, CTag, decltype(whole)::value, HD,
+                             decltype(wpr)::value>),
+        grid, dim3(DEC_BLOCK), 0, stream,
+        decode_args<CTag>(p, out, q, kv_cache, num_seqs, block_table,
+                          seq_lens, sliding_window, tmp_out, tmp_lse));
   };
   auto by_dim = [&](auto tag, auto ctag, auto whole, auto wpr) {
     if (head_dim == 64)
@@ -571,9 +126,9 @@ void paged_decode_attention(torch::Tensor out, torch::Tensor q,
   };
   using one = std::integral_constant<int, 1>;
   using four = std::integral_constant<int, DEC_WAVES>;
-  if (wave_rows)           by_type(std::true_type{}, one{});
-  else if (num_parts == 1) by_type(std::true_type{}, four{});
-  else                     by_type(std::false_type{}, four{});
+  if (p.wave_rows)           by_type(std::true_type{}, one{});
+  else if (p.num_parts == 1) by_type(std::true_type{}, four{});
+  else                       by_type(std::false_type{}, four{});
   HIP_CHECK_KERNEL();
 }
 

@@ -34,6 +34,13 @@ void prefill_attention(torch::Tensor out, torch::Tensor q,
                        torch::Tensor query_start_loc, torch::Tensor seq_lens,
                        double scale, int64_t num_decodes,
                        int64_t max_query_len, int64_t sliding_window);
+void mixed_attention(torch::Tensor out, torch::Tensor q,
+                     torch::Tensor kv_cache, torch::Tensor block_table,
+                     torch::Tensor query_start_loc, torch::Tensor seq_lens,
+                     double scale, int64_t num_decodes,
+                     int64_t max_decode_len, int64_t max_query_len,
+                     int64_t sliding_window, torch::Tensor tmp_out,
+                     torch::Tensor tmp_lse);
 torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
                         c10::optional<torch::Tensor> bias);
 torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w);
@@ -202,6 +209,11 @@ TORCH_LIBRARY(vllm_amd, m) {
         "Tensor block_table, Tensor query_start_loc, Tensor seq_lens, "
         "float scale, int num_decodes, int max_query_len, "
         "int sliding_window) -> ()");
+  m.def("mixed_attention(Tensor(a!) out, Tensor q, Tensor kv_cache, "
+        "Tensor block_table, Tensor query_start_loc, Tensor seq_lens, "
+        "float scale, int num_decodes, int max_decode_len, "
+        "int max_query_len, int sliding_window, Tensor(b!) tmp_out, "
+        "Tensor(c!) tmp_lse) -> ()");
   m.def("lt_linear(Tensor a, Tensor w, Tensor? bias) -> Tensor");
   m.def("linear_silu_and_mul(Tensor a, Tensor w) -> Tensor");
   m.def("lt_linear_fp8(Tensor a, Tensor w) -> Tensor");
@@ -328,6 +340,7 @@ TORCH_LIBRARY_IMPL(vllm_amd, CUDA, m) {
   m.impl("reshape_and_cache", &vllm_amd::reshape_and_cache);
   m.impl("paged_decode_attention", &vllm_amd::paged_decode_attention);
   m.impl("prefill_attention", &vllm_amd::prefill_attention);
+  m.impl("mixed_attention", &vllm_amd::mixed_attention);
   m.impl("lt_linear", &vllm_amd::lt_linear);
   m.impl("linear_silu_and_mul", &vllm_amd::linear_silu_and_mul);
   m.impl("lt_linear_fp8", &vllm_amd::lt_linear_fp8);

@@ -150,6 +150,28 @@ def rope_and_cache(positions, q, k, v, cos_sin_cache, rotary_dim, is_neox,
         reshape_and_cache(k, v, kv_cache, slot_mapping)
 
 
+def _attention_mixes(rows, reqs, tokens, heads, head_dim, kv_heads, parts,
+                     max_decode_len, max_seq_len, max_query_len):
+    """Whether decode rows and portions of prompts run in one launch
+    (csrc/attention_mixed.hip). Not short rows in numbers that take a wave
+    each, heads that one of the two kernels does not take, grids past 65535
+    units, nor rows that read less than a twentieth of the time that the
+    portions may take (5 TB/s against 0.8 PFLOP/s): there is nothing to run
+    beside them, and tiles are 1.5 % slower in the joint kernel (1 row x
+    1000 keys and 8191 tokens 651 and 661 us)."""
+    if not 0 < rows < reqs or head_dim not in (64, 128):
+        return False
+    if heads % kv_heads or heads // kv_heads > 8:
+        return False
+    if parts == 1 and max_decode_len <= 512 and rows * kv_heads >= 1024:
+        return False
+    read_us = rows * max_decode_len * kv_heads * head_dim * 4 / 5e6
+    tile_us = (tokens - rows) * max_seq_len * heads * head_dim * 2 / 8e8
+    tiles = -(-max_query_len * (heads // kv_heads) // 128)
+    return (read_us * 20 >= tile_us
+            and tiles * (reqs - rows) + rows * parts < 65536)
+
+
 def attention_unified(
     q,
     kv_cache,
@@ -197,6 +219,19 @@ def attention_unified(
         else:
             tmp_out = q.new_empty(0, dtype=torch.float32)
             tmp_lse = tmp_out
+        if (max_query_len <= 0 and num_decodes < num_reqs
+                and head_dim in (64, 128)):
+            qsl = query_start_loc
+            max_query_len = int((qsl[1:] - qsl[:-1]).max().item())
+        if _attention_mixes(num_decodes, num_reqs, num_tokens, num_heads,
+                            head_dim, kv_cache.shape[2], num_parts,
+                            max_decode_len, max_seq_len, max_query_len):
+            _C.mixed_attention(
+                out, q, kv_cache, block_table, query_start_loc, seq_lens,
+                scale, num_decodes, max_decode_len, max_query_len,
+                sliding_window, tmp_out, tmp_lse,
+            )
+            return out
         _C.paged_decode_attention(
             out[:num_decodes], q_dec, kv_cache, block_table, seq_lens,
             scale, max_decode_len, sliding_window, tmp_out, tmp_lse,
