@@ -18,6 +18,10 @@
 //     (4g..4g+3, 16+4g..) holds exactly the P^T fragment of those keys
 //     when the contraction runs over keys in that order, so P never
 //     moves between lanes.
+//   - Values are read as lines that leave L2 first: each is needed once,
+//     and they no longer push out what other workgroups are about to read
+//     (keys cannot be: a load takes half a line of each row, the other half
+//     would be fetched again).
 //   - P stays at more than 16 bits: it is split in two 16-bit parts
 //     (p = hi + lo, error 2^-17) and multiplied twice; the matrix cores
 //     are idle here anyway. Sums and outputs are fp32. Results are as far
@@ -27,10 +31,10 @@
 // Against the vector-ALU form it replaced (16 lanes per token, dot
 // products reduced with shuffles), us per layer at 32 query and 8 KV
 // heads of 128:
-//   1 x 1000 keys 46 -> 13; 256 x 129..2176 keys 349 -> 228 (5.3 TB/s);
-//   1024 x 129..176 keys 206 -> 121 (5.3 TB/s; 132 with the last 32 keys
-//   of a row read whole);
-//   64 x 4096..8192 keys, fp8 cache 371 -> 160 (5.2 TB/s).
+//   1 x 1000 keys 46 -> 8; 256 x 129..2176 keys 349 -> 203 (6.0 TB/s; 223
+//   with values read as everything else); 1024 x 129..176 keys 206 -> 111
+//   (119; 132 with the last 32 keys of a row read whole); 16 x 4096 keys 43
+//   (52); 64 x 4096..8192 keys, fp8 cache 371 -> 150 (159).
 //
 // The KV cache layout [2, blocks, kv_heads, block_size=64, D] keeps each
 // (block, head) tile contiguous (16 KB at D=128).
@@ -207,8 +211,8 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
     for (int i = 0; i < VN; ++i) {
       const int e = (i * WAVE_SIZE + lane) * EPV;
       const int r = min(max(e / HD, lo), hi);
-      vr[i] = *reinterpret_cast<const i32x4*>(tile + kv_plane_stride +
-                                              r * HD + e % HD);
+      vr[i] = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(
+          tile + kv_plane_stride + r * HD + e % HD));
     }
   };
 

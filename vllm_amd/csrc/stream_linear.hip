@@ -22,14 +22,18 @@
 //    order (arrivals.h; 2112 x 7168, 64 rows: 14.7 us in three parts, 21.3
 //    in one).
 //
-// us on weights from HBM, tuned library products -> these (floor at 6 TB/s):
+//  * Weights leave L2 first (lds_fill16_once): read once, they would push
+//    out x, which every workgroup reads (7168 x 16384, 64 rows 58 -> 49 us).
+//
+// us on weights from HBM, tuned library products -> these, in a graph, where
+// split products clear their counters by a launch of 2 us (floor at 6 TB/s):
 //                   1 row          8 rows         32 rows        64 rows
-//    4096 x 4096    10.5 ->  8.4   10.6 ->  8.4   11.8 -> 10.7   13.8 -> 13.1   (5.6)
-//    6144 x 4096    13.3 -> 11.8   14.5 -> 11.5   15.2 -> 13.9   17.9 -> 17.2   (8.4)
-//   28672 x 4096    51.7 -> 42.7   47.6 -> 42.4   48.3 -> 44.5   54.6 -> 47.4   (39)
-//    4096 x 14336   25.5 -> 23.2   25.7 -> 23.5   31.9 -> 27.1   37.6 -> 32.9   (20)
-//    2112 x 7168    12.2 ->  9.1   12.0 -> 10.6   15.8 -> 11.9   19.3 -> 14.7   (5.0)
-
+//    4096 x 4096    10.5 ->  7.5   10.6 ->  7.8   11.8 -> 11.4   13.8 -> 13.8   (5.6)
+//    6144 x 4096    13.3 -> 10.9   14.5 -> 11.4   15.2 -> 15.1   17.9 -> 16.6   (8.4)
+//   28672 x 4096    51.7 -> 38.9   47.6 -> 39.3   48.3 -> 40.6   54.6 -> 44.5   (39)
+//    4096 x 14336   25.5 -> 21.3   25.7 -> 22.0   31.9 -> 27.9   37.6 -> 34.4   (20)
+//    2112 x 7168    12.2 ->  9.4   12.0 -> 11.6   15.8 -> 14.0   19.3 -> 16.7   (5.0)
+//  128256 x 4096     179 ->  158    176 ->  159    192 ->  169    201 ->  194   (175)
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
 
@@ -130,7 +134,7 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     char* to = ring + slot * STEP;
 #pragma unroll
     for (int j = 0; j < 2 * NI; ++j)
-      lds_fill16(wbase + k, wat[j], to + j * SL_FILL);
+      lds_fill16_once(wbase + k, wat[j], to + j * SL_FILL);
 #pragma unroll
     for (int j = 0; j < XG; ++j)
       lds_fill16(reinterpret_cast<const char*>(x) + k, xat[j],
