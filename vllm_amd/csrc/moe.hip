@@ -11,13 +11,12 @@
 //
 // Two forms of the product, chosen by the average number of rows an
 // expert gets (ops/hip_ops.py):
-//   moe_stream_kernel  few rows: every weight is read once and used for at
-//                      most 64 rows, so HBM bounds it. Weights go straight
-//                      into MFMA fragments, no LDS and no barrier in the
-//                      loop. Weights may be stored in fragment order
+//   moe_rows_kernel    few rows: every weight is read once and used for at
+//                      most 64 rows, so HBM bounds it.
+//   moe_stream_kernel  the same for weights stored in fragment order
 //                      ([E][N/16][K/32][64 lanes][8], ops/hip_ops.py
-//                      moe_shuffle_weights): then a wave's load is one run
-//                      of 1 KB.
+//                      moe_shuffle_weights), or that do not begin on 16 B:
+//                      straight into MFMA fragments, no LDS in the loop.
 //   moe_tiles.hip      many rows: the matrix cores bound it; 128 or 256 x
 //                      256 tiles through LDS.
 //
@@ -32,7 +31,7 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
-#include "moe.h"
+#include "moe_rows.h"
 #include "tile_product.h"
 
 namespace vllm_amd {
@@ -200,16 +199,54 @@ static int split_of_grid(int m_tiles, int n_blocks) {
 }
 
 // --------------------------------------------------------------------------
-// Few rows. A workgroup takes 64 weight rows (32 gate + 32 up rows for
-// gated experts) of an expert and up to 64 token rows; its four waves take
-// a quarter of K each and add up at the end. A wave reads 64 weight rows
-// 128 B at a time straight into A fragments, the next 128 B while it
-// multiplies; token rows are B fragments, from L2. Two workgroups per CU
-// keep 128 KB of weights in flight. At 64 rows the matrix cores are 15 %
-// busy, so rows of padding cost nothing; 16-row groups past the tile's
-// last row are left out.
+// Few rows: weights are read once and used for at most 64 rows, so HBM bounds
+// it; at 64 rows the matrix cores are 15 % busy, so rows of padding cost
+// nothing. 8-row groups past the tile's last row are left out.
+//
+// Weights as they are stored: stream_product.h, 128 weight rows (64 gate + 64
+// up rows for gated experts) a workgroup, or 32 where those are too few to
+// fill the chip; LDS is filled in whole lines that leave L2 first. us by
+// fragments, as below, and so: 8 experts of 4096 x 14336, 2 a token, 1 token
+// 166 / 115, 4 409 / 330, 48 517 / 441 (6.4 TB/s), 90 592 / 457; 64 of 7168 x
+// 2048, 8 a token, 64 tokens 950 / 805; 128 of 2048 x 768 195 / 179.
+constexpr int SR_FILL = 128;   // workgroups that are enough
+
+template <typename Tag, int ACT, int NI>
+__launch_bounds__(THREADS, 1) __global__
+void moe_rows_kernel(const short* __restrict__ A,
+                     const short* __restrict__ W, int64_t expert_stride,
+                     short* __restrict__ C, int64_t ldc,
+                     const int* __restrict__ sorted,
+                     const int* __restrict__ expert_tiles, int K, int N,
+                     int topk_div, int total_flat, int m_tiles,
+                     int n_blocks) {
+  int tile, blk;
+  if (!tile_of_block(m_tiles, n_blocks, tile, blk)) return;
+  const int expert = expert_tiles[tile];
+  if (expert < 0) return;  // padding tile
+  __shared__ __align__(16) char lds[ROWS_LDS];
+  const int rows = rows_of_tile<BM>(sorted, tile, total_flat);
+  const int n0 = blk * (ACT == SILU_GATED ? NI * 8 : NI * 16);
+  const short* w = W + expert * expert_stride;
+  rows_body<Tag, ACT, NI>(lds, A, w, C, ldc, sorted, K, N, topk_div,
+                          tile * BM, rows, n0);
+}
+
+// Weights in fragment order, or that do not begin on 16 B: a workgroup takes
+// 64 weight rows (32 gate + 32 up rows for gated experts) of an expert and
+// up to 64 token rows; its four waves take a quarter of K each and add up at
+// the end. A wave reads 64 weight rows 128 B at a time straight into A
+// fragments, the next 128 B while it multiplies; token rows are B fragments,
+// from L2. Two workgroups per CU keep 128 KB of weights in flight.
 constexpr int ST_W = 64;     // weight rows per workgroup
 constexpr int ST_U = 2;      // 32-wide K steps per load
+
+// Runs of 1 KB (fragment order) leave L2 first; of half lines the other half
+// would be fetched again (519 -> 588 us for 48 tokens as above).
+template <int STEP> DEVINL s16x8 weights(const short* p) {
+  const s16x8* v = reinterpret_cast<const s16x8*>(p);
+  return STEP > 32 ? __builtin_nontemporal_load(v) : *v;
+}
 
 template <typename Tag, int ACT, int STEP, int MT>
 DEVINL void stream_body(const short* const (&wp)[4],
@@ -229,8 +266,7 @@ DEVINL void stream_body(const short* const (&wp)[4],
     for (int u = 0; u < ST_U; ++u) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        w[u][i] =
-            *reinterpret_cast<const s16x8*>(wp[i] + (int64_t)(s + u) * STEP);
+        w[u][i] = weights<STEP>(wp[i] + (int64_t)(s + u) * STEP);
 #pragma unroll
       for (int j = 0; j < MT; ++j)
         x[u][j] = *reinterpret_cast<const s16x8*>(xp[j] + (s + u) * 32);
@@ -265,8 +301,7 @@ DEVINL void stream_body(const short* const (&wp)[4],
   for (; s < s1; ++s) {   // an odd step is left
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const s16x8 w =
-          *reinterpret_cast<const s16x8*>(wp[i] + (int64_t)s * STEP);
+      const s16x8 w = weights<STEP>(wp[i] + (int64_t)s * STEP);
 #pragma unroll
       for (int j = 0; j < MT; ++j)
         acc[i][j] = mfma16<Tag>(
@@ -482,7 +517,17 @@ static void run_gemm(const torch::Tensor& a, const torch::Tensor& b,
               em <= sorted.numel());
   TORCH_CHECK(topk_div > 0 || a.size(0) >= em);
   if (em == 0) return;
-  const int cols = (form > 0 ? TL_W : ST_W) / (act == SILU_GATED ? 2 : 1);
+  const bool aligned = (uintptr_t)a.data_ptr() % 16 == 0 &&
+                       (uintptr_t)b.data_ptr() % 16 == 0 &&
+                       a.numel() * 2 < (1ll << 32) &&
+                       b_rows * K * 2 < (1ll << 32);
+  const bool by_rows = form == 0 && !shuf && aligned && K % SP_K == 0;
+  const int halves = act == SILU_GATED ? 2 : 1;
+  const bool wide =
+      (int64_t)m_tiles * ceil_div(N * halves, SR_WIDE) >= SR_FILL;
+  const int cols = (form > 0  ? TL_W
+                    : by_rows ? (wide ? SR_WIDE : SR_NARROW)
+                              : ST_W) / halves;
   const int n_blocks = ceil_div(N, cols);
   const int split = split_of_grid(m_tiles, n_blocks);
   const int64_t blocks =
@@ -491,10 +536,7 @@ static void run_gemm(const torch::Tensor& a, const torch::Tensor& b,
                : ((int64_t)m_tiles * n_blocks + 7) / 8 * 8;
   // (Tiles address rows and an expert's weights with 32 bits, and fill LDS
   // from them 16 B at a time.)
-  TORCH_CHECK(form == 0 || (a.numel() * 2 < (1ll << 32) &&
-                            b_rows * K * 2 < (1ll << 32) &&
-                            (uintptr_t)a.data_ptr() % 16 == 0 &&
-                            (uintptr_t)b.data_ptr() % 16 == 0));
+  TORCH_CHECK(form == 0 || aligned);
   TORCH_CHECK(blocks < (1ll << 30));
   auto stream = c10::hip::getCurrentHIPStream().stream();
   if (form > 0) {
@@ -515,6 +557,19 @@ static void run_gemm(const torch::Tensor& a, const torch::Tensor& b,
   auto launch = [&](auto tag, auto act_tag) {
     using Tag = decltype(tag);
     constexpr int ACT = decltype(act_tag)::value;
+    if (by_rows) {
+      auto rows = [&](auto kernel) {
+        hipLaunchKernelGGL(
+            kernel, grid, dim3(THREADS), 0, stream,
+            (const short*)a.data_ptr(), (const short*)b.data_ptr(),
+            b_rows * K, (short*)c.data_ptr(), c.size(1),
+            sorted.data_ptr<int>(), expert_tiles.data_ptr<int>(), K, N,
+            (int)topk_div, (int)total_flat, m_tiles, n_blocks);
+      };
+      if (wide) rows(moe_rows_kernel<Tag, ACT, SR_WIDE / 16>);
+      else      rows(moe_rows_kernel<Tag, ACT, SR_NARROW / 16>);
+      return;
+    }
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(
           kernel, grid, dim3(THREADS), 0, stream,

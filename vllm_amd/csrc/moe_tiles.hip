@@ -10,6 +10,13 @@
 // or experts of few rows) lay the four waves out along the weights; 32-row
 // groups without a row are left out.
 //
+// An expert that has at most 32 rows in all is no tile: its weights stream
+// past them (moe_rows.h; a few rows after whole tiles meet their weights in
+// L2 and stay a tile). Beside larger ones, us without and so: 64 experts of
+// 7168 x 2048, 8 a token, 100 tokens (0 to 46 rows) 987 / 854, 300 (4 to 139)
+// 1114 / 1031; 8 of 4096 x 14336, 2 a token, 100 tokens (15 to 41) 572 / 523.
+// With up to 64 rows 906, 1086 and 594.
+//
 // 64 experts of 7168 x 2048, 4096 tokens of 8, 50 to 1925 rows an expert:
 // 1.76 + 0.98 ms (eight waves by halves in turn 2.01 + 1.10); 512 rows each
 // 1.50 + 0.86 (1.28 and 1.12 PFLOP/s: the second, of 32 stages, pays the
@@ -20,7 +27,7 @@
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
 
-#include "moe.h"
+#include "moe_rows.h"
 #include "tile_product.h"
 
 namespace vllm_amd {
@@ -97,6 +104,8 @@ DEVINL void tile_body(char* lds, const TileArgs& t, const short* w,
       });
 }
 
+constexpr int TL_FEW = 32;   // rows of an expert that are no tile
+
 template <typename Tag, int ACT, int TM>
 __launch_bounds__(TP_THREADS, 1) __global__
 void moe_tile_kernel(const TileArgs t) {
@@ -107,10 +116,22 @@ void moe_tile_kernel(const TileArgs t) {
   using Whole = TileProduct<Tag, 2, 4, 4, 2, 3>;
   using Half = TileProduct<Tag, 1, 2, 4, 3, 3>;
   static_assert(Whole::TM == 256 && Half::TM == 128);
-  __shared__ __align__(16) char lds[TM == 256 ? Whole::LDS : Half::LDS];
+  static_assert(Whole::LDS <= ROWS_LDS && Half::LDS <= ROWS_LDS);
+  __shared__ __align__(16) char lds[ROWS_LDS];
   const int rows = rows_of_tile<TM>(t.sorted, tile, t.total_flat);
   const int n0 = blk * (ACT == SILU_GATED ? TL_W / 2 : TL_W);
   const short* w = t.w + t.expert_tiles[tile] * t.expert_stride;
+  if (rows <= TL_FEW &&
+      (tile == 0 || t.expert_tiles[tile - 1] != t.expert_tiles[tile])) {
+    constexpr int PER = SR_WIDE / (ACT == SILU_GATED ? 2 : 1);
+    for (int n = n0; n < min(n0 + TL_W / SR_WIDE * PER, t.N); n += PER) {
+      if (n > n0) __syncthreads();
+      rows_body<Tag, ACT, SR_WIDE / 16>(lds, t.a, w, t.c, t.ldc, t.sorted,
+                                        t.K, t.N, t.topk_div, tile * TM,
+                                        rows, n);
+    }
+    return;
+  }
   if constexpr (TM == 256) {
     if (rows > 128) {
       tile_body<Tag, ACT, 2, 4, 4, 2>(lds, t, w, tile * TM, rows, n0);

@@ -21,7 +21,6 @@
 //    over workgroups; the last one to arrive adds up the parts in their
 //    order (arrivals.h; 2112 x 7168, 64 rows: 14.7 us in three parts, 21.3
 //    in one).
-//
 //  * Weights leave L2 first (lds_fill16_once): read once, they would push
 //    out x, which every workgroup reads (7168 x 16384, 64 rows 58 -> 49 us).
 //
@@ -34,13 +33,15 @@
 //    4096 x 14336   25.5 -> 21.3   25.7 -> 22.0   31.9 -> 27.9   37.6 -> 34.4   (20)
 //    2112 x 7168    12.2 ->  9.4   12.0 -> 11.6   15.8 -> 14.0   19.3 -> 16.7   (5.0)
 //  128256 x 4096     179 ->  158    176 ->  159    192 ->  169    201 ->  194   (175)
+
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
 #include <cmath>
+
 #include "arrivals.h"
-#include "common.h"
+#include "stream_product.h"
 
 namespace vllm_amd {
 
@@ -52,8 +53,6 @@ torch::Tensor silu_and_mul(torch::Tensor x);
 namespace {
 
 constexpr int SL_ROWS = 64;      // rows of x at most
-constexpr int SL_K = 64;         // columns of K per step of a wave: 128 B
-constexpr int SL_FILL = 1024;    // bytes of a fill: 8 rows x 128 B
 constexpr int SL_PARTS = 8;      // of K, over workgroups
 constexpr int SL_JOBS = 1024;    // column tiles whose K is split
 constexpr int SL_LDS = 160 * 1024;
@@ -67,7 +66,7 @@ constexpr int SL_NFORMS = sizeof(SL_FORMS) / sizeof(Form);
 
 // xg: groups of 8 rows of x.
 constexpr int ring_bytes(Form f, int xg) {
-  return f.wv * f.d * (2 * f.ni + xg) * SL_FILL;
+  return f.wv * f.d * (2 * f.ni + xg) * SP_FILL;
 }
 constexpr int sums_bytes(Form f, int xg) {
   return f.wv * f.ni * ((xg + 1) / 2) * WAVE_SIZE * 16;
@@ -85,11 +84,9 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     const short* __restrict__ w, const short* __restrict__ bias, const int M,
     const int N, const int K, const int n_tiles, const int parts,
     f32x4* __restrict__ part_sums, unsigned* __restrict__ arrived) {
-  constexpr int MT = (XG + 1) / 2;      // 16-row groups of x
-  constexpr int FILLS = 2 * NI + XG;
-  constexpr int STEP = FILLS * SL_FILL;
+  using P = StreamProduct<Tag, NI, XG, WV, D>;
+  constexpr int MT = P::MT;
   constexpr int NO = SILU ? NI / 2 : NI;
-  static_assert(D > 1 && (D - 1) * FILLS < 64, "what a wait can count");
   extern __shared__ __align__(16) char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
@@ -99,116 +96,28 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
   const int part = blockIdx.x / n_tiles;
   const int n0 = tile * NO * 16;
 
-  // Steps of this workgroup's part of K, every WV-th for this wave.
-  const int steps = K / SL_K;
-  const int s0 = steps * part / parts;
-  const int s1 = steps * (part + 1) / parts;
-  const int n = s1 - s0 > wave ? (s1 - s0 - wave + WV - 1) / WV : 0;
-  const int turn = n > 0 ? (int)((blockIdx.x / 8) % (unsigned)n) : 0;
-
-  // Byte places of this lane's pieces in the tile's rows; rows past the
-  // end repeat the last. 16 B chunk c of row r lies at c ^ (r / 2 & 7), so
-  // that the 16 rows of a fragment read meet no bank twice.
-  const int frow = lane >> 3;
-  const char* wbase = reinterpret_cast<const char*>(w + (int64_t)n0 * K);
+  // Rows past the end repeat the last.
   uint32_t wat[2 * NI], xat[XG];
 #pragma unroll
   for (int i = 0; i < 2 * NI; ++i) {
-    const int r = i * 8 + frow;
-    const int c = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+    const int r = i * 8 + (lane >> 3);
     const int half = SILU && i >= NI ? 1 : 0;
-    wat[i] = (uint32_t)(min(r - half * NO * 16, N - 1 - n0) + half * N) *
-                 (uint32_t)(K * 2) + c;
+    wat[i] = sp_place(min(r - half * NO * 16, N - 1 - n0) + half * N, r, K);
   }
 #pragma unroll
   for (int i = 0; i < XG; ++i) {
-    const int r = i * 8 + frow;
-    xat[i] = (uint32_t)min(r, M - 1) * (uint32_t)(K * 2) +
-             ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+    const int r = i * 8 + (lane >> 3);
+    xat[i] = sp_place(min(r, M - 1), r, K);
   }
-  char* ring = lds + wave * (D * STEP);
-  auto fill = [&](int i, int slot) {
-    i = min(i, n - 1) + turn;
-    const int64_t k = (int64_t)(s0 + wave + (i >= n ? i - n : i) * WV) *
-                      (SL_K * 2);
-    char* to = ring + slot * STEP;
-#pragma unroll
-    for (int j = 0; j < 2 * NI; ++j)
-      lds_fill16_once(wbase + k, wat[j], to + j * SL_FILL);
-#pragma unroll
-    for (int j = 0; j < XG; ++j)
-      lds_fill16(reinterpret_cast<const char*>(x) + k, xat[j],
-                 to + (2 * NI + j) * SL_FILL);
-  };
+  const int steps = K / SP_K;
+  P::run(lds, wave, steps * part / parts, steps * (part + 1) / parts,
+         blockIdx.x / 8, reinterpret_cast<const char*>(w + (int64_t)n0 * K),
+         wat, reinterpret_cast<const char*>(x), xat);
 
-  f32x4 acc[NI][MT];
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // The product is formed transposed: a lane ends up with four neighbouring
-  // columns of row l16. (Of 8 rows the upper lanes repeat the lower.)
-  const int xrow = XG == 1 ? l16 & 7 : l16;
-  auto multiply = [&](int slot) {
-    const char* from = ring + slot * STEP;
-    s16x8 wf[2][NI], xf[2][MT];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-        wf[u][i] = *reinterpret_cast<const s16x8*>(
-            from + (i * 16 + l16) * 128 +
-            ((u * 4 + l4) ^ ((l16 >> 1) & 7)) * 16);
-#pragma unroll
-      for (int j = 0; j < MT; ++j)
-        xf[u][j] = *reinterpret_cast<const s16x8*>(
-            from + 2 * NI * SL_FILL + (j * 16 + xrow) * 128 +
-            ((u * 4 + l4) ^ ((xrow >> 1) & 7)) * 16);
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < MT; ++j)
-          acc[i][j] = mfma16<Tag>(wf[u][i], xf[u][j], acc[i][j]);
-  };
-  if (n > 0) {
-    // Short waves fill the last step more than once: the counts that the
-    // waits go by stay the same.
-#pragma unroll
-    for (int d = 0; d < D - 1; ++d) fill(d, d);
-    int slot = 0, i = 0;
-    for (; i + D - 1 < n; ++i) {
-      fill(i + D - 1, slot == 0 ? D - 1 : slot - 1);
-      lds_fill_wait<(D - 1) * FILLS>();
-      asm volatile("" ::: "memory");
-      multiply(slot);
-      // Read before it is filled again.
-      __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
-      asm volatile("" ::: "memory");
-      slot = slot + 1 == D ? 0 : slot + 1;
-    }
-    lds_fill_wait();
-    asm volatile("" ::: "memory");
-    for (; i < n; ++i) {
-      multiply(slot);
-      slot = slot + 1 == D ? 0 : slot + 1;
-    }
-  }
-
-  // Sums of all waves; each wave goes on with a share of the tiles.
-  constexpr int T = NI * MT;
+  // Each wave goes on with a share of the tiles.
+  constexpr int T = P::T;
   constexpr int TO = NO * MT;
   constexpr int PER = (TO + WV - 1) / WV;
-  f32x4* red = reinterpret_cast<f32x4*>(lds);
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j)
-      red[(wave * T + i * MT + j) * WAVE_SIZE + lane] = acc[i][j];
-  __syncthreads();
   constexpr int H = SILU ? 2 : 1;
   f32x4 v[PER][H];
 #pragma unroll
@@ -216,12 +125,7 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     const int t = u * WV + wave;
     if (t >= TO) break;
 #pragma unroll
-    for (int h = 0; h < H; ++h) {
-      v[u][h] = red[(h * TO + t) * WAVE_SIZE + lane];
-#pragma unroll
-      for (int q = 1; q < WV; ++q)
-        v[u][h] += red[(q * T + h * TO + t) * WAVE_SIZE + lane];
-    }
+    for (int h = 0; h < H; ++h) v[u][h] = P::sum(lds, h * TO + t);
   }
   if (parts > 1) {
     f32x4* sums = part_sums + (int64_t)tile * parts * T * WAVE_SIZE + lane;
@@ -293,7 +197,7 @@ Plan plan(int xg, int64_t rows_w, int K, bool silu) {
     const int64_t tiles = (rows_w + f.ni * 16 - 1) / (f.ni * 16);
     for (int parts : {1, 2, 3, 4, 6, 8}) {
       if (parts > 1 && (tiles > SL_JOBS || tiles * parts > 1100 ||
-                        K / SL_K / parts < f.wv))
+                        K / SP_K / parts < f.wv))
         continue;
       const double mb = (f.ni * 16 + xg * 8) * 2e-6 * K / parts;
       const double jobs = (double)(tiles * parts);
@@ -379,7 +283,7 @@ bool stream_linear_takes(const torch::Tensor& x, const torch::Tensor& w,
                          int64_t n) {
   const int64_t K = x.size(1);
   return x.size(0) > 0 && x.size(0) <= SL_ROWS && n > 0 && n % 4 == 0 &&
-         K > 0 && K % SL_K == 0 && K < (1 << 24) &&
+         K > 0 && K % SP_K == 0 && K < (1 << 24) &&
          w.size(0) < (1 << 30) && (w.size(0) + 160) * K * 2 < (1ll << 32) &&
          (x.scalar_type() == torch::kBFloat16 ||
           x.scalar_type() == torch::kHalf) &&

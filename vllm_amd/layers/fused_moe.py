@@ -234,10 +234,10 @@ class FusedMoE(nn.Module):
     def _maybe_shuffled(self, hidden):
         import os
 
-        # Fragment-major streaming is opt-in (VLLM_AMD_MOE_SHUF=1): 1 to
-        # 10 % faster where an expert gets few rows (8 experts of 4096 x
-        # 14336: 1 token 165 -> 146 us, 48 tokens 518 -> 500), for a
-        # second copy of the weights.
+        # Fragment-major streaming is opt-in (VLLM_AMD_MOE_SHUF=1) and no
+        # longer faster, for a second copy of the weights (8 experts of
+        # 4096 x 14336: 1 token 114 us as stored, 132 so, 48 tokens 445 and
+        # 443).
         if (not hidden.is_cuda
                 or os.environ.get("VLLM_AMD_MOE_SHUF", "0") != "1"):
             return None, None

@@ -483,11 +483,11 @@ def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
 
 # Form of the expert products by the average number of rows an expert
 # gets: below 24 weights are streamed past at most 64 rows, below 192 tiles
-# of 128 rows, from there 256. ms streamed / 128 / 256: 8 experts of 4096 x
-# 14336, 12 rows 0.54 / 0.57 / 0.59, 32 rows 0.74 / 0.61 / 0.62, 128 rows
-# 1.49 / 0.69 / 0.86, 256 rows 2.74 / 1.14 / 0.99; 64 experts of 7168 x
-# 2048, 16 rows 1.11 / 1.00 / 1.00, 64 rows 1.89 / 1.17 / 1.17, 192 rows
-# 4.21 / 1.79 / 1.79, 512 rows 10.2 / 3.70 / 3.20.
+# of 128 rows, from there 256 (in which an expert of at most 32 rows is
+# streamed as well). ms streamed / 128 / 256: 8 experts of 4096 x 14336, 12
+# rows 0.45 / 0.50 / 0.50, 32 rows 0.47 / 0.54 / 0.54, 128 rows 1.04 / 0.65 /
+# 0.66, 256 rows 1.92 / 1.01 / 0.95; 64 experts of 7168 x 2048, 16 rows 0.88 /
+# 0.88 / 0.88, 64 rows 1.51 / 1.07 / 1.07, 192 rows 2.96 / 1.54 / 1.30.
 _MOE_TILES_FROM = 24
 _MOE_WIDE_TILES_FROM = 192
 # The average says little where rows meet in few experts (equal prompts,
@@ -496,12 +496,10 @@ _MOE_WIDE_TILES_FROM = 192
 # an expert may get more than 64 (the batch holds more tokens) and one tile
 # per expert fills the chip. us streamed / 128, experts chosen evenly | by
 # half of the tokens | all the same: 64 experts of 7168 x 2048, 8 a token,
-# 80 tokens 1018 / 993 | 1023 / 985 | 350 / 201, 191 tokens 1177 / 1018 |
-# 1255 / 1005 | 526 / 225; 256 experts, 767 tokens 4591 / 3890 | 4916 /
-# 4004 | 1854 / 679; 128 of 2048 x 768, 65 tokens 237 / 238 | 216 / 219 |
-# 67 / 60. Not filled: 8 experts of 4096 x 14336, 2 a token, 65 tokens 530 /
-# 555 | 559 / 562 | 400 / 312. Fewer than 4: 128 of 2048 x 768, 1 a token,
-# 192 tokens 188 / 204 | 145 / 148 | 55 / 58.
+# 80 tokens 856 / 858 | 858 / 846 | 267 / 197, 191 tokens 923 / 888 | 959 /
+# 900 | 342 / 212; 128 of 2048 x 768, 65 tokens 209 / 218 | 210 / 220 | 51 /
+# 46. Not filled: 8 experts of 4096 x 14336, 2 a token, 65 tokens 439 / 516 |
+# 452 / 504 | 281 / 299.
 _MOE_STREAM_ROWS = 64
 _MOE_CHIP_TILES = 256
 
