@@ -1,6 +1,6 @@
-"""Linear layers on few rows (csrc/stream_linear.hip): sizes at the edges
-of its forms, parts and epilogues against fp32 products of the same
-operands."""
+"""Linear layers on few rows (csrc/stream_linear.hip) and on up to 256
+(csrc/tile_linear.hip): sizes at the edges of their forms, parts and
+epilogues against fp32 products of the same operands."""
 
 import pytest
 import torch
@@ -36,11 +36,17 @@ SHAPES = [(1, 8, 64), (8, 16, 128), (9, 2112, 7168), (16, 24, 192),
           (64, 2112, 7168), (64, 4096, 4096), (1, 4096, 4096),
           (64, 6144, 4096), (5, 28672, 512), (64, 28672, 512),
           (40, 22016, 256), (64, 37888, 256), (3, 128256, 128)]
+# Tiles of 128 and 256 weight rows, the last one ragged; row groups of 32 at
+# both ends of the 128- and 256-row forms; one stage of K, fewer than LDS
+# holds, and more.
+TILES = [(65, 32752, 64), (96, 65536, 128), (128, 32768, 320),
+         (129, 32752, 64), (161, 65472, 192), (200, 31744, 640),
+         (255, 32768, 448), (256, 65536, 64), (70, 30720, 1024)]
 
 
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("m,n,k", SHAPES + TILES)
 def test_linear(m, n, k, dtype):
     from vllm_amd.ops import hip_ops
     x, w = _operands(m, n, k, dtype)
@@ -52,10 +58,10 @@ def test_linear(m, n, k, dtype):
 
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("m,n,k", SHAPES + TILES)
 def test_linear_silu_and_mul(m, n, k, dtype):
     from vllm_amd.ops import hip_ops
-    x, w = _operands(m, 2 * n if n < 60000 else n, k, dtype)
+    x, w = _operands(m, 2 * n if n < 30000 else n, k, dtype)
     gate, up = (x.float() @ w.float().t()).chunk(2, -1)
     expect = torch.nn.functional.silu(gate) * up
     _check(hip_ops.linear_silu_and_mul(x, w), expect, dtype)

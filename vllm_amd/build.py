@@ -41,6 +41,7 @@ SOURCES = [
     CSRC / "latent_attention_tiles.hip",
     CSRC / "ssd.hip",
     CSRC / "stream_linear.hip",
+    CSRC / "tile_linear.hip",
     CSRC / "arrivals.cpp",
     CSRC / "gemm_hipblaslt.cpp",
     CSRC / "bindings.cpp",

@@ -32,6 +32,9 @@ bool stream_linear_takes(const torch::Tensor& x, const torch::Tensor& w,
                          int64_t n);
 torch::Tensor stream_linear(const torch::Tensor& x, const torch::Tensor& w,
                             const c10::optional<torch::Tensor>& bias);
+// tile_linear.hip
+bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
+                 const torch::Tensor& w, bool silu);
 
 namespace {
 
@@ -318,14 +321,19 @@ torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
   const int64_t K = sizes.back();
   auto a2 = a.reshape({-1, K}).contiguous();
   sizes.back() = w.size(0);
-  // Few rows stream the weights through a kernel of our own (which side is
-  // faster at which size: stream_linear.hip).
-  if (w.dim() == 2 && stream_linear_takes(a2, w, w.size(0)) &&
+  // Few rows stream the weights through a kernel of our own, and some more
+  // meet them in tiles (which side is faster at which size: stream_linear.hip
+  // and tile_linear.hip).
+  const bool ours =
+      w.dim() == 2 && a2.size(0) > 0 &&
       (!bias.has_value() ||
        (bias->scalar_type() == a2.scalar_type() && bias->is_contiguous() &&
-        bias->numel() == w.size(0))))
+        bias->numel() == w.size(0)));
+  if (ours && stream_linear_takes(a2, w, w.size(0)))
     return stream_linear(a2, w, bias).reshape(sizes);
   auto out = torch::empty({a2.size(0), w.size(0)}, a.options());
+  if (ours && !bias.has_value() && tile_linear(out, a2, w, false))
+    return out.reshape(sizes);
   run_matmul(out, a2, w, bias);
   return out.reshape(sizes);
 }

@@ -49,6 +49,9 @@ namespace vllm_amd {
 torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
                         c10::optional<torch::Tensor> bias);
 torch::Tensor silu_and_mul(torch::Tensor x);
+// tile_linear.hip
+bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
+                 const torch::Tensor& w, bool silu);
 
 namespace {
 
@@ -307,8 +310,8 @@ torch::Tensor stream_linear(const torch::Tensor& x, const torch::Tensor& w,
   return out;
 }
 
-// silu(x @ gate^T) * (x @ up^T), w = [gate; up]; in one launch where
-// stream_linear takes it (the products are then not rounded in between).
+// silu(x @ gate^T) * (x @ up^T), w = [gate; up]; in one launch where this file
+// or tile_linear takes it (the products are then not rounded in between).
 torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w) {
   TORCH_CHECK(w.dim() == 2 && w.size(0) % 2 == 0 && a.dim() >= 1 &&
               a.size(-1) == w.size(1) && a.scalar_type() == w.scalar_type(),
@@ -317,9 +320,12 @@ torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w) {
   auto x = a.reshape({-1, sizes.back()}).contiguous();
   const int64_t N = w.size(0) / 2;
   sizes.back() = N;
-  if (!stream_linear_takes(x, w, N))
-    return silu_and_mul(lt_linear(x, w, c10::nullopt)).reshape(sizes);
   auto out = torch::empty({x.size(0), N}, x.options());
+  if (!stream_linear_takes(x, w, N)) {
+    if (x.size(0) > 0 && tile_linear(out, x, w, true))
+      return out.reshape(sizes);
+    return silu_and_mul(lt_linear(x, w, c10::nullopt)).reshape(sizes);
+  }
   if (x.scalar_type() == torch::kBFloat16)
     launch<BF16Tag, true>(out, x, w, nullptr, (int)N);
   else

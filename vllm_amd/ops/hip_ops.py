@@ -97,10 +97,11 @@ def linear(x, weight, bias=None):
 
 def linear_silu_and_mul(x, weight):
     # The activation as the product's epilogue where few rows stream the
-    # weights (csrc/stream_linear.hip); other shapes take two launches.
+    # weights (csrc/stream_linear.hip) and in tiles of up to 256 rows
+    # (tile_linear.hip); other shapes take two launches.
     n2, k = weight.shape
     if (x.dtype == torch.float32 or n2 % 16 or k % 64
-            or x.numel() > 64 * k or x.numel() == 0):
+            or x.numel() > 256 * k or x.numel() == 0):
         return silu_and_mul(linear(x, weight))
     return _C.linear_silu_and_mul(x, weight)
 
