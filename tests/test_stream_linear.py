@@ -97,6 +97,7 @@ def test_replays():
     from vllm_amd.ops import hip_ops
     x, w = _operands(33, 2112, 7168, torch.bfloat16)
     side = torch.cuda.Stream()
+    torch.cuda.synchronize()
     with torch.cuda.stream(side):
         eager = hip_ops.linear(x, w)
     torch.cuda.synchronize()

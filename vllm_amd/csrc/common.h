@@ -246,6 +246,13 @@ DEVINL void reads_ahead() {
   }
 }
 
+// 16 B from global memory; ONCE: a line that nobody reads again, which
+// leaves the caches first.
+template <bool ONCE> DEVINL s16x8 load16(const short* p) {
+  const s16x8* v = reinterpret_cast<const s16x8*>(p);
+  return ONCE ? __builtin_nontemporal_load(v) : *v;
+}
+
 // 64 lanes x 16 B from global memory straight into LDS: lane i's 16 bytes
 // land at dst + 16 * i (dst the same in all lanes). No register receives
 // anything, so the kernel waits itself (lds_fill_wait, then a barrier for
