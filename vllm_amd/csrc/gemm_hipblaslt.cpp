@@ -1,4 +1,5 @@
-// Tuned hipBLASLt GEMM for the linear layers (bf16/fp16, TN, row-major).
+// Tuned hipBLASLt GEMM for the linear layers (bf16/fp16, TN, row-major)
+// whose rows are not few enough for stream_linear.hip or tile_linear.hip.
 //
 // torch's F.linear on ROCm picks heuristics that leave ~1.5-2x on the
 // table for both skinny decode shapes (weight-streaming bound) and big

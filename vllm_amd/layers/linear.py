@@ -5,8 +5,9 @@ Merged/QKV/RowParallel): weights are sharded at construction time; a
 RowParallelLinear forward ends in one RCCL all-reduce over xGMI — the
 dominant collective of TP decode (2 per decoder layer).
 
-On GPU, GEMMs go through the tuned hipBLASLt op (ops.linear — per-shape
-algo search, csrc/gemm_hipblaslt.cpp); on CPU, torch F.linear.
+On GPU, products go through ops.linear: kernels of our own for few rows
+(csrc/stream_linear.hip, csrc/tile_linear.hip), else tuned hipBLASLt
+(per-shape algo search, csrc/gemm_hipblaslt.cpp); on CPU, torch F.linear.
 """
 
 from __future__ import annotations

@@ -117,7 +117,8 @@ def attention_unified(
 
 
 def linear(x, weight, bias=None):
-    """x @ weight.T + bias — tuned hipBLASLt on GPU, F.linear on CPU."""
+    """x @ weight.T + bias — kernels of our own for few rows and tuned
+    hipBLASLt for others on GPU, F.linear on CPU."""
     return get_backend(x.device).linear(x, weight, bias)
 
 

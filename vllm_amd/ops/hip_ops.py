@@ -86,9 +86,10 @@ def gelu_and_mul(x):
 
 
 def linear(x, weight, bias=None):
-    # Tuned hipBLASLt GEMM (per-shape algo search on first use). Rows
-    # that are not 16-byte multiples fall outside its aligned kernels:
-    # those shapes go to torch's vendor GEMM instead.
+    # Few rows stream the weights (csrc/stream_linear.hip, tile_linear.hip),
+    # others take a tuned hipBLASLt GEMM (per-shape algo search on first
+    # use). Rows that are not 16-byte multiples fall outside the aligned
+    # kernels: those shapes go to torch's vendor GEMM instead.
     per16 = 4 if x.dtype == torch.float32 else 8
     if weight.shape[0] % per16 or weight.shape[1] % per16:
         return torch.nn.functional.linear(x, weight, bias)
