@@ -60,6 +60,7 @@ def test_merge(ctx, hq, hkv, hd, window, dtype, cache):
                                atol=2.0 ** -9)
 
 
+@torch.inference_mode()   # as the runner captures
 def test_replays_and_streams():
     """Counters are left zero: by replays, by eager calls beside them and by
     calls on other streams."""

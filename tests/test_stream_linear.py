@@ -91,6 +91,7 @@ def test_views_and_other_streams():
 
 
 @gpu
+@torch.inference_mode()   # as the runner captures
 def test_replays():
     """A captured product counts in its own counters: replays beside eager
     calls on the same and on another stream give the same."""
