@@ -81,6 +81,19 @@ def test_mla_decode_split_ignores_prompts(hip, rows, monkeypatch):
     assert split(8192) == split(0)
 
 
+@pytest.mark.parametrize("rows,kv,span,window,parts", [
+    (1, 8, 1000, 0, 8),       # none shorter than 128 keys
+    (1, 8, 8192, 0, 32),      # one workgroup a CU ...
+    (2, 8, 8192, 0, 16),
+    (3, 8, 8192, 0, 22),      # ... two
+    (1, 8, 200000, 0, 64),    # the lanes of a wave
+    (2, 256, 8192, 0, 4),     # none longer than 2048 keys
+    (1, 8, 8192, 97, 1),      # a window's keys
+])
+def test_decode_parts(hip, rows, kv, span, window, parts):
+    assert hip._decode_parts(rows, kv, span, window) == parts
+
+
 @pytest.mark.parametrize("tokens,topk,E,H,form", [
     (64, 8, 64, 7168, 0),      # one streamed tile holds any expert's rows
     (65, 8, 64, 7168, 1),      # no longer

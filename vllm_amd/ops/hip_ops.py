@@ -33,17 +33,20 @@ _DEC_FILL = 512
 def _decode_parts(rows, kv_heads, max_seq_len, sliding_window):
     """Into how many partitions a row's keys are split. Every partition
     costs a pass over its fp32 partials, so no more than fill the chip:
-    16 rows x 4096 keys (8 KV heads of 128) take 52 us in 4 partitions,
-    58 in 16. Partitions of more than 2048 keys leave ragged batches
+    16 rows x 4096 keys (8 KV heads of 128) take 43.7 us in 4 partitions,
+    46.4 in 16. Partitions of more than 2048 keys leave ragged batches
     waiting for their longest row; below that more partitions only
-    cost: 256 rows x 129..2176 keys take 227 us in 2, 248 in 9; 64 rows
-    x 4096..8192 fp8 keys 154 us in 4, 180 in 32. At most 64, the lanes
-    of the merging wave."""
+    cost: 256 rows x 129..2176 keys take 203 us in 2, 239 in 9; 64 rows
+    x 4096..8192 fp8 keys 149 us in 4, 173 in 32. One or two rows are
+    hardly ragged and one workgroup a CU does: one x 8000 keys 15.4 us in
+    32, 19.4 in 63; two x 8000 19.5 in 16, 20.9 in 32 (24 x 500..3000
+    45.7 in 2, 37.7 in 3). At most 64, the lanes of the merging wave."""
     span = max(max_seq_len, 1)
     if sliding_window > 0:
         span = min(span, sliding_window + 31)
     units = -(-span // _DEC_UNIT)
-    parts = max(-(-_DEC_FILL // max(rows * kv_heads, 1)),
+    fill = _DEC_FILL // 2 if rows <= 2 else _DEC_FILL
+    parts = max(-(-fill // max(rows * kv_heads, 1)),
                 -(-units // _DEC_MAX_UNITS))
     return max(1, min(parts, units, 64))
 
