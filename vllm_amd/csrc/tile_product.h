@@ -75,6 +75,7 @@ struct TileProduct {
   static constexpr int LDS = PA * AB + PW * WB;
   static constexpr int WW = NI * 32;         // weight rows of a wave
   static_assert(PA >= 2 && PW >= PA && LDS <= 160 * 1024);
+  static_assert(NI % 2 == 0, "products of a step go in pairs");
 
   // fill_a(step, i, dst) and fill_w: the wave's i-th fill of 8 rows of a
   // stage, rows (wave * FA + i) * 8 .. of the tile. done(J, acc) gets the
