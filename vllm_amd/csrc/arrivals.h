@@ -50,8 +50,7 @@ DEVINL float part_get(const float* p) {
 DEVINL bool last_to_arrive(unsigned* counter, unsigned total,
                            unsigned* flag) {
   // Every wave's parts are written through before the workgroup counts.
-  __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
-  asm volatile("" ::: "memory");
+  global_wait();
   __syncthreads();
   if (threadIdx.x == 0) {
     const unsigned before = __hip_atomic_fetch_add(

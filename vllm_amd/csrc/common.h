@@ -302,6 +302,19 @@ template <int N = 0> DEVINL void lds_fill_wait() {
   static_assert(N >= 0 && N < 64);
   __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
 }
+// All of this wave's LDS operations, or all of its loads and stores, are done.
+// The builtin says nothing of memory to the compiler: without a barrier on
+// either side an access might be moved past the wait that is meant for it.
+DEVINL void lds_wait() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+  asm volatile("" ::: "memory");
+}
+DEVINL void global_wait() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+  asm volatile("" ::: "memory");
+}
 // Workgroup barrier that waits for this wave's LDS operations but not for
 // its loads (__syncthreads may wait for both).
 DEVINL void lds_barrier() {

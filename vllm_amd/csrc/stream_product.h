@@ -104,8 +104,7 @@ template <typename Tag, int NI, int XG, int WV, int D> struct StreamProduct {
         asm volatile("" ::: "memory");
         multiply(slot);
         // Read before it is filled again.
-        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
-        asm volatile("" ::: "memory");
+        lds_wait();
         slot = slot + 1 == D ? 0 : slot + 1;
       }
       lds_fill_wait();
