@@ -94,6 +94,63 @@ def test_replays_and_streams():
             assert torch.equal(o, expect)
 
 
+def _nodes(graph):
+    import ctypes
+    hip = ctypes.CDLL("libamdhip64.so")
+    n = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()),
+                                None, ctypes.byref(n)) == 0
+    return n.value
+
+
+@torch.inference_mode()
+def test_captured_launches_share_counters():
+    """A graph clears counters once for each of its streams, not once for
+    each launch; graphs of one pool, captured one after the other without an
+    eager call between them, do not disturb each other."""
+    from vllm_amd.ops import hip_ops
+    ctx = [1500, 200, 0, 3000, 129]
+    q, kv, table, qsl, lens = _rows(ctx, 32, 8, 128, torch.bfloat16,
+                                    torch.bfloat16)
+    x = torch.randn(33, 7168, device="cuda").bfloat16()
+    w = torch.randn(2112, 7168, device="cuda").bfloat16() * 0.01
+
+    def call():
+        return (hip_ops.attention_unified(
+            q, kv, table, qsl, lens, 0.09, num_decodes=len(ctx),
+            max_seq_len=4096), hip_ops.linear(x, w))
+
+    expect = call()
+    main, side = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graphs, outs, pool = [], [], None
+    for _ in range(3):
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph, stream=main, pool=pool):
+            out = [call(), call()]
+            side.wait_stream(main)
+            with torch.cuda.stream(side):
+                out.append(call())
+            out.append(call())
+            main.wait_stream(side)
+        assert _nodes(graph) == 8 + 2   # kernels and a fill for each stream
+        graph.instantiate()
+        pool = graph.pool()
+        graphs.append(graph)
+        outs.append(out)
+    for i in (0, 1, 2, 0, 2, 1):
+        for o in outs[i]:
+            for t in o:
+                t.zero_()
+        torch.cuda.synchronize()
+        graphs[i].replay()
+        eager = call()
+        torch.cuda.synchronize()
+        for o in outs[i] + [eager]:
+            for t, e in zip(o, expect):
+                assert torch.equal(t, e)
+
+
 # More tiles than rows and fewer, one of each; a portion shorter than a
 # tile, after cached tokens; heads in groups of 1, 7 and 8; rows in one and
 # in several partitions; a window; an fp8 cache; a negative scale.
