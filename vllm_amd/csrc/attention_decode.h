@@ -145,7 +145,7 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
   const int seq = WPR > 1 ? row_block : row_block * DEC_WAVES + wave;
   if (WPR == 1 && seq >= a.num_seqs) return;   // (no barrier below then)
   const int part = WPR > 1 ? part_block : 0;
-  const int ctx = a.seq_lens[seq];
+  const int ctx = load_uniform(a.seq_lens + seq);
   const int num_q_heads = num_kv_heads * group;
   const int hq0 = kvh * group;
   const int t_lo = sliding_window > 0 ? max(0, ctx - sliding_window) : 0;
@@ -188,7 +188,8 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
   const int* bt = a.block_table + (int64_t)seq * a.max_blocks_per_req;
   auto tile_of = [&](int key0) {
     return kv_cache +
-           ((int64_t)bt[key0 >> 6] * num_kv_heads + kvh) * (64 * HD) +
+           ((int64_t)load_uniform(bt + (key0 >> 6)) * num_kv_heads + kvh) *
+               (64 * HD) +
            (key0 & 63) * HD;
   };
   i32x4 kr[KT][KN], vr[VN];

@@ -103,13 +103,13 @@ DEVINL void prefill_tile(const PrefillArgs<CTag>& a, const int kvh,
   const int sliding_window = a.sliding_window;
   const float scale_log2 = a.scale_log2;
   const int64_t kv_plane_stride = a.kv_plane_stride;
-  const int q_start = a.query_start_loc[req];
-  const int ql = a.query_start_loc[req + 1] - q_start;
+  const int q_start = load_uniform(a.query_start_loc + req);
+  const int ql = load_uniform(a.query_start_loc + req + 1) - q_start;
   const int rows = ql * group;
   const int tile = (rows + PF_ROWS - 1) / PF_ROWS - 1 - from_last;
   if (tile < 0) return;
   const int row0 = tile * PF_ROWS;
-  const int ctx = a.seq_lens[req];
+  const int ctx = load_uniform(a.seq_lens + req);
   const int num_q_heads = num_kv_heads * group;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
@@ -210,10 +210,10 @@ DEVINL void prefill_tile(const PrefillArgs<CTag>& a, const int kvh,
     }
   };
 
-  load(bt[kt0]);
+  load(load_uniform(bt + kt0));
   store(kt0);
-  if (kt0 + 1 < kt_end) load(bt[kt0 + 1]);
-  int phys = bt[min(kt0 + 2, kt_end - 1)];
+  if (kt0 + 1 < kt_end) load(load_uniform(bt + kt0 + 1));
+  int phys = load_uniform(bt + min(kt0 + 2, kt_end - 1));
   __syncthreads();
 
   for (int kt = kt0; kt < kt_end; ++kt) {
@@ -237,7 +237,7 @@ DEVINL void prefill_tile(const PrefillArgs<CTag>& a, const int kvh,
     if (kt + 1 < kt_end) store(kt + 1);
     if (kt + 2 < kt_end) {
       load(phys);
-      phys = bt[min(kt + 3, kt_end - 1)];
+      phys = load_uniform(bt + min(kt + 3, kt_end - 1));
     }
 
     // --- mask, only where the tile meets an edge -------------------------

@@ -253,6 +253,14 @@ template <bool ONCE> DEVINL s16x8 load16(const short* p) {
   return ONCE ? __builtin_nontemporal_load(v) : *v;
 }
 
+// A value that no lane's place decides and that the launch does not change:
+// by way of the scalar cache. (A pointer that comes in a structure is not
+// known to be free of aliases. The compiler then loads through it as a vector,
+// and such a load waits for all that were issued before it.)
+DEVINL int load_uniform(const int* p) {
+  return *(const __attribute__((address_space(4))) int*)p;
+}
+
 // 64 lanes x 16 B from global memory straight into LDS: lane i's 16 bytes
 // land at dst + 16 * i (dst the same in all lanes). No register receives
 // anything, so the kernel waits itself (lds_fill_wait, then a barrier for
