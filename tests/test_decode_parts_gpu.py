@@ -37,6 +37,11 @@ def _rows(ctx, hq, hkv, hd, dtype, cache_dtype):
     ([900, 64, 1500], 16, 2, 256, 0, torch.bfloat16, None),
     ([3000, 100, 500], 8, 8, 128, 300, torch.bfloat16, None),
     ([2176 - 7 * i for i in range(256)], 8, 2, 128, 0, torch.bfloat16, None),
+    # More counters than lines, and than a stream's set holds.
+    ([2100 + i if i % 9 == 0 else i % 150 for i in range(300)], 8, 4, 64, 0,
+     torch.bfloat16, None),
+    ([2500 if i % 65 == 0 else 1 + i % 70 for i in range(520)], 32, 32, 64, 0,
+     torch.float16, None),
 ])
 def test_merge(ctx, hq, hkv, hd, window, dtype, cache):
     from vllm_amd.ops import hip_ops
@@ -92,6 +97,38 @@ def test_replays_and_streams():
         assert torch.equal(out, expect)
         for o in beside:
             assert torch.equal(o, expect)
+
+
+def test_more_streams_than_sets():
+    """More streams than have counters of their own, and one that is not
+    torch's."""
+    import ctypes
+    from vllm_amd.ops import hip_ops
+    ctx = [1500, 200, 0, 3000, 129]
+    q, kv, table, qsl, lens = _rows(ctx, 32, 8, 128, torch.bfloat16,
+                                    torch.bfloat16)
+
+    def call():
+        return hip_ops.attention_unified(
+            q, kv, table, qsl, lens, 0.09, num_decodes=len(ctx),
+            max_seq_len=4096)
+
+    expect = call()
+    hip = ctypes.CDLL("libamdhip64.so")
+    handle = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(handle)) == 0
+    streams = [torch.cuda.Stream() for _ in range(34)]
+    streams += [torch.cuda.ExternalStream(handle.value)]
+    torch.cuda.synchronize()
+    outs = []
+    for _ in range(3):
+        for s in streams:
+            with torch.cuda.stream(s):
+                outs.append(call())
+    torch.cuda.synchronize()
+    assert hip.hipStreamDestroy(handle) == 0
+    for o in outs:
+        assert torch.equal(o, expect)
 
 
 def _nodes(graph):

@@ -8,6 +8,8 @@
 #include <map>
 #include <mutex>
 
+#include "arrivals.h"
+
 namespace vllm_amd {
 
 namespace {
@@ -50,13 +52,13 @@ struct Captured {
 // may end and come back as another stream while work is under way.
 at::Tensor arrival_counters(const at::Tensor& like, int64_t n) {
   constexpr size_t SETS = 32;
-  constexpr int64_t COUNTERS = 16384;
   auto opt = like.options().dtype(torch::kInt);
   const auto stream = c10::hip::getCurrentHIPStream();
   const int64_t id = stream.id();
   const auto capture = capture_of(stream.stream());
-  if (n > COUNTERS || (id != 0 && id % 2 == 0) || !capture.known)
-    return torch::zeros({n}, opt);
+  const int64_t blocks = (n + ARRIVAL_BLOCK - 1) / ARRIVAL_BLOCK;
+  if (blocks > 1 || (id != 0 && id % 2 == 0) || !capture.known)
+    return torch::zeros({blocks * ARRIVAL_BLOCK}, opt);
   // (Never destroyed: the runtime may be gone by then.)
   using Key = std::pair<int, int64_t>;
   static auto* sets = new std::map<Key, at::Tensor>();
@@ -71,14 +73,14 @@ at::Tensor arrival_counters(const at::Tensor& like, int64_t n) {
   if (capture.active) {
     auto it = captured->find(key);
     if (it != captured->end()) return it->second.counters;
-    auto t = torch::zeros({COUNTERS}, opt);
+    auto t = torch::zeros({ARRIVAL_BLOCK}, opt);
     if (captured->size() < SETS)
       captured->emplace(key, Captured{stream.stream(), capture, t});
     return t;
   }
   auto it = sets->find(key);
   if (it != sets->end()) return it->second;
-  auto t = torch::zeros({COUNTERS}, opt);
+  auto t = torch::zeros({ARRIVAL_BLOCK}, opt);
   if (sets->size() < SETS) sets->emplace(key, t);
   return t;
 }

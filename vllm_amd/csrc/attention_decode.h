@@ -436,7 +436,7 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
     float* w_lds = reinterpret_cast<float*>(lds);   // [group][MAX_PARTS]
     static_assert(MAX_GROUP * MAX_PARTS * 4 + 4 <= dec_lds<CTag, HD>);
     if (!last_to_arrive(
-            a.arrived + (int64_t)seq * num_kv_heads + kvh, used,
+            a.arrived, (int64_t)seq * num_kv_heads + kvh, used,
             reinterpret_cast<unsigned*>(w_lds + MAX_GROUP * MAX_PARTS)))
       return;
     const int64_t row0 = ((int64_t)seq * num_q_heads + hq0) * num_parts;

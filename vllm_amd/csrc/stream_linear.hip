@@ -140,7 +140,7 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
       for (int h = 0; h < H; ++h)
         part_put(sums + (part * T + h * TO + t) * WAVE_SIZE, v[u][h]);
     }
-    if (!last_to_arrive(arrived + tile, parts,
+    if (!last_to_arrive(arrived, tile, parts,
                         reinterpret_cast<unsigned*>(lds)))
       return;
 #pragma unroll
