@@ -116,6 +116,37 @@ def test_replays():
         assert torch.equal(again, eager)
 
 
+def _form(m, rows, k, silu=False):
+    try:
+        from vllm_amd.ops import hip_ops
+    except (ImportError, OSError) as e:
+        pytest.skip(f"extension not built: {e}")
+    return hip_ops._C.linear_form(m, rows, k, silu)
+
+
+# What is wide and short, or narrow with many rows, goes to the library;
+# what lies on the other side of each line does not.
+@pytest.mark.parametrize("m,rows,k,silu,kind", [
+    (8, 50272, 256, False, 0), (8, 50272, 320, False, 1),
+    (16, 50272, 512, False, 0), (16, 50272, 576, False, 1),
+    (17, 151936, 1024, False, 0), (32, 151936, 1088, False, 1),
+    (33, 151936, 1536, False, 0), (64, 151936, 1600, False, 1),
+    (1, 49144, 64, False, 1), (32, 49144, 64, False, 1),
+    (33, 24576, 1024, False, 0), (33, 24576, 1088, False, 1),
+    (33, 24568, 1024, False, 1),
+    (33, 256, 6144, False, 0), (64, 8, 8192, False, 0),
+    (32, 256, 7168, False, 1), (64, 264, 7168, False, 1),
+    (64, 256, 6080, False, 1), (64, 256, 8256, False, 1),
+    (64, 98304, 1024, True, 0), (64, 98304, 1088, True, 1),
+    (32, 98304, 64, True, 1), (64, 98272, 64, True, 1),
+    (64, 256, 7168, True, 1),
+    (64, 4096, 4096, False, 1), (64, 4096, 4080, False, 0),
+    (0, 4096, 4096, False, 0), (8, 262144, 8192, False, 0),   # 4 GB
+])
+def test_route_by_sizes(m, rows, k, silu, kind):
+    assert _form(m, rows, k, silu)[0] == kind
+
+
 def test_gated_silu_calls_what_is_hooked():
     """The fused pass goes past the modules only where nothing would be
     left out: a hook, a bias or an adapter still runs."""

@@ -44,6 +44,8 @@ void mixed_attention(torch::Tensor out, torch::Tensor q,
 torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
                         c10::optional<torch::Tensor> bias);
 torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w);
+std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
+                                 bool silu);
 torch::Tensor lt_linear_fp8(torch::Tensor a, torch::Tensor w);
 void dynamic_quant_fp8(torch::Tensor out, torch::Tensor scales,
                        torch::Tensor x);
@@ -216,6 +218,8 @@ TORCH_LIBRARY(vllm_amd, m) {
         "Tensor(c!) tmp_lse) -> ()");
   m.def("lt_linear(Tensor a, Tensor w, Tensor? bias) -> Tensor");
   m.def("linear_silu_and_mul(Tensor a, Tensor w) -> Tensor");
+  m.def("linear_form(int rows, int weight_rows, int k, bool silu) -> int[]",
+        &vllm_amd::linear_form);
   m.def("lt_linear_fp8(Tensor a, Tensor w) -> Tensor");
   m.def("dynamic_quant_fp8(Tensor(a!) out, Tensor(b!) scales, Tensor x)"
         " -> ()");

@@ -50,6 +50,7 @@ torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
                         c10::optional<torch::Tensor> bias);
 torch::Tensor silu_and_mul(torch::Tensor x);
 // tile_linear.hip
+int tile_linear_form(int64_t M, int64_t rows_w, int64_t K, bool silu);
 bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
                  const torch::Tensor& w, bool silu);
 
@@ -66,6 +67,11 @@ constexpr Form SL_FORMS[] = {{1, 8, 4}, {2, 4, 2}, {4, 4, 2},
                              {6, 4, 2}, {8, 4, 2}, {8, 2, 2},
                              {10, 2, 2}};
 constexpr int SL_NFORMS = sizeof(SL_FORMS) / sizeof(Form);
+
+// Groups of 8 rows of x that a launch for M rows is made for.
+constexpr int row_groups(int64_t M) {
+  return M <= 8 ? 1 : M <= 16 ? 2 : M <= 32 ? 4 : 8;
+}
 
 // xg: groups of 8 rows of x.
 constexpr int ring_bytes(Form f, int xg) {
@@ -255,8 +261,7 @@ void launch_form(torch::Tensor& out, const torch::Tensor& x,
 template <typename Tag, bool SILU>
 void launch(torch::Tensor& out, const torch::Tensor& x,
             const torch::Tensor& w, const short* bias, int N) {
-  const int groups = ceil_div((int)x.size(0), 8);
-  const int xg = groups <= 2 ? groups : groups <= 4 ? 4 : 8;
+  const int xg = row_groups(x.size(0));
   const Plan p = plan(xg, w.size(0), (int)x.size(1), SILU);
   auto by_rows = [&](auto form) {
     constexpr int I = decltype(form)::value;
@@ -280,20 +285,60 @@ void launch(torch::Tensor& out, const torch::Tensor& x,
 
 }  // namespace
 
+// Whether a product of M rows with rows_w weight rows (silu: n = rows_w / 2
+// columns of out) is one for this file, by its sizes. Up to 64 rows it is,
+// but for two kinds at which the tuned library is ahead:
+//  * Wide and short ones. Workgroups hardly begin before they end, and what
+//    they write is no longer little beside the weights. us, library and this:
+//    50272 x 768, 16 / 32 / 64 rows 18.4 and 18.9, 19.1 and 20.5, 20.5 and
+//    26.9, x 2048 40 and 36 (64 rows); 65536 x 256, 8 / 32 / 64 rows 9.8 and
+//    10.8, 12.5 and 13.0, 11.7 and 17.7; 32000 x 512, 32 / 64 rows 10.7 and
+//    9.5, 10.9 and 12.2. An activation as epilogue makes up for most of it
+//    (131072 x 512, 64 rows 49 and 51).
+//  * Narrow ones of more than 32 rows: a few workgroups take in all of x (128
+//    x 7168, 32 / 64 rows 8.3 and 7.1, 8.4 and 9.5; 512 x 7168, 64 rows 10.8
+//    and 10.2; 128 x 14336 12.9 and 12.8; where K is shorter the library takes
+//    5.2 to 12.7, by the algorithm that its race came to).
+bool stream_sizes(int64_t M, int64_t rows_w, int64_t n, int64_t K) {
+  if (M <= 0 || M > SL_ROWS || n <= 0 || n % 4 != 0 || K <= 0 ||
+      K % SP_K != 0 || K >= (1 << 24) || rows_w >= (1 << 30) ||
+      (rows_w + 160) * K * 2 >= (1ll << 32))
+    return false;
+  if (rows_w != n) return !(M > 32 && n >= 49152 && K <= 1024);
+  if (rows_w >= 49152 && K <= std::min(256 * row_groups(M), 1536))
+    return false;
+  if (M > 32 && rows_w >= 24576 && K <= 1024) return false;
+  return !(M > 32 && rows_w <= 256 && K >= 6144 && K <= 8192);
+}
+
 // Whether stream_linear takes the product: x [M, K] and w [rows, K], both
 // contiguous; out has n columns.
 bool stream_linear_takes(const torch::Tensor& x, const torch::Tensor& w,
                          int64_t n) {
-  const int64_t K = x.size(1);
-  return x.size(0) > 0 && x.size(0) <= SL_ROWS && n > 0 && n % 4 == 0 &&
-         K > 0 && K % SP_K == 0 && K < (1 << 24) &&
-         w.size(0) < (1 << 30) && (w.size(0) + 160) * K * 2 < (1ll << 32) &&
+  return stream_sizes(x.size(0), w.size(0), n, x.size(1)) &&
          (x.scalar_type() == torch::kBFloat16 ||
           x.scalar_type() == torch::kHalf) &&
-         w.scalar_type() == x.scalar_type() && w.size(1) == K &&
+         w.scalar_type() == x.scalar_type() && w.size(1) == x.size(1) &&
          x.is_contiguous() && w.is_contiguous() &&
          (uintptr_t)x.data_ptr() % 16 == 0 &&
          (uintptr_t)w.data_ptr() % 16 == 0;
+}
+
+// What a product of these sizes runs as, for 16-bit operands that begin on
+// 16 B: {0} the library, {1, 16-row groups of weights, waves, ring steps,
+// 8-row groups of x, parts of K} stream_linear, {2, weight rows of a tile}
+// tile_linear.
+std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
+                                 bool silu) {
+  const int64_t n = silu ? weight_rows / 2 : weight_rows;
+  if (stream_sizes(rows, weight_rows, n, k)) {
+    const int xg = row_groups(rows);
+    const Plan p = plan(xg, weight_rows, (int)k, silu);
+    const Form f = SL_FORMS[p.form];
+    return {1, f.ni, f.wv, f.d, xg, p.parts};
+  }
+  const int tile = tile_linear_form(rows, weight_rows, k, silu);
+  return tile == 0 ? std::vector<int64_t>{0} : std::vector<int64_t>{2, tile};
 }
 
 // x, w and bias as stream_linear_takes and lt_linear have checked them.

@@ -142,15 +142,21 @@ void launch(torch::Tensor& out, const torch::Tensor& x,
 
 }  // namespace
 
+// The form for a product of these sizes, 0 if it is not one for this file.
+int tile_linear_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
+  if (rows_w <= 0 || rows_w % (silu ? 16 : 8) != 0 || K <= 0 ||
+      K % TP_K != 0 || K >= (1 << 22) || (rows_w + 256) * K * 2 >= (1ll << 32))
+    return 0;
+  return tile_form(M, rows_w, silu);
+}
+
 // The product of x [M, K] and w [rows, K], both contiguous, into out [M, n],
 // if it is one that this file takes.
 bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
                  const torch::Tensor& w, bool silu) {
-  const int64_t M = x.size(0), K = x.size(1);
-  const int form = tile_form(M, w.size(0), silu);
-  if (form == 0 || out.size(1) % 8 != 0 || K <= 0 || K % TP_K != 0 ||
-      K >= (1 << 22) || (w.size(0) + 256) * K * 2 >= (1ll << 32) ||
-      w.size(1) != K || w.scalar_type() != x.scalar_type() ||
+  const int64_t K = x.size(1);
+  const int form = tile_linear_form(x.size(0), w.size(0), K, silu);
+  if (form == 0 || w.size(1) != K || w.scalar_type() != x.scalar_type() ||
       (x.scalar_type() != torch::kBFloat16 &&
        x.scalar_type() != torch::kHalf) ||
       !x.is_contiguous() || !w.is_contiguous() ||
