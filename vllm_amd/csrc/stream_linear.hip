@@ -155,9 +155,23 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
       if (t >= TO) break;
 #pragma unroll
       for (int h = 0; h < H; ++h) {
-        v[u][h] = part_get(sums + (h * TO + t) * WAVE_SIZE);
-        for (int q = 1; q < parts; ++q)
-          v[u][h] += part_get(sums + (q * T + h * TO + t) * WAVE_SIZE);
+        // On their way at once, added in their order (a read past the last
+        // part repeats it: with a branch each read waits for the one before).
+        const f32x4* at = sums + (h * TO + t) * WAVE_SIZE;
+        auto add = [&](auto n) {
+          constexpr int Q = decltype(n)::value;
+          f32x4 p[Q];
+#pragma unroll
+          for (int q = 0; q < Q; ++q)
+            p[q] = part_get(at + min(q, parts - 1) * (T * WAVE_SIZE));
+          v[u][h] = p[0];
+#pragma unroll
+          for (int q = 1; q < Q; ++q)
+            if (q < parts) v[u][h] += p[q];
+        };
+        if (parts == 2)     add(std::integral_constant<int, 2>{});
+        else if (parts < 5) add(std::integral_constant<int, 4>{});
+        else                add(std::integral_constant<int, SL_PARTS>{});
       }
     }
   }
@@ -296,8 +310,8 @@ void launch(torch::Tensor& out, const torch::Tensor& x,
 //    9.5, 10.9 and 12.2. An activation as epilogue makes up for most of it
 //    (131072 x 512, 64 rows 49 and 51).
 //  * Narrow ones of more than 32 rows: a few workgroups take in all of x (128
-//    x 7168, 32 / 64 rows 8.3 and 7.1, 8.4 and 9.5; 512 x 7168, 64 rows 10.8
-//    and 10.2; 128 x 14336 12.9 and 12.8; where K is shorter the library takes
+//    x 7168, 32 / 64 rows 8.4 and 7.2, 8.4 and 9.5; 512 x 7168, 64 rows 10.8
+//    and 9.8; 128 x 14336 12.9 and 11.4; where K is shorter the library takes
 //    5.2 to 12.7, by the algorithm that its race came to).
 bool stream_sizes(int64_t M, int64_t rows_w, int64_t n, int64_t K) {
   if (M <= 0 || M > SL_ROWS || n <= 0 || n % 4 != 0 || K <= 0 ||
