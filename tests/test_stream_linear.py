@@ -141,6 +141,11 @@ def _form(m, rows, k, silu=False):
     (32, 98304, 64, True, 1), (64, 98272, 64, True, 1),
     (64, 256, 7168, True, 1),
     (64, 4096, 4096, False, 1), (64, 4096, 4080, False, 0),
+    (65, 128256, 512, False, 0), (65, 128256, 576, False, 2),
+    (128, 32768, 1024, False, 0), (128, 32768, 1088, False, 2),
+    (256, 65536, 2048, False, 0), (256, 65536, 2112, False, 2),
+    (256, 65536, 64, True, 2), (257, 65536, 4096, True, 0),
+    (256, 4096, 4096, False, 0),                       # no full round
     (0, 4096, 4096, False, 0), (8, 262144, 8192, False, 0),   # 4 GB
 ])
 def test_route_by_sizes(m, rows, k, silu, kind):

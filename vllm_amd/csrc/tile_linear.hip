@@ -100,17 +100,25 @@ __global__ __launch_bounds__(TP_THREADS, 1) void tile_linear_kernel(
 }
 
 // 0: the library; else 128 or 256 weight rows a tile, for M rows by rows_w
-// weight rows. The share of its rounds over 256 CUs that a form keeps busy
-// decides: 256 where that is at least 95 % (for up to 128 rows of a plain
-// product in more than one round: 65536 x 4096 alone, 80 rows, 128 us, the
-// library 124), else 128 where that is one round. An activation, which saves a
-// launch and a pass, makes up for a third of one round, or a tenth of several.
-// us, this and the library: 28672 x 4096, 128 rows, 224 tiles of 128: 57.4 and
-// 57.2; 65536 x 4096, 128 rows, 512 tiles of 128: 136 and 125; 57344 x 4096
-// with the activation, 128 rows, 448 tiles: 118 and 102; 152064 x 3584, 256
-// rows, 594 tiles of 256: 288 and 259.
-int tile_form(int64_t M, int64_t rows_w, bool silu) {
-  if (M <= 64 || M > TI_ROWS) return 0;
+// weight rows of K.
+//
+// The share of its rounds over 256 CUs that a form keeps busy decides: 256
+// where that is at least 95 % (for up to 128 rows of a plain product in more
+// than one round: 65536 x 4096 alone, 80 rows, 128 us, the library 124), else
+// 128 where that is one round. An activation, which saves a launch and a pass,
+// makes up for a third of one round, or a tenth of several. us, this and the
+// library: 28672 x 4096, 128 rows, 224 tiles of 128: 57.4 and 57.2; 65536 x
+// 4096, 128 rows, 512 tiles of 128: 136 and 125; 57344 x 4096 with the
+// activation, 128 rows, 448 tiles: 118 and 102; 152064 x 3584, 256 rows, 594
+// tiles of 256: 288 and 259.
+//
+// Plain products whose K is at most eight times their rows write too much
+// beside what they read, and workgroups that end together wait for it. us, this
+// and the library: 65536 x 512, 256 rows 30.0 and 24.5, x 1024 39.7 and 37.9, x
+// 2048 73 and 76; 128256 x 256, 128 rows 30.6 and 26.2, x 1024 61.5 and 60.0,
+// 65 rows 54 and 62. An activation halves what is written.
+int tile_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
+  if (M <= 64 || M > TI_ROWS || (!silu && K <= 8 * M)) return 0;
   auto rounds = [&](int tile) { return (rows_w + tile * 256 - 1) / tile / 256; };
   auto busy = [&](int tile) {
     return (double)((rows_w + tile - 1) / tile) / (double)(rounds(tile) * 256);
@@ -147,7 +155,7 @@ int tile_linear_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
   if (rows_w <= 0 || rows_w % (silu ? 16 : 8) != 0 || K <= 0 ||
       K % TP_K != 0 || K >= (1 << 22) || (rows_w + 256) * K * 2 >= (1ll << 32))
     return 0;
-  return tile_form(M, rows_w, silu);
+  return tile_form(M, rows_w, K, silu);
 }
 
 // The product of x [M, K] and w [rows, K], both contiguous, into out [M, n],
