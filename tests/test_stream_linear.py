@@ -19,14 +19,14 @@ def _operands(m, n, k, dtype):
     return x, w * k ** -0.5
 
 
-def _check(out, expect, dtype):
+def _check(out, expect, dtype, k=0):
     # fp32 sums of exact products: what is left is the rounding of the
     # result (half a unit of the last of 7 stored bits in bf16, of 10 in
     # fp16: 2^-8 and 2^-11 of the value) and, near zero, of sums of terms
-    # of size 1 (K * 2^-24 at the very most, K up to 14336).
+    # of size 1 (K * 2^-24 at the very most, K up to 14336 where not given).
     unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     err = (out.float() - expect).abs() - expect.abs() * unit
-    assert err.max() <= 1e-3, err.max()
+    assert err.max() <= max(1e-3, k * 2.0 ** -24), err.max()
 
 
 # Row groups of 8, 16, 32 and 64 at both ends; columns that end within a
@@ -42,6 +42,20 @@ SHAPES = [(1, 8, 64), (8, 16, 128), (9, 2112, 7168), (16, 24, 192),
 TILES = [(65, 32752, 64), (96, 65536, 128), (128, 32768, 320),
          (129, 32752, 64), (161, 65472, 192), (200, 31744, 640),
          (255, 32768, 448), (256, 65536, 64), (70, 30720, 1024)]
+
+
+# The same where a plain product is not left to the library, and more tiles
+# than CUs.
+TILES += [(96, 32752, 1088), (200, 32752, 1664), (99, 131056, 832),
+          (130, 65520, 1088), (161, 131056, 1344), (70, 131056, 320)]
+# Weights that come to each form of stream_linear (plan() in the source), whole
+# and with K split: rows of weights that end within a tile, steps of K past
+# what a ring holds.
+FORMS = [(8, 2624), (8, 28672), (16, 832), (16, 3136), (16, 7168),
+         (1424, 7168), (4432, 832), (8288, 832), (4256, 14336), (4432, 8256),
+         (4432, 5184), (4256, 4160), (18160, 832), (8288, 7168),
+         (8288, 5184), (24848, 832), (24848, 1088), (8288, 18176),
+         (34016, 448), (34016, 1088)]
 
 
 @gpu
@@ -65,6 +79,23 @@ def test_linear_silu_and_mul(m, n, k, dtype):
     gate, up = (x.float() @ w.float().t()).chunk(2, -1)
     expect = torch.nn.functional.silu(gate) * up
     _check(hip_ops.linear_silu_and_mul(x, w), expect, dtype)
+
+
+@gpu
+@pytest.mark.parametrize("n,k", FORMS)
+@pytest.mark.parametrize("dtype,rows", [(torch.bfloat16, (8, 9, 32, 33)),
+                                        (torch.float16, (1, 16, 17, 64))])
+def test_forms(n, k, dtype, rows):
+    """Both ends of the row groups, with the activation and without."""
+    from vllm_amd.ops import hip_ops
+    for m in rows:
+        x, w = _operands(m, n, k, dtype)
+        expect = x.float() @ w.float().t()
+        _check(hip_ops.linear(x, w), expect, dtype, k)
+        if n % 16 == 0:
+            gate, up = expect.chunk(2, -1)
+            _check(hip_ops.linear_silu_and_mul(x, w),
+                   torch.nn.functional.silu(gate) * up, dtype, k)
 
 
 @gpu
@@ -150,6 +181,45 @@ def _form(m, rows, k, silu=False):
 ])
 def test_route_by_sizes(m, rows, k, silu, kind):
     assert _form(m, rows, k, silu)[0] == kind
+
+
+def _key(m, rows, k, silu):
+    """Which kernel: form, row groups, whether K is split; or tile, row form,
+    whether tiles take more than a round of the CUs."""
+    form = _form(m, rows, k, silu)
+    if form[0] == 1:
+        return ("stream", silu, form[1], form[4], form[5] > 1)
+    if form[0] == 2:
+        return ("tile", silu, form[1], m > 128, rows > form[1] * 256)
+    return None
+
+
+def _model_layers():
+    from vllm_amd.config import MODEL_PRESETS, get_model_spec
+    for name in MODEL_PRESETS:
+        s = get_model_spec(name)
+        h, hd = s.hidden_size, s.head_dim
+        for tp in (1, 2, 4, 8):
+            inter, kv = s.intermediate_size // tp, max(s.num_kv_heads // tp, 1)
+            heads = s.num_heads // tp
+            yield from (((heads + 2 * kv) * hd, h, False),
+                        (h, heads * hd, False), (h, inter, False),
+                        (2 * inter, h, False), (2 * inter, h, True),
+                        (s.vocab_size // tp, h, False))
+
+
+def test_shapes_reach_the_forms_of_models():
+    """Every kernel that a layer of a known model runs as, on 1 to 256 rows,
+    is one that the tests above run."""
+    edges = (1, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 256)
+    tested = {_key(m, n, k, silu) for n, k in FORMS for m in edges[:8]
+              for silu in (False, True) if not silu or n % 16 == 0}
+    tested |= {_key(m, n, k, silu) for m, n, k in TILES
+               for silu in (False, True)}
+    models = {_key(m, n, k, silu) for n, k, silu in _model_layers()
+              for m in edges if n > 0 and k > 0 and n % (16 if silu else 8) == 0}
+    assert len(models) > 30
+    assert models <= tested, sorted(models - tested, key=str)
 
 
 def test_gated_silu_calls_what_is_hooked():
