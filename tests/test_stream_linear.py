@@ -82,6 +82,23 @@ def test_linear_silu_and_mul(m, n, k, dtype):
 
 
 @gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(64, 65536, 64), (300, 65536, 64),
+                                   (1000, 8192, 64), (2048, 4096, 64),
+                                   (129, 50272, 192), (300, 24, 8192)])
+def test_library_race_takes_right_results_only(m, n, k, dtype):
+    """Shapes for which the library lists algorithms that compute something
+    else, among others; the call that tunes and those that follow."""
+    from vllm_amd.ops import hip_ops
+    x, w = _operands(m, n, k, dtype)
+    bias = torch.randn(n, dtype=dtype, device="cuda")
+    expect = x.float() @ w.float().t()
+    for _ in range(3):
+        _check(hip_ops.linear(x, w), expect, dtype)
+        _check(hip_ops.linear(x, w, bias), expect + bias.float(), dtype)
+
+
+@gpu
 @pytest.mark.parametrize("n,k", FORMS)
 @pytest.mark.parametrize("dtype,rows", [(torch.bfloat16, (8, 9, 32, 33)),
                                         (torch.float16, (1, 16, 17, 64))])
