@@ -247,7 +247,10 @@ def test_odd_places_take_plain_loads(hip, monkeypatch):
     (96, 4000, 1000, 32, 128, True),
     (8, 1000, 2000, 32, 128, True),
     (1, 1000, 8191, 32, 128, False),     # nothing to run beside
-    (256, 300, 500, 32, 128, False),     # a wave a row
+    (256, 300, 500, 32, 128, True),
+    (256, 128, 500, 32, 128, False),     # a wave a row
+    (512, 300, 500, 32, 128, False),     # a wave a row
+    (160, 128, 500, 32, 64, True),
     (8, 1000, 200, 72, 128, False),      # nine heads a KV head
     (8, 1000, 200, 32, 256, False),
     (8, 1000, 2000, 32, 64, True),
@@ -263,3 +266,46 @@ def test_rows_beside_portions(hip, rows, keys, new, heads, hd, mixed):
     names = [n for n, _ in hip._C.calls]
     assert names == (["mixed_attention"] if mixed else
                      ["paged_decode_attention", "prefill_attention"])
+
+
+@pytest.mark.parametrize("rows,keys,past,new,portions,window,fp8,mixed", [
+    (64, 2000, 0, 1000, 4, 0, False, True),
+    (64, 2000, 4000, 1000, 4, 0, False, False),   # tiles of one length
+    (64, 2000, 4000, 1000, 1, 0, False, True),    # of one portion
+    (64, 8000, 4000, 1000, 4, 0, False, True),    # their past is not known
+    (512, 2000, 4000, 1000, 4, 0, False, True),   # as much to read
+    (2, 2000, 0, 2000, 1, 0, False, True),
+    (2, 2000, 0, 2000, 1, 0, True, False),        # half the bytes
+    (3, 8000, 0, 4000, 1, 0, False, True),
+    (3, 8000, 0, 4000, 1, 128, False, False),     # the keys of a window
+])
+def test_rows_beside_portions_by_what_they_read(hip, rows, keys, past, new,
+                                                portions, window, fp8, mixed):
+    q = torch.empty(rows + new * portions, 32, 128, dtype=torch.bfloat16)
+    kv = torch.empty(2, 1, 8, 64, 128, dtype=torch.bfloat16)
+    if fp8:
+        kv = kv.to(torch.float8_e4m3fn)
+    lens = [keys] * rows + [past + new] * portions
+    starts = torch.tensor([0] + [1] * rows + [new] * portions).cumsum(0)
+    hip.attention_unified(
+        q, kv, torch.zeros(len(lens), 1, dtype=torch.int32),
+        starts.to(torch.int32), _lens(*lens), 0.1, num_decodes=rows,
+        max_seq_len=max(lens), max_query_len=new, max_decode_len=keys,
+        sliding_window=window)
+    names = [n for n, _ in hip._C.calls]
+    assert names == (["mixed_attention"] if mixed else
+                     ["paged_decode_attention", "prefill_attention"])
+
+
+def test_wave_rows_as_the_kernel_plans_them():
+    try:
+        from vllm_amd.ops import hip_ops
+    except (ImportError, OSError) as e:
+        pytest.skip(f"extension not built: {e}")
+    for units in (1, 1023, 1024, 1535, 1536, 4095, 4096):
+        for hd in (64, 128, 256):
+            for parts in (1, 2):
+                for span in (1, 128, 129, 512, 513):
+                    assert hip_ops._decode_waves(
+                        units, hd, parts, span) == hip_ops._C.decode_waves(
+                            units, hd, parts, span)

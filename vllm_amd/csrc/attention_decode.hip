@@ -15,6 +15,21 @@ __global__ __launch_bounds__(DEC_BLOCK, 2) void paged_decode_kernel(
                                          blockIdx.z, lds);
 }
 
+// Rows of a few steps leave three of a workgroup's four waves idle, and
+// starting and merging it costs more than its keys: from half the waves
+// that run at a time on, each takes a row of at most 128 keys of its own;
+// of up to 512 (the least that a captured step is told) where rows fill
+// the chip twice over. us, workgroup / wave a row, 32/8 heads of 128: 1024
+// rows x 1..32 keys 49 / 20, 33..64 56 / 35, 129..176 125 / 121, 512 377 /
+// 378; 128 x 1..128 11.1 / 9.3; 64 x 128 7.6 / 8.8, 512 x 1..512 104 / 106.
+// Heads of 256: 512 x 128 97.6 / 99.3, 1..128 49 / 45, 1..512 195 / 207.
+bool decode_waves(int64_t units, int64_t head_dim, int64_t num_parts,
+                  int64_t span) {
+  return num_parts == 1 &&
+         ((span <= 128 && units >= (head_dim == 64 ? 1536 : 1024)) ||
+          (span <= 512 && units >= 4096 && head_dim <= 128));
+}
+
 // Checks the operands of num_seqs decode rows and lays them out.
 DecodePlan plan_decode(const torch::Tensor& out, const torch::Tensor& q,
                        const torch::Tensor& kv_cache, int num_seqs,
@@ -54,19 +69,8 @@ DecodePlan plan_decode(const torch::Tensor& out, const torch::Tensor& q,
   const int part_len =
       (int)((span + (int64_t)num_parts * unit - 1) /
             ((int64_t)num_parts * unit)) * unit;
-  // Rows of a few steps leave three of a workgroup's four waves idle, and
-  // starting and merging it costs more than its keys: from half the waves
-  // that run at a time on, each takes a row of at most 128 keys of its own;
-  // of up to 512 (the least that a captured step is told) where rows fill
-  // the chip twice over. us, workgroup / wave a row, 32/8 heads of 128: 1024
-  // rows x 1..32 keys 49 / 20, 33..64 56 / 35, 129..176 125 / 121, 512 377 /
-  // 378; 128 x 1..128 11.1 / 9.3; 64 x 128 7.6 / 8.8, 512 x 1..512 104 / 106.
-  // Heads of 256: 512 x 128 97.6 / 99.3, 1..128 49 / 45, 1..512 195 / 207.
   const int64_t units = (int64_t)num_seqs * num_kv_heads;
-  const bool wave_rows =
-      num_parts == 1 &&
-      ((span <= 128 && units >= (head_dim == 64 ? 1536 : 1024)) ||
-       (span <= 512 && units >= 4096 && head_dim <= 128));
+  const bool wave_rows = decode_waves(units, head_dim, num_parts, span);
   torch::Tensor arrived;
   if (num_parts > 1) arrived = arrival_counters(q, units);
   return {num_parts, part_len, wave_rows, (float)scale * DEC_LOG2E, arrived};

@@ -34,6 +34,8 @@ void prefill_attention(torch::Tensor out, torch::Tensor q,
                        torch::Tensor query_start_loc, torch::Tensor seq_lens,
                        double scale, int64_t num_decodes,
                        int64_t max_query_len, int64_t sliding_window);
+bool decode_waves(int64_t units, int64_t head_dim, int64_t num_parts,
+                  int64_t span);
 void mixed_attention(torch::Tensor out, torch::Tensor q,
                      torch::Tensor kv_cache, torch::Tensor block_table,
                      torch::Tensor query_start_loc, torch::Tensor seq_lens,
@@ -211,6 +213,8 @@ TORCH_LIBRARY(vllm_amd, m) {
         "Tensor block_table, Tensor query_start_loc, Tensor seq_lens, "
         "float scale, int num_decodes, int max_query_len, "
         "int sliding_window) -> ()");
+  m.def("decode_waves(int units, int head_dim, int parts, int span) -> bool",
+        &vllm_amd::decode_waves);
   m.def("mixed_attention(Tensor(a!) out, Tensor q, Tensor kv_cache, "
         "Tensor block_table, Tensor query_start_loc, Tensor seq_lens, "
         "float scale, int num_decodes, int max_decode_len, "

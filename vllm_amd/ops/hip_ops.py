@@ -155,25 +155,49 @@ def rope_and_cache(positions, q, k, v, cos_sin_cache, rotary_dim, is_neox,
         reshape_and_cache(k, v, kv_cache, slot_mapping)
 
 
+def _decode_waves(units, head_dim, parts, span):
+    """Whether a wave takes a row of its own: plan_decode of
+    csrc/attention_decode.hip, for rows * KV heads units."""
+    return parts == 1 and (
+        (span <= 128 and units >= (1536 if head_dim == 64 else 1024))
+        or (span <= 512 and units >= 4096 and head_dim <= 128))
+
+
 def _attention_mixes(rows, reqs, tokens, heads, head_dim, kv_heads, parts,
-                     max_decode_len, max_seq_len, max_query_len):
+                     max_decode_len, max_seq_len, max_query_len,
+                     window=0, kv_bytes=2):
     """Whether decode rows and portions of prompts run in one launch
-    (csrc/attention_mixed.hip). Not short rows in numbers that take a wave
-    each, heads that one of the two kernels does not take, grids past 65535
-    units, nor rows that read less than a twentieth of the time that the
-    portions may take (5 TB/s against 0.8 PFLOP/s): there is nothing to run
-    beside them, and tiles are 1.5 % slower in the joint kernel (1 row x
-    1000 keys and 8191 tokens 651 and 661 us)."""
+    (csrc/attention_mixed.hip). Not rows that take a wave each (1024 x 64 keys
+    and 8 portions of 128 tokens 58 us in turn, 74 as workgroups in one
+    launch), heads that one of the two kernels does not take, nor grids past
+    65535 units. Nor rows that read (5 TB/s) less than a twentieth of the time
+    that the portions may take (0.8 PFLOP/s): they have hardly any effect (1
+    row x 1000 keys and 8000 tokens 587 us in turn, 588 in one launch). A
+    third where several portions come after more cached tokens than they are
+    long: their tiles are all of one length and fill the chip in step, which
+    rows among them disturb (4 portions of 1000 after 4000 beside 8 x 4000
+    keys 386 and 415 us, 16/2 heads 202 and 234; beside 64 x 2000, 8/8 heads,
+    215 and 181)."""
     if not 0 < rows < reqs or head_dim not in (64, 128):
         return False
     if heads % kv_heads or heads // kv_heads > 8:
         return False
-    if parts == 1 and max_decode_len <= 512 and rows * kv_heads >= 1024:
+    span = max_decode_len
+    if window > 0:
+        span = min(span, window + 31)
+    if _decode_waves(rows * kv_heads, head_dim, parts, span):
         return False
-    read_us = rows * max_decode_len * kv_heads * head_dim * 4 / 5e6
-    tile_us = (tokens - rows) * max_seq_len * heads * head_dim * 2 / 8e8
+    read_us = rows * span * kv_heads * head_dim * 2 * kv_bytes / 5e6
+    # (Cached tokens of portions are known only where the longest context is
+    # not a row's.)
+    alike = (reqs - rows > 1 and max_seq_len > max_decode_len
+             and max_seq_len >= 2 * max_query_len)
+    keys = max_seq_len - max_query_len / 2 if alike else max_seq_len / 2
+    if window > 0:
+        keys = min(keys, window)
+    tile_us = (tokens - rows) * keys * heads * head_dim * 4 / 8e8
     tiles = -(-max_query_len * (heads // kv_heads) // 128)
-    return (read_us * 20 >= tile_us
+    return (read_us * (3 if alike else 20) >= tile_us
             and tiles * (reqs - rows) + rows * parts < 65536)
 
 
@@ -230,7 +254,8 @@ def attention_unified(
             max_query_len = int((qsl[1:] - qsl[:-1]).max().item())
         if _attention_mixes(num_decodes, num_reqs, num_tokens, num_heads,
                             head_dim, kv_cache.shape[2], num_parts,
-                            max_decode_len, max_seq_len, max_query_len):
+                            max_decode_len, max_seq_len, max_query_len,
+                            sliding_window, kv_cache.element_size()):
             _C.mixed_attention(
                 out, q, kv_cache, block_table, query_start_loc, seq_lens,
                 scale, num_decodes, max_decode_len, max_query_len,
