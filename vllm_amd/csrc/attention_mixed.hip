@@ -19,16 +19,22 @@ constexpr int max_lds(int a, int b) { return a > b ? a : b; }
 // the last of each portion first, `rows` units (row, partition) pairs. Tiles
 // are spread evenly over the first `spread` units: over all where they are
 // at least two of three, otherwise so that they are two of three while they
-// last, as the last to start should be short. (One of two meets the order in
-// which workgroups are dealt to CUs: all tiles go to one half of them and
-// all rows to the other.)
+// last, as the last to start should be short.
+//
+// Workgroups of an XCD are dealt to its CUs four ways in turn, so work that
+// comes back every second or fourth unit meets on some CUs only: one tile of
+// two went to one half of them; short portions beside a long one leave units
+// without work, and every fourth was a tile (portions of 2000, 100 and 100 tokens
+// beside 8 x 4000 keys 129 us in turn, 147 in one launch, 91 now; 64 x 2000 with
+// a window of 512 62, 86, 50). So the units are turned by one place in each
+// group of four.
 //
 // 32/8 heads of 128, us one after the other and so: 96 rows x 100..4000
-// keys and portions of 400, 700 and 1001 tokens after 0 to 4096 341 -> 262
-// (one of two 320, runs of 256 tiles and 256 rows in turn 265); 200 rows x
-// 100..2000 and 2 of 100 and 200 tokens 176 -> 158; 16 rows x 100..300 and
-// 30 of 17..200 33.6 -> 28.7; 32/4 heads, 32 rows x 2000..4000 and 4 of
-// 1000..2000 162 -> 148 (runs of 256 in turn 183).
+// keys and portions of 400, 700 and 1001 tokens after 0 to 4096 311 -> 242;
+// 200 rows x 100..2000 and 2 of 100 and 200 tokens 154 -> 145; 16 rows x
+// 100..300 and 30 of 17..200 33.9 -> 29.1; 32/4 heads, 32 rows x 2000..4000
+// and 4 of 1000..2000 159 -> 133 (runs of 256 tiles and 256 rows in turn were
+// a fifth slower there).
 struct Mix { int tiles, rows, spread, num_prefills; };
 
 template <typename Tag, typename CTag, bool WHOLE, int HD>
@@ -40,9 +46,11 @@ __global__ __launch_bounds__(PF_BLOCK, 2) void mixed_attention_kernel(
   const auto before = [&](int n) {   // tiles among the first n units
     return (int)((int64_t)min(n, mix.spread) * mix.tiles / mix.spread);
   };
-  const int at = before(blockIdx.y);
-  const bool tile = before(blockIdx.y + 1) > at;
-  const int u = tile ? at : blockIdx.y - at;
+  int y = blockIdx.y;
+  if (y < ((mix.tiles + mix.rows) & ~3)) y = (y & ~3) | ((y + (y >> 2)) & 3);
+  const int at = before(y);
+  const bool tile = before(y + 1) > at;
+  const int u = tile ? at : y - at;
   if (tile)
     prefill_tile<Tag, CTag, HD>(p, kvh, d.num_seqs + u % mix.num_prefills,
                                 u / mix.num_prefills, lds);
