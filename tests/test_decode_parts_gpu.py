@@ -191,7 +191,7 @@ def test_captured_launches_share_counters():
 # More tiles than rows and fewer, one of each; a portion shorter than a
 # tile, after cached tokens; heads in groups of 1, 7 and 8; rows in one and
 # in several partitions; a window; an fp8 cache; a negative scale.
-@pytest.mark.parametrize("rows,new,past,hq,hkv,hd,window,dtype,cache,scale", [
+MIXED = [
     ([1000], [70], [0], 32, 8, 128, 0, torch.bfloat16, None, 0.09),
     ([0, 1, 129, 3000], [1, 300], [5, 64], 14, 2, 128, 0, torch.float16,
      None, 0.09),
@@ -200,7 +200,94 @@ def test_captured_launches_share_counters():
      torch.bfloat16, None, 0.09),
     ([700, 1500, 64], [200], [31], 8, 2, 128, 0, torch.bfloat16,
      torch.float8_e4m3fn, 0.09),
-])
+    ([300] * 37, [1000, 3, 129], [0, 900, 7], 8, 2, 64, 0, torch.bfloat16,
+     None, 0.1),
+]
+NAMES = "rows,new,past,hq,hkv,hd,window,dtype,cache,scale"
+
+
+def _step(rows, new, past, hq, hkv, hd, dtype, cache):
+    ctx = rows + [n + p for n, p in zip(new, past)]
+    _, kv, table, _, lens = _rows(ctx, hq, hkv, hd, dtype, cache or dtype)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(sum(ctx))
+    q = torch.randn(len(rows) + sum(new), hq, hd, device="cuda",
+                    generator=g).to(dtype)
+    qsl = torch.tensor([0] + [1] * len(rows) + new, device="cuda").cumsum(
+        0).to(torch.int32)
+    return q, kv, table, qsl, lens
+
+
+def _joint(q, kv, table, qsl, lens, rows, new, window, scale):
+    """mixed_attention, whatever the rule says of the sizes."""
+    from vllm_amd.ops import hip_ops
+    n, hq, hd = len(rows), q.shape[1], q.shape[2]
+    parts = hip_ops._decode_parts(n, kv.shape[2], max(rows), window)
+    tmp = [q.new_empty(n, hq, parts, w, dtype=torch.float32)
+           if parts > 1 else q.new_empty(0, dtype=torch.float32)
+           for w in (hd, 2)]
+    out = torch.empty_like(q)
+    hip_ops._C.mixed_attention(out, q, kv, table, qsl, lens, scale, n,
+                               max(rows), max(new), window, *tmp)
+    return out
+
+
+@pytest.mark.parametrize(NAMES, MIXED)
+def test_mixed_exact(rows, new, past, hq, hkv, hd, window, dtype, cache,
+                     scale):
+    """The joint launch against fp32: weights of portions and the result are
+    rounded to p bits (p = 8, 11), each off by 2^-p at most: 2^-p of the same
+    sums over |v|, and of the result once for their own sum and once for
+    itself."""
+    q, kv, table, qsl, lens = _step(rows, new, past, hq, hkv, hd, dtype,
+                                    cache)
+    out = _joint(q, kv, table, qsl, lens, rows, new, window, scale).float()
+    live = [i for i, c in enumerate(lens.tolist()) if c > 0]
+    starts = qsl.tolist()
+    take = torch.cat([torch.arange(starts[i], starts[i + 1]) for i in live])
+    lq = torch.tensor([0] + [starts[i + 1] - starts[i] for i in live],
+                      dtype=torch.int32, device="cuda").cumsum(0).int()
+
+    def exact(values):
+        return ref.attention_unified(
+            q[take].float(), values, table[live], lq, lens[live], scale,
+            num_decodes=len([i for i in live if i < len(rows)]),
+            sliding_window=window)
+
+    wide = kv.float()
+    expect, mag = exact(wide), exact(torch.stack([wide[0], wide[1].abs()]))
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    bound = eps * (mag + 2 * expect.abs()) + 2.0 ** -16
+    assert ((out[take] - expect).abs() <= bound).all()
+    dead = torch.ones(len(q), dtype=torch.bool)
+    dead[take] = False
+    assert (out[dead.cuda()] == 0).all()
+
+
+@torch.inference_mode()   # as the runner captures
+def test_mixed_replays():
+    case = MIXED[1]
+    q, kv, table, qsl, lens = _step(*case[:6], case[7], case[8])
+
+    def call():
+        return _joint(q, kv, table, qsl, lens, case[0], case[1], case[6],
+                      case[9])
+
+    expect = call()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for _ in range(4):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        beside = call()
+        torch.cuda.synchronize()
+        assert torch.equal(out, expect)
+        assert torch.equal(beside, expect)
+
+
+@pytest.mark.parametrize(NAMES, MIXED)
 def test_mixed(rows, new, past, hq, hkv, hd, window, dtype, cache, scale):
     """Rows and portions in one launch against each in its own: the same
     work by the same code, so the same but for the order in which the
