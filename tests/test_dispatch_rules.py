@@ -103,6 +103,9 @@ def test_decode_parts(hip, rows, kv, span, window, parts):
     (500, 1, 128, 2048, 0),    # below 4 rows an expert
     (512, 1, 128, 2048, 1),
     (1536, 8, 64, 7168, 2),
+    (383, 2, 16, 1024, 0),     # 16 x 4 tiles leave three quarters idle
+    (384, 2, 16, 1024, 1),
+    (192, 2, 16, 2048, 1),     # 16 x 8 tiles half of it
 ])
 def test_expert_form(hip, tokens, topk, E, H, form):
     """Where rows may meet in few experts the weights are not streamed

@@ -511,14 +511,21 @@ def mla_heads(q_nope, q_pe, w_uk, w_uv, kv_cache, block_table,
     return out
 
 
-# Form of the expert products by the average number of rows an expert
-# gets: below 24 weights are streamed past at most 64 rows, below 192 tiles
-# of 128 rows, from there 256 (in which an expert of at most 32 rows is
-# streamed as well). ms streamed / 128 / 256: 8 experts of 4096 x 14336, 12
-# rows 0.45 / 0.50 / 0.50, 32 rows 0.47 / 0.54 / 0.54, 128 rows 1.04 / 0.65 /
-# 0.66, 256 rows 1.92 / 1.01 / 0.95; 64 experts of 7168 x 2048, 16 rows 0.88 /
-# 0.88 / 0.88, 64 rows 1.51 / 1.07 / 1.07, 192 rows 2.96 / 1.54 / 1.30.
+# Form of the expert products by the average number of rows an expert gets:
+# below 24 weights are streamed past at most 64 rows, below 192 tiles of 128
+# rows, from there 256 (in which an expert of at most 32 rows is streamed as
+# well). ms streamed / 128 / 256, chosen evenly: 8 experts of 4096 x 14336, 12
+# rows 0.44 / 0.49 / 0.49, 32 rows 0.47 / 0.54 / 0.54 (0.61 / 0.53 / 0.53
+# where half of the tokens agree), 64 rows 0.76 / 0.57 / 0.57, 100 rows 0.94 /
+# 0.60 / 0.60; 64 experts of 7168 x 2048, 16 rows 0.87 / 0.86 / 0.87, 64 rows
+# 1.43 / 1.03 / 1.03.
+# Where one tile per expert leaves more than half of the chip idle, tiles are
+# worth it from 48 rows only: 16 experts of 1024 x 3584 without a gate, us
+# streamed / 128, 24 rows 70 / 82 (76 / 78 where half agree), 38 rows 76 / 82
+# (80 / 95), 50 rows 89 / 82 (85 / 94), 64 rows 96 / 63; 8 of 1024 x 2048, 32
+# rows 34 / 57, 48 rows 36 / 41, 64 rows 56 / 45.
 _MOE_TILES_FROM = 24
+_MOE_FEW_TILES_FROM = 48
 _MOE_WIDE_TILES_FROM = 192
 # The average says little where rows meet in few experts (equal prompts,
 # padded rows of a captured step): weights of an expert with more than 64
@@ -539,10 +546,10 @@ def _moe_form(tokens, total, E, H):
     expert) pairs of tokens rows of H, no pair twice."""
     if total >= _MOE_WIDE_TILES_FROM * E:
         return 2
-    if total >= _MOE_TILES_FROM * E:
+    chip = E * -(-H // 256) / _MOE_CHIP_TILES
+    if total >= (_MOE_TILES_FROM if chip >= 0.5 else _MOE_FEW_TILES_FROM) * E:
         return 1
-    return int(tokens > _MOE_STREAM_ROWS and total >= 4 * E
-               and E * -(-H // 256) >= _MOE_CHIP_TILES)
+    return int(tokens > _MOE_STREAM_ROWS and total >= 4 * E and chip >= 1)
 
 
 def _moe_hip_ok(hidden, w13, w2, activation):
