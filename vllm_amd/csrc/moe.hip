@@ -209,7 +209,12 @@ static int split_of_grid(int m_tiles, int n_blocks) {
 // fragments, as below, and so: 8 experts of 4096 x 14336, 2 a token, 1 token
 // 166 / 115, 4 409 / 330, 48 517 / 441 (6.4 TB/s), 90 592 / 457; 64 of 7168 x
 // 2048, 8 a token, 64 tokens 950 / 805; 128 of 2048 x 768 195 / 179.
-constexpr int SR_FILL = 128;   // workgroups that are enough
+// Workgroups that are enough (of the tiles that there may be; few of them
+// are empty). us with 128 and with 32 weight rows a workgroup: 16 experts of
+// 1024 x 3584 without a gate, second product in 128 and 512, 8 tokens of two
+// 47.3 and 42.1, in 136 and 544, 64 tokens 63.4 and 54.5; 8 of 1024 x 2048, first
+// product in 256 and 1024, 4 tokens 24.6 and 28.9.
+constexpr int SR_FILL = 192;
 
 template <typename Tag, int ACT, int NI>
 __launch_bounds__(THREADS, 1) __global__
