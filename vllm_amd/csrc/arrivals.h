@@ -4,7 +4,7 @@
 // Workgroups of a group run on different XCDs, whose L2s do not see each
 // other. Parts are written and read by agent-scope accesses, which go past
 // them; a release fence instead would write back all of L2 (2112 x 7168, 64
-// rows in three parts: 33 us with fences, 14.7 without).
+// rows in three parts: 33 us with fences, 14.3 without).
 #pragma once
 
 #include "common.h"

@@ -21,7 +21,12 @@
 //   - Values are read as lines that leave L2 first: each is needed once,
 //     and they no longer push out what other workgroups are about to read
 //     (keys cannot be: a load takes half a line of each row, the other half
-//     would be fetched again).
+//     would be fetched again). Rows that have most of their keys in common
+//     pay for it: 64 x 2000 keys, 1920 of them common, 32 heads ungrouped,
+//     147 -> 163 us, 128 x 16000, 15936 common, one KV head 83 -> 91, 256 x
+//     2000, 32/8 heads, 148 -> 151; with half in common there is a gain (256 x
+//     1000, 512 common, 113 -> 103). Asking each step whether a neighbour
+//     reads the same block gives those back and costs all others 2 to 5 %.
 //   - P stays at more than 16 bits: it is split in two 16-bit parts
 //     (p = hi + lo, error 2^-17) and multiplied twice; the matrix cores
 //     are idle here anyway. Sums and outputs are fp32. Results are as far
@@ -31,10 +36,10 @@
 // Against the vector-ALU form it replaced (16 lanes per token, dot
 // products reduced with shuffles), us per layer at 32 query and 8 KV
 // heads of 128:
-//   1 x 1000 keys 46 -> 8; 256 x 129..2176 keys 349 -> 203 (6.0 TB/s; 223
-//   with values read as everything else); 1024 x 129..176 keys 206 -> 111
-//   (119; 132 with the last 32 keys of a row read whole); 16 x 4096 keys 43
-//   (52); 64 x 4096..8192 keys, fp8 cache 371 -> 150 (159).
+//   1 x 1000 keys 46 -> 8; 256 x 129..2176 keys 349 -> 206 (5.9 TB/s; 225
+//   with values read as everything else); 1024 x 129..176 keys 206 -> 104
+//   (119; 132 with the last 32 keys of a row read whole); 16 x 4096 keys 45
+//   (51); 64 x 4096..8192 keys, fp8 cache 371 -> 144 (156).
 //
 // The KV cache layout [2, blocks, kv_heads, block_size=64, D] keeps each
 // (block, head) tile contiguous (16 KB at D=128).
@@ -87,8 +92,8 @@ DEVINL int dec_base(int ctx, int window) {
 // of its own, whole, for batches of short rows. A row of several partitions
 // (only where not WHOLE) leaves fp32 partials with their running maximum
 // (log2 domain) and sum; the last of its workgroups to arrive merges them.
-// (A second launch for that: 1 x 1000 keys 9.2 us, now 8.2; 4 x 8192 29.5,
-// now 25.9; 64 x 4096..8192 fp8 keys 156.2, now 156.0.)
+// (With a second launch for that: 1 x 1000 keys 9.4 us, now 7.8; 4 x 8192 32.4,
+// now 27.3.)
 template <typename CTag> struct DecodeArgs {
   short* out;            // [Tdec, Hq, D] (16-bit)
   float* tmp_out;        // [Tdec, Hq, parts, D]

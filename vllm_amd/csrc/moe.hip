@@ -50,8 +50,8 @@ constexpr int LDS_EXPERTS = 1024;   // whose counters fit LDS
 // prefix over the blocks cost 13 us (32 while a thread by itself filled up
 // its expert's last tile and read the blocks' counts one by one). Up to 2048
 // rows one workgroup does it all in one launch (48 rows on 8 experts: 6.5 ->
-// 4.1 us). Counters of more than 1024 experts
-// (LDS false) are in the scratch instead, one set per block all the same.
+// 3.6 us). Counters of more than 1024 experts (LDS false) are in the scratch
+// instead, one set per block all the same.
 constexpr int ALIGN_ROWS = 2048;   // rows per block
 
 // counts[e] -> off[e] = first row of expert e in tile order, and what the
@@ -207,7 +207,7 @@ static int split_of_grid(int m_tiles, int n_blocks) {
 // up rows for gated experts) a workgroup, or 32 where those are too few to
 // fill the chip; LDS is filled in whole lines that leave L2 first. us by
 // fragments, as below, and so: 8 experts of 4096 x 14336, 2 a token, 1 token
-// 166 / 115, 4 409 / 330, 48 517 / 441 (6.4 TB/s), 90 592 / 457; 64 of 7168 x
+// 166 / 115, 4 409 / 330, 48 517 / 435 (6.5 TB/s), 90 592 / 444; 64 of 7168 x
 // 2048, 8 a token, 64 tokens 950 / 805; 128 of 2048 x 768 195 / 179.
 // Workgroups that are enough (of the tiles that there may be; few of them
 // are empty). us with 128 and with 32 weight rows a workgroup: 16 experts of

@@ -19,20 +19,21 @@
 //    -> 45.7 us).
 //  * Enough workgroups of equal size (plan() below). Narrow layers split K
 //    over workgroups; the last one to arrive adds up the parts in their
-//    order (arrivals.h; 2112 x 7168, 64 rows: 14.7 us in three parts, 21.3
+//    order (arrivals.h; 2112 x 7168, 64 rows: 14.3 us in three parts, 21.3
 //    in one).
 //  * Weights leave L2 first (lds_fill16_once): read once, they would push
 //    out x, which every workgroup reads (7168 x 16384, 64 rows 58 -> 49 us).
 //
-// us on weights from HBM, tuned library products -> these, in a graph, where
-// split products clear their counters by a launch of 2 us (floor at 6 TB/s):
+// us on weights from HBM, tuned library products -> these, in a graph (in
+// brackets the weights' bytes at 6.6 TB/s, which streams of this kind reach on
+// average; the widest layer passes it):
 //                   1 row          8 rows         32 rows        64 rows
-//    4096 x 4096    10.5 ->  7.5   10.6 ->  7.8   11.8 -> 11.4   13.8 -> 13.8   (5.6)
-//    6144 x 4096    13.3 -> 10.9   14.5 -> 11.4   15.2 -> 15.1   17.9 -> 16.6   (8.4)
-//   28672 x 4096    51.7 -> 38.9   47.6 -> 39.3   48.3 -> 40.6   54.6 -> 44.5   (39)
-//    4096 x 14336   25.5 -> 21.3   25.7 -> 22.0   31.9 -> 27.9   37.6 -> 34.4   (20)
-//    2112 x 7168    12.2 ->  9.4   12.0 -> 11.6   15.8 -> 14.0   19.3 -> 16.7   (5.0)
-//  128256 x 4096     179 ->  158    176 ->  159    192 ->  169    201 ->  194   (175)
+//    4096 x 4096    10.4 ->  7.5   13.4 ->  7.6   11.7 ->  9.8   14.0 -> 12.4   (5.1)
+//    6144 x 4096    15.2 -> 11.1   14.2 -> 11.3   14.9 -> 14.8   18.2 -> 17.7   (7.6)
+//   28672 x 4096    48.9 -> 37.3   52.1 -> 37.4   52.4 -> 38.8   53.9 -> 42.9   (36)
+//    4096 x 14336   25.3 -> 20.3   25.4 -> 21.2   31.6 -> 25.0   37.5 -> 28.7   (18)
+//    2112 x 7168    12.2 ->  8.3   12.4 ->  9.8   16.0 -> 11.1   19.2 -> 14.3   (4.6)
+//  128256 x 4096     175 ->  154    174 ->  151    188 ->  163    199 ->  186   (159)
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
@@ -199,14 +200,14 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
 
 struct Plan { int form, parts; };
 
-// Form and parts of K by an estimate of the time, of which these bound it
-// (added as fourth powers): weights at 6 TB/s; all that enters workgroups, x
-// again in each, at 15 TB/s; what the fullest CU takes in at 60 GB/s, evened
-// out by two fifths where neighbours still run. A workgroup's start costs
-// 0.2 us of its CU, splitting K 1.5 us and the traffic of partial sums. The
-// constants are those that come closest to the best of all forms over 15
-// layers of 2112 x 7168 to 128256 x 4096 at 1 to 64 rows: 1.3 % from it on
-// average, 7 % at most.
+// Form and parts of K by an estimate of the time. Its terms (added as fourth
+// powers): weights at 6 TB/s; all that enters workgroups, x again in each, at
+// 15 TB/s; what the fullest CU takes in at 60 GB/s, evened out by two fifths
+// where neighbours still run. A workgroup's start costs 0.2 us of its CU,
+// splitting K 1.5 us and the traffic of partial sums. These are coefficients
+// of a fit and not bounds (the first is passed by a tenth): they come closest
+// to the best of all forms over 15 layers of 2112 x 7168 to 128256 x 4096 at 1
+// to 64 rows, 1.3 % from it on average, 7 % at most.
 Plan plan(int xg, int64_t rows_w, int K, bool silu) {
   Plan best{-1, 1};
   double least = 1e30;

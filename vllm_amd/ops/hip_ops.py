@@ -33,14 +33,14 @@ _DEC_FILL = 512
 def _decode_parts(rows, kv_heads, max_seq_len, sliding_window):
     """Into how many partitions a row's keys are split. Every partition
     costs a pass over its fp32 partials, so no more than fill the chip:
-    16 rows x 4096 keys (8 KV heads of 128) take 43.7 us in 4 partitions,
-    46.4 in 16. Partitions of more than 2048 keys leave ragged batches
+    16 rows x 4096 keys (8 KV heads of 128) take 45.3 us in 4 partitions,
+    50.3 in 16. Partitions of more than 2048 keys leave ragged batches
     waiting for their longest row; below that more partitions only
-    cost: 256 rows x 129..2176 keys take 203 us in 2, 239 in 9; 64 rows
-    x 4096..8192 fp8 keys 149 us in 4, 173 in 32. One or two rows are
-    hardly ragged and one workgroup a CU does: one x 8000 keys 15.4 us in
-    32, 19.4 in 63; two x 8000 19.5 in 16, 20.9 in 32 (24 x 500..3000
-    45.7 in 2, 37.7 in 3). At most 64, the lanes of the merging wave."""
+    cost: 256 rows x 129..2176 keys take 206 us in 2, 244 in 9; 64 rows
+    x 4096..8192 fp8 keys 144 us in 4, 172 in 32. For one or two rows one
+    workgroup a CU does: one x 8000 keys 13.2 us in 32, 16.3 in 63; two x
+    8000 16.9 in 16, 18.5 in 32 (24 x 500..3000 45.1 in 2, 40.4 in 3). At
+    most 64, the lanes of the merging wave."""
     span = max(max_seq_len, 1)
     if sliding_window > 0:
         span = min(span, sliding_window + 31)
