@@ -150,10 +150,10 @@ hipblasLtMatmulAlgo_t pick_algo(uint64_t key, hipblasLtMatmulDesc_t op_desc,
   HIP_CHECK(hipEventCreate(&ev1));
   auto time_algo = [&](const hipblasLtMatmulAlgo_t& algo,
                        int reps) -> float {
-    if (call(algo, out) != HIPBLAS_STATUS_SUCCESS)
+    if (call(algo, out, c.workspace) != HIPBLAS_STATUS_SUCCESS)
       return 1e30f;  // warm + probe
     HIP_CHECK(hipEventRecord(ev0, stream));
-    for (int r = 0; r < reps; ++r) (void)call(algo, out);
+    for (int r = 0; r < reps; ++r) (void)call(algo, out, c.workspace);
     HIP_CHECK(hipEventRecord(ev1, stream));
     HIP_CHECK(hipEventSynchronize(ev1));
     float ms = 1e30f;
@@ -176,12 +176,14 @@ hipblasLtMatmulAlgo_t pick_algo(uint64_t key, hipblasLtMatmulDesc_t op_desc,
             [](auto& x, auto& y) { return x.first < y.first; });
   HIP_CHECK(hipEventDestroy(ev0));
   HIP_CHECK(hipEventDestroy(ev1));
+  // (The workspace that all products share may be in use on another stream.)
+  const auto space = torch::empty({(int64_t)(kWorkspaceBytes / 4)},
+                                  out.options().dtype(torch::kFloat));
   auto run_clean = [&](int i, const torch::Tensor& to) {
-    torch::from_blob(c.workspace, {(int64_t)(kWorkspaceBytes / 4)},
-                     to.options().dtype(torch::kFloat))
-        .fill_(NAN);
+    space.fill_(NAN);
     to.fill_(NAN);
-    return call(results[i].algo, to) == HIPBLAS_STATUS_SUCCESS;
+    return call(results[i].algo, to, space.data_ptr()) ==
+           HIPBLAS_STATUS_SUCCESS;
   };
   const auto expect = torch::empty_like(out);
   int first = 0;
@@ -266,10 +268,10 @@ void run_matmul(torch::Tensor& out, const torch::Tensor& a,
                        (is_f32 ? (1ull << 63) : 0ull);
 
   auto call = [&](const hipblasLtMatmulAlgo_t& cand,
-                  const torch::Tensor& to) {
+                  const torch::Tensor& to, void* space) {
     return hipblasLtMatmul(
         c.handle, op_desc, &alpha, w.data_ptr(), lw, a.data_ptr(), la,
-        &beta, to.data_ptr(), lc, to.data_ptr(), lc, &cand, c.workspace,
+        &beta, to.data_ptr(), lc, to.data_ptr(), lc, &cand, space,
         kWorkspaceBytes, stream);
   };
   hipblasLtMatmulAlgo_t algo =
@@ -325,10 +327,10 @@ void run_matmul_fp8(torch::Tensor& out, const torch::Tensor& a,
   const uint64_t key = shape_key(M, N, K, false, false) ^ (1ull << 63);
 
   auto call = [&](const hipblasLtMatmulAlgo_t& cand,
-                  const torch::Tensor& to) {
+                  const torch::Tensor& to, void* space) {
     return hipblasLtMatmul(
         c.handle, op_desc, &alpha, w.data_ptr(), lw, a.data_ptr(), la,
-        &beta, to.data_ptr(), lc, to.data_ptr(), lc, &cand, c.workspace,
+        &beta, to.data_ptr(), lc, to.data_ptr(), lc, &cand, space,
         kWorkspaceBytes, stream);
   };
   hipblasLtMatmulAlgo_t algo =
