@@ -36,6 +36,7 @@ def _rows(ctx, hq, hkv, hd, dtype, cache_dtype):
     ([2000, 31, 640], 3, 1, 64, 0, torch.bfloat16, None),
     ([900, 64, 1500], 16, 2, 256, 0, torch.bfloat16, None),
     ([3000, 100, 500], 8, 8, 128, 300, torch.bfloat16, None),
+    ([4100, 1030], 16, 2, 256, 0, torch.float16, None),   # merged in two runs
     ([2176 - 7 * i for i in range(256)], 8, 2, 128, 0, torch.bfloat16, None),
     # More counters than lines, and than a stream's set holds.
     ([2100 + i if i % 9 == 0 else i % 150 for i in range(300)], 8, 4, 64, 0,

@@ -478,13 +478,23 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
     for (int e = e0; e < group * HD; e += DEC_BLOCK * 4) {
       const float* w = w_lds + e / HD * MAX_PARTS;
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int p0 = 0; p0 < used; p0 += AT_ONCE) {
+        // Reads past the last partition repeat it: with a branch each waits
+        // for the one before (16/2 heads of 256, 3 x 2916 keys 19.5 us, now
+        // 15.4).
+        f32x4 v[AT_ONCE];
+        if (e == e0 && p0 == 0) {
 #pragma unroll
-      for (int p = 0; p < AT_ONCE; ++p)
-        if (p < used) acc += (e == e0 ? first[p] : part_get(part_of(e, p))) *
-                             w[p];
-#pragma unroll 4
-      for (int p = AT_ONCE; p < used; ++p)
-        acc += part_get(part_of(e, p)) * w[p];
+          for (int i = 0; i < AT_ONCE; ++i) v[i] = first[i];
+        } else {
+#pragma unroll
+          for (int i = 0; i < AT_ONCE; ++i)
+            v[i] = part_get(part_of(e, min(p0 + i, used - 1)));
+        }
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i)
+          if (p0 + i < used) acc += v[i] * w[p0 + i];
+      }
       store4(e / HD, e % HD, acc);
     }
   }
