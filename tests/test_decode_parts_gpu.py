@@ -66,6 +66,29 @@ def test_merge(ctx, hq, hkv, hd, window, dtype, cache):
                                atol=2.0 ** -9)
 
 
+# A key's halves lie on neighbouring lanes where its row has 128 B or more:
+# every row size, with all of the columns that a group may have and with one.
+@pytest.mark.parametrize("group", [1, 8])
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("cache", [None, torch.float8_e4m3fn])
+@pytest.mark.parametrize("n", [5, 600])   # rows in parts, and a wave each
+def test_key_rows_by_halves(group, hd, cache, n):
+    from vllm_amd.ops import hip_ops
+    ctx = [(1, 2, 31, 33, 100)[i % 5] for i in range(n)]
+    if n == 5:
+        ctx[2:] = [700, 65, 1999]
+    q, kv, table, qsl, lens = _rows(ctx, 2 * group, 2, hd, torch.bfloat16,
+                                    cache or torch.bfloat16)
+    out = hip_ops.attention_unified(
+        q, kv, table, qsl, lens, hd ** -0.5, num_decodes=n,
+        max_seq_len=max(ctx))
+    expect = ref.attention_unified(q.float(), kv.float(), table, qsl, lens,
+                                   hd ** -0.5, num_decodes=n)
+    # The output's own rounding, as above.
+    torch.testing.assert_close(out.float(), expect, rtol=2.0 ** -8,
+                               atol=2.0 ** -9)
+
+
 @torch.inference_mode()   # as the runner captures
 def test_replays_and_streams():
     """Counters are left zero: by replays, by eager calls beside them and by

@@ -11,22 +11,28 @@
 //     current ones are free.
 //   - Scores are S^T = K Q^T on the matrix cores: a K row goes from HBM
 //     straight into the A fragment (16 B per lane), the query heads of
-//     the group are the 16 columns. No cross-lane sum per key and head,
+//     the group are the columns. No long cross-lane sum per key and head,
 //     which is what the vector-ALU form of this kernel spent its time on.
+//   - A group has at most 8 of the 16 columns. The other 8 hold the second
+//     half of the queries' columns, and two neighbouring rows of the
+//     fragment the halves of one key: the same products, but a load takes
+//     whole lines of 8 keys instead of half lines of 16, and a score is the
+//     sum of two lanes (one rotation). us on caches from HBM: 256 x
+//     129..2176 keys 210 -> 203, 64 x 4096..8192, fp8 cache 147 -> 144, 64 x
+//     100..4000, 28/4 heads 63 -> 58, 64 x 1000..4000, 16/4 heads of 256 126
+//     -> 119, 1 x 1000 8.7 -> 8.1; by quarters of a group of 4 no faster.
 //   - O^T = V^T P^T: V passes through this wave's own LDS slice to be
 //     transposed on the read. The lane that holds the scores of keys
 //     (4g..4g+3, 16+4g..) holds exactly the P^T fragment of those keys
 //     when the contraction runs over keys in that order, so P never
 //     moves between lanes.
-//   - Values are read as lines that leave L2 first: each is needed once,
-//     and they no longer push out what other workgroups are about to read
-//     (keys cannot be: a load takes half a line of each row, the other half
-//     would be fetched again). Rows that have most of their keys in common
-//     pay for it: 64 x 2000 keys, 1920 of them common, 32 heads ungrouped,
-//     147 -> 163 us, 128 x 16000, 15936 common, one KV head 83 -> 91, 256 x
-//     2000, 32/8 heads, 148 -> 151; with half in common there is a gain (256 x
-//     1000, 512 common, 113 -> 103). Asking each step whether a neighbour
-//     reads the same block gives those back and costs all others 2 to 5 %.
+//   - Keys and values are read as lines that leave L2 first: each is needed
+//     once, and they no longer push out what other workgroups are about to
+//     read. (Rows that have most of their keys in common: 64 x 2000 keys, 1920
+//     of them common, 32 heads ungrouped, 135 us; half lines of keys, which had
+//     to stay in L2 for the other half, 164, and nothing marked 147.) Where a
+//     wave is a row of few keys, keys are not marked: what a step holds past
+//     the row's end repeats its last key (200 x 1..60 keys 9.8 us, marked 10.2).
 //   - P stays at more than 16 bits: it is split in two 16-bit parts
 //     (p = hi + lo, error 2^-17) and multiplied twice; the matrix cores
 //     are idle here anyway. Sums and outputs are fp32. Results are as far
@@ -36,10 +42,9 @@
 // Against the vector-ALU form it replaced (16 lanes per token, dot
 // products reduced with shuffles), us per layer at 32 query and 8 KV
 // heads of 128:
-//   1 x 1000 keys 46 -> 8; 256 x 129..2176 keys 349 -> 206 (5.9 TB/s; 225
-//   with values read as everything else); 1024 x 129..176 keys 206 -> 104
-//   (119; 132 with the last 32 keys of a row read whole); 16 x 4096 keys 45
-//   (51); 64 x 4096..8192 keys, fp8 cache 371 -> 144 (156).
+//   1 x 1000 keys 46 -> 8; 256 x 129..2176 keys 349 -> 203 (6.0 TB/s);
+//   1024 x 129..176 keys 206 -> 107 (132 with the last 32 keys of a row read
+//   whole); 16 x 4096 keys 47; 64 x 4096..8192 keys, fp8 cache 371 -> 144.
 //
 // The KV cache layout [2, blocks, kv_heads, block_size=64, D] keeps each
 // (block, head) tile contiguous (16 KB at D=128).
@@ -80,6 +85,12 @@ template <typename CTag, int HD>
 constexpr int dec_keys =
     HD == 256 && sizeof(typename CacheTraits<CTag>::elem) == 2 ? 16
                                                                : DEC_KEYS;
+
+// Parts of a key row that lie on neighbouring lanes: one load of 16 / S rows
+// then takes whole lines of 128 B. (A row of 64 B is taken whole as it is.)
+template <typename CTag, int HD>
+constexpr int dec_split =
+    HD * sizeof(typename CacheTraits<CTag>::elem) >= 128 ? 2 : 1;
 
 // First key this row attends, rounded down so that a wave's 32 keys
 // never leave a cache block.
@@ -130,7 +141,12 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
   constexpr int KEYS = dec_keys<CTag, HD>;
   constexpr int KT = KEYS / 16;                   // score tiles
   constexpr int KF = HD / 32;                     // MFMA steps over D
-  constexpr int KN = HD * (int)sizeof(elem) / 64; // 16 B K loads per row
+  constexpr int S = dec_split<CTag, HD>;
+  static_assert(MAX_GROUP * S <= 16);
+  constexpr int NT = KT * S;                      // loaded tiles of 16 / S keys
+  constexpr int KN = HD * (int)sizeof(elem) / 64 / S;   // 16 B K loads of one
+  constexpr int QF = KF / S;                      // fragments of the queries
+  constexpr int KR = 4 / S;                       // keys of a lane in a tile
   constexpr int VN = KEYS * HD / EPV / WAVE_SIZE;
   constexpr int DS = HD / 16;                     // output column tiles
   constexpr int V_BYTES = KEYS * HD * 2;          // per wave
@@ -174,18 +190,20 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
 
   char* v_lds = lds + wave * V_BYTES;
 
-  // B fragments of the queries: column l16 is a head of the group, the
-  // others repeat head 0 and are never written out.
-  s16x8 qf[KF];
+  // B fragments of the queries: column h + 16 / S * part is that part of the
+  // columns of head h of the group (of head 0 where the group ends before).
+  const int part_q = l16 / (16 / S);
+  s16x8 qf[QF];
   {
+    const int h = l16 % (16 / S);
     const short* qb = a.q + (int64_t)seq * a.q_stride +
-                      (int64_t)(hq0 + (l16 < group ? l16 : 0)) * HD;
+                      (int64_t)(hq0 + (h < group ? h : 0)) * HD;
 #pragma unroll
-    for (int kk = 0; kk < KF; ++kk) {
-      // With an fp8 cache a 16 B load is two fragments' worth of one
-      // row, so the dims of a step are interleaved differently.
-      const int d = FP8 ? (kk >> 1) * 64 + l4 * 16 + (kk & 1) * 8
-                        : kk * 32 + l4 * 8;
+    for (int kk = 0; kk < QF; ++kk) {
+      // With an fp8 cache a 16 B load is two fragments' worth of one row.
+      constexpr int PER = FP8 ? 2 : 1;
+      const int d =
+          ((kk / PER * 4 + l4) * S + part_q) * EPV + kk % PER * 8;
       qf[kk] = *reinterpret_cast<const s16x8*>(qb + d);
     }
   }
@@ -197,18 +215,26 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
                (64 * HD) +
            (key0 & 63) * HD;
   };
-  i32x4 kr[KT][KN], vr[VN];
+  // Row l16 of tile t is part l16 % S of key k_row(t): a lane ends up with
+  // the scores of keys 16 * T + 4 * l4 + 0..3 however they are loaded.
+  auto k_row = [&](int t) {
+    const int p = l16 / S;
+    return t / S * 16 + p / KR * 4 + t % S * KR + p % KR;
+  };
+  i32x4 kr[NT][KN], vr[VN];
   // Rows of a step that the row does not attend repeat the nearest one it
   // does: they cost no bytes.
   auto load_k = [&](const elem* tile, int key0) {
     const int lo = t_lo - key0, hi = t_end - 1 - key0;
 #pragma unroll
-    for (int s = 0; s < KT; ++s) {
-      const int r = min(max(s * 16 + l16, lo), hi);
+    for (int t = 0; t < NT; ++t) {
+      const int r = min(max(k_row(t), lo), hi);
 #pragma unroll
-      for (int i = 0; i < KN; ++i)
-        kr[s][i] = *reinterpret_cast<const i32x4*>(
-            tile + r * HD + (i * 4 + l4) * EPV);
+      for (int i = 0; i < KN; ++i) {
+        const i32x4* at = reinterpret_cast<const i32x4*>(
+            tile + r * HD + ((i * 4 + l4) * S + l16 % S) * EPV);
+        kr[t][i] = WPR > 1 ? __builtin_nontemporal_load(at) : *at;
+      }
     }
   };
   auto load_v = [&](const elem* tile, int key0) {
@@ -238,10 +264,10 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
     // ---- S^T: rows are keys, columns heads -----------------------------
     f32x4 s[KT];
 #pragma unroll
-    for (int t = 0; t < KT; ++t) {
-      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT; ++t) {
+      f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kk = 0; kk < KF; ++kk) {
+      for (int kk = 0; kk < QF; ++kk) {
         s16x8 f;
         if constexpr (FP8) {
           const i32x4 r = kr[t][kk >> 1];
@@ -251,7 +277,15 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
         } else {
           f = __builtin_bit_cast(s16x8, kr[t][kk]);
         }
-        s[t] = mfma16<Tag>(f, qf[kk], s[t]);
+        c = mfma16<Tag>(f, qf[kk], c);
+      }
+      // Of each key the part that met its own columns; then the others'.
+#pragma unroll
+      for (int j = 0; j < KR; ++j) {
+        float y = c[j * S];
+        if constexpr (S == 2) y = part_q == 0 ? y : c[j * S + 1];
+        if constexpr (S == 2) y += row_ror<8>(y);
+        s[t / S][t % S * KR + j] = y;
       }
     }
     if constexpr (NEXT) load_k(next_tile, key0 + STRIDE);

@@ -346,6 +346,13 @@ DEVINL float wave_reduce_max(float v) {
   return v;
 }
 
+// The value of the lane N before this one in its group of 16, round it.
+template <int N> DEVINL float row_ror(float v) {
+  const int b = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(b, b, 0x120 + N, 0xf, 0xf, false));
+}
+
 // Reduce within 16-lane groups (used for MFMA row reductions).
 DEVINL float group16_reduce_max(float v) {
 #pragma unroll
