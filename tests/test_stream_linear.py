@@ -1,4 +1,4 @@
-"""Linear layers on few rows (csrc/stream_linear.hip) and on up to 256
+"""Linear layers on few rows (csrc/stream_linear.hip) and on up to 1024
 (csrc/tile_linear.hip): sizes at the edges of their forms, parts and
 epilogues against fp32 products of the same operands."""
 
@@ -48,6 +48,9 @@ TILES = [(65, 32752, 64), (96, 65536, 128), (128, 32768, 320),
 # than CUs.
 TILES += [(96, 32752, 1088), (200, 32752, 1664), (99, 131056, 832),
           (130, 65520, 1088), (161, 131056, 1344), (70, 131056, 320)]
+# Tiles of 64 weight rows, and of 256 that K is split over (with the
+# activation whole in one launch).
+TILES += [(66, 10688, 1664), (140, 10688, 1664), (66, 10944, 5120)]
 # Weights that come to each form of stream_linear (plan() in the source), whole
 # and with K split: rows of weights that end within a tile, steps of K past
 # what a ring holds.
@@ -223,6 +226,61 @@ def _model_layers():
                         (h, heads * hd, False), (h, inter, False),
                         (2 * inter, h, False), (2 * inter, h, True),
                         (s.vocab_size // tp, h, False))
+
+
+# K split over tiles, or whole in one round that is not full: 64, 128 and 256
+# weight rows a tile on 128 and 256 rows, and several tiles of rows; ragged rows
+# and columns, parts that are not alike, fewer stages than LDS holds.
+SPLIT = [(65, 2104, 7168, 64), (128, 3072, 8256, 64), (200, 2560, 6912, 64),
+         (96, 4088, 14336, 128), (128, 16384, 2048, 64), (250, 4096, 14336, 128),
+         (128, 18432, 7168, 256), (129, 24568, 1664, 128),
+         (256, 7160, 16384, 256), (257, 2112, 7168, 128), (700, 3584, 18944, 256),
+         (1023, 4096, 14336, 256), (600, 1536, 6208, 128)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k,cols", SPLIT)
+def test_tiles_in_parts(m, n, k, cols, dtype):
+    from vllm_amd.ops import hip_ops
+    kind, tile, parts = _form(m, n, k)
+    assert (kind, tile) == (2, cols) and (parts > 1 or n >= 16384)
+    x, w = _operands(m, n, k, dtype)
+    # What is read is written first: scratch that holds NaN.
+    junk = torch.full((64 << 20,), float("nan"), device="cuda")
+    del junk
+    out = hip_ops.linear(x, w)
+    _check(out, x.float() @ w.float().t(), dtype, k)
+    assert torch.equal(out, hip_ops.linear(x, w))
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_tiles_in_parts_replayed():
+    from vllm_amd.ops import hip_ops
+    x, w = _operands(130, 4096, 7168, torch.bfloat16)
+    eager = hip_ops.linear(x, w)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = hip_ops.linear(x, w)
+    for _ in range(4):
+        out.zero_()
+        graph.replay()
+        beside = hip_ops.linear(x, w)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager) and torch.equal(beside, eager)
+
+
+@pytest.mark.parametrize("m,n,k,form", [
+    (128, 4096, 5056, 0), (128, 4096, 5120, 2), (128, 1528, 7168, 0),
+    (129, 4096, 6080, 0), (129, 4096, 6144, 2), (1024, 4096, 10816, 0),
+    (1024, 4096, 10944, 2), (1025, 4096, 14336, 0), (1024, 5888, 28672, 0),
+    (128, 36864, 7168, 0), (160, 24576, 1280, 0), (160, 24576, 1344, 2),
+    (300, 24576, 5120, 0), (64, 4096, 14336, 1)])
+def test_route_of_split_tiles(m, n, k, form):
+    """Both sides of the lines in by_estimate (csrc/tile_linear.hip)."""
+    assert _form(m, n, k)[0] == form
 
 
 def test_shapes_reach_the_forms_of_models():

@@ -43,6 +43,7 @@
 
 #include "arrivals.h"
 #include "stream_product.h"
+#include "tile_linear.h"
 
 namespace vllm_amd {
 
@@ -51,7 +52,6 @@ torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
                         c10::optional<torch::Tensor> bias);
 torch::Tensor silu_and_mul(torch::Tensor x);
 // tile_linear.hip
-int tile_linear_form(int64_t M, int64_t rows_w, int64_t K, bool silu);
 bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
                  const torch::Tensor& w, bool silu);
 
@@ -341,8 +341,8 @@ bool stream_linear_takes(const torch::Tensor& x, const torch::Tensor& w,
 
 // What a product of these sizes runs as, for 16-bit operands that begin on
 // 16 B: {0} the library, {1, 16-row groups of weights, waves, ring steps,
-// 8-row groups of x, parts of K} stream_linear, {2, weight rows of a tile}
-// tile_linear.
+// 8-row groups of x, parts of K} stream_linear, {2, weight rows of a tile,
+// parts of K} tile_linear.
 std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
                                  bool silu) {
   const int64_t n = silu ? weight_rows / 2 : weight_rows;
@@ -352,8 +352,9 @@ std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
     const Form f = SL_FORMS[p.form];
     return {1, f.ni, f.wv, f.d, xg, p.parts};
   }
-  const int tile = tile_linear_form(rows, weight_rows, k, silu);
-  return tile == 0 ? std::vector<int64_t>{0} : std::vector<int64_t>{2, tile};
+  const TileForm tile = tile_linear_form(rows, weight_rows, k, silu);
+  if (tile.cols == 0) return {0};
+  return {2, tile.cols, tile.parts};
 }
 
 // x, w and bias as stream_linear_takes and lt_linear have checked them.

@@ -1,21 +1,33 @@
-// Linear layers on 65 to 256 rows, where one workgroup holds all rows of a
-// tile of columns (gfx950): out[M, N] = x[M, K] @ w[N, K]^T, and the same
+// Linear layers on 65 to 1024 rows, by tiles of all rows or of 256 of them
+// (gfx950): out[M, N] = x[M, K] @ w[N, K]^T, and for up to 256 rows the same
 // with silu(gate) * up of two halves of w as the epilogue.
 //
-// Between bound by the weights' way from HBM and by the matrix cores
-// (tile_product.h). Weights are read by one workgroup only and leave L2 first;
-// x stays. Nothing splits K here: partial sums of so many rows cost what the
-// split gains. So a layer must have nearly as many tiles as CUs run, or a
-// multiple of that, to be ahead of the tuned library (tile_form below).
+// Between bound by the weights' way from HBM and by what a CU takes in: rows of
+// x come from L2, but behind weights that are still under way, and a CU keeps
+// about 64 KB under way, so both together come at 50 to 60 GB/s a CU (125 where
+// nothing comes from HBM).
+//
+//  * Weights that one workgroup reads leave L2 first; x stays.
+//  * Workgroups begin at different stages of K, those that share weights at
+//    the same one: rows whose stride is a power of two meet on few channels
+//    otherwise. A window of some 60 stages, so that x stays in L2. 128 rows of
+//    weights alone at K = 16384 5.4 -> 7.0 TB/s; 28672 x 4096 with the
+//    activation, 128 rows 57 -> 52 us.
+//  * Layers with few tiles split K over workgroups until about one a CU runs,
+//    if K is long enough for the partial sums not to cost what that gains
+//    (by_estimate below); a second launch adds them.
 // us, library (and activation) -> this, weights from HBM:
-//   28672 x 4096 with the activation, 80 rows 59 -> 47, 256 rows 73 -> 61;
-//   22016 x 4096 with it, 192 rows 60 -> 54, 256 rows 64 -> 57; 129280 x 7168,
-//   80 rows 345 -> 313, 256 rows 405 -> 385; 128256 x 4096, 256 rows 275 -> 251;
-//   32000 x 4096, 80 rows 59 -> 52, 192 rows 67 -> 63.
+//   28672 x 4096 with the activation, 80 rows 59 -> 46, 256 rows 84 -> 66;
+//   22016 x 4096 with it, 192 rows 60 -> 54, 256 rows 64 -> 57; 128256 x 4096,
+//   128 rows 260 -> 176, 256 rows 289 -> 229; 4096 x 14336, 128 rows 52 -> 34,
+//   256 rows 65 -> 45, 512 rows 95 -> 69.
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
 
+#include <cmath>
+
+#include "tile_linear.h"
 #include "tile_product.h"
 
 namespace vllm_amd {
@@ -25,32 +37,51 @@ namespace {
 constexpr int TI_ROWS = 256;
 
 // N: columns of out. SILU: w has 2N rows, gate then up; a wave's gate rows,
-// then the up rows of the same columns.
-template <typename Tag, bool SILU, int WGM, int NI, int MI, int PA, int PW>
+// then the up rows of the same columns. ONCE: one workgroup reads a weight.
+// parts > 1 (not SILU): K is split, and the sums of a part go to `sums` in
+// blocks of 32 x 32: [parts][row blocks][column blocks][4][lane].
+template <typename Tag, bool SILU, bool ONCE, int WGM, int NI, int MI, int PA,
+          int PW>
 __global__ __launch_bounds__(TP_THREADS, 1) void tile_linear_kernel(
     short* __restrict__ out, const short* __restrict__ x,
     const short* __restrict__ w, const int M, const int N, const int K,
-    const int tiles) {
+    const int m_tiles, const int n_tiles, const int parts,
+    f32x4* __restrict__ sums) {
   using P = TileProduct<Tag, WGM, NI, MI, PA, PW>;
   __shared__ __align__(16) char lds[P::LDS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
   const int l32 = lane & 31;
   const int half = lane >> 5;
-  constexpr int NO = SILU ? NI / 2 : NI;
-  // Each XCD (workgroups go round them) takes a run of tiles.
-  const int run = (tiles + 7) / 8;
-  const int tile = blockIdx.x % 8 * run + blockIdx.x / 8;
-  if (blockIdx.x / 8 >= run || tile >= tiles) return;
-  const int n0 = tile * (P::TN / (SILU ? 2 : 1));
+  constexpr int H = SILU ? 2 : 1;
+  constexpr int NO = NI / H;
+  // Each XCD (workgroups go round them) takes a run of tiles; those beside
+  // each other have weights in common, then columns of K.
+  const int tiles = m_tiles * n_tiles, jobs = tiles * parts;
+  const int run = (jobs + 7) / 8;
+  const int xcd = blockIdx.x % 8, nth = blockIdx.x / 8;
+  const int job = xcd * run + nth;
+  if (nth >= run || job >= jobs) return;
+  const int part = job / tiles, tile = job % tiles;
+  const int m0 = tile % m_tiles * P::TM;
+  const int n0 = tile / m_tiles * (P::TN / H);
+  const int rows = min(M - m0, P::TM);
+  const int s0 = K / TP_K * part / parts;
+  const int steps = K / TP_K * (part + 1) / parts - s0;
+  const short* xt = x + (int64_t)m0 * K;
   const short* wt = w + (int64_t)n0 * K;
+  const int turn = (nth / m_tiles + xcd * 4) % steps;
+  auto stage = [&](int s) {
+    s += turn;
+    return (s0 + (s >= steps ? s - steps : s)) * TP_K;
+  };
 
   // Byte places of this lane's pieces; rows past the end repeat the last.
   uint32_t ap[P::FA], wp[P::FW];
 #pragma unroll
   for (int i = 0; i < P::FA; ++i) {
     const int r = (wave * P::FA + i) * 8 + (lane >> 3);
-    ap[i] = (uint32_t)min(r, M - 1) * (uint32_t)(K * 2) +
+    ap[i] = (uint32_t)min(r, rows - 1) * (uint32_t)(K * 2) +
             ((lane & 7) ^ tp_swap(r)) * 16;
   }
 #pragma unroll
@@ -66,19 +97,39 @@ __global__ __launch_bounds__(TP_THREADS, 1) void tile_linear_kernel(
             ((lane & 7) ^ tp_swap(r)) * 16;
   }
   P::run(
-      lds, K / TP_K, M,
-      [&](int s, int i, char* dst) { lds_fill16(x + s * TP_K, ap[i], dst); },
+      lds, steps, rows,
+      [&](int s, int i, char* dst) { lds_fill16(xt + stage(s), ap[i], dst); },
       [&](int s, int i, char* dst) {
-        lds_fill16_once(wt + s * TP_K, wp[i], dst);
+        if constexpr (ONCE) lds_fill16_once(wt + stage(s), wp[i], dst);
+        else lds_fill16(wt + stage(s), wp[i], dst);
       },
       [&](auto n, auto& acc) {
         constexpr int J = decltype(n)::value;
         const int wm = wave / P::WGN, wn = wave % P::WGN;
+        if (!SILU && parts > 1) {
+          const int cols = n_tiles * (P::TN / 32);
+#pragma unroll
+          for (int j = 0; j < J; ++j) {
+            const int rb = m0 / 32 + j * WGM + wm;
+            f32x4* to = sums + lane +
+                        (((int64_t)part * m_tiles * (P::TM / 32) + rb) * cols +
+                         n0 / 32 + wn * NI) *
+                            256;
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+              for (int b = 0; b < 4; ++b)
+                to[i * 256 + b * 64] =
+                    f32x4{acc[i][j][b * 4], acc[i][j][b * 4 + 1],
+                          acc[i][j][b * 4 + 2], acc[i][j][b * 4 + 3]};
+          }
+          return;
+        }
 #pragma unroll
         for (int j = 0; j < J; ++j) {
           const int row = (j * WGM + wm) * 32 + l32;
-          if (row >= M) continue;
-          short* o = out + (int64_t)row * N;
+          if (row >= rows) continue;
+          short* o = out + (int64_t)(m0 + row) * N;
 #pragma unroll
           for (int i = 0; i < NO; ++i) {
             f32x16 v = acc[i][j];
@@ -99,8 +150,114 @@ __global__ __launch_bounds__(TP_THREADS, 1) void tile_linear_kernel(
       });
 }
 
-// 0: the library; else 128 or 256 weight rows a tile, for M rows by rows_w
-// weight rows of K.
+// The parts of a product with K split, added in their order: half a block of
+// 32 x 32 a wave, eight parts on their way at once. (The last workgroup of a
+// tile to arrive would read all of its parts alone, 7 x 128 KB, at what one CU
+// takes in, and the code for it in the kernel above costs its loop registers:
+// 4096 x 14336, 256 rows, 8 parts 54.9 us so, 45.2 with this launch.)
+template <typename Tag>
+__global__ __launch_bounds__(256) void tile_sums_kernel(
+    short* __restrict__ out, const f32x4* __restrict__ sums, const int M,
+    const int N, const int row_blocks, const int col_blocks,
+    const int parts) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
+  const int lane = threadIdx.x % WAVE_SIZE;
+  const int unit = blockIdx.x * 4 + wave;
+  const int b = unit % 2 * 2, cb = unit / 2 % col_blocks;
+  const int rb = unit / 2 / col_blocks;
+  if (rb * 32 >= M) return;
+  const int64_t part = (int64_t)row_blocks * col_blocks * 256;
+  const f32x4* at =
+      sums + ((int64_t)rb * col_blocks + cb) * 256 + b * 64 + lane;
+  f32x16 v;
+  constexpr int Q = 8;
+  for (int p0 = 0; p0 < parts; p0 += Q) {
+    f32x4 t[Q][2];   // (a read past the last part repeats it)
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        t[q][c] = __builtin_nontemporal_load(
+            at + min(p0 + q, parts - 1) * part + c * 64);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float a = p0 == 0 ? t[0][c][r] : v[c * 4 + r] + t[0][c][r];
+#pragma unroll
+        for (int q = 1; q < Q; ++q)
+          if (p0 + q < parts) a += t[q][c][r];
+        v[c * 4 + r] = a;
+      }
+  }
+  const i32x4 chunk = row_chunk<Tag>(v, 0);
+  const int row = rb * 32 + (lane & 31);
+  const int col = cb * 32 + b * 8 + (lane >> 5) * 8;
+  if (row < M && col < N)
+    *reinterpret_cast<i32x4*>(out + (int64_t)row * N + col) = chunk;
+}
+
+// us of a product in tiles of `cols` weight rows with K in `parts`, for at most
+// 256 workgroups. A stage of 64 columns of K: what a CU takes in, rows of x and
+// weights, at 76 GB/s (one that has reads from HBM under way takes in no more,
+// whatever comes from L2 beside them); the weights' way from HBM; products.
+// These are coefficients of a fit and not bounds: 1800 times of 33 layers of
+// 512 x 7168 to 36864 x 7168 on 72 to 1024 rows are within 7 % of it (rms), and
+// the form that it prefers is 0.7 % slower than the best one on average.
+double estimate(int64_t M, int64_t N, int64_t K, int cols, int parts) {
+  const int64_t tm = M <= 128 ? 128 : 256;
+  const int64_t m_tiles = (M + tm - 1) / tm;
+  const double jobs = (double)(m_tiles * ((N + cols - 1) / cols) * parts);
+  const double rows = (double)(m_tiles == 1 ? (M + 31) / 32 * 32 : tm);
+  auto pow = [](double v) { return std::pow(v, 1.85); };
+  const double stage =
+      std::pow(pow((rows + cols) * 0.128 / 76.) +
+                   pow(cols * 128e-6 * jobs / (double)m_tiles / 8.) +
+                   pow(rows * cols * 128e-6 / 10.8),
+               1 / 1.85);
+  return (double)K / TP_K / parts * stage + 5.4 +
+         (parts > 1 ? 3.5 + parts * (double)M * (double)N * 4e-6 / 3.2 : 0.);
+}
+
+// The form of least estimate among those of one round that keep 60 % of the CUs
+// busy, where it is ahead of the library. With K whole: up to 256 rows. With K
+// split (up to 16 parts): from K = 5120 on up to 128 rows, above from 6144 on,
+// and only if K is long beside the 256 x 256 tiles of the output (170 columns
+// of K each, 90 of them), since partial sums cost 10 to 20 us. Below 1536
+// columns of output there is too little to split. us, the library and this (at
+// 128, 256 and 1024 rows if not said): 4096 x 14336 52 / 34, 65 / 45, 137 /
+// 116; 3584 x 18944 65 / 40, 80 / 52, 173 / 132; 7168 x 16384 71 / 54, 107 /
+// 72, and 512 rows 148 / 117; 2112 x 7168 25 / 17, 32 / 24, 49 / 45; 24576 x
+// 1536 27.6 / 23.0. On the other side of the lines: 4096 x 4096 17.3 / 17.0,
+// 21.0 / 25.1, 41 / 50; 4096 x 7168, 1024 rows 69 / 74; 8192 x 28672, 768 rows
+// 301 / 316; 36864 x 7168, 128 rows 118 / 121; 512 x 7168, 256 rows 12 / 15.6.
+TileForm by_estimate(int64_t M, int64_t N, int64_t K) {
+  TileForm best{0, 1};
+  if (M > 1024) return best;
+  const int64_t tm = M <= 128 ? 128 : 256;
+  const int64_t out_tiles = (M + 255) / 256 * ((N + 255) / 256);
+  const bool split = N >= 1536 && (M <= 128 ? K >= 5120
+                                            : K >= 6144 && out_tiles <= 90 &&
+                                                  K >= 170 * out_tiles);
+  double least = 1e30;
+  for (int cols : {64, 128, 256}) {
+    if (cols == 64 && M > 256) continue;
+    const int64_t tiles = (M + tm - 1) / tm * ((N + cols - 1) / cols);
+    for (int parts = 1; parts <= 16 && tiles * parts <= 256; ++parts) {
+      if (tiles * parts < 154 || K / TP_K / parts < 4 ||
+          (parts == 1 ? M > 256 || K <= 8 * M : !split))
+        continue;
+      const double t = estimate(M, N, K, cols, parts);
+      if (t < least) {
+        least = t;
+        best = {cols, parts};
+      }
+    }
+  }
+  return best;
+}
+
+// How M rows meet rows_w weight rows of K; cols 0: in the library.
 //
 // The share of its rounds over 256 CUs that a form keeps busy decides: 256
 // where that is at least 95 % (for up to 128 rows of a plain product in more
@@ -117,44 +274,81 @@ __global__ __launch_bounds__(TP_THREADS, 1) void tile_linear_kernel(
 // and the library: 65536 x 512, 256 rows 30.0 and 24.5, x 1024 39.7 and 37.9, x
 // 2048 73 and 76; 128256 x 256, 128 rows 30.6 and 26.2, x 1024 61.5 and 60.0,
 // 65 rows 54 and 62. An activation halves what is written.
-int tile_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
-  if (M <= 64 || M > TI_ROWS || (!silu && K <= 8 * M)) return 0;
-  auto rounds = [&](int tile) { return (rows_w + tile * 256 - 1) / tile / 256; };
-  auto busy = [&](int tile) {
-    return (double)((rows_w + tile - 1) / tile) / (double)(rounds(tile) * 256);
-  };
-  if (busy(256) >= 0.95 && (silu || M > 128 || rounds(256) > 1)) return 256;
-  const double least = rounds(128) > 1 ? (silu ? 0.9 : 2.) : silu ? 0.65 : 0.95;
-  return busy(128) >= least ? 128 : 0;
+TileForm tile_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
+  if (M <= 64 || (silu && M > TI_ROWS)) return {0, 1};
+  if (M <= TI_ROWS && (silu || K > 8 * M)) {
+    auto rounds = [&](int tile) {
+      return (rows_w + tile * 256 - 1) / tile / 256;
+    };
+    auto busy = [&](int tile) {
+      return (double)((rows_w + tile - 1) / tile) /
+             (double)(rounds(tile) * 256);
+    };
+    if (busy(256) >= 0.95 && (silu || M > 128 || rounds(256) > 1))
+      return {256, 1};
+    const double least =
+        rounds(128) > 1 ? (silu ? 0.9 : 2.) : silu ? 0.65 : 0.95;
+    if (busy(128) >= least) return {128, 1};
+  }
+  return silu ? TileForm{0, 1} : by_estimate(M, rows_w, K);
 }
 
 template <typename Tag, bool SILU>
 void launch(torch::Tensor& out, const torch::Tensor& x,
-            const torch::Tensor& w, int form) {
+            const torch::Tensor& w, TileForm form) {
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)out.size(1);
-  const int tiles = ceil_div(N, form / (SILU ? 2 : 1));
+  constexpr int H = SILU ? 2 : 1;
+  const int tm = M <= 128 ? 128 : 256;
+  const int m_tiles = ceil_div(M, tm), n_tiles = ceil_div(N, form.cols / H);
+  const int jobs = m_tiles * n_tiles * form.parts;
+  const int row_blocks = m_tiles * (tm / 32);
+  const int col_blocks = n_tiles * (form.cols / 32);
+  auto stream = c10::hip::getCurrentHIPStream().stream();
+  torch::Tensor sums;
+  if (form.parts > 1)
+    sums = torch::empty({(int64_t)form.parts * row_blocks * col_blocks * 1024},
+                        x.options().dtype(torch::kFloat));
+  f32x4* const to = form.parts > 1 ? (f32x4*)sums.data_ptr() : nullptr;
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(ceil_div(tiles, 8) * 8), dim3(TP_THREADS),
-                       0, c10::hip::getCurrentHIPStream().stream(),
-                       (short*)out.data_ptr(), (const short*)x.data_ptr(),
-                       (const short*)w.data_ptr(), M, N, K, tiles);
+    hipLaunchKernelGGL(kernel, dim3(ceil_div(jobs, 8) * 8), dim3(TP_THREADS),
+                       0, stream, (short*)out.data_ptr(),
+                       (const short*)x.data_ptr(), (const short*)w.data_ptr(),
+                       M, N, K, m_tiles, n_tiles, form.parts, to);
   };
   if (M <= 128) {
-    if (form == 128) go(tile_linear_kernel<Tag, SILU, 2, 2, 2, 5, 5>);
-    else             go(tile_linear_kernel<Tag, SILU, 1, 2, 4, 3, 3>);
-  } else {
-    if (form == 128) go(tile_linear_kernel<Tag, SILU, 2, 2, 4, 3, 3>);
-    else             go(tile_linear_kernel<Tag, SILU, 2, 4, 4, 2, 3>);
+    if (form.cols == 128)
+      go(tile_linear_kernel<Tag, SILU, true, 2, 2, 2, 5, 5>);
+    else if (form.cols == 256)
+      go(tile_linear_kernel<Tag, SILU, true, 1, 2, 4, 3, 3>);
+    else if constexpr (!SILU)
+      go(tile_linear_kernel<Tag, SILU, true, 4, 2, 1, 5, 5>);
+  } else if (m_tiles == 1) {
+    if (form.cols == 128)
+      go(tile_linear_kernel<Tag, SILU, true, 2, 2, 4, 3, 3>);
+    else if (form.cols == 256)
+      go(tile_linear_kernel<Tag, SILU, true, 2, 4, 4, 2, 3>);
+    else if constexpr (!SILU)
+      go(tile_linear_kernel<Tag, SILU, true, 4, 2, 2, 3, 3>);
+  } else if constexpr (!SILU) {
+    if (form.cols == 128)
+      go(tile_linear_kernel<Tag, SILU, false, 2, 2, 4, 3, 3>);
+    else
+      go(tile_linear_kernel<Tag, SILU, false, 2, 4, 4, 2, 3>);
   }
+  if (form.parts > 1)
+    hipLaunchKernelGGL((tile_sums_kernel<Tag>),
+                       dim3(ceil_div(row_blocks * col_blocks * 2, 4)),
+                       dim3(256), 0, stream, (short*)out.data_ptr(), to, M, N,
+                       row_blocks, col_blocks, form.parts);
 }
 
 }  // namespace
 
 // The form for a product of these sizes, 0 if it is not one for this file.
-int tile_linear_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
+TileForm tile_linear_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
   if (rows_w <= 0 || rows_w % (silu ? 16 : 8) != 0 || K <= 0 ||
       K % TP_K != 0 || K >= (1 << 22) || (rows_w + 256) * K * 2 >= (1ll << 32))
-    return 0;
+    return {0, 1};
   return tile_form(M, rows_w, K, silu);
 }
 
@@ -163,8 +357,8 @@ int tile_linear_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
 bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
                  const torch::Tensor& w, bool silu) {
   const int64_t K = x.size(1);
-  const int form = tile_linear_form(x.size(0), w.size(0), K, silu);
-  if (form == 0 || w.size(1) != K || w.scalar_type() != x.scalar_type() ||
+  const TileForm form = tile_linear_form(x.size(0), w.size(0), K, silu);
+  if (form.cols == 0 || w.size(1) != K || w.scalar_type() != x.scalar_type() ||
       (x.scalar_type() != torch::kBFloat16 &&
        x.scalar_type() != torch::kHalf) ||
       !x.is_contiguous() || !w.is_contiguous() ||

@@ -93,9 +93,6 @@ struct TileProduct {
       f32x16 acc[NI][J > 0 ? J : 1];
       loop<J>(lds, steps, wave, fill_a, fill_w, acc);
       done(n, acc);
-      // What was filled past the end must not land in another workgroup's
-      // LDS.
-      lds_fill_wait();
     };
     if (mine >= MI) go(std::integral_constant<int, MI>{});
     else if (MI > 3 && mine == 3) go(std::integral_constant<int, 3>{});
@@ -105,6 +102,16 @@ struct TileProduct {
   }
 
  private:
+  // The fills of n whole stages may be under way (where rows and weights are
+  // as far ahead; none elsewhere).
+  template <int MAX> static DEVINL void wait_but(int n) {
+    if constexpr (PA == PW && MAX > 0) {
+      if (n >= MAX) return lds_fill_wait<MAX * (FA + FW)>();
+      return wait_but<MAX - 1>(n);
+    }
+    lds_fill_wait();
+  }
+
   template <int J, typename FillA, typename FillW, int JA>
   static DEVINL void loop(char* lds, const int steps, const int wave,
                           FillA fill_a, FillW fill_w, f32x16 (&acc)[NI][JA]) {
@@ -123,12 +130,10 @@ struct TileProduct {
     const char* const a0 = lds + wm * 32 * TP_ROW;
     const char* const w0 = wlds + wn * WW * TP_ROW;
     auto fa = [&](int s, int i, int place) {
-      fill_a(min(s, steps - 1), i,
-             lds + place * AB + (wave * FA + i) * TP_FILL);
+      fill_a(s, i, lds + place * AB + (wave * FA + i) * TP_FILL);
     };
     auto fw = [&](int s, int i, int place) {
-      fill_w(min(s, steps - 1), i,
-             wlds + place * WB + (wave * FW + i) * TP_FILL);
+      fill_w(s, i, wlds + place * WB + (wave * FW + i) * TP_FILL);
     };
     s16x8 af[2][J > 0 ? J : 1], wf[2][NI];
     auto read = [&](int to, int ap, int wp, int k, int r) {
@@ -178,42 +183,58 @@ struct TileProduct {
     static_assert(AHEAD + FA < 64);
 #pragma unroll
     for (int t = 1 - PW; t < 0; ++t) {
-      if (t + PA - 1 >= 0) {
+      if (t + PA - 1 >= 0 && t + PA - 1 < steps) {
 #pragma unroll
         for (int i = t + PA - 1 == 0 ? 0 : FA / 2; i < FA; ++i)
           fa(t + PA - 1, i, t + PA - 1);
       }
+      if (t + PW - 1 < steps) {
 #pragma unroll
-      for (int i = 0; i < FW; ++i) fw(t + PW - 1, i, t + PW - 1);
-      if (t + PA >= 1) {
+        for (int i = 0; i < FW; ++i) fw(t + PW - 1, i, t + PW - 1);
+      }
+      if (t + PA >= 1 && t + PA < steps) {
 #pragma unroll
         for (int i = 0; i < FA / 2; ++i) fa(t + PA, i, (t + PA) % PA);
       }
     }
-    lds_fill_wait<AHEAD>();
+    if (steps >= PW) lds_fill_wait<AHEAD>();
+    else lds_fill_wait();
     lds_barrier();
 #pragma unroll
     for (int r = 0; r < F; ++r) read(0, 0, 0, 0, r);
     int ap = 0, wp = 0;
-#pragma unroll 1
-    for (int s = 0; s < steps; ++s) {
+    // MORE: fills of whole stages go on.
+    auto stage = [&](const int s, auto more) {
+      constexpr bool MORE = decltype(more)::value;
       const int an = ap == PA - 1 ? 0 : ap + 1, al = ap == 0 ? PA - 1 : ap - 1;
       const int wn_ = wp == PW - 1 ? 0 : wp + 1, wl = wp == 0 ? PW - 1 : wp - 1;
-      step(0, false, [&](int r) { read(1, ap, wp, 1, r); }, FA / 2,
-           [&](int f) { fa(s + PA - 1, FA / 2 + f, al); });
-      step(1, false, [&](int r) { read(0, ap, wp, 2, r); }, FW / 2,
-           [&](int f) { fw(s + PW - 1, f, wl); });
-      step(0, true, [&](int r) { read(1, ap, wp, 3, r); }, FW / 2,
-           [&](int f) { fw(s + PW - 1, FW / 2 + f, wl); });
+      step(0, false, [&](int r) { read(1, ap, wp, 1, r); }, FA / 2, [&](int f) {
+        if (MORE || s + PA - 1 < steps) fa(s + PA - 1, FA / 2 + f, al);
+      });
+      step(1, false, [&](int r) { read(0, ap, wp, 2, r); }, FW / 2, [&](int f) {
+        if (MORE || s + PW - 1 < steps) fw(s + PW - 1, f, wl);
+      });
+      step(0, true, [&](int r) { read(1, ap, wp, 3, r); }, FW / 2, [&](int f) {
+        if (MORE || s + PW - 1 < steps) fw(s + PW - 1, FW / 2 + f, wl);
+      });
       // The next stage has landed when only what was filled after it is
       // under way; past the barrier no wave reads this one again.
-      lds_fill_wait<AHEAD>();
+      if constexpr (MORE) lds_fill_wait<AHEAD>();
+      else wait_but<PW - 2>(steps - 2 - s);
       lds_barrier();
       step(1, true, [&](int r) { read(0, an, wn_, 0, r); }, FA / 2,
-           [&](int f) { fa(s + PA, f, ap); });
+           [&](int f) {
+             if (MORE || s + PA < steps) fa(s + PA, f, ap);
+           });
       ap = an;
       wp = wn_;
-    }
+    };
+    constexpr int LAST = PA > PW - 1 ? PA : PW - 1;   // stage MORE looks ahead
+    int s = 0;
+#pragma unroll 1
+    for (; s + LAST < steps; ++s) stage(s, std::true_type{});
+#pragma unroll 1
+    for (; s < steps; ++s) stage(s, std::false_type{});
   }
 };
 
