@@ -709,6 +709,17 @@ def test_head_matmul(T, H, K, N, dtype):
                  else 2**-10)
 
 
+# Four steps of K at once up to 256 workgroups (both sides), and five steps.
+@pytest.mark.parametrize("T,H,K,N", [(128, 128, 512, 128), (129, 86, 512, 128),
+                                     (3, 2, 640, 128)])
+def test_head_matmul_steps(T, H, K, N):
+    hip = _hip()
+    x = torch.randn(T, H, K, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(H, K, N, device="cuda", dtype=torch.bfloat16) * K**-0.5
+    assert_close(hip.head_matmul(x, w), ref.head_matmul(x, w),
+                 atol=2**-9, rtol=2**-8)   # as above
+
+
 @pytest.mark.parametrize("T,H,I,E,K,act", [
     (33, 128, 128, 6, 2, "relu2"),    # streamed, part of a 64-row tile
     (1100, 128, 64, 128, 2, "silu"),  # streamed, counted by blocks of rows
