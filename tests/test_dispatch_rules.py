@@ -81,6 +81,15 @@ def test_mla_decode_split_ignores_prompts(hip, rows, monkeypatch):
     assert split(8192) == split(0)
 
 
+@pytest.mark.parametrize("rows,heads,keys,parts", [
+    (1, 128, 60, 1), (1, 128, 1000, 8), (1, 128, 16000, 64),
+    (16, 128, 2000, 8), (64, 128, 130, 1), (128, 128, 1000, 1),
+    (128, 128, 2176, 2), (32, 128, 8192, 8), (200, 128, 2176, 1),
+    (300, 128, 500, 1), (1, 16, 4000, 32), (64, 16, 1000, 4)])
+def test_mla_split(hip, rows, heads, keys, parts):
+    assert hip._mla_split(rows, heads, keys) == parts
+
+
 @pytest.mark.parametrize("rows,kv,span,window,parts", [
     (1, 8, 1000, 0, 8),       # none shorter than 128 keys
     (1, 8, 8192, 0, 32),      # one workgroup a CU ...

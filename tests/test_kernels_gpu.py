@@ -662,6 +662,34 @@ def test_mla_decode_kernel(T, Hq, ctx):
     assert_close(out, expect, atol=4e-2, rtol=4e-2)
 
 
+# Workgroups of 32, 64 and 128 heads; heads that end within one, and within a
+# wave's 16; keys of one tile, whole and in parts.
+@pytest.mark.parametrize("T,Hq,wide,bound", [
+    (3, 128, 32, 200), (2, 72, 32, 64), (17, 128, 32, 900),
+    (64, 100, 32, 130), (24, 128, 64, 2176), (100, 90, 64, 500),
+    (100, 128, 128, 1500), (5, 33, 128, 1500)])
+def test_mla_decode_head_groups(T, Hq, wide, bound):
+    hip = _hip()
+    parts = hip._mla_split(T, Hq, bound)
+    n = 128
+    while n > 32 and Hq > n // 2 and T * parts * -(-Hq // (n // 2)) <= 256:
+        n //= 2
+    assert n == wide
+    ctx = [1 + (bound - 1) * i // max(T - 1, 1) for i in range(T - 1)] + [bound]
+    nb = -(-bound // 64)
+    kv = torch.randn(T * nb, 64, 576, dtype=torch.bfloat16, device="cuda")
+    bt = torch.randperm(T * nb, device="cuda").int().view(T, nb)
+    sl = torch.tensor(ctx, dtype=torch.int32, device="cuda")
+    qn = torch.randn(T, Hq, 512, dtype=torch.bfloat16, device="cuda") * 0.3
+    qp = torch.randn(T, Hq, 64, dtype=torch.bfloat16, device="cuda") * 0.3
+    out = hip.mla_decode(qn, qp, kv, bt, sl, 0.07, bound)
+    expect = ref.mla_attention(
+        qn.float(), qp.float(), kv.float(), bt,
+        torch.arange(T + 1, dtype=torch.int32, device="cuda"), sl, 0.07)
+    # As below: weights and results rounded to 16 bits, values up to 4.
+    assert_close(out, expect, atol=8 * 2**-8, rtol=2 * 2**-8)
+
+
 @pytest.mark.parametrize("heads,bs,dtype", [
     (128, 64, torch.bfloat16),   # whole tiles from one cache block
     (130, 16, torch.bfloat16),   # second head group nearly empty

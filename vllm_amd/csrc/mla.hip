@@ -33,8 +33,8 @@
 //     2^8. Where they are rounded to 16 (decode), the largest is kept at
 //     one and the rounded weights are summed: 3 % slower, 4 % closer to
 //     64-bit results.
-// Rows are split over a few partitions of the keys when there are fewer
-// than CUs; fp32 partials (256 KB per row and partition) are merged by
+// Rows are split over a few partitions of the keys, and heads over workgroups
+// (group_heads below), when there are fewer than CUs; fp32 partials (256 KB per row and partition) are merged by
 // mla_reduce_kernel, so partitions are few and long, and rows that fit one
 // are written at once. A portion of 2 tokens after 8190 takes 56 us in
 // 64 partitions, with the products around it, and 510 in one.
@@ -56,7 +56,7 @@ namespace mla {
 constexpr int LORA = 512;
 constexpr int ROPE = 64;
 constexpr int DK = LORA + ROPE;   // 576
-constexpr int HG = 128;           // heads per workgroup
+constexpr int HG = 128;           // heads per workgroup, at most
 constexpr int SUB = 64;           // keys per LDS tile
 constexpr int WAVES = 8;
 constexpr int THREADS = WAVES * WAVE_SIZE;
@@ -113,7 +113,7 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
                 int num_reqs,
                 float* __restrict__ tmp_out,  // [rows, Hq, parts, LORA]
                 float* __restrict__ tmp_lse,  // [rows, Hq, parts, 2]
-                int num_parts, int part_len) {
+                int num_parts, int part_len, int group_heads) {
   int req, row, ctx, first = 0;   // first: row 0 of the scratch
   if constexpr (PROMPT) {
     row = query_start_loc[num_reqs] - 1 - (int)blockIdx.x;
@@ -125,14 +125,14 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
     req = row = blockIdx.x;
     ctx = seq_lens[req];
   }
-  const int hg0 = blockIdx.z * HG;
+  const int hg0 = blockIdx.z * group_heads;
   const int part = PARTS ? blockIdx.y : 0;
   const int t_begin = PARTS ? part * part_len : 0;
   const int t_end =
       PARTS && part + 1 < num_parts ? min(ctx, t_begin + part_len) : ctx;
   if (t_begin >= t_end) {
     if (!PROMPT && part == 0) {   // a row without keys (padding) is zero
-      const int n = min(HG, num_heads - hg0) * (LORA / 8);
+      const int n = min(group_heads, num_heads - hg0) * (LORA / 8);
       short* ob = out + ((int64_t)row * num_heads + hg0) * LORA;
       for (int c = threadIdx.x; c < n; c += THREADS)
         *reinterpret_cast<i32x4*>(ob + c * 8) = i32x4{0, 0, 0, 0};
@@ -147,7 +147,8 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
   const int l16 = lane & 15;
   const int l4 = lane >> 4;
   const int head = hg0 + wave * 16 + l16;
-  const bool busy = hg0 + wave * 16 < num_heads;
+  const bool busy =
+      wave * 16 < group_heads && hg0 + wave * 16 < num_heads;
 
   s16x8 qf[DK / 32];
   {
@@ -292,7 +293,7 @@ void mla_kernel(short* __restrict__ out,           // [T, Hq, LORA]
 
   l_run += __shfl_xor(l_run, 16, 64);
   l_run += __shfl_xor(l_run, 32, 64);
-  if (head >= num_heads) return;
+  if (!busy || head >= num_heads) return;
   const int64_t hrow = (int64_t)row * num_heads + head;
   if (!PARTS || num_parts == 1 || ctx <= part_len) {   // nothing to merge
     const float inv_l = 1.f / l_run;
@@ -404,6 +405,23 @@ static int part_length(int64_t max_seq_len, int parts) {
                   SUB) * SUB;
 }
 
+// Heads that a workgroup takes, of `pairs` rows and partitions: fewer than 128
+// while a round of workgroups then still has room on 256 CUs. A tile of 64
+// heads takes two thirds of the time of one of 128, of 32 half, and each
+// workgroup reads its queries and writes its partials in proportion, so few
+// and short rows are done sooner, and others need fewer partitions. us at 128
+// heads with the merge, 128 / 64 / 32 heads a workgroup, each in its best
+// number of partitions: 1 x 200 keys 21.6 / 14.2 / 12.3, 1 x 4000 28.8 / 24.2 /
+// 22.0, 8 x 4000 37.0 / 31.4 / 34.7, 64 x 100..150 27.4 / 17.9 / 16.1, 76 x
+// 431..531 40.9 / 33.6, 128 x 1000 64.8 / 57.7; 32 x 8192 103 / 106, 128 x
+// 129..2176 85 / 96 (hip_ops.py chooses the partitions with this in mind).
+static int group_heads(int64_t pairs, int64_t Hq) {
+  int n = HG;
+  while (n > 32 && Hq > n / 2 && pairs * ceil_div((int)Hq, n / 2) <= 256)
+    n /= 2;
+  return n;
+}
+
 }  // namespace mla
 
 // Decode rows; the scratch says into how many partitions their keys go.
@@ -420,7 +438,8 @@ void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
   const int parts = parts_of(tmp_out, tmp_lse, T, Hq);
   const int part_len = part_length(max_seq_len, parts);
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  dim3 grid(T, parts, ceil_div(Hq, HG));
+  const int heads = group_heads((int64_t)T * parts, Hq);
+  dim3 grid(T, parts, ceil_div(Hq, heads));
   auto launch = [&](auto tag) {
     using Tag = decltype(tag);
     hipLaunchKernelGGL(
@@ -430,7 +449,8 @@ void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
         block_table.data_ptr<int>(), (int)block_table.size(1), nullptr,
         seq_lens.data_ptr<int>(), (float)scale * 1.4426950408889634f, Hq, bs,
         T, T, parts > 1 ? tmp_out.data_ptr<float>() : nullptr,
-        parts > 1 ? tmp_lse.data_ptr<float>() : nullptr, parts, part_len);
+        parts > 1 ? tmp_lse.data_ptr<float>() : nullptr, parts, part_len,
+        heads);
     if (parts > 1) {
       HIP_CHECK_KERNEL();
       hipLaunchKernelGGL((mla_reduce_kernel<Tag, false>), dim3(Hq, T),
@@ -462,7 +482,8 @@ void mla_prefill(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
   auto stream = c10::hip::getCurrentHIPStream().stream();
   const int parts = parts_of(tmp_out, tmp_lse, rows, Hq);
   const int part_len = part_length(max_seq_len, parts);
-  dim3 grid(rows, parts, ceil_div(Hq, HG));
+  const int heads = group_heads((int64_t)rows * parts, Hq);
+  dim3 grid(rows, parts, ceil_div(Hq, heads));
   auto launch = [&](auto tag, auto split) {
     using Tag = decltype(tag);
     constexpr bool PARTS = decltype(split)::value;
@@ -474,7 +495,8 @@ void mla_prefill(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
         query_start_loc.data_ptr<int>(), seq_lens.data_ptr<int>(),
         (float)scale * 1.4426950408889634f, Hq, (int)kv_cache.size(1),
         (int)num_decodes, reqs, PARTS ? tmp_out.data_ptr<float>() : nullptr,
-        PARTS ? tmp_lse.data_ptr<float>() : nullptr, parts, part_len);
+        PARTS ? tmp_lse.data_ptr<float>() : nullptr, parts, part_len,
+        heads);
     if constexpr (PARTS) {
       HIP_CHECK_KERNEL();
       hipLaunchKernelGGL((mla_reduce_kernel<Tag, true>), dim3(Hq, rows),
