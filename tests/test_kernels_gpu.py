@@ -738,14 +738,16 @@ def test_head_matmul(T, H, K, N, dtype):
 
 
 # Four steps of K at once up to 256 workgroups (both sides), and five steps.
+# Off from sums that are not rounded by the result's own rounding: 2^-8 of it
+# (from rounded ones by twice that, where a sum lies between two results).
 @pytest.mark.parametrize("T,H,K,N", [(128, 128, 512, 128), (129, 86, 512, 128),
                                      (3, 2, 640, 128)])
 def test_head_matmul_steps(T, H, K, N):
     hip = _hip()
     x = torch.randn(T, H, K, device="cuda", dtype=torch.bfloat16)
     w = torch.randn(H, K, N, device="cuda", dtype=torch.bfloat16) * K**-0.5
-    assert_close(hip.head_matmul(x, w), ref.head_matmul(x, w),
-                 atol=2**-9, rtol=2**-8)   # as above
+    assert_close(hip.head_matmul(x, w), ref.head_matmul(x.float(), w.float()),
+                 atol=2**-9, rtol=2**-8)
 
 
 @pytest.mark.parametrize("T,H,I,E,K,act", [

@@ -9,6 +9,7 @@
 #include <hip/hip_fp16.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #define WAVE_SIZE 64
 
@@ -144,6 +145,37 @@ template <> DEVINL f32x16 mfma32<FP16Tag>(s16x8 a, s16x8 b, f32x16 c) {
       __builtin_bit_cast(h16x8, a), __builtin_bit_cast(h16x8, b), c, 0, 0, 0);
 }
 
+// c += a b, 16 x 16 x 32, c in accumulation registers and in its place. The
+// builtin names result and sum apart: where all 256 accumulation registers
+// are taken the compiler then moves them about (8192 x 28672 x 4096 by
+// tile_product.h 1.08 PFLOP/s, 1.43 so). The compiler knows nothing of
+// what may stand right before and after the instruction, so accumulators come
+// and go through acc_fence.
+template <typename Tag> DEVINL void mfma16_acc(f32x4& c, s16x8 a, s16x8 b) {
+  if constexpr (std::is_same_v<Tag, BF16Tag>)
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                 : "+a"(c)
+                 : "v"(a), "v"(b));
+  else
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0"
+                 : "+a"(c)
+                 : "v"(a), "v"(b));
+}
+// Between other instructions that write or read the accumulators and products
+// that do: the waits of either side (up to 19 states after a product of eight
+// passes) lie between them.
+template <int N, int M> DEVINL void acc_fence(f32x4 (&acc)[N][M]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < M; ++j) asm volatile("" : "+a"(acc[i][j]));
+  asm volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < M; ++j) asm volatile("" : "+a"(acc[i][j]));
+}
+
 // Two floats rounded (nearest even) to a packed 16-bit pair.
 template <typename Tag> DEVINL int pack2(float a, float b);
 template <> DEVINL int pack2<BF16Tag>(float a, float b) {
@@ -200,6 +232,22 @@ template <typename Tag> DEVINL i32x4 row_chunk(const f32x16& c, int b) {
   const unsigned y1 = pack2<Tag>(c[b * 4 + 6], c[b * 4 + 7]);
   const auto s0 = __builtin_amdgcn_permlane32_swap(x0, y0, false, false);
   const auto s1 = __builtin_amdgcn_permlane32_swap(x1, y1, false, false);
+  const int a0 = s0[0], a1 = s1[0], b0 = s0[1], b1 = s1[1];
+  return i32x4{a0, a1, b0, b1};
+}
+
+// The same of two 16 x 16 products with the columns of 16 x 16 in a row: lane
+// l16 of group l4 holds rows 4 * l4 + 0..3 of each, and gets eight rows from
+// row_start16() of the pair's 32 on.
+DEVINL int row_start16() {
+  const int l4 = threadIdx.x % WAVE_SIZE >> 4;
+  return (l4 & 1) * 16 + (l4 >> 1) * 8;
+}
+template <typename Tag> DEVINL i32x4 row_chunk16(f32x4 a, f32x4 b) {
+  const auto s0 = __builtin_amdgcn_permlane16_swap(
+      pack2<Tag>(a[0], a[1]), pack2<Tag>(b[0], b[1]), false, false);
+  const auto s1 = __builtin_amdgcn_permlane16_swap(
+      pack2<Tag>(a[2], a[3]), pack2<Tag>(b[2], b[3]), false, false);
   const int a0 = s0[0], a1 = s1[0], b0 = s0[1], b1 = s1[1];
   return i32x4{a0, a1, b0, b1};
 }

@@ -1,8 +1,8 @@
 // Grouped expert products for experts of many rows (gfx950): 128 or 256 x
 // 256 tiles of tile_product.h, the matrix cores bound them. The product is
 // formed transposed (weight rows are the A operand), so a lane ends up with
-// four neighbouring columns of one row, eight after a trade with the other
-// half wave (16 B stores). Gated experts: a tile is 128 gate rows and the up
+// four neighbouring columns of one row, eight after a trade with another
+// quarter of the wave (16 B stores). Gated experts: a tile is 128 gate rows and the up
 // rows of the same columns, a wave's gate groups before its up groups, and
 // the activation is the epilogue.
 //
@@ -18,10 +18,10 @@
 // With up to 64 rows 906, 1086 and 594.
 //
 // 64 experts of 7168 x 2048, 4096 tokens of 8, 50 to 1925 rows an expert:
-// 1.76 + 0.98 ms (eight waves by halves in turn 2.01 + 1.10); 512 rows each
-// 1.50 + 0.86 (1.28 and 1.12 PFLOP/s: the second, of 32 stages, pays the
-// start and end of its tiles). What uneven rows cost beyond their padding
-// is weights read twice: tiles of an expert that are not in step do not
+// 1.76 + 0.95 ms (eight waves by halves in turn 2.01 + 1.10); 512 rows each
+// 1.47 + 0.84 (1.31 and 1.14 PFLOP/s: the second, of 32 stages, pays the start
+// and end of its tiles; by products of 32 x 32 x 16 1.50 + 0.86). What uneven rows cost beyond their
+// padding is weights read twice: tiles of an expert that are not in step do not
 // meet in L2 (8.3 GB instead of 4.1 in the first product).
 
 #include <torch/all.h>
@@ -35,16 +35,15 @@ namespace vllm_amd {
 namespace moe {
 
 // One tile by TileProduct; `row0` is its first row in tile order.
-template <typename Tag, int ACT, int WGM, int NI, int MI, int PA>
+template <typename Tag, int ACT, int WGM, int NG, int MG, int PA>
 DEVINL void tile_body(char* lds, const TileArgs& t, const short* w,
                       const int row0, const int rows, const int n0) {
-  using P = TileProduct<Tag, WGM, NI, MI, PA, 3>;
+  using P = TileProduct<Tag, WGM, NG, MG, PA, 3>;
   static_assert(P::TN == TL_W && P::WW * P::WGN == TL_W);
   constexpr bool GATED = ACT == SILU_GATED;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
-  const int l32 = lane & 31;
-  const int half = lane >> 5;
+  const int l16 = lane & 15;
   const int N = t.N;
 
   uint32_t ap[P::FA], wp[P::FW];   // byte places of this lane's pieces
@@ -74,31 +73,30 @@ DEVINL void tile_body(char* lds, const TileArgs& t, const short* w,
       [&](int s, int i, char* dst) { lds_fill16(w + s * TP_K, wp[i], dst); },
       [&](auto n, auto& acc) {
         constexpr int J = decltype(n)::value;
-        constexpr int NO = GATED ? NI / 2 : NI;
-        // Register r of acc[i][j]: weight row i*32 + 8*(r/4) + 4*half + r%4
-        // of the wave, row l32 of its group j.
+        constexpr int NO = GATED ? P::NI / 2 : P::NI;
         const int wm = wave / P::WGN, wn = wave % P::WGN;
+        const int col0 = n0 + wn * NO * 16 + row_start16();
 #pragma unroll
         for (int j = 0; j < J; ++j) {
-          const int row = (j * WGM + wm) * 32 + l32;
+          const int row = P::row_of(j, wm) + l16;
           if (row >= rows) continue;
           short* c = t.c + (int64_t)(row0 + row) * t.ldc;
 #pragma unroll
-          for (int i = 0; i < NO; ++i) {
-            f32x16 v = acc[i][j];
+          for (int i = 0; i < NO; i += 2) {
+            f32x4 v[2];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              if constexpr (GATED)
-                v[r] = silu_mul(v[r], acc[i + NI / 2][j][r]);
-              else if constexpr (ACT == RELU2)
-                v[r] = relu2(v[r]);
-            }
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int b = 0; b < 4; b += 2) {
-              const i32x4 o = row_chunk<Tag>(v, b);
-              const int col = n0 + wn * NO * 32 + i * 32 + b * 8 + half * 8;
-              if (col < N) *reinterpret_cast<i32x4*>(c + col) = o;
-            }
+              for (int r = 0; r < 4; ++r) {
+                const float a = acc[i + h][j][r];
+                if constexpr (GATED)
+                  v[h][r] = silu_mul(a, acc[i + h + NO][j][r]);
+                else
+                  v[h][r] = ACT == RELU2 ? relu2(a) : a;
+              }
+            const i32x4 o = row_chunk16<Tag>(v[0], v[1]);
+            const int col = col0 + i * 16;
+            if (col < N) *reinterpret_cast<i32x4*>(c + col) = o;
           }
         }
       });

@@ -39,22 +39,22 @@ constexpr int TI_ROWS = 256;
 // N: columns of out. SILU: w has 2N rows, gate then up; a wave's gate rows,
 // then the up rows of the same columns. ONCE: one workgroup reads a weight.
 // parts > 1 (not SILU): K is split, and the sums of a part go to `sums` in
-// blocks of 32 x 32: [parts][row blocks][column blocks][4][lane].
-template <typename Tag, bool SILU, bool ONCE, int WGM, int NI, int MI, int PA,
+// blocks of 32 x 32: [parts][row blocks][column blocks][2][2][lane], those of
+// 16 weight rows and in them of 16 rows.
+template <typename Tag, bool SILU, bool ONCE, int WGM, int NG, int MG, int PA,
           int PW>
 __global__ __launch_bounds__(TP_THREADS, 1) void tile_linear_kernel(
     short* __restrict__ out, const short* __restrict__ x,
     const short* __restrict__ w, const int M, const int N, const int K,
     const int m_tiles, const int n_tiles, const int parts,
     f32x4* __restrict__ sums) {
-  using P = TileProduct<Tag, WGM, NI, MI, PA, PW>;
+  using P = TileProduct<Tag, WGM, NG, MG, PA, PW>;
   __shared__ __align__(16) char lds[P::LDS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
-  const int l32 = lane & 31;
-  const int half = lane >> 5;
+  const int l16 = lane & 15;
   constexpr int H = SILU ? 2 : 1;
-  constexpr int NO = NI / H;
+  constexpr int NO = P::NI / H;
   // Each XCD (workgroups go round them) takes a run of tiles; those beside
   // each other have weights in common, then columns of K.
   const int tiles = m_tiles * n_tiles, jobs = tiles * parts;
@@ -106,45 +106,37 @@ __global__ __launch_bounds__(TP_THREADS, 1) void tile_linear_kernel(
       [&](auto n, auto& acc) {
         constexpr int J = decltype(n)::value;
         const int wm = wave / P::WGN, wn = wave % P::WGN;
-        if (!SILU && parts > 1) {
-          const int cols = n_tiles * (P::TN / 32);
-#pragma unroll
-          for (int j = 0; j < J; ++j) {
-            const int rb = m0 / 32 + j * WGM + wm;
-            f32x4* to = sums + lane +
-                        (((int64_t)part * m_tiles * (P::TM / 32) + rb) * cols +
-                         n0 / 32 + wn * NI) *
-                            256;
-#pragma unroll
-            for (int i = 0; i < NI; ++i)
-#pragma unroll
-              for (int b = 0; b < 4; ++b)
-                to[i * 256 + b * 64] =
-                    f32x4{acc[i][j][b * 4], acc[i][j][b * 4 + 1],
-                          acc[i][j][b * 4 + 2], acc[i][j][b * 4 + 3]};
-          }
-          return;
-        }
+        const int col0 = n0 + wn * NO * 16 + row_start16();
+        const int cols = n_tiles * (P::TN / 32);
 #pragma unroll
         for (int j = 0; j < J; ++j) {
-          const int row = (j * WGM + wm) * 32 + l32;
+          if (!SILU && parts > 1) {
+            const int rb = (m0 + P::row_of(j, wm)) / 32;
+            f32x4* to = sums + lane + j % 2 * 64 +
+                        (((int64_t)part * m_tiles * (P::TM / 32) + rb) * cols +
+                         n0 / 32 + wn * NG) *
+                            256;
+#pragma unroll
+            for (int i = 0; i < P::NI; ++i) to[i * 128] = acc[i][j];
+            continue;
+          }
+          const int row = P::row_of(j, wm) + l16;
           if (row >= rows) continue;
           short* o = out + (int64_t)(m0 + row) * N;
 #pragma unroll
-          for (int i = 0; i < NO; ++i) {
-            f32x16 v = acc[i][j];
-            const int c0 = n0 + (wn * NO + i) * 32;
+          for (int i = 0; i < NO; i += 2) {
+            f32x4 v[2] = {acc[i][j], acc[i + 1][j]};
             if constexpr (SILU) {
 #pragma unroll
-              for (int r = 0; r < 16; ++r)
-                v[r] = v[r] / (1.f + __expf(-v[r])) * acc[i + NI / 2][j][r];
-            }
+              for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int b = 0; b < 4; b += 2) {
-              const i32x4 chunk = row_chunk<Tag>(v, b);
-              const int col = c0 + b * 8 + half * 8;
-              if (col < N) *reinterpret_cast<i32x4*>(o + col) = chunk;
+                for (int r = 0; r < 4; ++r)
+                  v[h][r] = v[h][r] / (1.f + __expf(-v[h][r])) *
+                            acc[i + h + NO][j][r];
             }
+            const i32x4 chunk = row_chunk16<Tag>(v[0], v[1]);
+            const int col = col0 + i * 16;
+            if (col < N) *reinterpret_cast<i32x4*>(o + col) = chunk;
           }
         }
       });
@@ -163,13 +155,13 @@ __global__ __launch_bounds__(256) void tile_sums_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
   const int unit = blockIdx.x * 4 + wave;
-  const int b = unit % 2 * 2, cb = unit / 2 % col_blocks;
+  const int b = unit % 2, cb = unit / 2 % col_blocks;
   const int rb = unit / 2 / col_blocks;
   if (rb * 32 >= M) return;
   const int64_t part = (int64_t)row_blocks * col_blocks * 256;
   const f32x4* at =
       sums + ((int64_t)rb * col_blocks + cb) * 256 + b * 64 + lane;
-  f32x16 v;
+  f32x4 v[2];
   constexpr int Q = 8;
   for (int p0 = 0; p0 < parts; p0 += Q) {
     f32x4 t[Q][2];   // (a read past the last part repeats it)
@@ -178,21 +170,21 @@ __global__ __launch_bounds__(256) void tile_sums_kernel(
 #pragma unroll
       for (int c = 0; c < 2; ++c)
         t[q][c] = __builtin_nontemporal_load(
-            at + min(p0 + q, parts - 1) * part + c * 64);
+            at + min(p0 + q, parts - 1) * part + c * 128);
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        float a = p0 == 0 ? t[0][c][r] : v[c * 4 + r] + t[0][c][r];
+        float a = p0 == 0 ? t[0][c][r] : v[c][r] + t[0][c][r];
 #pragma unroll
         for (int q = 1; q < Q; ++q)
           if (p0 + q < parts) a += t[q][c][r];
-        v[c * 4 + r] = a;
+        v[c][r] = a;
       }
   }
-  const i32x4 chunk = row_chunk<Tag>(v, 0);
-  const int row = rb * 32 + (lane & 31);
-  const int col = cb * 32 + b * 8 + (lane >> 5) * 8;
+  const i32x4 chunk = row_chunk16<Tag>(v[0], v[1]);
+  const int row = rb * 32 + b * 16 + (lane & 15);
+  const int col = cb * 32 + row_start16();
   if (row < M && col < N)
     *reinterpret_cast<i32x4*>(out + (int64_t)row * N + col) = chunk;
 }

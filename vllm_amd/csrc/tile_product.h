@@ -4,23 +4,28 @@
 // without -amdgpu-mfma-vgpr-form: 256 accumulators a lane leave no room in
 // the vector registers.
 //
-// What bounds it. A wave of 128 x 128 reads 8 fragments of 32 x 16 from LDS
-// for 16 products of 32 x 32 x 16 (64 B a clock of the 128 that LDS gives;
-// eight waves of 64 x 128 read 96, and with what is filled that is all there
-// is). With one wave a SIMD nothing else hides a wait, so nothing waits:
-//  * fragments of the next 16 columns are read one at a time between this
-//    step's products, the order of products being that in which fragments
-//    arrive (pinned by scheduling barriers: the compiler would move reads to
-//    their use);
+// What bounds it. Large products the chip's power: the matrix cores are busy
+// three quarters of the cycles, at 1.7 to 1.8 GHz. Products of 16 x 16 x 32 move
+// half the accumulators per flop that those of 32 x 32 x 16 do (random values
+// from registers alone: 2.02 and 1.77 PFLOP/s). Small ones what a CU takes in:
+// about 64 KB are under way, so 50 to 60 GB/s beside reads from HBM.
+//  * A wave of 128 x 128 reads 16 fragments of 16 x 32 from LDS for 64 products
+//    (half of what LDS gives; eight waves of 64 x 128 read 96 B a clock, and
+//    with what is filled that is all there is). With one wave a SIMD nothing
+//    else hides a wait, so nothing waits: fragments of the next 32 columns are
+//    read between this step's products, the order of products being that in
+//    which fragments arrive (pinned by scheduling barriers: the compiler would
+//    move reads to their use);
 //  * fills go straight from global memory to LDS, a few between products of
 //    every step: all at once they back up behind each other;
-//  * one barrier per 64 columns, before the last of their four steps, by
+//  * one barrier per 64 columns, before the last of their two steps, by
 //    when all of their fragments are in registers. From there on their
 //    places are filled again, that of the rows first. (Beside 256 x 256
 //    tiles LDS has two places for rows and three for weights, which come
 //    from further away.)
-// 8192 x 28672 x 4096 in bf16: 1.39 PFLOP/s, 8192 x 4096 x 14336 1.44 (eight
-// waves by halves in turn 1.0; the tuned library 1.57 and 1.60).
+// 8192 x 4096 x 14336 in bf16: 1.50 PFLOP/s, 8192 x 28672 x 4096 1.43, 2048 x
+// 8192 x 4096 1.40 (32 x 32 x 16 1.43, 1.36 and 1.29; eight waves by halves in
+// turn 1.0; the tuned library 1.60 and 1.57 of the first two).
 #pragma once
 
 #include <type_traits>
@@ -59,27 +64,35 @@ template <int NI, int J> struct TpOrder {
   }
 };
 
-// WGM: waves along the rows (4 / WGM along the weights). NI, MI: 32-row
+// WGM: waves along the rows (4 / WGM along the weights). NG, MG: 32-row
 // groups of weights and of rows a wave takes. PA, PW: stages of rows and of
 // weights that LDS holds. The waves' groups of rows alternate, so that in a
 // tile with few rows they have as many each.
-template <typename Tag, int WGM, int NI, int MI, int PA, int PW>
+template <typename Tag, int WGM, int NG, int MG, int PA, int PW>
 struct TileProduct {
   static constexpr int WGN = 4 / WGM;
-  static constexpr int TM = WGM * MI * 32;
-  static constexpr int TN = WGN * NI * 32;
+  static constexpr int NI = NG * 2;          // 16-row groups of weights
+  static constexpr int TM = WGM * MG * 32;
+  static constexpr int TN = WGN * NG * 32;
   static constexpr int AB = TM * TP_ROW;     // bytes of a stage
   static constexpr int WB = TN * TP_ROW;
   static constexpr int FA = TM / 8 / 4;      // fills a wave
   static constexpr int FW = TN / 8 / 4;
   static constexpr int LDS = PA * AB + PW * WB;
-  static constexpr int WW = NI * 32;         // weight rows of a wave
+  static constexpr int WW = NG * 32;         // weight rows of a wave
   static_assert(PA >= 2 && PW >= PA && LDS <= 160 * 1024);
-  static_assert(NI % 2 == 0, "products of a step go in pairs");
+
+  // First row in the tile of 16-row group j of a wave that is wm-th along
+  // the rows.
+  static DEVINL int row_of(int j, int wm) {
+    return (j / 2 * WGM + wm) * 32 + j % 2 * 16;
+  }
 
   // fill_a(step, i, dst) and fill_w: the wave's i-th fill of 8 rows of a
   // stage, rows (wave * FA + i) * 8 .. of the tile. done(J, acc) gets the
-  // sums of the J groups of rows of this wave that hold any of `rows`.
+  // sums of the J 16-row groups of this wave in the 32-row groups that hold
+  // any of `rows`: register r of acc[i][j] is weight row i*16 + 4*l4 + r of
+  // the wave, row l16 of its group j.
   template <typename FillA, typename FillW, typename Done>
   static DEVINL void run(char* lds, const int steps, const int rows,
                          FillA fill_a, FillW fill_w, Done done) {
@@ -89,15 +102,15 @@ struct TileProduct {
     const int groups = (min(rows, TM) + 31) / 32;
     const int mine = (groups - wm + WGM - 1) / WGM;
     auto go = [&](auto n) {
-      constexpr int J = decltype(n)::value;
-      f32x16 acc[NI][J > 0 ? J : 1];
+      constexpr int J = decltype(n)::value * 2;
+      f32x4 acc[NI][J > 0 ? J : 1];
       loop<J>(lds, steps, wave, fill_a, fill_w, acc);
-      done(n, acc);
+      done(std::integral_constant<int, J>{}, acc);
     };
-    if (mine >= MI) go(std::integral_constant<int, MI>{});
-    else if (MI > 3 && mine == 3) go(std::integral_constant<int, 3>{});
-    else if (MI > 2 && mine == 2) go(std::integral_constant<int, 2>{});
-    else if (MI > 1 && mine == 1) go(std::integral_constant<int, 1>{});
+    if (mine >= MG) go(std::integral_constant<int, MG>{});
+    else if (MG > 3 && mine == 3) go(std::integral_constant<int, 3>{});
+    else if (MG > 2 && mine == 2) go(std::integral_constant<int, 2>{});
+    else if (MG > 1 && mine == 1) go(std::integral_constant<int, 1>{});
     else go(std::integral_constant<int, 0>{});
   }
 
@@ -114,20 +127,20 @@ struct TileProduct {
 
   template <int J, typename FillA, typename FillW, int JA>
   static DEVINL void loop(char* lds, const int steps, const int wave,
-                          FillA fill_a, FillW fill_w, f32x16 (&acc)[NI][JA]) {
+                          FillA fill_a, FillW fill_w, f32x4 (&acc)[NI][JA]) {
     constexpr TpOrder<NI, J> O{};
     constexpr int M = NI * J, F = NI + J;
-    constexpr int G = M > 1 ? M / 2 : 1;     // pairs of products of a step
+    constexpr int G = M > 0 ? M / 4 : 1;     // fours of products of a step
+    static_assert(M % 4 == 0);
     const int lane = threadIdx.x % WAVE_SIZE;
-    const int l32 = lane & 31;
-    const int half = lane >> 5;
+    const int l16 = lane & 15;
+    const int l4 = lane >> 4;
     const int wm = wave / WGN, wn = wave % WGN;
-    int at[4];   // byte places of this lane's fragments of a group
+    int at[2];   // byte places of this lane's fragments of a group
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      at[k] = l32 * TP_ROW + ((k * 2 + half) ^ tp_swap(l32)) * 16;
+    for (int k = 0; k < 2; ++k)
+      at[k] = l16 * TP_ROW + ((k * 4 + l4) ^ tp_swap(l16)) * 16;
     char* const wlds = lds + PA * AB;
-    const char* const a0 = lds + wm * 32 * TP_ROW;
     const char* const w0 = wlds + wn * WW * TP_ROW;
     auto fa = [&](int s, int i, int place) {
       fill_a(s, i, lds + place * AB + (wave * FA + i) * TP_FILL);
@@ -138,32 +151,31 @@ struct TileProduct {
     s16x8 af[2][J > 0 ? J : 1], wf[2][NI];
     auto read = [&](int to, int ap, int wp, int k, int r) {
       if constexpr (J > 0) {
+        const int x = O.ix[r];
         if (O.w[r])
-          wf[to][O.ix[r]] = *reinterpret_cast<const s16x8*>(
-              w0 + wp * WB + O.ix[r] * 32 * TP_ROW + at[k]);
+          wf[to][x] = *reinterpret_cast<const s16x8*>(
+              w0 + wp * WB + x * 16 * TP_ROW + at[k]);
         else
-          af[to][O.ix[r]] = *reinterpret_cast<const s16x8*>(
-              a0 + ap * AB + O.ix[r] * WGM * 32 * TP_ROW + at[k]);
+          af[to][x] = *reinterpret_cast<const s16x8*>(
+              lds + ap * AB + row_of(x, wm) * TP_ROW + at[k]);
       }
     };
-    // Products from fragments `cur`; between them READS of the next step's
-    // fragments, by the pair in which they come (all in the first half where
-    // a barrier follows), and n fills.
-    auto step = [&](const int cur, const bool soon, auto reads, const int n,
-                    auto fills) {
+    // Products from fragments `cur`; between them, all in the first half, the
+    // reads of the next step's fragments, and n fills.
+    auto step = [&](const int cur, auto reads, const int n, auto fills) {
 #pragma unroll
       for (int g = 0; g < G; ++g) {
 #pragma unroll
         for (int r = 0; r < F; ++r)
-          if (r * G / (soon ? 2 * F : F) == g) reads(r);
+          if (r * G / (2 * F) == g) reads(r);
 #pragma unroll
         for (int f = 0; f < n; ++f)
           if ((2 * f + 1) * G / (2 * n) == g) fills(f);
-        if constexpr (M > 1) {
+        if constexpr (M > 0) {
 #pragma unroll
-          for (int q = 2 * g; q < 2 * g + 2; ++q)
-            acc[O.i[q]][O.j[q]] = mfma32<Tag>(
-                wf[cur][O.i[q]], af[cur][O.j[q]], acc[O.i[q]][O.j[q]]);
+          for (int q = 4 * g; q < 4 * g + 4; ++q)
+            mfma16_acc<Tag>(acc[O.i[q]][O.j[q]], wf[cur][O.i[q]],
+                            af[cur][O.j[q]]);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -172,69 +184,59 @@ struct TileProduct {
 #pragma unroll
       for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int j = 0; j < J; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        for (int j = 0; j < J; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      acc_fence(acc);
     }
-    // In the order in which the loop goes on: what it waits for is counted.
-    constexpr int AHEAD_A = FW + (PA - 2) * (FA + FW);
+    // Stage s fills weights of stage s + PW - 1 in its first step and rows of
+    // stage s + PA in its second, as long as there are any; the wait between
+    // them for the next stage leaves what was filled after it.
+    constexpr int AHEAD_A = (PA - 1) * FW + (PA - 2) * FA;
     constexpr int AHEAD_W = (PW - 2) * (FA + FW);
     constexpr int AHEAD = AHEAD_A < AHEAD_W ? AHEAD_A : AHEAD_W;
     static_assert(AHEAD + FA < 64);
+    constexpr int LAST = PA > PW - 1 ? PA : PW - 1;
 #pragma unroll
-    for (int t = 1 - PW; t < 0; ++t) {
-      if (t + PA - 1 >= 0 && t + PA - 1 < steps) {
-#pragma unroll
-        for (int i = t + PA - 1 == 0 ? 0 : FA / 2; i < FA; ++i)
-          fa(t + PA - 1, i, t + PA - 1);
-      }
-      if (t + PW - 1 < steps) {
+    for (int t = -LAST - 1; t < 0; ++t) {
+      if (t + PW - 1 >= 0 && t + PW - 1 < steps) {
 #pragma unroll
         for (int i = 0; i < FW; ++i) fw(t + PW - 1, i, t + PW - 1);
       }
-      if (t + PA >= 1 && t + PA < steps) {
+      if (t + PA >= 0 && t + PA < steps) {
 #pragma unroll
-        for (int i = 0; i < FA / 2; ++i) fa(t + PA, i, (t + PA) % PA);
+        for (int i = 0; i < FA; ++i) fa(t + PA, i, t + PA);
       }
     }
-    if (steps >= PW) lds_fill_wait<AHEAD>();
+    if (steps >= PW) lds_fill_wait<AHEAD + FA>();
     else lds_fill_wait();
     lds_barrier();
 #pragma unroll
     for (int r = 0; r < F; ++r) read(0, 0, 0, 0, r);
     int ap = 0, wp = 0;
-    // MORE: fills of whole stages go on.
+    // MORE: fills go on in the whole stage.
     auto stage = [&](const int s, auto more) {
       constexpr bool MORE = decltype(more)::value;
-      const int an = ap == PA - 1 ? 0 : ap + 1, al = ap == 0 ? PA - 1 : ap - 1;
+      const int an = ap == PA - 1 ? 0 : ap + 1;
       const int wn_ = wp == PW - 1 ? 0 : wp + 1, wl = wp == 0 ? PW - 1 : wp - 1;
-      step(0, false, [&](int r) { read(1, ap, wp, 1, r); }, FA / 2, [&](int f) {
-        if (MORE || s + PA - 1 < steps) fa(s + PA - 1, FA / 2 + f, al);
-      });
-      step(1, false, [&](int r) { read(0, ap, wp, 2, r); }, FW / 2, [&](int f) {
+      step(0, [&](int r) { read(1, ap, wp, 1, r); }, FW, [&](int f) {
         if (MORE || s + PW - 1 < steps) fw(s + PW - 1, f, wl);
-      });
-      step(0, true, [&](int r) { read(1, ap, wp, 3, r); }, FW / 2, [&](int f) {
-        if (MORE || s + PW - 1 < steps) fw(s + PW - 1, FW / 2 + f, wl);
       });
       // The next stage has landed when only what was filled after it is
       // under way; past the barrier no wave reads this one again.
       if constexpr (MORE) lds_fill_wait<AHEAD>();
       else wait_but<PW - 2>(steps - 2 - s);
       lds_barrier();
-      step(1, true, [&](int r) { read(0, an, wn_, 0, r); }, FA / 2,
-           [&](int f) {
-             if (MORE || s + PA < steps) fa(s + PA, f, ap);
-           });
+      step(1, [&](int r) { read(0, an, wn_, 0, r); }, FA, [&](int f) {
+        if (MORE || s + PA < steps) fa(s + PA, f, ap);
+      });
       ap = an;
       wp = wn_;
     };
-    constexpr int LAST = PA > PW - 1 ? PA : PW - 1;   // stage MORE looks ahead
     int s = 0;
 #pragma unroll 1
     for (; s + LAST < steps; ++s) stage(s, std::true_type{});
 #pragma unroll 1
     for (; s < steps; ++s) stage(s, std::false_type{});
+    if constexpr (J > 0) acc_fence(acc);
   }
 };
 
