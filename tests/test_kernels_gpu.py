@@ -346,6 +346,29 @@ def test_prefill_attention_edges(hd, group, dtype, cache_dtype, window,
     assert_close(out, expect, atol=atol, rtol=atol / 4)
 
 
+@pytest.mark.parametrize("hd,cache_dtype", [
+    (64, torch.bfloat16), (128, torch.bfloat16), (256, torch.bfloat16),
+    (64, torch.float8_e4m3fn), (128, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_prefill_attention_tile_counts(hd, cache_dtype, window):
+    """One to seven key tiles a workgroup, odd and even, from an odd and an
+    even tile on. Tolerance as above."""
+    hip = _hip()
+    ctx = [64 * i - 3 for i in range(1, 8)] + [64 * i + 2 for i in range(1, 8)]
+    q_lens = [1 + i % 3 for i in range(len(ctx))]
+    n = len(ctx)
+    q, cache, bt, qsl, sl = _make_paged(n, q_lens, ctx, 8, 2, D=hd)
+    cache = cache.to(cache_dtype)
+    out = hip.attention_unified(q, cache, bt, qsl, sl, hd**-0.5,
+                                num_decodes=0, max_seq_len=max(ctx),
+                                max_query_len=max(q_lens),
+                                sliding_window=window)
+    expect = ref.attention_unified(q.float(), cache.float(), bt, qsl, sl,
+                                   hd**-0.5, sliding_window=window)
+    atol = 3 * 4 * 2**-8
+    assert_close(out, expect, atol=atol, rtol=atol / 4)
+
+
 def test_model_forward_matches_cpu_reference():
     """Tiny Llama forward on GPU (bf16, HIP kernels) vs CPU fp32 torch
     reference: logits must be directionally identical (cosine > 0.99)."""

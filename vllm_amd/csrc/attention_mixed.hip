@@ -30,10 +30,10 @@ constexpr int max_lds(int a, int b) { return a > b ? a : b; }
 // group of four.
 //
 // 32/8 heads of 128, us one after the other and so: 96 rows x 100..4000
-// keys and portions of 400, 700 and 1001 tokens after 0 to 4096 311 -> 242;
-// 200 rows x 100..2000 and 2 of 100 and 200 tokens 154 -> 145; 16 rows x
-// 100..300 and 30 of 17..200 33.9 -> 29.1; 32/4 heads, 32 rows x 2000..4000
-// and 4 of 1000..2000 159 -> 133 (runs of 256 tiles and 256 rows in turn were
+// keys and portions of 400, 700 and 1001 tokens after 0 to 4096 291 -> 208;
+// 200 rows x 100..2000 and 2 of 100 and 200 tokens 152 -> 140; 16 rows x
+// 100..300 and 30 of 17..200 30.7 -> 27.9; 32/4 heads, 32 rows x 2000..4000
+// and 4 of 1000..2000 140 -> 124 (runs of 256 tiles and 256 rows in turn were
 // a fifth slower there).
 struct Mix { int tiles, rows, spread, num_prefills; };
 

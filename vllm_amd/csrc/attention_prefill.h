@@ -2,12 +2,19 @@
 // MI355X (gfx950, CDNA4): the work of a workgroup (kernels:
 // attention_prefill.hip, and attention_mixed.hip beside decode rows).
 //
-// What bounds it: the matrix cores, with the exponentials and LDS reads
-// close behind (per 32 x 64 scores of a wave: 1024 cycles of MFMA at
-// D=128, about as many of vector ALU and, over four waves, of LDS). So:
+// What bounds it: the matrix cores, with the exponentials close behind (per
+// 32 x 64 scores of a wave at D=128: 1024 cycles of MFMA, about as many of
+// vector ALU, half as many of LDS), and over milliseconds the chip's power
+// (1.75 GHz). So:
 //   - 32x32x16 MFMA, four waves of 32 rows: half the LDS bytes per flop
-//     of 16-row fragments. Two workgroups per CU fit at D=128, so one
-//     wave's softmax runs under another's products.
+//     of 16-row fragments. Two workgroups per CU fit at D=128.
+//   - A wave's vector work runs under its own products: the maximum of a
+//     tile's scores under the first half of the next tile's, its weights
+//     under the second half and under the results of the weights before them
+//     (one after the other, two waves a SIMD: matrix cores 44 % and vector ALU
+//     49 % of the cycles, hardly any at once; now 59 %). Scheduling barriers
+//     pin the order; other shares of products a group, 3 to 8 fragments read
+//     ahead and wave priorities measured the same.
 //   - The rows of a tile are (token, query head) pairs of ONE KV head:
 //     the heads of a group share every K/V tile they read, the causal
 //     edge of a tile is only 128 / group tokens wide, and a short
@@ -19,25 +26,31 @@
 //     the keys in the order in which the score registers hold them.
 //   - V^T fragments come from transposing LDS reads of the row-major
 //     tile: no scatter when the tile is stored.
-//   - K/V tiles are double-buffered: the tile after next is in flight in
-//     registers while two are in LDS, one barrier per tile.
+//   - K and V have two places each in LDS and are filled straight from the
+//     cache (8-bit ones by way of registers, which widen): V a tile ahead, K
+//     two, one barrier per tile.
+//   - Tiles are taken in pairs, so that scores stay in the registers where
+//     they were formed. Of an even number the last takes scores that nobody
+//     asked for with it; forms of their own for it needed scratch and made
+//     short prompts wait for code (8192 tokens 552 us, 64 short ones 57).
 //   - The 16-bit weights are summed as they are rounded (one dot product
 //     instruction a pair), so that their rounding cancels in the quotient,
 //     and the row's largest weight is exactly one: accumulators are
 //     rescaled whenever a maximum moves. Letting it grow by 2^8 first
 //     would save 3 % and raise the distance to 64-bit results by 2 to 7 %
 //     (now 1 % below that of unrounded sums).
-//   - Results are stored 16 B a lane (8 B: 59 us for the short prompts
-//     below, 53 now).
-// Against 16x16x32 fragments on 16-row waves with V scattered into LDS:
-// one 8192-token prompt, 32/8 heads of 128: 4.70 -> 0.67 ms (820 TFLOP/s);
-// 64 prompts of 33..223 tokens: 207 -> 54 us; 4 x 2048 tokens, 16/8 heads
-// of 256: 2.59 -> 0.26 ms.
+//   - Results are stored 16 B a lane.
+// Scores, weights and results one after the other -> so, us, 32/8 heads of
+// 128: one prompt of 8192 tokens 615 -> 527 (1.04 PFLOP/s), with an 8-bit cache
+// 599 -> 551; 2048 63 -> 52; 512 after 1536 to 15872, 4 such 410 -> 312; 64 of
+// 33..223 48.7 -> 44.6; 4 x 2048 tokens, 16/8 heads of 256, 284 -> 211.
 //
 // Role of the reference's triton_unified_attention.py:179 (prefill side)
 // and prefix_prefill.py.
 
 #pragma once
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -117,10 +130,6 @@ DEVINL void prefill_tile(const PrefillArgs<CTag>& a, const int kvh,
   const int l32 = lane & 31;
   const int half = lane >> 5;
 
-  // [tok][d], chunks moved; [tok][d], segments moved
-  auto* k_lds = reinterpret_cast<short(*)[TILE]>(lds);
-  auto* v_lds = reinterpret_cast<short(*)[TILE]>(lds + 2 * TILE * 2);
-
   // --- this lane's row: token and head --------------------------------
   const int row = row0 + wave * 32 + l32;
   const int row_safe = min(row, rows - 1);
@@ -158,112 +167,170 @@ DEVINL void prefill_tile(const PrefillArgs<CTag>& a, const int kvh,
   const int kt_end = last_pos / KVTILE + 1;
 
   const int* bt = a.block_table + (int64_t)req * a.max_blocks_per_req;
-  i32x4 kr[LD], vr[LD];
-  auto load = [&](int phys) {
-    const elem* src =
-        a.kv_cache + ((int64_t)phys * num_kv_heads + kvh) * (KVTILE * HD);
+  auto block_of = [&](int kt) { return load_uniform(bt + min(kt, kt_end - 1)); };
+
+  // A tile of keys (PLANE 0) or values (1) on its way to a place in LDS: fills,
+  // or, where it has to be widened, registers until land().
+  i32x4 kv_reg[2][FP8 ? LD : 1];
+  auto fetch = [&](auto plane, int phys, int place) {
+    constexpr int PLANE = decltype(plane)::value;
+    const elem* src = a.kv_cache + PLANE * kv_plane_stride +
+                      ((int64_t)phys * num_kv_heads + kvh) * TILE;
 #pragma unroll
     for (int i = 0; i < LD; ++i) {
-      kr[i] = *reinterpret_cast<const i32x4*>(
-          src + (i * PF_BLOCK + threadIdx.x) * EPV);
-      vr[i] = *reinterpret_cast<const i32x4*>(
-          src + kv_plane_stride + (i * PF_BLOCK + threadIdx.x) * EPV);
+      if constexpr (FP8)
+        kv_reg[PLANE][i] = *reinterpret_cast<const i32x4*>(
+            src + (i * PF_BLOCK + threadIdx.x) * EPV);
+      else {
+        // What lies in LDS where this lane's 16 B land.
+        constexpr int ROWS = PF_BLOCK * 8 / HD;   // of a piece
+        const int r = threadIdx.x * 8 / HD, c = threadIdx.x * 8 % HD / 8;
+        const int at = PLANE == 0 ? k_chunk<HD>(i * ROWS + r, c) * 8
+                                  : v_seg<HD>(i * ROWS + r, c >> 1) * 16 +
+                                        (c & 1) * 8;
+        lds_fill16(src + i * PF_BLOCK * EPV, (uint32_t)(r * HD + at) * 2,
+                   lds + (PLANE * 2 + place) * TILE * 2 +
+                       (i * PF_BLOCK + wave * WAVE_SIZE) * 16);
+      }
     }
   };
-  auto store = [&](int kt) {
-    const int b = kt & 1;
-    if (kt * KVTILE + KVTILE > ctx) {
-      // Rows no token has been written to yet may hold anything, and
-      // their zero weight does not stop a NaN.
+  auto land = [&](auto plane, int kt, int place) {
+    constexpr int PLANE = decltype(plane)::value;
+    // Values of rows no token has been written to yet may hold anything, and
+    // their zero weight does not stop a NaN.
+    const bool edge = PLANE == 1 && kt * KVTILE + KVTILE > ctx;
+    short* to = reinterpret_cast<short*>(lds) + (PLANE * 2 + place) * TILE;
+    if constexpr (FP8) {
 #pragma unroll
       for (int i = 0; i < LD; ++i) {
-        const int key = kt * KVTILE + (i * PF_BLOCK + threadIdx.x) * EPV / HD;
+        const int e = (i * PF_BLOCK + threadIdx.x) * EPV;
+        const int r = e / HD;
+        const int c = (e % HD) / 8;
+        i32x4 v = kv_reg[PLANE][i];
+        if (edge) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) vr[i][j] = key < ctx ? vr[i][j] : 0;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < LD; ++i) {
-      const int e = (i * PF_BLOCK + threadIdx.x) * EPV;
-      const int r = e / HD;
-      const int c = (e % HD) / 8;
-#pragma unroll
-      for (int h = 0; h < EPV / 8; ++h) {
-        i32x4 kv, vv;
-        if constexpr (FP8) {
-          const int2 k0 = fp8x4_widen<Tag>(kr[i][h * 2]);
-          const int2 k1 = fp8x4_widen<Tag>(kr[i][h * 2 + 1]);
-          kv = i32x4{k0.x, k0.y, k1.x, k1.y};
-          const int2 x = fp8x4_widen<Tag>(vr[i][h * 2]);
-          const int2 y = fp8x4_widen<Tag>(vr[i][h * 2 + 1]);
-          vv = i32x4{x.x, x.y, y.x, y.y};
-        } else {
-          kv = kr[i];
-          vv = vr[i];
+          for (int j = 0; j < 4; ++j) v[j] = kt * KVTILE + r < ctx ? v[j] : 0;
         }
-        *reinterpret_cast<i32x4*>(
-            &k_lds[b][r * HD + k_chunk<HD>(r, c + h) * 8]) = kv;
-        *reinterpret_cast<i32x4*>(
-            &v_lds[b][r * HD + v_seg<HD>(r, (c + h) >> 1) * 16 +
-                      ((c + h) & 1) * 8]) = vv;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int2 x = fp8x4_widen<Tag>(v[h * 2]);
+          const int2 y = fp8x4_widen<Tag>(v[h * 2 + 1]);
+          const int at = PLANE == 0 ? k_chunk<HD>(r, c + h) * 8
+                                    : v_seg<HD>(r, (c + h) >> 1) * 16 +
+                                          ((c + h) & 1) * 8;
+          *reinterpret_cast<i32x4*>(to + r * HD + at) =
+              i32x4{x.x, x.y, y.x, y.y};
+        }
+      }
+    } else if (edge) {
+#pragma unroll
+      for (int i = 0; i < LD; ++i) {
+        const int e = (i * PF_BLOCK + threadIdx.x) * EPV;
+        if (kt * KVTILE + e / HD >= ctx)
+          *reinterpret_cast<i32x4*>(to + e) = i32x4{0, 0, 0, 0};
       }
     }
   };
-
-  load(load_uniform(bt + kt0));
-  store(kt0);
-  if (kt0 + 1 < kt_end) load(load_uniform(bt + kt0 + 1));
-  int phys = load_uniform(bt + min(kt0 + 2, kt_end - 1));
-  __syncthreads();
-
-  for (int kt = kt0; kt < kt_end; ++kt) {
-    const int b = kt & 1;
-    // --- S^T: 64 keys x 32 rows -----------------------------------------
-    f32x16 s[2];
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
-      const int key = n * 32 + l32;
-#pragma unroll
-      for (int kk = 0; kk < KF; ++kk) {
-        const s16x8 f = *reinterpret_cast<const s16x8*>(
-            &k_lds[b][key * HD + k_chunk<HD>(key, kk * 2 + half) * 8]);
-        s[n] = mfma32<Tag>(f, qf[kk], s[n]);
-      }
+  // All fills of this wave have landed (what follows stays behind them).
+  auto landed = [&] {
+    if constexpr (!FP8) {
+      lds_fill_wait();
+      asm volatile("" ::: "memory");
     }
-    // The other buffer was last read before the barrier that opened this
-    // iteration.
-    if (kt + 1 < kt_end) store(kt + 1);
-    if (kt + 2 < kt_end) {
-      load(phys);
-      phys = load_uniform(bt + min(kt + 3, kt_end - 1));
-    }
+  };
+  constexpr std::integral_constant<int, 0> KEYS{};
+  constexpr std::integral_constant<int, 1> VALUES{};
 
+  // Products of a step in their order: the first and the second 32 keys of the
+  // next tile's scores, then the four chunks of 16 keys of this one's results.
+  constexpr int QK = 2 * KF, ALL = QK + 4 * DS;
+  constexpr int AHEAD = 4;                       // fragments read ahead
+  int k_at[KF], v_at[DS];   // first fragments of a tile, in its bytes
+#pragma unroll
+  for (int kk = 0; kk < KF; ++kk)
+    k_at[kk] = (l32 * HD + k_chunk<HD>(l32, kk * 2 + half) * 8) * 2;
+#pragma unroll
+  for (int i = 0; i < DS; ++i) {
+    const int r = half * 4 + ((lane & 15) >> 2);
+    v_at[i] = (r * HD + v_seg<HD>(r, i * 2 + ((lane >> 4) & 1)) * 16 +
+               (lane & 3) * 4) * 2;
+  }
+  auto fragment = [&](int m, int k_place, int v_place) -> s16x8 {
+    if (m < QK)   // (the moves of rows 16 and 32 apart are the same)
+      return *reinterpret_cast<const s16x8*>(
+          lds + k_place * TILE * 2 + m / KF * 32 * HD * 2 + k_at[m % KF]);
+    const char* v = lds + (2 + v_place) * TILE * 2 +
+                    (m - QK) / DS * 16 * HD * 2 + v_at[(m - QK) % DS];
+    const s16x4 c0 = lds_read_tr(v), c1 = lds_read_tr(v + 8 * HD * 2);
+    return __builtin_shufflevector(c0, c1, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  const f32x16 zero = {};
+  const int first = block_of(kt0);
+  int next = block_of(kt0 + 1), second = block_of(kt0 + 2);
+
+  // One tile: its scores s become weights and results, between the products of
+  // the next one's scores t (MORE; where there is none, of what lies there).
+  auto tile_step = [&](const int kt, f32x16 (&s)[2], f32x16 (&t)[2],
+                       const int place, auto more) {
+    constexpr bool MORE = decltype(more)::value;
+    constexpr int FIRST = MORE ? 0 : QK;
+    if constexpr (MORE) {
+      // (Of either place the last read lies before the barrier.)
+      if (kt + 1 < kt_end) fetch(VALUES, next, 1 - place);
+      if (kt + 2 < kt_end) fetch(KEYS, second, place);
+      next = second;
+      second = block_of(kt + 3);
+    }
+    s16x8 frag[AHEAD], pf[4];
+    auto read = [&](int m) {
+      if (m >= FIRST && m < ALL)
+        frag[m % AHEAD] = fragment(m, 1 - place, place);
+    };
+    auto product = [&](int m) {
+      if (m < QK)
+        t[m / KF] = mfma32<Tag>(frag[m % AHEAD], qf[m % KF],
+                                m % KF == 0 ? zero : t[m / KF]);
+      else
+        o[(m - QK) % DS] = mfma32<Tag>(frag[m % AHEAD], pf[(m - QK) / DS],
+                                       o[(m - QK) % DS]);
+      read(m + AHEAD);
+    };
     // --- mask, only where the tile meets an edge -------------------------
     // Register r of subtile n is key n*32 + 8*(r/4) + 4*half + r%4.
     const int key_base = kt * KVTILE + half * 4;
     if (kt * KVTILE + KVTILE - 1 > first_pos ||
         (sliding_window > 0 && kt * KVTILE <= last_pos - sliding_window)) {
-      const int lo = sliding_window > 0 ? qpos - sliding_window : -1;
+      const int hi = qpos - key_base;
+      const int lo = sliding_window > 0 ? hi - sliding_window : -1;
 #pragma unroll
       for (int n = 0; n < 2; ++n)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int key = key_base + n * 32 + 8 * (r >> 2) + (r & 3);
-          s[n][r] = (key <= qpos) & (key > lo) ? s[n][r] : PF_NEG;
+          const int key = n * 32 + 8 * (r >> 2) + (r & 3);
+          s[n][r] = key <= hi && key > lo ? s[n][r] : PF_NEG;
         }
     }
+#pragma unroll
+    for (int m = FIRST; m < FIRST + AHEAD; ++m) read(m);
 
     // --- running softmax --------------------------------------------------
     // med3 with +inf is a maximum that the compiler fuses in threes (fmaxf
     // first quiets each score: 37 more instructions a tile, 2 %).
     float mx = PF_NEG;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      mx = __builtin_amdgcn_fmed3f(mx, s[0][r], INFINITY);
-      mx = __builtin_amdgcn_fmed3f(mx, s[1][r], INFINITY);
+    for (int g = 0; g < 8; ++g) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = g * 2; r < g * 2 + 2; ++r) {
+        mx = __builtin_amdgcn_fmed3f(mx, s[0][r], INFINITY);
+        mx = __builtin_amdgcn_fmed3f(mx, s[1][r], INFINITY);
+      }
+      if constexpr (MORE) {
+#pragma unroll
+        for (int m = KF * g / 8; m < KF * (g + 1) / 8; ++m) product(m);
+      }
     }
+    __builtin_amdgcn_sched_barrier(0);
     mx = half_max(mx);
     if (__any(mx > m_run)) {
       const float m_new = fmaxf(m_run, mx);
@@ -275,12 +342,18 @@ DEVINL void prefill_tile(const PrefillArgs<CTag>& a, const int kvh,
     }
     // A row that has seen no key yet (a window's first tile) weighs none.
     const float shift = m_run > PF_NEG ? -m_run * scale_log2 : 0.f;
-    s16x8 pf[4];
+
+    // --- weights, and O^T += V^T P^T ---------------------------------------
+    // Half a chunk of weights a group, then as many products as weights are
+    // there for.
+    constexpr int TO[9] = {8, 11, 14, 17, 20, 22, 24, 26, 28};
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      i32x4 pk;
+    for (int g = 0; g < 8; ++g) {
+      __builtin_amdgcn_sched_barrier(0);
+      const int c = g / 2;
+      i32x4 pk = g % 2 ? __builtin_bit_cast(i32x4, pf[c]) : i32x4{};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = g % 2 * 2; j < g % 2 * 2 + 2; ++j) {
         const int r = (c & 1) * 8 + j * 2;
         const float p0 = __builtin_amdgcn_exp2f(
             __builtin_fmaf(s[c >> 1][r], scale_log2, shift));
@@ -290,28 +363,44 @@ DEVINL void prefill_tile(const PrefillArgs<CTag>& a, const int kvh,
         l_run = add_pair<Tag>(pk[j], l_run);
       }
       pf[c] = __builtin_bit_cast(s16x8, pk);
+      const int m0 = TO[g] * KF / 8, m1 = TO[g + 1] * KF / 8;
+#pragma unroll
+      for (int m = m0; m < m1; ++m)
+        if (m >= FIRST) product(m);
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = TO[8] * KF / 8; m < ALL; ++m) product(m);
+    if constexpr (MORE) {
+      landed();
+      if (kt + 1 < kt_end) land(VALUES, kt + 1, 1 - place);
+      if (kt + 2 < kt_end) land(KEYS, kt + 2, place);
+    }
+    lds_barrier();
+  };
 
-    // --- O^T += V^T P^T ----------------------------------------------------
-    const int vrow = half * 4 + ((lane & 15) >> 2);
-    const int vcol = (lane & 3) * 4;
+  fetch(KEYS, first, 0);
+  fetch(VALUES, first, 0);
+  if (!FP8 && kt0 + 1 < kt_end) fetch(KEYS, next, 1);
+  landed();
+  land(KEYS, kt0, 0);
+  land(VALUES, kt0, 0);
+  if (FP8 && kt0 + 1 < kt_end) fetch(KEYS, next, 1);
+  lds_barrier();
+  f32x16 sa[2], sb[2];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int r0 = c * 16 + vrow;
-#pragma unroll
-      for (int i = 0; i < DS; ++i) {
-        const int seg = i * 2 + ((lane >> 4) & 1);
-        const s16x4 c0 = lds_read_tr(
-            &v_lds[b][r0 * HD + v_seg<HD>(r0, seg) * 16 + vcol]);
-        const s16x4 c1 = lds_read_tr(
-            &v_lds[b][(r0 + 8) * HD + v_seg<HD>(r0 + 8, seg) * 16 + vcol]);
-        o[i] = mfma32<Tag>(
-            __builtin_shufflevector(c0, c1, 0, 1, 2, 3, 4, 5, 6, 7), pf[c],
-            o[i]);
-      }
-    }
-    __syncthreads();
+  for (int m = 0; m < QK; ++m)
+    sa[m / KF] = mfma32<Tag>(fragment(m, 0, 0), qf[m % KF],
+                             m % KF == 0 ? zero : sa[m / KF]);
+  if (FP8 && kt0 + 1 < kt_end) land(KEYS, kt0 + 1, 1);
+  lds_barrier();   // the first keys' place is free
+  int kt = kt0;
+#pragma unroll 1
+  for (; kt + 1 < kt_end; kt += 2) {
+    tile_step(kt, sa, sb, 0, std::true_type{});
+    tile_step(kt + 1, sb, sa, 1, std::true_type{});
   }
+  if (kt < kt_end) tile_step(kt, sa, sb, 0, std::false_type{});
 
   // --- epilogue: column l32 is this lane's row ---------------------------
   l_run += __shfl_xor(l_run, 32, 64);

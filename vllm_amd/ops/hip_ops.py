@@ -173,12 +173,12 @@ def _attention_mixes(rows, reqs, tokens, heads, head_dim, kv_heads, parts,
     launch), heads that one of the two kernels does not take, nor grids past
     65535 units. Nor rows that read (5 TB/s) less than a twentieth of the time
     that the portions may take (0.8 PFLOP/s): they have hardly any effect (1
-    row x 1000 keys and 8000 tokens 587 us in turn, 588 in one launch). A
-    third where several portions come after more cached tokens than they are
-    long: their tiles are all of one length and fill the chip in step, which
-    rows among them disturb (4 portions of 1000 after 4000 beside 8 x 4000
-    keys 386 and 415 us, 16/2 heads 202 and 234; beside 64 x 2000, 8/8 heads,
-    215 and 181)."""
+    row x 1000 keys and 8000 tokens 518 us in turn, 522 in one launch). A
+    third where portions come after more cached tokens than they are long:
+    their tiles are all of one length and fill the chip in step, which rows
+    among them disturb (4 portions of 1000 after 4000 beside 8 x 4000 keys,
+    16/2 heads, 177 and 200 us, one of 2000 after 6000 beside 32 x 1000, 32/8
+    heads, 265 and 307; the 4 beside 64 x 2000, 8/8 heads, 182 and 144)."""
     if not 0 < rows < reqs or head_dim not in (64, 128):
         return False
     if heads % kv_heads or heads // kv_heads > 8:
@@ -191,7 +191,7 @@ def _attention_mixes(rows, reqs, tokens, heads, head_dim, kv_heads, parts,
     read_us = rows * span * kv_heads * head_dim * 2 * kv_bytes / 5e6
     # (Cached tokens of portions are known only where the longest context is
     # not a row's.)
-    alike = (reqs - rows > 1 and max_seq_len > max_decode_len
+    alike = (max_seq_len > max_decode_len
              and max_seq_len >= 2 * max_query_len)
     keys = max_seq_len - max_query_len / 2 if alike else max_seq_len / 2
     if window > 0:
