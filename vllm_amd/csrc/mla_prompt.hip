@@ -20,7 +20,8 @@
 // two, which is one unless their largest is below 1/4 or from 2^15.
 // 128 heads, prompts of 300, 1300 and 2301 tokens: 2.02 -> 0.63 ms with
 // everything between queries and results (latent form before); one of
-// 8192 13.1 -> 3.80 ms, four of 2048 4.48 -> 1.36 ms.
+// 8192 13.1 -> 3.80 ms, four of 2048 4.48 -> 1.36 ms (before the last change to
+// mla_prompt_kernel's order, which takes 7 % off it).
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
@@ -267,18 +268,20 @@ void mla_expand_kernel(short* __restrict__ k_out,   // [heads, reqs, S, D] fp16
 // keys of one token) and O^T = V^T P^T with V^T by transposing reads, as
 // for ordinary heads; per tile 24 + 32 products a wave (weights are hi + lo),
 // 40 KB of fragment reads and 32 exponentials a lane, so the matrix cores
-// bound it. Two tiles alternate, filled straight from global memory, one
-// barrier a tile: 80 KB, two workgroups a CU, one's softmax under the
-// other's products. Accumulators are rescaled when a maximum has grown by
-// 2^8. 3901 tokens as above: 0.50 ms, 820 TFLOP/s with both halves of the
-// weights. All tiles of a head run on one XCD, late ones (most keys) first;
+// bound it. As there (attention_prefill.h), a tile's maximum and weights are
+// taken between the products of the next tile's scores and of its own results;
+// two places of keys and of values, filled straight from global memory, one
+// barrier a tile: 80 KB, two workgroups a CU. Accumulators are rescaled when a
+// maximum has grown by 2^8. 3901 tokens as above: 0.45 ms, 910 TFLOP/s with
+// both halves of the weights (scores, weights and results one after the other
+// 0.485). All tiles of a head run on one XCD, late ones (most keys) first;
 // where fewer than eight heads run at a time, a head's tiles go to several.
 constexpr int PA_M = 128;
 constexpr int PA_KEYS = 64;
 constexpr int PA_THREADS = 4 * WAVE_SIZE;
 constexpr int PA_K = PA_KEYS * D * 2;          // bytes: keys, values
 constexpr int PA_PE = PA_KEYS * ROPE * 2;      // rotary parts
-constexpr int PA_BUF = 2 * PA_K + PA_PE;
+constexpr int PA_KEY_BYTES = PA_K + PA_PE;     // two places, then two of values
 
 DEVINL float half_max(float x) {
   const auto sw = __builtin_amdgcn_permlane32_swap(
@@ -315,7 +318,7 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
   const int pos0 = ctx - ql;             // of the portion's first token
   const int row0 = tile * PA_M;
 
-  __shared__ __align__(16) char lds[2 * PA_BUF];
+  __shared__ __align__(16) char lds[2 * (PA_KEY_BYTES + PA_K)];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
   const int l32 = lane & 31;
@@ -375,25 +378,37 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
   const short* pb = pe + (int64_t)r * S * ROPE;
   // Rows past the context repeat the last one: their weight is zero, and
   // what was never written could be NaN.
-  auto fill = [&](int kt, int buf) {
-    char* dst = lds + buf * PA_BUF;
+  auto fill_keys = [&](int kt, int place) {
+    char* dst = lds + place * PA_KEY_BYTES;
     const int last = ctx - 1 - kt * PA_KEYS;
     const int64_t t0 = (int64_t)kt * PA_KEYS;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = (wave * 4 + i) * 4 + (lane >> 4);
-      const int64_t at = (t0 + min(row, last)) * D;
-      lds_fill16(kb + at + chunk256(row, lane & 15) * 8,
+      lds_fill16(kb + t0 * D,
+                 (uint32_t)(min(row, last) * D + chunk256(row, lane & 15) * 8) *
+                     2,
                  dst + (wave * 4 + i) * 1024);
-      lds_fill16(vb + at + seg256_chunk(row, lane & 15) * 8,
-                 dst + PA_K + (wave * 4 + i) * 1024);
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int row = (wave * 2 + i) * 8 + (lane >> 3);
-      lds_fill16(pb + (t0 + min(row, last)) * ROPE +
-                     chunk128(row, lane & 7) * 8,
-                 dst + 2 * PA_K + (wave * 2 + i) * 1024);
+      lds_fill16(pb + t0 * ROPE,
+                 (uint32_t)(min(row, last) * ROPE +
+                            chunk128(row, lane & 7) * 8) * 2,
+                 dst + PA_K + (wave * 2 + i) * 1024);
+    }
+  };
+  auto fill_values = [&](int kt, int place) {
+    char* dst = lds + 2 * PA_KEY_BYTES + place * PA_K;
+    const int last = ctx - 1 - kt * PA_KEYS;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = (wave * 4 + i) * 4 + (lane >> 4);
+      lds_fill16(vb + (int64_t)kt * PA_KEYS * D,
+                 (uint32_t)(min(row, last) * D +
+                            seg256_chunk(row, lane & 15) * 8) * 2,
+                 dst + (wave * 4 + i) * 1024);
     }
   };
 
@@ -406,98 +421,174 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
 
   const int wave_first = pos0 + row0 + wave * 32;
   const int wave_last = pos0 + min(row0 + wave * 32 + 31, ql - 1);
-  fill(0, 0);
+
+  // Fragments of a step in the order of their products: the first and the
+  // second 32 keys of the next tile's scores (one product each), then the four
+  // chunks of 16 keys of this one's results (two, by the weights' parts).
+  constexpr int KF = (D + ROPE) / 16, DS = D / 32;
+  constexpr int QK = 2 * KF, ALL = QK + 4 * DS;
+  constexpr int AHEAD = 4;   // fragments read ahead
+  int k_at[KF], v_at[DS];    // first fragments of a tile, in its bytes
+#pragma unroll
+  for (int kk = 0; kk < D / 16; ++kk)
+    k_at[kk] = l32 * 256 + chunk256(l32, kk * 2 + half) * 16;
+#pragma unroll
+  for (int kk = 0; kk < ROPE / 16; ++kk)
+    k_at[D / 16 + kk] = PA_K + l32 * 128 + chunk128(l32, kk * 2 + half) * 16;
+#pragma unroll
+  for (int i = 0; i < DS; ++i) {
+    const int row = half * 4 + ((lane & 15) >> 2);
+    v_at[i] = row * 256 + seg256(row, i * 2 + ((lane >> 4) & 1)) * 32 +
+              (lane & 3) * 8;
+  }
+  auto fragment = [&](int m, int k_place, int v_place) -> s16x8 {
+    if (m < QK)   // (the moves of rows 16 and 32 apart are the same)
+      return *reinterpret_cast<const s16x8*>(
+          lds + k_place * PA_KEY_BYTES +
+          m / KF * 32 * (m % KF < D / 16 ? 256 : 128) + k_at[m % KF]);
+    const char* at = lds + 2 * PA_KEY_BYTES + v_place * PA_K +
+                     (m - QK) / DS * 16 * 256 + v_at[(m - QK) % DS];
+    const s16x4 a = lds_read_tr(at), b = lds_read_tr(at + 8 * 256);
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  const f32x16 zero = {};
+
   auto run = [&](auto shifts) {
     constexpr bool SHIFTS = decltype(shifts)::value;
-#pragma unroll 1
-    for (int kt = 0; kt < kt_end; ++kt) {
-      lds_fill_wait();
+    // Product m of the scores t of tile kt.
+    auto score = [&](const int kt, const int m, const s16x8 f,
+                     f32x16 (&t)[2]) {
+      const int n = m / KF, kk = m % KF;
+      if (kk < D / 16)
+        t[n] = mfma32<FP16Tag>(f, qf[kk], kk == 0 ? zero : t[n]);
+      else
+        t[n] = mfma32<Tag>(f, qf[kk], t[n]);
+      if constexpr (SHIFTS) {
+        if (kk == D / 32 - 1)
+          t[n] *= __builtin_ldexpf(1.f, min(ke[kt * 2] - ke[kt * 2 + 1], 127));
+        if (kk == D / 16 - 1) t[n] *= __builtin_ldexpf(1.f, ke[kt * 2 + 1]);
+      }
+    };
+    // One tile: its scores s become weights and results, between the products
+    // of the next one's scores t (MORE; where there is none, of what lies
+    // there).
+    auto tile_step = [&](const int kt, f32x16 (&s)[2], f32x16 (&t)[2],
+                         const int place, auto more) {
+      constexpr bool MORE = decltype(more)::value;
+      constexpr int FIRST = MORE ? 0 : QK;
+      if constexpr (MORE) {
+        // (Of either place the last read lies before the barrier.)
+        if (kt + 1 < kt_end) fill_values(kt + 1, 1 - place);
+        if (kt + 2 < kt_end) fill_keys(kt + 2, place);
+      }
+      if (kt * PA_KEYS <= wave_last) {   // else no key for these tokens
+        s16x8 frag[AHEAD], p_hi[4], p_lo[4];
+        const int nt = min(kt + 1, kt_end - 1);
+        auto read = [&](int m) {
+          if (m >= FIRST && m < ALL)
+            frag[m % AHEAD] = fragment(m, 1 - place, place);
+        };
+        auto product = [&](int m) {
+          const s16x8 f = frag[m % AHEAD];
+          if (m < QK) {
+            score(nt, m, f, t);
+          } else {
+            const int c = (m - QK) / DS, i = (m - QK) % DS;
+            o[i] = mfma32<Tag>(f, p_lo[c], o[i]);
+            o[i] = mfma32<Tag>(f, p_hi[c], o[i]);
+          }
+          read(m + AHEAD);
+        };
+        // Register e of s[n] is key n*32 + 8*(e/4) + 4*half + e%4.
+        if (kt * PA_KEYS + PA_KEYS - 1 > wave_first) {
+          const int left = qpos - kt * PA_KEYS - half * 4;
+#pragma unroll
+          for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+              s[n][e] = n * 32 + 8 * (e >> 2) + (e & 3) <= left ? s[n][e] : NEG;
+        }
+#pragma unroll
+        for (int m = FIRST; m < FIRST + AHEAD; ++m) read(m);
+        float mx = NEG;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int e = g * 4; e < g * 4 + 4; ++e) {
+            mx = __builtin_amdgcn_fmed3f(mx, s[0][e], INFINITY);
+            mx = __builtin_amdgcn_fmed3f(mx, s[1][e], INFINITY);
+          }
+          if constexpr (MORE) {
+#pragma unroll
+            for (int m = KF * g / 4; m < KF * (g + 1) / 4; ++m) product(m);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        mx = half_max(mx) * scale;
+        if (__any(mx - m_run > GROWTH)) {
+          const float m_new = fmaxf(m_run, mx);
+          const float f = __builtin_amdgcn_exp2f(m_run - m_new);
+          l_run *= f;
+#pragma unroll
+          for (int i = 0; i < DS; ++i) o[i] *= f;
+          m_run = m_new;
+        }
+        // --- weights, and O^T += V^T P^T, 16 keys at a time ----------------
+        // Half a chunk of weights a group, then as many products as weights
+        // are there for.
+        constexpr int TO[9] = {KF, 16, 20, 25, 28, 30, 32, 34, 36};
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+          __builtin_amdgcn_sched_barrier(0);
+          const int c = g / 2;
+          i32x4 hi = {}, lo = {};
+          if (g % 2) {
+            hi = __builtin_bit_cast(i32x4, p_hi[c]);
+            lo = __builtin_bit_cast(i32x4, p_lo[c]);
+          }
+#pragma unroll
+          for (int j = g % 2 * 2; j < g % 2 * 2 + 2; ++j) {
+            const int e = (c & 1) * 8 + j * 2;
+            const float p0 = __builtin_amdgcn_exp2f(
+                __builtin_fmaf(s[c >> 1][e], scale, -m_run));
+            const float p1 = __builtin_amdgcn_exp2f(
+                __builtin_fmaf(s[c >> 1][e + 1], scale, -m_run));
+            hi[j] = pack2<Tag>(p0, p1);
+            l_run += p0 + p1;
+            lo[j] = pack2<Tag>(p0 - unpack_lo<Tag>(hi[j]),
+                               p1 - unpack_hi<Tag>(hi[j]));
+          }
+          p_hi[c] = __builtin_bit_cast(s16x8, hi);
+          p_lo[c] = __builtin_bit_cast(s16x8, lo);
+#pragma unroll
+          for (int m = TO[g]; m < TO[g + 1]; ++m)
+            if (m >= FIRST) product(m);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = TO[8]; m < ALL; ++m) product(m);
+      }
+      if constexpr (MORE) lds_fill_wait();
       lds_barrier();
-      if (kt + 1 < kt_end) fill(kt + 1, (kt + 1) & 1);
-      if (kt * PA_KEYS > wave_last) continue;   // no key for these tokens
-      const char* t = lds + (kt & 1) * PA_BUF;
-      // --- S^T: 64 keys x 32 tokens ----------------------------------------
-      f32x16 s[2];
+    };
+
+    fill_keys(0, 0);
+    fill_values(0, 0);
+    if (kt_end > 1) fill_keys(1, 1);
+    lds_fill_wait();
+    lds_barrier();
+    f32x16 sa[2], sb[2];
 #pragma unroll
-      for (int n = 0; n < 2; ++n) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) s[n][e] = 0.f;
-        const int key = n * 32 + l32;
-#pragma unroll
-        for (int kk = 0; kk < D / 16; ++kk) {
-          s[n] = mfma32<FP16Tag>(
-              *reinterpret_cast<const s16x8*>(
-                  t + key * 256 + chunk256(key, kk * 2 + half) * 16),
-              qf[kk], s[n]);
-          if (SHIFTS && kk == D / 32 - 1)
-            s[n] *= __builtin_ldexpf(1.f,
-                                     min(ke[kt * 2] - ke[kt * 2 + 1], 127));
-        }
-        if constexpr (SHIFTS) s[n] *= __builtin_ldexpf(1.f, ke[kt * 2 + 1]);
-#pragma unroll
-        for (int kk = 0; kk < ROPE / 16; ++kk)
-          s[n] = mfma32<Tag>(
-              *reinterpret_cast<const s16x8*>(
-                  t + 2 * PA_K + key * 128 + chunk128(key, kk * 2 + half) * 16),
-              qf[D / 16 + kk], s[n]);
-      }
-      // Register e of s[n] is key n*32 + 8*(e/4) + 4*half + e%4.
-      if (kt * PA_KEYS + PA_KEYS - 1 > wave_first) {
-        const int left = qpos - kt * PA_KEYS - half * 4;
-#pragma unroll
-        for (int n = 0; n < 2; ++n)
-#pragma unroll
-          for (int e = 0; e < 16; ++e)
-            s[n][e] = n * 32 + 8 * (e >> 2) + (e & 3) <= left ? s[n][e] : NEG;
-      }
-      float mx = NEG;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        mx = __builtin_amdgcn_fmed3f(mx, s[0][e], INFINITY);
-        mx = __builtin_amdgcn_fmed3f(mx, s[1][e], INFINITY);
-      }
-      mx = half_max(mx) * scale;
-      if (__any(mx - m_run > GROWTH)) {
-        const float m_new = fmaxf(m_run, mx);
-        const float f = __builtin_amdgcn_exp2f(m_run - m_new);
-        l_run *= f;
-#pragma unroll
-        for (int i = 0; i < D / 32; ++i) o[i] *= f;
-        m_run = m_new;
-      }
-      // --- O^T += V^T P^T, 16 keys at a time -------------------------------
-      const int vrow = half * 4 + ((lane & 15) >> 2);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        i32x4 hi, lo;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int e = (c & 1) * 8 + j * 2;
-          const float p0 = __builtin_amdgcn_exp2f(
-              __builtin_fmaf(s[c >> 1][e], scale, -m_run));
-          const float p1 = __builtin_amdgcn_exp2f(
-              __builtin_fmaf(s[c >> 1][e + 1], scale, -m_run));
-          hi[j] = pack2<Tag>(p0, p1);
-          l_run += p0 + p1;
-          lo[j] = pack2<Tag>(p0 - unpack_lo<Tag>(hi[j]),
-                             p1 - unpack_hi<Tag>(hi[j]));
-        }
-        const s16x8 p_hi = __builtin_bit_cast(s16x8, hi);
-        const s16x8 p_lo = __builtin_bit_cast(s16x8, lo);
-        const int r0 = c * 16 + vrow;
-#pragma unroll
-        for (int i = 0; i < D / 32; ++i) {
-          const int seg = i * 2 + ((lane >> 4) & 1);
-          const char* at = t + PA_K + (lane & 3) * 8;
-          const s16x4 a = lds_read_tr(at + r0 * 256 + seg256(r0, seg) * 32);
-          const s16x4 b =
-              lds_read_tr(at + (r0 + 8) * 256 + seg256(r0 + 8, seg) * 32);
-          const s16x8 vf = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
-          o[i] = mfma32<Tag>(vf, p_lo, o[i]);
-          o[i] = mfma32<Tag>(vf, p_hi, o[i]);
-        }
-      }
+    for (int m = 0; m < QK; ++m) score(0, m, fragment(m, 0, 0), sa);
+    lds_barrier();   // the first keys' place is free
+    int kt = 0;
+#pragma unroll 1
+    for (; kt + 1 < kt_end; kt += 2) {
+      tile_step(kt, sa, sb, 0, std::true_type{});
+      tile_step(kt + 1, sb, sa, 1, std::true_type{});
     }
+    if (kt < kt_end) tile_step(kt, sa, sb, 0, std::false_type{});
   };
   if (__any(shifted != 0)) run(std::true_type{});
   else run(std::false_type{});
