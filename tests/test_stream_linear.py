@@ -51,6 +51,8 @@ TILES += [(96, 32752, 1088), (200, 32752, 1664), (99, 131056, 832),
 # Tiles of 64 weight rows, and of 256 that K is split over (with the
 # activation whole in one launch).
 TILES += [(66, 10688, 1664), (140, 10688, 1664), (66, 10944, 5120)]
+# More than one round of tiles of 128 weight rows (plain, up to 64 rows).
+TILES += [(40, 88064, 2048)]
 # Weights that come to each form of stream_linear (plan() in the source), whole
 # and with K split: rows of weights that end within a tile, steps of K past
 # what a ring holds.
@@ -277,10 +279,45 @@ def test_tiles_in_parts_replayed():
     (129, 4096, 6080, 0), (129, 4096, 6144, 2), (1024, 4096, 10816, 0),
     (1024, 4096, 10944, 2), (1025, 4096, 14336, 0), (1024, 5888, 28672, 0),
     (128, 36864, 7168, 0), (160, 24576, 1280, 0), (160, 24576, 1344, 2),
-    (300, 24576, 5120, 0), (64, 4096, 14336, 1)])
+    (300, 24576, 5120, 0)])
 def test_route_of_split_tiles(m, n, k, form):
     """Both sides of the lines in by_estimate (csrc/tile_linear.hip)."""
     assert _form(m, n, k)[0] == form
+
+
+@pytest.mark.parametrize("m,n,k,silu,form", [
+    (32, 65536, 4096, False, 1), (33, 65536, 4096, False, 2),
+    (64, 65536, 2048, False, 2), (64, 65536, 1984, False, 1),
+    (64, 98304, 4096, False, 2), (64, 98304, 5184, False, 1),
+    (33, 55808, 9216, True, 2), (33, 55552, 9216, True, 1),
+    (64, 27904, 5120, False, 2), (64, 27904, 5184, False, 1),
+    (64, 27752, 4096, False, 1), (64, 4096, 14336, False, 2),
+    (64, 4096, 14272, False, 1), (64, 4096, 14336, True, 1),
+    (33, 2304, 14336, False, 2), (33, 2296, 14336, False, 1),
+    (33, 20480, 14336, False, 2), (33, 20488, 14336, False, 1)])
+def test_route_of_few_rows(m, n, k, silu, form):
+    """Both sides of the lines for 33 to 64 rows in tile_form."""
+    assert _form(m, n, k, silu)[0] == form
+
+
+# Tiles on 33 to 64 rows: a wave with both of its 32-row groups, and without.
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(33, 65520, 2048), (64, 27904, 2048),
+                                   (40, 98304, 2112), (64, 2312, 14336),
+                                   (47, 20472, 14400)])
+def test_tiles_of_few_rows(m, n, k, dtype):
+    from vllm_amd.ops import hip_ops
+    assert _form(m, n, k)[0] == 2
+    x, w = _operands(m, n, k, dtype)
+    expect = x.float() @ w.float().t()
+    _check(hip_ops.linear(x, w), expect, dtype, k)
+    bias = torch.randn(n, device="cuda").to(dtype)
+    _check(hip_ops.linear(x, w, bias), expect + bias.float(), dtype, k)
+    if n % 16 == 0 and _form(m, n, k, True)[0] == 2:
+        gate, up = expect.chunk(2, -1)
+        _check(hip_ops.linear_silu_and_mul(x, w),
+               torch.nn.functional.silu(gate) * up, dtype, k)
 
 
 def test_shapes_reach_the_forms_of_models():

@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "common.h"
+#include "tile_linear.h"
 
 namespace vllm_amd {
 
@@ -371,7 +372,10 @@ torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
       (!bias.has_value() ||
        (bias->scalar_type() == a2.scalar_type() && bias->is_contiguous() &&
         bias->numel() == w.size(0)));
-  if (ours && stream_linear_takes(a2, w, w.size(0)))
+  if (ours &&
+      (bias.has_value() ||
+       !tile_linear_first(a2.size(0), w.size(0), K, false)) &&
+      stream_linear_takes(a2, w, w.size(0)))
     return stream_linear(a2, w, bias).reshape(sizes);
   auto out = torch::empty({a2.size(0), w.size(0)}, a.options());
   if (ours && !bias.has_value() && tile_linear(out, a2, w, false))

@@ -34,6 +34,8 @@
 //    4096 x 14336   25.3 -> 20.3   25.4 -> 21.2   31.6 -> 25.0   37.5 -> 28.7   (18)
 //    2112 x 7168    12.2 ->  8.3   12.4 ->  9.8   16.0 -> 11.1   19.2 -> 14.3   (4.6)
 //  128256 x 4096     175 ->  154    174 ->  151    188 ->  163    199 ->  186   (159)
+// (From 33 rows on tile_linear.hip takes the third, the fourth and the last
+// without a bias: 42, 28 and 172 on 64.)
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
@@ -302,7 +304,8 @@ void launch(torch::Tensor& out, const torch::Tensor& x,
 
 // Whether a product of M rows with rows_w weight rows (silu: n = rows_w / 2
 // columns of out) is one for this file, by its sizes. Up to 64 rows it is,
-// but for two kinds at which the tuned library is ahead:
+// but for two kinds at which the tuned library is ahead (and callers ask
+// tile_linear_first before):
 //  * Wide and short ones. Workgroups hardly begin before they end, and what
 //    they write is no longer little beside the weights. us, library and this:
 //    50272 x 768, 16 / 32 / 64 rows 18.4 and 18.9, 19.1 and 20.5, 20.5 and
@@ -346,7 +349,8 @@ bool stream_linear_takes(const torch::Tensor& x, const torch::Tensor& w,
 std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
                                  bool silu) {
   const int64_t n = silu ? weight_rows / 2 : weight_rows;
-  if (stream_sizes(rows, weight_rows, n, k)) {
+  if (!tile_linear_first(rows, weight_rows, k, silu) &&
+      stream_sizes(rows, weight_rows, n, k)) {
     const int xg = row_groups(rows);
     const Plan p = plan(xg, weight_rows, (int)k, silu);
     const Form f = SL_FORMS[p.form];
@@ -382,7 +386,8 @@ torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w) {
   const int64_t N = w.size(0) / 2;
   sizes.back() = N;
   auto out = torch::empty({x.size(0), N}, x.options());
-  if (!stream_linear_takes(x, w, N)) {
+  if (tile_linear_first(x.size(0), w.size(0), x.size(1), true) ||
+      !stream_linear_takes(x, w, N)) {
     if (x.size(0) > 0 && tile_linear(out, x, w, true))
       return out.reshape(sizes);
     return silu_and_mul(lt_linear(x, w, c10::nullopt)).reshape(sizes);

@@ -1,4 +1,4 @@
-// Linear layers on 65 to 1024 rows, by tiles of all rows or of 256 of them
+// Linear layers on 33 to 1024 rows, by tiles of all rows or of 256 of them
 // (gfx950): out[M, N] = x[M, K] @ w[N, K]^T, and for up to 256 rows the same
 // with silu(gate) * up of two halves of w as the epilogue.
 //
@@ -249,7 +249,22 @@ TileForm by_estimate(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
-// How M rows meet rows_w weight rows of K; cols 0: in the library.
+// How M rows meet rows_w weight rows of K; cols 0: in the library, or up to 64
+// rows in stream_linear.hip.
+//
+// On 33 to 64 rows stream_linear splits K over the waves of a workgroup, which
+// takes x in for 16 to 128 weight rows; a tile takes it in for 128 or 256. So
+// tiles are ahead where their rounds keep the CUs busy, the more the shorter K
+// is, and where K is long enough to be split here. us, stream_linear and this,
+// 64 rows: 128256 x 4096 190 and 172; 57344 x 4096 90 and 75; 102400 x 2048
+// (0.78 of two rounds) 96 and 80, 152064 x 3584 216 and 207; 57344 x 8192 with
+// the activation 159 and 146; 28672 x 4096 with it 41.9 and 40.9; 4096 x 14336
+// 30.2 and 27.7, 7168 x 16384 52.9 and 45.0, 8192 x 28672 103 and 83. On the
+// other side: 145000 x 5504 by tiles of 128 311 and 330; 36864 x 7168 97 and
+// 120 (0.56 of a round); 24576 x 1536 18.1 and 18.7; 10944 x 5120 32.9 and 30.7,
+// but 29.1 and 30.0 on 33 rows; 12288 x 5120 29.5 and 31.0; 2048 x 16384 on 33
+// rows 18.6 and 20.0; 23672 x 22016 180 and 208. 5500 sizes inside: 0.90 of
+// stream_linear's time on average, none above 1.05.
 //
 // The share of its rounds over 256 CUs that a form keeps busy decides: 256
 // where that is at least 95 % (for up to 128 rows of a plain product in more
@@ -267,15 +282,20 @@ TileForm by_estimate(int64_t M, int64_t N, int64_t K) {
 // 2048 73 and 76; 128256 x 256, 128 rows 30.6 and 26.2, x 1024 61.5 and 60.0,
 // 65 rows 54 and 62. An activation halves what is written.
 TileForm tile_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
-  if (M <= 64 || (silu && M > TI_ROWS)) return {0, 1};
-  if (M <= TI_ROWS && (silu || K > 8 * M)) {
-    auto rounds = [&](int tile) {
-      return (rows_w + tile * 256 - 1) / tile / 256;
-    };
-    auto busy = [&](int tile) {
-      return (double)((rows_w + tile - 1) / tile) /
-             (double)(rounds(tile) * 256);
-    };
+  if (M <= 32 || (silu && M > TI_ROWS)) return {0, 1};
+  auto rounds = [&](int tile) {
+    return (rows_w + tile * 256 - 1) / tile / 256;
+  };
+  auto busy = [&](int tile) {
+    return (double)((rows_w + tile - 1) / tile) / (double)(rounds(tile) * 256);
+  };
+  if (M <= 64) {
+    if (K < 2048) return {0, 1};
+    if (busy(256) >= (rounds(256) == 1 ? 0.85 : K <= 4096 ? 0.75 : 0.9))
+      return {256, 1};
+    if (K <= 5120 && busy(128) >= 0.85) return {128, 1};
+    if (silu || K < 14336 || rows_w < 2304 || rows_w > 20480) return {0, 1};
+  } else if (M <= TI_ROWS && (silu || K > 8 * M)) {
     if (busy(256) >= 0.95 && (silu || M > 128 || rounds(256) > 1))
       return {256, 1};
     const double least =
