@@ -427,7 +427,6 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
   // chunks of 16 keys of this one's results (two, by the weights' parts).
   constexpr int KF = (D + ROPE) / 16, DS = D / 32;
   constexpr int QK = 2 * KF, ALL = QK + 4 * DS;
-  constexpr int AHEAD = 4;   // fragments read ahead
   int k_at[KF], v_at[DS];    // first fragments of a tile, in its bytes
 #pragma unroll
   for (int kk = 0; kk < D / 16; ++kk)
@@ -441,11 +440,22 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
     v_at[i] = row * 256 + seg256(row, i * 2 + ((lane >> 4) & 1)) * 32 +
               (lane & 3) * 8;
   }
-  auto fragment = [&](int m, int k_place, int v_place) -> s16x8 {
-    if (m < QK)   // (the moves of rows 16 and 32 apart are the same)
+  auto fragment = [&](int m, int k_place, int v_place, auto again) -> s16x8 {
+    if (m < QK) {   // (the moves of rows 16 and 32 apart are the same)
+      int at = k_at[m % KF];
+      if constexpr (decltype(again)::value) {
+        // Formed anew, not kept: there is no register left for it.
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        const int row = l & 31, c = m % KF * 2 + (l >> 5);
+        at = m % KF < D / 16
+                 ? row * 256 + chunk256(row, c) * 16
+                 : PA_K + row * 128 + chunk128(row, c - D / 8) * 16;
+      }
       return *reinterpret_cast<const s16x8*>(
           lds + k_place * PA_KEY_BYTES +
-          m / KF * 32 * (m % KF < D / 16 ? 256 : 128) + k_at[m % KF]);
+          m / KF * 32 * (m % KF < D / 16 ? 256 : 128) + at);
+    }
     const char* at = lds + 2 * PA_KEY_BYTES + v_place * PA_K +
                      (m - QK) / DS * 16 * 256 + v_at[(m - QK) % DS];
     const s16x4 a = lds_read_tr(at), b = lds_read_tr(at + 8 * 256);
@@ -455,6 +465,10 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
 
   auto run = [&](auto shifts) {
     constexpr bool SHIFTS = decltype(shifts)::value;
+    // Fragments read ahead. (Scratch for the rare form with shifts would cost
+    // all launches: one prompt of 22 tokens 6.9 us with 44 B of it, 6.6 with
+    // none.)
+    constexpr int AHEAD = SHIFTS ? 1 : 4;
     // Product m of the scores t of tile kt.
     auto score = [&](const int kt, const int m, const s16x8 f,
                      f32x16 (&t)[2]) {
@@ -486,7 +500,7 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
         const int nt = min(kt + 1, kt_end - 1);
         auto read = [&](int m) {
           if (m >= FIRST && m < ALL)
-            frag[m % AHEAD] = fragment(m, 1 - place, place);
+            frag[m % AHEAD] = fragment(m, 1 - place, place, shifts);
         };
         auto product = [&](int m) {
           const s16x8 f = frag[m % AHEAD];
@@ -580,8 +594,11 @@ void mla_prompt_kernel(short* __restrict__ out,            // [T, Hq, D]
     lds_barrier();
     f32x16 sa[2], sb[2];
 #pragma unroll
-    for (int m = 0; m < QK; ++m) score(0, m, fragment(m, 0, 0), sa);
-    lds_barrier();   // the first keys' place is free
+    for (int m = 0; m < QK; ++m) {
+      score(0, m, fragment(m, 0, 0, shifts), sa);
+      if (SHIFTS && m % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    if (kt_end > 1) lds_barrier();   // the first keys' place is free
     int kt = 0;
 #pragma unroll 1
     for (; kt + 1 < kt_end; kt += 2) {
