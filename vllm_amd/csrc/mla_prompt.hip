@@ -20,8 +20,8 @@
 // two, which is one unless their largest is below 1/4 or from 2^15.
 // 128 heads, prompts of 300, 1300 and 2301 tokens: 2.02 -> 0.63 ms with
 // everything between queries and results (latent form before); one of
-// 8192 13.1 -> 3.80 ms, four of 2048 4.48 -> 1.36 ms (before the last change to
-// mla_prompt_kernel's order, which takes 7 % off it).
+// 8192 13.1 -> 3.80 ms, four of 2048 4.48 -> 1.36 ms (with mla_prompt_kernel
+// one step after the other; as it is it takes 7 % less).
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>
