@@ -150,7 +150,8 @@ template <> DEVINL f32x16 mfma32<FP16Tag>(s16x8 a, s16x8 b, f32x16 c) {
 // are taken the compiler then moves them about (8192 x 28672 x 4096 by
 // tile_product.h 1.08 PFLOP/s, 1.43 so). The compiler knows nothing of
 // what may stand right before and after the instruction, so accumulators come
-// and go through acc_fence.
+// and go through acc_fence; that nothing else was put beside one is checked in
+// the built kernels (tests/test_product_waits.py).
 template <typename Tag> DEVINL void mfma16_acc(f32x4& c, s16x8 a, s16x8 b) {
   if constexpr (std::is_same_v<Tag, BF16Tag>)
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
@@ -162,18 +163,15 @@ template <typename Tag> DEVINL void mfma16_acc(f32x4& c, s16x8 a, s16x8 b) {
                  : "v"(a), "v"(b));
 }
 // Between other instructions that write or read the accumulators and products
-// that do: the waits of either side (up to 19 states after a product of eight
-// passes) lie between them.
+// that do: the waits of either side (two states before a product, eight after)
+// lie before and behind the point where the compiler may move them.
 template <int N, int M> DEVINL void acc_fence(f32x4 (&acc)[N][M]) {
+  asm volatile("s_nop 15");
 #pragma unroll
   for (int i = 0; i < N; ++i)
 #pragma unroll
     for (int j = 0; j < M; ++j) asm volatile("" : "+a"(acc[i][j]));
-  asm volatile("s_nop 15\n\ts_nop 15");
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-#pragma unroll
-    for (int j = 0; j < M; ++j) asm volatile("" : "+a"(acc[i][j]));
+  asm volatile("s_nop 15");
 }
 
 // Two floats rounded (nearest even) to a packed 16-bit pair.
