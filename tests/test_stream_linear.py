@@ -274,6 +274,27 @@ def test_tiles_in_parts_replayed():
         assert torch.equal(out, eager) and torch.equal(beside, eager)
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (700, 3584, 18944), (768, 7168, 16384), (600, 2112, 7168),
+    (1024, 2112, 7168), (512, 4096, 14336), (64, 7168, 16384),
+    (256, 30720, 3840)])
+def test_tiles_that_share_weights_begin_together(m, n, k):
+    """Also where an XCD's run of workgroups is no multiple of the row tiles;
+    every tile and part is somebody's."""
+    _, cols, parts = _form(m, n, k)
+    from vllm_amd.ops import hip_ops
+    flat = hip_ops._C.linear_starts(m, n, k, False)
+    jobs = [tuple(flat[i:i + 5]) for i in range(0, len(flat), 5)]
+    m_tiles, n_tiles = -(-m // (128 if m <= 128 else 256)), -(-n // cols)
+    assert sorted(j[1:4] for j in jobs) == [
+        (p, a, b) for p in range(parts) for a in range(m_tiles)
+        for b in range(n_tiles)]
+    begin = {}
+    for xcd, part, _, tile, first in jobs:
+        assert begin.setdefault((xcd, part, tile), first) == first
+    assert len(set(begin.values())) > 1
+
+
 @pytest.mark.parametrize("m,n,k,form", [
     (128, 4096, 5056, 0), (128, 4096, 5120, 2), (128, 1528, 7168, 0),
     (129, 4096, 6080, 0), (129, 4096, 6144, 2), (1024, 4096, 10816, 0),

@@ -48,6 +48,8 @@ torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
 torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w);
 std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
                                  bool silu);
+std::vector<int64_t> linear_starts(int64_t rows, int64_t weight_rows,
+                                   int64_t k, bool silu);
 torch::Tensor lt_linear_fp8(torch::Tensor a, torch::Tensor w);
 void dynamic_quant_fp8(torch::Tensor out, torch::Tensor scales,
                        torch::Tensor x);
@@ -224,6 +226,8 @@ TORCH_LIBRARY(vllm_amd, m) {
   m.def("linear_silu_and_mul(Tensor a, Tensor w) -> Tensor");
   m.def("linear_form(int rows, int weight_rows, int k, bool silu) -> int[]",
         &vllm_amd::linear_form);
+  m.def("linear_starts(int rows, int weight_rows, int k, bool silu) -> int[]",
+        &vllm_amd::linear_starts);
   m.def("lt_linear_fp8(Tensor a, Tensor w) -> Tensor");
   m.def("dynamic_quant_fp8(Tensor(a!) out, Tensor(b!) scales, Tensor x)"
         " -> ()");

@@ -8,9 +8,9 @@
 // nothing comes from HBM).
 //
 //  * Weights that one workgroup reads leave L2 first; x stays.
-//  * Workgroups begin at different stages of K, those that share weights at
-//    the same one: rows whose stride is a power of two meet on few channels
-//    otherwise. A window of some 60 stages, so that x stays in L2. 128 rows of
+//  * Workgroups begin at different stages of K, those of an XCD that share
+//    weights at the same one (tile_job): rows whose stride is a power of two
+//    meet on few channels otherwise. A window of some 60 stages, so that x stays in L2. 128 rows of
 //    weights alone at K = 16384 5.4 -> 7.0 TB/s; 28672 x 4096 with the
 //    activation, 128 rows 57 -> 52 us.
 //  * Layers with few tiles split K over workgroups until about one a CU runs,
@@ -55,22 +55,20 @@ __global__ __launch_bounds__(TP_THREADS, 1) void tile_linear_kernel(
   const int l16 = lane & 15;
   constexpr int H = SILU ? 2 : 1;
   constexpr int NO = P::NI / H;
-  // Each XCD (workgroups go round them) takes a run of tiles; those beside
-  // each other have weights in common, then columns of K.
-  const int tiles = m_tiles * n_tiles, jobs = tiles * parts;
+  const int jobs = m_tiles * n_tiles * parts;
   const int run = (jobs + 7) / 8;
   const int xcd = blockIdx.x % 8, nth = blockIdx.x / 8;
-  const int job = xcd * run + nth;
-  if (nth >= run || job >= jobs) return;
-  const int part = job / tiles, tile = job % tiles;
-  const int m0 = tile % m_tiles * P::TM;
-  const int n0 = tile / m_tiles * (P::TN / H);
+  if (nth >= run || xcd * run + nth >= jobs) return;
+  const TileJob t = tile_job(xcd, nth, run, m_tiles, n_tiles);
+  const int part = t.part;
+  const int m0 = t.m_tile * P::TM;
+  const int n0 = t.n_tile * (P::TN / H);
   const int rows = min(M - m0, P::TM);
-  const int s0 = K / TP_K * part / parts;
-  const int steps = K / TP_K * (part + 1) / parts - s0;
+  const int s0 = tile_part(K / TP_K, part, parts);
+  const int steps = tile_part(K / TP_K, part + 1, parts) - s0;
   const short* xt = x + (int64_t)m0 * K;
   const short* wt = w + (int64_t)n0 * K;
-  const int turn = (nth / m_tiles + xcd * 4) % steps;
+  const int turn = t.turn % steps;
   auto stage = [&](int s) {
     s += turn;
     return (s0 + (s >= steps ? s - steps : s)) * TP_K;
@@ -362,6 +360,28 @@ TileForm tile_linear_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
       K % TP_K != 0 || K >= (1 << 22) || (rows_w + 256) * K * 2 >= (1ll << 32))
     return {0, 1};
   return tile_form(M, rows_w, K, silu);
+}
+
+// For the tests: {XCD, part of K, row tile, weight tile, first stage in the
+// part} of every workgroup of a product of these sizes; nothing if it is not
+// one for this file.
+std::vector<int64_t> linear_starts(int64_t rows, int64_t weight_rows,
+                                   int64_t k, bool silu) {
+  const TileForm form = tile_linear_form(rows, weight_rows, k, silu);
+  std::vector<int64_t> out;
+  if (form.cols == 0) return out;
+  const int m_tiles = ceil_div((int)rows, rows <= 128 ? 128 : 256);
+  const int n_tiles = ceil_div((int)weight_rows, form.cols);
+  const int jobs = m_tiles * n_tiles * form.parts;
+  const int run = ceil_div(jobs, 8), stages = (int)k / TP_K;
+  for (int xcd = 0; xcd < 8; ++xcd)
+    for (int nth = 0; nth < run && xcd * run + nth < jobs; ++nth) {
+      const TileJob t = tile_job(xcd, nth, run, m_tiles, n_tiles);
+      const int steps = tile_part(stages, t.part + 1, form.parts) -
+                        tile_part(stages, t.part, form.parts);
+      out.insert(out.end(), {xcd, t.part, t.m_tile, t.n_tile, t.turn % steps});
+    }
+  return out;
 }
 
 // The product of x [M, K] and w [rows, K], both contiguous, into out [M, n],
