@@ -206,13 +206,15 @@ def test_route_by_sizes(m, rows, k, silu, kind):
 
 
 def _key(m, rows, k, silu):
-    """Which kernel: form, row groups, whether K is split; or tile, row form,
-    whether tiles take more than a round of the CUs."""
+    """Which kernel: form, row groups, whether K is split; or tile, tiles of
+    rows (of 128 or 256, or several), whether K is split, whether tiles take
+    more than a round of the CUs."""
     form = _form(m, rows, k, silu)
     if form[0] == 1:
         return ("stream", silu, form[1], form[4], form[5] > 1)
     if form[0] == 2:
-        return ("tile", silu, form[1], m > 128, rows > form[1] * 256)
+        return ("tile", silu, form[1], (m > 128) + (m > 256), form[2] > 1,
+                rows > form[1] * 256)
     return None
 
 
@@ -322,11 +324,13 @@ def test_route_of_few_rows(m, n, k, silu, form):
 
 
 # Tiles on 33 to 64 rows: a wave with both of its 32-row groups, and without.
+FEW = [(33, 65520, 2048), (64, 27904, 2048), (40, 98304, 2112),
+       (64, 2312, 14336), (47, 20472, 14400)]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("m,n,k", [(33, 65520, 2048), (64, 27904, 2048),
-                                   (40, 98304, 2112), (64, 2312, 14336),
-                                   (47, 20472, 14400)])
+@pytest.mark.parametrize("m,n,k", FEW)
 def test_tiles_of_few_rows(m, n, k, dtype):
     from vllm_amd.ops import hip_ops
     assert _form(m, n, k)[0] == 2
@@ -342,13 +346,16 @@ def test_tiles_of_few_rows(m, n, k, dtype):
 
 
 def test_shapes_reach_the_forms_of_models():
-    """Every kernel that a layer of a known model runs as, on 1 to 256 rows,
+    """Every kernel that a layer of a known model runs as, on 1 to 1024 rows,
     is one that the tests above run."""
-    edges = (1, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 256)
+    edges = (1, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 256, 257, 512, 513,
+             768, 769, 1024)
     tested = {_key(m, n, k, silu) for n, k in FORMS for m in edges[:8]
               for silu in (False, True) if not silu or n % 16 == 0}
     tested |= {_key(m, n, k, silu) for m, n, k in TILES
                for silu in (False, True)}
+    tested |= {_key(m, n, k, False) for m, n, k, _ in SPLIT}
+    tested |= {_key(m, n, k, False) for m, n, k in FEW}
     models = {_key(m, n, k, silu) for n, k, silu in _model_layers()
               for m in edges if n > 0 and k > 0 and n % (16 if silu else 8) == 0}
     assert len(models) > 30
