@@ -50,7 +50,8 @@ TILES += [(96, 32752, 1088), (200, 32752, 1664), (99, 131056, 832),
           (130, 65520, 1088), (161, 131056, 1344), (70, 131056, 320)]
 # Tiles of 64 weight rows, and of 256 that K is split over (with the
 # activation whole in one launch).
-TILES += [(66, 10688, 1664), (140, 10688, 1664), (66, 10944, 5120)]
+TILES += [(66, 10688, 1664), (140, 10688, 1664), (66, 10944, 5120),
+          (140, 15432, 1664)]
 # More than one round of tiles of 128 weight rows (plain, up to 64 rows).
 TILES += [(40, 88064, 2048)]
 # Weights that come to each form of stream_linear (plan() in the source), whole
@@ -302,7 +303,12 @@ def test_tiles_that_share_weights_begin_together(m, n, k):
     (129, 4096, 6080, 0), (129, 4096, 6144, 2), (1024, 4096, 10816, 0),
     (1024, 4096, 10944, 2), (1025, 4096, 14336, 0), (1024, 5888, 28672, 0),
     (128, 36864, 7168, 0), (160, 24576, 1280, 0), (160, 24576, 1344, 2),
-    (300, 24576, 5120, 0)])
+    (300, 24576, 5120, 0),
+    # K whole: the share of a round that tiles keep busy.
+    (128, 42752, 4096, 2), (128, 42496, 4096, 0),
+    (192, 24576, 7232, 2), (192, 24448, 7232, 0), (192, 24448, 7168, 2),
+    (192, 15424, 4096, 2), (192, 15360, 4096, 0), (192, 15424, 5184, 0),
+    (128, 9856, 4096, 2), (128, 9792, 4096, 0)])
 def test_route_of_split_tiles(m, n, k, form):
     """Both sides of the lines in by_estimate (csrc/tile_linear.hip)."""
     assert _form(m, n, k)[0] == form

@@ -209,18 +209,29 @@ double estimate(int64_t M, int64_t N, int64_t K, int cols, int parts) {
          (parts > 1 ? 3.5 + parts * (double)M * (double)N * 4e-6 / 3.2 : 0.);
 }
 
-// The form of least estimate among those of one round that keep 60 % of the CUs
-// busy, where it is ahead of the library. With K whole: up to 256 rows. With K
-// split (up to 16 parts): from K = 5120 on up to 128 rows, above from 6144 on,
-// and only if K is long beside the 256 x 256 tiles of the output (170 columns
-// of K each, 90 of them), since partial sums cost 10 to 20 us. Below 1536
-// columns of output there is too little to split. us, the library and this (at
-// 128, 256 and 1024 rows if not said): 4096 x 14336 52 / 34, 65 / 45, 137 /
-// 116; 3584 x 18944 65 / 40, 80 / 52, 173 / 132; 7168 x 16384 71 / 54, 107 /
-// 72, and 512 rows 148 / 117; 2112 x 7168 25 / 17, 32 / 24, 49 / 45; 24576 x
-// 1536 27.6 / 23.0. On the other side of the lines: 4096 x 4096 17.3 / 17.0,
-// 21.0 / 25.1, 41 / 50; 4096 x 7168, 1024 rows 69 / 74; 8192 x 28672, 768 rows
-// 301 / 316; 36864 x 7168, 128 rows 118 / 121; 512 x 7168, 256 rows 12 / 15.6.
+// The form of least estimate among those of one round that keep enough of the
+// CUs busy, where it is ahead of the library.
+//
+// With K split (up to 16 parts) 60 % are enough. From K = 5120 on up to 128
+// rows, above from 6144 on, and only if K is long beside the 256 x 256 tiles of
+// the output (170 columns of K each, 90 of them), since partial sums cost 10 to
+// 20 us. Below 1536 columns of output there is too little to split. us, the
+// library and this (at 128, 256 and 1024 rows if not said): 4096 x 14336 52 /
+// 34, 65 / 45, 137 / 116; 3584 x 18944 65 / 40, 80 / 52, 173 / 132; 7168 x
+// 16384 71 / 54, 107 / 72, and 512 rows 148 / 117; 2112 x 7168 25 / 17, 32 / 24,
+// 49 / 45. On the other side of the lines: 4096 x 4096 17.3 / 17.0, 21.0 / 25.1,
+// 41 / 50; 4096 x 7168, 1024 rows 69 / 74; 8192 x 28672, 768 rows 301 / 316; 512
+// x 7168, 256 rows 12 / 15.6. Of 2300 sizes inside 0.74 of the library's time
+// on average, one above 1.02 (1.026).
+//
+// With K whole, up to 256 rows: 65 %, and 75 % where K is long (the library
+// begins K at several places: 19712 x 9728, 148 rows, 60 % busy 105 / 113; 39680
+// x 10240, 68 rows, 61 % 157 / 169; 22272 x 5632, 95 rows, 68 % 57 / 61; 43456 x
+// 11968, 154 rows, 66 % 216 / 229; inside 22016 x 4096, 192 rows, 67 % 62 / 52).
+// Tiles of 64 take x in for few weights: up to 128 rows 60 % are enough (24576 x
+// 1536 27.6 / 23.0), above only nearly all, and K up to 5120 (256 rows: 16384 x
+// 4096 52 / 48, 71 % 11568 x 4096 39 / 45, 88 % 14336 x 4096 45 / 47; 15872 x
+// 7168 78 / 82). Of 1200 sizes inside 0.87 on average, two above 1.03 (1.05).
 TileForm by_estimate(int64_t M, int64_t N, int64_t K) {
   TileForm best{0, 1};
   if (M > 1024) return best;
@@ -233,8 +244,12 @@ TileForm by_estimate(int64_t M, int64_t N, int64_t K) {
   for (int cols : {64, 128, 256}) {
     if (cols == 64 && M > 256) continue;
     const int64_t tiles = (M + tm - 1) / tm * ((N + cols - 1) / cols);
+    const int64_t lengthy = cols == 256 ? 8192 : M <= 128 ? 5120 : 7168;
+    const int64_t whole = cols > 64 ? (K > lengthy ? 192 : 167)
+                          : M <= 128 ? 154 : K <= 5120 ? 241 : 257;
     for (int parts = 1; parts <= 16 && tiles * parts <= 256; ++parts) {
-      if (tiles * parts < 154 || K / TP_K / parts < 4 ||
+      if (tiles * parts < (parts == 1 ? whole : 154) ||
+          K / TP_K / parts < 4 ||
           (parts == 1 ? M > 256 || K <= 8 * M : !split))
         continue;
       const double t = estimate(M, N, K, cols, parts);
