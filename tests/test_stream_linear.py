@@ -321,9 +321,16 @@ def test_route_of_split_tiles(m, n, k, form):
     (33, 55808, 9216, True, 2), (33, 55552, 9216, True, 1),
     (64, 27904, 5120, False, 2), (64, 27904, 5184, False, 1),
     (64, 27752, 4096, False, 1), (64, 4096, 14336, False, 2),
-    (64, 4096, 14272, False, 1), (64, 4096, 14336, True, 1),
-    (33, 2304, 14336, False, 2), (33, 2296, 14336, False, 1),
-    (33, 20480, 14336, False, 2), (33, 20488, 14336, False, 1)])
+    (64, 4096, 8448, False, 2), (64, 4096, 8384, False, 1),
+    (33, 4096, 10432, False, 2), (33, 4096, 10368, False, 1),
+    (33, 2808, 14400, False, 2), (33, 2808, 14336, False, 1),
+    (33, 2816, 10432, False, 2), (64, 4096, 14336, True, 1),
+    (33, 2304, 14400, False, 2), (33, 2296, 14400, False, 1),
+    (33, 19456, 14336, False, 2), (33, 19464, 14336, False, 1),
+    (48, 16384, 10368, False, 2),    # never tiles of 64 with K whole
+    (64, 31744, 4096, True, 2), (64, 31872, 4096, True, 1),
+    (64, 32768, 3072, True, 2), (64, 98304, 4096, True, 1),
+    (64, 100352, 4096, True, 2)])
 def test_route_of_few_rows(m, n, k, silu, form):
     """Both sides of the lines for 33 to 64 rows in tile_form."""
     assert _form(m, n, k, silu)[0] == form
@@ -331,7 +338,8 @@ def test_route_of_few_rows(m, n, k, silu, form):
 
 # Tiles on 33 to 64 rows: a wave with both of its 32-row groups, and without.
 FEW = [(33, 65520, 2048), (64, 27904, 2048), (40, 98304, 2112),
-       (64, 2312, 14336), (47, 20472, 14400)]
+       (64, 2312, 14336), (47, 19448, 14400), (33, 2824, 10432),
+       (64, 13824, 8448)]
 
 
 @pytest.mark.gpu

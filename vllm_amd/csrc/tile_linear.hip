@@ -250,7 +250,7 @@ TileForm by_estimate(int64_t M, int64_t N, int64_t K) {
     for (int parts = 1; parts <= 16 && tiles * parts <= 256; ++parts) {
       if (tiles * parts < (parts == 1 ? whole : 154) ||
           K / TP_K / parts < 4 ||
-          (parts == 1 ? M > 256 || K <= 8 * M : !split))
+          (parts == 1 ? M > 256 || M <= 64 || K <= 8 * M : !split))
         continue;
       const double t = estimate(M, N, K, cols, parts);
       if (t < least) {
@@ -268,16 +268,22 @@ TileForm by_estimate(int64_t M, int64_t N, int64_t K) {
 // On 33 to 64 rows stream_linear splits K over the waves of a workgroup, which
 // takes x in for 16 to 128 weight rows; a tile takes it in for 128 or 256. So
 // tiles are ahead where their rounds keep the CUs busy, the more the shorter K
-// is, and where K is long enough to be split here. us, stream_linear and this,
-// 64 rows: 128256 x 4096 190 and 172; 57344 x 4096 90 and 75; 102400 x 2048
-// (0.78 of two rounds) 96 and 80, 152064 x 3584 216 and 207; 57344 x 8192 with
-// the activation 159 and 146; 28672 x 4096 with it 41.9 and 40.9; 4096 x 14336
-// 30.2 and 27.7, 7168 x 16384 52.9 and 45.0, 8192 x 28672 103 and 83. On the
-// other side: 145000 x 5504 by tiles of 128 311 and 330; 36864 x 7168 97 and
-// 120 (0.56 of a round); 24576 x 1536 18.1 and 18.7; 10944 x 5120 32.9 and 30.7,
-// but 29.1 and 30.0 on 33 rows; 12288 x 5120 29.5 and 31.0; 2048 x 16384 on 33
-// rows 18.6 and 20.0; 23672 x 22016 180 and 208. 5500 sizes inside: 0.90 of
-// stream_linear's time on average, none above 1.05.
+// is, and where K is long enough to be split here: from 10400 on 33 rows (the
+// crossing lies between 8700 and 11000 by the weight rows) to 8400 on 64 (6600
+// to 8700), later where there are few weight rows, whose parts are many. us,
+// stream_linear and this, 64 rows: 128256 x 4096 190 and 172; 57344 x 4096 90
+// and 75; 102400 x 2048 (0.78 of two rounds) 96 and 80, 152064 x 3584 216 and
+// 207; 57344 x 8192 with the activation 159 and 146; 28672 x 4096 with it 41.9
+// and 40.9; on 33 and 64 rows 5120 x 10240 27.3 and 24.8, 29.7 and 25.9; 3072 x
+// 12288 23.0 and 21.6, 25.5 and 22.4; 8192 x 10240 35.1 and 33.5, 38.5 and 34.7;
+// 7168 x 16384 on 64 52.9 and 45.0, 8192 x 28672 103 and 83. On the other side:
+// 145000 x 5504 by tiles of 128 311 and 330; 24576 x 1536 18.1 and 18.7; 12288 x
+// 5120 29.5 and 31.0; 8192 x 8192 on 33 and 64 27.9 and 31.1, 29.7 and 31.1; 5120
+// x 8192 on 33 21.8 and 22.0; 2560 x 10752 on 48 4 % behind; 22880 x 12096 on 40
+// 13 % (two parts). Where all CUs take gate and up rows at a stride of 8 KB they
+// meet on few channels: 32768 x 4096 with the activation 43.3 and 50.4, 31600 x
+// 4096 42.6 and 42.0. 8100 sizes inside: 0.90 of stream_linear's time on average,
+// one in 180 above 1.02, seven above 1.05 (1.074: 7168 x 13312 on 33).
 //
 // The share of its rounds over 256 CUs that a form keeps busy decides: 256
 // where that is at least 95 % (for up to 128 rows of a plain product in more
@@ -304,10 +310,16 @@ TileForm tile_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
   };
   if (M <= 64) {
     if (K < 2048) return {0, 1};
-    if (busy(256) >= (rounds(256) == 1 ? 0.85 : K <= 4096 ? 0.75 : 0.9))
+    if (busy(256) >= (rounds(256) == 1 ? 0.85
+                      : K > 4096       ? 0.9
+                      : silu           ? 0.76
+                                       : 0.75))
       return {256, 1};
-    if (K <= 5120 && busy(128) >= 0.85) return {128, 1};
-    if (silu || K < 14336 || rows_w < 2304 || rows_w > 20480) return {0, 1};
+    const bool meet = silu && K % 4096 == 0 && busy(128) > 0.97;
+    if (K <= 5120 && busy(128) >= 0.85 && !meet) return {128, 1};
+    if (silu || rows_w < 2304 || rows_w > 19456 ||
+        K < 12500 - 64 * M + (rows_w < 2816 ? 4000 : 0))
+      return {0, 1};
   } else if (M <= TI_ROWS && (silu || K > 8 * M)) {
     if (busy(256) >= 0.95 && (silu || M > 128 || rounds(256) > 1))
       return {256, 1};
