@@ -90,6 +90,34 @@ def test_mla_split(hip, rows, heads, keys, parts):
     assert hip._mla_split(rows, heads, keys) == parts
 
 
+@pytest.mark.parametrize("rows,heads,told,parts", [
+    (4, 64, 8192, 64), (6, 64, 6000, 42), (3, 128, 8192, 42),
+    (8, 64, 4096, 32), (4, 128, 16384, 64),    # shorter rows would lose
+    (1, 128, 4096, 32), (128, 128, 1000, 1),   # as many, or they gain too
+    (3, 128, 0, 1)])
+def test_mla_split_of_rows_shorter_than_told(hip, rows, heads, told, parts):
+    """Partitions get longer than two tiles only where rows much shorter than
+    the bound do not pay for it: captured steps are told the longest that
+    rows may become."""
+    assert hip._mla_split(rows, heads, told) == parts
+
+
+def test_mla_heads_of_a_workgroup_as_the_kernel_plans_them():
+    """_mla_split counts on the rule of csrc/mla.hip."""
+    try:
+        from vllm_amd.ops import hip_ops
+    except (ImportError, OSError) as e:
+        pytest.skip(f"extension not built: {e}")
+    seen = set()
+    for heads in (1, 16, 32, 33, 64, 65, 72, 100, 128, 129, 160, 256):
+        for pairs in (0, 1, 15, 16, 32, 63, 64, 65, 85, 86, 127, 128, 129, 255,
+                      256, 257, 4096, 1 << 20):
+            n = hip_ops._mla_group_heads(pairs, heads)
+            assert n == torch.ops.vllm_amd.mla_group_heads(pairs, heads)
+            seen.add(n)
+    assert seen == {32, 64, 128}
+
+
 @pytest.mark.parametrize("rows,kv,span,window,parts", [
     (1, 8, 1000, 0, 8),       # none shorter than 128 keys
     (1, 8, 8192, 0, 32),      # one workgroup a CU ...

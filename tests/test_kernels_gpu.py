@@ -694,10 +694,7 @@ def test_mla_decode_kernel(T, Hq, ctx):
 def test_mla_decode_head_groups(T, Hq, wide, bound):
     hip = _hip()
     parts = hip._mla_split(T, Hq, bound)
-    n = 128
-    while n > 32 and Hq > n // 2 and T * parts * -(-Hq // (n // 2)) <= 256:
-        n //= 2
-    assert n == wide
+    assert hip._C.mla_group_heads(T * parts, Hq) == wide
     ctx = [1 + (bound - 1) * i // max(T - 1, 1) for i in range(T - 1)] + [bound]
     nb = -(-bound // 64)
     kv = torch.randn(T * nb, 64, 576, dtype=torch.bfloat16, device="cuda")

@@ -424,6 +424,10 @@ static int group_heads(int64_t pairs, int64_t Hq) {
 
 }  // namespace mla
 
+int64_t mla_group_heads(int64_t pairs, int64_t heads) {
+  return mla::group_heads(pairs, heads);
+}
+
 // Decode rows; the scratch says into how many partitions their keys go.
 void mla_decode(torch::Tensor out, torch::Tensor q_nope, torch::Tensor q_pe,
                 torch::Tensor kv_cache, torch::Tensor block_table,

@@ -335,46 +335,58 @@ def _mla_parts(rows, heads, max_seq_len):
                       -(-max_seq_len // _MLA_PART_MIN), 64))
 
 
+def _mla_group_heads(pairs, heads):
+    """Heads that a workgroup takes (csrc/mla.hip, group_heads) of so many
+    rows and partitions: the fewest of 32, 64 and 128 that one round of
+    workgroups has room for."""
+    n = 128
+    while n > 32 and heads > n // 2 and pairs * -(-heads // (n // 2)) <= _MLA_FILL:
+        n //= 2
+    return n
+
+
 @functools.lru_cache(maxsize=1024)
 def _mla_split(rows, heads, max_seq_len):
     """Into how many partitions the kernel splits a row's keys: as
     _mla_parts says or, where that is 5 % less by an estimate, as many as
-    leave room for workgroups of fewer heads (the kernel takes the fewest
-    of 32, 64 and 128 that one round of workgroups has room for). The
-    estimate, in us: a start and the queries' way in, tiles of 64 keys, and
-    with partitions a launch and their traffic. Its coefficients come from a
-    fit of 528 times at 16, 64 and 128 heads, 1 to 200 rows and 60 to 16000
-    keys, which they meet within 5 %; the choice is 9 % faster than
-    _mla_parts on average and slower nowhere among them."""
-    def wide(parts):
-        n = 128
-        while (n > 32 and heads > n // 2
-               and rows * parts * -(-heads // (n // 2)) <= _MLA_FILL):
-            n //= 2
-        return n
+    leave room for workgroups of fewer heads. The estimate, in us: a start and the queries' way in,
+    tiles of 64 keys, and with partitions a launch and their traffic. Its
+    coefficients come from a fit of 528 times at 16, 64 and 128 heads, 1 to
+    200 rows and 60 to 16000 keys, which they meet within 5 %.
+    max_seq_len is a bound, for captured steps the longest that rows may
+    become: longer partitions must not be behind either where rows have a
+    quarter or a sixteenth of it (4 rows, 64 heads, told 8192: of 491 keys
+    16.0 in 64 partitions, 20.4 in 32). Of 820 times at 16 to 128 heads, 1 to
+    160 rows, told 100 to 16384 keys and having all, 0.6, a quarter or 0.06
+    of them, 0.89 of _mla_parts' on average; 26 above 1.02, all at less than
+    35 us, the worst 1.09 (64 rows, 16 heads, 120 keys told 200: 11.5)."""
+    first = _mla_parts(rows, heads, max_seq_len)
 
-    def us(parts):
-        n = wide(parts)
-        groups = rows * parts * -(-heads // n)
-        took = min(n, heads)
+    def us(parts, keys):
+        wide = _mla_group_heads(rows * parts, heads)
+        took = min(wide, heads)
+        part_tiles = max(1, -(-max_seq_len // (64 * parts)))
+        used = min(parts, -(-keys // (64 * part_tiles)))
+        groups = rows * used * -(-heads // wide)
         tile = 2.1 if took <= 32 else 2.3 if took <= 64 else 3.15
-        tiles = -(-max_seq_len // (64 * parts)) * -(-groups // _MLA_FILL)
+        tiles = min(part_tiles, -(-keys // 64)) * -(-groups // _MLA_FILL)
         t = (3.8 + 9.8 * took / 128
              + tiles * tile * (1 + 0.25 * min(groups / _MLA_FILL, 1)))
         if parts > 1:
-            t += 2.2 + 0.16 * parts + rows * parts * heads * 4.5e-4
+            t += 2.2 + 0.16 * used + rows * used * heads * 4.5e-4
         return t
 
-    best = _mla_parts(rows, heads, max_seq_len)
-    least = us(best) * 0.95
+    shorter = [max(1, max_seq_len // n) for n in (4, 16)]
+    limits = [us(first, keys) for keys in shorter]
+    best, least = first, us(first, max_seq_len) * 0.95
     for n in (32, 64):
         room = _MLA_FILL // max(1, rows * -(-heads // n))
-        for keys in (64, 128):
-            parts = min(room, -(-max_seq_len // keys), 64)
-            if parts > 0 and us(parts) < least:
-                best, least = parts, us(parts)
-        if room and us(1) < least:
-            best, least = 1, us(1)
+        parts_of = [min(room, -(-max_seq_len // keys), 64)
+                    for keys in (64, 128)] + [1] * (room > 0)
+        for parts in parts_of:
+            if parts > 0 and us(parts, max_seq_len) < least and all(
+                    us(parts, k) <= u for k, u in zip(shorter, limits)):
+                best, least = parts, us(parts, max_seq_len)
     return best
 
 
