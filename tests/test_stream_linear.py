@@ -243,6 +243,25 @@ SPLIT = [(65, 2104, 7168, 64), (128, 3072, 8256, 64), (200, 2560, 6912, 64),
          (1023, 4096, 14336, 256), (600, 1536, 6208, 128)]
 
 
+def _poison(spare):
+    """All memory that the caching allocator holds free, and `spare` bytes
+    more, is NaN in 16 and in 32 bits; what it has reserved by now."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    more = [torch.empty(n, dtype=torch.uint8, device="cuda")
+            for n in (spare, 1 << 20)]   # large ones, and small ones apart
+    free = [b["size"] for seg in torch.cuda.memory_snapshot()
+            for b in seg["blocks"] if b["state"] == "inactive"]
+    junk = [torch.empty(n, dtype=torch.uint8, device="cuda") for n in free]
+    for t in more + junk:
+        t.fill_(0xFF)
+    del more, junk, t
+    left = [b["size"] for seg in torch.cuda.memory_snapshot()
+            for b in seg["blocks"] if b["state"] == "inactive"]
+    assert sum(left) >= spare
+    return torch.cuda.memory_reserved()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k,cols", SPLIT)
@@ -251,10 +270,12 @@ def test_tiles_in_parts(m, n, k, cols, dtype):
     kind, tile, parts = _form(m, n, k)
     assert (kind, tile) == (2, cols) and (parts > 1 or n >= 16384)
     x, w = _operands(m, n, k, dtype)
-    # What is read is written first: scratch that holds NaN.
-    junk = torch.full((64 << 20,), float("nan"), device="cuda")
-    del junk
+    # What is read is written first: wherever the scratch comes from, it
+    # holds NaN.
+    reserved = _poison(256 << 20)
     out = hip_ops.linear(x, w)
+    torch.cuda.synchronize()
+    assert torch.cuda.memory_reserved() == reserved
     _check(out, x.float() @ w.float().t(), dtype, k)
     assert torch.equal(out, hip_ops.linear(x, w))
 
