@@ -88,9 +88,16 @@ constexpr int dec_keys =
 
 // Parts of a key row that lie on neighbouring lanes: one load of 16 / S rows
 // then takes whole lines of 128 B. (A row of 64 B is taken whole as it is.)
-template <typename CTag, int HD>
+// Where a wave is a row and the cache has 8 bits, half lines are ahead: a step
+// of 32 keys is one load a lane either way, and the sums of two lanes come on
+// top (us, whole and half lines, 16/8 heads: 600 rows x 1..350 keys 53.3 and
+// 47.7, from HBM 74 and 71; 1000 x 1..120 the same).
+template <typename CTag, int HD, int WPR>
 constexpr int dec_split =
-    HD * sizeof(typename CacheTraits<CTag>::elem) >= 128 ? 2 : 1;
+    HD * sizeof(typename CacheTraits<CTag>::elem) >= 128 &&
+            (WPR > 1 || sizeof(typename CacheTraits<CTag>::elem) == 2)
+        ? 2
+        : 1;
 
 // First key this row attends, rounded down so that a wave's 32 keys
 // never leave a cache block.
@@ -141,7 +148,7 @@ DEVINL void decode_rows(const DecodeArgs<CTag>& a, const int kvh,
   constexpr int KEYS = dec_keys<CTag, HD>;
   constexpr int KT = KEYS / 16;                   // score tiles
   constexpr int KF = HD / 32;                     // MFMA steps over D
-  constexpr int S = dec_split<CTag, HD>;
+  constexpr int S = dec_split<CTag, HD, WPR>;
   static_assert(MAX_GROUP * S <= 16);
   constexpr int NT = KT * S;                      // loaded tiles of 16 / S keys
   constexpr int KN = HD * (int)sizeof(elem) / 64 / S;   // 16 B K loads of one
