@@ -38,7 +38,8 @@ constexpr int max_lds(int a, int b) { return a > b ? a : b; }
 struct Mix { int tiles, rows, spread, num_prefills; };
 
 template <typename Tag, typename CTag, bool WHOLE, int HD>
-__global__ __launch_bounds__(PF_BLOCK, 2) void mixed_attention_kernel(
+__global__ __launch_bounds__(PF_BLOCK, pf_per_cu<HD>)
+void mixed_attention_kernel(
     const DecodeArgs<CTag> d, const PrefillArgs<CTag> p, const Mix mix) {
   static_assert(PF_BLOCK == DEC_BLOCK);
   __shared__ __align__(16) char lds[max_lds(pf_lds<HD>, dec_lds<CTag, HD>)];

@@ -99,6 +99,12 @@ template <typename CTag> struct PrefillArgs {
 
 // Bytes of LDS of a workgroup: two tiles each of keys and of values.
 template <int HD> constexpr int pf_lds = 4 * KVTILE * HD * 2;
+// Workgroups that a CU is to hold, by registers. Three with heads of 64: an
+// 8-bit cache left to itself takes two registers too many for that, and short
+// prompts wait for a second round (53 of 124 tokens, 32/4 heads 25.1 us, so
+// 21.6; 23 of 107, 32/8 heads 12.0 and 10.5). Four spill (1.25 to 1.4 times).
+template <int HD>
+constexpr int pf_per_cu = HD == 256 ? 1 : HD == 64 ? 3 : 2;
 
 // Tile `from_last` of a request's rows, counted from the last one.
 template <typename Tag, typename CTag, int HD>
@@ -244,7 +250,8 @@ DEVINL void prefill_tile(const PrefillArgs<CTag>& a, const int kvh,
   // Products of a step in their order: the first and the second 32 keys of the
   // next tile's scores, then the four chunks of 16 keys of this one's results.
   constexpr int QK = 2 * KF, ALL = QK + 4 * DS;
-  constexpr int AHEAD = 4;                       // fragments read ahead
+  // Fragments read ahead (with a fourth there would be scratch for these).
+  constexpr int AHEAD = FP8 && HD == 64 ? 3 : 4;
   int k_at[KF], v_at[DS];   // first fragments of a tile, in its bytes
 #pragma unroll
   for (int kk = 0; kk < KF; ++kk)

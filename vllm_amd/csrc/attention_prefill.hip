@@ -8,7 +8,7 @@
 namespace vllm_amd {
 
 template <typename Tag, typename CTag, int HD>
-__global__ __launch_bounds__(PF_BLOCK, HD == 256 ? 1 : 2)
+__global__ __launch_bounds__(PF_BLOCK, pf_per_cu<HD>)
 void prefill_attention_kernel(const PrefillArgs<CTag> a,
                               const int num_decodes) {
   __shared__ __align__(16) char lds[pf_lds<HD>];
