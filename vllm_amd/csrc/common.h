@@ -10,6 +10,7 @@
 
 #include <cstdint>
 #include <type_traits>
+#include <utility>
 
 #define WAVE_SIZE 64
 
@@ -172,6 +173,17 @@ template <int N, int M> DEVINL void acc_fence(f32x4 (&acc)[N][M]) {
 #pragma unroll
     for (int j = 0; j < M; ++j) asm volatile("" : "+a"(acc[i][j]));
   asm volatile("s_nop 15");
+}
+
+// f(0) to f(N - 1), each with its number as a constant. (Unrolled loops stay
+// loops where their bodies are long, and arrays of registers then go to
+// scratch.)
+template <int N, typename F, int... I>
+DEVINL void unrolled(F f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F> DEVINL void unrolled(F f) {
+  unrolled<N>(f, std::make_integer_sequence<int, N>{});
 }
 
 // Two floats rounded (nearest even) to a packed 16-bit pair.
@@ -348,6 +360,27 @@ DEVINL void lds_fill16_once(const void* base, uint32_t at, void* dst) {
       :
       : "s"(to), "v"(at), "s"(base)
       : "memory", "m0");
+}
+// mfma16_acc and, behind it, a fill of the 16 * 64 bytes `off` after `to` (an
+// address in LDS; off a constant). The place goes to m0 before the product, so
+// that the wait between the two holds the product, and the next product does
+// not wait for the instructions of a fill of its own.
+template <bool ONCE, typename Tag>
+DEVINL void mfma16_acc_fill(f32x4& c, s16x8 a, s16x8 b, const void* base,
+                            uint32_t at, uint32_t to, int off) {
+#define VLLM_AMD_PRODUCT_FILL(TYPE, HINT)                          \
+  asm volatile("s_add_u32 m0, %3, %4\n\t"                          \
+               "v_mfma_f32_16x16x32_" TYPE " %0, %1, %2, %0\n\t"   \
+               "global_load_lds_dwordx4 %5, %6" HINT               \
+               : "+a"(c)                                           \
+               : "v"(a), "v"(b), "s"(to), "i"(off), "v"(at), "s"(base) \
+               : "memory", "m0", "scc")
+  constexpr bool BF16 = std::is_same_v<Tag, BF16Tag>;
+  if constexpr (BF16 && ONCE)      VLLM_AMD_PRODUCT_FILL("bf16", " nt");
+  else if constexpr (BF16)         VLLM_AMD_PRODUCT_FILL("bf16", "");
+  else if constexpr (ONCE)         VLLM_AMD_PRODUCT_FILL("f16", " nt");
+  else                             VLLM_AMD_PRODUCT_FILL("f16", "");
+#undef VLLM_AMD_PRODUCT_FILL
 }
 // At most N (< 64) of this wave's loads still under way; the builtin, so
 // that the compiler knows its own older loads to be done as well and does

@@ -67,10 +67,10 @@ DEVINL void tile_body(char* lds, const TileArgs& t, const short* w,
     wp[i] = (uint32_t)src * (uint32_t)t.K * 2 +
             ((lane & 7) ^ tp_swap(r)) * 16;
   }
-  P::run(
+  P::template run<false>(
       lds, t.K / TP_K, rows,
-      [&](int s, int i, char* dst) { lds_fill16(t.a + s * TP_K, ap[i], dst); },
-      [&](int s, int i, char* dst) { lds_fill16(w + s * TP_K, wp[i], dst); },
+      [&](int s, int i) { return FillSource{t.a + s * TP_K, ap[i]}; },
+      [&](int s, int i) { return FillSource{w + s * TP_K, wp[i]}; },
       [&](auto n, auto& acc) {
         constexpr int J = decltype(n)::value;
         constexpr int NO = GATED ? P::NI / 2 : P::NI;

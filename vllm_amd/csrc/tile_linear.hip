@@ -94,13 +94,10 @@ __global__ __launch_bounds__(TP_THREADS, 1) void tile_linear_kernel(
     wp[i] = (uint32_t)src * (uint32_t)(K * 2) +
             ((lane & 7) ^ tp_swap(r)) * 16;
   }
-  P::run(
+  P::template run<ONCE>(
       lds, steps, rows,
-      [&](int s, int i, char* dst) { lds_fill16(xt + stage(s), ap[i], dst); },
-      [&](int s, int i, char* dst) {
-        if constexpr (ONCE) lds_fill16_once(wt + stage(s), wp[i], dst);
-        else lds_fill16(wt + stage(s), wp[i], dst);
-      },
+      [&](int s, int i) { return FillSource{xt + stage(s), ap[i]}; },
+      [&](int s, int i) { return FillSource{wt + stage(s), wp[i]}; },
       [&](auto n, auto& acc) {
         constexpr int J = decltype(n)::value;
         const int wm = wave / P::WGN, wn = wave % P::WGN;
