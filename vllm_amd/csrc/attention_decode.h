@@ -17,10 +17,15 @@
 //     half of the queries' columns, and two neighbouring rows of the
 //     fragment the halves of one key: the same products, but a load takes
 //     whole lines of 8 keys instead of half lines of 16, and a score is the
-//     sum of two lanes (one rotation). us on caches from HBM: 256 x
-//     129..2176 keys 210 -> 203, 64 x 4096..8192, fp8 cache 147 -> 144, 64 x
-//     100..4000, 28/4 heads 63 -> 58, 64 x 1000..4000, 16/4 heads of 256 126
-//     -> 119, 1 x 1000 8.7 -> 8.1; by quarters of a group of 4 no faster.
+//     sum of two lanes (one rotation). us, half lines and whole, marked as
+//     below: keys that no cache holds, 32 x 4096 keys 108 and 91, 64 x 4096 221
+//     and 179, 1 x 1000 8.7 and 8.2, 16 x 128 6.2 and 5.3, 4 x 20 4.44 and
+//     4.46; keys that the last-level cache may hold in part, 256 x 129..2176
+//     210 and 203, 64 x 4096..8192 with an 8-bit cache 147 and 145, 32 x 4096
+//     87 either way. By quarters of a group of 4 no faster. What a window of
+//     1024 keys reads again and again from the last-level cache is 8 % slower
+//     (119 x 5600, 28/4 heads 44 and 48; from memory 80 and 56), rows of up to
+//     60 keys in L2 0.1 us.
 //   - O^T = V^T P^T: V passes through this wave's own LDS slice to be
 //     transposed on the read. The lane that holds the scores of keys
 //     (4g..4g+3, 16+4g..) holds exactly the P^T fragment of those keys
@@ -32,7 +37,8 @@
 //     of them common, 32 heads ungrouped, 135 us; half lines of keys, which had
 //     to stay in L2 for the other half, 164, and nothing marked 147.) Where a
 //     wave is a row of few keys, keys are not marked: what a step holds past
-//     the row's end repeats its last key (200 x 1..60 keys 9.8 us, marked 10.2).
+//     the row's end repeats its last key (200 x 1..60 keys 9.8 us, marked
+//     10.2).
 //   - P stays at more than 16 bits: it is split in two 16-bit parts
 //     (p = hi + lo, error 2^-17) and multiplied twice; the matrix cores
 //     are idle here anyway. Sums and outputs are fp32. Results are as far
@@ -43,8 +49,9 @@
 // products reduced with shuffles), us per layer at 32 query and 8 KV
 // heads of 128:
 //   1 x 1000 keys 46 -> 8; 256 x 129..2176 keys 349 -> 203 (6.0 TB/s);
-//   1024 x 129..176 keys 206 -> 107 (132 with the last 32 keys of a row read
-//   whole); 16 x 4096 keys 47; 64 x 4096..8192 keys, fp8 cache 371 -> 144.
+//   1024 x 129..176 keys 206 -> 108 (132 with the last 32 keys of a row read
+//   whole), 118 between the other work of a model's layer; 16 x 4096 keys 46;
+//   64 x 4096..8192 keys, fp8 cache 371 -> 145.
 //
 // The KV cache layout [2, blocks, kv_heads, block_size=64, D] keeps each
 // (block, head) tile contiguous (16 KB at D=128).

@@ -11,10 +11,10 @@
 //   - A wave's vector work runs under its own products: the maximum of a
 //     tile's scores under the first half of the next tile's, its weights
 //     under the second half and under the results of the weights before them
-//     (one after the other, two waves a SIMD: matrix cores 44 % and vector ALU
-//     49 % of the cycles, hardly any at once; now 59 %). Scheduling barriers
-//     pin the order; other shares of products a group, 3 to 8 fragments read
-//     ahead and wave priorities measured the same.
+//     (one after the other, two waves a SIMD: matrix cores 42 % and vector ALU
+//     46 % of the cycles, hardly any at once; now 55 and 52 %). Scheduling
+//     barriers pin the order; other shares of products a group, 3 to 8 fragments
+//     read ahead and wave priorities measured the same.
 //   - The rows of a tile are (token, query head) pairs of ONE KV head:
 //     the heads of a group share every K/V tile they read, the causal
 //     edge of a tile is only 128 / group tokens wide, and a short

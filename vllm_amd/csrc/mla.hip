@@ -34,14 +34,14 @@
 //     one and the rounded weights are summed: 3 % slower, 4 % closer to
 //     64-bit results.
 // Rows are split over a few partitions of the keys, and heads over workgroups
-// (group_heads below), when there are fewer than CUs; fp32 partials (256 KB per row and partition) are merged by
-// mla_reduce_kernel, so partitions are few and long, and rows that fit one
-// are written at once. A portion of 2 tokens after 8190 takes 56 us in
-// 64 partitions, with the products around it, and 510 in one.
-// 128 heads: 128 rows x 129..2176 keys 1025 -> 88 us with the merge (four
-// waves of 16 heads on 32-key tiles, V stored transposed, before); prompts
-// of 300, 1300 and 2301 tokens 1.32 ms (750 TFLOP/s counting P once; a
-// composition of library products in fp32 before, 24 ms).
+// (group_heads below), when there are fewer than CUs; fp32 partials (256 KB per
+// row and partition) are merged by mla_reduce_kernel, so partitions are few and
+// long, and rows that fit one are written at once. A portion of 2 tokens after
+// 8190 takes 56 us in 64 partitions, with the products around it, and 510 in
+// one. 128 heads: 128 rows x 129..2176 keys 1025 -> 88 us with the merge (four
+// waves of 16 heads on 32-key tiles, V stored transposed, before); prompts of
+// 300, 1300 and 2301 tokens 1.32 ms (750 TFLOP/s counting P once; a composition
+// of library products in fp32 before, 24 ms).
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>

@@ -2,9 +2,9 @@
 // 256 tiles of tile_product.h, the matrix cores bound them. The product is
 // formed transposed (weight rows are the A operand), so a lane ends up with
 // four neighbouring columns of one row, eight after a trade with another
-// quarter of the wave (16 B stores). Gated experts: a tile is 128 gate rows and the up
-// rows of the same columns, a wave's gate groups before its up groups, and
-// the activation is the epilogue.
+// quarter of the wave (16 B stores). Gated experts: a tile is 128 gate rows and
+// the up rows of the same columns, a wave's gate groups before its up groups,
+// and the activation is the epilogue.
 //
 // Tiles of at most 128 rows (what is left of an expert after whole tiles,
 // or experts of few rows) lay the four waves out along the weights; 32-row
@@ -20,9 +20,10 @@
 // 64 experts of 7168 x 2048, 4096 tokens of 8, 50 to 1925 rows an expert:
 // 1.76 + 0.95 ms (eight waves by halves in turn 2.01 + 1.10); 512 rows each
 // 1.47 + 0.84 (1.31 and 1.14 PFLOP/s: the second, of 32 stages, pays the start
-// and end of its tiles; by products of 32 x 32 x 16 1.50 + 0.86). What uneven rows cost beyond their
-// padding is weights read twice: tiles of an expert that are not in step do not
-// meet in L2 (8.3 GB instead of 4.1 in the first product).
+// and end of its tiles; by products of 32 x 32 x 16 1.50 + 0.86). What uneven
+// rows cost beyond their padding is weights read twice: tiles of an expert that
+// are not in step do not meet in L2 (8.3 GB instead of 4.1 in the first
+// product).
 
 #include <torch/all.h>
 #include <c10/hip/HIPStream.h>

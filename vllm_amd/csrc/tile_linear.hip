@@ -3,16 +3,18 @@
 // with silu(gate) * up of two halves of w as the epilogue.
 //
 // Between bound by the weights' way from HBM and by what a CU takes in: rows of
-// x come from L2, but behind weights that are still under way, and a CU keeps
-// about 64 KB under way, so both together come at 50 to 60 GB/s a CU (125 where
-// nothing comes from HBM).
+// x come from L2 (100 GB/s a CU, alone), weights from HBM (23 GB/s a CU where
+// all read, 5.9 TB/s), and where both come one waits for the other rather than
+// beside it, however much is under way: 128 rows of x and 64 of weights a stage
+// at 49 GB/s a CU (4.2 TB/s of weights), 256 and 64 at 59 (3.0), 256 and 128 at
+// 58 (4.9), 128 and 128 at 46 (5.9).
 //
 //  * Weights that one workgroup reads leave L2 first; x stays.
 //  * Workgroups begin at different stages of K, those of an XCD that share
 //    weights at the same one (tile_job): rows whose stride is a power of two
-//    meet on few channels otherwise. A window of some 60 stages, so that x stays in L2. 128 rows of
-//    weights alone at K = 16384 5.4 -> 7.0 TB/s; 28672 x 4096 with the
-//    activation, 128 rows 57 -> 52 us.
+//    meet on few channels otherwise. A window of some 60 stages, so that x
+//    stays in L2. 128 rows of weights alone at K = 16384 5.4 -> 7.0 TB/s; 28672
+//    x 4096 with the activation, 128 rows 57 -> 52 us.
 //  * Layers with few tiles split K over workgroups until about one a CU runs,
 //    if K is long enough for the partial sums not to cost what that gains
 //    (by_estimate below); a second launch adds them.
@@ -186,9 +188,9 @@ __global__ __launch_bounds__(256) void tile_sums_kernel(
 
 // us of a product in tiles of `cols` weight rows with K in `parts`, for at most
 // 256 workgroups. A stage of 64 columns of K: what a CU takes in, rows of x and
-// weights, at 76 GB/s (one that has reads from HBM under way takes in no more,
-// whatever comes from L2 beside them); the weights' way from HBM; products.
-// These are coefficients of a fit and not bounds: 1800 times of 33 layers of
+// weights; the weights' way from HBM; products, each by a rate, and between
+// their sum and the largest. The rates (a CU's 76 GB/s and 10.8 TFLOP/s, 8 TB/s) are
+// coefficients of a fit and not bounds: 1800 times of 33 layers of
 // 512 x 7168 to 36864 x 7168 on 72 to 1024 rows are within 7 % of it (rms), and
 // the form that it prefers is 0.7 % slower than the best one on average.
 double estimate(int64_t M, int64_t N, int64_t K, int cols, int parts) {
@@ -215,20 +217,21 @@ double estimate(int64_t M, int64_t N, int64_t K, int cols, int parts) {
 // 20 us. Below 1536 columns of output there is too little to split. us, the
 // library and this (at 128, 256 and 1024 rows if not said): 4096 x 14336 52 /
 // 34, 65 / 45, 137 / 116; 3584 x 18944 65 / 40, 80 / 52, 173 / 132; 7168 x
-// 16384 71 / 54, 107 / 72, and 512 rows 148 / 117; 2112 x 7168 25 / 17, 32 / 24,
-// 49 / 45. On the other side of the lines: 4096 x 4096 17.3 / 17.0, 21.0 / 25.1,
-// 41 / 50; 4096 x 7168, 1024 rows 69 / 74; 8192 x 28672, 768 rows 301 / 316; 512
-// x 7168, 256 rows 12 / 15.6. Of 2300 sizes inside 0.74 of the library's time
-// on average, one above 1.02 (1.026).
+// 16384 71 / 54, 107 / 72, and 512 rows 148 / 117; 2112 x 7168 25 / 17, 32 /
+// 24, 49 / 45. On the other side of the lines: 4096 x 4096 17.3 / 17.0, 21.0 /
+// 25.1, 41 / 50; 4096 x 7168, 1024 rows 69 / 74; 8192 x 28672, 768 rows 301 /
+// 316; 512 x 7168, 256 rows 12 / 15.6. Of 2300 sizes inside 0.74 of the
+// library's time on average, one above 1.02 (1.026).
 //
 // With K whole, up to 256 rows: 65 %, and 75 % where K is long (the library
-// begins K at several places: 19712 x 9728, 148 rows, 60 % busy 105 / 113; 39680
-// x 10240, 68 rows, 61 % 157 / 169; 22272 x 5632, 95 rows, 68 % 57 / 61; 43456 x
-// 11968, 154 rows, 66 % 216 / 229; inside 22016 x 4096, 192 rows, 67 % 62 / 52).
-// Tiles of 64 take x in for few weights: up to 128 rows 60 % are enough (24576 x
-// 1536 27.6 / 23.0), above only nearly all, and K up to 5120 (256 rows: 16384 x
-// 4096 52 / 48, 71 % 11568 x 4096 39 / 45, 88 % 14336 x 4096 45 / 47; 15872 x
-// 7168 78 / 82). Of 1200 sizes inside 0.87 on average, two above 1.03 (1.05).
+// begins K at several places: 19712 x 9728, 148 rows, 60 % busy 105 / 113;
+// 39680 x 10240, 68 rows, 61 % 157 / 169; 22272 x 5632, 95 rows, 68 % 57 / 61;
+// 43456 x 11968, 154 rows, 66 % 216 / 229; inside 22016 x 4096, 192 rows, 67 %
+// 62 / 52). Tiles of 64 take x in for few weights: up to 128 rows 60 % are
+// enough (24576 x 1536 27.6 / 23.0), above only nearly all, and K up to 5120
+// (256 rows: 16384 x 4096 52 / 48, 71 % 11568 x 4096 39 / 45, 88 % 14336 x 4096
+// 45 / 47; 15872 x 7168 78 / 82). Of 1200 sizes inside 0.87 on average, two
+// above 1.03 (1.05).
 TileForm by_estimate(int64_t M, int64_t N, int64_t K) {
   TileForm best{0, 1};
   if (M > 1024) return best;
@@ -272,15 +275,16 @@ TileForm by_estimate(int64_t M, int64_t N, int64_t K) {
 // and 75; 102400 x 2048 (0.78 of two rounds) 96 and 80, 152064 x 3584 216 and
 // 207; 57344 x 8192 with the activation 159 and 146; 28672 x 4096 with it 41.9
 // and 40.9; on 33 and 64 rows 5120 x 10240 27.3 and 24.8, 29.7 and 25.9; 3072 x
-// 12288 23.0 and 21.6, 25.5 and 22.4; 8192 x 10240 35.1 and 33.5, 38.5 and 34.7;
-// 7168 x 16384 on 64 52.9 and 45.0, 8192 x 28672 103 and 83. On the other side:
-// 145000 x 5504 by tiles of 128 311 and 330; 24576 x 1536 18.1 and 18.7; 12288 x
-// 5120 29.5 and 31.0; 8192 x 8192 on 33 and 64 27.9 and 31.1, 29.7 and 31.1; 5120
-// x 8192 on 33 21.8 and 22.0; 2560 x 10752 on 48 4 % behind; 22880 x 12096 on 40
-// 13 % (two parts). Where all CUs take gate and up rows at a stride of 8 KB they
-// meet on few channels: 32768 x 4096 with the activation 43.3 and 50.4, 31600 x
-// 4096 42.6 and 42.0. 8100 sizes inside: 0.90 of stream_linear's time on average,
-// one in 180 above 1.02, seven above 1.05 (1.074: 7168 x 13312 on 33).
+// 12288 23.0 and 21.6, 25.5 and 22.4; 8192 x 10240 35.1 and 33.5, 38.5 and
+// 34.7; 7168 x 16384 on 64 52.9 and 45.0, 8192 x 28672 103 and 83. On the other
+// side: 145000 x 5504 by tiles of 128 311 and 330; 24576 x 1536 18.1 and 18.7;
+// 12288 x 5120 29.5 and 31.0; 8192 x 8192 on 33 and 64 27.9 and 31.1, 29.7 and
+// 31.1; 5120 x 8192 on 33 21.8 and 22.0; 2560 x 10752 on 48 4 % behind; 22880 x
+// 12096 on 40 13 % (two parts). Where all CUs take gate and up rows at a stride
+// of 8 KB they meet on few channels: 32768 x 4096 with the activation 43.3 and
+// 50.4, 31600 x 4096 42.6 and 42.0. 8100 sizes inside: 0.90 of stream_linear's
+// time on average, one in 180 above 1.02, seven above 1.05 (1.074: 7168 x 13312
+// on 33).
 //
 // The share of its rounds over 256 CUs that a form keeps busy decides: 256
 // where that is at least 95 % (for up to 128 rows of a plain product in more

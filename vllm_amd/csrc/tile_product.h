@@ -8,7 +8,7 @@
 // three quarters of the cycles, at 1.7 to 1.8 GHz. Products of 16 x 16 x 32
 // move half the accumulators per flop that those of 32 x 32 x 16 do (random
 // values from registers alone: 2.02 and 1.77 PFLOP/s). Small ones what a CU
-// takes in: about 64 KB are under way, so 50 to 60 GB/s beside reads from HBM.
+// takes in: 46 to 60 GB/s of rows from L2 and weights from HBM together.
 //  * A wave of 128 x 128 reads 16 fragments of 16 x 32 from LDS for 64 products
 //    (half of what LDS gives; eight waves of 64 x 128 read 96 B a clock, and
 //    with what is filled that is all there is). With one wave a SIMD nothing
