@@ -620,6 +620,25 @@ def test_moe_grouped_gemm_kernel(T, H, I, E, K):
     assert_close(out, expect, atol=8e-2, rtol=8e-2)
 
 
+# An expert of more row tiles than a wave finds at a time, between one of a row
+# and one of a group and a tile.
+def test_moe_expert_of_many_tiles():
+    hip = _hip()
+    H, I, E = 128, 64, 4
+    rows = [1, 66 * 256 + 5, 2300, 0]
+    T = sum(rows)
+    assert hip._moe_form(T, T, E, H) == 2
+    hidden = torch.randn(T, H, dtype=torch.bfloat16, device="cuda") * 0.3
+    w13 = torch.randn(E, 2 * I, H, dtype=torch.bfloat16, device="cuda") * 0.2
+    w2 = torch.randn(E, H, I, dtype=torch.bfloat16, device="cuda") * 0.2
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))
+    ids = ids[torch.randperm(T)].view(T, 1).cuda()
+    w = torch.rand(T, 1, device="cuda")
+    out = hip.fused_moe_hip(hidden, w13, w2, w, ids)
+    expect = ref.fused_moe(hidden.float(), w13.float(), w2.float(), w, ids)
+    assert_close(out, expect, atol=8e-2, rtol=8e-2)
+
+
 # Captured under inference mode like the engine's own captures: the
 # default CUDA generator's capture state may have been created by an
 # earlier inference-mode step, and capture_begin updates it in place.

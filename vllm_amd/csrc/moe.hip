@@ -457,6 +457,30 @@ int64_t moe_tile_rows(int64_t form) {
   return form == 2 ? 256 : form == 1 ? 128 : moe::BM;
 }
 
+// For the tests: {XCD, row tile, column block} of every tile in the order of
+// its workgroup, where expert_of[i] is the expert of row tile i.
+std::vector<int64_t> moe_tile_order(std::vector<int64_t> expert_of,
+                                    int64_t n_blocks, int64_t split) {
+  using namespace moe;
+  std::vector<int64_t> out;
+  const int tiles = (int)expert_of.size();
+  for (int xcd = 0; xcd < 8; ++xcd) {
+    const TilePart p = tile_part_of(xcd, tiles, (int)n_blocks, (int)split);
+    const int blocks = p.n1 - p.n0;
+    const bool one = p.m1 - p.m0 <= TILE_GROUP;
+    for (int l = 0; l < (p.m1 - p.m0) * blocks; ++l) {
+      int first = p.m0 + l / blocks, end = first, m, n;
+      const int64_t expert = expert_of[first];
+      while (first > p.m0 && (one || expert_of[first - 1] == expert)) --first;
+      while (end < p.m1 && (one || expert_of[end] == expert)) ++end;
+      tile_of_run(first, end - first, blocks, l - (first - p.m0) * blocks, m,
+                  n);
+      out.insert(out.end(), {xcd, m, n + p.n0});
+    }
+  }
+  return out;
+}
+
 // scratch: ceil(total / 2048) * num_experts ints where total > 2048, and
 // 2 * num_experts more for more than 1024 experts.
 void moe_align(torch::Tensor topk_ids, int64_t num_experts, int64_t tile_rows,
