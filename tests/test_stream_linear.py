@@ -121,6 +121,168 @@ def test_forms(n, k, dtype, rows):
                    torch.nn.functional.silu(gate) * up, dtype, k)
 
 
+# Products of norms: every form on up to 16 rows, K whole and split, steps that
+# end within the eight of a fill of gains, rows that end within eight.
+NORMS = [(1, 24, 64), (8, 2624, 7168), (3, 6144, 4096), (9, 6144, 4096),
+         (16, 28672, 4096), (2, 28672, 4096), (7, 4608, 3584), (1, 832, 576),
+         (16, 4432, 8256), (5, 8288, 832), (12, 34016, 1088), (8, 64, 14336),
+         (16, 18160, 8192)]
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k", NORMS)
+def test_norm_linear(m, n, k):
+    from vllm_amd.ops import hip_ops
+    assert hip_ops._C.layer_streams(m, k, n, 64, 128, 64)
+    x, w = _operands(m, n, k, torch.bfloat16)
+    x = x * torch.logspace(-6, 3, m, device="cuda")[:, None].bfloat16()
+    torch.manual_seed(m * k + n)
+    gain = 1 + 0.1 * torch.randn(k, device="cuda").bfloat16()
+    bias = torch.randn(n, device="cuda").bfloat16()
+    root = (x.float().square().mean(-1, keepdim=True) + 1e-6).rsqrt()
+    y = x.float() * root * gain.float()
+    expect = y @ w.float().t()
+    # Rows are rounded once, each value by up to 2^-8 of it (half a unit of
+    # the last of 7 stored bits), at random: errors of a sum's terms add up as
+    # roots of sums of squares, and seven deviations (2^-8 / sqrt(3) each at
+    # most) are more than any of these results is off.
+    size = (y.square() @ w.float().square().t()).sqrt()
+
+    def check(out, want):
+        assert (out.float() - want).abs().le(
+            want.abs() * 2.0 ** -8 + 7 * size * 2.0 ** -8 / 3 ** 0.5
+            + 1e-5).all()
+
+    check(hip_ops.norm_linear(x, gain, 1e-6, w), expect)
+    check(hip_ops.norm_linear(x, gain, 1e-6, w, bias), expect + bias.float())
+    if n % 16 == 0:
+        gate, up = expect.chunk(2, -1)
+        # d(silu(g) u) <= 1.1 |u| dg + (|g| + 0.3) du, sizes alike.
+        size = (1.1 * up.abs() + gate.abs() + 0.3) * size.reshape(
+            m, 2, -1).amax(1)
+        check(hip_ops.norm_linear(x, gain, 1e-6, w, silu=True),
+              torch.nn.functional.silu(gate) * up)
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(1, 24, 64), (8, 4096, 4096),
+                                   (9, 2112, 7168), (16, 4104, 14336),
+                                   (33, 4096, 14336), (70, 4096, 4096)])
+def test_linear_add(m, n, k, dtype):
+    from vllm_amd.ops import hip_ops
+    x, w = _operands(m, n, k, dtype)
+    residual = torch.randn(m, n, device="cuda").to(dtype)
+    bias = torch.randn(n, device="cuda").to(dtype)
+    expect = x.float() @ w.float().t() + residual.float()
+    # Where the sum is a launch of its own the product is rounded before.
+    slack = 0 if m <= 16 else (expect - residual.float()).abs().max() * 2e-3
+
+    def check(out, want):
+        unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+        err = (out.float() - want).abs() - want.abs() * unit
+        assert err.max() <= slack * 4 + max(1e-3, k * 2.0 ** -24)
+
+    check(hip_ops.linear_add(x, w, None, residual), expect)
+    check(hip_ops.linear_add(x, w, bias, residual), expect + bias.float())
+
+
+@gpu
+def test_norms_that_are_not_fused_are_the_same():
+    """Rows in fp16 and more rows: a norm, then the product."""
+    from vllm_amd.ops import hip_ops
+    for m, dtype in ((8, torch.float16), (17, torch.bfloat16),
+                     (300, torch.bfloat16)):
+        x, w = _operands(m, 1024, 512, dtype)
+        gain = torch.rand(512, device="cuda").to(dtype)
+        y = hip_ops.rms_norm(x, gain, 1e-5)
+        assert torch.equal(hip_ops.norm_linear(x, gain, 1e-5, w),
+                           hip_ops.linear(y, w))
+        assert torch.equal(hip_ops.norm_linear(x, gain, 1e-5, w, silu=True),
+                           hip_ops.linear_silu_and_mul(y, w))
+
+
+@gpu
+@pytest.mark.parametrize("rows", [1, 8, 16, 17])
+@pytest.mark.parametrize("model", ["llama-3-8b", "qwen2.5-7b"])
+def test_layers_on_the_residual_stream(model, rows):
+    """A step of few rows with norms in products, beside the same step whose
+    last layer has a hook, which keeps every module's call."""
+    import dataclasses
+
+    from vllm_amd import ops
+    from vllm_amd.config import ModelConfig, get_model_spec
+    from vllm_amd.models.registry import get_model_class
+    from vllm_amd.worker.forward_context import (
+        AttentionMetadata, ForwardContext, set_forward_context)
+    spec = dataclasses.replace(get_model_spec(model), num_layers=2,
+                               vocab_size=1024)
+    config = ModelConfig(model=model, dtype="bf16", spec=spec,
+                         max_model_len=256)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows)
+    with torch.inference_mode():
+        with torch.device("cuda"):
+            net = get_model_class(spec.architecture)(config).eval()
+        for p in net.parameters():
+            p.data.normal_(generator=g).mul_(p.shape[-1] ** -0.5)
+            if p.dim() == 1:
+                p.data.add_(1.0)
+        lens = torch.arange(1, rows + 1, device="cuda", dtype=torch.int32)
+        meta = AttentionMetadata(
+            query_start_loc=torch.arange(rows + 1, device="cuda",
+                                         dtype=torch.int32),
+            seq_lens=lens, block_table=torch.arange(
+                rows, device="cuda", dtype=torch.int32)[:, None].contiguous(),
+            slot_mapping=torch.arange(rows, device="cuda") * 64
+            + lens.long() - 1,
+            num_reqs=rows, num_actual_tokens=rows, max_query_len=1,
+            max_seq_len=rows, num_decodes=rows)
+        cache = torch.randn(2, rows, spec.num_kv_heads, 64, spec.head_dim,
+                            device="cuda", generator=g).bfloat16()
+        ids = torch.arange(rows, device="cuda")
+
+        def step():
+            ctx = ForwardContext(attn_metadata=meta, kv_caches=[
+                cache.clone() for _ in range(2)])
+            with set_forward_context(ctx):
+                return net(ids, lens.long() - 1), ctx.kv_caches
+
+        embeds = net.model.embed_tokens(ids)
+        assert net.model.layers[0].streams()
+        assert ops.layer_streams(embeds, *net.model.stream_sizes) == (
+            rows <= 16)
+        out, caches = step()
+        seen = []
+        net.model.layers[1].register_forward_hook(
+            lambda m, args, res: seen.append(res))
+        expect, old = step()
+    assert len(seen) == 1 and seen[0][1] is not None
+    if rows > 16:
+        assert torch.equal(out, expect)
+    # Two layers, each with five roundings by 2^-8 / sqrt(3) of a value at
+    # random: sqrt(10) of them, 0.007 of the result's size, and twice that.
+    for a, b in [(out, expect)] + list(zip(caches, old)):
+        assert ((a.float() - b.float()).norm()
+                <= 0.015 * b.float().norm())
+
+
+def test_layers_that_stream():
+    """Sizes by which layers go without norms of their own."""
+    try:
+        from vllm_amd.ops import hip_ops
+    except (ImportError, OSError) as e:
+        pytest.skip(f"extension not built: {e}")
+    llama = (4096, 6144, 4096, 28672, 14336)
+    takes = hip_ops._C.layer_streams
+    assert takes(1, *llama) and takes(16, *llama) and not takes(17, *llama)
+    assert not takes(0, *llama)
+    assert takes(16, 8192, 10240, 8192, 57344, 28672)
+    assert not takes(8, 4096, 6144, 4096, 28672, 14272)
+    assert not takes(8, 4080, 6144, 4096, 28672, 14336)   # K in steps of 64
+    assert not takes(1, 256, 65536, 256, 2048, 1024)      # wide and short
+
+
 @gpu
 def test_views_and_other_streams():
     """Operands that begin off 16 B take the library; launches on several

@@ -46,6 +46,14 @@ void mixed_attention(torch::Tensor out, torch::Tensor q,
 torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
                         c10::optional<torch::Tensor> bias);
 torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w);
+torch::Tensor linear_add(torch::Tensor a, torch::Tensor w,
+                         c10::optional<torch::Tensor> bias,
+                         torch::Tensor residual);
+torch::Tensor norm_linear(torch::Tensor a, torch::Tensor gains, double eps,
+                          torch::Tensor w, c10::optional<torch::Tensor> bias,
+                          bool silu);
+bool layer_streams(int64_t rows, int64_t hidden, int64_t qkv, int64_t heads,
+                   int64_t gate_up, int64_t inner);
 std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
                                  bool silu);
 std::vector<int64_t> linear_starts(int64_t rows, int64_t weight_rows,
@@ -227,6 +235,13 @@ TORCH_LIBRARY(vllm_amd, m) {
         "Tensor(c!) tmp_lse) -> ()");
   m.def("lt_linear(Tensor a, Tensor w, Tensor? bias) -> Tensor");
   m.def("linear_silu_and_mul(Tensor a, Tensor w) -> Tensor");
+  m.def("linear_add(Tensor a, Tensor w, Tensor? bias, Tensor residual) "
+        "-> Tensor");
+  m.def("norm_linear(Tensor a, Tensor gains, float eps, Tensor w, "
+        "Tensor? bias, bool silu) -> Tensor");
+  m.def("layer_streams(int rows, int hidden, int qkv, int heads, "
+        "int gate_up, int inner) -> bool",
+        &vllm_amd::layer_streams);
   m.def("linear_form(int rows, int weight_rows, int k, bool silu) -> int[]",
         &vllm_amd::linear_form);
   m.def("linear_starts(int rows, int weight_rows, int k, bool silu) -> int[]",
@@ -362,6 +377,8 @@ TORCH_LIBRARY_IMPL(vllm_amd, CUDA, m) {
   m.impl("mixed_attention", &vllm_amd::mixed_attention);
   m.impl("lt_linear", &vllm_amd::lt_linear);
   m.impl("linear_silu_and_mul", &vllm_amd::linear_silu_and_mul);
+  m.impl("linear_add", &vllm_amd::linear_add);
+  m.impl("norm_linear", &vllm_amd::norm_linear);
   m.impl("lt_linear_fp8", &vllm_amd::lt_linear_fp8);
   m.impl("dynamic_quant_fp8", &vllm_amd::dynamic_quant_fp8);
   m.impl("scale_rows_cols", &vllm_amd::scale_rows_cols);

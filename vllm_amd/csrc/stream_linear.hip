@@ -53,6 +53,8 @@ namespace vllm_amd {
 torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
                         c10::optional<torch::Tensor> bias);
 torch::Tensor silu_and_mul(torch::Tensor x);
+torch::Tensor rms_norm(torch::Tensor x, torch::Tensor weight, double eps);
+torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w);
 // tile_linear.hip
 bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
                  const torch::Tensor& w, bool silu);
@@ -60,6 +62,7 @@ bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
 namespace {
 
 constexpr int SL_ROWS = 64;      // rows of x at most
+constexpr int SL_NORM_ROWS = 16; // ... that are normalized on their way
 constexpr int SL_PARTS = 8;      // of K, over workgroups
 constexpr int SL_JOBS = 1024;    // column tiles whose K is split
 constexpr int SL_LDS = 160 * 1024;
@@ -80,24 +83,41 @@ constexpr int row_groups(int64_t M) {
 constexpr int ring_bytes(Form f, int xg) {
   return f.wv * f.d * (2 * f.ni + xg) * SP_FILL;
 }
-constexpr int sums_bytes(Form f, int xg) {
-  return f.wv * f.ni * ((xg + 1) / 2) * WAVE_SIZE * 16;
+constexpr int sums_bytes(Form f, int xg, bool norm) {
+  return f.wv * (f.ni * ((xg + 1) / 2) + norm) * WAVE_SIZE * 16;
 }
-constexpr int lds_bytes(Form f, int xg) {
-  return ring_bytes(f, xg) > sums_bytes(f, xg) ? ring_bytes(f, xg)
-                                               : sums_bytes(f, xg);
+// norm_steps: steps of K of a workgroup that takes gains, else 0.
+constexpr int lds_bytes(Form f, int xg, int norm_steps = 0) {
+  const int sums = sums_bytes(f, xg, norm_steps > 0);
+  return (ring_bytes(f, xg) > sums ? ring_bytes(f, xg) : sums) +
+         (norm_steps > 0 ? f.wv * sp_gain_bytes(norm_steps, f.wv) : 0);
 }
+
+// What a product has beside its operands, all of it optional.
+struct Beside {
+  const short* bias = nullptr;       // [N]
+  const short* residual = nullptr;   // [M, N], added to the result
+  const short* gains = nullptr;      // [K], of the RMS norm of x
+  float eps = 0.f;
+};
 
 // N: columns of out. SILU: w has 2N rows, gate then up; a tile is NI / 2
 // groups of gate rows and the NI / 2 groups of the same columns' up rows.
-template <typename Tag, int NI, int XG, int WV, int D, bool SILU>
+// NORM: the product of x's RMS norm. A row's root comes out of the sum (what
+// meets the weights is x * gain, rounded as the normalized row would be), so a
+// workgroup needs its squares at the end only, and has them, since all of x
+// passes through it. With the residual as epilogue a layer of few rows keeps
+// no launch for its norms: they took 3.5 us each beside products of 7 to 37
+// (four layers of 4096 and the logits, 1 row 526 -> 508 us, 8 rows 534 -> 512).
+template <typename Tag, int NI, int XG, int WV, int D, bool SILU, bool NORM>
 __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     short* __restrict__ out, const short* __restrict__ x,
-    const short* __restrict__ w, const short* __restrict__ bias, const int M,
+    const short* __restrict__ w, const Beside beside, const int M,
     const int N, const int K, const int n_tiles, const int parts,
     f32x4* __restrict__ part_sums, unsigned* __restrict__ arrived) {
-  using P = StreamProduct<Tag, NI, XG, WV, D>;
+  using P = StreamProduct<Tag, NI, XG, WV, D, NORM>;
   constexpr int MT = P::MT;
+  static_assert(!NORM || MT == 1);
   constexpr int NO = SILU ? NI / 2 : NI;
   extern __shared__ __align__(16) char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
@@ -124,10 +144,12 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
   const int steps = K / SP_K;
   P::run(lds, wave, steps * part / parts, steps * (part + 1) / parts,
          blockIdx.x / 8, reinterpret_cast<const char*>(w + (int64_t)n0 * K),
-         wat, reinterpret_cast<const char*>(x), xat);
+         wat, reinterpret_cast<const char*>(x), xat,
+         reinterpret_cast<const char*>(beside.gains));
 
   // Each wave goes on with a share of the tiles.
   constexpr int T = P::T;
+  constexpr int TN = P::TN;
   constexpr int TO = NO * MT;
   constexpr int PER = (TO + WV - 1) / WV;
   constexpr int H = SILU ? 2 : 1;
@@ -139,16 +161,21 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
 #pragma unroll
     for (int h = 0; h < H; ++h) v[u][h] = P::sum(lds, h * TO + t);
   }
+  float squares = 0.f;
+  if constexpr (NORM) squares = P::sum(lds, T)[0];
   if (parts > 1) {
-    f32x4* sums = part_sums + (int64_t)tile * parts * T * WAVE_SIZE + lane;
+    f32x4* sums = part_sums + (int64_t)tile * parts * TN * WAVE_SIZE + lane;
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
       const int t = u * WV + wave;
       if (t >= TO) break;
 #pragma unroll
       for (int h = 0; h < H; ++h)
-        part_put(sums + (part * T + h * TO + t) * WAVE_SIZE, v[u][h]);
+        part_put(sums + (part * TN + h * TO + t) * WAVE_SIZE, v[u][h]);
     }
+    if (NORM && wave == 0)
+      part_put(reinterpret_cast<float*>(sums + (part * TN + T) * WAVE_SIZE),
+               squares);
     if (!last_to_arrive(arrived, tile, parts,
                         reinterpret_cast<unsigned*>(lds)))
       return;
@@ -166,7 +193,7 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
           f32x4 p[Q];
 #pragma unroll
           for (int q = 0; q < Q; ++q)
-            p[q] = part_get(at + min(q, parts - 1) * (T * WAVE_SIZE));
+            p[q] = part_get(at + min(q, parts - 1) * (TN * WAVE_SIZE));
           v[u][h] = p[0];
 #pragma unroll
           for (int q = 1; q < Q; ++q)
@@ -177,7 +204,19 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
         else                add(std::integral_constant<int, SL_PARTS>{});
       }
     }
+    if constexpr (NORM) {
+      float p[SL_PARTS];
+#pragma unroll
+      for (int q = 0; q < SL_PARTS; ++q)
+        p[q] = part_get(reinterpret_cast<const float*>(
+            sums + (min(q, parts - 1) * TN + T) * WAVE_SIZE));
+      squares = p[0];
+#pragma unroll
+      for (int q = 1; q < SL_PARTS; ++q)
+        if (q < parts) squares += p[q];
+    }
   }
+  const float root = NORM ? rsqrtf(squares / K + beside.eps) : 1.f;
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
     const int t = u * WV + wave;
@@ -185,15 +224,26 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     const int row = (t % MT) * 16 + l16;
     const int col = n0 + (t / MT) * 16 + l4 * 4;
     f32x4 o = v[u][0];
+    if constexpr (NORM) {
+#pragma unroll
+      for (int h = 0; h < H; ++h) v[u][h] *= root;
+      o = v[u][0];
+    }
     if constexpr (SILU) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         o[r] = o[r] / (1.f + __expf(-o[r])) * v[u][1][r];
     }
     if (row >= M || col >= N || (XG == 1 && l16 >= 8)) continue;
-    if (!SILU && bias != nullptr) {
+    if (!SILU && beside.bias != nullptr) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] += to_f32<Tag>(bias[col + r]);
+      for (int r = 0; r < 4; ++r) o[r] += to_f32<Tag>(beside.bias[col + r]);
+    }
+    if (!SILU && !NORM && beside.residual != nullptr) {
+      const s16x4 a = *reinterpret_cast<const s16x4*>(
+          beside.residual + (int64_t)row * N + col);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] += to_f32<Tag>(a[r]);
     }
     *reinterpret_cast<int2*>(out + (int64_t)row * N + col) =
         int2{pack2<Tag>(o[0], o[1]), pack2<Tag>(o[2], o[3])};
@@ -210,26 +260,26 @@ struct Plan { int form, parts; };
 // of a fit and not bounds (the first is passed by a tenth): they come closest
 // to the best of all forms over 15 layers of 2112 x 7168 to 128256 x 4096 at 1
 // to 64 rows, 1.3 % from it on average, 7 % at most.
-Plan plan(int xg, int64_t rows_w, int K, bool silu) {
+Plan plan(int xg, int64_t rows_w, int K, bool silu, bool norm = false) {
   Plan best{-1, 1};
   double least = 1e30;
   auto fourth = [](double v) { return v * v * v * v; };
   for (int i = 0; i < SL_NFORMS; ++i) {
     const Form f = SL_FORMS[i];
     // Two waves have too little on the way where four fit.
-    if (lds_bytes(f, xg) > SL_LDS || (f.wv == 2 && xg < 8) ||
-        (silu && f.ni % 2 != 0))
-      continue;
+    if ((f.wv == 2 && xg < 8) || (silu && f.ni % 2 != 0)) continue;
     const int64_t tiles = (rows_w + f.ni * 16 - 1) / (f.ni * 16);
     for (int parts : {1, 2, 3, 4, 6, 8}) {
       if (parts > 1 && (tiles > SL_JOBS || tiles * parts > 1100 ||
                         K / SP_K / parts < f.wv))
         continue;
+      const int lds = lds_bytes(f, xg, norm ? ceil_div(K / SP_K, parts) : 0);
+      if (lds > SL_LDS) continue;
       const double mb = (f.ni * 16 + xg * 8) * 2e-6 * K / parts;
       const double jobs = (double)(tiles * parts);
       const double cus = (double)((tiles * parts + 255) / 256);
       const double load =
-          cus > 1 && lds_bytes(f, xg) * 2 > SL_LDS
+          cus > 1 && lds * 2 > SL_LDS
               ? cus
               : 0.6 * cus + 0.4 * std::max(1.0, jobs / 256);
       double t = std::sqrt(std::sqrt(fourth(rows_w * 2e-6 * K / 6.0) +
@@ -246,46 +296,52 @@ Plan plan(int xg, int64_t rows_w, int K, bool silu) {
   return best;
 }
 
-template <typename Tag, int I, int XG, bool SILU>
+template <typename Tag, int I, int XG, bool SILU, bool NORM>
 void launch_form(torch::Tensor& out, const torch::Tensor& x,
-                 const torch::Tensor& w, const short* bias, int N,
+                 const torch::Tensor& w, const Beside& beside, int N,
                  int parts) {
   constexpr Form f = SL_FORMS[I];
-  if constexpr (lds_bytes(f, XG) <= SL_LDS && (f.wv > 2 || XG == 8) &&
-                (!SILU || f.ni % 2 == 0)) {
+  if constexpr (lds_bytes(f, XG, NORM) <= SL_LDS && (f.wv > 2 || XG == 8) &&
+                (!SILU || f.ni % 2 == 0) && (!NORM || XG <= 2)) {
+    const int lds =
+        lds_bytes(f, XG, NORM ? ceil_div((int)x.size(1) / SP_K, parts) : 0);
     const int M = (int)x.size(0), K = (int)x.size(1);
     const int cols = f.ni * 16 / (SILU ? 2 : 1);
     const int tiles = ceil_div(N, cols);
     torch::Tensor sums, arrived;
     if (parts > 1) {
-      sums = torch::empty({(int64_t)tiles * parts * f.ni * ((XG + 1) / 2) *
-                           WAVE_SIZE * 4},
+      sums = torch::empty({(int64_t)tiles * parts *
+                           (f.ni * ((XG + 1) / 2) + NORM) * WAVE_SIZE * 4},
                           x.options().dtype(torch::kFloat));
       arrived = arrival_counters(x, tiles);
     }
     hipLaunchKernelGGL(
-        (stream_linear_kernel<Tag, f.ni, XG, f.wv, f.d, SILU>),
-        dim3(tiles * parts), dim3(f.wv * WAVE_SIZE), lds_bytes(f, XG),
+        (stream_linear_kernel<Tag, f.ni, XG, f.wv, f.d, SILU, NORM>),
+        dim3(tiles * parts), dim3(f.wv * WAVE_SIZE), lds,
         c10::hip::getCurrentHIPStream().stream(), (short*)out.data_ptr(),
-        (const short*)x.data_ptr(), (const short*)w.data_ptr(), bias, M, N, K,
-        tiles, parts, parts > 1 ? (f32x4*)sums.data_ptr() : nullptr,
+        (const short*)x.data_ptr(), (const short*)w.data_ptr(), beside, M, N,
+        K, tiles, parts, parts > 1 ? (f32x4*)sums.data_ptr() : nullptr,
         parts > 1 ? (unsigned*)arrived.data_ptr() : nullptr);
   } else {
     TORCH_CHECK(false, "stream_linear: form does not fit");
   }
 }
 
-template <typename Tag, bool SILU>
+template <typename Tag, bool SILU, bool NORM = false>
 void launch(torch::Tensor& out, const torch::Tensor& x,
-            const torch::Tensor& w, const short* bias, int N) {
+            const torch::Tensor& w, const Beside& beside, int N) {
   const int xg = row_groups(x.size(0));
-  const Plan p = plan(xg, w.size(0), (int)x.size(1), SILU);
+  const Plan p = plan(xg, w.size(0), (int)x.size(1), SILU, NORM);
   auto by_rows = [&](auto form) {
     constexpr int I = decltype(form)::value;
-    if (xg == 1) launch_form<Tag, I, 1, SILU>(out, x, w, bias, N, p.parts);
-    else if (xg == 2) launch_form<Tag, I, 2, SILU>(out, x, w, bias, N, p.parts);
-    else if (xg == 4) launch_form<Tag, I, 4, SILU>(out, x, w, bias, N, p.parts);
-    else launch_form<Tag, I, 8, SILU>(out, x, w, bias, N, p.parts);
+    auto groups = [&](auto n) {
+      launch_form<Tag, I, decltype(n)::value, SILU, NORM>(out, x, w, beside,
+                                                          N, p.parts);
+    };
+    if (xg == 1) groups(std::integral_constant<int, 1>{});
+    else if (xg == 2) groups(std::integral_constant<int, 2>{});
+    else if (xg == 4) groups(std::integral_constant<int, 4>{});
+    else groups(std::integral_constant<int, 8>{});
   };
   static_assert(SL_NFORMS == 7);
   switch (p.form) {
@@ -361,16 +417,111 @@ std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
   return {2, tile.cols, tile.parts};
 }
 
-// x, w and bias as stream_linear_takes and lt_linear have checked them.
-torch::Tensor stream_linear(const torch::Tensor& x, const torch::Tensor& w,
-                            const c10::optional<torch::Tensor>& bias) {
+// x, w and what is beside them as stream_linear_takes and the callers have
+// checked them.
+static torch::Tensor stream_linear_beside(const torch::Tensor& x,
+                                          const torch::Tensor& w,
+                                          const Beside& beside) {
   const int64_t N = w.size(0);
   auto out = torch::empty({x.size(0), N}, x.options());
-  const short* b = bias.has_value() ? (const short*)bias->data_ptr() : nullptr;
   if (x.scalar_type() == torch::kBFloat16)
-    launch<BF16Tag, false>(out, x, w, b, (int)N);
+    launch<BF16Tag, false>(out, x, w, beside, (int)N);
   else
-    launch<FP16Tag, false>(out, x, w, b, (int)N);
+    launch<FP16Tag, false>(out, x, w, beside, (int)N);
+  HIP_CHECK_KERNEL();
+  return out;
+}
+
+torch::Tensor stream_linear(const torch::Tensor& x, const torch::Tensor& w,
+                            const c10::optional<torch::Tensor>& bias) {
+  Beside beside;
+  if (bias.has_value()) beside.bias = (const short*)bias->data_ptr();
+  return stream_linear_beside(x, w, beside);
+}
+
+static bool bias_fits(const c10::optional<torch::Tensor>& bias,
+                      const torch::Tensor& w) {
+  return !bias.has_value() ||
+         (bias->scalar_type() == w.scalar_type() && bias->is_contiguous() &&
+          bias->numel() == w.size(0));
+}
+
+// a @ w^T + bias + residual; in one launch, rounded once, where this file
+// takes the product.
+torch::Tensor linear_add(torch::Tensor a, torch::Tensor w,
+                         c10::optional<torch::Tensor> bias,
+                         torch::Tensor residual) {
+  TORCH_CHECK(a.dim() == 2 && w.dim() == 2 && a.size(1) == w.size(1) &&
+                  a.scalar_type() == w.scalar_type() &&
+                  residual.dim() == 2 && residual.size(0) == a.size(0) &&
+                  residual.size(1) == w.size(0) &&
+                  residual.scalar_type() == a.scalar_type() &&
+                  residual.device() == a.device(),
+              "linear_add: [M, K] x [N, K] + [M, N]");
+  auto x = a.contiguous();
+  if (x.size(0) == 0 || !residual.is_contiguous() ||
+      (uintptr_t)residual.data_ptr() % 8 != 0 || !bias_fits(bias, w) ||
+      tile_linear_first(x.size(0), w.size(0), x.size(1), false) ||
+      !stream_linear_takes(x, w, w.size(0)))
+    return lt_linear(x, w, bias) + residual;
+  Beside beside;
+  if (bias.has_value()) beside.bias = (const short*)bias->data_ptr();
+  beside.residual = (const short*)residual.data_ptr();
+  return stream_linear_beside(x, w, beside);
+}
+
+// Whether the norm of `rows` rows goes with the product (bf16 only: fp16 rows
+// times gains may pass 65504 where normalized ones do not). Up to 16 rows: a
+// step's rows are multiplied by its gains in every workgroup, and from 17 on
+// the gains no longer fit beside the widest form's weights.
+static bool norm_sizes(int64_t rows, int64_t weight_rows, int64_t k,
+                       bool silu) {
+  return rows <= SL_NORM_ROWS &&
+         stream_sizes(rows, weight_rows, silu ? weight_rows / 2 : weight_rows,
+                      k) &&
+         plan(row_groups(rows), weight_rows, (int)k, silu, true).form >= 0;
+}
+
+// Whether a decoder layer's products of `rows` rows go without launches for
+// its norms: `qkv` and `gate_up` weight rows on the norms of `hidden` columns,
+// and products back to `hidden` columns from `heads` and `inner` ones.
+bool layer_streams(int64_t rows, int64_t hidden, int64_t qkv, int64_t heads,
+                   int64_t gate_up, int64_t inner) {
+  return norm_sizes(rows, qkv, hidden, false) &&
+         norm_sizes(rows, gate_up, hidden, true) && gate_up == 2 * inner &&
+         stream_sizes(rows, hidden, hidden, heads) &&
+         stream_sizes(rows, hidden, hidden, inner);
+}
+
+// linear (or, silu, linear_silu_and_mul) of rms_norm(a, gains, eps); in one
+// launch where norm_sizes says so.
+torch::Tensor norm_linear(torch::Tensor a, torch::Tensor gains, double eps,
+                          torch::Tensor w, c10::optional<torch::Tensor> bias,
+                          bool silu) {
+  TORCH_CHECK(a.dim() == 2 && w.dim() == 2 && a.size(1) == w.size(1) &&
+                  a.scalar_type() == w.scalar_type() && gains.dim() == 1 &&
+                  gains.size(0) == a.size(1) &&
+                  gains.scalar_type() == a.scalar_type() &&
+                  gains.device() == a.device(),
+              "norm_linear: [M, K] x [N, K], gains [K]");
+  TORCH_CHECK(!silu || (w.size(0) % 2 == 0 && !bias.has_value()),
+              "norm_linear: the activation takes [gate; up] without a bias");
+  auto x = a.contiguous();
+  const int64_t N = silu ? w.size(0) / 2 : w.size(0);
+  if (x.scalar_type() != torch::kBFloat16 || x.size(0) == 0 ||
+      !gains.is_contiguous() || (uintptr_t)gains.data_ptr() % 16 != 0 ||
+      !bias_fits(bias, w) || !stream_linear_takes(x, w, N) ||
+      !norm_sizes(x.size(0), w.size(0), x.size(1), silu)) {
+    auto y = rms_norm(x, gains, eps);
+    return silu ? linear_silu_and_mul(y, w) : lt_linear(y, w, bias);
+  }
+  Beside beside;
+  if (bias.has_value()) beside.bias = (const short*)bias->data_ptr();
+  beside.gains = (const short*)gains.data_ptr();
+  beside.eps = (float)eps;
+  auto out = torch::empty({x.size(0), N}, x.options());
+  if (silu) launch<BF16Tag, true, true>(out, x, w, beside, (int)N);
+  else      launch<BF16Tag, false, true>(out, x, w, beside, (int)N);
   HIP_CHECK_KERNEL();
   return out;
 }
@@ -393,9 +544,9 @@ torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w) {
     return silu_and_mul(lt_linear(x, w, c10::nullopt)).reshape(sizes);
   }
   if (x.scalar_type() == torch::kBFloat16)
-    launch<BF16Tag, true>(out, x, w, nullptr, (int)N);
+    launch<BF16Tag, true>(out, x, w, Beside{}, (int)N);
   else
-    launch<FP16Tag, true>(out, x, w, nullptr, (int)N);
+    launch<FP16Tag, true>(out, x, w, Beside{}, (int)N);
   HIP_CHECK_KERNEL();
   return out.reshape(sizes);
 }

@@ -11,4 +11,7 @@ def hooked(*modules) -> bool:
     or those registered for all modules."""
     if _module._global_forward_hooks or _module._global_forward_pre_hooks:
         return True
-    return any(m._forward_hooks or m._forward_pre_hooks for m in modules)
+    for m in modules:
+        if m._forward_hooks or m._forward_pre_hooks:
+            return True
+    return False

@@ -82,6 +82,23 @@ def gated_silu(proj, act, x):
     return act(proj(x))
 
 
+def plain(*projs) -> bool:
+    """Whether the projections are products with bf16 weights on one rank and
+    nothing else that would have to be called. (Asked for every layer of
+    small steps: what is absent is looked up where it would be, since a
+    module's own way to say so takes a microsecond.)"""
+    for p in projs:
+        weight = p._parameters["weight"]
+        if ("weight_fp8" in p._buffers
+                or p.__dict__.get("lora_slices") is not None
+                or weight.dtype != torch.bfloat16
+                or type(p) not in (QKVParallelLinear, RowParallelLinear,
+                                   MergedColumnParallelLinear)
+                or p.__dict__.get("gather_output")):
+            return False
+    return get_tp_world_size() == 1 and not hooked(*projs)
+
+
 class ReplicatedLinear(nn.Module):
     def __init__(self, input_size, output_size, bias=False, dtype=None):
         super().__init__()

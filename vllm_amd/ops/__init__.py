@@ -127,6 +127,27 @@ def linear_silu_and_mul(x, weight):
     return get_backend(x.device).linear_silu_and_mul(x, weight)
 
 
+def norm_linear(x, gain, eps, weight, bias=None, silu=False):
+    """linear (silu: linear_silu_and_mul) of rms_norm(x, gain, eps)."""
+    return get_backend(x.device).norm_linear(x, gain, eps, weight, bias,
+                                             silu)
+
+
+def linear_add(x, weight, bias, residual):
+    """linear(x, weight, bias) + residual."""
+    return get_backend(x.device).linear_add(x, weight, bias, residual)
+
+
+def layer_streams(x, qkv, heads, gate_up, inner):
+    """Whether a decoder layer on x [rows, hidden] is faster by norm_linear
+    and linear_add than with norms of its own: qkv and gate_up rows of weights
+    behind the norms, and heads and inner columns before the products back to
+    the hidden size."""
+    return (x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous()
+            and get_backend(x.device).layer_streams(
+                x.shape[0], x.shape[1], qkv, heads, gate_up, inner))
+
+
 def linear_fp8(x, w_fp8, w_scale, bias=None):
     """W8A8 fp8 linear: dynamic per-token activation scales, per-channel
     weight scales. fp8 MFMA GEMM on GPU; bit-matching fp32 simulation on

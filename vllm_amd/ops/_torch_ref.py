@@ -181,6 +181,17 @@ def quantize_weight_fp8(w):
     return q, scales
 
 
+def norm_linear(x, gain, eps, weight, bias=None, silu=False):
+    y = rms_norm(x, gain, eps)
+    if silu:
+        return linear_silu_and_mul(y, weight)
+    return linear(y, weight, bias)
+
+
+def linear_add(x, weight, bias, residual):
+    return linear(x, weight, bias) + residual
+
+
 def linear_fp8(x, w_fp8, w_scale, bias=None):
     """W8A8 fp8 linear, CPU reference: quantize activations per-token
     exactly as the GPU path does, then compute in fp32 on dequantized

@@ -111,6 +111,21 @@ def linear_silu_and_mul(x, weight):
     return _C.linear_silu_and_mul(x, weight)
 
 
+def norm_linear(x, gain, eps, weight, bias=None, silu=False):
+    return _C.norm_linear(x, gain, eps, weight, bias, silu)
+
+
+def linear_add(x, weight, bias, residual):
+    return _C.linear_add(x, weight, bias, residual)
+
+
+@functools.lru_cache(maxsize=None)
+def layer_streams(rows, hidden, qkv, heads, gate_up, inner):
+    # Up to 16 rows, for layers whose products all stream their weights
+    # (csrc/stream_linear.hip).
+    return _C.layer_streams(rows, hidden, qkv, heads, gate_up, inner)
+
+
 def quant_fp8_dynamic(x):
     # Per-token dynamic quant (csrc/quant_fp8.hip): one workgroup/row.
     M, K = x.shape
