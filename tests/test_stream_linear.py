@@ -164,6 +164,57 @@ def test_norm_linear(m, n, k):
               torch.nn.functional.silu(gate) * up)
 
 
+# Heads whose halves hold one to four groups of 16 columns (the widest form has
+# four), whole and with K split; both cache types; rows that are padding.
+@gpu
+@pytest.mark.parametrize("m,hq,hkv,d,k,kv", [
+    (1, 32, 8, 128, 4096, torch.bfloat16),
+    (16, 28, 4, 128, 3584, torch.bfloat16),
+    (8, 32, 8, 128, 4096, torch.float8_e4m3fn),
+    (9, 2, 1, 64, 4096, torch.bfloat16), (7, 4, 4, 32, 128, torch.bfloat16),
+    (3, 160, 8, 128, 8192, torch.float8_e4m3fn),
+    (2, 16, 8, 256, 3072, torch.bfloat16),
+    (5, 2, 2, 96, 512, torch.bfloat16),
+    (17, 8, 2, 128, 512, torch.bfloat16)])   # as steps of their own
+def test_norm_qkv_rope_cache(m, hq, hkv, d, k, kv):
+    """Against the steps that it stands for, on the same rounded sums."""
+    from vllm_amd.ops import hip_ops
+    rows = (hq + 2 * hkv) * d
+    x, w = _operands(m, rows, k, torch.bfloat16)
+    torch.manual_seed(m * k + rows)
+    gain = 1 + 0.1 * torch.randn(k, device="cuda").bfloat16()
+    turn = torch.randn(300, d, device="cuda")
+    positions = torch.randint(0, 300, (m,), device="cuda")
+    slots = torch.randperm(5 * 16, device="cuda")[:m]
+    slots[m // 2] = -1 if m > 2 else slots[m // 2]
+    for bias in (None, torch.randn(rows, device="cuda").bfloat16()):
+        caches = [torch.zeros(2, 5, hkv, 16, d, device="cuda").to(kv)
+                  for _ in range(2)]
+        q = hip_ops.norm_qkv_rope_cache(x, gain, 1e-6, w, bias, positions,
+                                        turn, caches[0], slots)
+        qkv = hip_ops.norm_linear(x, gain, 1e-6, w, bias).view(m, -1, d)
+        q2, k2, v2 = qkv.split([hq, hkv, hkv], dim=1)
+        hip_ops.rope_and_cache(positions, q2, k2, v2, turn, d, True,
+                               caches[1], slots)
+        # Forms may differ in the order of their sums: an ulp or two of what
+        # is rounded, turned (by up to five here) and rounded again.
+        a, b = (c.view(torch.uint8) if kv != torch.bfloat16 else c
+                for c in caches)
+        top = q2.float().abs().max()
+        assert (q.float() - q2.float()).abs().max() <= top * 2.0 ** -7
+        assert q.shape == q2.shape
+        if kv == torch.bfloat16:
+            assert (a.float() - b.float()).abs().max() <= top * 2.0 ** -7
+        else:   # neighbours among 8-bit values, where they are not the same
+            assert ((a != b).float().mean() < 0.02
+                    and (a.int() - b.int()).abs().max() <= 1)
+        assert (caches[0].float() != 0).any()
+        used = torch.zeros(80, dtype=torch.bool, device="cuda")
+        used[slots[slots >= 0]] = True
+        kept = caches[0].float().transpose(2, 3).reshape(2, 80, -1)
+        assert (kept[:, ~used] == 0).all()
+
+
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [(1, 24, 64), (8, 4096, 4096),

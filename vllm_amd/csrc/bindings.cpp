@@ -52,6 +52,10 @@ torch::Tensor linear_add(torch::Tensor a, torch::Tensor w,
 torch::Tensor norm_linear(torch::Tensor a, torch::Tensor gains, double eps,
                           torch::Tensor w, c10::optional<torch::Tensor> bias,
                           bool silu);
+torch::Tensor norm_qkv_rope_cache(
+    torch::Tensor a, torch::Tensor gains, double eps, torch::Tensor w,
+    c10::optional<torch::Tensor> bias, torch::Tensor positions,
+    torch::Tensor slots, torch::Tensor cos_sin, torch::Tensor kv_cache);
 bool layer_streams(int64_t rows, int64_t hidden, int64_t qkv, int64_t heads,
                    int64_t gate_up, int64_t inner);
 std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
@@ -239,6 +243,9 @@ TORCH_LIBRARY(vllm_amd, m) {
         "-> Tensor");
   m.def("norm_linear(Tensor a, Tensor gains, float eps, Tensor w, "
         "Tensor? bias, bool silu) -> Tensor");
+  m.def("norm_qkv_rope_cache(Tensor a, Tensor gains, float eps, Tensor w, "
+        "Tensor? bias, Tensor positions, Tensor slots, Tensor cos_sin, "
+        "Tensor(a!) kv_cache) -> Tensor");
   m.def("layer_streams(int rows, int hidden, int qkv, int heads, "
         "int gate_up, int inner) -> bool",
         &vllm_amd::layer_streams);
@@ -379,6 +386,7 @@ TORCH_LIBRARY_IMPL(vllm_amd, CUDA, m) {
   m.impl("linear_silu_and_mul", &vllm_amd::linear_silu_and_mul);
   m.impl("linear_add", &vllm_amd::linear_add);
   m.impl("norm_linear", &vllm_amd::norm_linear);
+  m.impl("norm_qkv_rope_cache", &vllm_amd::norm_qkv_rope_cache);
   m.impl("lt_linear_fp8", &vllm_amd::lt_linear_fp8);
   m.impl("dynamic_quant_fp8", &vllm_amd::dynamic_quant_fp8);
   m.impl("scale_rows_cols", &vllm_amd::scale_rows_cols);

@@ -55,6 +55,9 @@ torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
 torch::Tensor silu_and_mul(torch::Tensor x);
 torch::Tensor rms_norm(torch::Tensor x, torch::Tensor weight, double eps);
 torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w);
+void rope_and_cache(torch::Tensor positions, torch::Tensor q, torch::Tensor k,
+                    torch::Tensor v, torch::Tensor cos_sin_cache, int64_t rot,
+                    torch::Tensor kv_cache, torch::Tensor slot_mapping);
 // tile_linear.hip
 bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
                  const torch::Tensor& w, bool silu);
@@ -101,24 +104,46 @@ struct Beside {
   float eps = 0.f;
 };
 
-// N: columns of out. SILU: w has 2N rows, gate then up; a tile is NI / 2
-// groups of gate rows and the NI / 2 groups of the same columns' up rows.
+// What becomes of two halves of weight rows: nothing (one row a column),
+// silu(gate) * up, or the rotation of a head's halves.
+enum { SINGLE = 0, SILU = 1, ROPE = 2 };
+
+// Weights of query, key and value heads. out gets the rotated queries [M,
+// q_heads, 2 * half], the cache [2, blocks, kv_heads, block_size, 2 * half] the
+// rotated keys and the values.
+struct Heads {
+  const int64_t* positions = nullptr;   // [M]
+  const int64_t* slots = nullptr;       // [M]
+  const float* cos_sin = nullptr;       // [positions, cos half | sin half]
+  void* kv_cache = nullptr;
+  int64_t plane = 0;                    // elements from keys to values
+  int half = 0, q_heads = 0, kv_heads = 0, block_size = 0;
+  bool fp8 = false;
+};
+
+// N: columns of out. PAIR SILU: w has 2N rows, gate then up; a tile is NI / 2
+// groups of gate rows and the NI / 2 groups of the same columns' up rows. ROPE:
+// N counts pairs of a head's columns that turn together, and a tile is NI / 2
+// groups of first and of second ones of one head. (The launch for rotation and
+// cache took 2.9 us of a layer: the same, 1 row 508 -> 498 us, 8 rows 512 ->
+// 502. What it read is asked for behind the first fills here, as the residual
+// is, or it would be waited for at the end.)
 // NORM: the product of x's RMS norm. A row's root comes out of the sum (what
 // meets the weights is x * gain, rounded as the normalized row would be), so a
 // workgroup needs its squares at the end only, and has them, since all of x
 // passes through it. With the residual as epilogue a layer of few rows keeps
 // no launch for its norms: they took 3.5 us each beside products of 7 to 37
 // (four layers of 4096 and the logits, 1 row 526 -> 508 us, 8 rows 534 -> 512).
-template <typename Tag, int NI, int XG, int WV, int D, bool SILU, bool NORM>
+template <typename Tag, int NI, int XG, int WV, int D, int PAIR, bool NORM>
 __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     short* __restrict__ out, const short* __restrict__ x,
-    const short* __restrict__ w, const Beside beside, const int M,
-    const int N, const int K, const int n_tiles, const int parts,
+    const short* __restrict__ w, const Beside beside, const Heads heads,
+    const int M, const int N, const int K, const int n_tiles, const int parts,
     f32x4* __restrict__ part_sums, unsigned* __restrict__ arrived) {
   using P = StreamProduct<Tag, NI, XG, WV, D, NORM>;
   constexpr int MT = P::MT;
   static_assert(!NORM || MT == 1);
-  constexpr int NO = SILU ? NI / 2 : NI;
+  constexpr int NO = PAIR ? NI / 2 : NI;
   extern __shared__ __align__(16) char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
@@ -127,32 +152,73 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
   const int tile = blockIdx.x % n_tiles;
   const int part = blockIdx.x / n_tiles;
   const int n0 = tile * NO * 16;
+  // Weight row of column n0, and how far the other half's lies.
+  const int head = PAIR == ROPE ? n0 / heads.half : 0;
+  const int w0 = n0 + head * heads.half;
+  const int apart = PAIR == ROPE ? heads.half : N;
 
   // Rows past the end repeat the last.
   uint32_t wat[2 * NI], xat[XG];
 #pragma unroll
   for (int i = 0; i < 2 * NI; ++i) {
     const int r = i * 8 + (lane >> 3);
-    const int half = SILU && i >= NI ? 1 : 0;
-    wat[i] = sp_place(min(r - half * NO * 16, N - 1 - n0) + half * N, r, K);
+    const int half = PAIR && i >= NI ? 1 : 0;
+    wat[i] =
+        sp_place(min(r - half * NO * 16, N - 1 - n0) + half * apart, r, K);
   }
 #pragma unroll
   for (int i = 0; i < XG; ++i) {
     const int r = i * 8 + (lane >> 3);
     xat[i] = sp_place(min(r, M - 1), r, K);
   }
-  const int steps = K / SP_K;
-  P::run(lds, wave, steps * part / parts, steps * (part + 1) / parts,
-         blockIdx.x / 8, reinterpret_cast<const char*>(w + (int64_t)n0 * K),
-         wat, reinterpret_cast<const char*>(x), xat,
-         reinterpret_cast<const char*>(beside.gains));
-
-  // Each wave goes on with a share of the tiles.
+  // Afterwards each wave goes on with a share of the tiles.
   constexpr int T = P::T;
   constexpr int TN = P::TN;
   constexpr int TO = NO * MT;
   constexpr int PER = (TO + WV - 1) / WV;
-  constexpr int H = SILU ? 2 : 1;
+  constexpr int H = PAIR ? 2 : 1;
+  s16x4 residual[PER];
+  f32x4 cos[PER], sin[PER];
+  int64_t slot = -1;
+  auto early = [&] {
+    if constexpr (PAIR == SINGLE && !NORM) {
+      if (beside.residual == nullptr) return;
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const int t = min(u * WV + wave, TO - 1);
+        const int row = min((t % MT) * 16 + l16, M - 1);
+        const int col = min(n0 + (t / MT) * 16 + l4 * 4, N - 4);
+        residual[u] = *reinterpret_cast<const s16x4*>(
+            beside.residual + (int64_t)row * N + col);
+      }
+    }
+    if constexpr (PAIR == ROPE) {
+      // By way of the scalar cache: a wait for a load would be one for the
+      // fills before it.
+      int pos = 0;
+#pragma unroll
+      for (int r = 0; r < XG * 8; ++r) {
+        const int p = load_uniform(
+            reinterpret_cast<const int*>(heads.positions + min(r, M - 1)));
+        if (l16 == r) pos = p;
+      }
+      slot = heads.slots[min(l16, M - 1)];
+      const float* turn = heads.cos_sin + (int64_t)pos * (2 * heads.half);
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const int t = min(u * WV + wave, TO - 1);
+        const int p = n0 - head * heads.half + (t / MT) * 16 + l4 * 4;
+        cos[u] = *reinterpret_cast<const f32x4*>(turn + p);
+        sin[u] = *reinterpret_cast<const f32x4*>(turn + heads.half + p);
+      }
+    }
+  };
+  const int steps = K / SP_K;
+  P::run(lds, wave, steps * part / parts, steps * (part + 1) / parts,
+         blockIdx.x / 8, reinterpret_cast<const char*>(w + (int64_t)w0 * K),
+         wat, reinterpret_cast<const char*>(x), xat,
+         reinterpret_cast<const char*>(beside.gains), early);
+
   f32x4 v[PER][H];
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
@@ -229,21 +295,78 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
       for (int h = 0; h < H; ++h) v[u][h] *= root;
       o = v[u][0];
     }
-    if constexpr (SILU) {
+    if constexpr (PAIR == SILU) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         o[r] = o[r] / (1.f + __expf(-o[r])) * v[u][1][r];
     }
     if (row >= M || col >= N || (XG == 1 && l16 >= 8)) continue;
-    if (!SILU && beside.bias != nullptr) {
+    if constexpr (PAIR == ROPE) {
+      const int half = heads.half, p = col - head * half;
+      int2 to[2];
+      float y[2][4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        f32x4 z = v[u][h];
+        if (beside.bias != nullptr) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            z[r] += to_f32<Tag>(beside.bias[(2 * head + h) * half + p + r]);
+        }
+        // Rounded as a product of its own would leave them.
+        to[h] = int2{pack2<Tag>(z[0], z[1]), pack2<Tag>(z[2], z[3])};
+        y[h][0] = unpack_lo<Tag>(to[h].x);
+        y[h][1] = unpack_hi<Tag>(to[h].x);
+        y[h][2] = unpack_lo<Tag>(to[h].y);
+        y[h][3] = unpack_hi<Tag>(to[h].y);
+      }
+      if (head < heads.q_heads + heads.kv_heads) {
+        float a[4], b[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          a[r] = __builtin_fmaf(y[0][r], cos[u][r], -(y[1][r] * sin[u][r]));
+          b[r] = __builtin_fmaf(y[0][r], sin[u][r], y[1][r] * cos[u][r]);
+        }
+        to[0] = int2{pack2<Tag>(a[0], a[1]), pack2<Tag>(a[2], a[3])};
+        to[1] = int2{pack2<Tag>(b[0], b[1]), pack2<Tag>(b[2], b[3])};
+      }
+      if (head < heads.q_heads) {
+        short* q = out + ((int64_t)row * heads.q_heads + head) * (2 * half) + p;
+        *reinterpret_cast<int2*>(q) = to[0];
+        *reinterpret_cast<int2*>(q + half) = to[1];
+        continue;
+      }
+      if (slot < 0) continue;   // padding
+      const bool value = head >= heads.q_heads + heads.kv_heads;
+      const int kvh = head - heads.q_heads - (value ? heads.kv_heads : 0);
+      const int64_t at = (value ? heads.plane : 0) + p +
+                         ((slot / heads.block_size * heads.kv_heads + kvh) *
+                              heads.block_size + slot % heads.block_size) *
+                             (2 * half);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (heads.fp8) {
+          const uint32_t x0 = f32_to_fp8_e4m3(unpack_lo<Tag>(to[h].x));
+          const uint32_t x1 = f32_to_fp8_e4m3(unpack_hi<Tag>(to[h].x));
+          const uint32_t x2 = f32_to_fp8_e4m3(unpack_lo<Tag>(to[h].y));
+          const uint32_t x3 = f32_to_fp8_e4m3(unpack_hi<Tag>(to[h].y));
+          *reinterpret_cast<uint32_t*>((uint8_t*)heads.kv_cache + at +
+                                       h * half) =
+              x0 | x1 << 8 | x2 << 16 | x3 << 24;
+        } else {
+          *reinterpret_cast<int2*>((short*)heads.kv_cache + at + h * half) =
+              to[h];
+        }
+      }
+      continue;
+    }
+    if (PAIR == SINGLE && beside.bias != nullptr) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] += to_f32<Tag>(beside.bias[col + r]);
     }
-    if (!SILU && !NORM && beside.residual != nullptr) {
-      const s16x4 a = *reinterpret_cast<const s16x4*>(
-          beside.residual + (int64_t)row * N + col);
+    if (PAIR == SINGLE && !NORM && beside.residual != nullptr) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] += to_f32<Tag>(a[r]);
+      for (int r = 0; r < 4; ++r) o[r] += to_f32<Tag>(residual[u][r]);
     }
     *reinterpret_cast<int2*>(out + (int64_t)row * N + col) =
         int2{pack2<Tag>(o[0], o[1]), pack2<Tag>(o[2], o[3])};
@@ -260,14 +383,18 @@ struct Plan { int form, parts; };
 // of a fit and not bounds (the first is passed by a tenth): they come closest
 // to the best of all forms over 15 layers of 2112 x 7168 to 128256 x 4096 at 1
 // to 64 rows, 1.3 % from it on average, 7 % at most.
-Plan plan(int xg, int64_t rows_w, int K, bool silu, bool norm = false) {
+// half: 0, or columns of half a head, which tiles must not pass.
+Plan plan(int xg, int64_t rows_w, int K, bool silu, bool norm = false,
+          int half = 0) {
   Plan best{-1, 1};
   double least = 1e30;
   auto fourth = [](double v) { return v * v * v * v; };
   for (int i = 0; i < SL_NFORMS; ++i) {
     const Form f = SL_FORMS[i];
     // Two waves have too little on the way where four fit.
-    if ((f.wv == 2 && xg < 8) || (silu && f.ni % 2 != 0)) continue;
+    if ((f.wv == 2 && xg < 8) || ((silu || half > 0) && f.ni % 2 != 0) ||
+        (half > 0 && half % (f.ni * 8) != 0))
+      continue;
     const int64_t tiles = (rows_w + f.ni * 16 - 1) / (f.ni * 16);
     for (int parts : {1, 2, 3, 4, 6, 8}) {
       if (parts > 1 && (tiles > SL_JOBS || tiles * parts > 1100 ||
@@ -296,17 +423,17 @@ Plan plan(int xg, int64_t rows_w, int K, bool silu, bool norm = false) {
   return best;
 }
 
-template <typename Tag, int I, int XG, bool SILU, bool NORM>
+template <typename Tag, int I, int XG, int PAIR, bool NORM>
 void launch_form(torch::Tensor& out, const torch::Tensor& x,
-                 const torch::Tensor& w, const Beside& beside, int N,
-                 int parts) {
+                 const torch::Tensor& w, const Beside& beside,
+                 const Heads& heads, int N, int parts) {
   constexpr Form f = SL_FORMS[I];
   if constexpr (lds_bytes(f, XG, NORM) <= SL_LDS && (f.wv > 2 || XG == 8) &&
-                (!SILU || f.ni % 2 == 0) && (!NORM || XG <= 2)) {
+                (!PAIR || f.ni % 2 == 0) && (!NORM || XG <= 2)) {
     const int lds =
         lds_bytes(f, XG, NORM ? ceil_div((int)x.size(1) / SP_K, parts) : 0);
     const int M = (int)x.size(0), K = (int)x.size(1);
-    const int cols = f.ni * 16 / (SILU ? 2 : 1);
+    const int cols = f.ni * 16 / (PAIR ? 2 : 1);
     const int tiles = ceil_div(N, cols);
     torch::Tensor sums, arrived;
     if (parts > 1) {
@@ -316,27 +443,29 @@ void launch_form(torch::Tensor& out, const torch::Tensor& x,
       arrived = arrival_counters(x, tiles);
     }
     hipLaunchKernelGGL(
-        (stream_linear_kernel<Tag, f.ni, XG, f.wv, f.d, SILU, NORM>),
+        (stream_linear_kernel<Tag, f.ni, XG, f.wv, f.d, PAIR, NORM>),
         dim3(tiles * parts), dim3(f.wv * WAVE_SIZE), lds,
         c10::hip::getCurrentHIPStream().stream(), (short*)out.data_ptr(),
-        (const short*)x.data_ptr(), (const short*)w.data_ptr(), beside, M, N,
-        K, tiles, parts, parts > 1 ? (f32x4*)sums.data_ptr() : nullptr,
+        (const short*)x.data_ptr(), (const short*)w.data_ptr(), beside, heads,
+        M, N, K, tiles, parts, parts > 1 ? (f32x4*)sums.data_ptr() : nullptr,
         parts > 1 ? (unsigned*)arrived.data_ptr() : nullptr);
   } else {
     TORCH_CHECK(false, "stream_linear: form does not fit");
   }
 }
 
-template <typename Tag, bool SILU, bool NORM = false>
+template <typename Tag, int PAIR, bool NORM = false>
 void launch(torch::Tensor& out, const torch::Tensor& x,
-            const torch::Tensor& w, const Beside& beside, int N) {
+            const torch::Tensor& w, const Beside& beside, int N,
+            const Heads& heads = Heads{}) {
   const int xg = row_groups(x.size(0));
-  const Plan p = plan(xg, w.size(0), (int)x.size(1), SILU, NORM);
+  const Plan p = plan(xg, w.size(0), (int)x.size(1), PAIR == SILU, NORM,
+                      heads.half);
   auto by_rows = [&](auto form) {
     constexpr int I = decltype(form)::value;
     auto groups = [&](auto n) {
-      launch_form<Tag, I, decltype(n)::value, SILU, NORM>(out, x, w, beside,
-                                                          N, p.parts);
+      launch_form<Tag, I, decltype(n)::value, PAIR, NORM>(
+          out, x, w, beside, heads, N, p.parts);
     };
     if (xg == 1) groups(std::integral_constant<int, 1>{});
     else if (xg == 2) groups(std::integral_constant<int, 2>{});
@@ -425,9 +554,9 @@ static torch::Tensor stream_linear_beside(const torch::Tensor& x,
   const int64_t N = w.size(0);
   auto out = torch::empty({x.size(0), N}, x.options());
   if (x.scalar_type() == torch::kBFloat16)
-    launch<BF16Tag, false>(out, x, w, beside, (int)N);
+    launch<BF16Tag, SINGLE>(out, x, w, beside, (int)N);
   else
-    launch<FP16Tag, false>(out, x, w, beside, (int)N);
+    launch<FP16Tag, SINGLE>(out, x, w, beside, (int)N);
   HIP_CHECK_KERNEL();
   return out;
 }
@@ -475,11 +604,11 @@ torch::Tensor linear_add(torch::Tensor a, torch::Tensor w,
 // step's rows are multiplied by its gains in every workgroup, and from 17 on
 // the gains no longer fit beside the widest form's weights.
 static bool norm_sizes(int64_t rows, int64_t weight_rows, int64_t k,
-                       bool silu) {
+                       bool silu, int half = 0) {
   return rows <= SL_NORM_ROWS &&
          stream_sizes(rows, weight_rows, silu ? weight_rows / 2 : weight_rows,
                       k) &&
-         plan(row_groups(rows), weight_rows, (int)k, silu, true).form >= 0;
+         plan(row_groups(rows), weight_rows, (int)k, silu, true, half).form >= 0;
 }
 
 // Whether a decoder layer's products of `rows` rows go without launches for
@@ -520,8 +649,76 @@ torch::Tensor norm_linear(torch::Tensor a, torch::Tensor gains, double eps,
   beside.gains = (const short*)gains.data_ptr();
   beside.eps = (float)eps;
   auto out = torch::empty({x.size(0), N}, x.options());
-  if (silu) launch<BF16Tag, true, true>(out, x, w, beside, (int)N);
-  else      launch<BF16Tag, false, true>(out, x, w, beside, (int)N);
+  if (silu) launch<BF16Tag, SILU, true>(out, x, w, beside, (int)N);
+  else      launch<BF16Tag, SINGLE, true>(out, x, w, beside, (int)N);
+  HIP_CHECK_KERNEL();
+  return out;
+}
+
+// Queries of rms_norm(a, gains, eps) @ w^T (+ bias), w = [q heads; k heads; v
+// heads], rotated over all of a head, with the rotated keys and the values in
+// the cache; in one launch where norm_sizes says so of tiles within a head's
+// halves, else as the steps it stands for. [M, q_heads, D], whose rows may lie
+// apart.
+torch::Tensor norm_qkv_rope_cache(
+    torch::Tensor a, torch::Tensor gains, double eps, torch::Tensor w,
+    c10::optional<torch::Tensor> bias, torch::Tensor positions,
+    torch::Tensor slots, torch::Tensor cos_sin, torch::Tensor kv_cache) {
+  TORCH_CHECK(a.dim() == 2 && w.dim() == 2 && a.size(1) == w.size(1) &&
+                  kv_cache.dim() == 5 && kv_cache.size(0) == 2 &&
+                  kv_cache.is_contiguous(),
+              "norm_qkv_rope_cache: [M, K] x [rows, K], cache [2, blocks, "
+              "heads, block, D]");
+  const int64_t M = a.size(0), D = kv_cache.size(4), Hkv = kv_cache.size(2);
+  const int64_t Hq = w.size(0) / D - 2 * Hkv;
+  TORCH_CHECK(Hq > 0 && w.size(0) == (Hq + 2 * Hkv) * D,
+              "norm_qkv_rope_cache: rows of w are heads");
+  TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32 &&
+                  cos_sin.is_contiguous() && cos_sin.dim() == 2 &&
+                  cos_sin.size(1) == D &&
+                  positions.scalar_type() == torch::kInt64 &&
+                  slots.scalar_type() == torch::kInt64 &&
+                  positions.is_contiguous() && slots.is_contiguous() &&
+                  positions.numel() >= M && slots.numel() >= M,
+              "norm_qkv_rope_cache: fp32 table [positions, D], int64 "
+              "positions and slots");
+  TORCH_CHECK(kv_cache.scalar_type() == a.scalar_type() ||
+                  kv_cache.scalar_type() == torch::kFloat8_e4m3fn,
+              "norm_qkv_rope_cache: cache of the rows' type or e4m3");
+  auto x = a.contiguous();
+  const int half = (int)D / 2;
+  if (x.scalar_type() != torch::kBFloat16 ||
+      gains.scalar_type() != torch::kBFloat16 || gains.numel() != x.size(1) ||
+      !gains.is_contiguous() || (uintptr_t)gains.data_ptr() % 16 != 0 ||
+      (uintptr_t)cos_sin.data_ptr() % 16 != 0 ||
+      (uintptr_t)kv_cache.data_ptr() % 16 != 0 || D % 32 != 0 ||
+      !bias_fits(bias, w) || M == 0 ||
+      !stream_linear_takes(x, w, w.size(0)) ||
+      !norm_sizes(M, w.size(0), x.size(1), false, half)) {
+    auto qkv = norm_linear(x, gains, eps, w, bias, false);
+    auto rows = qkv.view({M, Hq + 2 * Hkv, D});
+    auto q = rows.narrow(1, 0, Hq);
+    rope_and_cache(positions, q, rows.narrow(1, Hq, Hkv),
+                   rows.narrow(1, Hq + Hkv, Hkv), cos_sin, D, kv_cache, slots);
+    return q;
+  }
+  Beside beside;
+  if (bias.has_value()) beside.bias = (const short*)bias->data_ptr();
+  beside.gains = (const short*)gains.data_ptr();
+  beside.eps = (float)eps;
+  Heads heads;
+  heads.positions = positions.data_ptr<int64_t>();
+  heads.slots = slots.data_ptr<int64_t>();
+  heads.cos_sin = cos_sin.data_ptr<float>();
+  heads.kv_cache = kv_cache.data_ptr();
+  heads.plane = kv_cache.stride(0);
+  heads.half = half;
+  heads.q_heads = (int)Hq;
+  heads.kv_heads = (int)Hkv;
+  heads.block_size = (int)kv_cache.size(3);
+  heads.fp8 = kv_cache.scalar_type() == torch::kFloat8_e4m3fn;
+  auto out = torch::empty({M, Hq, D}, x.options());
+  launch<BF16Tag, ROPE, true>(out, x, w, beside, (int)(w.size(0) / 2), heads);
   HIP_CHECK_KERNEL();
   return out;
 }
@@ -544,9 +741,9 @@ torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w) {
     return silu_and_mul(lt_linear(x, w, c10::nullopt)).reshape(sizes);
   }
   if (x.scalar_type() == torch::kBFloat16)
-    launch<BF16Tag, true>(out, x, w, Beside{}, (int)N);
+    launch<BF16Tag, SILU>(out, x, w, Beside{}, (int)N);
   else
-    launch<FP16Tag, true>(out, x, w, Beside{}, (int)N);
+    launch<FP16Tag, SILU>(out, x, w, Beside{}, (int)N);
   HIP_CHECK_KERNEL();
   return out.reshape(sizes);
 }

@@ -22,6 +22,10 @@ constexpr __host__ __device__ int sp_gain_bytes(int steps, int waves) {
   return ((steps + waves - 1) / waves + 7) / 8 * SP_FILL;
 }
 
+struct Nothing {
+  DEVINL void operator()() const {}
+};
+
 // NI: 16-row groups of weights; XG: groups of 8 rows of x; WV: waves that
 // multiply (of NW in the workgroup), each with a ring of D steps.
 // NORM: the rows of x are multiplied by gains, one for each column of K, on
@@ -46,13 +50,17 @@ struct StreamProduct {
   // rows l4 * 4 .. + 3 of row l16. NORM: sum(T)[j] is the sum of squares of
   // row l16 of the j-th 16 over these steps; the gains take
   // sp_gain_bytes(s1 - s0, WV) of LDS behind LDS for each wave.
+  // early(): what the caller loads for the end, asked for behind the first
+  // fills, which it would keep waiting before them.
+  template <typename Early = Nothing>
   static DEVINL void run(char* lds, const int wave, const int s0,
                          const int s1, const int turn_seed,
                          const char* __restrict__ w,
                          const uint32_t (&wat)[2 * NI],
                          const char* __restrict__ x,
                          const uint32_t (&xat)[XG],
-                         const char* __restrict__ gains = nullptr) {
+                         const char* __restrict__ gains = nullptr,
+                         const Early& early = Early{}) {
     const int lane = threadIdx.x % WAVE_SIZE;
     const int l16 = lane & 15;
     const int l4 = lane >> 4;
@@ -139,11 +147,13 @@ struct StreamProduct {
           for (int j = 0; j < MT; ++j)
             acc[i][j] = mfma16<Tag>(wf[u][i], xf[u][j], acc[i][j]);
     };
+    if (n == 0) early();
     if (n > 0) {
       // Short waves fill the last step more than once: the counts that the
       // waits go by stay the same.
 #pragma unroll
       for (int d = 0; d < D - 1; ++d) fill(d, d);
+      early();
       int slot = 0, i = 0;
       for (; i + D - 1 < n; ++i) {
         fill(i + D - 1, slot == 0 ? D - 1 : slot - 1);

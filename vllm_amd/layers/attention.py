@@ -69,11 +69,7 @@ class Attention(nn.Module):
             # what matters, not values).
             return self._profile_attention(q, k, v, meta).reshape(T, -1)
 
-        kv_cache = ctx.kv_caches[self.layer_idx]
-        use_w = (self.kv_group == "window"
-                 and meta.block_table_w is not None)
-        slot_mapping = meta.slot_mapping_w if use_w else meta.slot_mapping
-        block_table = meta.block_table_w if use_w else meta.block_table
+        kv_cache, slot_mapping = self.written(ctx)
         if rotary is not None:
             positions, rope = rotary
             ops.rope_and_cache(positions, q, k, v, rope.cos_sin_cache,
@@ -81,10 +77,26 @@ class Attention(nn.Module):
                                slot_mapping)
         else:
             ops.reshape_and_cache(k, v, kv_cache, slot_mapping)
+        return self.attend(q, ctx)
+
+    def _by_window(self, meta) -> bool:
+        return self.kv_group == "window" and meta.block_table_w is not None
+
+    def written(self, ctx):
+        """The cache that the step's keys and values go to, and where."""
+        meta = ctx.attn_metadata
+        return (ctx.kv_caches[self.layer_idx],
+                meta.slot_mapping_w if self._by_window(meta)
+                else meta.slot_mapping)
+
+    def attend(self, q, ctx) -> torch.Tensor:
+        """Attention of q [T, Hq, D] over the cache, which holds the step's
+        keys and values by now."""
+        meta = ctx.attn_metadata
         out = ops.attention_unified(
             q,
-            kv_cache,
-            block_table,
+            ctx.kv_caches[self.layer_idx],
+            meta.block_table_w if self._by_window(meta) else meta.block_table,
             meta.query_start_loc,
             meta.seq_lens,
             self.scale,
@@ -94,7 +106,7 @@ class Attention(nn.Module):
             max_query_len=meta.max_query_len,
             max_decode_len=meta.max_decode_len,
         )
-        return out.reshape(T, -1)
+        return out.reshape(q.shape[0], -1)
 
     def _profile_attention(self, q, k, v, meta) -> torch.Tensor:
         """Cache-less varlen attention for the memory-profiling dummy run."""

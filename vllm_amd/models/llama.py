@@ -140,6 +140,25 @@ class LlamaAttention(nn.Module):
         return self.attn(q, k, v, rotary=(positions, self.rotary_emb))
 
 
+    def turns_in_projection(self, positions, ctx) -> bool:
+        """Whether norm_qkv_rope_cache does what happens between the norm
+        and attention: heads turned over their whole width, as neighbours of
+        half a width, and a cache of the kernel's types."""
+        attn, rope = self.attn, self.rotary_emb
+        if (self.q_norm is not None or not ctx.kv_caches
+                or type(attn) is not Attention
+                or type(rope) is not RotaryEmbedding
+                or rope.rotary_dim != self.head_dim or not rope.is_neox
+                or positions.dtype != torch.int64
+                or not positions.is_contiguous() or hooked(attn, rope)):
+            return False
+        kv_cache, slots = attn.written(ctx)
+        return (kv_cache.dtype in (torch.bfloat16, torch.float8_e4m3fn)
+                and kv_cache.dim() == 5 and kv_cache.is_contiguous()
+                and slots.dtype == torch.int64 and slots.is_contiguous()
+                and positions.dim() == 1)
+
+
 class LlamaDecoderLayer(nn.Module):
     def __init__(self, spec: ModelSpec, layer_idx: int, dtype, max_position,
                  cache_idx: int = -1):
@@ -204,12 +223,20 @@ class LlamaDecoderLayer(nn.Module):
         """The layer on the residual stream itself: norms on the way into
         products, and sums as products' epilogues (four layers of 4096 and
         the logits, 1 row of 1000 keys 526 -> 508 us, 8 short rows 534 ->
-        512)."""
+        512), and rotation and cache write too (498 and 502)."""
         attn, mlp = self.self_attn, self.mlp
         norm, proj = self.input_layernorm, attn.qkv_proj
-        x = ops.norm_linear(hidden, norm.weight, norm.eps, proj.weight,
-                            proj.bias)
-        x, proj = attn.attend(positions, x), attn.o_proj
+        ctx, rope = get_forward_context(), attn.rotary_emb
+        if attn.turns_in_projection(positions, ctx):
+            kv_cache, slots = attn.attn.written(ctx)
+            x = ops.norm_qkv_rope_cache(
+                hidden, norm.weight, norm.eps, proj.weight, proj.bias,
+                positions, rope.cos_sin_cache, kv_cache, slots)
+            x = attn.attn.attend(x, ctx)
+        else:
+            x = attn.attend(positions, ops.norm_linear(
+                hidden, norm.weight, norm.eps, proj.weight, proj.bias))
+        proj = attn.o_proj
         hidden = ops.linear_add(x, proj.weight, proj.bias, hidden)
         norm = self.post_attention_layernorm
         x = ops.norm_linear(hidden, norm.weight, norm.eps,

@@ -133,6 +133,15 @@ def norm_linear(x, gain, eps, weight, bias=None, silu=False):
                                              silu)
 
 
+def norm_qkv_rope_cache(x, gain, eps, weight, bias, positions, cos_sin_cache,
+                        kv_cache, slot_mapping):
+    """norm_linear by the weights of query, key and value heads, then
+    rope_and_cache over whole heads; the rotated queries [T, Hq, D]."""
+    return get_backend(x.device).norm_qkv_rope_cache(
+        x, gain, eps, weight, bias, positions, cos_sin_cache, kv_cache,
+        slot_mapping)
+
+
 def linear_add(x, weight, bias, residual):
     """linear(x, weight, bias) + residual."""
     return get_backend(x.device).linear_add(x, weight, bias, residual)

@@ -188,6 +188,18 @@ def norm_linear(x, gain, eps, weight, bias=None, silu=False):
     return linear(y, weight, bias)
 
 
+def norm_qkv_rope_cache(x, gain, eps, weight, bias, positions, cos_sin_cache,
+                        kv_cache, slot_mapping):
+    head_dim, kv_heads = kv_cache.shape[4], kv_cache.shape[2]
+    qkv = norm_linear(x, gain, eps, weight, bias)
+    q, k, v = qkv.view(x.shape[0], -1, head_dim).split(
+        [qkv.shape[1] // head_dim - 2 * kv_heads, kv_heads, kv_heads], dim=1)
+    q = q.contiguous()
+    rope_and_cache(positions, q, k, v, cos_sin_cache, head_dim, True,
+                   kv_cache, slot_mapping)
+    return q
+
+
 def linear_add(x, weight, bias, residual):
     return linear(x, weight, bias) + residual
 

@@ -115,6 +115,12 @@ def norm_linear(x, gain, eps, weight, bias=None, silu=False):
     return _C.norm_linear(x, gain, eps, weight, bias, silu)
 
 
+def norm_qkv_rope_cache(x, gain, eps, weight, bias, positions, cos_sin_cache,
+                        kv_cache, slot_mapping):
+    return _C.norm_qkv_rope_cache(x, gain, eps, weight, bias, positions,
+                                  slot_mapping, cos_sin_cache, kv_cache)
+
+
 def linear_add(x, weight, bias, residual):
     return _C.linear_add(x, weight, bias, residual)
 
