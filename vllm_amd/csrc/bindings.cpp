@@ -57,7 +57,7 @@ torch::Tensor norm_qkv_rope_cache(
     c10::optional<torch::Tensor> bias, torch::Tensor positions,
     torch::Tensor slots, torch::Tensor cos_sin, torch::Tensor kv_cache);
 bool layer_streams(int64_t rows, int64_t hidden, int64_t qkv, int64_t heads,
-                   int64_t gate_up, int64_t inner);
+                   int64_t gate_up, int64_t inner, int64_t half);
 std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
                                  bool silu);
 std::vector<int64_t> linear_starts(int64_t rows, int64_t weight_rows,
@@ -247,7 +247,7 @@ TORCH_LIBRARY(vllm_amd, m) {
         "Tensor? bias, Tensor positions, Tensor slots, Tensor cos_sin, "
         "Tensor(a!) kv_cache) -> Tensor");
   m.def("layer_streams(int rows, int hidden, int qkv, int heads, "
-        "int gate_up, int inner) -> bool",
+        "int gate_up, int inner, int half) -> bool",
         &vllm_amd::layer_streams);
   m.def("linear_form(int rows, int weight_rows, int k, bool silu) -> int[]",
         &vllm_amd::linear_form);

@@ -61,11 +61,12 @@ void rope_and_cache(torch::Tensor positions, torch::Tensor q, torch::Tensor k,
 // tile_linear.hip
 bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
                  const torch::Tensor& w, bool silu);
+bool tile_linear_add(torch::Tensor& out, const torch::Tensor& x,
+                     const torch::Tensor& w, bool silu, const short* residual);
 
 namespace {
 
 constexpr int SL_ROWS = 64;      // rows of x at most
-constexpr int SL_NORM_ROWS = 16; // ... that are normalized on their way
 constexpr int SL_PARTS = 8;      // of K, over workgroups
 constexpr int SL_JOBS = 1024;    // column tiles whose K is split
 constexpr int SL_LDS = 160 * 1024;
@@ -142,7 +143,6 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     f32x4* __restrict__ part_sums, unsigned* __restrict__ arrived) {
   using P = StreamProduct<Tag, NI, XG, WV, D, NORM>;
   constexpr int MT = P::MT;
-  static_assert(!NORM || MT == 1);
   constexpr int NO = PAIR ? NI / 2 : NI;
   extern __shared__ __align__(16) char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
@@ -178,8 +178,10 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
   constexpr int PER = (TO + WV - 1) / WV;
   constexpr int H = PAIR ? 2 : 1;
   s16x4 residual[PER];
+  s16x4 bias[PER][2];   // (of turned pairs)
   f32x4 cos[PER], sin[PER];
-  int64_t slot = -1;
+  constexpr int SAME = WV % MT == 0 ? 1 : PER;   // row groups of a wave's tiles
+  int64_t slots[SAME];
   auto early = [&] {
     if constexpr (PAIR == SINGLE && !NORM) {
       if (beside.residual == nullptr) return;
@@ -195,21 +197,36 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     if constexpr (PAIR == ROPE) {
       // By way of the scalar cache: a wait for a load would be one for the
       // fills before it.
-      int pos = 0;
+      int pos[SAME];
 #pragma unroll
-      for (int r = 0; r < XG * 8; ++r) {
-        const int p = load_uniform(
-            reinterpret_cast<const int*>(heads.positions + min(r, M - 1)));
-        if (l16 == r) pos = p;
+      for (int u = 0; u < SAME; ++u) {
+        const int r0 = (u * WV + wave) % MT * 16;
+        pos[u] = 0;
+#pragma unroll
+        for (int r = 0; r < (XG == 1 ? 8 : 16); ++r) {
+          const int p = load_uniform(reinterpret_cast<const int*>(
+              heads.positions + min(r0 + r, M - 1)));
+          if (l16 == r) pos[u] = p;
+        }
       }
-      slot = heads.slots[min(l16, M - 1)];
-      const float* turn = heads.cos_sin + (int64_t)pos * (2 * heads.half);
+#pragma unroll
+      for (int u = 0; u < SAME; ++u)
+        slots[u] =
+            heads.slots[min((u * WV + wave) % MT * 16 + l16, M - 1)];
 #pragma unroll
       for (int u = 0; u < PER; ++u) {
         const int t = min(u * WV + wave, TO - 1);
         const int p = n0 - head * heads.half + (t / MT) * 16 + l4 * 4;
+        const float* turn =
+            heads.cos_sin + (int64_t)pos[u % SAME] * (2 * heads.half);
         cos[u] = *reinterpret_cast<const f32x4*>(turn + p);
         sin[u] = *reinterpret_cast<const f32x4*>(turn + heads.half + p);
+        if (beside.bias != nullptr) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            bias[u][h] = *reinterpret_cast<const s16x4*>(
+                beside.bias + (2 * head + h) * heads.half + p);
+        }
       }
     }
   };
@@ -227,8 +244,8 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
 #pragma unroll
     for (int h = 0; h < H; ++h) v[u][h] = P::sum(lds, h * TO + t);
   }
-  float squares = 0.f;
-  if constexpr (NORM) squares = P::sum(lds, T)[0];
+  f32x4 squares = {0.f, 0.f, 0.f, 0.f};   // of four groups of 16 rows
+  if constexpr (NORM) squares = P::sum(lds, T);
   if (parts > 1) {
     f32x4* sums = part_sums + (int64_t)tile * parts * TN * WAVE_SIZE + lane;
 #pragma unroll
@@ -240,8 +257,7 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
         part_put(sums + (part * TN + h * TO + t) * WAVE_SIZE, v[u][h]);
     }
     if (NORM && wave == 0)
-      part_put(reinterpret_cast<float*>(sums + (part * TN + T) * WAVE_SIZE),
-               squares);
+      part_put(sums + (part * TN + T) * WAVE_SIZE, squares);
     if (!last_to_arrive(arrived, tile, parts,
                         reinterpret_cast<unsigned*>(lds)))
       return;
@@ -271,18 +287,19 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
       }
     }
     if constexpr (NORM) {
-      float p[SL_PARTS];
+      f32x4 p[SL_PARTS];
 #pragma unroll
       for (int q = 0; q < SL_PARTS; ++q)
-        p[q] = part_get(reinterpret_cast<const float*>(
-            sums + (min(q, parts - 1) * TN + T) * WAVE_SIZE));
+        p[q] = part_get(sums + (min(q, parts - 1) * TN + T) * WAVE_SIZE);
       squares = p[0];
 #pragma unroll
       for (int q = 1; q < SL_PARTS; ++q)
         if (q < parts) squares += p[q];
     }
   }
-  const float root = NORM ? rsqrtf(squares / K + beside.eps) : 1.f;
+  f32x4 roots;
+#pragma unroll
+  for (int j = 0; j < MT; ++j) roots[j] = rsqrtf(squares[j] / K + beside.eps);
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
     const int t = u * WV + wave;
@@ -291,6 +308,9 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     const int col = n0 + (t / MT) * 16 + l4 * 4;
     f32x4 o = v[u][0];
     if constexpr (NORM) {
+      float root = roots[0];
+#pragma unroll
+      for (int j = 1; j < MT; ++j) root = t % MT == j ? roots[j] : root;
 #pragma unroll
       for (int h = 0; h < H; ++h) v[u][h] *= root;
       o = v[u][0];
@@ -310,8 +330,7 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
         f32x4 z = v[u][h];
         if (beside.bias != nullptr) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            z[r] += to_f32<Tag>(beside.bias[(2 * head + h) * half + p + r]);
+          for (int r = 0; r < 4; ++r) z[r] += to_f32<Tag>(bias[u][h][r]);
         }
         // Rounded as a product of its own would leave them.
         to[h] = int2{pack2<Tag>(z[0], z[1]), pack2<Tag>(z[2], z[3])};
@@ -336,6 +355,7 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
         *reinterpret_cast<int2*>(q + half) = to[1];
         continue;
       }
+      const int64_t slot = slots[u % SAME];
       if (slot < 0) continue;   // padding
       const bool value = head >= heads.q_heads + heads.kv_heads;
       const int kvh = head - heads.q_heads - (value ? heads.kv_heads : 0);
@@ -429,7 +449,7 @@ void launch_form(torch::Tensor& out, const torch::Tensor& x,
                  const Heads& heads, int N, int parts) {
   constexpr Form f = SL_FORMS[I];
   if constexpr (lds_bytes(f, XG, NORM) <= SL_LDS && (f.wv > 2 || XG == 8) &&
-                (!PAIR || f.ni % 2 == 0) && (!NORM || XG <= 2)) {
+                (!PAIR || f.ni % 2 == 0)) {
     const int lds =
         lds_bytes(f, XG, NORM ? ceil_div((int)x.size(1) / SP_K, parts) : 0);
     const int M = (int)x.size(0), K = (int)x.size(1);
@@ -589,10 +609,17 @@ torch::Tensor linear_add(torch::Tensor a, torch::Tensor w,
               "linear_add: [M, K] x [N, K] + [M, N]");
   auto x = a.contiguous();
   if (x.size(0) == 0 || !residual.is_contiguous() ||
-      (uintptr_t)residual.data_ptr() % 8 != 0 || !bias_fits(bias, w) ||
-      tile_linear_first(x.size(0), w.size(0), x.size(1), false) ||
-      !stream_linear_takes(x, w, w.size(0)))
+      (uintptr_t)residual.data_ptr() % 8 != 0 || !bias_fits(bias, w))
     return lt_linear(x, w, bias) + residual;
+  const bool tiles = !bias.has_value() &&
+                     tile_linear_first(x.size(0), w.size(0), x.size(1), false);
+  if (tiles || !stream_linear_takes(x, w, w.size(0))) {
+    auto out = torch::empty({x.size(0), w.size(0)}, x.options());
+    if (!bias.has_value() &&
+        tile_linear_add(out, x, w, false, (const short*)residual.data_ptr()))
+      return out;
+    return lt_linear(x, w, bias) + residual;
+  }
   Beside beside;
   if (bias.has_value()) beside.bias = (const short*)bias->data_ptr();
   beside.residual = (const short*)residual.data_ptr();
@@ -600,26 +627,46 @@ torch::Tensor linear_add(torch::Tensor a, torch::Tensor w,
 }
 
 // Whether the norm of `rows` rows goes with the product (bf16 only: fp16 rows
-// times gains may pass 65504 where normalized ones do not). Up to 16 rows: a
-// step's rows are multiplied by its gains in every workgroup, and from 17 on
-// the gains no longer fit beside the widest form's weights.
+// times gains may pass 65504 where normalized ones do not). Up to 32 rows, if
+// the gains leave room for the form that the product takes without them, and
+// with half a head's columns up to 64 rows in any form, since a launch for the
+// rotation goes too. us with the launches that go, and in one (4096 x 6144 with
+// the rotation, 4096 x 28672 and 3584 x 37888 with the activation): 8 rows 16.0
+// and 12.0, 38.0 and 35.5, 48.0 and 45.9; 32 rows 19.1 and 14.4, 39.5 and 41.4
+// (another form: not taken), 53.1 and 51.5; 64 rows 22.8 and 18.8, tiles, 53.7
+// and 59.7 (rows are multiplied by gains in two waves: not taken).
 static bool norm_sizes(int64_t rows, int64_t weight_rows, int64_t k,
                        bool silu, int half = 0) {
-  return rows <= SL_NORM_ROWS &&
-         stream_sizes(rows, weight_rows, silu ? weight_rows / 2 : weight_rows,
-                      k) &&
-         plan(row_groups(rows), weight_rows, (int)k, silu, true, half).form >= 0;
+  if (tile_linear_first(rows, weight_rows, k, silu) ||
+      !stream_sizes(rows, weight_rows, silu ? weight_rows / 2 : weight_rows,
+                    k))
+    return false;
+  const int xg = row_groups(rows);
+  const Plan with = plan(xg, weight_rows, (int)k, silu, true, half);
+  if (half > 0) return with.form >= 0;
+  const Plan without = plan(xg, weight_rows, (int)k, silu);
+  return rows <= 32 && with.form == without.form &&
+         with.parts == without.parts;
 }
 
-// Whether a decoder layer's products of `rows` rows go without launches for
-// its norms: `qkv` and `gate_up` weight rows on the norms of `hidden` columns,
-// and products back to `hidden` columns from `heads` and `inner` ones.
+// Whether the residual goes with the product, without a bias.
+static bool add_sizes(int64_t rows, int64_t weight_rows, int64_t k) {
+  if (tile_linear_first(rows, weight_rows, k, false))
+    return tile_linear_form(rows, weight_rows, k, false).parts > 1;
+  return stream_sizes(rows, weight_rows, weight_rows, k);
+}
+
+// Whether a decoder layer of up to 64 rows has fewer launches if products take
+// its norms, sums and rotation along: `qkv` and `gate_up` weight rows on norms
+// of `hidden` columns, products back to them from `heads` and `inner` columns,
+// heads of twice `half` columns that turn as a whole (0: others). Sums must be
+// epilogues, or launches would only move; a norm may stay one.
 bool layer_streams(int64_t rows, int64_t hidden, int64_t qkv, int64_t heads,
-                   int64_t gate_up, int64_t inner) {
-  return norm_sizes(rows, qkv, hidden, false) &&
-         norm_sizes(rows, gate_up, hidden, true) && gate_up == 2 * inner &&
-         stream_sizes(rows, hidden, hidden, heads) &&
-         stream_sizes(rows, hidden, hidden, inner);
+                   int64_t gate_up, int64_t inner, int64_t half) {
+  return gate_up == 2 * inner && rows > 0 && rows <= SL_ROWS &&
+         add_sizes(rows, hidden, heads) && add_sizes(rows, hidden, inner) &&
+         (norm_sizes(rows, qkv, hidden, false, (int)half) ||
+          norm_sizes(rows, gate_up, hidden, true));
 }
 
 // linear (or, silu, linear_silu_and_mul) of rms_norm(a, gains, eps); in one
@@ -692,7 +739,8 @@ torch::Tensor norm_qkv_rope_cache(
       !gains.is_contiguous() || (uintptr_t)gains.data_ptr() % 16 != 0 ||
       (uintptr_t)cos_sin.data_ptr() % 16 != 0 ||
       (uintptr_t)kv_cache.data_ptr() % 16 != 0 || D % 32 != 0 ||
-      !bias_fits(bias, w) || M == 0 ||
+      !bias_fits(bias, w) ||
+      (bias.has_value() && (uintptr_t)bias->data_ptr() % 8 != 0) || M == 0 ||
       !stream_linear_takes(x, w, w.size(0)) ||
       !norm_sizes(M, w.size(0), x.size(1), false, half)) {
     auto qkv = norm_linear(x, gains, eps, w, bias, false);

@@ -101,7 +101,11 @@ struct StreamProduct {
     // The product is formed transposed. (Of 8 rows the upper lanes repeat
     // the lower.)
     const int xrow = XG == 1 ? l16 & 7 : l16;
-    float squares[MT] = {};
+    // Rows by themselves: their sums of squares are the diagonal. (Matrix cores
+    // have time; by the vector ALU, in a chain, the same within 2 %.)
+    f32x4 squares[MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) squares[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto multiply = [&](int slot, int i) {
       const char* from = ring + slot * STEP;
       s16x8 wf[2][NI], xf[2][MT];
@@ -126,15 +130,12 @@ struct StreamProduct {
           const i32x4 gf = *reinterpret_cast<const i32x4*>(g + u * 64);
 #pragma unroll
           for (int j = 0; j < MT; ++j) {
+            squares[j] = mfma16<Tag>(xf[u][j], xf[u][j], squares[j]);
             i32x4 f = __builtin_bit_cast(i32x4, xf[u][j]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float a = unpack_lo<Tag>(f[e]), b = unpack_hi<Tag>(f[e]);
-              squares[j] += a * a;
-              squares[j] += b * b;
-              f[e] = pack2<Tag>(a * unpack_lo<Tag>(gf[e]),
-                                b * unpack_hi<Tag>(gf[e]));
-            }
+            for (int e = 0; e < 4; ++e)
+              f[e] = pack2<Tag>(unpack_lo<Tag>(f[e]) * unpack_lo<Tag>(gf[e]),
+                                unpack_hi<Tag>(f[e]) * unpack_hi<Tag>(gf[e]));
             xf[u][j] = __builtin_bit_cast(s16x8, f);
           }
         }
@@ -183,8 +184,11 @@ struct StreamProduct {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
-          v[j] = squares[j] + __shfl_xor(squares[j], 16, WAVE_SIZE);
-          v[j] += __shfl_xor(v[j], 32, WAVE_SIZE);
+          float own = squares[j][0];   // of row l16, in group l16 / 4
+#pragma unroll
+          for (int r = 1; r < 4; ++r)
+            own = (l16 & 3) == r ? squares[j][r] : own;
+          v[j] = __shfl(own, (l16 >> 2) * 16 + l16, WAVE_SIZE);
         }
         red[(wave * TN + T) * WAVE_SIZE + lane] = v;
       }

@@ -146,9 +146,9 @@ __global__ __launch_bounds__(TP_THREADS, 1) void tile_linear_kernel(
 // 4096 x 14336, 256 rows, 8 parts 54.9 us so, 45.2 with this launch.)
 template <typename Tag>
 __global__ __launch_bounds__(256) void tile_sums_kernel(
-    short* __restrict__ out, const f32x4* __restrict__ sums, const int M,
-    const int N, const int row_blocks, const int col_blocks,
-    const int parts) {
+    short* __restrict__ out, const f32x4* __restrict__ sums,
+    const short* __restrict__ residual, const int M, const int N,
+    const int row_blocks, const int col_blocks, const int parts) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE_SIZE);
   const int lane = threadIdx.x % WAVE_SIZE;
   const int unit = blockIdx.x * 4 + wave;
@@ -158,6 +158,17 @@ __global__ __launch_bounds__(256) void tile_sums_kernel(
   const int64_t part = (int64_t)row_blocks * col_blocks * 256;
   const f32x4* at =
       sums + ((int64_t)rb * col_blocks + cb) * 256 + b * 64 + lane;
+  const int row = rb * 32 + b * 16 + (lane & 15);
+  s16x4 add[2] = {};
+  if (residual != nullptr && row < M) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int col = cb * 32 + c * 16 + (lane >> 4) * 4;
+      if (col < N)
+        add[c] = *reinterpret_cast<const s16x4*>(residual + (int64_t)row * N +
+                                                 col);
+    }
+  }
   f32x4 v[2];
   constexpr int Q = 8;
   for (int p0 = 0; p0 < parts; p0 += Q) {
@@ -179,8 +190,13 @@ __global__ __launch_bounds__(256) void tile_sums_kernel(
         v[c][r] = a;
       }
   }
+  if (residual != nullptr) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[c][r] += to_f32<Tag>(add[c][r]);
+  }
   const i32x4 chunk = row_chunk16<Tag>(v[0], v[1]);
-  const int row = rb * 32 + b * 16 + (lane & 15);
   const int col = cb * 32 + row_start16();
   if (row < M && col < N)
     *reinterpret_cast<i32x4*>(out + (int64_t)row * N + col) = chunk;
@@ -333,7 +349,8 @@ TileForm tile_form(int64_t M, int64_t rows_w, int64_t K, bool silu) {
 
 template <typename Tag, bool SILU>
 void launch(torch::Tensor& out, const torch::Tensor& x,
-            const torch::Tensor& w, TileForm form) {
+            const torch::Tensor& w, TileForm form,
+            const short* residual = nullptr) {
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)out.size(1);
   constexpr int H = SILU ? 2 : 1;
   const int tm = M <= 128 ? 128 : 256;
@@ -376,8 +393,8 @@ void launch(torch::Tensor& out, const torch::Tensor& x,
   if (form.parts > 1)
     hipLaunchKernelGGL((tile_sums_kernel<Tag>),
                        dim3(ceil_div(row_blocks * col_blocks * 2, 4)),
-                       dim3(256), 0, stream, (short*)out.data_ptr(), to, M, N,
-                       row_blocks, col_blocks, form.parts);
+                       dim3(256), 0, stream, (short*)out.data_ptr(), to,
+                       residual, M, N, row_blocks, col_blocks, form.parts);
 }
 
 }  // namespace
@@ -413,12 +430,15 @@ std::vector<int64_t> linear_starts(int64_t rows, int64_t weight_rows,
 }
 
 // The product of x [M, K] and w [rows, K], both contiguous, into out [M, n],
-// if it is one that this file takes.
-bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
-                 const torch::Tensor& w, bool silu) {
+// if it is one that this file takes. With a residual [M, n] (8 B places, not
+// beside an activation) the sum of both, if K is split: it is added with the
+// parts then.
+bool tile_linear_add(torch::Tensor& out, const torch::Tensor& x,
+                     const torch::Tensor& w, bool silu,
+                     const short* residual) {
   const int64_t K = x.size(1);
   const TileForm form = tile_linear_form(x.size(0), w.size(0), K, silu);
-  if (form.cols == 0 || w.size(1) != K || w.scalar_type() != x.scalar_type() ||
+  if (form.cols == 0 || (residual != nullptr && (silu || form.parts == 1)) || w.size(1) != K || w.scalar_type() != x.scalar_type() ||
       (x.scalar_type() != torch::kBFloat16 &&
        x.scalar_type() != torch::kHalf) ||
       !x.is_contiguous() || !w.is_contiguous() ||
@@ -426,13 +446,18 @@ bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
     return false;
   if (x.scalar_type() == torch::kBFloat16) {
     if (silu) launch<BF16Tag, true>(out, x, w, form);
-    else      launch<BF16Tag, false>(out, x, w, form);
+    else      launch<BF16Tag, false>(out, x, w, form, residual);
   } else {
     if (silu) launch<FP16Tag, true>(out, x, w, form);
-    else      launch<FP16Tag, false>(out, x, w, form);
+    else      launch<FP16Tag, false>(out, x, w, form, residual);
   }
   HIP_CHECK_KERNEL();
   return true;
+}
+
+bool tile_linear(torch::Tensor& out, const torch::Tensor& x,
+                 const torch::Tensor& w, bool silu) {
+  return tile_linear_add(out, x, w, silu, nullptr);
 }
 
 }  // namespace vllm_amd

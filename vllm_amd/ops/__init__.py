@@ -147,14 +147,15 @@ def linear_add(x, weight, bias, residual):
     return get_backend(x.device).linear_add(x, weight, bias, residual)
 
 
-def layer_streams(x, qkv, heads, gate_up, inner):
-    """Whether a decoder layer on x [rows, hidden] is faster by norm_linear
-    and linear_add than with norms of its own: qkv and gate_up rows of weights
-    behind the norms, and heads and inner columns before the products back to
-    the hidden size."""
+def layer_streams(x, qkv, heads, gate_up, inner, half):
+    """Whether a decoder layer on x [rows, hidden] is faster by
+    norm_qkv_rope_cache, norm_linear and linear_add than by norms, rotation and
+    sums of their own: qkv and gate_up rows of weights behind the norms, heads
+    and inner columns before the products back to the hidden size, half a
+    head's columns if heads turn as a whole, else 0."""
     return (x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous()
             and get_backend(x.device).layer_streams(
-                x.shape[0], x.shape[1], qkv, heads, gate_up, inner))
+                x.shape[0], x.shape[1], qkv, heads, gate_up, inner, half))
 
 
 def linear_fp8(x, w_fp8, w_scale, bias=None):

@@ -126,10 +126,9 @@ def linear_add(x, weight, bias, residual):
 
 
 @functools.lru_cache(maxsize=None)
-def layer_streams(rows, hidden, qkv, heads, gate_up, inner):
-    # Up to 16 rows, for layers whose products all stream their weights
-    # (csrc/stream_linear.hip).
-    return _C.layer_streams(rows, hidden, qkv, heads, gate_up, inner)
+def layer_streams(rows, hidden, qkv, heads, gate_up, inner, half):
+    # Up to 64 rows (csrc/stream_linear.hip).
+    return _C.layer_streams(rows, hidden, qkv, heads, gate_up, inner, half)
 
 
 def quant_fp8_dynamic(x):
