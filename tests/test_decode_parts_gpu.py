@@ -66,6 +66,29 @@ def test_merge(ctx, hq, hkv, hd, window, dtype, cache):
                                atol=2.0 ** -9)
 
 
+# Rows at the ends of what one partition takes in one, two and three steps of
+# its waves, and past it.
+@pytest.mark.parametrize("hd,cache", [(64, None), (128, None), (256, None),
+                                      (128, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("told", [129, 256, 257, 384, 385])
+def test_short_rows(hd, cache, told):
+    from vllm_amd.ops import hip_ops
+    ctx = [told, 1, 128, 129, min(told, 256), 64, 0]
+    q, kv, table, qsl, lens = _rows(ctx, 8, 2, hd, torch.bfloat16,
+                                    cache or torch.bfloat16)
+    out = hip_ops.attention_unified(
+        q, kv, table, qsl, lens, hd ** -0.5, num_decodes=len(ctx),
+        max_seq_len=told)
+    assert (out[-1] == 0).all()
+    n = len(ctx) - 1
+    expect = ref.attention_unified(q[:n].float(), kv.float(), table[:n],
+                                   qsl[:n + 1], lens[:n], hd ** -0.5,
+                                   num_decodes=n)
+    # The output's own rounding, as above.
+    torch.testing.assert_close(out[:n].float(), expect, rtol=2.0 ** -8,
+                               atol=2.0 ** -9)
+
+
 # A key's halves lie on neighbouring lanes where its row has 128 B or more:
 # every row size, with all of the columns that a group may have and with one.
 @pytest.mark.parametrize("group", [1, 8])

@@ -131,6 +131,20 @@ def test_decode_parts(hip, rows, kv, span, window, parts):
     assert hip._decode_parts(rows, kv, span, window) == parts
 
 
+@pytest.mark.parametrize("rows,kv,span,hd,size,parts", [
+    (1, 8, 384, 128, 2, 1), (1, 8, 385, 128, 2, 4),    # not worth a merge
+    (16, 8, 384, 64, 1, 1), (1, 2, 256, 256, 2, 1), (1, 2, 257, 256, 2, 3),
+    (4, 8, 8192, 128, 2, 8), (4, 8, 8192, 128, 1, 16),  # one a CU, two
+    (3, 8, 8192, 128, 2, 10), (5, 8, 8192, 128, 2, 6),
+    (7, 8, 8192, 128, 2, 4), (9, 8, 8192, 128, 2, 8),   # 224 CUs, 216
+    (16, 8, 2000, 128, 2, 2), (17, 8, 2000, 128, 2, 4),
+    (16, 8, 8192, 128, 2, 4),     # none longer than 2048 keys
+    (1, 28, 8192, 128, 2, 9)])
+def test_decode_parts_of_short_and_few_rows(hip, rows, kv, span, hd, size,
+                                            parts):
+    assert hip._decode_parts(rows, kv, span, 0, hd, size) == parts
+
+
 @pytest.mark.parametrize("tokens,topk,E,H,form", [
     (64, 8, 64, 7168, 0),      # one streamed tile holds any expert's rows
     (65, 8, 64, 7168, 1),      # no longer

@@ -31,7 +31,8 @@ _DEC_MAX_UNITS = 16
 _DEC_FILL = 512
 
 
-def _decode_parts(rows, kv_heads, max_seq_len, sliding_window):
+def _decode_parts(rows, kv_heads, max_seq_len, sliding_window, head_dim=128,
+                  kv_bytes=1):
     """Into how many partitions a row's keys are split. Every partition
     costs a pass over its fp32 partials, so no more than fill the chip:
     16 rows x 4096 keys (8 KV heads of 128) take 45.3 us in 4 partitions,
@@ -40,15 +41,34 @@ def _decode_parts(rows, kv_heads, max_seq_len, sliding_window):
     cost: 256 rows x 129..2176 keys take 206 us in 2, 244 in 9; 64 rows
     x 4096..8192 fp8 keys 144 us in 4, 172 in 32. For one or two rows one
     workgroup a CU does: one x 8000 keys 13.2 us in 32, 16.3 in 63; two x
-    8000 16.9 in 16, 18.5 in 32 (24 x 500..3000 45.1 in 2, 40.4 in 3). At
-    most 64, the lanes of the merging wave."""
+    8000 16.9 in 16, 18.5 in 32 (24 x 500..3000 45.1 in 2, 40.4 in 3). So
+    it does for more rows with a cache of 16 bits, where partitions come out
+    that 220 of the 256 CUs have one: us in one, and two, a CU, rows alike
+    and from a fifth on (8 KV heads of 128) 4 x 2500 11.7 and 14.1, 10.7 and
+    12.4; 8 x 4000 23.5 and 24.6, 17.5 and 19.5; 16 x 1200 16.7 and 18.0,
+    13.5 and 15.2, x 4000 44.7 and 43.5, 30.7 and 33.2; 2 heads of 256, 6 x
+    4000 17.2 and 21.5; of 9 rows, 216 CUs, x 800..4000 21.4 and 20.3, with 8
+    bits 16 x 800..4000 23.9 and 20.2. At most 64, the lanes of the merging
+    wave.
+
+    Three steps of a workgroup's waves take no longer than to merge, two of
+    twice the steps with heads of 256: us in one partition and in those of
+    128 keys, 8 KV heads of 128, 1 x 160 4.9 and 6.5, 1 x 384 6.7 and 7.2, 1
+    x 400 7.9 and 7.2, 16 x 256 6.3 and 8.5, 40 x 384 14.5 and 16.3; 2 of
+    256, 1 x 256 8.8 and 10.3, 1 x 384 11.2 and 10.5."""
     span = max(max_seq_len, 1)
     if sliding_window > 0:
         span = min(span, sliding_window + 31)
+    if span <= _DEC_UNIT * (3 if head_dim <= 128 else 2):
+        return 1
     units = -(-span // _DEC_UNIT)
+    groups = max(rows * kv_heads, 1)
     fill = _DEC_FILL // 2 if rows <= 2 else _DEC_FILL
-    parts = max(-(-fill // max(rows * kv_heads, 1)),
-                -(-units // _DEC_MAX_UNITS))
+    parts = -(-fill // groups)
+    one = _DEC_FILL // 2 // groups
+    if kv_bytes > 1 and groups <= 128 and one * groups >= 220:
+        parts = one
+    parts = max(parts, -(-units // _DEC_MAX_UNITS))
     return max(1, min(parts, units, 64))
 
 
@@ -256,7 +276,8 @@ def attention_unified(
         if max_decode_len <= 0:
             max_decode_len = max_seq_len
         num_parts = _decode_parts(num_decodes, kv_cache.shape[2],
-                                  max_decode_len, sliding_window)
+                                  max_decode_len, sliding_window, head_dim,
+                                  kv_cache.element_size())
         if num_parts > 1:
             tmp_out = torch.empty(
                 num_decodes, num_heads, num_parts, head_dim,
