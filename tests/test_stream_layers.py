@@ -1,0 +1,133 @@
+"""Small steps pass by the modules of a layer only where these do what their
+classes say: anything replaced, wrapped or added is called as before."""
+
+import pytest
+import torch
+import torch.nn as nn
+
+from vllm_amd import ops
+from vllm_amd.config import ModelConfig, get_model_spec
+from vllm_amd.models.registry import get_model_class
+from vllm_amd.worker.forward_context import (
+    AttentionMetadata,
+    ForwardContext,
+    set_forward_context,
+)
+
+
+@pytest.fixture
+def net(monkeypatch):
+    """A model on the CPU whose steps are all small enough."""
+    monkeypatch.setattr(ops, "layer_streams", lambda *args: True)
+    name = "tiny-llama-128"
+    spec = get_model_spec(name)
+    torch.manual_seed(0)
+    model = get_model_class(spec.architecture)(
+        ModelConfig(model=name, dtype="bf16", max_model_len=64)).eval()
+    for p in model.parameters():
+        nn.init.normal_(p, std=0.05)
+    return model
+
+
+def _step(model):
+    """Three rows that decode, with a hook-free count of fused layers."""
+    spec = model.config.spec
+    torch.manual_seed(1)
+    caches = [torch.randn(2, 3, spec.num_kv_heads, 64,
+                          spec.head_dim).bfloat16()
+              for _ in range(spec.num_layers)]
+    lens = torch.tensor([4, 9, 30], dtype=torch.int32)
+    meta = AttentionMetadata(
+        query_start_loc=torch.arange(4, dtype=torch.int32), seq_lens=lens,
+        block_table=torch.arange(3, dtype=torch.int32)[:, None],
+        slot_mapping=torch.arange(3) * 64 + lens.long() - 1, num_reqs=3,
+        num_actual_tokens=3, max_query_len=1, max_seq_len=30, num_decodes=3)
+    fused = []
+    inner = ops.linear_add
+    ops.linear_add = lambda *args: fused.append(1) or inner(*args)
+    try:
+        with torch.inference_mode(), set_forward_context(
+                ForwardContext(attn_metadata=meta, kv_caches=caches)):
+            out = model(torch.tensor([7, 3, 1]), lens.long() - 1)
+    finally:
+        ops.linear_add = inner
+    return out, caches, len(fused)
+
+
+def _by_modules(model, monkeypatch):
+    """The step as all modules' calls."""
+    with monkeypatch.context() as m:
+        m.setattr(ops, "layer_streams", lambda *args: False)
+        return _step(model)
+
+
+def _same(got, expect):
+    assert got[2] == expect[2] == 0
+    assert torch.equal(got[0], expect[0])
+    for a, b in zip(got[1], expect[1]):
+        assert torch.equal(a, b)
+
+
+class Wrapped(nn.Module):
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+        self.calls = 0
+
+    def forward(self, *args, **kwargs):
+        self.calls += 1
+        return self.inner(*args, **kwargs)
+
+    def split_qkv(self, qkv):
+        return self.inner.split_qkv(qkv)
+
+
+PROJECTIONS = ["self_attn.qkv_proj", "self_attn.o_proj", "mlp.gate_up_proj",
+               "mlp.down_proj"]
+
+
+def test_plain_layers_are_passed_by(net, monkeypatch):
+    out, caches, fused = _step(net)
+    assert fused == 2 * net.config.spec.num_layers
+    expect = _by_modules(net, monkeypatch)
+    for a, b in [(out, expect[0]), *zip(caches, expect[1])]:
+        # A few roundings of 2^-8 apart.
+        assert (a - b).norm() <= 2.0 ** -5 * b.norm()
+
+
+@pytest.mark.parametrize("name", PROJECTIONS)
+def test_wrapped_projections_are_called(net, monkeypatch, name):
+    layer = net.model.layers[0]
+    parent, attr = name.split(".")
+    wrapped = Wrapped(layer.get_submodule(name))
+    setattr(getattr(layer, parent), attr, wrapped)
+    assert not layer.streams()
+    got = _step(net)
+    assert wrapped.calls == 1
+    _same(got, _by_modules(net, monkeypatch))
+
+
+@pytest.mark.parametrize("name", PROJECTIONS)
+def test_parametrized_weights_are_asked_for(net, monkeypatch, name):
+    class Twice(nn.Module):
+        def forward(self, w):
+            return w * 2
+
+    layer = net.model.layers[0]
+    nn.utils.parametrize.register_parametrization(
+        layer.get_submodule(name), "weight", Twice())
+    assert not layer.streams()
+    _same(_step(net), _by_modules(net, monkeypatch))
+
+
+@pytest.mark.parametrize("name", PROJECTIONS)
+def test_adapters_and_fp8_weights_are_not_plain(net, name):
+    layer = net.model.layers[0]
+    proj = layer.get_submodule(name)
+    assert layer.streams()
+    proj.lora_slices = [(0, 8, "a")]
+    assert not layer.streams()
+    proj.lora_slices = None
+    assert layer.streams()
+    proj.quantize_fp8()
+    assert not layer.streams()

@@ -88,12 +88,13 @@ def plain(*projs) -> bool:
     small steps: what is absent is looked up where it would be, since a
     module's own way to say so takes a microsecond.)"""
     for p in projs:
-        weight = p._parameters["weight"]
-        if ("weight_fp8" in p._buffers
+        if type(p) not in (QKVParallelLinear, RowParallelLinear,
+                           MergedColumnParallelLinear):
+            return False   # (a parametrized one has a class of its own, too)
+        weight = p._parameters.get("weight")
+        if (weight is None or weight.dtype != torch.bfloat16
+                or "weight_fp8" in p._buffers
                 or p.__dict__.get("lora_slices") is not None
-                or weight.dtype != torch.bfloat16
-                or type(p) not in (QKVParallelLinear, RowParallelLinear,
-                                   MergedColumnParallelLinear)
                 or p.__dict__.get("gather_output")):
             return False
     return get_tp_world_size() == 1 and not hooked(*projs)

@@ -139,7 +139,6 @@ class LlamaAttention(nn.Module):
                 k.reshape(-1, self.head_dim).contiguous()).view(k.shape)
         return self.attn(q, k, v, rotary=(positions, self.rotary_emb))
 
-
     def turns_in_projection(self, positions, ctx) -> bool:
         """Whether norm_qkv_rope_cache does what happens between the norm
         and attention: heads turned over their whole width, as neighbours of
@@ -215,8 +214,8 @@ class LlamaDecoderLayer(nn.Module):
         a, m = attn._modules, mlp._modules
         gate_up, act = m["gate_up_proj"], m["act_fn"]
         return (type(act) is SiluAndMul
-                and gate_up.bias is None
                 and plain(a["qkv_proj"], a["o_proj"], gate_up, m["down_proj"])
+                and gate_up.bias is None
                 and not hooked(self, attn, mlp, act, n1, n2))
 
     def forward_stream(self, positions, hidden):
