@@ -131,3 +131,67 @@ def test_adapters_and_fp8_weights_are_not_plain(net, name):
     assert layer.streams()
     proj.quantize_fp8()
     assert not layer.streams()
+
+
+MODULES = PROJECTIONS + ["", "self_attn", "self_attn.attn",
+                         "self_attn.rotary_emb", "mlp", "mlp.act_fn",
+                         "input_layernorm", "post_attention_layernorm"]
+# Called with what they are called with by the layer's modules, beside
+# products that take norms and sums along.
+BESIDE = ["self_attn.attn", "self_attn.rotary_emb"]
+
+
+@pytest.mark.parametrize("name", MODULES)
+def test_replaced_forwards_are_called(net, monkeypatch, name):
+    module = net.model.layers[0].get_submodule(name)
+    calls, inner = [], module.forward
+    module.forward = lambda *a, **kw: calls.append(1) or inner(*a, **kw)
+    got = _step(net)
+    assert len(calls) == 1
+    if name not in BESIDE:
+        _same(got, _by_modules(net, monkeypatch))
+
+
+@pytest.mark.parametrize("name", MODULES)
+def test_replaced_forwards_of_classes_are_called(net, monkeypatch, name):
+    cls = type(net.model.layers[0].get_submodule(name))
+    calls, inner = [], cls.forward
+    monkeypatch.setattr(
+        cls, "forward", lambda *a, **kw: calls.append(1) or inner(*a, **kw))
+    got = _step(net)
+    assert len(calls) >= net.config.spec.num_layers
+    if name not in BESIDE:
+        _same(got, _by_modules(net, monkeypatch))
+
+
+def test_layers_of_other_classes_are_called(net, monkeypatch):
+    from vllm_amd.models.llama import LlamaDecoderLayer
+
+    class Scaled(LlamaDecoderLayer):
+        def forward(self, positions, hidden, residual):
+            hidden, residual = super().forward(positions, hidden, residual)
+            return hidden * 0.5, residual
+
+    net.model.layers[0].__class__ = Scaled
+    _same(_step(net), _by_modules(net, monkeypatch))
+    wrapped = net.model.layers[0] = Wrapped(net.model.layers[0])
+    _same(_step(net), _by_modules(net, monkeypatch))
+    assert wrapped.calls == 2
+
+
+@pytest.mark.parametrize("change", ["hook", "forward", "wrap"])
+def test_the_last_norm_is_called_as_before(net, monkeypatch, change):
+    """With the sublayer's output and the residual apart."""
+    seen = []
+    norm = net.model.norm
+    if change == "hook":
+        norm.register_forward_pre_hook(lambda m, args: seen.append(len(args)))
+    elif change == "forward":
+        norm.forward = lambda *args: seen.append(len(args)) or type(
+            norm).forward(norm, *args)
+    else:
+        net.model.norm = Wrapped(norm)
+        norm.register_forward_pre_hook(lambda m, args: seen.append(len(args)))
+    got = _step(net)
+    assert seen == [2]
+    _same(got, _by_modules(net, monkeypatch))

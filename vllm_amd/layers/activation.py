@@ -6,8 +6,10 @@ import torch
 import torch.nn as nn
 
 from vllm_amd import ops
+from vllm_amd.layers.hooks import passed_by
 
 
+@passed_by
 class SiluAndMul(nn.Module):
     """silu(x[..., :d]) * x[..., d:] — fused gate*up for LLaMA MLPs."""
 

@@ -12,10 +12,11 @@ import torch
 import torch.nn as nn
 
 from vllm_amd import ops
-from vllm_amd.layers.hooks import hooked
+from vllm_amd.layers.hooks import hooked, passed_by
 from vllm_amd.worker.forward_context import get_forward_context
 
 
+@passed_by
 class Attention(nn.Module):
     def __init__(
         self,

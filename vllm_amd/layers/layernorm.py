@@ -9,8 +9,10 @@ import torch
 import torch.nn as nn
 
 from vllm_amd import ops
+from vllm_amd.layers.hooks import passed_by
 
 
+@passed_by
 class RMSNorm(nn.Module):
     def __init__(self, hidden_size: int, eps: float = 1e-6, dtype=None):
         super().__init__()

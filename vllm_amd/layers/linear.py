@@ -19,7 +19,7 @@ import torch.nn as nn
 
 from vllm_amd import ops
 from vllm_amd.layers.activation import SiluAndMul
-from vllm_amd.layers.hooks import hooked
+from vllm_amd.layers.hooks import hooked, passed_by
 from vllm_amd.parallel.state import (
     get_tp_rank,
     get_tp_world_size,
@@ -100,6 +100,7 @@ def plain(*projs) -> bool:
     return get_tp_world_size() == 1 and not hooked(*projs)
 
 
+@passed_by
 class ReplicatedLinear(nn.Module):
     def __init__(self, input_size, output_size, bias=False, dtype=None):
         super().__init__()
@@ -120,6 +121,7 @@ class ReplicatedLinear(nn.Module):
     quantize_fp8 = _quantize_fp8
 
 
+@passed_by
 class ColumnParallelLinear(nn.Module):
     """Output-dim sharded: Y_local = X @ W_local^T. No communication in
     forward (unless gather_output)."""
@@ -186,6 +188,7 @@ class ColumnParallelLinear(nn.Module):
         return full.chunk(tp, dim=0)[rank]
 
 
+@passed_by
 class MergedColumnParallelLinear(ColumnParallelLinear):
     """Several column-parallel projections fused into one GEMM
     (e.g. gate_proj + up_proj). Each sub-output is sharded separately."""
@@ -209,6 +212,7 @@ class MergedColumnParallelLinear(ColumnParallelLinear):
                          dim=0)
 
 
+@passed_by
 class QKVParallelLinear(ColumnParallelLinear):
     """Fused QKV projection, head-aware sharding. KV heads are replicated
     when tp > num_kv_heads."""
@@ -282,6 +286,7 @@ class QKVParallelLinear(ColumnParallelLinear):
                           v.chunk(kv_chunks, dim=0)[kv_rank]], dim=0)
 
 
+@passed_by
 class RowParallelLinear(nn.Module):
     """Input-dim sharded: Y = sum_ranks(X_local @ W_local^T) via all-reduce.
     The all-reduce is the per-layer TP collective (reference linear.py:1767)."""

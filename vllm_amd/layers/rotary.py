@@ -14,6 +14,7 @@ import torch
 import torch.nn as nn
 
 from vllm_amd import ops
+from vllm_amd.layers.hooks import passed_by
 
 
 def _compute_inv_freq(rotary_dim: int, theta: float) -> torch.Tensor:
@@ -88,6 +89,7 @@ def _apply_yarn_scaling(inv_freq: torch.Tensor, scaling: dict, dim: int,
     return out, float(mscale * attn_factor)
 
 
+@passed_by
 class RotaryEmbedding(nn.Module):
     def __init__(
         self,

@@ -17,7 +17,7 @@ from vllm_amd.layers.activation import SiluAndMul
 from vllm_amd.layers.attention import Attention
 from vllm_amd.worker.forward_context import get_forward_context
 from vllm_amd.layers.embedding import ParallelLMHead, VocabParallelEmbedding
-from vllm_amd.layers.hooks import hooked
+from vllm_amd.layers.hooks import hooked, passed_by
 from vllm_amd.layers.layernorm import LayerNorm, RMSNorm
 from vllm_amd.layers.linear import (
     MergedColumnParallelLinear,
@@ -35,6 +35,7 @@ from vllm_amd.parallel.state import (
 )
 
 
+@passed_by
 class LlamaMLP(nn.Module):
     def __init__(self, spec: ModelSpec, dtype: torch.dtype):
         super().__init__()
@@ -71,6 +72,7 @@ class LlamaMLP(nn.Module):
         return self.down_proj(x, reduce_results=reduce_results)
 
 
+@passed_by
 class LlamaAttention(nn.Module):
     def __init__(self, spec: ModelSpec, layer_idx: int, dtype: torch.dtype,
                  max_position: int, cache_idx: int = -1):
@@ -158,6 +160,7 @@ class LlamaAttention(nn.Module):
                 and positions.dim() == 1)
 
 
+@passed_by
 class LlamaDecoderLayer(nn.Module):
     def __init__(self, spec: ModelSpec, layer_idx: int, dtype, max_position,
                  cache_idx: int = -1):
@@ -308,6 +311,15 @@ class LlamaModel(nn.Module):
                               dtype=dtype)
                      if is_last_pp_rank() else None)
 
+    def streams(self, layers) -> bool:
+        """Whether all layers go on the residual stream, or none: what hooks,
+        or modules in the place of others, are called with stays the same.
+        (The last norm gets the sum as one.)"""
+        return (all([type(layer) is LlamaDecoderLayer and layer.streams()
+                     for layer in layers])
+                and (self.norm is None or type(self.norm) is RMSNorm
+                     and not hooked(self.norm)))
+
     def forward(self, input_ids, positions, hidden_in=None):
         ctx = get_forward_context()
         if self.embed_tokens is not None:
@@ -332,9 +344,8 @@ class LlamaModel(nn.Module):
             r = get_tp_rank()
             hidden = hidden[r * shard:(r + 1) * shard]
         layers = list(self.layers)[self.lo:self.hi]
-        # All layers or none: what a hook on one of them sees stays the same.
         if (sp == 1 and ops.layer_streams(hidden, *self.stream_sizes)
-                and all([layer.streams() for layer in layers])):
+                and self.streams(layers)):
             for layer in layers:
                 hidden = layer.forward_stream(positions, hidden)
             return hidden if self.norm is None else self.norm(hidden)
