@@ -195,3 +195,45 @@ def test_the_last_norm_is_called_as_before(net, monkeypatch, change):
     got = _step(net)
     assert seen == [2]
     _same(got, _by_modules(net, monkeypatch))
+
+
+@pytest.mark.parametrize("name", ["q_a_proj", "kv_a_proj_with_mqa",
+                                  "kv_a_layernorm", "rotary_emb"])
+def test_wrapped_modules_of_latent_attention_are_called(name):
+    from vllm_amd.models.deepseek import DeepseekMLAAttention
+
+    spec = get_model_spec("tiny-deepseek")
+    torch.manual_seed(0)
+    block = DeepseekMLAAttention(spec, 0, torch.float32, 64)
+    for p in block.parameters():
+        nn.init.normal_(p, std=0.05)
+
+    def step():
+        torch.manual_seed(1)
+        cache = torch.randn(2, 64, spec.kv_lora_rank + spec.qk_rope_head_dim)
+        meta = AttentionMetadata(
+            query_start_loc=torch.arange(3, dtype=torch.int32),
+            seq_lens=torch.tensor([4, 9], dtype=torch.int32),
+            block_table=torch.tensor([[0], [1]], dtype=torch.int32),
+            slot_mapping=torch.tensor([3, 64 + 8]), num_reqs=2,
+            num_actual_tokens=2, max_query_len=1, max_seq_len=9,
+            num_decodes=2)
+        x = torch.randn(2, spec.hidden_size)
+        with torch.inference_mode(), set_forward_context(
+                ForwardContext(attn_metadata=meta, kv_caches=[cache])):
+            return block(torch.tensor([3, 8]), x), cache
+
+    expect = step()
+    wrapped = Wrapped(getattr(block, name))
+    setattr(block, name, wrapped)
+    got = step()
+    assert wrapped.calls == 1
+    for a, b in zip(got, expect):
+        torch.testing.assert_close(a, b)
+
+    class OnGpu(torch.Tensor):
+        """Takes the path that GPU tensors take."""
+        is_cuda = True
+
+    block._a_projs(torch.randn(2, spec.hidden_size).as_subclass(OnGpu))
+    block.double()

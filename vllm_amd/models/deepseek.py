@@ -98,10 +98,16 @@ class DeepseekMLAAttention(nn.Module):
         self._join_a_projs()
         return self
 
+    def _a_projs_are_plain(self) -> bool:
+        return (type(self.q_a_proj) is ReplicatedLinear
+                and type(self.kv_a_proj_with_mqa) is ReplicatedLinear)
+
     def _joined_a_projs(self):
         """The weights of the two projections of the hidden state as one
         matrix, or None where they do not lie one behind the other in one
-        storage."""
+        storage, or are another module's than these."""
+        if not self._a_projs_are_plain():
+            return None
         q, kv = self.q_a_proj.weight, self.kv_a_proj_with_mqa.weight
         if (q.numel() == 0 or kv.numel() == 0 or q.dtype != kv.dtype
                 or q.device != kv.device
@@ -118,7 +124,8 @@ class DeepseekMLAAttention(nn.Module):
         behind the other, so that _a_projs can take them as one matrix.
         Weights that lie so already stay where they are: a move that
         changes nothing leaves captured graphs and shared memory valid."""
-        if self.q_a_proj is None or self._joined_a_projs() is not None:
+        if (not self._a_projs_are_plain()
+                or self._joined_a_projs() is not None):
             return
         q, kv = self.q_a_proj.weight, self.kv_a_proj_with_mqa.weight
         if q.numel() == 0 or q.dtype != kv.dtype or q.device != kv.device:
@@ -133,7 +140,8 @@ class DeepseekMLAAttention(nn.Module):
         22.7, 3901 132 / 102, 8192 215 / 218)."""
         q, kv = self.q_a_proj, self.kv_a_proj_with_mqa
         both = None
-        if (hidden.is_cuda and hidden.shape[0] <= 4096 and q.bias is None
+        if (hidden.is_cuda and hidden.shape[0] <= 4096
+                and self._a_projs_are_plain() and q.bias is None
                 and kv.bias is None and not hooked(q, kv)):
             both = self._joined_a_projs()
         if both is None:
@@ -183,14 +191,16 @@ class DeepseekMLAAttention(nn.Module):
             out = ops.head_matmul(o_c, self.w_uv)
         else:
             kv_cache = ctx.kv_caches[self.layer_idx]
-            if hooked(self.kv_a_layernorm, self.rotary_emb):
+            norm, rope = self.kv_a_layernorm, self.rotary_emb
+            if (type(norm) is not RMSNorm or type(rope) is not RotaryEmbedding
+                    or hooked(norm, rope)):
                 c_kv, q_pe, k_pe = self._prepare(positions, q_pe, kv_a)
                 ops.concat_and_cache_mla(c_kv, k_pe, kv_cache,
                                          meta.slot_mapping)
             else:
                 q_pe = ops.mla_prepare(
-                    positions, q_pe, kv_a, self.kv_a_layernorm.weight,
-                    self.kv_a_layernorm.eps, self.rotary_emb.cos_sin_cache,
+                    positions, q_pe, kv_a, norm.weight, norm.eps,
+                    rope.cos_sin_cache,
                     kv_cache, meta.slot_mapping)
             out = ops.mla_heads(
                 q_nope, q_pe, self.w_uk, self.w_uv, kv_cache,
