@@ -181,7 +181,9 @@ def test_norm_linear(m, n, k):
     (50, 2, 1, 64, 4096, torch.bfloat16), (64, 64, 8, 128, 8192,
                                            torch.bfloat16),
     (5, 2, 2, 96, 512, torch.bfloat16),
-    (65, 8, 2, 128, 512, torch.bfloat16)])   # as steps of their own
+    (65, 8, 2, 128, 512, torch.bfloat16),   # as steps of their own
+    (4, 8, 2, 40, 512, torch.bfloat16),
+    (3, 16, 4, 72, 576, torch.float8_e4m3fn)])   # heads not of 16s
 def test_norm_qkv_rope_cache(m, hq, hkv, d, k, kv):
     """Against the steps that it stands for."""
     from vllm_amd.ops import hip_ops

@@ -137,6 +137,16 @@ def norm_linear(x, gain, eps, weight, bias=None, silu=False):
 
 def norm_qkv_rope_cache(x, gain, eps, weight, bias, positions, cos_sin_cache,
                         kv_cache, slot_mapping):
+    kv_heads, head_dim = kv_cache.shape[2], kv_cache.shape[4]
+    if head_dim % 16:
+        # rope_and_cache knows what to do with these.
+        qkv = norm_linear(x, gain, eps, weight, bias).view(
+            x.shape[0], -1, head_dim)
+        q, k, v = qkv.split([qkv.shape[1] - 2 * kv_heads, kv_heads, kv_heads],
+                            dim=1)
+        rope_and_cache(positions, q, k, v, cos_sin_cache, head_dim, True,
+                       kv_cache, slot_mapping)
+        return q
     return _C.norm_qkv_rope_cache(x, gain, eps, weight, bias, positions,
                                   slot_mapping, cos_sin_cache, kv_cache)
 
