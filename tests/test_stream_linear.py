@@ -252,6 +252,42 @@ def test_linear_add(m, n, k, dtype):
 
 
 @gpu
+@pytest.mark.parametrize("op,operands", [
+    ("lt_linear", "wb"), ("linear_silu_and_mul", "w"), ("linear_add", "wbr"),
+    ("norm_linear", "gwb"), ("norm_qkv_rope_cache", "gwbpstc"),
+    ("lt_linear_fp8", "w")])
+def test_operands_elsewhere_are_refused(op, operands):
+    """Before anything is launched: their addresses mean nothing there."""
+    from vllm_amd.ops import hip_ops
+    call = getattr(hip_ops._C, op)
+    rows, d, heads = 8, 64, 4
+    x, w = _operands(rows, heads * d, 512, torch.bfloat16)
+    have = dict(
+        w=w, b=w[:, 0].contiguous(), g=x[0].clone(), r=x[:, :256].clone(),
+        p=torch.zeros(rows, dtype=torch.int64, device="cuda"),
+        s=torch.arange(rows, device="cuda"),
+        t=torch.zeros(16, d, device="cuda"),
+        c=torch.zeros(2, 1, 1, 16, d, dtype=x.dtype, device="cuda"))
+    order = dict(lt_linear="wb", linear_silu_and_mul="w", linear_add="wbr",
+                 norm_linear="g.wb", norm_qkv_rope_cache="g.wbpstc",
+                 lt_linear_fp8="w")[op]
+    if op == "lt_linear_fp8":
+        x, have["w"] = (t.to(torch.float8_e4m3fn) for t in (x, w))
+
+    def run(elsewhere):
+        args = [1e-6 if o == "." else
+                have[o].cpu() if o == elsewhere else have[o] for o in order]
+        if op == "norm_linear":
+            args.append(False)
+        return call(x, *args)
+
+    run(None)
+    for o in operands:
+        with pytest.raises(RuntimeError, match="operands on"):
+            run(o)
+
+
+@gpu
 def test_norms_that_are_not_fused_are_the_same():
     """Rows in fp16 and more rows: a norm, then the product."""
     from vllm_amd.ops import hip_ops

@@ -352,6 +352,8 @@ void run_matmul_fp8(torch::Tensor& out, const torch::Tensor& a,
 }  // namespace
 
 torch::Tensor lt_linear_fp8(torch::Tensor a, torch::Tensor w) {
+  TORCH_CHECK(w.device() == a.device(), "operands on ", w.device(), " and ",
+              a.device());
   auto out = torch::empty({a.size(0), w.size(0)},
                           a.options().dtype(torch::kBFloat16));
   run_matmul_fp8(out, a, w);
@@ -360,6 +362,10 @@ torch::Tensor lt_linear_fp8(torch::Tensor a, torch::Tensor w) {
 
 torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
                         c10::optional<torch::Tensor> bias) {
+  // (An operand elsewhere would be read by its address there.)
+  TORCH_CHECK(w.device() == a.device() &&
+                  (!bias.has_value() || bias->device() == a.device()),
+              "operands on ", w.device(), " and ", a.device());
   auto sizes = a.sizes().vec();
   const int64_t K = sizes.back();
   auto a2 = a.reshape({-1, K}).contiguous();

@@ -42,6 +42,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
 
 #include "arrivals.h"
 #include "stream_product.h"
@@ -588,6 +589,17 @@ torch::Tensor stream_linear(const torch::Tensor& x, const torch::Tensor& w,
   return stream_linear_beside(x, w, beside);
 }
 
+// (An operand elsewhere would be read by its address there.)
+static void check_device(const torch::Tensor& a,
+                         std::initializer_list<const torch::Tensor*> others,
+                         const c10::optional<torch::Tensor>& bias) {
+  for (const torch::Tensor* t : others)
+    TORCH_CHECK(t->device() == a.device(), "operands on ", t->device(),
+                " and ", a.device());
+  TORCH_CHECK(!bias.has_value() || bias->device() == a.device(),
+              "operands on ", bias->device(), " and ", a.device());
+}
+
 static bool bias_fits(const c10::optional<torch::Tensor>& bias,
                       const torch::Tensor& w) {
   return !bias.has_value() ||
@@ -604,9 +616,9 @@ torch::Tensor linear_add(torch::Tensor a, torch::Tensor w,
                   a.scalar_type() == w.scalar_type() &&
                   residual.dim() == 2 && residual.size(0) == a.size(0) &&
                   residual.size(1) == w.size(0) &&
-                  residual.scalar_type() == a.scalar_type() &&
-                  residual.device() == a.device(),
+                  residual.scalar_type() == a.scalar_type(),
               "linear_add: [M, K] x [N, K] + [M, N]");
+  check_device(a, {&w, &residual}, bias);
   auto x = a.contiguous();
   if (x.size(0) == 0 || !residual.is_contiguous() ||
       (uintptr_t)residual.data_ptr() % 8 != 0 || !bias_fits(bias, w))
@@ -677,9 +689,9 @@ torch::Tensor norm_linear(torch::Tensor a, torch::Tensor gains, double eps,
   TORCH_CHECK(a.dim() == 2 && w.dim() == 2 && a.size(1) == w.size(1) &&
                   a.scalar_type() == w.scalar_type() && gains.dim() == 1 &&
                   gains.size(0) == a.size(1) &&
-                  gains.scalar_type() == a.scalar_type() &&
-                  gains.device() == a.device(),
+                  gains.scalar_type() == a.scalar_type(),
               "norm_linear: [M, K] x [N, K], gains [K]");
+  check_device(a, {&gains, &w}, bias);
   TORCH_CHECK(!silu || (w.size(0) % 2 == 0 && !bias.has_value()),
               "norm_linear: the activation takes [gate; up] without a bias");
   auto x = a.contiguous();
@@ -732,6 +744,7 @@ torch::Tensor norm_qkv_rope_cache(
   TORCH_CHECK(kv_cache.scalar_type() == a.scalar_type() ||
                   kv_cache.scalar_type() == torch::kFloat8_e4m3fn,
               "norm_qkv_rope_cache: cache of the rows' type or e4m3");
+  check_device(a, {&gains, &w, &positions, &slots, &cos_sin, &kv_cache}, bias);
   auto x = a.contiguous();
   const int half = (int)D / 2;
   if (x.scalar_type() != torch::kBFloat16 ||
@@ -777,6 +790,7 @@ torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w) {
   TORCH_CHECK(w.dim() == 2 && w.size(0) % 2 == 0 && a.dim() >= 1 &&
               a.size(-1) == w.size(1) && a.scalar_type() == w.scalar_type(),
               "linear_silu_and_mul: [.., K] x [2N, K]");
+  check_device(a, {&w}, c10::nullopt);
   auto sizes = a.sizes().vec();
   auto x = a.reshape({-1, sizes.back()}).contiguous();
   const int64_t N = w.size(0) / 2;
