@@ -303,6 +303,28 @@ def test_norms_that_are_not_fused_are_the_same():
 
 
 @gpu
+@pytest.mark.parametrize("m,n,k", [(8, 1030, 512), (70, 1030, 512),
+                                   (8, 1028, 520), (70, 1028, 512)])
+def test_rows_of_no_whole_16_bytes_beside_norms_and_sums(m, n, k):
+    """These are no products of the aligned kernels (hip_ops.linear)."""
+    from vllm_amd.ops import hip_ops
+    x, w = _operands(m, n, k, torch.bfloat16)
+    gain = torch.rand(k, device="cuda").bfloat16()
+    residual = torch.randn(m, n, device="cuda").bfloat16()
+    y = hip_ops.rms_norm(x, gain, 1e-6)
+    for got, want in [
+            (hip_ops.linear_add(x, w, None, residual),
+             hip_ops.linear(x, w).float() + residual.float()),
+            (hip_ops.norm_linear(x, gain, 1e-6, w),
+             hip_ops.linear(y, w).float()),
+            (hip_ops.norm_linear(x, gain, 1e-6, w, silu=True),
+             hip_ops.linear_silu_and_mul(y, w).float())]:
+        # Rounded twice at most on either side.
+        assert ((got.float() - want).abs()
+                <= 2.0 ** -6 * (want.abs() + want.abs().mean())).all()
+
+
+@gpu
 @pytest.mark.parametrize("rows", [1, 8, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("model", ["llama-3-8b", "qwen2.5-7b"])
 def test_layers_on_the_residual_stream(model, rows):

@@ -50,10 +50,11 @@
 
 namespace vllm_amd {
 
-// gemm_hipblaslt.cpp, elementwise.hip
+// gemm_hipblaslt.cpp, elementwise.hip, pooled_attention.hip
 torch::Tensor lt_linear(torch::Tensor a, torch::Tensor w,
                         c10::optional<torch::Tensor> bias);
 torch::Tensor silu_and_mul(torch::Tensor x);
+torch::Tensor silu_and_mul_any(torch::Tensor x);
 torch::Tensor rms_norm(torch::Tensor x, torch::Tensor weight, double eps);
 torch::Tensor linear_silu_and_mul(torch::Tensor a, torch::Tensor w);
 void rope_and_cache(torch::Tensor positions, torch::Tensor q, torch::Tensor k,
@@ -600,6 +601,16 @@ static void check_device(const torch::Tensor& a,
               "operands on ", bias->device(), " and ", a.device());
 }
 
+// A product by itself. (Rows that are not multiples of 16 B fall outside the
+// aligned kernels, the library's own among them.)
+static torch::Tensor product(const torch::Tensor& x, const torch::Tensor& w,
+                             const c10::optional<torch::Tensor>& bias) {
+  const int64_t per16 = 16 / x.element_size();
+  if (w.size(0) % per16 != 0 || w.size(1) % per16 != 0)
+    return at::linear(x, w, bias);
+  return lt_linear(x, w, bias);
+}
+
 static bool bias_fits(const c10::optional<torch::Tensor>& bias,
                       const torch::Tensor& w) {
   return !bias.has_value() ||
@@ -622,7 +633,7 @@ torch::Tensor linear_add(torch::Tensor a, torch::Tensor w,
   auto x = a.contiguous();
   if (x.size(0) == 0 || !residual.is_contiguous() ||
       (uintptr_t)residual.data_ptr() % 8 != 0 || !bias_fits(bias, w))
-    return lt_linear(x, w, bias) + residual;
+    return product(x, w, bias) + residual;
   const bool tiles = !bias.has_value() &&
                      tile_linear_first(x.size(0), w.size(0), x.size(1), false);
   if (tiles || !stream_linear_takes(x, w, w.size(0))) {
@@ -630,7 +641,7 @@ torch::Tensor linear_add(torch::Tensor a, torch::Tensor w,
     if (!bias.has_value() &&
         tile_linear_add(out, x, w, false, (const short*)residual.data_ptr()))
       return out;
-    return lt_linear(x, w, bias) + residual;
+    return product(x, w, bias) + residual;
   }
   Beside beside;
   if (bias.has_value()) beside.bias = (const short*)bias->data_ptr();
@@ -701,7 +712,10 @@ torch::Tensor norm_linear(torch::Tensor a, torch::Tensor gains, double eps,
       !bias_fits(bias, w) || !stream_linear_takes(x, w, N) ||
       !norm_sizes(x.size(0), w.size(0), x.size(1), silu)) {
     auto y = rms_norm(x, gains, eps);
-    return silu ? linear_silu_and_mul(y, w) : lt_linear(y, w, bias);
+    if (!silu) return product(y, w, bias);
+    if (w.size(0) % 16 == 0 && w.size(1) % 8 == 0)
+      return linear_silu_and_mul(y, w);
+    return silu_and_mul_any(product(y, w, c10::nullopt));
   }
   Beside beside;
   if (bias.has_value()) beside.bias = (const short*)bias->data_ptr();
