@@ -442,6 +442,28 @@ def test_lt_linear(m, k, n, bias):
     assert_close(out, expect, atol=5e-2, rtol=5e-2)
 
 
+@pytest.mark.parametrize("first", ["fp32", "fp8"])
+def test_algorithms_are_chosen_by_types(first):
+    """Products of the same sizes in fp32 and in fp8, one after the other:
+    each runs by an algorithm of its own types."""
+    hip = _hip()
+    m, n, k = (272, 640, 512) if first == "fp32" else (272, 512, 640)
+    a = torch.randint(-4, 5, (m, k), device="cuda").float() / 4
+    w = torch.randint(-4, 5, (n, k), device="cuda").float() / 4
+    expect = a @ w.t()   # fp8 holds these, fp32 their sums
+
+    def fp32():
+        assert torch.equal(hip._C.lt_linear(a, w, None), expect)
+
+    def fp8():
+        out = hip._C.lt_linear_fp8(a.to(torch.float8_e4m3fn),
+                                   w.to(torch.float8_e4m3fn))
+        assert torch.equal(out, expect.bfloat16())
+
+    for run in (fp32, fp8) if first == "fp32" else (fp8, fp32):
+        run()
+
+
 def test_fused_moe_matches_reference():
     T, H, I, E, K = 37, 256, 512, 4, 2
     hidden = torch.randn(T, H, dtype=torch.bfloat16, device="cuda") * 0.1

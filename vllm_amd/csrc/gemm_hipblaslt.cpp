@@ -21,8 +21,9 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <mutex>
-#include <unordered_map>
+#include <tuple>
 #include <vector>
 
 #include "common.h"
@@ -58,10 +59,22 @@ namespace {
 
 constexpr size_t kWorkspaceBytes = 128ull * 1024 * 1024;
 
+// What an algorithm is chosen for, in full: products of other types are other
+// products, whatever their sizes.
+struct ProductKey {
+  int64_t m, n, k;
+  hipDataType in, out;
+  bool bias;
+  bool operator<(const ProductKey& o) const {
+    return std::tie(m, n, k, in, out, bias) <
+           std::tie(o.m, o.n, o.k, o.in, o.out, o.bias);
+  }
+};
+
 struct LtContext {
   hipblasLtHandle_t handle{nullptr};
   void* workspace{nullptr};
-  std::unordered_map<uint64_t, hipblasLtMatmulAlgo_t> algo_cache;
+  std::map<ProductKey, hipblasLtMatmulAlgo_t> algo_cache;
   std::mutex mu;
 };
 
@@ -73,12 +86,6 @@ LtContext& ctx() {
     HIP_CHECK(hipMalloc(&c.workspace, kWorkspaceBytes));
   });
   return c;
-}
-
-uint64_t shape_key(int64_t m, int64_t n, int64_t k, bool bf16, bool bias) {
-  // m<=2^24 buckets suffice; key layout: [m:24][n:20][k:18][dtype:1][bias:1]
-  return ((uint64_t)m << 40) ^ ((uint64_t)n << 20) ^ ((uint64_t)k << 2) ^
-         ((uint64_t)bf16 << 1) ^ (uint64_t)bias;
 }
 
 // Cache lookup, or race hipBLASLt's candidate algorithms for this
@@ -98,11 +105,11 @@ uint64_t shape_key(int64_t m, int64_t n, int64_t k, bool bf16, bool bias) {
 // winner is the fastest whose result is that of the heuristic's first choice,
 // out of memory that nothing has been left in.
 template <typename Call>
-hipblasLtMatmulAlgo_t pick_algo(uint64_t key, hipblasLtMatmulDesc_t op_desc,
+hipblasLtMatmulAlgo_t pick_algo(const ProductKey& key,
+                                hipblasLtMatmulDesc_t op_desc,
                                 hipblasLtMatrixLayout_t lw,
                                 hipblasLtMatrixLayout_t la,
                                 hipblasLtMatrixLayout_t lc,
-                                hipDataType dt_in, hipDataType dt_out,
                                 hipStream_t stream, const torch::Tensor& out,
                                 Call call) {
   auto& c = ctx();
@@ -131,7 +138,7 @@ hipblasLtMatmulAlgo_t pick_algo(uint64_t key, hipblasLtMatmulDesc_t op_desc,
     std::vector<hipblasLtMatmulHeuristicResult_t> all;
     if (hipblaslt_ext::getAllAlgos(
             c.handle, hipblaslt_ext::GemmType::HIPBLASLT_GEMM,
-            HIPBLAS_OP_T, HIPBLAS_OP_N, dt_in, dt_in, dt_out, dt_out,
+            HIPBLAS_OP_T, HIPBLAS_OP_N, key.in, key.in, key.out, key.out,
             HIPBLAS_COMPUTE_32F, all) == HIPBLAS_STATUS_SUCCESS) {
       const float alpha = 1.f, beta = 0.f;
       for (auto& r : all) {
@@ -265,8 +272,6 @@ void run_matmul(torch::Tensor& out, const torch::Tensor& a,
   HIPBLASLT_CHECK(hipblasLtMatrixLayoutCreate(&lc, dt, N, M, N));
 
   const float alpha = 1.f, beta = 0.f;
-  const uint64_t key = shape_key(M, N, K, is_bf16, has_bias) ^
-                       (is_f32 ? (1ull << 63) : 0ull);
 
   auto call = [&](const hipblasLtMatmulAlgo_t& cand,
                   const torch::Tensor& to, void* space) {
@@ -276,7 +281,8 @@ void run_matmul(torch::Tensor& out, const torch::Tensor& a,
         kWorkspaceBytes, stream);
   };
   hipblasLtMatmulAlgo_t algo =
-      pick_algo(key, op_desc, lw, la, lc, dt, dt, stream, out, call);
+      pick_algo({M, N, K, dt, dt, has_bias}, op_desc, lw, la, lc, stream, out,
+                call);
 
   HIPBLASLT_CHECK(hipblasLtMatmul(
       c.handle, op_desc, &alpha, w.data_ptr(), lw, a.data_ptr(), la, &beta,
@@ -291,7 +297,7 @@ void run_matmul(torch::Tensor& out, const torch::Tensor& a,
 
 // fp8 e4m3 x fp8 e4m3 -> bf16 raw GEMM (no scaling — the caller rescales
 // rows/cols in one fused pass; see quant_fp8.hip). Same tuned-algo cache
-// as the bf16 path, keyed with dtype bit = 0 and a distinct fp8 marker.
+// as the 16-bit and fp32 products.
 // gfx950 fp8 MFMA peak is ~2x bf16, so big prefill GEMMs roughly double.
 void run_matmul_fp8(torch::Tensor& out, const torch::Tensor& a,
                     const torch::Tensor& w) {
@@ -323,9 +329,6 @@ void run_matmul_fp8(torch::Tensor& out, const torch::Tensor& a,
   HIPBLASLT_CHECK(hipblasLtMatrixLayoutCreate(&lc, HIP_R_16BF, N, M, N));
 
   const float alpha = 1.f, beta = 0.f;
-  // fp8 keys get a high tag bit so they can't collide with bf16/fp16
-  // keys of the same shape.
-  const uint64_t key = shape_key(M, N, K, false, false) ^ (1ull << 63);
 
   auto call = [&](const hipblasLtMatmulAlgo_t& cand,
                   const torch::Tensor& to, void* space) {
@@ -335,8 +338,8 @@ void run_matmul_fp8(torch::Tensor& out, const torch::Tensor& a,
         kWorkspaceBytes, stream);
   };
   hipblasLtMatmulAlgo_t algo =
-      pick_algo(key, op_desc, lw, la, lc, HIP_R_8F_E4M3, HIP_R_16BF,
-                stream, out, call);
+      pick_algo({M, N, K, HIP_R_8F_E4M3, HIP_R_16BF, false}, op_desc, lw, la,
+                lc, stream, out, call);
 
   HIPBLASLT_CHECK(hipblasLtMatmul(
       c.handle, op_desc, &alpha, w.data_ptr(), lw, a.data_ptr(), la, &beta,
