@@ -324,8 +324,16 @@ def test_rows_of_no_whole_16_bytes_beside_norms_and_sums(m, n, k):
                 <= 2.0 ** -6 * (want.abs() + want.abs().mean())).all()
 
 
+# A step of 65 rows goes by modules on both sides. Of llama-3-8b's, one ended in a
+# segmentation fault of the host in the first call of the projection back to the
+# hidden state (lt_linear, 65 x 4096 x 4096, bf16, no bias, within the race of
+# the library's algorithms, in inference mode). Its cause is not known.
+ONE_MORE = pytest.param(65, marks=pytest.mark.skip(
+    reason="the race of 65 x 4096 x 4096 ended a process once, cause unknown"))
+
+
 @gpu
-@pytest.mark.parametrize("rows", [1, 8, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("rows", [1, 8, 16, 17, 32, 33, 64, ONE_MORE])
 @pytest.mark.parametrize("model", ["llama-3-8b", "qwen2.5-7b"])
 def test_layers_on_the_residual_stream(model, rows):
     """A step of few rows with norms in products, beside the same step whose
@@ -372,7 +380,8 @@ def test_layers_on_the_residual_stream(model, rows):
 
         embeds = net.model.embed_tokens(ids)
         assert net.model.layers[0].streams()
-        assert ops.layer_streams(embeds, *net.model.stream_sizes)
+        assert ops.layer_streams(embeds, *net.model.stream_sizes) == (
+            rows <= 64)
         out, caches = step()
         seen = []
         net.model.layers[1].register_forward_hook(

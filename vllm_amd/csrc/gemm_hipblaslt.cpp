@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "common.h"
+#include "fault_note.h"
 #include "tile_linear.h"
 
 namespace vllm_amd {
@@ -92,18 +93,30 @@ LtContext& ctx() {
 // (desc, layouts) once — `call` runs the matmul with a given algo — and
 // cache the winner.
 //
-// Candidate pool: the heuristic's 48 PLUS the library's FULL algorithm
-// list (hipblaslt_ext::getAllAlgos, shape-filtered by
-// matmulIsAlgoSupported) — the heuristic alone left ~40% on the table
-// for the decode-shape GEMMs (profiles/r01_summary.md). Two-phase race:
-// one timed rep over every supported candidate, then a longer rerace of
-// the top finishers. VLLM_AMD_GEMM_TUNE=quick restores heuristic-only.
+// Candidate pool: the heuristic's 48 and, where it gains anything, the
+// library's full algorithm list (hipblaslt_ext::getAllAlgos, shape-filtered by
+// matmulIsAlgoSupported). Two-phase race: one timed rep over every supported
+// candidate, then a longer rerace of the top finishers.
+// VLLM_AMD_GEMM_TUNE=quick restores heuristic-only.
 //
 // The full list holds algorithms that say they support a shape and compute
 // something else, and they are fast: at K = 64 they won the race of 64 to 2048
 // rows x 65536 columns with sums of what the workspace held before. So the
 // winner is the fastest whose result is that of the heuristic's first choice,
 // out of memory that nothing has been left in.
+//
+// Nothing vouches for them but that, and a process has ended in a segmentation
+// fault of the host within a race of 65 x 4096 x 4096, for a cause that is not
+// known. So they stay out where they gain nothing: products of 65 to 128 rows
+// with 16 MB of weights and more in 16 bits. us by the heuristic's alone and by
+// all, each the better of two races: 72 rows 4096 x 4096 14.8 and 14.9, 6144 x
+// 4096 19.5 and 19.5, 37888 x 3584 56.3 and 56.5, 5120 x 4096 17.0 and 16.6, 128
+// rows 20.4 and 20.6, 112 rows 4608 x 3584 18.2 and 17.8, 2048 x 4096 10.7 and
+// 10.8 (and a first call of 60 ms takes 10).
+// Smaller weights gain (96 rows, 3072 x 1024 8.6 and 6.6, 1024 x 2048 8.5 and
+// 6.5), and so do some products of more rows (250 x 24576 x 1536 31.4 and 29.5,
+// 1024 x 37888 x 3584 254 and 230). Whatever is called next is noted, so that
+// a process that does not come back says what it was.
 template <typename Call>
 hipblasLtMatmulAlgo_t pick_algo(const ProductKey& key,
                                 hipblasLtMatmulDesc_t op_desc,
@@ -130,18 +143,40 @@ hipblasLtMatmulAlgo_t pick_algo(const ProductKey& key,
       c.handle, op_desc, lw, la, lc, lc, pref, kMaxAlgos, results.data(),
       &found));
   HIPBLASLT_CHECK(hipblasLtMatmulPreferenceDestroy(pref));
-  TORCH_CHECK(found > 0, "hipBLASLt: no algorithms for this GEMM");
   results.resize(found);
+  // (Of one that did not succeed nothing else holds.)
+  const auto failed = [](const hipblasLtMatmulHeuristicResult_t& r) {
+    return r.state != HIPBLAS_STATUS_SUCCESS;
+  };
+  results.erase(std::remove_if(results.begin(), results.end(), failed),
+                results.end());
+  found = (int)results.size();
+  TORCH_CHECK(found > 0, "hipBLASLt: no algorithms for this GEMM");
 
+  FaultNote note;
+  auto say = [&](const char* what, int i, int n) {
+    note.say("algorithms of a library product, %lld x %lld x %lld (rows, "
+             "columns, K; types %d to %d%s): %s, %d of %d (%d by its "
+             "heuristic)", (long long)key.m, (long long)key.n,
+             (long long)key.k, (int)key.in, (int)key.out,
+             key.bias ? ", bias" : "", what, i, n, found);
+  };
   const char* tune = getenv("VLLM_AMD_GEMM_TUNE");
-  if (tune == nullptr || strcmp(tune, "quick") != 0) {
+  const bool gains = key.m <= 64 || key.m > 128 ||
+                     key.n * key.k < (1 << 23) || key.in == HIP_R_32F ||
+                     key.in == HIP_R_8F_E4M3;
+  if (gains && (tune == nullptr || strcmp(tune, "quick") != 0)) {
+    say("listing", 0, 0);
     std::vector<hipblasLtMatmulHeuristicResult_t> all;
     if (hipblaslt_ext::getAllAlgos(
             c.handle, hipblaslt_ext::GemmType::HIPBLASLT_GEMM,
             HIPBLAS_OP_T, HIPBLAS_OP_N, key.in, key.in, key.out, key.out,
             HIPBLAS_COMPUTE_32F, all) == HIPBLAS_STATUS_SUCCESS) {
       const float alpha = 1.f, beta = 0.f;
-      for (auto& r : all) {
+      for (size_t i = 0; i < all.size(); ++i) {
+        auto& r = all[i];
+        if (failed(r)) continue;
+        say("asked whether supported", (int)i, (int)all.size());
         size_t ws = 0;
         if (hipblaslt_ext::matmulIsAlgoSupported(c.handle, op_desc, &alpha,
                                                  lw, la, &beta, lc, lc,
@@ -171,14 +206,18 @@ hipblasLtMatmulAlgo_t pick_algo(const ProductKey& key,
   // Phase A: one rep each over the whole pool.
   std::vector<std::pair<float, int>> ranked;
   ranked.reserve(results.size());
-  for (int i = 0; i < (int)results.size(); ++i)
+  for (int i = 0; i < (int)results.size(); ++i) {
+    say("timed", i, (int)results.size());
     ranked.emplace_back(time_algo(results[i].algo, 1), i);
+  }
   std::sort(ranked.begin(), ranked.end(),
             [](auto& x, auto& y) { return x.first < y.first; });
   // Phase B: rerace the 12 fastest with more reps.
   for (int j = 0; j < std::min<int>(12, (int)ranked.size()); ++j)
-    if (ranked[j].first < 1e30f)
+    if (ranked[j].first < 1e30f) {
+      say("timed again", ranked[j].second, (int)results.size());
       ranked[j].first = time_algo(results[ranked[j].second].algo, 8);
+    }
   std::sort(ranked.begin(),
             ranked.begin() + std::min<int>(12, (int)ranked.size()),
             [](auto& x, auto& y) { return x.first < y.first; });
@@ -188,6 +227,7 @@ hipblasLtMatmulAlgo_t pick_algo(const ProductKey& key,
   const auto space = torch::empty({(int64_t)(kWorkspaceBytes / 4)},
                                   out.options().dtype(torch::kFloat));
   auto run_clean = [&](int i, const torch::Tensor& to) {
+    say("compared", i, (int)results.size());
     space.fill_(NAN);
     to.fill_(NAN);
     return call(results[i].algo, to, space.data_ptr()) ==
