@@ -164,8 +164,8 @@ def test_norm_linear(m, n, k):
               torch.nn.functional.silu(gate) * up)
 
 
-# Heads whose halves hold one to four groups of 16 columns (the widest form has
-# four), whole and with K split; both cache types; rows that are padding.
+# Heads of several sizes in forms of one and two groups of 16 columns of a half,
+# whole and with K split; both cache types; rows that are padding.
 @gpu
 @pytest.mark.parametrize("m,hq,hkv,d,k,kv", [
     (1, 32, 8, 128, 4096, torch.bfloat16),
@@ -186,6 +186,35 @@ def test_norm_linear(m, n, k):
     (3, 16, 4, 72, 576, torch.float8_e4m3fn)])   # heads not of 16s
 def test_norm_qkv_rope_cache(m, hq, hkv, d, k, kv):
     """Against the steps that it stands for."""
+    _check_norm_qkv_rope_cache(m, hq, hkv, d, k, kv)
+
+
+# Every form that takes the rotation along, for 8, 16, 32 and 64 rows, with K
+# whole and split: 16-row groups of weights, waves, ring steps, 8-row groups of
+# x, parts of K.
+@gpu
+@pytest.mark.parametrize("m,hq,hkv,d,k,form", [
+    (1, 1, 1, 32, 128, (2, 4, 2, 1, 1)), (7, 1, 1, 32, 2048, (2, 4, 2, 1, 6)),
+    (9, 1, 1, 32, 128, (2, 4, 2, 2, 1)), (16, 1, 1, 32, 2048, (2, 4, 2, 2, 4)),
+    (17, 1, 1, 32, 128, (2, 4, 2, 4, 1)), (31, 1, 1, 32, 2048, (2, 4, 2, 4, 4)),
+    (33, 1, 1, 32, 128, (2, 4, 2, 8, 1)), (64, 1, 1, 32, 2048, (2, 4, 2, 8, 3)),
+    (8, 32, 32, 64, 128, (4, 4, 2, 1, 1)), (3, 64, 1, 64, 11840, (4, 4, 2, 1, 3)),
+    (13, 96, 2, 64, 128, (4, 4, 2, 2, 1)), (16, 64, 2, 64, 8192, (4, 4, 2, 2, 3)),
+    (32, 80, 16, 64, 128, (4, 4, 2, 4, 1)), (17, 64, 1, 64, 5952, (4, 4, 2, 4, 3)),
+    (50, 80, 16, 64, 128, (4, 4, 2, 8, 1)), (64, 64, 1, 64, 4096, (4, 4, 2, 8, 3)),
+    (5, 28, 28, 96, 128, (6, 4, 2, 1, 1)), (2, 72, 8, 96, 16384, (6, 4, 2, 1, 2)),
+    (16, 72, 8, 96, 128, (6, 4, 2, 2, 1)), (9, 72, 8, 96, 8192, (6, 4, 2, 2, 2)),
+    (32, 72, 8, 96, 128, (6, 4, 2, 4, 1)), (20, 72, 8, 96, 4096, (6, 4, 2, 4, 2)),
+    (8, 80, 16, 128, 128, (8, 4, 2, 1, 1)), (16, 40, 40, 128, 128, (8, 4, 2, 2, 1)),
+    (11, 128, 1, 128, 16384, (8, 4, 2, 2, 3))])
+def test_norm_qkv_rope_cache_in_every_form(m, hq, hkv, d, k, form):
+    from vllm_amd.ops import hip_ops
+    assert hip_ops._C.linear_form(m, (hq + 2 * hkv) * d, k, False, True,
+                                  d // 2) == [1, *form]
+    _check_norm_qkv_rope_cache(m, hq, hkv, d, k, torch.bfloat16)
+
+
+def _check_norm_qkv_rope_cache(m, hq, hkv, d, k, kv):
     from vllm_amd.ops import hip_ops
     rows = (hq + 2 * hkv) * d
     x, w = _operands(m, rows, k, torch.bfloat16)
@@ -413,6 +442,29 @@ def test_layers_that_stream():
     assert not takes(33, 4096, 6144, 4096, 28672, 14336, 0)
     # Residuals that no epilogue takes: tiles with K whole.
     assert not takes(64, 32768, 6144, 4096, 28672, 14336, 64)
+
+
+@pytest.mark.parametrize("rows,weights,k,half,form", [
+    (1, 6144, 4096, 64, [1, 2, 4, 2, 1, 1]),    # the form without the norm
+    (64, 6144, 4096, 64, [1, 2, 4, 2, 8, 1]),
+    (16, 24576, 8192, 64, [1, 8, 4, 2, 2, 1]),  # a wider one
+    (32, 9216, 3072, 48, [1, 2, 4, 2, 4, 1]),   # heads of 96
+    (64, 9216, 3072, 48, [0]),
+    (64, 10240, 8192, 64, [1, 4, 4, 2, 8, 3]),  # K split in both
+    (16, 3840, 11840, 48, [1, 2, 4, 2, 2, 2]),
+    (1, 4096, 7680, 64, [0]),                   # whole, half of the chip
+    (16, 2304, 768, 32, [1, 2, 4, 2, 2, 1]),    # launches are most of it
+    (8, 18432, 4096, 64, [0]),                  # a narrower one
+    (33, 24576, 8192, 64, [0]),                 # two waves, three parts
+    (33, 27648, 4096, 64, [0]),
+    (33, 18432, 4096, 0, [0]),                  # no rotation, past 32 rows
+    (32, 18432, 4096, 0, [1, 6, 4, 2, 4, 1])])
+def test_forms_of_norms_and_rotations(rows, weights, k, half, form):
+    try:
+        from vllm_amd.ops import hip_ops
+    except (ImportError, OSError) as e:
+        pytest.skip(f"extension not built: {e}")
+    assert hip_ops._C.linear_form(rows, weights, k, False, True, half) == form
 
 
 @gpu

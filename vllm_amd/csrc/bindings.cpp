@@ -59,7 +59,7 @@ torch::Tensor norm_qkv_rope_cache(
 bool layer_streams(int64_t rows, int64_t hidden, int64_t qkv, int64_t heads,
                    int64_t gate_up, int64_t inner, int64_t half);
 std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
-                                 bool silu);
+                                 bool silu, bool norm, int64_t half);
 std::vector<int64_t> linear_starts(int64_t rows, int64_t weight_rows,
                                    int64_t k, bool silu);
 int64_t mla_group_heads(int64_t pairs, int64_t heads);
@@ -249,7 +249,8 @@ TORCH_LIBRARY(vllm_amd, m) {
   m.def("layer_streams(int rows, int hidden, int qkv, int heads, "
         "int gate_up, int inner, int half) -> bool",
         &vllm_amd::layer_streams);
-  m.def("linear_form(int rows, int weight_rows, int k, bool silu) -> int[]",
+  m.def("linear_form(int rows, int weight_rows, int k, bool silu, "
+        "bool norm=False, int half=0) -> int[]",
         &vllm_amd::linear_form);
   m.def("linear_starts(int rows, int weight_rows, int k, bool silu) -> int[]",
         &vllm_amd::linear_starts);

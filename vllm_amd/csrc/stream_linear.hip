@@ -182,8 +182,7 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
   s16x4 residual[PER];
   s16x4 bias[PER][2];   // (of turned pairs)
   f32x4 cos[PER], sin[PER];
-  constexpr int SAME = WV % MT == 0 ? 1 : PER;   // row groups of a wave's tiles
-  int64_t slots[SAME];
+  int64_t slot = 0;
   auto early = [&] {
     if constexpr (PAIR == SINGLE && !NORM) {
       if (beside.residual == nullptr) return;
@@ -199,28 +198,21 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     if constexpr (PAIR == ROPE) {
       // By way of the scalar cache: a wait for a load would be one for the
       // fills before it.
-      int pos[SAME];
+      static_assert(WV % MT == 0, "a wave's tiles are of the same rows");
+      const int r0 = wave % MT * 16;
+      int pos = 0;
 #pragma unroll
-      for (int u = 0; u < SAME; ++u) {
-        const int r0 = (u * WV + wave) % MT * 16;
-        pos[u] = 0;
-#pragma unroll
-        for (int r = 0; r < (XG == 1 ? 8 : 16); ++r) {
-          const int p = load_uniform(reinterpret_cast<const int*>(
-              heads.positions + min(r0 + r, M - 1)));
-          if (l16 == r) pos[u] = p;
-        }
+      for (int r = 0; r < (XG == 1 ? 8 : 16); ++r) {
+        const int p = load_uniform(reinterpret_cast<const int*>(
+            heads.positions + min(r0 + r, M - 1)));
+        if (l16 == r) pos = p;
       }
-#pragma unroll
-      for (int u = 0; u < SAME; ++u)
-        slots[u] =
-            heads.slots[min((u * WV + wave) % MT * 16 + l16, M - 1)];
+      slot = heads.slots[min(r0 + l16, M - 1)];
+      const float* turn = heads.cos_sin + (int64_t)pos * (2 * heads.half);
 #pragma unroll
       for (int u = 0; u < PER; ++u) {
         const int t = min(u * WV + wave, TO - 1);
         const int p = n0 - head * heads.half + (t / MT) * 16 + l4 * 4;
-        const float* turn =
-            heads.cos_sin + (int64_t)pos[u % SAME] * (2 * heads.half);
         cos[u] = *reinterpret_cast<const f32x4*>(turn + p);
         sin[u] = *reinterpret_cast<const f32x4*>(turn + heads.half + p);
         if (beside.bias != nullptr) {
@@ -357,7 +349,6 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
         *reinterpret_cast<int2*>(q + half) = to[1];
         continue;
       }
-      const int64_t slot = slots[u % SAME];
       if (slot < 0) continue;   // padding
       const bool value = head >= heads.q_heads + heads.kv_heads;
       const int kvh = head - heads.q_heads - (value ? heads.kv_heads : 0);
@@ -395,7 +386,7 @@ __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
   }
 }
 
-struct Plan { int form, parts; };
+struct Plan { int form, parts; double us; };
 
 // Form and parts of K by an estimate of the time. Its terms (added as fourth
 // powers): weights at 6 TB/s; all that enters workgroups, x again in each, at
@@ -408,13 +399,14 @@ struct Plan { int form, parts; };
 // half: 0, or columns of half a head, which tiles must not pass.
 Plan plan(int xg, int64_t rows_w, int K, bool silu, bool norm = false,
           int half = 0) {
-  Plan best{-1, 1};
-  double least = 1e30;
+  Plan best{-1, 1, 1e30};
   auto fourth = [](double v) { return v * v * v * v; };
   for (int i = 0; i < SL_NFORMS; ++i) {
     const Form f = SL_FORMS[i];
-    // Two waves have too little on the way where four fit.
-    if ((f.wv == 2 && xg < 8) || ((silu || half > 0) && f.ni % 2 != 0) ||
+    // Two waves have too little on the way where four fit, and are slow to
+    // multiply rows by gains (4096 x 27648 with the rotation, 33 rows 47.7 us
+    // in launches and 54.9 in one).
+    if ((f.wv == 2 && (xg < 8 || norm)) || ((silu || half > 0) && f.ni % 2 != 0) ||
         (half > 0 && half % (f.ni * 8) != 0))
       continue;
     const int64_t tiles = (rows_w + f.ni * 16 - 1) / (f.ni * 16);
@@ -436,10 +428,7 @@ Plan plan(int xg, int64_t rows_w, int K, bool silu, bool norm = false,
                                      fourth(load * mb / 0.06))) +
                  0.2 * jobs / 256;
       if (parts > 1) t += 1.5 + 0.04 * parts * f.ni * xg;
-      if (t < least) {
-        least = t;
-        best = {i, parts};
-      }
+      if (t < best.us) best = {i, parts, t};
     }
   }
   return best;
@@ -450,7 +439,8 @@ void launch_form(torch::Tensor& out, const torch::Tensor& x,
                  const torch::Tensor& w, const Beside& beside,
                  const Heads& heads, int N, int parts) {
   constexpr Form f = SL_FORMS[I];
-  if constexpr (lds_bytes(f, XG, NORM) <= SL_LDS && (f.wv > 2 || XG == 8) &&
+  if constexpr (lds_bytes(f, XG, NORM) <= SL_LDS &&
+                (f.wv > 2 || (XG == 8 && !NORM)) &&
                 (!PAIR || f.ni % 2 == 0)) {
     const int lds =
         lds_bytes(f, XG, NORM ? ceil_div((int)x.size(1) / SP_K, parts) : 0);
@@ -549,25 +539,6 @@ bool stream_linear_takes(const torch::Tensor& x, const torch::Tensor& w,
          (uintptr_t)w.data_ptr() % 16 == 0;
 }
 
-// What a product of these sizes runs as, for 16-bit operands that begin on
-// 16 B: {0} the library, {1, 16-row groups of weights, waves, ring steps,
-// 8-row groups of x, parts of K} stream_linear, {2, weight rows of a tile,
-// parts of K} tile_linear.
-std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
-                                 bool silu) {
-  const int64_t n = silu ? weight_rows / 2 : weight_rows;
-  if (!tile_linear_first(rows, weight_rows, k, silu) &&
-      stream_sizes(rows, weight_rows, n, k)) {
-    const int xg = row_groups(rows);
-    const Plan p = plan(xg, weight_rows, (int)k, silu);
-    const Form f = SL_FORMS[p.form];
-    return {1, f.ni, f.wv, f.d, xg, p.parts};
-  }
-  const TileForm tile = tile_linear_form(rows, weight_rows, k, silu);
-  if (tile.cols == 0) return {0};
-  return {2, tile.cols, tile.parts};
-}
-
 // x, w and what is beside them as stream_linear_takes and the callers have
 // checked them.
 static torch::Tensor stream_linear_beside(const torch::Tensor& x,
@@ -651,13 +622,28 @@ torch::Tensor linear_add(torch::Tensor a, torch::Tensor w,
 
 // Whether the norm of `rows` rows goes with the product (bf16 only: fp16 rows
 // times gains may pass 65504 where normalized ones do not). Up to 32 rows, if
-// the gains leave room for the form that the product takes without them, and
-// with half a head's columns up to 64 rows in any form, since a launch for the
-// rotation goes too. us with the launches that go, and in one (4096 x 6144 with
-// the rotation, 4096 x 28672 and 3584 x 37888 with the activation): 8 rows 16.0
-// and 12.0, 38.0 and 35.5, 48.0 and 45.9; 32 rows 19.1 and 14.4, 39.5 and 41.4
-// (another form: not taken), 53.1 and 51.5; 64 rows 22.8 and 18.8, tiles, 53.7
-// and 59.7 (rows are multiplied by gains in two waves: not taken).
+// the gains leave room for the form that the product takes without them. us with
+// the launches that go, and in one (4096 x 6144 with the rotation, 4096 x 28672
+// and 3584 x 37888 with the activation): 8 rows 16.0 and 12.0, 38.0 and 35.5,
+// 48.0 and 45.9; 32 rows 19.1 and 14.4, 39.5 and 41.4 (another form: not
+// taken), 53.1 and 51.5; 64 rows 22.8 and 18.8, tiles, and two waves.
+//
+// half: columns of half a head, if the rotation goes with the product too. Then
+// up to 64 rows in that form. Heads whose halves its tiles do not fit (64
+// columns, and 96 weight rows of a tile) take another one. That may cost more
+// than the launches, up to 60 % of the product, and where depends on how tiles
+// come out on 256 CUs, which the estimate knows to 2 us at best. So other forms
+// are taken, unless the estimate is that far behind, by what held for 139 of
+// 141 products of 128 to 12288 columns (two lost 3 %). us apart and in one:
+//  * K split over workgroups: 10240 x 8192, 33 and 64 rows 43.3 and 43.3, 46.6
+//    and 44.7; 3840 x 11840, 16 rows 26.6 and 20.5. (Not split, of narrow
+//    layers: 4096 x 7680, 1 row 17.6 and 20.1.)
+//  * wider tiles: 24576 x 8192, 16 rows 76.1 and 61.8. (Narrower ones: 18432 x
+//    4096, 8 rows 30.7 and 34.5.)
+//  * 32 weight rows for 64, up to 32 rows: 9216 x 3072 (heads of 96), 16 and 32
+//    rows 19.6 and 17.2, 21.7 and 20.6. (64 rows 25.9 and 36.4.)
+//  * up to 16 rows of up to 2048 columns, where launches are most of the time:
+//    2304 x 768 8.9 and 5.1.
 static bool norm_sizes(int64_t rows, int64_t weight_rows, int64_t k,
                        bool silu, int half = 0) {
   if (tile_linear_first(rows, weight_rows, k, silu) ||
@@ -666,10 +652,36 @@ static bool norm_sizes(int64_t rows, int64_t weight_rows, int64_t k,
     return false;
   const int xg = row_groups(rows);
   const Plan with = plan(xg, weight_rows, (int)k, silu, true, half);
-  if (half > 0) return with.form >= 0;
   const Plan without = plan(xg, weight_rows, (int)k, silu);
-  return rows <= 32 && with.form == without.form &&
-         with.parts == without.parts;
+  if (with.form < 0) return false;
+  if (with.form == without.form && with.parts == without.parts)
+    return half > 0 || rows <= 32;
+  const Form f = SL_FORMS[with.form], other = SL_FORMS[without.form];
+  return half > 0 && with.us < without.us + 2 &&
+         (with.parts > 1 || (f.ni > other.ni && other.ni > 1) ||
+          (f.ni == 2 && other.ni == 4 && rows <= 32) ||
+          (k <= 2048 && rows <= 16));
+}
+
+// What a product of these sizes runs as, for 16-bit operands that begin on
+// 16 B: {0} the library, {1, 16-row groups of weights, waves, ring steps,
+// 8-row groups of x, parts of K} stream_linear, {2, weight rows of a tile,
+// parts of K} tile_linear. norm: of a norm's rows, with half a head's columns
+// where heads turn as a whole; {0} where the norm is a launch of its own.
+std::vector<int64_t> linear_form(int64_t rows, int64_t weight_rows, int64_t k,
+                                 bool silu, bool norm, int64_t half) {
+  const int64_t n = silu ? weight_rows / 2 : weight_rows;
+  if (norm && !norm_sizes(rows, weight_rows, k, silu, (int)half)) return {0};
+  if (!tile_linear_first(rows, weight_rows, k, silu) &&
+      stream_sizes(rows, weight_rows, n, k)) {
+    const int xg = row_groups(rows);
+    const Plan p = plan(xg, weight_rows, (int)k, silu, norm, (int)half);
+    const Form f = SL_FORMS[p.form];
+    return {1, f.ni, f.wv, f.d, xg, p.parts};
+  }
+  const TileForm tile = tile_linear_form(rows, weight_rows, k, silu);
+  if (tile.cols == 0) return {0};
+  return {2, tile.cols, tile.parts};
 }
 
 // Whether the residual goes with the product, without a bias.
