@@ -430,6 +430,8 @@ def test_layers_that_stream():
         from vllm_amd.ops import hip_ops
     except (ImportError, OSError) as e:
         pytest.skip(f"extension not built: {e}")
+    # Asked in every step, of any number of rows: what is kept is bounded.
+    assert hip_ops.layer_streams.cache_info().maxsize is not None
     llama = (4096, 6144, 4096, 28672, 14336, 64)
     takes = hip_ops._C.layer_streams
     assert takes(1, *llama) and takes(64, *llama) and not takes(65, *llama)

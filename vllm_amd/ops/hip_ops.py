@@ -155,9 +155,9 @@ def linear_add(x, weight, bias, residual):
     return _C.linear_add(x, weight, bias, residual)
 
 
-@functools.lru_cache(maxsize=None)
+@functools.lru_cache(maxsize=1024)
 def layer_streams(rows, hidden, qkv, heads, gate_up, inner, half):
-    # Up to 64 rows (csrc/stream_linear.hip).
+    # Up to 64 rows (csrc/stream_linear.hip). (Prompts come in any number.)
     return _C.layer_streams(rows, hidden, qkv, heads, gate_up, inner, half)
 
 
