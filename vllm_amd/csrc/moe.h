@@ -79,9 +79,12 @@ DEVINL bool tile_of_block(const int* __restrict__ expert_tiles, int tiles,
   const int expert = __builtin_amdgcn_readlane(it, 32);
   const uint64_t other =
       __ballot(near < p.m0 || near >= p.m1 || it != expert);
-  const uint32_t low = (uint32_t)other, high = (uint32_t)(other >> 32);
-  int first = at - (low ? __builtin_clz(low) : 32);
-  int end = at + (high ? __builtin_ctz(high) : 32);
+  // (A bit behind the 32 to either side ends the count. As a select of 32
+  // where there is none, the compiler had it read another compare's
+  // condition: tests/test_conditions.py.)
+  const uint64_t low = other << 32, high = other >> 32;
+  int first = at - __builtin_clzll(low | 1ull << 31);
+  int end = at + __builtin_ctzll(high | 1ull << 32);
   for (bool more = low == 0; more && first > p.m0; ) {
     const int i = first - 1 - lane;
     const uint64_t o =
