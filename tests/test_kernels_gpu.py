@@ -643,21 +643,33 @@ def test_moe_grouped_gemm_kernel(T, H, I, E, K):
 
 
 # An expert of more row tiles than a wave finds at a time, between one of a row
-# and one of a group and a tile.
+# and one of a group and a tile: 77 row tiles, in the second product all of them
+# on every XCD (24 column blocks in 8 parts).
 def test_moe_expert_of_many_tiles():
     hip = _hip()
-    H, I, E = 128, 64, 4
+    H, I, E = 6144, 64, 4
     rows = [1, 66 * 256 + 5, 2300, 0]
     T = sum(rows)
     assert hip._moe_form(T, T, E, H) == 2
-    hidden = torch.randn(T, H, dtype=torch.bfloat16, device="cuda") * 0.3
+    experts = [e for e, n in enumerate(rows) for _ in range(-(-n // 256))]
+    flat = hip._C.moe_tile_order(experts, H // 256, 8)
+    assert {(m, n) for m, n in zip(flat[1::3], flat[2::3])} == {
+        (m, n) for m in range(len(experts)) for n in range(H // 256)}
+    assert flat[::3].count(0) == len(experts) * 3   # an eighth of the blocks
+    hidden = torch.randn(T, H, dtype=torch.bfloat16, device="cuda") * 0.04
     w13 = torch.randn(E, 2 * I, H, dtype=torch.bfloat16, device="cuda") * 0.2
     w2 = torch.randn(E, H, I, dtype=torch.bfloat16, device="cuda") * 0.2
     ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))
     ids = ids[torch.randperm(T)].view(T, 1).cuda()
     w = torch.rand(T, 1, device="cuda")
     out = hip.fused_moe_hip(hidden, w13, w2, w, ids)
-    expect = ref.fused_moe(hidden.float(), w13.float(), w2.float(), w, ids)
+    # An expert at a time: the reference's products are of all tokens.
+    expect = torch.empty_like(hidden, dtype=torch.float32)
+    for e in range(E):
+        mine = ids[:, 0] == e
+        gate, up = (hidden[mine].float() @ w13[e].float().t()).chunk(2, -1)
+        act = torch.nn.functional.silu(gate) * up
+        expect[mine] = act @ w2[e].float().t() * w[mine]
     assert_close(out, expect, atol=8e-2, rtol=8e-2)
 
 
