@@ -64,7 +64,8 @@ std::vector<int64_t> linear_starts(int64_t rows, int64_t weight_rows,
                                    int64_t k, bool silu);
 int64_t mla_group_heads(int64_t pairs, int64_t heads);
 std::vector<int64_t> moe_tile_order(std::vector<int64_t> expert_of,
-                                    int64_t n_blocks, int64_t split);
+                                    int64_t n_blocks, int64_t split,
+                                    int64_t tile_rows);
 torch::Tensor lt_linear_fp8(torch::Tensor a, torch::Tensor w);
 void dynamic_quant_fp8(torch::Tensor out, torch::Tensor scales,
                        torch::Tensor x);
@@ -254,7 +255,8 @@ TORCH_LIBRARY(vllm_amd, m) {
         &vllm_amd::linear_form);
   m.def("linear_starts(int rows, int weight_rows, int k, bool silu) -> int[]",
         &vllm_amd::linear_starts);
-  m.def("moe_tile_order(int[] expert_of, int n_blocks, int split) -> int[]",
+  m.def("moe_tile_order(int[] expert_of, int n_blocks, int split, "
+        "int tile_rows=256) -> int[]",
         &vllm_amd::moe_tile_order);
   m.def("mla_group_heads(int pairs, int heads) -> int",
         &vllm_amd::mla_group_heads);

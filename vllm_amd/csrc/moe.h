@@ -34,11 +34,20 @@ DEVINL bool tile_of_block(int m_tiles, int n_blocks, int& m, int& n) {
 // an expert, in equal groups of at most eight, go through the column blocks
 // together: those beside each other share weights, and the blocks rows, in its
 // L2. ms, groups of eight that end anywhere in an expert and these: 64 experts
-// of 7168 x 2048, 8 a token, 4096 tokens 2.75 and 2.66, 1600 unevenly 1.53 and
-// 1.42; 128 of 2048 x 768, 512 tokens 0.253 and 0.243; 8 of 4096 x 14336, 2 a
-// token, 4096 tokens 2.41 and 2.33. Where a part has eight row tiles at most
-// they are one group (the same 8 experts, 400 tokens, a tile each: 0.606, one
-// expert after another 0.633).
+// of 7168 x 2048, 8 a token, 4096 tokens 2.70 and 2.65, 1600 unevenly 1.58 and
+// 1.45; 128 of 2048 x 768, 512 tokens 0.267 and 0.260; 8 of 4096 x 14336, 2 a
+// token, 1700 tokens 1.30 and 1.22, 4096 2.40 and 2.37.
+//
+// Where a part has eight row tiles at most they are one group (the same 8
+// experts, 400 tokens, a tile each: 0.606, one expert after another 0.633). Nor
+// do groups end with their experts where an XCD has all of 16 tiles of 128 rows
+// or fewer: experts of one tile and of two, side by side, wait for weights and
+// multiply at the same time. Of these 8 experts with 330 to 740 tokens (9 to 16
+// tiles, 32 samples), groups that end with their experts took 1.9 % more on
+// average, from 3.7 % less to 6.2 % more (0.670 and 0.712). With tiles of 256 rows
+// they gain 1.3 % from 12 tiles on, and with fewer it is even (-3 to 3 %); as
+// many experts as tiles have nothing to mix (16 of 5120 x 8192, 1 a token, 1000
+// tokens 0.769 and 0.752).
 constexpr int TILE_GROUP = 8;
 struct TilePart { int m0, m1, n0, n1; };   // of an XCD
 inline __host__ __device__ TilePart tile_part_of(int xcd, int tiles,
@@ -59,48 +68,71 @@ inline __host__ __device__ void tile_of_run(int first, int tiles, int blocks,
   m = first + r0 + (q - r0 * blocks) % rows;
   n = (q - r0 * blocks) / rows;
 }
+// Tile l of a part. expert_of(i): of row tile i; ballot(f): the lanes of a wave
+// that f(lane) is true for, of a device's or the host's. few: the part has all
+// row tiles, of 128 rows.
+template <typename Expert, typename Ballot>
+inline __host__ __device__ void tile_of_part(const TilePart& p, bool few,
+                                             int l, const Expert& expert_of,
+                                             const Ballot& ballot, int& m,
+                                             int& n) {
+  const int tiles = p.m1 - p.m0, blocks = p.n1 - p.n0;
+  int first = p.m0, end = p.m1;
+  if (tiles > TILE_GROUP) {
+    if (few && tiles <= 2 * TILE_GROUP && ballot([&](int lane) {
+          const int i = p.m0 + (lane < tiles - 1 ? lane : tiles - 2);
+          return expert_of(i) == expert_of(i + 1);
+        })) {
+      // (Eight and the rest. In two halves 14 tiles lost 3 %.)
+      const int g = l / (TILE_GROUP * blocks), q = l % (TILE_GROUP * blocks);
+      first += g * TILE_GROUP;
+      const int rows = end - first < TILE_GROUP ? end - first : TILE_GROUP;
+      m = first + q % rows;
+      n = p.n0 + q / rows;
+      return;
+    }
+    // The run that row tile `at` is in: 32 to either side come at once.
+    const int at = p.m0 + l / blocks;
+    const int expert = expert_of(at);
+    auto others = [&](int from, int step) -> uint64_t {
+      return ballot([&](int lane) {
+        const int i = from + lane * step;
+        const int in = i < p.m0 ? p.m0 : i < p.m1 ? i : p.m1 - 1;
+        return i != in || expert_of(in) != expert;
+      });
+    };
+    const uint64_t near = others(at - 32, 1);
+    // (A bit behind the 32 to either side ends the count. As a select of 32
+    // where there is none, the compiler had it read another compare's
+    // condition: tests/test_conditions.py.)
+    const uint64_t low = near << 32, high = near >> 32;
+    first = at - __builtin_clzll(low | 1ull << 31);
+    end = at + __builtin_ctzll(high | 1ull << 32);
+    for (bool more = low == 0; more;) {
+      const uint64_t o = others(first - 1, -1);
+      first -= o ? __builtin_ctzll(o) : WAVE_SIZE;
+      more = o == 0;
+    }
+    for (bool more = high == 0; more;) {
+      const uint64_t o = others(end, 1);
+      end += o ? __builtin_ctzll(o) : WAVE_SIZE;
+      more = o == 0;
+    }
+  }
+  tile_of_run(first, end - first, blocks, l - (first - p.m0) * blocks, m, n);
+  n += p.n0;
+}
+template <int TM>
 DEVINL bool tile_of_block(const int* __restrict__ expert_tiles, int tiles,
                           int n_blocks, int split, int& m, int& n) {
   const TilePart p =
       tile_part_of((int)blockIdx.x & 7, tiles, n_blocks, split);
-  const int blocks = p.n1 - p.n0;
   const int l = (int)blockIdx.x >> 3;
-  if (l >= (p.m1 - p.m0) * blocks) return false;
-  if (p.m1 - p.m0 <= TILE_GROUP) {
-    tile_of_run(p.m0, p.m1 - p.m0, blocks, l, m, n);
-    n += p.n0;
-    return true;
-  }
-  // The run that row tile `at` is in: 32 to either side come at once.
-  const int at = p.m0 + l / blocks;
-  const int lane = threadIdx.x % WAVE_SIZE;
-  const int near = at - 32 + lane;
-  const int it = expert_tiles[min(max(near, p.m0), p.m1 - 1)];
-  const int expert = __builtin_amdgcn_readlane(it, 32);
-  const uint64_t other =
-      __ballot(near < p.m0 || near >= p.m1 || it != expert);
-  // (A bit behind the 32 to either side ends the count. As a select of 32
-  // where there is none, the compiler had it read another compare's
-  // condition: tests/test_conditions.py.)
-  const uint64_t low = other << 32, high = other >> 32;
-  int first = at - __builtin_clzll(low | 1ull << 31);
-  int end = at + __builtin_ctzll(high | 1ull << 32);
-  for (bool more = low == 0; more && first > p.m0; ) {
-    const int i = first - 1 - lane;
-    const uint64_t o =
-        __ballot(i < p.m0 || expert_tiles[max(i, p.m0)] != expert);
-    first -= o ? __builtin_ctzll(o) : WAVE_SIZE;
-    more = o == 0;
-  }
-  for (bool more = high == 0; more; ) {
-    const int i = end + lane;
-    const uint64_t o =
-        __ballot(i >= p.m1 || expert_tiles[min(i, p.m1 - 1)] != expert);
-    end += o ? __builtin_ctzll(o) : WAVE_SIZE;
-    more = o == 0;
-  }
-  tile_of_run(first, end - first, blocks, l - (first - p.m0) * blocks, m, n);
-  n += p.n0;
+  if (l >= (p.m1 - p.m0) * (p.n1 - p.n0)) return false;
+  tile_of_part(
+      p, TM == 128 && split == 8, l,
+      [&](int i) { return expert_tiles[i]; },
+      [&](auto f) { return __ballot(f((int)threadIdx.x % WAVE_SIZE)); }, m, n);
   return true;
 }
 

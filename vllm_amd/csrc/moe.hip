@@ -458,24 +458,29 @@ int64_t moe_tile_rows(int64_t form) {
 }
 
 // For the tests: {XCD, row tile, column block} of every tile in the order of
-// its workgroup, where expert_of[i] is the expert of row tile i.
+// its workgroup, where expert_of[i] is the expert of row tile i, and tile_rows
+// 128 or 256.
 std::vector<int64_t> moe_tile_order(std::vector<int64_t> expert_of,
-                                    int64_t n_blocks, int64_t split) {
+                                    int64_t n_blocks, int64_t split,
+                                    int64_t tile_rows) {
   using namespace moe;
   std::vector<int64_t> out;
-  const int tiles = (int)expert_of.size();
   for (int xcd = 0; xcd < 8; ++xcd) {
-    const TilePart p = tile_part_of(xcd, tiles, (int)n_blocks, (int)split);
-    const int blocks = p.n1 - p.n0;
-    const bool one = p.m1 - p.m0 <= TILE_GROUP;
-    for (int l = 0; l < (p.m1 - p.m0) * blocks; ++l) {
-      int first = p.m0 + l / blocks, end = first, m, n;
-      const int64_t expert = expert_of[first];
-      while (first > p.m0 && (one || expert_of[first - 1] == expert)) --first;
-      while (end < p.m1 && (one || expert_of[end] == expert)) ++end;
-      tile_of_run(first, end - first, blocks, l - (first - p.m0) * blocks, m,
-                  n);
-      out.insert(out.end(), {xcd, m, n + p.n0});
+    const TilePart p = tile_part_of(xcd, (int)expert_of.size(),
+                                    (int)n_blocks, (int)split);
+    for (int l = 0; l < (p.m1 - p.m0) * (p.n1 - p.n0); ++l) {
+      int m = 0, n = 0;
+      tile_of_part(
+          p, tile_rows == 128 && split == 8, l,
+          [&](int i) { return expert_of.at(i); },
+          [&](auto f) {
+            uint64_t lanes = 0;
+            for (int lane = 0; lane < WAVE_SIZE; ++lane)
+              lanes |= (uint64_t)f(lane) << lane;
+            return lanes;
+          },
+          m, n);
+      out.insert(out.end(), {xcd, m, n});
     }
   }
   return out;

@@ -109,8 +109,8 @@ template <typename Tag, int ACT, int TM>
 __launch_bounds__(TP_THREADS, 1) __global__
 void moe_tile_kernel(const TileArgs t) {
   int tile, blk;
-  if (!tile_of_block(t.expert_tiles, t.expert_tiles[t.m_tiles], t.n_blocks,
-                     t.split, tile, blk))
+  if (!tile_of_block<TM>(t.expert_tiles, t.expert_tiles[t.m_tiles],
+                         t.n_blocks, t.split, tile, blk))
     return;
   using Whole = TileProduct<Tag, 2, 4, 4, 2, 3>;
   using Half = TileProduct<Tag, 1, 2, 4, 3, 3>;
