@@ -418,10 +418,21 @@ def test_layers_on_the_residual_stream(model, rows):
         expect, old = step()
     assert len(seen) == 1 and seen[0][1] is not None
     # Two layers, each with five roundings by 2^-8 / sqrt(3) of a value at
-    # random: sqrt(10) of them, 0.007 of the result's size, and twice that.
-    for a, b in [(out, expect)] + list(zip(caches, old)):
-        assert ((a.float() - b.float()).norm()
-                <= 0.015 * b.float().norm())
+    # random: sqrt(10) of them, 0.007 of the result's size, and twice that. Of
+    # caches, what the step wrote: row r's key and value, in place r of block r.
+    every = torch.arange(rows, device="cuda")
+
+    def written(c):
+        return c[:, every, :, every].float()
+
+    for a, b in [(out.float(), expect.float())] + [
+            (written(a), written(b)) for a, b in zip(caches, old)]:
+        assert (a - b).norm() <= 0.015 * b.norm()
+    for c in caches + old:
+        assert not torch.equal(written(c), written(cache))
+        rest = c.clone()   # over what it wrote, the state before
+        rest[:, every, :, every] = cache[:, every, :, every]
+        assert torch.equal(rest, cache)
 
 
 def test_layers_that_stream():
