@@ -98,7 +98,8 @@ inline __host__ __device__ void tile_of_part(const TilePart& p, bool few,
       return ballot([&](int lane) {
         const int i = from + lane * step;
         const int in = i < p.m0 ? p.m0 : i < p.m1 ? i : p.m1 - 1;
-        return i != in || expert_of(in) != expert;
+        const bool other = expert_of(in) != expert;   // (no branch)
+        return (i != in) | other;
       });
     };
     const uint64_t near = others(at - 32, 1);
