@@ -66,8 +66,8 @@ class FaultNote {
     const int n = vsnprintf(slot_->line, sizeof slot_->line - 1, format, args);
     va_end(args);
     if (n <= 0) return;
-    const int end = n < (int)sizeof slot_->line - 2 ? n
-                                                    : (int)sizeof slot_->line - 2;
+    const int room = (int)sizeof slot_->line - 2;
+    const int end = n < room ? n : room;
     slot_->line[end] = '\n';
     slot_->length.store(end + 1);
   }

@@ -131,12 +131,15 @@ struct Heads {
 // cache took 2.9 us of a layer: the same, 1 row 508 -> 498 us, 8 rows 512 ->
 // 502. What it read is asked for behind the first fills here, as the residual
 // is, or it would be waited for at the end.)
-// NORM: the product of x's RMS norm. A row's root comes out of the sum (what
-// meets the weights is x * gain, rounded as the normalized row would be), so a
+// NORM: the product of x's RMS norm. A row's root comes out of the sum, so a
 // workgroup needs its squares at the end only, and has them, since all of x
-// passes through it. With the residual as epilogue a layer of few rows keeps
-// no launch for its norms: they took 3.5 us each beside products of 7 to 37
-// (four layers of 4096 and the logits, 1 row 526 -> 508 us, 8 rows 534 -> 512).
+// passes through it. What meets the weights is x * gain instead of x * root *
+// gain, rounded once to the same bits. Where a row lies between powers of two
+// is another place then, so the rounding's share of the result is 0.93 to 1.05
+// of what it was, by the rows' size. With the residual as epilogue a layer of
+// few rows keeps no launch for its norms: they took 3.5 us each beside products
+// of 7 to 37 (four layers of 4096 and the logits, 1 row 526 -> 508 us, 8 rows 534
+// -> 512).
 template <typename Tag, int NI, int XG, int WV, int D, int PAIR, bool NORM>
 __global__ __launch_bounds__(WV * WAVE_SIZE) void stream_linear_kernel(
     short* __restrict__ out, const short* __restrict__ x,

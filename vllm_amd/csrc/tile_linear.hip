@@ -438,7 +438,9 @@ bool tile_linear_add(torch::Tensor& out, const torch::Tensor& x,
                      const short* residual) {
   const int64_t K = x.size(1);
   const TileForm form = tile_linear_form(x.size(0), w.size(0), K, silu);
-  if (form.cols == 0 || (residual != nullptr && (silu || form.parts == 1)) || w.size(1) != K || w.scalar_type() != x.scalar_type() ||
+  if (form.cols == 0 ||
+      (residual != nullptr && (silu || form.parts == 1)) || w.size(1) != K ||
+      w.scalar_type() != x.scalar_type() ||
       (x.scalar_type() != torch::kBFloat16 &&
        x.scalar_type() != torch::kHalf) ||
       !x.is_contiguous() || !w.is_contiguous() ||

@@ -47,9 +47,13 @@ def _decode_parts(rows, kv_heads, max_seq_len, sliding_window, head_dim=128,
     and from a fifth on (8 KV heads of 128) 4 x 2500 11.7 and 14.1, 10.7 and
     12.4; 8 x 4000 23.5 and 24.6, 17.5 and 19.5; 16 x 1200 16.7 and 18.0,
     13.5 and 15.2, x 4000 44.7 and 43.5, 30.7 and 33.2; 2 heads of 256, 6 x
-    4000 17.2 and 21.5; of 9 rows, 216 CUs, x 800..4000 21.4 and 20.3, with 8
-    bits 16 x 800..4000 23.9 and 20.2. At most 64, the lanes of the merging
-    wave.
+    4000 17.2 and 21.5; 10 rows, 240 CUs, x 4000 29.7 and 30.2, 21.7 and 22.9;
+    14, 224 CUs, x 2000 21.1 and 22.7, 17.5 and 18.4; of 9 rows, 216 CUs, x
+    800..4000 21.4 and 20.3, of 13, 208 CUs, x 1200 14.8 and 17.2, 13.1 and
+    12.7; with 8 bits 16 x 800..4000 23.9 and 20.2. (Of 148 shapes of 3 to 16
+    rows in one a CU 9 lose more than 1 %, most of them uneven rows of 800 keys:
+    5 x 160..800 8.8 and 8.5, with heads of 256 11.4 and 10.3.) At most 64, the
+    lanes of the merging wave.
 
     Three steps of a workgroup's waves take no longer than to merge, two of
     twice the steps with heads of 256: us in one partition and in those of
