@@ -133,6 +133,29 @@ def test_adapters_and_fp8_weights_are_not_plain(net, name):
     assert not layer.streams()
 
 
+@pytest.mark.parametrize("name", PROJECTIONS + [
+    "self_attn", "mlp", "mlp.act_fn", "input_layernorm",
+    "post_attention_layernorm"])
+def test_functions_in_the_place_of_modules_are_called(net, monkeypatch, name):
+    layer = net.model.layers[0]
+    parent, _, attr = name.rpartition(".")
+    parent = layer.get_submodule(parent)
+    module, calls = layer.get_submodule(name), []
+    class Function:
+        def __call__(self, *args, **kwargs):
+            calls.append(1)
+            return module(*args, **kwargs)
+
+        def __getattr__(self, what):
+            return getattr(module, what)
+
+    delattr(parent, attr)
+    setattr(parent, attr, Function())
+    got = _step(net)
+    assert len(calls) == 1
+    _same(got, _by_modules(net, monkeypatch))
+
+
 MODULES = PROJECTIONS + ["", "self_attn", "self_attn.attn",
                          "self_attn.rotary_emb", "mlp", "mlp.act_fn",
                          "input_layernorm", "post_attention_layernorm"]

@@ -207,17 +207,17 @@ class LlamaDecoderLayer(nn.Module):
     def streams(self) -> bool:
         """Whether forward_stream does what forward would: a gated layer
         with RMS norms and plain products, no module of which is hooked."""
-        m = self._modules
-        attn, mlp, n1, n2 = (m["self_attn"], m["mlp"], m["input_layernorm"],
-                             m["post_attention_layernorm"])
+        m = self._modules.get
+        attn, mlp, n1, n2 = (m("self_attn"), m("mlp"), m("input_layernorm"),
+                             m("post_attention_layernorm"))
         if (self.parallel_residual or type(attn) is not LlamaAttention
                 or type(mlp) is not LlamaMLP or not mlp.gated
                 or type(n1) is not RMSNorm or type(n2) is not RMSNorm):
             return False
-        a, m = attn._modules, mlp._modules
-        gate_up, act = m["gate_up_proj"], m["act_fn"]
+        a, m = attn._modules.get, mlp._modules.get
+        gate_up, act = m("gate_up_proj"), m("act_fn")
         return (type(act) is SiluAndMul
-                and plain(a["qkv_proj"], a["o_proj"], gate_up, m["down_proj"])
+                and plain(a("qkv_proj"), a("o_proj"), gate_up, m("down_proj"))
                 and gate_up.bias is None
                 and not hooked(self, attn, mlp, act, n1, n2))
 
