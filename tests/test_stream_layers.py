@@ -107,6 +107,17 @@ def test_wrapped_projections_are_called(net, monkeypatch, name):
     _same(got, _by_modules(net, monkeypatch))
 
 
+def test_a_wrapped_rotation_is_called(net, monkeypatch):
+    attn = net.model.layers[0].self_attn
+    expect = _by_modules(net, monkeypatch)
+    attn.rotary_emb = wrapped = Wrapped(attn.rotary_emb)
+    got = _by_modules(net, monkeypatch)
+    assert wrapped.calls == 1
+    _same(got, expect)
+    _step(net)
+    assert wrapped.calls == 2
+
+
 @pytest.mark.parametrize("name", PROJECTIONS)
 def test_parametrized_weights_are_asked_for(net, monkeypatch, name):
     class Twice(nn.Module):

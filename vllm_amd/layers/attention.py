@@ -13,6 +13,7 @@ import torch.nn as nn
 
 from vllm_amd import ops
 from vllm_amd.layers.hooks import hooked, passed_by
+from vllm_amd.layers.rotary import RotaryEmbedding
 from vllm_amd.worker.forward_context import get_forward_context
 
 
@@ -61,7 +62,9 @@ class Attention(nn.Module):
         if v.dim() == 2:
             v = v.view(T, self.num_kv_heads, self.head_dim)
 
-        if rotary is not None and (not ctx.kv_caches or hooked(rotary[1])):
+        if rotary is not None and (not ctx.kv_caches
+                                   or type(rotary[1]) is not RotaryEmbedding
+                                   or hooked(rotary[1])):
             rotary[1](rotary[0], q, k)
             rotary = None
         if not ctx.kv_caches:
