@@ -643,16 +643,20 @@ def test_moe_grouped_gemm_kernel(T, H, I, E, K):
 
 
 # An expert of more row tiles than a wave finds at a time, between one of a row
-# and one of a group and a tile: 77 row tiles, in the second product all of them
-# on every XCD (24 column blocks in 8 parts).
-def test_moe_expert_of_many_tiles():
+# and one of a group and a tile: 77 row tiles of 256, in the second product all
+# of them on every XCD (24 column blocks in 8 parts); and of 128, beside 400.
+@pytest.mark.parametrize("form,rows", [
+    (2, [1, 66 * 256 + 5, 2300, 0]),
+    (1, [1, 66 * 128 + 5, 1100, 0] + [3] * 396)])
+def test_moe_expert_of_many_tiles(form, rows):
     hip = _hip()
-    H, I, E = 6144, 64, 4
-    rows = [1, 66 * 256 + 5, 2300, 0]
+    H, I, E = 6144, 64, len(rows)
     T = sum(rows)
-    assert hip._moe_form(T, T, E, H) == 2
-    experts = [e for e, n in enumerate(rows) for _ in range(-(-n // 256))]
-    flat = hip._C.moe_tile_order(experts, H // 256, 8)
+    assert hip._moe_form(T, T, E, H) == form
+    tile = 128 * form
+    experts = [e for e, n in enumerate(rows) for _ in range(-(-n // tile))]
+    assert experts.count(1) == 67
+    flat = hip._C.moe_tile_order(experts, H // 256, 8, tile)
     assert {(m, n) for m, n in zip(flat[1::3], flat[2::3])} == {
         (m, n) for m in range(len(experts)) for n in range(H // 256)}
     assert flat[::3].count(0) == len(experts) * 3   # an eighth of the blocks
